@@ -142,7 +142,11 @@ int litenn_hip_permute(int dev, void* dst, int dtype, const size_t* src_shape, s
  * matrix cores (the rows padded to a multiple of 16; one padded tile costs about as much as three
  * single-row launches): weights and activations are rounded to fp16 once each (activation rows are first scaled
  * by a power of two into the fp16 range), products accumulate in f32; relative L2 error about
- * 4e-4.  LITENN_HIP_MATMUL_PRECISE in `flags` keeps f32 operands (GEMV path) for any m.
+ * 4e-4.  LITENN_HIP_MATMUL_PRECISE in `flags` keeps f32 operands for any m: Q4_0, Q8_0, Q4_K, Q5_K and Q6_K
+ * with k <= 16384 and m >= 8 on the matrix cores (weights as exact integers, every activation as two halves that carry
+ * its Float32 digits, block scales and sums in f32: the streaming GEMV's accuracy), in scratch of the
+ * device's memory pool or in a given workspace if it has 4.125 * m * k bytes and some (m rounded up to 32, k
+ * to 256); without such room, and for the other formats, row by row through the GEMV, which needs none.
  * The matrix-core path needs a device workspace of litenn_hip_mul_mat_q_workspace_bytes(m, k):
  * litenn_hip_mul_mat_q takes it from the device's memory pool in stream order (hipMallocAsync /
  * hipFreeAsync on the call's stream: no wait for the stream, opts->synchronize is honoured; only

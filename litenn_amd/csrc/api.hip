@@ -15,6 +15,12 @@ namespace litenn_hip
 	int launch_gemv(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y,
 	                const float* residual, hipStream_t stream);
 	size_t gemm_scratch_halves(size_t m, size_t k);
+	size_t exact_scratch_bytes(size_t m, size_t k);
+	bool exact_gemm_takes(int fmt, const void* wq, size_t n, size_t k);
+	bool launch_exact_rows(const float* x, size_t m, size_t k, const float* norm_w, double eps, const float* up,
+	                       void* scratch, hipStream_t stream);
+	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
+	                       const float* residual, const void* scratch, hipStream_t stream);
 	bool launch_gemm(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y,
 	                 const float* residual, void* scratch_halves, float* partial, size_t partial_floats,
 	                 hipStream_t stream);
@@ -760,6 +766,10 @@ static bool is_weight_format(int fmt)
 // tile costs about as much as three single-row GEMVs (Q4_K 14336 x 4096: 14.6 us against 8.2 each).
 static constexpr size_t kMatrixCoreMinRows = 4;
 
+// From this many rows on a matmul with Float32 operands shares the weights between its rows.  Two launches and their
+// scratch from the pool take the host 21 us, a row of the streaming kernel 3.4 us and more of the GPU.
+static constexpr size_t kExactMinRows = 8;
+
 extern "C" size_t litenn_hip_mul_mat_q_workspace_bytes(size_t m, size_t k)
 {
 	return m >= kMatrixCoreMinRows ? 2 * gemm_scratch_halves(m, k) : 0;
@@ -869,6 +879,37 @@ extern "C" int litenn_hip_mul_mat_q_ws(int dev, int fmt, const void* wq, size_t 
 			return 0;
 		}
 		return finish(action, opts);
+	}
+	// Several rows with Float32 operands share the weights on the matrix cores (csrc/exact.hip) where there is room for
+	// the rows taken apart: in the caller's workspace, or, where none was given, from the device's memory pool.  A
+	// call that finds no room, or whose stream is being captured, streams the weights row by row, which needs none.
+	if (m >= kExactMinRows && exact_gemm_takes(fmt, wq, n, k))
+	{
+		const size_t need = exact_scratch_bytes(m, k);
+		StreamScratch scratch(s);
+		void* room = workspace && workspace_bytes >= need ? workspace : nullptr;
+		if (!workspace && scratch.allocate(need) == hipSuccess)
+		{
+			room = scratch.get();
+		}
+		else if (!workspace)
+		{
+			(void)hipGetLastError(); // no memory to be had is no error here
+		}
+		if (room && launch_exact_rows(xf, m, k, nullptr, 0.0, nullptr, room, s))
+		{
+			launch_exact_gemm(fmt, 1, &wq, &n, k, m, &yf, rf, room, s);
+			if (scratch.blocking())
+			{
+				const hipError_t launched = hipGetLastError();
+				const hipError_t drained = hipStreamSynchronize(s);
+				if (launched != hipSuccess || drained != hipSuccess)
+				{
+					return fail_hip(action, launched != hipSuccess ? launched : drained);
+				}
+			}
+			return finish_with(widened, action, opts);
+		}
 	}
 	launch_gemv(fmt, wq, n, k, xf, m, yf, rf, s);
 	return finish_with(widened, action, opts);

@@ -1,0 +1,1001 @@
+// Quantised matmul of several activation rows with Float32 operands on the matrix cores:
+//   Y[M, N] = X[M, K] . deq(W)[N, K]^T  (+ residual)
+// with the accuracy of the Float32 streaming kernel (csrc/gemv.hip), which would read the weights once
+// per row.  No operand is rounded to 16 bits:
+//
+//   * A GGUF weight is a small integer times a scale.  The integers (or, for the K-quants with six-bit
+//     sub-scales, integer times sub-scale: at most 63 * 31 < 2048) are exact in binary16 and are what
+//     the matrix cores multiply; the block's Float32 scale is applied to the Float32 sum of its
+//     products.
+//   * An activation is scaled by a power of two per row and taken apart into two binary16 values, hi =
+//     half(x) and lo = half(x - hi), which together carry 22 to 24 significant bits; both are
+//     multiplied by the same integers and accumulate in the same Float32 registers.
+//   * The minimum term of Q4_K and Q5_K, dmin * sum_j m_j (sum of sub-block j's activations), is one
+//     more product per 256 elements: the eight sums, taken apart the same way, against the eight
+//     six-bit minima.
+//
+// Against 64 bits the result is as close as the streaming kernel's (relative L2 1.0e-7 to 2.1e-7 over
+// K = 256 .. 14336 and every format; the streaming kernel has 1.4e-7 to 2.5e-7).
+//
+// What bounds it: few rows are the weights' stream and the launch; many rows, the LDS reads of the fragments (two
+// per pair of products) and the latency in front of them: a product issues every 100 cycles and SIMD where
+// it takes 32.  Row by row through the streaming kernel the same calls took, us, before -> now with the rows'
+// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 56; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
+//
+// v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
+// weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
+#include "common.hpp"
+
+#include <algorithm>
+
+namespace litenn_hip
+{
+	namespace
+	{
+		typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+		typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+		typedef float floatx16 __attribute__((ext_vector_type(16)));
+		typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+		typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+		constexpr int kTile = 32;     // activation rows and weight rows of one product
+		constexpr int kChunk = 256;   // K elements of the outer loop's step: four stages of four MFMA steps
+		constexpr int kFrag = 1024;   // bytes of an operand fragment: 64 lanes x 8 halves
+		constexpr int kStageBytes = 8 * kFrag;           // one tile, 64 elements: (hi, lo) x 4 steps
+		constexpr int kTileChunkBytes = 4 * kStageBytes; // one tile, 256 elements
+		constexpr float kSumScale = 1.0f / 64.0f; // sums of 32 activations back into the binary16 range
+
+		// ---- weight blocks -> binary16 integers -------------------------------------------------------
+		// A wavefront copies the raw blocks of its 32 NG rows for one 256-element chunk into a slot of its own in
+		// LDS, 16-byte pieces in a row's order (eight neighbouring lanes fetch one 128-byte line; a lane that
+		// fetched its own row's bytes instead took 29 us for Q8_0 4096 x 4096, most of it in the vector memory
+		// path).  From there lane (r, h) = (lane % 32, lane / 32) takes, of weight row r, elements 16 s + 8 h .. + 7
+		// of step s (K in natural order).  A stage is 64 elements = steps 0..3.  Blocks are only 2-byte aligned.
+		typedef const __attribute__((address_space(3))) uint8_t* lds_bytes_t;
+		__device__ __forceinline__ u32x2 load8(lds_bytes_t p)
+		{
+			typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+			return *(const __attribute__((address_space(3))) u32x2_a2*)(p);
+		}
+		__device__ __forceinline__ u32x4 load16(lds_bytes_t p)
+		{
+			typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+			return *(const __attribute__((address_space(3))) u32x4_a2*)(p);
+		}
+		__device__ __forceinline__ uint32_t load2(lds_bytes_t p) { return *(const __attribute__((address_space(3))) uint16_t*)(p); }
+
+		__device__ __forceinline__ half2v as_half2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
+
+		// bytes 0, 1 and 2, 3 of v as the halves 1024 + byte (0x6400 | byte)
+		__device__ __forceinline__ half2v biased01(uint32_t v) { return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)); }
+		__device__ __forceinline__ half2v biased23(uint32_t v) { return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)); }
+
+		__device__ __forceinline__ half8 join(half2v a, half2v b, half2v c, half2v d)
+		{
+			return half8{ a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y };
+		}
+		// eight unsigned bytes minus `bias`
+		__device__ __forceinline__ half8 bytes_minus(uint32_t a, uint32_t b, float bias)
+		{
+			const _Float16 m = static_cast<_Float16>(-1024.0f - bias);
+			const half2v off = { m, m };
+			return join(biased01(a) + off, biased23(a) + off, biased01(b) + off, biased23(b) + off);
+		}
+		// eight unsigned bytes (at most 31) times the integer `scale` (at most 63): (1024 + q) s - 1024 s, fused
+		__device__ __forceinline__ half8 bytes_times(uint32_t a, uint32_t b, uint32_t scale)
+		{
+			const half2v s = as_half2(0x64006400u | (scale * 0x00010001u)) - half2v{ 1024, 1024 };
+			const half2v off = s * half2v{ -1024, -1024 };
+			return join(__builtin_elementwise_fma(biased01(a), s, off), __builtin_elementwise_fma(biased23(a), s, off),
+			            __builtin_elementwise_fma(biased01(b), s, off), __builtin_elementwise_fma(biased23(b), s, off));
+		}
+
+		// Formats:
+		//   kBlock        elements of a block, kChunkBytes bytes of 256 elements
+		//   kScaleSteps   steps whose products share one scale: after them the sum is scaled and added
+		//   Head          what the lane needs of the chunk as a whole
+		//   kMins         whether a minimum term follows each chunk
+		// Rows whose last chunk is not whole (blocks of 32 only) load their last block again in the missing blocks'
+		// places and scale it by 0 (`blocks` whole blocks of the chunk are there).
+		struct Q4_0X
+		{
+			static constexpr int kBlock = 32, kChunkBytes = 8 * 18, kScaleSteps = 2;
+			static constexpr bool kMins = false;
+			struct Head {};
+			struct Raw { u32x2 q[2]; uint32_t d[2]; };
+			static __device__ __forceinline__ Head head(lds_bytes_t, int) { return {}; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int blocks)
+			{
+				Raw r;
+#pragma unroll
+				for (int b = 0; b < 2; ++b)
+				{
+					const int block = 2 * st + b;
+					lds_bytes_t p = chunk + 18 * block;
+					r.d[b] = block < blocks ? load2(p) : 0u;
+					r.q[b] = load8(p + 2 + 8 * h);
+				}
+				return r;
+			}
+			static __device__ __forceinline__ half8 frag(const Head&, const Raw& r, int, int t)
+			{
+				const u32x2 q = r.q[t >> 1];
+				const int sh = 4 * (t & 1);
+				return bytes_minus((q.x >> sh) & 0x0f0f0f0fu, (q.y >> sh) & 0x0f0f0f0fu, 8.0f);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw& r, int, int t) { return f16_bits_to_f32(r.d[t >> 1]); }
+			static __device__ __forceinline__ float chunk_scale(const Head&) { return 1.0f; }
+		};
+
+		struct Q8_0X
+		{
+			static constexpr int kBlock = 32, kChunkBytes = 8 * 34, kScaleSteps = 2;
+			static constexpr bool kMins = false;
+			struct Head {};
+			struct Raw { u32x2 q[4]; uint32_t d[2]; };
+			static __device__ __forceinline__ Head head(lds_bytes_t, int) { return {}; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int blocks)
+			{
+				Raw r;
+#pragma unroll
+				for (int b = 0; b < 2; ++b)
+				{
+					const int block = 2 * st + b;
+					lds_bytes_t p = chunk + 34 * block;
+					r.d[b] = block < blocks ? load2(p) : 0u;
+					r.q[2 * b] = load8(p + 2 + 8 * h);
+					r.q[2 * b + 1] = load8(p + 18 + 8 * h);
+				}
+				return r;
+			}
+			static __device__ __forceinline__ half8 frag(const Head&, const Raw& r, int, int t)
+			{
+				return bytes_minus(r.q[t].x ^ 0x80808080u, r.q[t].y ^ 0x80808080u, 128.0f);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw& r, int, int t) { return f16_bits_to_f32(r.d[t >> 1]); }
+			static __device__ __forceinline__ float chunk_scale(const Head&) { return 1.0f; }
+		};
+
+		struct Q4_KX
+		{
+			static constexpr int kBlock = 256, kChunkBytes = 144, kScaleSteps = 16;
+			static constexpr bool kMins = true;
+			struct Head { u32x4 w; }; // d, dmin, 12 bytes of six-bit scales and minima
+			struct Raw { u32x2 q[2]; };
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return { load16(chunk) }; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int)
+			{
+				lds_bytes_t p = chunk + 16 + 32 * st + 8 * h;
+				return { { load8(p), load8(p + 16) } };
+			}
+			// get_scale_min_k4 of the ggml block definition, four sub-blocks to a dword
+			static __device__ __forceinline__ uint32_t scales(const u32x4& w, int four)
+			{
+				return four == 0 ? w.y & 0x3f3f3f3fu : (w.w & 0x0f0f0f0fu) | ((w.y >> 2) & 0x30303030u);
+			}
+			static __device__ __forceinline__ uint32_t minima(const u32x4& w, int four)
+			{
+				return four == 0 ? w.z & 0x3f3f3f3fu : ((w.w >> 4) & 0x0f0f0f0fu) | ((w.z >> 2) & 0x30303030u);
+			}
+			// steps 0, 1: low nibbles (sub-block 2 st); steps 2, 3: high nibbles (2 st + 1)
+			static __device__ __forceinline__ half8 frag(const Head& hd, const Raw& r, int st, int t)
+			{
+				const int sh = 4 * (t >> 1), sub = 2 * st + (t >> 1);
+				const uint32_t s = (scales(hd.w, sub >> 2) >> (8 * (sub & 3))) & 0xffu;
+				const u32x2 q = r.q[t & 1];
+				return bytes_times((q.x >> sh) & 0x0f0f0f0fu, (q.y >> sh) & 0x0f0f0f0fu, s);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
+			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.w.x); }
+			static __device__ __forceinline__ half8 min_frag(const Head& hd) { return bytes_minus(minima(hd.w, 0), minima(hd.w, 1), 0.0f); }
+			static __device__ __forceinline__ float min_scale(const Head& hd) { return -f16_bits_to_f32(hd.w.x >> 16); }
+		};
+
+		struct Q5_KX
+		{
+			static constexpr int kBlock = 256, kChunkBytes = 176, kScaleSteps = 16;
+			static constexpr bool kMins = true;
+			struct Head { u32x4 w; u32x2 fifth[2]; };
+			struct Raw { u32x2 q[2]; };
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int h)
+			{
+				return { load16(chunk), { load8(chunk + 16 + 8 * h), load8(chunk + 32 + 8 * h) } };
+			}
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int)
+			{
+				lds_bytes_t p = chunk + 48 + 32 * st + 8 * h;
+				return { { load8(p), load8(p + 16) } };
+			}
+			static __device__ __forceinline__ half8 frag(const Head& hd, const Raw& r, int st, int t)
+			{
+				const int sh = 4 * (t >> 1), sub = 2 * st + (t >> 1);
+				const uint32_t s = (Q4_KX::scales(hd.w, sub >> 2) >> (8 * (sub & 3))) & 0xffu;
+				const u32x2 q = r.q[t & 1], f = hd.fifth[t & 1]; // bit `sub` of a byte is its element's fifth bit
+				return bytes_times(((q.x >> sh) & 0x0f0f0f0fu) | (((f.x >> sub) & 0x01010101u) << 4),
+				                   ((q.y >> sh) & 0x0f0f0f0fu) | (((f.y >> sub) & 0x01010101u) << 4), s);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
+			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.w.x); }
+			static __device__ __forceinline__ half8 min_frag(const Head& hd)
+			{
+				return bytes_minus(Q4_KX::minima(hd.w, 0), Q4_KX::minima(hd.w, 1), 0.0f);
+			}
+			static __device__ __forceinline__ float min_scale(const Head& hd) { return -f16_bits_to_f32(hd.w.x >> 16); }
+		};
+
+		struct Q6_KX
+		{
+			// six bits and a signed byte of sub-scale per 16 elements: their product does not fit a half, so every
+			// step is scaled on its own
+			static constexpr int kBlock = 256, kChunkBytes = 210, kScaleSteps = 1;
+			static constexpr bool kMins = false;
+			struct Head { u32x4 sc; uint32_t d; };
+			struct Raw { u32x2 low[4], high[2]; }; // half st / 2 of the block: [32 x (first, second)] x 16-element runs
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return { load16(chunk + 192), load2(chunk + 208) }; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int)
+			{
+				lds_bytes_t ql = chunk + 64 * (st >> 1) + 8 * h;
+				lds_bytes_t qh = chunk + 128 + 32 * (st >> 1) + 8 * h;
+				return { { load8(ql), load8(ql + 16), load8(ql + 32), load8(ql + 48) }, { load8(qh), load8(qh + 16) } };
+			}
+			// quarter i = 2 (st % 2) + t / 2 of the half, elements 16 (t % 2) + 8 h .. of its 32
+			static __device__ __forceinline__ half8 frag(const Head&, const Raw& r, int st, int t)
+			{
+				const int sh = 4 * (st & 1), top = 2 * (2 * (st & 1) + (t >> 1));
+				const u32x2 q = r.low[2 * (t >> 1) + (t & 1)], f = r.high[t & 1];
+				return bytes_minus(((q.x >> sh) & 0x0f0f0f0fu) | (((f.x >> top) & 0x03030303u) << 4),
+				                   ((q.y >> sh) & 0x0f0f0f0fu) | (((f.y >> top) & 0x03030303u) << 4), 32.0f);
+			}
+			static __device__ __forceinline__ float scale(const Head& hd, const Raw&, int st, int t)
+			{
+				const int sub = 4 * st + t;
+				const uint32_t w = sub < 4 ? hd.sc.x : sub < 8 ? hd.sc.y : sub < 12 ? hd.sc.z : hd.sc.w;
+				return static_cast<float>(static_cast<int8_t>(w >> (8 * (sub & 3))));
+			}
+			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.d); }
+		};
+
+		// 16-byte pieces of a row's chunk: from the 16-byte boundary at or below it.  Rows are whole blocks apart from
+		// an address of any alignment, so a chunk may begin up to 14 bytes behind its first piece.  The slot's
+		// rows are a multiple of 16 bytes but not of 32 apart: 32 lanes then read over 64 banks two to a bank.
+		template <typename F>
+		constexpr int slot_pieces() { return (F::kChunkBytes + 14 + 15) / 16; }
+		template <typename F>
+		constexpr int slot_stride() { return 16 * (slot_pieces<F>() | 1); }
+
+		// ---- activations -> fragments -----------------------------------------------------------------
+		// [tile of 32 rows][chunk][step][hi, lo] fragments, then [tile][chunk] fragments of sub-block sums
+		// (halves 0..7 of lane (r, 0): hi parts, of lane (r, 1): lo parts), then a factor per row.
+		struct RowsLayout
+		{
+			size_t sums, factors, bytes;
+			__host__ __device__ RowsLayout(size_t tiles, size_t chunks)
+			{
+				sums = tiles * chunks * kTileChunkBytes;
+				factors = sums + tiles * chunks * kFrag;
+				bytes = factors + tiles * kTile * sizeof(float);
+			}
+		};
+
+		constexpr int kHeldItems = 8; // 8-element items of a row per thread: rows up to 16384 wide
+
+		// One workgroup per row.  The producers of csrc/gemm.hip's pre-pass may run first: RMSNorm with f64
+		// accumulation (norm_w) or SwiGLU's silu(x) * up.
+		__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
+		                                                         int m, int m_pad, int k, int chunks,
+		                                                         const float* __restrict__ norm_w, double eps,
+		                                                         const float* __restrict__ up)
+		{
+			__shared__ float red[4];
+			__shared__ double red64[4];
+			// eight rows share every 128-byte line of the layout: XCD x (workgroups are dealt out round-robin)
+			// takes the row octets x, x + 8, ... so that its L2 puts whole lines together
+			const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
+			const int row = (((nth >> 3) << 3) + xcd) * 8 + (nth & 7);
+			if (row >= m_pad)
+			{
+				return;
+			}
+			const RowsLayout at(m_pad / kTile, chunks);
+			const int tile = row / kTile, r = row % kTile;
+			uint8_t* frags = out + static_cast<size_t>(tile) * chunks * kTileChunkBytes + r * 16;
+			uint8_t* sums = out + at.sums + static_cast<size_t>(tile) * chunks * kFrag + r * 16;
+			float* factors = reinterpret_cast<float*>(out + at.factors);
+			const int items = chunks * (kChunk / 8);
+			float held[kHeldItems][8];
+			double ss = 0.0;
+			float mx = 0.0f;
+#pragma unroll
+			for (int u = 0; u < kHeldItems; ++u)
+			{
+				const int it = threadIdx.x + 256 * u;
+#pragma unroll
+				for (int e = 0; e < 8; ++e)
+				{
+					held[u][e] = 0.0f;
+				}
+				if (row < m && 8 * it < k)
+				{
+					const size_t o = static_cast<size_t>(row) * k + 8 * it;
+					const float4 a = *reinterpret_cast<const float4*>(x + o);
+					const float4 b = *reinterpret_cast<const float4*>(x + o + 4);
+					held[u][0] = a.x, held[u][1] = a.y, held[u][2] = a.z, held[u][3] = a.w;
+					held[u][4] = b.x, held[u][5] = b.y, held[u][6] = b.z, held[u][7] = b.w;
+					if (up)
+					{
+						const float4 ua = *reinterpret_cast<const float4*>(up + o);
+						const float4 ub = *reinterpret_cast<const float4*>(up + o + 4);
+						const float uu[8] = { ua.x, ua.y, ua.z, ua.w, ub.x, ub.y, ub.z, ub.w };
+#pragma unroll
+						for (int e = 0; e < 8; ++e)
+						{
+							const float gv = held[u][e];
+							const float sig = __fdiv_rn(1.0f, __fadd_rn(1.0f, expf(-gv)));
+							held[u][e] = __fmul_rn(__fmul_rn(gv, sig), uu[e]);
+						}
+					}
+#pragma unroll
+					for (int e = 0; e < 8; ++e)
+					{
+						const double v = static_cast<double>(held[u][e]);
+						ss += v * v;
+					}
+				}
+			}
+			if (norm_w)
+			{
+				for (int off = 32; off > 0; off >>= 1)
+				{
+					ss += __shfl_xor(ss, off, 64);
+				}
+				if ((threadIdx.x & 63) == 0)
+				{
+					red64[threadIdx.x >> 6] = ss;
+				}
+				__syncthreads();
+				const double total = red64[0] + red64[1] + red64[2] + red64[3];
+				const double inv = 1.0 / sqrt(total / static_cast<double>(k) + eps);
+#pragma unroll
+				for (int u = 0; u < kHeldItems; ++u)
+				{
+					const int it = threadIdx.x + 256 * u;
+					if (row < m && 8 * it < k)
+					{
+						const float4 wa = *reinterpret_cast<const float4*>(norm_w + 8 * it);
+						const float4 wb = *reinterpret_cast<const float4*>(norm_w + 8 * it + 4);
+						const float ww[8] = { wa.x, wa.y, wa.z, wa.w, wb.x, wb.y, wb.z, wb.w };
+#pragma unroll
+						for (int e = 0; e < 8; ++e)
+						{
+							held[u][e] = static_cast<float>(static_cast<double>(held[u][e]) * inv * static_cast<double>(ww[e]));
+						}
+					}
+				}
+			}
+			// the largest finite magnitude (infinities and NaN keep their values below)
+#pragma unroll
+			for (int u = 0; u < kHeldItems; ++u)
+			{
+#pragma unroll
+				for (int e = 0; e < 8; ++e)
+				{
+					const float a = fabsf(held[u][e]);
+					mx = a <= 3.402823466e38f ? fmaxf(mx, a) : mx;
+				}
+			}
+			mx = wave_max(mx);
+			if ((threadIdx.x & 63) == 0)
+			{
+				red[threadIdx.x >> 6] = mx;
+			}
+			__syncthreads();
+			mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+			// x 2^shift has its largest magnitude in [2^14, 2^15); the inverse stays a normal number
+			const int shift = mx > 0.0f ? min(14 - ilogbf(mx), 126) : 0;
+#pragma unroll
+			for (int u = 0; u < kHeldItems; ++u)
+			{
+				const int it = threadIdx.x + 256 * u;
+				double sum = 0.0;
+				if (it < items)
+				{
+					half8 hi, lo;
+#pragma unroll
+					for (int e = 0; e < 8; ++e)
+					{
+						const float v = ldexpf(held[u][e], shift);
+						hi[e] = static_cast<_Float16>(v);
+						const float rest = v - static_cast<float>(hi[e]);
+						lo[e] = static_cast<_Float16>(fabsf(v) <= 65504.0f ? rest : 0.0f); // (inf - inf)
+						sum += static_cast<double>(v);
+					}
+					uint8_t* dst = frags + static_cast<size_t>(it >> 1) * (2 * kFrag) + (it & 1) * 512;
+					*reinterpret_cast<half8*>(dst) = hi;
+					*reinterpret_cast<half8*>(dst + kFrag) = lo;
+				}
+				// four neighbouring threads hold one sub-block of 32 elements
+				sum += __shfl_xor(sum, 1, 64);
+				sum += __shfl_xor(sum, 2, 64);
+				if (it < items && (threadIdx.x & 3) == 0)
+				{
+					const float v = static_cast<float>(sum * kSumScale);
+					const _Float16 hi = static_cast<_Float16>(v);
+					const double rest = sum * kSumScale - static_cast<double>(static_cast<float>(hi));
+					const _Float16 lo = static_cast<_Float16>(fabsf(v) <= 65504.0f ? static_cast<float>(rest) : 0.0f);
+					uint8_t* dst = sums + static_cast<size_t>(it >> 5) * kFrag + ((it >> 2) & 7) * 2;
+					*reinterpret_cast<_Float16*>(dst) = hi;
+					*reinterpret_cast<_Float16*>(dst + 512) = lo;
+				}
+			}
+			if (threadIdx.x == 0)
+			{
+				factors[row] = row < m ? ldexpf(1.0f, -shift) : 0.0f;
+			}
+		}
+
+		// ---- the product ------------------------------------------------------------------------------
+		struct ExactMats
+		{
+			const uint8_t* w[3];
+			float* y[3];
+			int n[3];
+			int first_block[3]; // grid x index of each matrix's first workgroup (INT_MAX when unused)
+		};
+
+		// Workgroups that share a strip of weight rows follow each other on one XCD (as in csrc/gemm.hip)
+		__device__ __forceinline__ void exact_grid_position(int& grid_x, int& grid_y)
+		{
+			grid_x = blockIdx.x, grid_y = blockIdx.y;
+			if (gridDim.y > 1)
+			{
+				const int gx = gridDim.x, gy = gridDim.y, full = gx & ~7, l = grid_x + gx * grid_y;
+				if (l < full * gy)
+				{
+					grid_x = (l / (8 * gy)) * 8 + (l & 7);
+					grid_y = (l >> 3) % gy;
+				}
+				else
+				{
+					grid_x = full + (l - full * gy) % (gx - full);
+					grid_y = (l - full * gy) / (gx - full);
+				}
+			}
+		}
+
+		// A wavefront multiplies NG groups of 32 weight rows by MT tiles of 32 activation rows over one of KS
+		// ranges of K; the KS sums meet in LDS at the end, added in K order.  Two levels of sums, a chunk's and
+		// the range's, keep the rounding of long rows down.  WN wavefronts side by side share the activation
+		// fragments of a range through LDS (two buffers of one 64-element stage, the next two stages travelling
+		// through registers while the current one is multiplied); with WN = 1 nobody shares them and they go to
+		// registers directly, each refilled for the next stage once it has been used.  The raw blocks of the
+		// next chunk travel through registers into the wavefront's slot meanwhile.
+		template <typename F, int NG, int MT, int WN, int KS>
+		__global__ __launch_bounds__(64 * WN * KS) void exact_gemm_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
+		                                                                  const float* residual, int k, int m, int m_tiles,
+		                                                                  int chunks, size_t row_bytes)
+		{
+			constexpr bool kShared = WN > 1;
+			constexpr int kPieces = kShared ? MT * 8 / WN : 1; // 1 KB pieces a wavefront stages
+			static_assert(!kShared || kPieces * WN == MT * 8, "activation pieces / wavefront split");
+			constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>();
+			constexpr int kRowPieces = NG * kTile * P;
+			constexpr int kWLoads = (kRowPieces + 63) / 64;
+			constexpr int kRingBytes = kShared ? KS * 2 * MT * kStageBytes : 0;
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
+			int grid_x, grid_y;
+			exact_grid_position(grid_x, grid_y);
+			const int which = (grid_x >= mats.first_block[1]) + (grid_x >= mats.first_block[2]);
+			const uint8_t* w = which == 0 ? mats.w[0] : (which == 1 ? mats.w[1] : mats.w[2]);
+			float* y = which == 0 ? mats.y[0] : (which == 1 ? mats.y[1] : mats.y[2]);
+			const int n = which == 0 ? mats.n[0] : (which == 1 ? mats.n[1] : mats.n[2]);
+			const int block_x = grid_x - (which == 0 ? 0 : (which == 1 ? mats.first_block[1] : mats.first_block[2]));
+			const int lane = threadIdx.x & 63;
+			const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int part = wave / WN, wv = wave % WN;
+			const int r = lane & 31, h = lane >> 5;
+			const int n_base = (block_x * WN + wv) * (NG * kTile);
+			const int mt_base = grid_y * MT;
+			const int per = (chunks + KS - 1) / KS;
+			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
+
+			// ---- weights: piece i of this lane is piece (64 i + lane) % P of row (64 i + lane) / P; the last pieces of a
+			// partial chunk, and of an aligned one, lie behind the row: they fetch the row's last piece again
+			uint8_t* const slot = lds + kRingBytes + wave * (NG * kTile * kStride);
+			const uint8_t* piece_row[kWLoads]; // the 16-byte boundary at or below the row's start
+			int piece_at[kWLoads], piece_last[kWLoads], piece_slot[kWLoads];
+#pragma unroll
+			for (int i = 0; i < kWLoads; ++i)
+			{
+				const int id = min(64 * i + lane, kRowPieces - 1), row = id / P;
+				const uintptr_t start = reinterpret_cast<uintptr_t>(w) + static_cast<size_t>(min(n_base + row, n - 1)) * row_bytes;
+				const int mis = static_cast<int>(start & 15);
+				piece_row[i] = reinterpret_cast<const uint8_t*>(start - mis);
+				piece_at[i] = mis; // byte offset of the chunk's start from the row's first piece, plus piece offset below
+				piece_last[i] = static_cast<int>((mis + row_bytes - 1) & ~size_t{ 15 });
+				piece_slot[i] = row * kStride + 16 * (id - row * P);
+			}
+			u32x4 moving[kWLoads];
+			const auto request_w = [&](int c) {
+#pragma unroll
+				for (int i = 0; i < kWLoads; ++i)
+				{
+					const int id = min(64 * i + lane, kRowPieces - 1);
+					const int at = min(((piece_at[i] + c * F::kChunkBytes) & ~15) + 16 * (id % P), piece_last[i]);
+					moving[i] = *reinterpret_cast<const u32x4*>(piece_row[i] + at);
+				}
+			};
+			const auto deposit_w = [&]() {
+#pragma unroll
+				for (int i = 0; i < kWLoads; ++i)
+				{
+					if (64 * (i + 1) <= kRowPieces || 64 * i + lane < kRowPieces)
+					{
+						*reinterpret_cast<u32x4*>(slot + piece_slot[i]) = moving[i];
+					}
+				}
+			};
+			int row_mis[NG];
+#pragma unroll
+			for (int q = 0; q < NG; ++q)
+			{
+				const size_t start = reinterpret_cast<uintptr_t>(w) + static_cast<size_t>(min(n_base + kTile * q + r, n - 1)) * row_bytes;
+				row_mis[q] = static_cast<int>(start & 15);
+			}
+			const auto lane_chunk = [&](int q, int c) {
+				return (lds_bytes_t)(slot) + (kTile * q + r) * kStride + ((row_mis[q] + c * F::kChunkBytes) & 15);
+			};
+
+			const RowsLayout at(m_tiles, chunks);
+			const uint8_t* tiles[MT]; // this lane's 16 bytes of the tile's first fragment
+			const uint8_t* sum_tiles[MT];
+#pragma unroll
+			for (int t = 0; t < MT; ++t)
+			{
+				const size_t tile = min(mt_base + t, m_tiles - 1);
+				tiles[t] = xs + tile * chunks * kTileChunkBytes + lane * 16;
+				sum_tiles[t] = xs + at.sums + tile * chunks * kFrag + lane * 16;
+			}
+
+			floatx16 acc[NG][MT], p[NG][MT];
+#pragma unroll
+			for (int q = 0; q < NG; ++q)
+			{
+#pragma unroll
+				for (int t = 0; t < MT; ++t)
+				{
+					acc[q][t] = floatx16{};
+				}
+			}
+
+			// ---- activations
+			half8 direct[kShared ? 1 : MT][4][2]; // WN = 1
+			u32x4 staged[2][kPieces];             // WN > 1: the next two stages on their way
+			uint8_t* const ring = lds + part * (2 * MT * kStageBytes);
+			const auto request = [&](u32x4 (&into)[kPieces], int c, int st) {
+#pragma unroll
+				for (int i = 0; i < kPieces; ++i)
+				{
+					const int piece = i * WN + wv, t = piece >> 3;
+					const size_t tile = min(mt_base + t, m_tiles - 1);
+					into[i] = *reinterpret_cast<const u32x4*>(xs + (tile * chunks + c) * kTileChunkBytes + st * kStageBytes +
+					                                            (piece & 7) * kFrag + lane * 16);
+				}
+			};
+			const auto deposit = [&](const u32x4 (&from)[kPieces], int buffer) {
+#pragma unroll
+				for (int i = 0; i < kPieces; ++i)
+				{
+					*reinterpret_cast<u32x4*>(ring + buffer * (MT * kStageBytes) + (i * WN + wv) * kFrag + lane * 16) = from[i];
+				}
+			};
+			const auto fetch_direct = [&](int c, int st, int s) {
+#pragma unroll
+				for (int t = 0; t < MT; ++t)
+				{
+#pragma unroll
+					for (int e = 0; e < 2; ++e)
+					{
+						direct[t][s][e] = *reinterpret_cast<const half8*>(tiles[t] + static_cast<size_t>(c) * kTileChunkBytes +
+						                                                  st * kStageBytes + (2 * s + e) * kFrag);
+					}
+				}
+			};
+
+			half8 sum_frag[MT];
+			if (c_begin < c_end)
+			{
+				request_w(c_begin);
+				if constexpr (kShared)
+				{
+					request(staged[0], c_begin, 0);
+					request(staged[1], c_begin, 1);
+				}
+				else
+				{
+#pragma unroll
+					for (int s = 0; s < 4; ++s)
+					{
+						fetch_direct(c_begin, 0, s);
+					}
+				}
+				deposit_w();
+				if constexpr (kShared)
+				{
+					deposit(staged[0], 0);
+				}
+			}
+			if constexpr (kShared)
+			{
+				__syncthreads();
+			}
+			int buffer = 0;
+			for (int i = 0; i < per; ++i)
+			{
+				const int c = c_begin + i;
+				const bool live = c < c_end; // (uniform: a shorter range only passes the barriers)
+				const int next = min(c + 1, c_end - 1);
+				typename F::Head head[NG];
+				floatx16 sum[F::kScaleSteps < 16 ? NG : 1][MT]; // the chunk's
+				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
+				if (live)
+				{
+					request_w(next);
+#pragma unroll
+					for (int q = 0; q < NG; ++q)
+					{
+						head[q] = F::head(lane_chunk(q, c), h);
+					}
+					if constexpr (F::kMins)
+					{
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+							sum_frag[t] = *reinterpret_cast<const half8*>(sum_tiles[t] + static_cast<size_t>(c) * kFrag);
+						}
+					}
+				}
+#pragma unroll
+				for (int st = 0; st < 4; ++st)
+				{
+					if (live)
+					{
+						typename F::Raw raw[NG];
+#pragma unroll
+						for (int q = 0; q < NG; ++q)
+						{
+							raw[q] = F::load(lane_chunk(q, c), st, h, blocks);
+						}
+						if constexpr (kShared)
+						{
+							request(staged[st & 1], st < 2 ? c : next, (st + 2) & 3);
+						}
+#pragma unroll
+						for (int s = 0; s < 4; ++s)
+						{
+							half8 b[NG];
+#pragma unroll
+							for (int q = 0; q < NG; ++q)
+							{
+								b[q] = F::frag(head[q], raw[q], st, s);
+							}
+							const int step = 4 * st + s;
+							const bool fresh = step % F::kScaleSteps == 0;
+#pragma unroll
+							for (int t = 0; t < MT; ++t)
+							{
+								half8 a[2];
+#pragma unroll
+								for (int e = 0; e < 2; ++e)
+								{
+									if constexpr (kShared)
+									{
+										a[e] = *reinterpret_cast<const half8*>(ring + buffer * (MT * kStageBytes) + t * kStageBytes +
+										                                       (2 * s + e) * kFrag + lane * 16);
+									}
+									else
+									{
+										a[e] = direct[t][s][e];
+									}
+								}
+#pragma unroll
+								for (int q = 0; q < NG; ++q)
+								{
+									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b[q], fresh ? floatx16{} : p[q][t], 0, 0, 0);
+									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b[q], p[q][t], 0, 0, 0);
+								}
+							}
+							if constexpr (!kShared)
+							{
+								fetch_direct(st < 3 ? c : next, (st + 1) & 3, s);
+							}
+							if constexpr (F::kScaleSteps < 16)
+							{
+								if (step % F::kScaleSteps == F::kScaleSteps - 1)
+								{
+#pragma unroll
+									for (int q = 0; q < NG; ++q)
+									{
+										const float d = F::scale(head[q], raw[q], st, s);
+#pragma unroll
+										for (int t = 0; t < MT; ++t)
+										{
+#pragma unroll
+											for (int e = 0; e < 16; ++e)
+											{
+												sum[q][t][e] = step == F::kScaleSteps - 1 ? d * p[q][t][e] : fmaf(d, p[q][t][e], sum[q][t][e]);
+											}
+										}
+									}
+								}
+							}
+						}
+						if constexpr (kShared)
+						{
+							deposit(staged[(st + 1) & 1], buffer ^ 1);
+						}
+					}
+					if constexpr (kShared)
+					{
+						__syncthreads();
+					}
+					buffer ^= 1;
+				}
+				if (live)
+				{
+#pragma unroll
+					for (int q = 0; q < NG; ++q)
+					{
+						const float d = F::chunk_scale(head[q]);
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+#pragma unroll
+							for (int e = 0; e < 16; ++e)
+							{
+								acc[q][t][e] = fmaf(d, F::kScaleSteps < 16 ? sum[q % (F::kScaleSteps < 16 ? NG : 1)][t][e] : p[q][t][e], acc[q][t][e]);
+							}
+						}
+						if constexpr (F::kMins)
+						{
+							const half8 b = F::min_frag(head[q]);
+							const float dm = F::min_scale(head[q]) * (1.0f / kSumScale);
+#pragma unroll
+							for (int t = 0; t < MT; ++t)
+							{
+								const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, floatx16{}, 0, 0, 0);
+#pragma unroll
+								for (int e = 0; e < 16; ++e)
+								{
+									acc[q][t][e] = fmaf(dm, s[e], acc[q][t][e]);
+								}
+							}
+						}
+					}
+					deposit_w(); // (the wavefront's own reads of the slot are behind it in its instruction stream)
+				}
+			}
+
+			if constexpr (KS > 1)
+			{
+				// ranges 1 .. KS - 1 hand their sums to range 0
+				__syncthreads();
+				floatx16* const handed = reinterpret_cast<floatx16*>(lds);
+				if (part > 0)
+				{
+#pragma unroll
+					for (int q = 0; q < NG; ++q)
+					{
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+#pragma unroll
+							for (int e = 0; e < 16; e += 4)
+							{
+								float4* dst = reinterpret_cast<float4*>(handed + (((part - 1) * WN + wv) * NG * MT + q * MT + t) * 64) + (e / 4) * 64 + lane;
+								*dst = float4{ acc[q][t][e], acc[q][t][e + 1], acc[q][t][e + 2], acc[q][t][e + 3] };
+							}
+						}
+					}
+				}
+				__syncthreads();
+				if (part > 0)
+				{
+					return;
+				}
+#pragma unroll
+				for (int other = 1; other < KS; ++other)
+				{
+#pragma unroll
+					for (int q = 0; q < NG; ++q)
+					{
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+#pragma unroll
+							for (int e = 0; e < 16; e += 4)
+							{
+								const float4 v = *(reinterpret_cast<const float4*>(handed + (((other - 1) * WN + wv) * NG * MT + q * MT + t) * 64) + (e / 4) * 64 + lane);
+								acc[q][t][e] += v.x;
+								acc[q][t][e + 1] += v.y;
+								acc[q][t][e + 2] += v.z;
+								acc[q][t][e + 3] += v.w;
+							}
+						}
+					}
+				}
+			}
+
+			// lane (r, h) holds weight row r and activation rows 8 (e / 4) + 4 h + e % 4
+			const float* factors = reinterpret_cast<const float*>(xs + at.factors);
+#pragma unroll
+			for (int t = 0; t < MT; ++t)
+			{
+#pragma unroll
+				for (int e = 0; e < 16; ++e)
+				{
+					const int mm = (mt_base + t) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
+					if (mm < m)
+					{
+						const float us = factors[mm];
+#pragma unroll
+						for (int q = 0; q < NG; ++q)
+						{
+							const int col = n_base + kTile * q + r;
+							if (col < n)
+							{
+								const size_t o = static_cast<size_t>(mm) * n + col;
+								float v = acc[q][t][e] * us;
+								if (residual)
+								{
+									v = residual[o] + v;
+								}
+								y[o] = v;
+							}
+						}
+					}
+				}
+			}
+		}
+
+		struct ExactCall
+		{
+			int count;
+			const uint8_t* w[3];
+			float* y[3];
+			int n[3];
+			int total_rows; // of all matrices
+			const uint8_t* xs;
+			const float* residual;
+			int k, m, m_tiles, chunks;
+			size_t row_bytes;
+			hipStream_t stream;
+		};
+
+		template <typename F, int NG, int MT, int WN, int KS>
+		void launch_variant(const ExactCall& c)
+		{
+			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * 2 * MT * kStageBytes : 0) +
+			                         static_cast<size_t>(WN) * KS * NG * kTile * slot_stride<F>();
+			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * NG * MT * 64 * 64;
+			constexpr size_t lds = rings > sums ? rings : sums;
+			static_assert(lds <= 160 * 1024, "LDS");
+			ExactMats mats{};
+			int blocks = 0;
+			for (int i = 0; i < 3; ++i)
+			{
+				mats.first_block[i] = 0x7fffffff;
+				if (i < c.count)
+				{
+					mats.w[i] = c.w[i];
+					mats.y[i] = c.y[i];
+					mats.n[i] = c.n[i];
+					mats.first_block[i] = blocks;
+					blocks += (c.n[i] + WN * NG * kTile - 1) / (WN * NG * kTile);
+				}
+			}
+			const auto kernel = &exact_gemm_kernel<F, NG, MT, WN, KS>;
+			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+			exact_gemm_kernel<F, NG, MT, WN, KS><<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
+			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
+		}
+
+		template <typename F>
+		void launch_exact_format(const ExactCall& c)
+		{
+			const int strips = (c.total_rows + kTile - 1) / kTile, units = strips * c.m_tiles;
+			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each
+			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 234 against 301 of the
+			// forms below, at 64 rows 53 against 62.  Not for Q6_K, whose scaling per step wants the registers.
+			if (F::kScaleSteps > 1 && (strips + 3) / 4 * ((c.m_tiles + 1) / 2) >= 200 && c.m_tiles > 1)
+			{
+				launch_variant<F, 1, 2, 4, 2>(c);
+			}
+			// Otherwise a wavefront keeps to itself and the ranges of K fill the card.  Q6_K saves a second decode with two
+			// tiles once there are enough of them (4096 x 14336 at 300 rows 168 against 207; at 45 rows 52 against 44).
+			else if (F::kScaleSteps == 1 && units >= 512 && c.m_tiles > 1)
+			{
+				launch_variant<F, 1, 2, 1, 8>(c);
+			}
+			// Eight ranges while there are few tiles (Q8_0 4096 x 4096 at 3 rows 14.7 against 16.6 with four, Q6_K
+			// 4096 x 14336 at 45 rows 44 against 54), four from there on (Q4_K 14336 x 4096 at 8 rows 18.1 against
+			// 20.7 with eight) and for short rows (Q8_0 1024 x 1024 7.2 against 8.1).
+			else if (units <= 256 && c.chunks >= 8)
+			{
+				launch_variant<F, 1, 1, 1, 8>(c);
+			}
+			else
+			{
+				launch_variant<F, 1, 1, 1, 4>(c);
+			}
+		}
+	} // namespace
+
+	// bytes of scratch the rows of an m x k activation matrix take
+	size_t exact_scratch_bytes(size_t m, size_t k)
+	{
+		const size_t tiles = (m + kTile - 1) / kTile, chunks = (k + kChunk - 1) / kChunk;
+		return RowsLayout(tiles, chunks).bytes;
+	}
+
+	// Whether launch_exact_gemm takes a matrix: one of the formats above, rows that start on 2 bytes.
+	bool exact_gemm_takes(int fmt, const void* wq, size_t n, size_t k)
+	{
+		switch (fmt)
+		{
+		case LITENN_FMT_Q4_0: case LITENN_FMT_Q8_0: case LITENN_FMT_Q4_K: case LITENN_FMT_Q5_K: case LITENN_FMT_Q6_K: break;
+		default: return false;
+		}
+		return n > 0 && n <= 0x3fffffffu && row_bytes(fmt, k) != 0 && reinterpret_cast<uintptr_t>(wq) % 2 == 0;
+	}
+
+	// Takes the rows of X' = x, RMSNorm(x) * norm_w or silu(x) * up apart into `scratch` (exact_scratch_bytes,
+	// 16-byte aligned) for any number of launch_exact_gemm calls of the same m and k.  Returns false, launching
+	// nothing, for rows it does not take.
+	bool launch_exact_rows(const float* x, size_t m, size_t k, const float* norm_w, double eps, const float* up, void* scratch,
+	                       hipStream_t stream)
+	{
+		const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+		if (!scratch || m == 0 || m > (size_t{ 1 } << 20) || k == 0 || k % 32 != 0 || k > static_cast<size_t>(kHeldItems) * 256 * 8 ||
+		    !aligned(x) || !aligned(scratch) || !aligned(norm_w) || !aligned(up) || (norm_w && up))
+		{
+			return false;
+		}
+		const int chunks = static_cast<int>((k + kChunk - 1) / kChunk);
+		const int m_pad = static_cast<int>((m + kTile - 1) / kTile * kTile);
+		split_rows_kernel<<<dim3(static_cast<unsigned>((m_pad + 63) / 64 * 64)), dim3(256), 0, stream>>>(
+		    x, static_cast<uint8_t*>(scratch), static_cast<int>(m), m_pad, static_cast<int>(k), chunks, norm_w, eps, up);
+		return true;
+	}
+
+	// y_i[M, n_i] = X' . deq(W_i)^T (+ residual, which may alias y; single matrix) for up to three matrices of
+	// one format over rows that launch_exact_rows has taken apart.
+	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
+	                       const float* residual, const void* scratch, hipStream_t stream)
+	{
+		ExactCall c{};
+		c.count = count;
+		for (int i = 0; i < count; ++i)
+		{
+			c.w[i] = static_cast<const uint8_t*>(wq[i]);
+			c.y[i] = y[i];
+			c.n[i] = static_cast<int>(n[i]);
+			c.total_rows += c.n[i];
+		}
+		c.xs = static_cast<const uint8_t*>(scratch);
+		c.residual = residual;
+		c.k = static_cast<int>(k);
+		c.m = static_cast<int>(m);
+		c.m_tiles = static_cast<int>((m + kTile - 1) / kTile);
+		c.chunks = static_cast<int>((k + kChunk - 1) / kChunk);
+		c.row_bytes = row_bytes(fmt, k);
+		c.stream = stream;
+		switch (fmt)
+		{
+		case LITENN_FMT_Q4_0: launch_exact_format<Q4_0X>(c); break;
+		case LITENN_FMT_Q8_0: launch_exact_format<Q8_0X>(c); break;
+		case LITENN_FMT_Q4_K: launch_exact_format<Q4_KX>(c); break;
+		case LITENN_FMT_Q5_K: launch_exact_format<Q5_KX>(c); break;
+		default: launch_exact_format<Q6_KX>(c); break;
+		}
+	}
+} // namespace litenn_hip

@@ -22,6 +22,12 @@ namespace litenn_hip
 	int launch_gemv(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y,
 	                const float* residual, hipStream_t stream);
 	size_t gemm_scratch_halves(size_t m, size_t k);
+	size_t exact_scratch_bytes(size_t m, size_t k);
+	bool exact_gemm_takes(int fmt, const void* wq, size_t n, size_t k);
+	bool launch_exact_rows(const float* x, size_t m, size_t k, const float* norm_w, double eps, const float* up,
+	                       void* scratch, hipStream_t stream);
+	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
+	                       const float* residual, const void* scratch, hipStream_t stream);
 	bool launch_gemm_group(int fmt, int count, const void* const* wq, const size_t* n, size_t k, const float* x,
 	                       size_t m, float* const* y, const float* residual, const float* norm_w, double eps,
 	                       const float* up, void* scratch_halves, float* partial, size_t partial_floats,
@@ -176,6 +182,8 @@ namespace
 			}
 			// (q/k/v projections in two formats share a launch that wants the rows in both fragment orders)
 			m->xh_halves = std::max(gemm_scratch_halves(rows, std::max({ d, qw, ff })), 2 * gemm_scratch_halves(rows, d));
+			// or, with Float32 operands, the rows taken apart into two halves each
+			m->xh_halves = std::max(m->xh_halves, (exact_scratch_bytes(rows, std::max({ d, qw, ff })) + 1) / 2);
 			LITENN_HIP_TRY(kAction, hipMalloc(&m->xh, 2 * m->xh_halves));
 			m->cap_rows = rows;
 		}
@@ -199,27 +207,70 @@ namespace
 		return 0;
 	}
 
-	// From this many rows on (and unless f32 operands are asked for) a matmul goes to the matrix cores:
-	// one padded 16-row tile costs about as much as three single-row GEMVs.
+	// From this many rows on a matmul goes to the matrix cores: one padded tile costs about as much as three
+	// single-row GEMVs (with Float32 operands: 12.5 us + bytes / 2.2 TB/s against 3.3 us + bytes / 5.1 TB/s per row).
 	constexpr size_t kGemmMinRows = 4;
 	// From this many rows on the prompt's attention runs tiled on the matrix cores.
 	constexpr size_t kAttnTileMinRows = 16;
+
+	bool is_quantised(const Weight& w) { return w.fmt != LITENN_FMT_F16 && w.fmt != LITENN_FMT_F32; }
+
+	// Several rows with Float32 operands through the matrix cores (csrc/exact.hip): the rows of x, RMSNorm(x) * norm_w
+	// or silu(x) * up are taken apart once for all `count` matrices of one width; consecutive matrices of
+	// one format share a launch.  False, with nothing launched, where a matrix or the rows are not its.
+	bool exact_group(litenn_hip_llama* m, int count, const Weight* const* ws, float* const* ys, const float* x, size_t rows,
+	                 const float* residual, const float* norm_w, const float* up, hipStream_t s)
+	{
+		for (int i = 0; i < count; ++i)
+		{
+			if (ws[i]->k != ws[0]->k || !exact_gemm_takes(ws[i]->fmt, ws[i]->data, ws[i]->n, ws[i]->k))
+			{
+				return false;
+			}
+		}
+		const size_t k = ws[0]->k;
+		if (rows < kGemmMinRows || exact_scratch_bytes(rows, k) > 2 * m->xh_halves ||
+		    !launch_exact_rows(x, rows, k, norm_w, m->p.rms_norm_epsilon, up, m->xh, s))
+		{
+			return false;
+		}
+		for (int i = 0; i < count;)
+		{
+			const void* w[3];
+			size_t n[3];
+			int j = i;
+			for (; j < count && ws[j]->fmt == ws[i]->fmt; ++j)
+			{
+				w[j - i] = ws[j]->data;
+				n[j - i] = ws[j]->n;
+			}
+			launch_exact_gemm(ws[i]->fmt, j - i, w, n, k, rows, ys + i, residual, m->xh, s);
+			i = j;
+		}
+		return true;
+	}
 
 	// partial: null, or m->xn while it is idle (the GEMM may leave the products of K's later ranges there)
 	void matmul(litenn_hip_llama* m, const Weight& w, const float* x, size_t rows, float* y, const float* residual,
 	            float* partial, unsigned flags, hipStream_t s)
 	{
-		const bool quant = w.fmt != LITENN_FMT_F16 && w.fmt != LITENN_FMT_F32;
-		if (rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE) && quant && w.k % 256 == 0 &&
-		    launch_gemm(w.fmt, w.data, w.n, w.k, x, rows, y, residual, m->xh, partial, partial ? m->xn_floats : 0, s))
+		if (rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE))
 		{
-			return;
+			if (is_quantised(w) && w.k % 256 == 0 &&
+			    launch_gemm(w.fmt, w.data, w.n, w.k, x, rows, y, residual, m->xh, partial, partial ? m->xn_floats : 0, s))
+			{
+				return;
+			}
 		}
-		launch_gemv(w.fmt, w.data, w.n, w.k, x, rows, y, residual, s);
+		const Weight* ws[1] = { &w };
+		if (!exact_group(m, 1, ws, &y, x, rows, residual, nullptr, nullptr, s))
+		{
+			launch_gemv(w.fmt, w.data, w.n, w.k, x, rows, y, residual, s);
+		}
 	}
 
 	// Multi-row form of an operator group: y_i = X' . W_i^T (+ residual) with X' = x, RMSNorm(x) * norm_w
-	// or silu(x) * up.  On the matrix cores the producer runs inside the fp16 pre-pass and matrices of
+	// or silu(x) * up.  On the matrix cores the producer runs inside the pre-pass and matrices of
 	// one format share a launch; otherwise it is composed from the stand-alone kernels (`tmp` takes
 	// the producer's result).
 	void matmul_group(litenn_hip_llama* m, int count, const Weight* const* ws, float* const* ys, const float* x,
@@ -232,8 +283,8 @@ namespace
 		{
 			same = same && ws[i]->fmt == w0.fmt && ws[i]->k == w0.k;
 		}
-		const bool quant = w0.fmt != LITENN_FMT_F16 && w0.fmt != LITENN_FMT_F32;
-		if (same && rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE) && quant && w0.k % 256 == 0)
+		const bool rounded = rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE);
+		if (same && rounded && is_quantised(w0) && w0.k % 256 == 0)
 		{
 			const void* w[3] = { nullptr, nullptr, nullptr };
 			size_t n[3] = { 0, 0, 0 };
@@ -247,6 +298,10 @@ namespace
 			{
 				return;
 			}
+		}
+		if (!rounded && exact_group(m, count, ws, ys, x, rows, residual, norm_w, up, s))
+		{
+			return;
 		}
 		const float* in = x;
 		if (norm_w)
@@ -477,10 +532,11 @@ namespace
 			                        L.wq.k == L.wk.k && L.wk.k == L.wv.k &&
 			                        launch_gemm_group_mixed(qkv_fmt, 3, qkv_w, qkv_n, L.wq.k, m->x, rows, qkv_out, L.attn_norm,
 			                                                m->p.rms_norm_epsilon, m->xh, m->xh_halves, s);
+			const bool exact = rows >= kGemmMinRows && (flags & LITENN_HIP_MATMUL_PRECISE); // (formats do not matter to its rows)
 			for (int i = 0; i < 3 && !one_launch;)
 			{
 				int j = i + 1;
-				while (j < 3 && qkv[j]->fmt == qkv[i]->fmt && qkv[j]->k == qkv[i]->k)
+				while (j < 3 && (exact || qkv[j]->fmt == qkv[i]->fmt) && qkv[j]->k == qkv[i]->k)
 				{
 					++j;
 				}

@@ -1,0 +1,79 @@
+"""The quantised matmul of several rows with Float32 operands (integer weights times split activations on the
+matrix cores) against the numpy decoder and a product in 64 bits.  Sizes lie at the edges of its tiles (32 rows of
+either side, 256 elements of K) and on both sides of every rule that picks a form.
+
+Bound: a weight is exact, an activation keeps 22 bits and more (relative error 2^-23 at most), and Float32 sums of
+k random products of like size err by about sqrt(log2 k) 2^-24 of |x| |W| / sqrt(k), the size such a sum has (a single
+output may happen to cancel to less, which no summation order can follow); 1e-6 is four times what is seen."""
+import numpy as np
+import pytest
+
+import np_decoders
+from litenn_amd import synth
+from litenn_amd.formats import Q4_0, Q4_K, Q5_K, Q6_K, Q8_0
+from litenn_amd.llama import MATMUL_PRECISE
+
+pytestmark = pytest.mark.gpu
+FORMATS = [Q4_0, Q8_0, Q4_K, Q5_K, Q6_K]
+
+
+def errors(hip, fmt, m, n, k, residual=False):
+    wq = synth.model_weights(fmt, n, k, 21, m, n)
+    x = synth.activations(m, k, 22, m)
+    x[m // 2] *= np.float32(1e-20)  # every row keeps its own scale
+    res = synth.activations(m, n, 23, 1) if residual else None
+    got = hip.mul_mat_q(fmt, hip.Tensor.from_numpy(wq), n, k, hip.Tensor.from_numpy(x),
+                        residual=hip.Tensor.from_numpy(res) if residual else None, flags=MATMUL_PRECISE).numpy()
+    w = np_decoders.decode(fmt, wq, k).astype(np.float64)
+    want = x.astype(np.float64) @ w.T
+    size = np.linalg.norm(x.astype(np.float64), axis=1) * np.linalg.norm(w) / np.sqrt(k)
+    if residual:
+        want += res
+        size = np.hypot(size, np.linalg.norm(res, axis=1))
+    return np.linalg.norm(got - want, axis=1) / size
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(8, 33, 256), (9, 1, 2048), (31, 65, 512), (32, 64, 4096), (33, 500, 2304), (65, 129, 768),
+                                   (300, 5200, 256), (70, 7000, 256), (130, 3300, 512), (12, 9000, 256), (3, 60, 512)])
+def test_rows_of_every_form(hip, fmt, m, n, k):
+    assert errors(hip, fmt, m, n, k, residual=m % 2 == 0).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt", [Q4_0, Q8_0])
+@pytest.mark.parametrize("m,n,k", [(8, 17, 32), (40, 70, 288), (9, 40, 1056), (200, 3300, 96)])
+def test_rows_that_end_inside_a_chunk(hip, fmt, m, n, k):
+    assert errors(hip, fmt, m, n, k).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_non_finite_and_tiny_activations(hip, fmt):
+    m, n, k = 9, 70, 512
+    wq = synth.model_weights(fmt, n, k, 5, 1)
+    x = synth.activations(m, k, 6, 1)
+    w, t = hip.Tensor.from_numpy(wq), hip.Tensor.from_numpy
+    clean = hip.mul_mat_q(fmt, w, n, k, t(x), flags=MATMUL_PRECISE).numpy()
+    x[0, 3], x[1, 9], x[2], x[3] = np.inf, np.nan, 0.0, x[3] * np.float32(1e-42)
+    got = hip.mul_mat_q(fmt, w, n, k, t(x), flags=MATMUL_PRECISE).numpy()
+    assert not np.any(np.isfinite(got[0])) and np.all(np.isnan(got[1])) and np.all(got[2] == 0.0)
+    assert np.all(np.abs(got[3]) <= 1e-38)
+    assert np.array_equal(got[4:], clean[4:])
+
+
+def test_a_workspace_that_holds_the_rows_is_used_and_a_smaller_one_is_enough(hip):
+    """The same bits out of the pool's memory and a caller's; with less room the rows go through the streaming kernel."""
+    import ctypes as C
+    from litenn_amd import _lib
+    fmt, m, n, k = Q4_K, 40, 200, 512
+    wq = synth.model_weights(fmt, n, k, 5, 2)
+    x = synth.activations(m, k, 6, 2)
+    w, xt = hip.Tensor.from_numpy(wq), hip.Tensor.from_numpy(x)
+    want = hip.mul_mat_q(fmt, w, n, k, xt, flags=MATMUL_PRECISE).numpy()
+    for size, same in ((64 * 512 * 5, True), (1024, False)):
+        room = hip.Tensor.from_numpy(np.zeros(size, np.uint8))
+        y = hip.Tensor.from_numpy(np.full((m, n), np.nan, np.float32))
+        _lib.check(_lib.load().litenn_hip_mul_mat_q_ws(0, fmt, w.ptr, n, k, xt.ptr, 0, m, y.ptr, None, MATMUL_PRECISE, room.ptr,
+                                                       C.c_size_t(size), None))
+        got = y.numpy()
+        assert np.array_equal(got, want) == same
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
