@@ -4,6 +4,7 @@
 // weight stream; they are written to keep f32 (f64 for the norm) semantics of the
 // reference chains and to read every operand once.
 #include "common.hpp"
+#include "attn_rows.hpp"
 #include "attn_math.hpp"
 
 #include <algorithm>
@@ -1086,6 +1087,11 @@ namespace litenn_hip
 	                        const int* past_dev, size_t past_host, size_t n_head, size_t n_kv_head, size_t head_dim,
 	                        float* out, size_t splits, float* partial, int* counters, hipStream_t s)
 	{
+		// several rows share the keys on the matrix cores
+		if (!past_dev && launch_attn_rows_causal(q, kcache, vcache, cache_dtype, m, past_host, n_head, n_kv_head, head_dim, out, s))
+		{
+			return;
+		}
 		launch_attn_any(q, const_cast<void*>(kcache), const_cast<void*>(vcache), cache_dtype, m, past_dev, past_host,
 		                n_head, n_kv_head, head_dim, out, splits, partial, counters, nullptr, s);
 	}
@@ -1191,8 +1197,37 @@ namespace litenn_hip
 	                     double logit_softcap, const float* mask, const float* sinks, bool causal, size_t key_offset,
 	                     size_t query_offset, float* out, hipStream_t s)
 	{
-		AttnExt x;
 		const double score_scale = logit_softcap != 0.0 ? scale / logit_softcap : scale;
+		if (attn_rows_pays(m, keys, cache_dtype == LITENN_F32))
+		{
+			RowsAttn a;
+			a.q = q;
+			a.ldq = a.ldo = n_head * head_dim;
+			a.k = kcache;
+			a.v = vcache;
+			a.ldk = a.ldv = n_kv_head * head_dim;
+			a.k_head = a.v_head = head_dim;
+			a.heads = static_cast<int>(n_head);
+			a.share = static_cast<int>(n_head / n_kv_head);
+			a.dim = a.vdim = static_cast<int>(head_dim);
+			a.rows = static_cast<int>(m);
+			a.keys = static_cast<int>(keys);
+			a.causal = causal;
+			a.q_at = static_cast<long long>(query_offset) - static_cast<long long>(key_offset);
+			a.scale = static_cast<float>(score_scale);
+			a.apply_scale = (scale != 1.0 || logit_softcap != 0.0) && score_scale != 1.0;
+			a.softcap = static_cast<float>(logit_softcap);
+			a.apply_cap = logit_softcap != 1.0;
+			a.mask = mask;
+			a.max_bias = max_bias;
+			a.sinks = sinks;
+			a.out = out;
+			if (launch_attn_rows(a, cache_dtype == LITENN_F32, s))
+			{
+				return;
+			}
+		}
+		AttnExt x;
 		x.mask = mask;
 		x.sinks = sinks;
 		x.score_scale = static_cast<float>(score_scale);

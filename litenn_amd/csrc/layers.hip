@@ -4,6 +4,7 @@
 // (recurrent step, and a chunked form whose contractions run on the Float32 matrix instructions).
 // Norms, positions, scores, softmax and everything inside a recurrence are Float32.  The reference
 // has no counterpart of these layers.
+#include "attn_rows.hpp"
 #include "layer_device.hpp"
 
 #include <algorithm>
@@ -1613,6 +1614,39 @@ namespace litenn_hip
 		const dim3 rows(a.rows, a.shape.heads);
 		if (a.f32)
 		{
+			if (attn_rows_pays(a.rows, std::min(a.keys, a.shape.window), true))
+			{
+				RowsAttn r;
+				r.q = a.q;
+				r.ldq = a.ldq;
+				r.k = a.kv;
+				r.v = static_cast<const float*>(a.kv) + a.v_first;
+				r.ldk = r.ldv = a.ldkv;
+				r.k_head = a.k_head;
+				r.v_head = a.v_head;
+				r.ring = a.kv_ring;
+				r.ring_first = a.kv_first;
+				r.heads = a.shape.heads;
+				r.share = a.shape.share;
+				r.dim = a.shape.dim;
+				r.vdim = a.shape.vdim;
+				r.rows = a.rows;
+				r.keys = a.keys;
+				r.q_at = static_cast<long long>(a.q_base) - a.key_base;
+				r.window = a.shape.window;
+				r.apply_scale = true;
+				r.scale = a.shape.scale;
+				r.sinks = a.shape.sink;
+				r.gate = a.gate;
+				r.ldg = a.ldg;
+				r.out_scale = a.out_scale;
+				r.out = static_cast<float*>(a.out);
+				r.ldo = a.ldo;
+				if (launch_attn_rows(r, true, s))
+				{
+					return;
+				}
+			}
 			window_attn_row_kernel<float><<<rows, dim3(64), 0, s>>>(a);
 			return;
 		}

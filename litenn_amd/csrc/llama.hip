@@ -505,7 +505,7 @@ namespace
 
 	// Enqueues the decoder over `rows` tokens whose ids are at `ids` (device); positions start at
 	// counters[0].  Logits are produced for the last `logit_rows` rows into m->logits.
-	void forward_rows(litenn_hip_llama* m, const int32_t* ids, size_t rows, size_t logit_rows, unsigned flags)
+	void forward_rows(litenn_hip_llama* m, const int32_t* ids, size_t rows, size_t logit_rows, unsigned flags, size_t past)
 	{
 		static const bool fuse_token = !(getenv("LITENN_HIP_FUSE") && getenv("LITENN_HIP_FUSE")[0] == '0');
 		if (rows == 1 && logit_rows == 1 && fuse_token)
@@ -517,6 +517,9 @@ namespace
 		const size_t d = m->p.embedding_length;
 		const size_t H = m->p.head_count, KH = m->p.head_count_kv, hd = m->head_dim;
 		const int* past_dev = m->d_counters;
+		// a captured step (one row) reads its position on the device; a prompt's rows are launched for theirs
+		const int* attn_past_dev = rows == 1 ? past_dev : nullptr;
+		const size_t attn_past = rows == 1 ? 0 : past;
 		launch_get_rows_q(m->tok_embd.fmt, m->tok_embd.data, m->tok_embd.n, d, ids, rows, m->x, m->d_err, s);
 		for (Layer& L : m->layers)
 		{
@@ -548,9 +551,9 @@ namespace
 			                       m->p.rope_dimension_count, m->cos_t, m->sin_t, s);
 			// a prompt's rows go through the matrix cores (fp16 operands) unless f32 operands are asked for
 			if (rows < kAttnTileMinRows || (flags & LITENN_HIP_MATMUL_PRECISE) ||
-			    !launch_attn_tile(m->q, L.kcache, L.vcache, m->p.kv_dtype, rows, past_dev, 0, H, KH, hd, m->attn, s))
+			    !launch_attn_tile(m->q, L.kcache, L.vcache, m->p.kv_dtype, rows, attn_past_dev, attn_past, H, KH, hd, m->attn, s))
 			{
-				launch_attn_decode(m->q, L.kcache, L.vcache, m->p.kv_dtype, rows, past_dev, 0, H, KH, hd, m->attn,
+				launch_attn_decode(m->q, L.kcache, L.vcache, m->p.kv_dtype, rows, attn_past_dev, attn_past, H, KH, hd, m->attn,
 				                   rows == 1 ? m->attn_splits : 1, m->attn_partial, m->attn_counters, s);
 			}
 			matmul(m, L.wo, m->attn, rows, m->x, m->x, m->xn, flags, s); // x = x + attn . Wo (xn is idle here)
@@ -595,9 +598,9 @@ int litenn_hip_llama::ensure_rows(size_t rows) { return ensure_scratch(this, row
 
 void litenn_hip_llama::prepare() { (void)block_fused_ready(this); }
 
-void litenn_hip_llama::forward(const int32_t* ids, size_t rows, size_t logit_rows, unsigned flags, int)
+void litenn_hip_llama::forward(const int32_t* ids, size_t rows, size_t logit_rows, unsigned flags, int past)
 {
-	forward_rows(this, ids, rows, logit_rows, flags);
+	forward_rows(this, ids, rows, logit_rows, flags, static_cast<size_t>(past));
 }
 
 bool litenn_hip_llama::give_up_waiting()
