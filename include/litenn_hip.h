@@ -291,8 +291,8 @@ int litenn_hip_argmax(int dev, const void* x, size_t rows, size_t n, void* out_i
 /* y[m, n] (f32) = x . W^T over BFloat16 weights whose rows are `pitch` elements apart, pitch being k
  * rounded up to a multiple of 64 and the elements behind the k-th zero.  x is [m, pitch] Float32 or
  * BFloat16 (what lies behind the k-th element of a row is not used).  One Float32 row streams the
- * weights once; other Float32 calls use the Float32 matrix instructions, BFloat16 ones the bfloat16
- * ones.  Accumulation is Float32 throughout. */
+ * weights once; other Float32 calls take every activation apart into three bfloat16 values, exactly, and use
+ * the bfloat16 matrix instructions as BFloat16 calls do.  Accumulation is Float32 throughout. */
 int litenn_hip_linear_bf16(int dev, const void* w, size_t n, size_t k, size_t pitch, const void* x, int x_dtype, size_t m,
                            void* y, const litenn_hip_exec* opts);
 

@@ -8,6 +8,7 @@
 #include "dense.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace litenn_hip
 {
@@ -339,8 +340,8 @@ namespace litenn_hip
 		}
 
 		// ------------------------------------------------------------------
-		// Many rows, bfloat16 operands: BM activation rows x BN weight rows per workgroup of four
-		// wavefronts, K in tiles of 64 double-buffered in LDS (global -> registers two tiles ahead -> LDS
+		// Many rows: BM activation rows x BN weight rows per group of four wavefronts, bfloat16 operands (Float32 ones:
+		// below), K in tiles of 64 double-buffered in LDS (global -> registers two tiles ahead -> LDS
 		// while the previous tile is multiplied), v_mfma_f32_16x16x32_bf16 with the weights as the A operand, so that a lane
 		// ends up with four consecutive outputs of one activation row.  The 16-byte pieces of a 128-byte
 		// LDS row are permuted by the row's low three bits: the 16 rows a fragment read touches then fall
@@ -445,38 +446,64 @@ namespace litenn_hip
 			}
 		}
 
-		// WM x WN wavefronts share the tile
-		template <int BM, int BN, int WM, int WN>
-		__global__ __launch_bounds__(256) void dense_tile_kernel(const TileArgs args)
+		// A Float32 as three values whose upper halves are bfloat16 and whose sum it is: eight significant bits, the next
+		// eight, the rest.  An infinity or a NaN is the first one, the others zero.
+		__device__ __forceinline__ void cut_in_three(uint32_t bits, uint32_t (&part)[3])
+		{
+			const bool special = (bits & 0x7f800000u) == 0x7f800000u;
+			const uint32_t quiet = (bits & 0x007fffffu) != 0u ? 0x00400000u : 0u;
+			part[0] = (bits | (special ? quiet : 0u)) & 0xffff0000u;
+			const float rest = special ? 0.0f : __uint_as_float(bits) - __uint_as_float(part[0]);
+			part[1] = __float_as_uint(rest) & 0xffff0000u;
+			part[2] = __float_as_uint(rest - __uint_as_float(part[1]));
+		}
+
+		// WM x WN wavefronts share the tile.
+		//
+		// F32: Float32 operands.  The weights are bfloat16 as they are; an activation is the sum of three bfloat16 values
+		// of eight bits each, cut off its front one after the other, which is exact, so that three products per operand
+		// pair give what one of Float32 operands gives, at 48 cycles per 32 elements of K where v_mfma_f32_16x16x4_f32
+		// takes 256.  The activations are taken apart on their way into LDS.
+		//
+		// KG groups of four wavefronts share the tile and cut its K walk into as many ranges, each through buffers of its
+		// own; their sums meet in LDS at the end, in K order.  A step of one group alone is a chain of latencies
+		// (request, LDS, barrier, products that feed each other): with few tiles the ranges fill the SIMDs.
+		template <int BM, int BN, int WM, int WN, int KG, bool F32>
+		__global__ __launch_bounds__(256 * KG) void dense_tile_kernel(const TileArgs args)
 		{
 			static_assert(WM * WN == 4, "four wavefronts");
+			constexpr int P = F32 ? 3 : 1; // parts of an activation
+			typedef std::conditional_t<F32, float, uint16_t> operand;
 			constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
 			constexpr int LA = BM / 32, LW = BN / 32; // 16-byte pieces a thread stages per K tile
-			__shared__ __attribute__((aligned(16))) uint16_t xs[2][BM * kTileK];
-			__shared__ __attribute__((aligned(16))) uint16_t ws[2][BN * kTileK];
+			extern __shared__ __attribute__((aligned(16))) uint16_t tile_lds[]; // per group: activations [2][P][BM][64], weights [2][BN][64]
+			const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+			uint16_t* const xs = tile_lds + group * (2 * kTileK * (P * BM + BN));
+			uint16_t* const ws = xs + 2 * P * BM * kTileK;
 			const DenseRows& d = args.d;
 			int tm, tn;
 			if (!tile_of(args, tm, tn))
 			{
 				return;
 			}
-			const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+			const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
 			const int j = lane & 15, g = lane >> 4;
 			const int wm = wave / WN, wn = wave % WN;
 			const int m0 = tm * BM, n0 = tn * BN;
 			const int k = d.w.k;
-			// this workgroup's share of K
-			const int all_steps = d.w.pitch / kTileK, part = static_cast<int>(blockIdx.y);
-			const int first_step = all_steps * part / d.splits;
-			const int steps = all_steps * (part + 1) / d.splits - first_step;
+			// this group's share of K, and the steps every group makes
+			const int all_steps = d.w.pitch / kTileK, parts = d.splits * KG, part = static_cast<int>(blockIdx.y) * KG + group;
+			const int first_step = all_steps * part / parts;
+			const int steps = all_steps * (part + 1) / parts - first_step;
+			const int rounds = (all_steps + parts - 1) / parts;
 
 			const int ch = tid & 7, row = tid >> 3; // this thread's piece column and first row
-			const uint16_t* xp[LA];
+			const operand* xp[LA];
 			const uint16_t* wp[LW];
 #pragma unroll
 			for (int i = 0; i < LA; ++i)
 			{
-				xp[i] = static_cast<const uint16_t*>(d.a) + static_cast<size_t>(operand_row(d, m0 + row + 32 * i)) * d.lda + ch * 8;
+				xp[i] = static_cast<const operand*>(d.a) + static_cast<size_t>(operand_row(d, m0 + row + 32 * i)) * d.lda + ch * 8;
 			}
 #pragma unroll
 			for (int i = 0; i < LW; ++i)
@@ -484,12 +511,17 @@ namespace litenn_hip
 				wp[i] = d.w.w + static_cast<size_t>(min(n0 + row + 32 * i, d.w.n - 1)) * d.w.pitch + ch * 8;
 			}
 			// two K tiles travel at any time: tile t in register set t & 1 until it is staged
-			u32x4 rx[2][LA], rw[2][LW];
+			constexpr int kWords = F32 ? 2 : 1; // of a piece of eight activations
+			u32x4 rx[2][LA][kWords], rw[2][LW];
 			const auto request = [&](int step, int set) {
 #pragma unroll
 				for (int i = 0; i < LA; ++i)
 				{
-					rx[set][i] = *reinterpret_cast<const u32x4*>(xp[i] + step * kTileK);
+#pragma unroll
+					for (int w = 0; w < kWords; ++w)
+					{
+						rx[set][i][w] = *reinterpret_cast<const u32x4*>(xp[i] + step * kTileK + 4 * w);
+					}
 				}
 #pragma unroll
 				for (int i = 0; i < LW; ++i)
@@ -506,10 +538,11 @@ namespace litenn_hip
 					for (int i = 0; i < LA; ++i)
 					{
 #pragma unroll
-						for (int e = 0; e < 4; ++e)
+						for (int e = 0; e < 4 * kWords; ++e)
 						{
-							const uint32_t keep = left >= 2 * e + 2 ? 0xffffffffu : left == 2 * e + 1 ? 0xffffu : 0u;
-							rx[set][i][e] &= keep;
+							const uint32_t keep = F32 ? (e < left ? 0xffffffffu : 0u)
+							                          : left >= 2 * e + 2 ? 0xffffffffu : left == 2 * e + 1 ? 0xffffu : 0u;
+							rx[set][i][e / 4][e % 4] &= keep;
 						}
 					}
 				}
@@ -517,12 +550,37 @@ namespace litenn_hip
 #pragma unroll
 				for (int i = 0; i < LA; ++i)
 				{
-					*reinterpret_cast<u32x4*>(&xs[set][(row + 32 * i) * kTileK + slot]) = rx[set][i];
+					uint16_t* const dst = xs + set * (P * BM * kTileK) + (row + 32 * i) * kTileK + slot;
+					if constexpr (F32)
+					{
+						u32x4 part[3];
+#pragma unroll
+						for (int e = 0; e < 4; ++e)
+						{
+							uint32_t lo[3], hi[3];
+							cut_in_three(rx[set][i][e / 2][2 * (e % 2)], lo);
+							cut_in_three(rx[set][i][e / 2][2 * (e % 2) + 1], hi);
+#pragma unroll
+							for (int p = 0; p < 3; ++p)
+							{
+								part[p][e] = __builtin_amdgcn_perm(hi[p], lo[p], 0x07060302u); // the upper halves
+							}
+						}
+#pragma unroll
+						for (int p = 0; p < 3; ++p)
+						{
+							*reinterpret_cast<u32x4*>(dst + p * (BM * kTileK)) = part[p];
+						}
+					}
+					else
+					{
+						*reinterpret_cast<u32x4*>(dst) = rx[set][i][0];
+					}
 				}
 #pragma unroll
 				for (int i = 0; i < LW; ++i)
 				{
-					*reinterpret_cast<u32x4*>(&ws[set][(row + 32 * i) * kTileK + slot]) = rw[set][i];
+					*reinterpret_cast<u32x4*>(ws + set * (BN * kTileK) + (row + 32 * i) * kTileK + slot) = rw[set][i];
 				}
 			};
 
@@ -540,58 +598,105 @@ namespace litenn_hip
 #pragma unroll
 				for (int ks = 0; ks < 2; ++ks)
 				{
-					bf16x8 wf[TN], xf[TM];
+					bf16x8 wf[TN], xf[P][TM];
 #pragma unroll
 					for (int a = 0; a < TN; ++a)
 					{
 						const int r = wn * (BN / WN) + 16 * a + j;
-						wf[a] = *reinterpret_cast<const bf16x8*>(&ws[buf][r * kTileK + (((4 * ks + g) ^ (r & 7)) * 8)]);
+						wf[a] = *reinterpret_cast<const bf16x8*>(ws + buf * (BN * kTileK) + r * kTileK + (((4 * ks + g) ^ (r & 7)) * 8));
 					}
 #pragma unroll
 					for (int b = 0; b < TM; ++b)
 					{
 						const int r = wm * (BM / WM) + 16 * b + j;
-						xf[b] = *reinterpret_cast<const bf16x8*>(&xs[buf][r * kTileK + (((4 * ks + g) ^ (r & 7)) * 8)]);
+#pragma unroll
+						for (int p = 0; p < P; ++p)
+						{
+							xf[p][b] = *reinterpret_cast<const bf16x8*>(xs + (buf * P + p) * (BM * kTileK) + r * kTileK + (((4 * ks + g) ^ (r & 7)) * 8));
+						}
 					}
 #pragma unroll
-					for (int a = 0; a < TN; ++a)
+					for (int p = P - 1; p >= 0; --p) // small parts first
 					{
 #pragma unroll
-						for (int b = 0; b < TM; ++b)
+						for (int a = 0; a < TN; ++a)
 						{
-							acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a], xf[b], acc[a][b], 0, 0, 0);
+#pragma unroll
+							for (int b = 0; b < TM; ++b)
+							{
+								acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a], xf[p][b], acc[a][b], 0, 0, 0);
+							}
 						}
 					}
 				}
 			};
 			// past the last tile it is requested and staged again: a branch around the loads would make every
 			// wait behind it a wait for all of them
-			request(first_step, 0);
-			request(first_step + min(1, steps - 1), 1);
-			stage(first_step, 0);
+			// (a group without a step walks on its neighbour's first one and multiplies nothing)
+			const auto at = [&](int step) { return min(first_step + max(0, min(step, steps - 1)), all_steps - 1); };
+			request(at(0), 0);
+			request(at(1), 1);
+			stage(at(0), 0);
 			__syncthreads();
 			// tile `step` is in LDS buffer `set`, tile step + 1 in the other register set
 			const auto advance = [&](int step, int set) {
-				request(first_step + min(step + 2, steps - 1), set);
-				if constexpr (BM * BN < 128 * 128)
+				request(at(step + 2), set);
+				if constexpr (BM * BN < 128 * 128 && !F32)
 				{
 					// on their way before the products, not behind them (the largest tile, whose products take
 					// longer than the loads, runs better scheduled freely)
 					__builtin_amdgcn_sched_barrier(0);
 				}
-				multiply(set);
-				stage(first_step + min(step + 1, steps - 1), set ^ 1);
+				if (KG == 1 || step < steps)
+				{
+					multiply(set);
+				}
+				stage(at(step + 1), set ^ 1);
 				__syncthreads();
 			};
 			int step = 0;
-			for (; step + 1 < steps; step += 2)
+			for (; step + 1 < rounds; step += 2)
 			{
 				advance(step, 0);
 				advance(step + 1, 1);
 			}
-			if (step < steps)
+			if (step < rounds)
 			{
 				advance(step, 0);
+			}
+			if constexpr (KG > 1)
+			{
+				floatx4* const handed = reinterpret_cast<floatx4*>(tile_lds);
+				if (group > 0)
+				{
+#pragma unroll
+					for (int a = 0; a < TN; ++a)
+					{
+#pragma unroll
+						for (int b = 0; b < TM; ++b)
+						{
+							handed[((group - 1) * 4 + wave) * (TN * TM * 64) + (a * TM + b) * 64 + lane] = acc[a][b];
+						}
+					}
+				}
+				__syncthreads();
+				if (group > 0)
+				{
+					return;
+				}
+#pragma unroll
+				for (int other = 0; other < KG - 1; ++other)
+				{
+#pragma unroll
+					for (int a = 0; a < TN; ++a)
+					{
+#pragma unroll
+						for (int b = 0; b < TM; ++b)
+						{
+							acc[a][b] += handed[(other * 4 + wave) * (TN * TM * 64) + (a * TM + b) * 64 + lane];
+						}
+					}
+				}
 			}
 #pragma unroll
 			for (int b = 0; b < TM; ++b)
@@ -600,124 +705,7 @@ namespace litenn_hip
 #pragma unroll
 				for (int a = 0; a < TN; ++a)
 				{
-					store_outputs<uint16_t>(d, m, n0 + wn * (BN / WN) + 16 * a + 4 * g, acc[a][b]);
-				}
-			}
-		}
-
-		// ------------------------------------------------------------------
-		// Many rows, Float32 operands: 64 x 64 per workgroup, K in tiles of 32, v_mfma_f32_16x16x4_f32.  The
-		// contraction index is dealt out so that a lane's four consecutive elements of a row (one 16-byte
-		// LDS read) serve four instructions: step r of a 16-wide block takes element 4 g + r from lane
-		// group g, for both operands.
-		// ------------------------------------------------------------------
-		constexpr int kF32Tile = 64, kF32K = 32, kF32Stride = 36;
-
-		__global__ __launch_bounds__(256) void dense_tile_f32_kernel(const TileArgs args)
-		{
-			__shared__ __attribute__((aligned(16))) float xs[kF32Tile * kF32Stride];
-			__shared__ __attribute__((aligned(16))) float ws[kF32Tile * kF32Stride];
-			const DenseRows& d = args.d;
-			int tm, tn;
-			if (!tile_of(args, tm, tn))
-			{
-				return;
-			}
-			const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-			const int j = lane & 15, g = lane >> 4;
-			const int wm = wave >> 1, wn = wave & 1;
-			const int m0 = tm * kF32Tile, n0 = tn * kF32Tile;
-			const int k = d.w.k;
-			const int steps = d.w.pitch / kF32K;
-			const int xrow = tid >> 3, xc = (tid & 7) * 4;  // two rows (xrow, xrow + 32), four floats
-			const int wrow = tid >> 2, wc = (tid & 3) * 8;  // one row, eight weights
-			const float* xp[2];
-#pragma unroll
-			for (int i = 0; i < 2; ++i)
-			{
-				xp[i] = static_cast<const float*>(d.a) + static_cast<size_t>(operand_row(d, m0 + xrow + 32 * i)) * d.lda + xc;
-			}
-			const uint16_t* wp = d.w.w + static_cast<size_t>(min(n0 + wrow, d.w.n - 1)) * d.w.pitch + wc;
-			floatx4 rx[2];
-			u32x4 rw;
-			const auto request = [&](int step) {
-#pragma unroll
-				for (int i = 0; i < 2; ++i)
-				{
-					rx[i] = *reinterpret_cast<const floatx4*>(xp[i] + step * kF32K);
-				}
-				rw = *reinterpret_cast<const u32x4*>(wp + step * kF32K);
-			};
-			floatx4 acc[2][2];
-#pragma unroll
-			for (int a = 0; a < 2; ++a)
-			{
-#pragma unroll
-				for (int b = 0; b < 2; ++b)
-				{
-					acc[a][b] = floatx4{ 0.0f, 0.0f, 0.0f, 0.0f };
-				}
-			}
-			request(0);
-			for (int step = 0; step < steps; ++step)
-			{
-				const int left = k - step * kF32K - xc;
-#pragma unroll
-				for (int i = 0; i < 2; ++i)
-				{
-					floatx4 v = rx[i];
-#pragma unroll
-					for (int e = 0; e < 4; ++e)
-					{
-						v[e] = e < left ? v[e] : 0.0f;
-					}
-					*reinterpret_cast<floatx4*>(&xs[(xrow + 32 * i) * kF32Stride + xc]) = v;
-				}
-#pragma unroll
-				for (int e = 0; e < 2; ++e)
-				{
-					*reinterpret_cast<floatx4*>(&ws[wrow * kF32Stride + wc + 4 * e]) =
-					    floatx4{ __uint_as_float(rw[2 * e] << 16), __uint_as_float(rw[2 * e] & 0xffff0000u),
-						         __uint_as_float(rw[2 * e + 1] << 16), __uint_as_float(rw[2 * e + 1] & 0xffff0000u) };
-				}
-				__syncthreads();
-				if (step + 1 < steps)
-				{
-					request(step + 1);
-				}
-#pragma unroll
-				for (int kb = 0; kb < kF32K; kb += 16)
-				{
-					floatx4 wf[2], xf[2];
-#pragma unroll
-					for (int t = 0; t < 2; ++t)
-					{
-						wf[t] = *reinterpret_cast<const floatx4*>(&ws[(wn * 32 + 16 * t + j) * kF32Stride + kb + 4 * g]);
-						xf[t] = *reinterpret_cast<const floatx4*>(&xs[(wm * 32 + 16 * t + j) * kF32Stride + kb + 4 * g]);
-					}
-#pragma unroll
-					for (int r = 0; r < 4; ++r)
-					{
-#pragma unroll
-						for (int a = 0; a < 2; ++a)
-						{
-#pragma unroll
-							for (int b = 0; b < 2; ++b)
-							{
-								acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[a][r], xf[b][r], acc[a][b], 0, 0, 0);
-							}
-						}
-					}
-				}
-				__syncthreads();
-			}
-#pragma unroll
-			for (int b = 0; b < 2; ++b)
-			{
-#pragma unroll
-				for (int a = 0; a < 2; ++a)
-				{
-					store_outputs<float>(d, m0 + wm * 32 + 16 * b + j, n0 + wn * 32 + 16 * a + 4 * g, acc[a][b]);
+					store_outputs<operand>(d, m, n0 + wn * (BN / WN) + 16 * a + 4 * g, acc[a][b]);
 				}
 			}
 		}
@@ -741,13 +729,16 @@ namespace litenn_hip
 			dense_row_kernel<R><<<dim3(blocks), dim3(kRowThreads), lds, s>>>(args);
 		}
 
-		template <int BM, int BN, int WM, int WN>
+		template <int BM, int BN, int WM, int WN, int KG, bool F32>
 		void launch_tile(TileArgs& args, hipStream_t s)
 		{
+			constexpr size_t lds = sizeof(uint16_t) * KG * 2 * kTileK * ((F32 ? 3 : 1) * BM + BN);
+			static_assert(lds <= 160 * 1024 && sizeof(float) * (KG - 1) * BM * BN <= lds, "LDS");
+			allow_dynamic_lds(reinterpret_cast<const void*>(&dense_tile_kernel<BM, BN, WM, WN, KG, F32>), lds);
 			args.m_tiles = (args.d.m + BM - 1) / BM;
 			args.n_tiles = (args.d.w.n + BN - 1) / BN;
 			const int per = (args.m_tiles * args.n_tiles + 7) / 8;
-			dense_tile_kernel<BM, BN, WM, WN><<<dim3(8 * per, args.d.splits), dim3(256), 0, s>>>(args);
+			dense_tile_kernel<BM, BN, WM, WN, KG, F32><<<dim3(8 * per, args.d.splits), dim3(256 * KG), lds, s>>>(args);
 		}
 
 		int tiles(const DenseRows& d, int bm, int bn) { return ((d.m + bm - 1) / bm) * ((d.w.n + bn - 1) / bn); }
@@ -797,29 +788,49 @@ namespace litenn_hip
 			return;
 		}
 		TileArgs args{ a, 0, 0 };
+		// Tallest tile that still gives a SIMD two wavefronts, from one workgroup's groups if need be.  Figures: us, kernel
+		// alone, the next smaller choice against the one taken.
+		const int steps = a.w.pitch / kTileK / a.splits;
+		const auto work = [&](int bm, int bn) { return tiles(a, bm, bn) * a.splits; };
 		if (a.f32)
 		{
-			args.m_tiles = (a.m + kF32Tile - 1) / kF32Tile;
-			args.n_tiles = (a.w.n + kF32Tile - 1) / kF32Tile;
-			const int per = (args.m_tiles * args.n_tiles + 7) / 8;
-			dense_tile_f32_kernel<<<dim3(8 * per), dim3(256), 0, s>>>(args);
-			return;
+			// width 2048 at 500 rows: ff 11264 rows 109 -> 100 (one group), 2048 rows 50 -> 39 (two)
+			if (a.m > 32 && work(64, 128) >= 384)
+			{
+				launch_tile<64, 128, 2, 2, 1, true>(args, s);
+			}
+			else if (a.m > 32 && work(64, 128) >= 192)
+			{
+				launch_tile<64, 128, 2, 2, 2, true>(args, s);
+			}
+			else // width 2048 at 30 rows: 4096 rows 28 -> 19 against one group's 64 x 64
+			{
+				launch_tile<32, 64, 1, 4, 2, true>(args, s);
+			}
 		}
-		if (a.m <= 32)
+		else if (a.m > 64 && tiles(a, 128, 128) >= 384) // width 2048 at 777 rows, 6432 rows 53 -> 45
 		{
-			launch_tile<32, 64, 1, 4>(args, s);
+			launch_tile<128, 128, 2, 2, 1, false>(args, s);
 		}
-		else if (tiles(a, 128, 128) >= 384)
+		else if (a.m > 64 && work(128, 64) >= 384) // 28672 x 4096 at 100 rows 75 -> 65
 		{
-			launch_tile<128, 128, 2, 2>(args, s);
+			launch_tile<128, 64, 2, 2, 1, false>(args, s);
 		}
-		else if (a.m > 64 && tiles(a, 128, 64) >= 192)
+		else if (a.m > 64 && work(128, 64) >= 192 && steps >= 48) // 2048 x 5632 at 777 rows 49 -> 42; 5632 x 1024 at 300 rows 13 -> 21
 		{
-			launch_tile<128, 64, 2, 2>(args, s);
+			launch_tile<128, 64, 2, 2, 2, false>(args, s);
 		}
-		else
+		else if (a.m > 32 && work(64, 64) >= 384) // 5632 x 1024 at 300 rows 16 -> 13
 		{
-			launch_tile<64, 64, 2, 2>(args, s);
+			launch_tile<64, 64, 2, 2, 1, false>(args, s);
+		}
+		else if (a.m > 32 && work(64, 64) >= 192) // 6144 x 4096 at 100 rows 29 (one group) -> 23
+		{
+			launch_tile<64, 64, 2, 2, 2, false>(args, s);
+		}
+		else // 4096 x 1536 at 100 rows 12 -> 9, width 2048 at 30 rows 149 -> 123 for all products
+		{
+			launch_tile<32, 64, 1, 4, 2, false>(args, s);
 		}
 	}
 } // namespace litenn_hip

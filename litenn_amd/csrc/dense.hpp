@@ -69,11 +69,11 @@ namespace litenn_hip
 		void* c = nullptr;
 		int ldc = 0; // a multiple of 4 for the operand types
 		int out = kOutF32;
-		// kOutF32 with bfloat16 operands: the products of `splits` ranges of K, split_stride floats apart, to be
+		// kOutF32: the products of `splits` ranges of K, split_stride floats apart, to be
 		// added by the reader (see dense_rows_splits)
 		int splits = 1;
 		size_t split_stride = 0;
-		bool f32 = false; // Float32 operands (the bfloat16 weights widened exactly), f32 matrix instructions
+		bool f32 = false; // Float32 operands
 		ClampedGlu act;
 		float softcap = 0.0f; // kOutF32: > 0: c becomes softcap tanh(c / softcap)
 	};

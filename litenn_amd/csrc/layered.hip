@@ -965,7 +965,7 @@ namespace litenn_hip
 				d.c = y;
 				d.ldc = ld_y;
 				d.f32 = f32;
-				d.splits = parts = !f32 && rows <= kSplitRows ? dense_rows_splits(w, rows) : 1;
+				d.splits = parts = rows <= kSplitRows ? dense_rows_splits(w, rows) : 1;
 				d.split_stride = part_stride;
 				launch_dense_rows(d, stream);
 				pending = after;

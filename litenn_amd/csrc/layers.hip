@@ -1530,11 +1530,16 @@ namespace litenn_hip
 			return;
 		}
 		const dim3 grid(a.rows), threads(256);
-		if (a.f32)
+		const bool one = !a.sub || a.sub_parts == 1;
+		if (a.f32 && one)
 		{
 			add_norm_kernel<float, 1><<<grid, threads, 0, s>>>(a);
 		}
-		else if (!a.sub || a.sub_parts == 1)
+		else if (a.f32)
+		{
+			add_norm_kernel<float, kDenseMaxSplits><<<grid, threads, 0, s>>>(a);
+		}
+		else if (one)
 		{
 			add_norm_kernel<uint16_t, 1><<<grid, threads, 0, s>>>(a);
 		}
