@@ -501,7 +501,11 @@ namespace litenn_hip
 			// ---- weights: piece i of this lane is piece (64 i + lane) % P of row (64 i + lane) / P; the last pieces of a
 			// partial chunk, and of an aligned one, lie behind the row: they fetch the row's last piece again
 			uint8_t* const slot = lds + kRingBytes + wave * (NG * kTile * kStride);
-			const uint8_t* piece_row[kWLoads]; // the 16-byte boundary at or below the row's start
+			// (addresses of the global segment: a load through a generic pointer counts as an LDS access too, and every
+			// wait for LDS would wait for it)
+			typedef const __attribute__((address_space(1))) uint8_t* global_bytes_t;
+			typedef const __attribute__((address_space(1))) u32x4* global_u32x4_t;
+			global_bytes_t piece_row[kWLoads]; // the 16-byte boundary at or below the row's start
 			int piece_at[kWLoads], piece_last[kWLoads], piece_slot[kWLoads];
 #pragma unroll
 			for (int i = 0; i < kWLoads; ++i)
@@ -509,7 +513,7 @@ namespace litenn_hip
 				const int id = min(64 * i + lane, kRowPieces - 1), row = id / P;
 				const uintptr_t start = reinterpret_cast<uintptr_t>(w) + static_cast<size_t>(min(n_base + row, n - 1)) * row_bytes;
 				const int mis = static_cast<int>(start & 15);
-				piece_row[i] = reinterpret_cast<const uint8_t*>(start - mis);
+				piece_row[i] = (global_bytes_t)(start - mis);
 				piece_at[i] = mis; // byte offset of the chunk's start from the row's first piece, plus piece offset below
 				piece_last[i] = static_cast<int>((mis + row_bytes - 1) & ~size_t{ 15 });
 				piece_slot[i] = row * kStride + 16 * (id - row * P);
@@ -521,7 +525,7 @@ namespace litenn_hip
 				{
 					const int id = min(64 * i + lane, kRowPieces - 1);
 					const int at = min(((piece_at[i] + c * F::kChunkBytes) & ~15) + 16 * (id % P), piece_last[i]);
-					moving[i] = *reinterpret_cast<const u32x4*>(piece_row[i] + at);
+					moving[i] = *(global_u32x4_t)(piece_row[i] + at);
 				}
 			};
 			const auto deposit_w = [&]() {
