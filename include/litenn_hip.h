@@ -244,8 +244,10 @@ int litenn_hip_attn_decode_noalloc(int dev, const void* q, const void* kcache, c
  * run on the matrix cores (fp16 operands: q / sqrt(d)
  * and the softmax weights are rounded once, f32 accumulation and softmax; relative L2 error
  * about 3e-4), tiled so that the keys are read once per 64 rows instead of once per row.
- * flags: LITENN_HIP_MATMUL_PRECISE keeps the f32 row kernel of litenn_hip_attn_decode, which
- * every other shape uses as well. */
+ * flags: LITENN_HIP_MATMUL_PRECISE keeps f32 operands, as every other shape does: 8 rows and more
+ * (16 on an F32 cache) on 96 keys and more, with heads of at most 128, run on the matrix cores as
+ * sums of 16-bit parts that carry the f32 operands, fewer in the row kernel of
+ * litenn_hip_attn_decode. */
 int litenn_hip_attn_rows(int dev, const void* q, const void* kcache, const void* vcache, int cache_dtype, size_t m,
                          size_t past, size_t n_head, size_t n_kv_head, size_t head_dim, void* out, unsigned flags,
                          const litenn_hip_exec* opts);
@@ -269,7 +271,8 @@ typedef struct litenn_hip_attn_ext_opts
  * k / v [keys, n_kv_head, head_dim] F16 or F32, out [m, n_head, head_dim] F32; query head h reads kv
  * head h / (n_head / n_kv_head).  o == NULL means no option (scale 1, no mask).  The LLaMA lowering
  * uses none of the options and goes through litenn_hip_attn_decode / litenn_hip_attn_rows; this
- * entry point is a plain f32 row kernel.  The tanh is (exp(2x) - 1) / (exp(2x) + 1) in f32 as in the
+ * entry point computes with f32 operands throughout (the kernels and limits that
+ * LITENN_HIP_MATMUL_PRECISE selects there).  The tanh is (exp(2x) - 1) / (exp(2x) + 1) in f32 as in the
  * reference, NaN once 2x exceeds 88.  Refused: max_bias without a mask (the reference's text), a
  * causal mask that hides every key from the first row (key_position_offset beyond
  * query_position_offset; the reference computes a softmax over scores of -1e9 there), more than

@@ -15,10 +15,12 @@
 //     six products whose terms reach 2^-24 are formed.
 // Scores, softmax and sums are Float32 as in the row kernels.
 //
-// One wavefront fits a SIMD (256 + 88 registers, most of them the queries' two halves and the outputs), so a tile
-// is one chain: stage, 16 products, softmax, 16 products.  200 rows on 1000 keys (32 heads of 128 over 8, mask,
-// slopes, soft cap and sinks) take 66 us where the row kernel took 1365, of which 21 are the options' arithmetic;
-// against 64 bits 3.8e-7, as before.
+// A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
+// a SIMD (250 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
+// where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
+// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) take 30 us, with mask, slopes, soft cap and sinks 35,
+// where the row kernel took 1365; one wavefront a SIMD, two of them sharing their keys, took 46 and 59.  Against 64
+// bits 3.8e-7, as before.  Float32 keys and values (three times the products, one wavefront a SIMD): 89 and 101 us.
 #include "common.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
@@ -100,24 +102,28 @@ namespace litenn_hip
 			return head < head_log2 ? pow(m0, static_cast<double>(head + 1)) : pow(m1, static_cast<double>(2 * (head - head_log2) + 1));
 		}
 
-		// Bytes between staged rows: keys are read 16 bytes per row by consecutive rows (16 rows cover the 64 banks
-		// once), values as four rows of 64 bytes (four rows cover them once).
+		// Rows of keys and values lie 2 D bytes apart in LDS, their 16-byte pieces permuted by the row so that the 64 banks
+		// are covered evenly: keys are read as a piece of each of 16 rows, values as 64 bytes of each of four.
 		template <int D>
-		constexpr int key_stride() { return 2 * D + 16; }
+		__device__ __forceinline__ int key_slot(int row, int piece) { return piece ^ (D == 128 ? row & 15 : (row >> 1) & 7); }
 		template <int D>
-		constexpr int value_stride() { return 2 * D + 64; }
+		__device__ __forceinline__ int value_slot(int row, int piece)
+		{
+			return piece ^ (D == 128 ? (row & 3) << 2 | ((row >> 2) & 3) : (row & 2) << 1);
+		}
 
 		// A workgroup takes 32 QW query rows of one head; its KW groups of QW wavefronts take the key tiles in turn,
 		// each group with its own buffers, and merge at the end.
 		template <typename O, int D, int QW, int KW>
-		__global__ __launch_bounds__(64 * QW * KW) void attn_rows_kernel(const RowsAttn a)
+		__global__ __launch_bounds__(64 * QW * KW, O::kStored == 1 ? 2 : 1) void attn_rows_kernel(const RowsAttn a)
 		{
 			typedef typename O::frag frag;
 			typedef typename O::stored stored;
-			constexpr int KS = key_stride<D>(), VS = value_stride<D>();
-			constexpr int kKeyBytes = kKeys * KS, kValueBytes = kKeys * VS; // of one piece
-			constexpr int kGroupBytes = O::kStored * (kKeyBytes + kValueBytes);
-			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KW][keys, values]; later the groups' results
+			constexpr int RS = 2 * D, kTileBytes = kKeys * RS; // of one part of the keys or the values
+			constexpr int kGroupBytes = 2 * O::kStored * kTileBytes;
+			// The second half of the queries waits in LDS where every wavefront has the same ones and registers are short
+			constexpr bool kQueriesInLds = O::kSplit == 2 && QW == 1 && D == 128;
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KW][keys, values], queries; later the groups' results
 			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 			const int group = wave / QW, qw = wave % QW;
 			const int tid = qw * 64 + lane; // within the group
@@ -149,17 +155,30 @@ namespace litenn_hip
 			frag q[D / 16][O::kSplit];
 			float unscale = 1.0f;
 			{
+				// (whole groups of eight; one behind the head's last loads the first again and is dropped: the loads must not
+				// hang on branches, or each waits for the one before)
 				const float* src = a.q + static_cast<size_t>(row_c) * a.ldq + static_cast<size_t>(head) * a.dim;
 				float v[D / 16][8];
 				float mx = 0.0f;
 #pragma unroll
 				for (int s = 0; s < D / 16; ++s)
 				{
+					const int d = 16 * s + 8 * h;
+					const floatx4_a4* at = reinterpret_cast<const floatx4_a4*>(src + (d < a.dim ? d : 0));
+					const floatx4 x = at[0], y = at[1];
 #pragma unroll
 					for (int e = 0; e < 8; ++e)
 					{
-						const int d = 16 * s + 8 * h + e;
-						v[s][e] = d < a.dim ? src[d] : 0.0f;
+						v[s][e] = e < 4 ? x[e & 3] : y[e & 3];
+					}
+				}
+#pragma unroll
+				for (int s = 0; s < D / 16; ++s)
+				{
+#pragma unroll
+					for (int e = 0; e < 8; ++e)
+					{
+						v[s][e] = 16 * s + 8 * h < a.dim ? v[s][e] : 0.0f;
 						const float m = fabsf(v[s][e]);
 						mx = m <= 3.402823466e38f ? fmaxf(mx, m) : mx;
 					}
@@ -181,18 +200,24 @@ namespace litenn_hip
 					}
 				}
 			}
-			float slope = 1.0f;
-			bool apply_slope = false;
-			if (a.mask && a.max_bias > 0.0)
+			uint8_t* const q_lds = lds + KW * kGroupBytes + lane * 16;
+			if constexpr (kQueriesInLds)
 			{
-				const double sl = row_alibi_slope(head, a.heads, a.max_bias);
-				slope = static_cast<float>(sl);
-				apply_slope = sl != 1.0;
+				if (group == 0)
+				{
+#pragma unroll
+					for (int s = 0; s < D / 16; ++s)
+					{
+						*reinterpret_cast<frag*>(q_lds + 1024 * s) = q[s][1];
+					}
+				}
+				__syncthreads();
 			}
+			const float slope = a.mask && a.max_bias > 0.0 ? static_cast<float>(row_alibi_slope(head, a.heads, a.max_bias)) : 1.0f;
 			const float* const mask_row = a.mask ? a.mask + static_cast<size_t>(row_c) * keys : nullptr;
 
 			// a dot product's score (the causal mask and the window aside)
-			const auto score_of = [&](float v, int key) {
+			const auto score_of = [&](float v, float mv) {
 				if (a.apply_scale)
 				{
 					v = __fmul_rn(v, a.scale);
@@ -207,43 +232,47 @@ namespace litenn_hip
 						v = __fmul_rn(v, a.softcap);
 					}
 				}
-				if (mask_row)
+				if (a.mask)
 				{
-					float mv = mask_row[key];
-					if (apply_slope)
-					{
-						mv = __fmul_rn(mv, slope);
-					}
-					v = __fadd_rn(v, mv);
+					v = __fadd_rn(v, __fmul_rn(mv, slope)); // (a slope of 1 leaves the mask as it is)
 				}
 				return v;
 			};
 
 			// ---- staging: a thread moves 8-element pieces of rows
 			uint8_t* const k_lds = lds + group * kGroupBytes;
-			uint8_t* const v_lds = k_lds + O::kStored * kKeyBytes;
-			constexpr int kRowPieces = D / 8, kPieces = kKeys * kRowPieces / (64 * QW);
-			static_assert(kPieces * 64 * QW == kKeys * kRowPieces, "pieces per thread");
+			uint8_t* const v_lds = k_lds + O::kStored * kTileBytes;
+			constexpr int kRowPieces = D / 8, kPieces = kKeys * kRowPieces / (64 * QW), kRowStep = 64 * QW / kRowPieces;
+			static_assert(kPieces * 64 * QW == kKeys * kRowPieces && kRowStep * kRowPieces == 64 * QW, "pieces per thread");
 			constexpr int kWords = sizeof(stored) / 2; // 16-byte words of a piece
+			const int piece_row = tid / kRowPieces, piece = tid % kRowPieces; // first row, and the same column in all of them
 			u32x4 kr[kPieces][kWords], vr[kPieces][kWords];
-			const auto request = [&](int tile) {
+			const uint32_t ldk = static_cast<uint32_t>(a.ldk), ldv = static_cast<uint32_t>(a.ldv);
+			// (a piece behind the head's last loads the first again and is zeroed on its way into LDS)
+			const stored* const k_piece = kb + (8 * piece < a.dim ? 8 * piece : 0);
+			const stored* const v_piece = vb + (8 * piece < a.vdim ? 8 * piece : 0);
+			const auto request = [&](u32x4 (&into)[kPieces][kWords], const stored* from, uint32_t ld, int tile) {
 #pragma unroll
 				for (int i = 0; i < kPieces; ++i)
 				{
-					const int c = tid + 64 * QW * i, key = min(first + tile * kKeys + c / kRowPieces, last - 1), d = (c % kRowPieces) * 8;
-					const size_t at = buffer_row(key);
+					const uint32_t at = buffer_row(min(first + tile * kKeys + piece_row + kRowStep * i, last - 1));
 #pragma unroll
 					for (int w = 0; w < kWords; ++w)
 					{
-						kr[i][w] = d < a.dim ? *reinterpret_cast<const u32x4*>(kb + at * a.ldk + d + 4 * w) : u32x4{ 0u, 0u, 0u, 0u };
-						vr[i][w] = d < a.vdim ? *reinterpret_cast<const u32x4*>(vb + at * a.ldv + d + 4 * w) : u32x4{ 0u, 0u, 0u, 0u };
+						into[i][w] = *reinterpret_cast<const u32x4*>(from + static_cast<uint64_t>(at) * ld + 4 * w);
 					}
 				}
 			};
-			const auto store_piece = [&](uint8_t* dst, int piece_bytes, const u32x4 (&w)[kWords]) {
+			const auto store_piece = [&](uint8_t* dst, const u32x4 (&w)[kWords], bool there) {
+				u32x4 v[kWords];
+#pragma unroll
+				for (int i = 0; i < kWords; ++i)
+				{
+					v[i] = there ? w[i] : u32x4{ 0u, 0u, 0u, 0u };
+				}
 				if constexpr (O::kStored == 1)
 				{
-					*reinterpret_cast<u32x4*>(dst) = w[0];
+					*reinterpret_cast<u32x4*>(dst) = v[0];
 				}
 				else
 				{
@@ -251,22 +280,29 @@ namespace litenn_hip
 #pragma unroll
 					for (int e = 0; e < 8; ++e)
 					{
-						O::split(__uint_as_float(w[e / 4][e % 4]), e, f);
+						O::split(__uint_as_float(v[e / 4][e % 4]), e, f);
 					}
 #pragma unroll
 					for (int p = 0; p < O::kStored; ++p)
 					{
-						*reinterpret_cast<frag*>(dst + p * piece_bytes) = f[p];
+						*reinterpret_cast<frag*>(dst + p * kTileBytes) = f[p];
 					}
 				}
 			};
-			const auto deposit = [&]() {
+			const auto deposit_keys = [&]() {
 #pragma unroll
 				for (int i = 0; i < kPieces; ++i)
 				{
-					const int c = tid + 64 * QW * i, key = c / kRowPieces, d = (c % kRowPieces) * 8;
-					store_piece(k_lds + key * KS + 2 * d, kKeyBytes, kr[i]);
-					store_piece(v_lds + key * VS + 2 * d, kValueBytes, vr[i]);
+					const int key = piece_row + kRowStep * i;
+					store_piece(k_lds + key * RS + 16 * key_slot<D>(key, piece), kr[i], 8 * piece < a.dim);
+				}
+			};
+			const auto deposit_values = [&]() {
+#pragma unroll
+				for (int i = 0; i < kPieces; ++i)
+				{
+					const int key = piece_row + kRowStep * i;
+					store_piece(v_lds + key * RS + 16 * value_slot<D>(key, piece), vr[i], 8 * piece < a.vdim);
 				}
 			};
 			const auto meet = [&]() {
@@ -287,20 +323,48 @@ namespace litenn_hip
 				o[b] = floatx16{};
 			}
 			float run_m = -INFINITY, run_l = 0.0f; // run_l: of this lane's keys
+			// Keys travel while the previous tile's values are used and go into LDS once its scores are formed, values the
+			// other way round: one of the two is in registers at a time.
+			const auto tile_at = [&](int step) { return min(step * KW + group, tiles - 1); };
 			if (steps > 0)
 			{
-				request(min(group, tiles - 1));
+				request(kr, k_piece, ldk, tile_at(0));
+				deposit_keys();
+				request(vr, v_piece, ldv, tile_at(0));
 			}
 			for (int step = 0; step < steps; ++step)
 			{
 				const int tile = step * KW + group;
 				const bool live = tile < tiles; // a group without a tile left goes through the motions on the last one
 				const int base = first + min(tile, tiles - 1) * kKeys;
-				meet(); // the previous tile has been consumed
-				deposit();
-				request(min(tile + KW, tiles - 1));
-				meet();
-
+				// the tile's mask: four runs of four keys (at the mask's end the last whole run there is, shifted below)
+				float mask[16];
+				if (a.mask)
+				{
+#pragma unroll
+					for (int e = 0; e < 16; e += 4)
+					{
+						const int key = base + 2 * e + 4 * h, from = max(0, min(key, keys - 4));
+						const floatx4 x = *reinterpret_cast<const floatx4_a4*>(mask_row + from);
+#pragma unroll
+						for (int i = 0; i < 4; ++i)
+						{
+							mask[e + i] = x[i];
+						}
+						if (base + kKeys > keys)
+						{
+#pragma unroll
+							for (int i = 0; i < 3; ++i)
+							{
+								const bool shifted = key - from > i;
+								mask[e] = shifted ? mask[e + 1] : mask[e];
+								mask[e + 1] = shifted ? mask[e + 2] : mask[e + 1];
+								mask[e + 2] = shifted ? mask[e + 3] : mask[e + 2];
+							}
+						}
+					}
+				}
+				meet(); // the tile's keys are there, the previous tile's values have been used
 				floatx16 s = {};
 #pragma unroll
 				for (int st = 0; st < D / 16; ++st)
@@ -308,10 +372,19 @@ namespace litenn_hip
 #pragma unroll
 					for (int p = 0; p < O::kProducts; ++p)
 					{
-						const frag kf = *reinterpret_cast<const frag*>(k_lds + O::stored_of[p] * kKeyBytes + j * KS + 32 * st + 16 * h);
-						s = O::multiply(kf, q[st][O::split_of[p]], s);
+						const frag kf = *reinterpret_cast<const frag*>(k_lds + O::stored_of[p] * kTileBytes + j * RS + 16 * key_slot<D>(j, 2 * st + h));
+						if constexpr (kQueriesInLds)
+						{
+							s = O::multiply(kf, p == 0 ? q[st][0] : *reinterpret_cast<const frag*>(q_lds + 1024 * st), s);
+						}
+						else
+						{
+							s = O::multiply(kf, q[st][O::split_of[p]], s);
+						}
 					}
 				}
+				deposit_values();
+				request(kr, k_piece, ldk, tile_at(step + 1));
 				// lane (j, h) holds keys base + 8 (e / 4) + 4 h + e % 4 of query j
 				float sc[16];
 				float top = -INFINITY;
@@ -320,7 +393,7 @@ namespace litenn_hip
 				{
 					const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
 					const bool visible = live && key >= lo && key < hi;
-					const float v = score_of(s[e] * unscale, visible ? key : lo);
+					const float v = score_of(s[e] * unscale, mask[e]);
 					sc[e] = visible ? v : -INFINITY;
 					top = fmaxf(top, sc[e]);
 				}
@@ -349,7 +422,10 @@ namespace litenn_hip
 				}
 				// step u: keys 16 u + 4 h + 0..3 and 16 u + 8 + 4 h + 0..3.  Sixteen lanes read four keys' rows of
 				// sixteen dimensions, eight bytes each, and get the four keys of one dimension
-				const int v_off = ((lane & 15) >> 2) * VS + (lane & 3) * 8 + ((lane >> 4) & 1) * 32;
+				meet(); // the tile's values are there, its keys have been used
+				deposit_keys();
+				request(vr, v_piece, ldv, tile_at(step + 1));
+				const int v_row = 4 * h + ((lane & 15) >> 2), v_col = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), v_byte = (lane & 1) * 8;
 #pragma unroll
 				for (int u = 0; u < 2; ++u)
 				{
@@ -361,9 +437,10 @@ namespace litenn_hip
 						for (int p = 0; p < O::kStored; ++p)
 						{
 							typedef __attribute__((address_space(3))) short4v* lds_short4;
-							const uint8_t* at = v_lds + p * kValueBytes + (16 * u + 4 * h) * VS + 64 * b + v_off;
-							const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at)));
-							const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + 8 * VS)));
+							const int r0 = 16 * u + v_row, r1 = r0 + 8;
+							const uint8_t* const at = v_lds + p * kTileBytes + v_byte;
+							const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + r0 * RS + 16 * value_slot<D>(r0, 4 * b + v_col))));
+							const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + r1 * RS + 16 * value_slot<D>(r1, 4 * b + v_col))));
 							vf[p] = __builtin_bit_cast(frag, u32x4{ x.x, x.y, y.x, y.y });
 						}
 #pragma unroll
@@ -471,7 +548,7 @@ namespace litenn_hip
 					{
 						dot = fmaf(src[d], widen(kr0[d]), dot);
 					}
-					const float v = score_of(dot, key);
+					const float v = score_of(dot, a.mask ? mask_row[key] : 0.0f);
 					const float new_m = fmaxf(run_m, v), ref_m = new_m == -INFINITY ? 0.0f : new_m;
 					const float corr = expf(run_m - ref_m), p = expf(v - ref_m);
 					run_m = new_m;
@@ -526,7 +603,7 @@ namespace litenn_hip
 		template <typename O, int D, int QW, int KW>
 		void launch_form(const RowsAttn& a, hipStream_t s)
 		{
-			constexpr size_t tiles = static_cast<size_t>(KW) * O::kStored * kKeys * (key_stride<D>() + value_stride<D>());
+			constexpr size_t tiles = static_cast<size_t>(KW) * O::kStored * kKeys * 4 * D + (O::kSplit == 2 && QW == 1 && D == 128 ? 64 * D : 0);
 			constexpr size_t merge = static_cast<size_t>(KW - 1) * QW * (D / 2 + 2) * 64 * sizeof(float);
 			constexpr size_t lds = tiles > merge ? tiles : merge;
 			static_assert(lds <= 160 * 1024, "LDS");
@@ -541,15 +618,20 @@ namespace litenn_hip
 			{
 				launch_form<FloatOperands, D, 2, 2>(a, s);
 			}
-			// Wavefronts that keep to themselves and share out the keys, except where there are few key tiles (us, 32 heads
-			// of 128: 200 rows on 1000 keys 45 against 63 with pairs on shared tiles, 220 rows on 128 keys about even, 33 rows on 33 keys 19 against 14)
-			else if (a.keys > 4 * kKeys)
-			{
-				launch_form<HalfOperands, D, 1, 4>(a, s);
-			}
 			else
 			{
-				launch_form<HalfOperands, D, 2, 2>(a, s);
+				// Eight wavefronts on a head's rows, one workgroup to a CU, while all of them fit the 256 CUs at once and each wavefront
+				// has two tiles; else four, two workgroups to a CU (us for eight and four: 200 rows on 1000 keys 35 and 39, 16 on
+				// 4000 79 and 105, 128 on 128 19 and 14, 512 on 1024 64 and 47, 1500 on 4000 447 and 401).
+				const size_t groups = static_cast<size_t>(a.heads) * ((a.rows + 31) / 32);
+				if (groups <= 256 && a.keys >= 512)
+				{
+					launch_form<HalfOperands, D, 1, 8>(a, s);
+				}
+				else
+				{
+					launch_form<HalfOperands, D, 1, 4>(a, s);
+				}
 			}
 		}
 	} // namespace
@@ -587,7 +669,7 @@ namespace litenn_hip
 		const int piece = f32 ? 4 : 8; // elements of 16 bytes
 		if (a.rows <= 0 || a.heads <= 0 || a.dim % 8 != 0 || a.vdim % 8 != 0 || a.dim <= 0 || a.vdim <= 0 || a.dim > 128 || a.vdim > 128 ||
 		    a.ldk % piece != 0 || a.ldv % piece != 0 || a.k_head % piece != 0 || a.v_head % piece != 0 || a.ldo % 4 != 0 ||
-		    !aligned(a.k) || !aligned(a.v) || !aligned(a.out) || (a.rows + 31) / 32 > 65535)
+		    a.ldk > 0xffffffffu || a.ldv > 0xffffffffu || (a.mask && a.keys < 4) || !aligned(a.k) || !aligned(a.v) || !aligned(a.out) || (a.rows + 31) / 32 > 65535)
 		{
 			return false;
 		}

@@ -34,7 +34,7 @@ namespace litenn_hip
 	};
 
 	// Whether the rows are many enough, and the keys they see, for the tiles to pay (us against the row kernels, 32 heads of
-	// 128: Float16 keys, 12 rows on 100 keys 17 against 20, 32 rows on 32 keys 14 against 13, 8 on 1024 38 against 131;
+	// 128: Float16 keys, 12 rows on 100 keys 13 against 20, 32 rows on 32 keys 14 against 13, 8 on 1024 26 against 131;
 	// Float32 keys, 8 rows on 300 keys 37 against 37, heads of 64 24 against 19).
 	inline bool attn_rows_pays(size_t rows, size_t keys, bool f32) { return rows >= (f32 ? 16u : 8u) && keys >= 96; }
 
