@@ -135,7 +135,9 @@ int litenn_hip_permute(int dev, void* dst, int dtype, const size_t* src_shape, s
  * from and returned to the device's memory pool in stream order, see below).
  * residual (f32 [m, n]) may be NULL; when given, y = residual + x.W
  * (the Add at tools/gguf/LLaMABuilder.cpp:652-653,661-663).  residual may alias y.
- * m == 1..3 runs the streaming GEMV, row by row (f32 operands).  m >= 4 (with k a multiple of 256;
+ * m == 1 runs the streaming GEMV (f32 operands).  m == 2 and 3 against Q4_0, Q8_0, Q4_K, Q5_K or Q6_K keep f32
+ * operands as under LITENN_HIP_MATMUL_PRECISE below; other formats go row by row through the GEMV.  m >= 4 (with k a
+ * multiple of 256;
  * the threshold was 16 in earlier versions of this library, and a caller that sized a workspace
  * for 4 <= m < 16 by that rule - zero bytes - must size it with
  * litenn_hip_mul_mat_q_workspace_bytes now) runs on the
@@ -143,10 +145,11 @@ int litenn_hip_permute(int dev, void* dst, int dtype, const size_t* src_shape, s
  * single-row launches): weights and activations are rounded to fp16 once each (activation rows are first scaled
  * by a power of two into the fp16 range), products accumulate in f32; relative L2 error about
  * 4e-4.  LITENN_HIP_MATMUL_PRECISE in `flags` keeps f32 operands for any m: Q4_0, Q8_0, Q4_K, Q5_K and Q6_K
- * with k <= 16384 and m >= 8 on the matrix cores (weights as exact integers, every activation as two halves that carry
- * its Float32 digits, block scales and sums in f32: the streaming GEMV's accuracy), in scratch of the
- * device's memory pool or in a given workspace if it has 4.125 * m * k bytes and some (m rounded up to 32, k
- * to 256); without such room, and for the other formats, row by row through the GEMV, which needs none.
+ * on the matrix cores (weights as exact integers, every activation as two halves that carry its Float32 digits,
+ * block scales and sums in f32: the streaming GEMV's accuracy), 2 to 8 rows in one launch without scratch, more with
+ * k <= 16384 in scratch of the device's memory pool or in a given workspace if it has 4.125 * m * k bytes and some
+ * (m rounded up to 32, k to 256); without such room, and for the other formats, row by row through the GEMV, which
+ * needs none.
  * The matrix-core path needs a device workspace of litenn_hip_mul_mat_q_workspace_bytes(m, k):
  * litenn_hip_mul_mat_q takes it from the device's memory pool in stream order (hipMallocAsync /
  * hipFreeAsync on the call's stream: no wait for the stream, opts->synchronize is honoured; only

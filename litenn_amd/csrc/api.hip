@@ -19,6 +19,8 @@ namespace litenn_hip
 	bool exact_gemm_takes(int fmt, const void* wq, size_t n, size_t k);
 	bool launch_exact_rows(const float* x, size_t m, size_t k, const float* norm_w, double eps, const float* up,
 	                       void* scratch, hipStream_t stream);
+	bool launch_exact_few(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y, const float* residual,
+	                      hipStream_t stream);
 	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
 	                       const float* residual, const void* scratch, hipStream_t stream);
 	bool launch_gemm(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y,
@@ -766,8 +768,12 @@ static bool is_weight_format(int fmt)
 // tile costs about as much as three single-row GEMVs (Q4_K 14336 x 4096: 14.6 us against 8.2 each).
 static constexpr size_t kMatrixCoreMinRows = 4;
 
-// From this many rows on a matmul with Float32 operands shares the weights between its rows.  Two launches and their
-// scratch from the pool take the host 21 us, a row of the streaming kernel 3.4 us and more of the GPU.
+// Up to this many rows with Float32 operands share the weights in one launch that needs no scratch (Q4_K 14336 x 4096 at
+// 8 rows 19.4 us, through scratch 25.6; the next row would double the fragments).
+static constexpr size_t kFewRows = 8;
+
+// From this many rows on a matmul with Float32 operands shares the weights between its rows through scratch (formats
+// or rows that the form above does not take go one by one below it).
 static constexpr size_t kExactMinRows = 8;
 
 extern "C" size_t litenn_hip_mul_mat_q_workspace_bytes(size_t m, size_t k)
@@ -833,6 +839,13 @@ extern "C" int litenn_hip_mul_mat_q_ws(int dev, int fmt, const void* wq, size_t 
 	float* yf = static_cast<float*>(y);
 	const float* rf = static_cast<const float*>(residual);
 	const bool quant = fmt != LITENN_FMT_F16 && fmt != LITENN_FMT_F32;
+	// Few rows share the weights in one launch without scratch (csrc/exact.hip, Float32 operands)
+	const bool keeps_f32 = (flags & LITENN_HIP_MATMUL_PRECISE) || m < kMatrixCoreMinRows || k % 256 != 0;
+	if (m >= 2 && m <= kFewRows && keeps_f32 && exact_gemm_takes(fmt, wq, n, k) &&
+	    launch_exact_few(fmt, wq, n, k, xf, m, yf, rf, s))
+	{
+		return finish_with(widened, action, opts);
+	}
 	if (m >= kMatrixCoreMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE) && quant && k % 256 == 0)
 	{
 		// the matrix-core path rounds the activations to fp16 into a workspace

@@ -171,6 +171,18 @@ namespace litenn_hip
 		return v;
 	}
 
+	// The largest of the wavefront's values, none of them negative or NaN (what a DPP step does not reach reads 0).
+	__device__ __forceinline__ float wave_max_nonnegative(float v)
+	{
+		v = fmaxf(v, dpp_f32<0xB1>(v));
+		v = fmaxf(v, dpp_f32<0x4E>(v));
+		v = fmaxf(v, dpp_f32<0x141>(v));
+		v = fmaxf(v, dpp_f32<0x140>(v));
+		v = fmaxf(v, dpp_f32<0x142, 0xA>(v));
+		v = fmaxf(v, dpp_f32<0x143, 0xC>(v));
+		return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+	}
+
 	__device__ __forceinline__ float wave_max(float v)
 	{
 		for (int off = 32; off > 0; off >>= 1)

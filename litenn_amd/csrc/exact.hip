@@ -4,7 +4,7 @@
 // per row.  No operand is rounded to 16 bits:
 //
 //   * A GGUF weight is a small integer times a scale.  The integers (or, for the K-quants with six-bit
-//     sub-scales, integer times sub-scale: at most 63 * 31 < 2048) are exact in binary16 and are what
+//     sub-scales, integer times sub-scale: at most 63 * 16 and some) are exact in binary16 and are what
 //     the matrix cores multiply; the block's Float32 scale is applied to the Float32 sum of its
 //     products.
 //   * An activation is scaled by a power of two per row and taken apart into two binary16 values, hi =
@@ -14,13 +14,13 @@
 //     more product per 256 elements: the eight sums, taken apart the same way, against the eight
 //     six-bit minima.
 //
-// Against 64 bits the result is as close as the streaming kernel's (relative L2 1.0e-7 to 2.1e-7 over
-// K = 256 .. 14336 and every format; the streaming kernel has 1.4e-7 to 2.5e-7).
+// Against 64 bits the result is as close as the streaming kernel's (relative L2 0.8e-7 to 1.2e-7 over
+// K = 256 .. 14336 and every format; the streaming kernel has 0.9e-7 to 2.6e-7).
 //
 // What bounds it: few rows are the weights' stream and the launch; many rows, the LDS reads of the fragments (two
 // per pair of products) and the latency in front of them: a product issues every 100 cycles and SIMD where
 // it takes 32.  Row by row through the streaming kernel the same calls took, us, before -> now with the rows'
-// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 56; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
+// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 45; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
 //
 // v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
 // weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
@@ -33,7 +33,10 @@ namespace litenn_hip
 	namespace
 	{
 		typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+		typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 		typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+		typedef float floatx4 __attribute__((ext_vector_type(4)));
+		typedef floatx4 floatx4_a4 __attribute__((aligned(4)));
 		typedef float floatx16 __attribute__((ext_vector_type(16)));
 		typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 		typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -52,16 +55,24 @@ namespace litenn_hip
 		// path).  From there lane (r, h) = (lane % 32, lane / 32) takes, of weight row r, elements 16 s + 8 h .. + 7
 		// of step s (K in natural order).  A stage is 64 elements = steps 0..3.  Blocks are only 2-byte aligned.
 		typedef const __attribute__((address_space(3))) uint8_t* lds_bytes_t;
-		__device__ __forceinline__ u32x2 load8(lds_bytes_t p)
+		// `p` is on 8 bytes and `at` a constant once unrolled: LDS reads off their alignment are served lane by lane, which
+		// was most of the time of Q6_K's and Q8_0's matmuls, so what lies on 2 bytes is put together from dwords
+		__device__ __forceinline__ u32x2 load8(lds_bytes_t p, int at)
 		{
-			typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
-			return *(const __attribute__((address_space(3))) u32x2_a2*)(p);
+			typedef const __attribute__((address_space(3))) uint32_t* words_t;
+			if (at % 8 == 0)
+			{
+				return *(const __attribute__((address_space(3))) u32x2*)(p + at);
+			}
+			if (at % 4 == 0)
+			{
+				const words_t w = (words_t)(p + at);
+				return { w[0], w[1] };
+			}
+			const words_t w = (words_t)(p + at - 2);
+			return { __builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16) };
 		}
-		__device__ __forceinline__ u32x4 load16(lds_bytes_t p)
-		{
-			typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
-			return *(const __attribute__((address_space(3))) u32x4_a2*)(p);
-		}
+		__device__ __forceinline__ u32x4 load16(lds_bytes_t p) { return *(const __attribute__((address_space(3))) u32x4*)(p); }
 		__device__ __forceinline__ uint32_t load2(lds_bytes_t p) { return *(const __attribute__((address_space(3))) uint16_t*)(p); }
 
 		__device__ __forceinline__ half2v as_half2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
@@ -81,20 +92,42 @@ namespace litenn_hip
 			const half2v off = { m, m };
 			return join(biased01(a) + off, biased23(a) + off, biased01(b) + off, biased23(b) + off);
 		}
-		// eight unsigned bytes (at most 31) times the integer `scale` (at most 63): (1024 + q) s - 1024 s, fused
-		__device__ __forceinline__ half8 bytes_times(uint32_t a, uint32_t b, uint32_t scale)
+		// Integer q times sub-scale s, less about kCentre s: (1024 + q) s + off with off = -(1024 + centre) s rounded to a half,
+		// fused.  What is taken off is the integer -off - 1024 s = centred_by, exactly.
+		__device__ __forceinline__ half2v centre_offset(half2v s, float centre)
+		{
+			const _Float16 m = static_cast<_Float16>(-1024.0f - centre);
+			return s * half2v{ m, m };
+		}
+		__device__ __forceinline__ half2v centred_by(half2v s, float centre)
+		{
+			return -__builtin_elementwise_fma(s, half2v{ 1024, 1024 }, centre_offset(s, centre));
+		}
+		// eight unsigned bytes (at most 31) times the integer `scale` (at most 63), centred
+		__device__ __forceinline__ half8 bytes_times(uint32_t a, uint32_t b, uint32_t scale, float centre)
 		{
 			const half2v s = as_half2(0x64006400u | (scale * 0x00010001u)) - half2v{ 1024, 1024 };
-			const half2v off = s * half2v{ -1024, -1024 };
+			const half2v off = centre_offset(s, centre);
 			return join(__builtin_elementwise_fma(biased01(a), s, off), __builtin_elementwise_fma(biased23(a), s, off),
 			            __builtin_elementwise_fma(biased01(b), s, off), __builtin_elementwise_fma(biased23(b), s, off));
+		}
+		// what that took off, for the eight scales a, b, as the factors of sums times kSumScale (at most 960 * 64: a half)
+		__device__ __forceinline__ half8 centres(uint32_t a, uint32_t b, float centre)
+		{
+			const half2v off = { -1024, -1024 };
+			const _Float16 f = static_cast<_Float16>(1.0f / kSumScale);
+			return half8{ f, f, f, f, f, f, f, f } * join(centred_by(biased01(a) + off, centre), centred_by(biased23(a) + off, centre), centred_by(biased01(b) + off, centre),
+			            centred_by(biased23(b) + off, centre));
 		}
 
 		// Formats:
 		//   kBlock        elements of a block, kChunkBytes bytes of 256 elements
 		//   kScaleSteps   steps whose products share one scale: after them the sum is scaled and added
 		//   Head          what the lane needs of the chunk as a whole
-		//   kMins         whether a minimum term follows each chunk
+		//   kMins         whether a minimum term follows each chunk.  The integers are then taken about kCentre, the middle of
+		//                 their range, lower, and what that takes from the sum is added back per chunk, a product more over the
+		//                 sub-blocks' sums: the sums on the way stay as small as the result (relative error at Q5_K, 33 rows
+		//                 of 2048, 1.66e-7 without it)
 		// Rows whose last chunk is not whole (blocks of 32 only) load their last block again in the missing blocks'
 		// places and scale it by 0 (`blocks` whole blocks of the chunk are there).
 		struct Q4_0X
@@ -111,9 +144,8 @@ namespace litenn_hip
 				for (int b = 0; b < 2; ++b)
 				{
 					const int block = 2 * st + b;
-					lds_bytes_t p = chunk + 18 * block;
-					r.d[b] = block < blocks ? load2(p) : 0u;
-					r.q[b] = load8(p + 2 + 8 * h);
+					r.d[b] = block < blocks ? load2(chunk + 18 * block) : 0u;
+					r.q[b] = load8(chunk + 8 * h, 18 * block + 2);
 				}
 				return r;
 			}
@@ -141,10 +173,9 @@ namespace litenn_hip
 				for (int b = 0; b < 2; ++b)
 				{
 					const int block = 2 * st + b;
-					lds_bytes_t p = chunk + 34 * block;
-					r.d[b] = block < blocks ? load2(p) : 0u;
-					r.q[2 * b] = load8(p + 2 + 8 * h);
-					r.q[2 * b + 1] = load8(p + 18 + 8 * h);
+					r.d[b] = block < blocks ? load2(chunk + 34 * block) : 0u;
+					r.q[2 * b] = load8(chunk + 8 * h, 34 * block + 2);
+					r.q[2 * b + 1] = load8(chunk + 8 * h, 34 * block + 18);
 				}
 				return r;
 			}
@@ -160,13 +191,14 @@ namespace litenn_hip
 		{
 			static constexpr int kBlock = 256, kChunkBytes = 144, kScaleSteps = 16;
 			static constexpr bool kMins = true;
+			static constexpr float kCentre = 8.0f;
 			struct Head { u32x4 w; }; // d, dmin, 12 bytes of six-bit scales and minima
 			struct Raw { u32x2 q[2]; };
 			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return { load16(chunk) }; }
 			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int)
 			{
 				lds_bytes_t p = chunk + 16 + 32 * st + 8 * h;
-				return { { load8(p), load8(p + 16) } };
+				return { { load8(p, 0), load8(p, 16) } };
 			}
 			// get_scale_min_k4 of the ggml block definition, four sub-blocks to a dword
 			static __device__ __forceinline__ uint32_t scales(const u32x4& w, int four)
@@ -183,11 +215,12 @@ namespace litenn_hip
 				const int sh = 4 * (t >> 1), sub = 2 * st + (t >> 1);
 				const uint32_t s = (scales(hd.w, sub >> 2) >> (8 * (sub & 3))) & 0xffu;
 				const u32x2 q = r.q[t & 1];
-				return bytes_times((q.x >> sh) & 0x0f0f0f0fu, (q.y >> sh) & 0x0f0f0f0fu, s);
+				return bytes_times((q.x >> sh) & 0x0f0f0f0fu, (q.y >> sh) & 0x0f0f0f0fu, s, kCentre);
 			}
 			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
 			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.w.x); }
 			static __device__ __forceinline__ half8 min_frag(const Head& hd) { return bytes_minus(minima(hd.w, 0), minima(hd.w, 1), 0.0f); }
+			static __device__ __forceinline__ half8 centre_frag(const Head& hd) { return centres(scales(hd.w, 0), scales(hd.w, 1), kCentre); }
 			static __device__ __forceinline__ float min_scale(const Head& hd) { return -f16_bits_to_f32(hd.w.x >> 16); }
 		};
 
@@ -195,16 +228,17 @@ namespace litenn_hip
 		{
 			static constexpr int kBlock = 256, kChunkBytes = 176, kScaleSteps = 16;
 			static constexpr bool kMins = true;
+			static constexpr float kCentre = 15.0f; // (1040 * 63 is no half)
 			struct Head { u32x4 w; u32x2 fifth[2]; };
 			struct Raw { u32x2 q[2]; };
 			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int h)
 			{
-				return { load16(chunk), { load8(chunk + 16 + 8 * h), load8(chunk + 32 + 8 * h) } };
+				return { load16(chunk), { load8(chunk + 8 * h, 16), load8(chunk + 8 * h, 32) } };
 			}
 			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int)
 			{
 				lds_bytes_t p = chunk + 48 + 32 * st + 8 * h;
-				return { { load8(p), load8(p + 16) } };
+				return { { load8(p, 0), load8(p, 16) } };
 			}
 			static __device__ __forceinline__ half8 frag(const Head& hd, const Raw& r, int st, int t)
 			{
@@ -212,7 +246,7 @@ namespace litenn_hip
 				const uint32_t s = (Q4_KX::scales(hd.w, sub >> 2) >> (8 * (sub & 3))) & 0xffu;
 				const u32x2 q = r.q[t & 1], f = hd.fifth[t & 1]; // bit `sub` of a byte is its element's fifth bit
 				return bytes_times(((q.x >> sh) & 0x0f0f0f0fu) | (((f.x >> sub) & 0x01010101u) << 4),
-				                   ((q.y >> sh) & 0x0f0f0f0fu) | (((f.y >> sub) & 0x01010101u) << 4), s);
+				                   ((q.y >> sh) & 0x0f0f0f0fu) | (((f.y >> sub) & 0x01010101u) << 4), s, kCentre);
 			}
 			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
 			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.w.x); }
@@ -220,6 +254,7 @@ namespace litenn_hip
 			{
 				return bytes_minus(Q4_KX::minima(hd.w, 0), Q4_KX::minima(hd.w, 1), 0.0f);
 			}
+			static __device__ __forceinline__ half8 centre_frag(const Head& hd) { return centres(Q4_KX::scales(hd.w, 0), Q4_KX::scales(hd.w, 1), kCentre); }
 			static __device__ __forceinline__ float min_scale(const Head& hd) { return -f16_bits_to_f32(hd.w.x >> 16); }
 		};
 
@@ -231,12 +266,12 @@ namespace litenn_hip
 			static constexpr bool kMins = false;
 			struct Head { u32x4 sc; uint32_t d; };
 			struct Raw { u32x2 low[4], high[2]; }; // half st / 2 of the block: [32 x (first, second)] x 16-element runs
-			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return { load16(chunk + 192), load2(chunk + 208) }; }
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return { load16(chunk + 192), load2(chunk + 222) }; } // (the last piece ends with the block)
 			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int h, int)
 			{
 				lds_bytes_t ql = chunk + 64 * (st >> 1) + 8 * h;
 				lds_bytes_t qh = chunk + 128 + 32 * (st >> 1) + 8 * h;
-				return { { load8(ql), load8(ql + 16), load8(ql + 32), load8(ql + 48) }, { load8(qh), load8(qh + 16) } };
+				return { { load8(ql, 0), load8(ql, 16), load8(ql, 32), load8(ql, 48) }, { load8(qh, 0), load8(qh, 16) } };
 			}
 			// quarter i = 2 (st % 2) + t / 2 of the half, elements 16 (t % 2) + 8 h .. of its 32
 			static __device__ __forceinline__ half8 frag(const Head&, const Raw& r, int st, int t)
@@ -255,11 +290,10 @@ namespace litenn_hip
 			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.d); }
 		};
 
-		// 16-byte pieces of a row's chunk: from the 16-byte boundary at or below it.  Rows are whole blocks apart from
-		// an address of any alignment, so a chunk may begin up to 14 bytes behind its first piece.  The slot's
-		// rows are a multiple of 16 bytes but not of 32 apart: 32 lanes then read over 64 banks two to a bank.
+		// 16-byte pieces of a row's chunk, the last one moved back so that it ends with the chunk.  The rows of a slot are a
+		// multiple of 16 bytes but not of 32 apart: 32 lanes then read over 64 banks two to a bank.
 		template <typename F>
-		constexpr int slot_pieces() { return (F::kChunkBytes + 14 + 15) / 16; }
+		constexpr int slot_pieces() { return (F::kChunkBytes + 15) / 16; }
 		template <typename F>
 		constexpr int slot_stride() { return 16 * (slot_pieces<F>() | 1); }
 
@@ -462,6 +496,78 @@ namespace litenn_hip
 			}
 		}
 
+		// A wavefront's share of the weights on their way: the raw blocks of 32 NG rows for one chunk, from memory (where
+		// they lie on 2 bytes) to the wavefront's slot in LDS (where a row's chunk begins on 16).  The P pieces of a row fall
+		// into groups of 16, 8, 4, 2 and 1 (the bits of P); a load takes one group of as many rows as there are lanes for, so
+		// that a lane's place in the row stays the same from load to load and its addresses are one sum.  Nothing behind
+		// the matrix is fetched: rows behind the last are the last, and a row's chunk that is not whole comes element
+		// by element, its missing part being the row's last two bytes.
+		template <typename F, int NG>
+		struct WeightPieces
+		{
+			static constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>(), kRows = NG * kTile;
+			static constexpr int loads_of(int width) { return (P & width) != 0 ? (kRows * width + 63) / 64 : 0; }
+			static constexpr int kLoads = loads_of(16) + loads_of(8) + loads_of(4) + loads_of(2) + loads_of(1);
+			static constexpr int kSlotBytes = kRows * kStride;
+			static_assert(P < 32, "pieces");
+			// (addresses of the global segment: a load through a generic pointer counts as an LDS access too, and every
+			// wait for LDS would wait for it)
+			typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+			typedef const __attribute__((address_space(1))) uint8_t* global_bytes_t;
+			typedef const __attribute__((address_space(1))) u32x4_a2* global_u32x4_t;
+			typedef const __attribute__((address_space(1))) uint16_t* global_u16_t;
+			global_bytes_t base; // the first row
+			int row_bytes, rows_left;
+			uint8_t* slot;
+
+			__device__ __forceinline__ WeightPieces(uint8_t* slot_, const uint8_t* w, int n_base, int n, size_t row_bytes_)
+			    : base((global_bytes_t)(w + static_cast<size_t>(min(n_base, n - 1)) * row_bytes_)), row_bytes(static_cast<int>(row_bytes_)),
+			      rows_left(max(n - n_base, 1)), slot(slot_)
+			{
+			}
+			// calls f(load, lane's row, lane's piece)
+			template <typename Fn>
+			static __device__ __forceinline__ void each(int lane, Fn f)
+			{
+				int load = 0, first = 0;
+#pragma unroll
+				for (int width = 16; width >= 1; width /= 2)
+				{
+#pragma unroll
+					for (int i = 0; i < loads_of(width); ++i)
+					{
+						f(load++, (i * (64 / width) + lane / width) % kRows, first + lane % width);
+					}
+					first += P & width;
+				}
+			}
+			__device__ __forceinline__ void request(u32x4 (&moving)[kLoads], int c, int lane) const
+			{
+				const int from = c * F::kChunkBytes;
+				if (F::kBlock < kChunk && from + F::kChunkBytes > row_bytes)
+				{
+					each(lane, [&](int i, int row, int piece) {
+#pragma unroll
+						for (int e = 0; e < 8; ++e)
+						{
+							const global_u16_t at = (global_u16_t)(base + min(row, rows_left - 1) * row_bytes + min(from + 16 * piece + 2 * e, row_bytes - 2));
+							moving[i][e / 2] = e % 2 == 0 ? *at : moving[i][e / 2] | static_cast<uint32_t>(*at) << 16;
+						}
+					});
+					return;
+				}
+				each(lane, [&](int i, int row, int piece) {
+					moving[i] = *(global_u32x4_t)(base + min(row, rows_left - 1) * row_bytes + (from + min(16 * piece, F::kChunkBytes - 16)));
+				});
+			}
+			__device__ __forceinline__ void deposit(const u32x4 (&moving)[kLoads], int lane) const
+			{
+				each(lane, [&](int i, int row, int piece) { *reinterpret_cast<u32x4*>(slot + row * kStride + 16 * piece) = moving[i]; });
+			}
+			// the lane's row of group q in the slot
+			__device__ __forceinline__ lds_bytes_t chunk(int q, int lane) const { return (lds_bytes_t)(slot) + (kTile * q + (lane & 31)) * kStride; }
+		};
+
 		// A wavefront multiplies NG groups of 32 weight rows by MT tiles of 32 activation rows over one of KS
 		// ranges of K; the KS sums meet in LDS at the end, added in K order.  Two levels of sums, a chunk's and
 		// the range's, keep the rounding of long rows down.  WN wavefronts side by side share the activation
@@ -477,9 +583,7 @@ namespace litenn_hip
 			constexpr bool kShared = WN > 1;
 			constexpr int kPieces = kShared ? MT * 8 / WN : 1; // 1 KB pieces a wavefront stages
 			static_assert(!kShared || kPieces * WN == MT * 8, "activation pieces / wavefront split");
-			constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>();
-			constexpr int kRowPieces = NG * kTile * P;
-			constexpr int kWLoads = (kRowPieces + 63) / 64;
+			typedef WeightPieces<F, NG> W;
 			constexpr int kRingBytes = kShared ? KS * 2 * MT * kStageBytes : 0;
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
 			int grid_x, grid_y;
@@ -498,56 +602,8 @@ namespace litenn_hip
 			const int per = (chunks + KS - 1) / KS;
 			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
 
-			// ---- weights: piece i of this lane is piece (64 i + lane) % P of row (64 i + lane) / P; the last pieces of a
-			// partial chunk, and of an aligned one, lie behind the row: they fetch the row's last piece again
-			uint8_t* const slot = lds + kRingBytes + wave * (NG * kTile * kStride);
-			// (addresses of the global segment: a load through a generic pointer counts as an LDS access too, and every
-			// wait for LDS would wait for it)
-			typedef const __attribute__((address_space(1))) uint8_t* global_bytes_t;
-			typedef const __attribute__((address_space(1))) u32x4* global_u32x4_t;
-			global_bytes_t piece_row[kWLoads]; // the 16-byte boundary at or below the row's start
-			int piece_at[kWLoads], piece_last[kWLoads], piece_slot[kWLoads];
-#pragma unroll
-			for (int i = 0; i < kWLoads; ++i)
-			{
-				const int id = min(64 * i + lane, kRowPieces - 1), row = id / P;
-				const uintptr_t start = reinterpret_cast<uintptr_t>(w) + static_cast<size_t>(min(n_base + row, n - 1)) * row_bytes;
-				const int mis = static_cast<int>(start & 15);
-				piece_row[i] = (global_bytes_t)(start - mis);
-				piece_at[i] = mis; // byte offset of the chunk's start from the row's first piece, plus piece offset below
-				piece_last[i] = static_cast<int>((mis + row_bytes - 1) & ~size_t{ 15 });
-				piece_slot[i] = row * kStride + 16 * (id - row * P);
-			}
-			u32x4 moving[kWLoads];
-			const auto request_w = [&](int c) {
-#pragma unroll
-				for (int i = 0; i < kWLoads; ++i)
-				{
-					const int id = min(64 * i + lane, kRowPieces - 1);
-					const int at = min(((piece_at[i] + c * F::kChunkBytes) & ~15) + 16 * (id % P), piece_last[i]);
-					moving[i] = *(global_u32x4_t)(piece_row[i] + at);
-				}
-			};
-			const auto deposit_w = [&]() {
-#pragma unroll
-				for (int i = 0; i < kWLoads; ++i)
-				{
-					if (64 * (i + 1) <= kRowPieces || 64 * i + lane < kRowPieces)
-					{
-						*reinterpret_cast<u32x4*>(slot + piece_slot[i]) = moving[i];
-					}
-				}
-			};
-			int row_mis[NG];
-#pragma unroll
-			for (int q = 0; q < NG; ++q)
-			{
-				const size_t start = reinterpret_cast<uintptr_t>(w) + static_cast<size_t>(min(n_base + kTile * q + r, n - 1)) * row_bytes;
-				row_mis[q] = static_cast<int>(start & 15);
-			}
-			const auto lane_chunk = [&](int q, int c) {
-				return (lds_bytes_t)(slot) + (kTile * q + r) * kStride + ((row_mis[q] + c * F::kChunkBytes) & 15);
-			};
+			const W weights(lds + kRingBytes + wave * W::kSlotBytes, w, n_base, n, row_bytes);
+			u32x4 moving[W::kLoads];
 
 			const RowsLayout at(m_tiles, chunks);
 			const uint8_t* tiles[MT]; // this lane's 16 bytes of the tile's first fragment
@@ -560,7 +616,7 @@ namespace litenn_hip
 				sum_tiles[t] = xs + at.sums + tile * chunks * kFrag + lane * 16;
 			}
 
-			floatx16 acc[NG][MT], p[NG][MT];
+			floatx16 acc[NG][MT], p[NG][MT], first[F::kMins ? NG : 1][MT]; // first: of the chunk's first half, where kScaleSteps is 16
 #pragma unroll
 			for (int q = 0; q < NG; ++q)
 			{
@@ -608,7 +664,7 @@ namespace litenn_hip
 			half8 sum_frag[MT];
 			if (c_begin < c_end)
 			{
-				request_w(c_begin);
+				weights.request(moving, c_begin, lane);
 				if constexpr (kShared)
 				{
 					request(staged[0], c_begin, 0);
@@ -622,7 +678,7 @@ namespace litenn_hip
 						fetch_direct(c_begin, 0, s);
 					}
 				}
-				deposit_w();
+				weights.deposit(moving, lane);
 				if constexpr (kShared)
 				{
 					deposit(staged[0], 0);
@@ -643,11 +699,11 @@ namespace litenn_hip
 				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
 				if (live)
 				{
-					request_w(next);
+					weights.request(moving, next, lane);
 #pragma unroll
 					for (int q = 0; q < NG; ++q)
 					{
-						head[q] = F::head(lane_chunk(q, c), h);
+						head[q] = F::head(weights.chunk(q, lane), h);
 					}
 					if constexpr (F::kMins)
 					{
@@ -667,7 +723,7 @@ namespace litenn_hip
 #pragma unroll
 						for (int q = 0; q < NG; ++q)
 						{
-							raw[q] = F::load(lane_chunk(q, c), st, h, blocks);
+							raw[q] = F::load(weights.chunk(q, lane), st, h, blocks);
 						}
 						if constexpr (kShared)
 						{
@@ -683,7 +739,7 @@ namespace litenn_hip
 								b[q] = F::frag(head[q], raw[q], st, s);
 							}
 							const int step = 4 * st + s;
-							const bool fresh = step % F::kScaleSteps == 0;
+							const bool fresh = step % min(F::kScaleSteps, 8) == 0;
 #pragma unroll
 							for (int t = 0; t < MT; ++t)
 							{
@@ -711,6 +767,21 @@ namespace litenn_hip
 							if constexpr (!kShared)
 							{
 								fetch_direct(st < 3 ? c : next, (st + 1) & 3, s);
+							}
+							if constexpr (F::kMins)
+							{
+								if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
+								{
+#pragma unroll
+									for (int q = 0; q < NG; ++q)
+									{
+#pragma unroll
+										for (int t = 0; t < MT; ++t)
+										{
+											first[q][t] = p[q][t];
+										}
+									}
+								}
 							}
 							if constexpr (F::kScaleSteps < 16)
 							{
@@ -750,6 +821,15 @@ namespace litenn_hip
 					for (int q = 0; q < NG; ++q)
 					{
 						const float d = F::chunk_scale(head[q]);
+						if constexpr (F::kMins)
+						{
+							const half8 b = F::centre_frag(head[q]);
+#pragma unroll
+							for (int t = 0; t < MT; ++t)
+							{
+								p[q][t] = first[q][t] + __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, p[q][t], 0, 0, 0);
+							}
+						}
 #pragma unroll
 						for (int t = 0; t < MT; ++t)
 						{
@@ -775,7 +855,7 @@ namespace litenn_hip
 							}
 						}
 					}
-					deposit_w(); // (the wavefront's own reads of the slot are behind it in its instruction stream)
+					weights.deposit(moving, lane); // (the wavefront's own reads of the slot are behind it in its instruction stream)
 				}
 			}
 
@@ -861,6 +941,252 @@ namespace litenn_hip
 			}
 		}
 
+		// ---- few rows: up to MR activation rows, one launch, no scratch ---------------------------------
+		// A workgroup takes 32 weight rows; its KS wavefronts take ranges of K and meet in LDS at the end.  Each takes
+		// the activations apart by itself, a chunk of 256 at a time and with a power of two per chunk and row: a
+		// lane holds four neighbouring elements of every row, and the parts go to fragments in the wavefront's LDS.
+		// Rows 0 .. MR - 1 of a fragment are the high parts, 16 .. 16 + MR - 1 the low ones, so that one product forms both;
+		// their sums lie in one lane (elements e and e + 8 of the result).  Bound by a wavefront's chain per chunk (blocks
+		// and activations into LDS, 16 products); a row more costs its preparation, 32 instructions.  us against the streaming
+		// kernel once per row: Q8_0 4096 x 4096 at 3 rows 10.9 / 18.2, Q4_K 14336 x 4096 at 4 rows 15.8 / 31.1, Q6_K 4096 x
+		// 14336 at 7 rows 33 / 90.
+		template <int MR>
+		struct FewRows
+		{
+			static constexpr int kPart = MR * 16, kHalf = 2 * kPart + 16; // bytes of a step's part, of eight elements' parts (16: 64 banks)
+			static constexpr int kSums = 32 * kHalf;                      // sub-block sums: [hi, lo][row][8 halves]
+			static constexpr int kUnused = kSums + 2 * kPart; // what lanes with nothing to write write
+			static constexpr int kBytes = kUnused + 256;
+			static constexpr int kValues = MR > 8 ? 8 : 4; // results of a lane
+		};
+
+		template <typename F, int MR, int KS>
+		__global__ __launch_bounds__(64 * KS, 2) void exact_few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, float* y,
+		                                                            const float* residual, int n, int k, int m, int chunks, size_t row_bytes)
+		{
+			typedef FewRows<MR> R;
+			typedef WeightPieces<F, 1> W;
+			constexpr int NE = R::kValues;
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][slot, fragments]; later the KS sums
+			const int lane = threadIdx.x & 63;
+			const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int r = lane & 31, h = lane >> 5;
+			const int n_base = blockIdx.x * kTile;
+			const int per = (chunks + KS - 1) / KS;
+			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
+			uint8_t* const mine = lds + part * (W::kSlotBytes + R::kBytes);
+			uint8_t* const frags = mine + W::kSlotBytes;
+			const W weights(mine, w, n_base, n, row_bytes);
+
+			// (nothing here may hang on a branch or look at what it loads: the next chunk's loads would be waited for at once)
+			floatx4 xv[MR];
+			const float* rows[MR];
+#pragma unroll
+			for (int i = 0; i < MR; ++i)
+			{
+				rows[i] = x + static_cast<size_t>(min(i, m - 1)) * k;
+			}
+			const auto request_x = [&](int c) {
+				const int at = min(c * kChunk + 4 * lane, k - 4);
+#pragma unroll
+				for (int i = 0; i < MR; ++i)
+				{
+					xv[i] = *reinterpret_cast<const floatx4_a4*>(rows[i] + at);
+				}
+			};
+			float unscale[MR];
+			// lane l holds elements 4 l .. 4 l + 3: step l / 4, half l / 2 % 2, first or second four of its eight
+			uint8_t* const frag_to = frags + (lane >> 1) * R::kHalf + (lane & 1) * 8;
+			// the sub-block sum of lanes 8 j .. 8 j + 7 is lane 8 j's to write, the others' go nowhere
+			const int sum_at = (lane & 7) == 0 ? R::kSums + (lane >> 3) * 2 : R::kUnused + lane * 4;
+			const int sum_row = (lane & 7) == 0 ? 16 : 0, sum_low = (lane & 7) == 0 ? R::kPart : 2;
+			const auto deposit_x = [&](int c) {
+				const bool there = F::kBlock == kChunk || c * kChunk + 4 * lane < k;
+#pragma unroll
+				for (int i = 0; i < MR; ++i)
+				{
+					float v[4];
+#pragma unroll
+					for (int e = 0; e < 4; ++e)
+					{
+						v[e] = there ? xv[i][e] : 0.0f;
+					}
+					// Times 2^shift the largest is in [2^14, 2^15); the inverse stays a normal number.  (An infinity, or a NaN
+					// aside from it, leaves the row's results infinite or NaN whatever becomes of the chunk's other elements.)
+					const float mx = wave_max_nonnegative(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+					const int shift = min(141 - static_cast<int>(static_cast<uint32_t>(__float_as_int(mx)) >> 23), 126);
+					const float scale = __int_as_float((127 + shift) << 23);
+					unscale[i] = __int_as_float((127 - shift) << 23);
+					half4 hi, lo;
+					float sum = 0.0f;
+#pragma unroll
+					for (int e = 0; e < 4; ++e)
+					{
+						v[e] *= scale;
+						hi[e] = static_cast<_Float16>(v[e]);
+						lo[e] = static_cast<_Float16>(fmaxf(v[e] - static_cast<float>(hi[e]), -16.0f)); // (inf - inf: any number will do)
+						sum += v[e];
+					}
+					*reinterpret_cast<half4*>(frag_to + 16 * i) = hi;
+					*reinterpret_cast<half4*>(frag_to + R::kPart + 16 * i) = lo;
+					if constexpr (F::kMins)
+					{
+						// eight neighbouring lanes hold one sub-block of 32 elements
+						sum += dpp_f32<0xB1>(sum);
+						sum += dpp_f32<0x4E>(sum);
+						sum += dpp_f32<0x141>(sum);
+						const float s = sum * kSumScale;
+						const _Float16 high = static_cast<_Float16>(s);
+						*reinterpret_cast<_Float16*>(frags + sum_at + sum_row * i) = high;
+						*reinterpret_cast<_Float16*>(frags + sum_at + sum_row * i + sum_low) = static_cast<_Float16>(fmaxf(s - static_cast<float>(high), -16.0f));
+					}
+				}
+			};
+			const uint8_t* const frag_from = frags + h * R::kHalf + (r >> 4) * R::kPart + min(r & 15, m - 1) * 16;
+			const uint8_t* const sums_from = frags + R::kSums + h * R::kPart + min(r & 15, m - 1) * 16;
+
+			float acc[NE];
+#pragma unroll
+			for (int e = 0; e < NE; ++e)
+			{
+				acc[e] = 0.0f;
+			}
+			u32x4 moving[2][W::kLoads]; // the next two chunks
+			if (c_begin < c_end)
+			{
+				weights.request(moving[0], c_begin, lane);
+				request_x(c_begin);
+				weights.request(moving[1], min(c_begin + 1, c_end - 1), lane);
+			}
+			const auto step = [&](int c, u32x4 (&arrived)[W::kLoads]) {
+				weights.deposit(arrived, lane);
+				deposit_x(c);
+				request_x(min(c + 1, c_end - 1));
+				weights.request(arrived, min(c + 2, c_end - 1), lane);
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
+				lds_bytes_t const chunk = weights.chunk(0, lane);
+				const typename F::Head head = F::head(chunk, h);
+				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
+				floatx16 p;
+				half8 sums;
+				float sum[NE];
+#pragma unroll
+				for (int st = 0; st < 4; ++st)
+				{
+					const typename F::Raw raw = F::load(chunk, st, h, blocks);
+#pragma unroll
+					for (int s = 0; s < 4; ++s)
+					{
+						const int at = 4 * st + s;
+						const half8 a = *reinterpret_cast<const half8*>(frag_from + 2 * at * R::kHalf);
+						p = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, F::frag(head, raw, st, s), at % min(F::kScaleSteps, 4) == 0 ? floatx16{} : p, 0, 0, 0);
+						if constexpr (F::kMins)
+						{
+							if (s == 3)
+							{
+								if (st == 3)
+								{
+									sums = r < 16 ? *reinterpret_cast<const half8*>(sums_from) : half8{}; // (into the high parts' rows alone)
+									p = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, F::centre_frag(head), p, 0, 0, 0);
+								}
+#pragma unroll
+								for (int e = 0; e < NE; ++e)
+								{
+									sum[e] = st == 0 ? p[e] + p[e + 8] : sum[e] + (p[e] + p[e + 8]);
+								}
+							}
+						}
+						if constexpr (F::kScaleSteps < 16)
+						{
+							if (at % F::kScaleSteps == F::kScaleSteps - 1)
+							{
+								const float d = F::scale(head, raw, st, s);
+#pragma unroll
+								for (int e = 0; e < NE; ++e)
+								{
+									sum[e] = at == F::kScaleSteps - 1 ? d * (p[e] + p[e + 8]) : fmaf(d, p[e] + p[e + 8], sum[e]);
+								}
+							}
+						}
+						if constexpr (F::kScaleSteps < 16)
+						{
+							// (the stage's sums now and not later: all stages' products at once are more than the registers hold)
+							if (s == 3)
+							{
+#pragma unroll
+								for (int e = 0; e < NE; ++e)
+								{
+									asm volatile("" : "+v"(sum[e]));
+								}
+							}
+						}
+					}
+				}
+				const float d = F::chunk_scale(head);
+				if constexpr (F::kMins)
+				{
+					const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, F::min_frag(head), floatx16{}, 0, 0, 0);
+					const float dm = F::min_scale(head) * (1.0f / kSumScale);
+#pragma unroll
+					for (int e = 0; e < NE; ++e)
+					{
+						sum[e] = fmaf(dm, s[e], d * sum[e]);
+					}
+				}
+				else
+				{
+#pragma unroll
+					for (int e = 0; e < NE; ++e)
+					{
+						sum[e] = d * sum[e];
+					}
+				}
+				// lane (r, h) holds weight row r and activation rows 8 (e / 4) + 4 h + e % 4
+#pragma unroll
+				for (int e = 0; e < NE; ++e)
+				{
+					const int row = 8 * (e / 4) + (e & 3);
+					acc[e] = fmaf(sum[e], h ? unscale[row + 4 < MR ? row + 4 : 0] : unscale[row < MR ? row : 0], acc[e]);
+				}
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			};
+			for (int c = c_begin; c < c_end; c += 2)
+			{
+				step(c, moving[0]);
+				if (c + 1 < c_end)
+				{
+					step(c + 1, moving[1]);
+				}
+			}
+			__syncthreads();
+			float* const handed = reinterpret_cast<float*>(lds); // [KS][activation row][weight row]
+#pragma unroll
+			for (int e = 0; e < NE; ++e)
+			{
+				const int row = 8 * (e / 4) + 4 * h + (e & 3);
+				if (row < m)
+				{
+					handed[(part * MR + row) * kTile + r] = acc[e];
+				}
+			}
+			__syncthreads();
+			for (int i = threadIdx.x; i < m * kTile; i += 64 * KS)
+			{
+				const int row = i / kTile, col = n_base + i % kTile;
+				float v = handed[i];
+#pragma unroll
+				for (int p = 1; p < KS; ++p)
+				{
+					v += handed[p * MR * kTile + i];
+				}
+				if (col < n)
+				{
+					const size_t o = static_cast<size_t>(row) * n + col;
+					y[o] = residual ? residual[o] + v : v;
+				}
+			}
+		}
+
 		struct ExactCall
 		{
 			int count;
@@ -879,7 +1205,7 @@ namespace litenn_hip
 		void launch_variant(const ExactCall& c)
 		{
 			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * 2 * MT * kStageBytes : 0) +
-			                         static_cast<size_t>(WN) * KS * NG * kTile * slot_stride<F>();
+			                         static_cast<size_t>(WN) * KS * WeightPieces<F, NG>::kSlotBytes;
 			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * NG * MT * 64 * 64;
 			constexpr size_t lds = rings > sums ? rings : sums;
 			static_assert(lds <= 160 * 1024, "LDS");
@@ -908,7 +1234,7 @@ namespace litenn_hip
 		{
 			const int strips = (c.total_rows + kTile - 1) / kTile, units = strips * c.m_tiles;
 			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each
-			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 234 against 301 of the
+			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 262 against 301 of the
 			// forms below, at 64 rows 53 against 62.  Not for Q6_K, whose scaling per step wants the registers.
 			if (F::kScaleSteps > 1 && (strips + 3) / 4 * ((c.m_tiles + 1) / 2) >= 200 && c.m_tiles > 1)
 			{
@@ -932,6 +1258,57 @@ namespace litenn_hip
 				launch_variant<F, 1, 1, 1, 4>(c);
 			}
 		}
+
+		struct FewCall
+		{
+			const uint8_t* w;
+			const float* x;
+			float* y;
+			const float* residual;
+			int n, k, m, chunks;
+			size_t row_bytes;
+			hipStream_t stream;
+		};
+
+		template <typename F, int MR, int KS>
+		void launch_few(const FewCall& c)
+		{
+			constexpr size_t tiles = static_cast<size_t>(KS) * (WeightPieces<F, 1>::kSlotBytes + FewRows<MR>::kBytes);
+			constexpr size_t sums = static_cast<size_t>(KS) * MR * kTile * sizeof(float);
+			constexpr size_t lds = tiles > sums ? tiles : sums;
+			static_assert(lds <= 160 * 1024, "LDS");
+			allow_dynamic_lds(reinterpret_cast<const void*>(&exact_few_kernel<F, MR, KS>), lds);
+			exact_few_kernel<F, MR, KS><<<dim3((c.n + kTile - 1) / kTile), dim3(64 * KS), lds, c.stream>>>(
+			    c.w, c.x, c.y, c.residual, c.n, c.k, c.m, c.chunks, c.row_bytes);
+		}
+
+		template <typename F, int MR>
+		void launch_few_rows(const FewCall& c)
+		{
+			// Eight ranges of K where 8192 weight rows and fewer leave CUs idle, else four (us at 3 rows: Q8_0 4096 x 4096 10.9
+			// with eight, 11.8 with four; Q6_K 4096 x 14336 24.7 and 30.2; Q4_0 11008 x 4096 16.4 and 14.3).
+			if (c.n <= 8192 && c.chunks >= 8)
+			{
+				launch_few<F, MR, 8>(c);
+			}
+			else
+			{
+				launch_few<F, MR, 4>(c);
+			}
+		}
+
+		template <typename F>
+		void launch_few_format(const FewCall& c)
+		{
+			switch (c.m)
+			{
+			case 1: case 2: launch_few_rows<F, 2>(c); break;
+			case 3: launch_few_rows<F, 3>(c); break;
+			case 4: launch_few_rows<F, 4>(c); break;
+			case 5: case 6: launch_few_rows<F, 6>(c); break;
+			default: launch_few_rows<F, 8>(c); break;
+			}
+		}
 	} // namespace
 
 	// bytes of scratch the rows of an m x k activation matrix take
@@ -949,7 +1326,7 @@ namespace litenn_hip
 		case LITENN_FMT_Q4_0: case LITENN_FMT_Q8_0: case LITENN_FMT_Q4_K: case LITENN_FMT_Q5_K: case LITENN_FMT_Q6_K: break;
 		default: return false;
 		}
-		return n > 0 && n <= 0x3fffffffu && row_bytes(fmt, k) != 0 && reinterpret_cast<uintptr_t>(wq) % 2 == 0;
+		return n > 0 && n <= 0x3fffffffu && row_bytes(fmt, k) != 0 && row_bytes(fmt, k) < (size_t{ 1 } << 25) && reinterpret_cast<uintptr_t>(wq) % 2 == 0;
 	}
 
 	// Takes the rows of X' = x, RMSNorm(x) * norm_w or silu(x) * up apart into `scratch` (exact_scratch_bytes,
@@ -1001,5 +1378,27 @@ namespace litenn_hip
 		case LITENN_FMT_Q5_K: launch_exact_format<Q5_KX>(c); break;
 		default: launch_exact_format<Q6_KX>(c); break;
 		}
+	}
+
+	// Y[M, N] = X . deq(W)^T (+ residual, which may alias y) for at most 8 rows, a matrix that exact_gemm_takes.
+	// Returns false, launching nothing, for more.
+	bool launch_exact_few(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y, const float* residual,
+	                      hipStream_t stream)
+	{
+		if (m == 0 || m > 8 || k < 4)
+		{
+			return false;
+		}
+		const FewCall c{ static_cast<const uint8_t*>(wq), x, y, residual, static_cast<int>(n), static_cast<int>(k), static_cast<int>(m),
+			             static_cast<int>((k + kChunk - 1) / kChunk), row_bytes(fmt, k), stream };
+		switch (fmt)
+		{
+		case LITENN_FMT_Q4_0: launch_few_format<Q4_0X>(c); break;
+		case LITENN_FMT_Q8_0: launch_few_format<Q8_0X>(c); break;
+		case LITENN_FMT_Q4_K: launch_few_format<Q4_KX>(c); break;
+		case LITENN_FMT_Q5_K: launch_few_format<Q5_KX>(c); break;
+		default: launch_few_format<Q6_KX>(c); break;
+		}
+		return true;
 	}
 } // namespace litenn_hip

@@ -60,6 +60,48 @@ def test_non_finite_and_tiny_activations(hip, fmt):
     assert np.array_equal(got[4:], clean[4:])
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("n,k", [(33, 256), (1, 2048), (70, 2304), (64, 768), (8200, 2048), (500, 4096)])
+@pytest.mark.parametrize("m", [2, 3, 4, 5, 6, 7, 8])
+def test_few_rows(hip, fmt, m, n, k):
+    assert errors(hip, fmt, m, n, k, residual=m % 2 == 0).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt", [Q4_0, Q8_0])
+@pytest.mark.parametrize("m,n,k", [(2, 17, 32), (4, 33, 288), (7, 40, 1056), (3, 70, 2080)])
+def test_few_rows_that_end_inside_a_chunk(hip, fmt, m, n, k):
+    assert errors(hip, fmt, m, n, k).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+def test_few_rows_with_non_finite_and_tiny_activations(hip, fmt):
+    m, n, k = 6, 70, 768
+    wq = synth.model_weights(fmt, n, k, 5, 1)
+    x = synth.activations(m, k, 6, 1)
+    w, t = hip.Tensor.from_numpy(wq), hip.Tensor.from_numpy
+    clean = hip.mul_mat_q(fmt, w, n, k, t(x), flags=MATMUL_PRECISE).numpy()
+    x[0, 3], x[1, 9], x[2], x[3] = np.inf, np.nan, 0.0, x[3] * np.float32(1e-42)
+    got = hip.mul_mat_q(fmt, w, n, k, t(x), flags=MATMUL_PRECISE).numpy()
+    assert not np.any(np.isfinite(got[0])) and np.all(np.isnan(got[1])) and np.all(got[2] == 0.0)
+    assert np.all(np.abs(got[3]) <= 1e-38)
+    assert np.array_equal(got[4:], clean[4:])
+
+
+@pytest.mark.parametrize("fmt,m", [(Q8_0, 3), (Q4_K, 5), (Q6_K, 2)])
+def test_few_rows_at_addresses_of_least_alignment(hip, fmt, m):
+    """Weights on 2 bytes, activations on 4, each the end of its allocation."""
+    n, k = 37, 512
+    wq, x = synth.model_weights(fmt, n, k, 5, 3), synth.activations(m, k, 6, 3)
+    want = hip.mul_mat_q(fmt, hip.Tensor.from_numpy(wq), n, k, hip.Tensor.from_numpy(x), flags=MATMUL_PRECISE).numpy()
+    from litenn_amd import _lib
+    w = hip.Tensor.from_numpy(np.concatenate([np.zeros(2, np.uint8), wq.reshape(-1)]))
+    xt = hip.Tensor.from_numpy(np.concatenate([np.zeros(1, np.float32), x.reshape(-1)]))
+    y = hip.Tensor.from_numpy(np.full((m, n), np.nan, np.float32))
+    at = lambda t, o: (t.ptr.value if hasattr(t.ptr, "value") else t.ptr) + o
+    _lib.check(_lib.load().litenn_hip_mul_mat_q(0, fmt, at(w, 2), n, k, at(xt, 4), 0, m, y.ptr, None, MATMUL_PRECISE, None))
+    assert np.array_equal(y.numpy(), want)
+
+
 def test_a_workspace_that_holds_the_rows_is_used_and_a_smaller_one_is_enough(hip):
     """The same bits out of the pool's memory and a caller's; with less room the rows go through the streaming kernel."""
     import ctypes as C
