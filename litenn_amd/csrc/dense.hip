@@ -794,8 +794,9 @@ namespace litenn_hip
 		const auto work = [&](int bm, int bn) { return tiles(a, bm, bn) * a.splits; };
 		if (a.f32)
 		{
-			// width 2048 at 500 rows: ff 11264 rows 109 -> 100 (one group), 2048 rows 50 -> 39 (two)
-			if (a.m > 32 && work(64, 128) >= 384)
+			// width 2048 at 500 rows: ff 11264 rows 109 -> 100 (one group), 2048 rows 50 -> 39 (two); 288 workgroups of one group
+			// 59, of two, which have a CU to themselves, 69
+			if (a.m > 32 && work(64, 128) > 256)
 			{
 				launch_tile<64, 128, 2, 2, 1, true>(args, s);
 			}
@@ -812,21 +813,29 @@ namespace litenn_hip
 		{
 			launch_tile<128, 128, 2, 2, 1, false>(args, s);
 		}
-		else if (a.m > 64 && work(128, 64) >= 384) // 28672 x 4096 at 100 rows 75 -> 65
+		else if (a.m > 64 && (work(128, 64) >= 384 || (a.splits == 1 && work(128, 64) > 256))) // 28672 x 4096 at 100 rows 75 -> 65
 		{
 			launch_tile<128, 64, 2, 2, 1, false>(args, s);
 		}
-		else if (a.m > 64 && work(128, 64) >= 192 && steps >= 48) // 2048 x 5632 at 777 rows 49 -> 42; 5632 x 1024 at 300 rows 13 -> 21
+		// (a workgroup of two groups has a CU to itself: 2048 x 5632 at 777 rows, 224 of them, 49 -> 42, at 1254 rows, 320, 66 -> 77;
+		// 5632 x 1024 at 300 rows 13 -> 21)
+		else if (a.m > 64 && work(128, 64) >= 192 && steps >= 48)
 		{
 			launch_tile<128, 64, 2, 2, 2, false>(args, s);
 		}
-		else if (a.m > 32 && work(64, 64) >= 384) // 5632 x 1024 at 300 rows 16 -> 13
+		else if (a.m > 32 && work(64, 64) > 288) // 5632 x 1024 at 300 rows 16 -> 13; of 320 workgroups 11.7 with one group, 12.6 with two
 		{
 			launch_tile<64, 64, 2, 2, 1, false>(args, s);
 		}
 		else if (a.m > 32 && work(64, 64) >= 192) // 6144 x 4096 at 100 rows 29 (one group) -> 23
 		{
 			launch_tile<64, 64, 2, 2, 2, false>(args, s);
+		}
+		// short walks have nothing to share, long ones run at the memory's rate (32000 x 1024, 2048, 4096 at one row: one group 15, 33, 54,
+		// two 16, 28, 56)
+		else if (work(32, 64) > 384 && (steps <= 16 || steps >= 64))
+		{
+			launch_tile<32, 64, 1, 4, 1, false>(args, s);
 		}
 		else // 4096 x 1536 at 100 rows 12 -> 9, width 2048 at 30 rows 149 -> 123 for all products
 		{
