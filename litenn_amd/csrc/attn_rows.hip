@@ -13,8 +13,7 @@
 //     by 2^14) are two halves each, hi + lo: two products per operand pair.
 //   * Float32 keys, values, queries and weights are three bfloat16 values each, which carry their 24 bits; the
 //     six products whose terms reach 2^-24 are formed.
-// Scores, softmax and sums are Float32 as in the row kernels.  Long prompts whose caller allows Float16 operands take the
-// same kernel with queries and weights rounded once (RoundedOperands; csrc/attn_tile.hip has the rule).
+// Scores, softmax and sums are Float32 as in the row kernels.
 //
 // A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
 // a SIMD (250 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
@@ -57,7 +56,6 @@ namespace litenn_hip
 		{
 			typedef half8 frag;
 			typedef uint16_t stored;
-			static constexpr bool kExact = true;
 			static constexpr int kStored = 1, kSplit = 2, kProducts = 2; // pieces of a key or value, of a query or weight
 			static constexpr int stored_of[2] = { 0, 0 }, split_of[2] = { 0, 1 };
 			static constexpr float kWeightScale = 16384.0f;
@@ -71,25 +69,10 @@ namespace litenn_hip
 				return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 			}
 		};
-		struct RoundedOperands // the same with queries and weights rounded to halves once
-		{
-			typedef half8 frag;
-			typedef uint16_t stored;
-			static constexpr bool kExact = false;
-			static constexpr int kStored = 1, kSplit = 1, kProducts = 1;
-			static constexpr int stored_of[1] = { 0 }, split_of[1] = { 0 };
-			static constexpr float kWeightScale = 16384.0f;
-			static __device__ __forceinline__ void split(float v, int e, frag (&out)[1]) { out[0][e] = static_cast<_Float16>(v); }
-			static __device__ __forceinline__ floatx16 multiply(frag a, frag b, floatx16 c)
-			{
-				return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-			}
-		};
 		struct FloatOperands
 		{
 			typedef bf16x8 frag;
 			typedef float stored;
-			static constexpr bool kExact = true;
 			static constexpr int kStored = 3, kSplit = 3, kProducts = 6;
 			static constexpr int stored_of[6] = { 0, 0, 1, 1, 0, 2 }, split_of[6] = { 0, 1, 0, 1, 2, 0 };
 			static constexpr float kWeightScale = 1.0f;
@@ -157,7 +140,6 @@ namespace litenn_hip
 			const auto sees_from = [&](int i) { return static_cast<int>(max(0ll, q_at + i - a.window + 1)); };
 			const auto sees_to = [&](int i) { return a.causal ? static_cast<int>(min(static_cast<long long>(keys), q_at + i + 1)) : keys; };
 			const int lo = sees_from(row_c), hi = sees_to(row_c);
-			const int wave_lo = sees_from(min(q_first + 32 * qw + 31, a.rows - 1)), wave_hi = sees_to(min(q_first + 32 * qw, a.rows - 1));
 			const int first = sees_from(q_first), last = sees_to(min(q_first + 32 * QW, a.rows) - 1);
 			const int tiles = (last - first + kKeys - 1) / kKeys;
 			const int steps = (tiles + KW - 1) / KW;
@@ -202,7 +184,7 @@ namespace litenn_hip
 					}
 				}
 				int shift = 0;
-				if constexpr (O::kStored == 1)
+				if constexpr (O::kSplit == 2)
 				{
 					mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
 					shift = mx > 0.0f ? min(8 - ilogbf(mx), 126) : 0;
@@ -234,9 +216,6 @@ namespace litenn_hip
 			const float slope = a.mask && a.max_bias > 0.0 ? static_cast<float>(row_alibi_slope(head, a.heads, a.max_bias)) : 1.0f;
 			const float* const mask_row = a.mask ? a.mask + static_cast<size_t>(row_c) * keys : nullptr;
 
-			// (rounded operands have no options, and take the maximum and the weights in powers of two)
-			const auto exp_of = [](float d) { return O::kExact ? exp_f32(d) : __builtin_amdgcn_exp2f(d); };
-			const float scale2 = a.scale * 1.44269502f * unscale;
 			// a dot product's score (the causal mask and the window aside)
 			const auto score_of = [&](float v, float mv) {
 				if (a.apply_scale)
@@ -360,7 +339,7 @@ namespace litenn_hip
 				const int base = first + min(tile, tiles - 1) * kKeys;
 				// the tile's mask: four runs of four keys (at the mask's end the last whole run there is, shifted below)
 				float mask[16];
-				if (O::kExact && a.mask)
+				if (a.mask)
 				{
 #pragma unroll
 					for (int e = 0; e < 16; e += 4)
@@ -412,33 +391,23 @@ namespace litenn_hip
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
 				{
-					sc[e] = O::kExact ? score_of(s[e] * unscale, mask[e]) : s[e] * scale2;
-				}
-				if (!live || base < wave_lo || base + kKeys > wave_hi) // some key is not everyone's to see
-				{
-#pragma unroll
-					for (int e = 0; e < 16; ++e)
-					{
-						const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
-						sc[e] = live && key >= lo && key < hi ? sc[e] : -INFINITY;
-					}
-				}
-#pragma unroll
-				for (int e = 0; e < 16; ++e)
-				{
+					const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
+					const bool visible = live && key >= lo && key < hi;
+					const float v = score_of(s[e] * unscale, mask[e]);
+					sc[e] = visible ? v : -INFINITY;
 					top = fmaxf(top, sc[e]);
 				}
 				top = fmaxf(top, __shfl_xor(top, 32, 64));
 				const float new_m = fmaxf(run_m, top);
 				const float ref_m = new_m == -INFINITY ? 0.0f : new_m; // (no visible key yet: every exponent is -inf)
-				const float corr = exp_of(run_m - ref_m);
+				const float corr = exp_f32(run_m - ref_m);
 				run_m = new_m;
 				float sum = 0.0f;
 				frag w[2][O::kSplit];
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
 				{
-					const float p = exp_of(sc[e] - ref_m);
+					const float p = exp_f32(sc[e] - ref_m);
 					sum += p;
 					O::split(p * O::kWeightScale, e & 7, w[e >> 3]);
 				}
@@ -515,7 +484,7 @@ namespace litenn_hip
 					const float* src = xch + (other * QW + qw) * kWaveFloats;
 					const float other_m = src[D / 2 * 64 + lane], other_l = src[(D / 2 + 1) * 64 + lane];
 					const float all_m = fmaxf(run_m, other_m), ref_m = all_m == -INFINITY ? 0.0f : all_m;
-					const float w0 = exp_of(run_m - ref_m), w1 = exp_of(other_m - ref_m);
+					const float w0 = exp_f32(run_m - ref_m), w1 = exp_f32(other_m - ref_m);
 					run_m = all_m;
 					run_l = run_l * w0 + other_l * w1;
 #pragma unroll
@@ -643,15 +612,8 @@ namespace litenn_hip
 		}
 
 		template <int D>
-		void launch_dim(const RowsAttn& a, bool f32, hipStream_t s, bool rounded)
+		void launch_dim(const RowsAttn& a, bool f32, hipStream_t s)
 		{
-			if (rounded)
-			{
-				// wavefronts that share their keys: here the key's loads count (us with the host's part, 1024 rows on 2048 keys, 32
-				// heads: two by two 115, alone by four 130, two by four 121, four by two 123)
-				launch_form<RoundedOperands, D, 2, 2>(a, s);
-				return;
-			}
 			if (f32)
 			{
 				launch_form<FloatOperands, D, 2, 2>(a, s);
@@ -674,12 +636,11 @@ namespace litenn_hip
 		}
 	} // namespace
 
-	// Causal attention of m rows at positions past .. past + m - 1 (operands as in launch_attn_decode); `rounded`: queries
-	// and weights may be rounded to halves
+	// Causal attention of m rows at positions past .. past + m - 1 (operands as in launch_attn_decode)
 	bool launch_attn_rows_causal(const float* q, const void* kcache, const void* vcache, int cache_dtype, size_t m,
-	                             size_t past, size_t n_head, size_t n_kv_head, size_t head_dim, float* out, hipStream_t s, bool rounded)
+	                             size_t past, size_t n_head, size_t n_kv_head, size_t head_dim, float* out, hipStream_t s)
 	{
-		if ((!rounded && !attn_rows_pays(m, past + m, cache_dtype == LITENN_F32)) || m > 0x3fffffffu || n_head > 65535 || past + m > 0x3fffffffu)
+		if (!attn_rows_pays(m, past + m, cache_dtype == LITENN_F32) || m > 0x3fffffffu || n_head > 65535 || past + m > 0x3fffffffu)
 		{
 			return false;
 		}
@@ -699,12 +660,11 @@ namespace litenn_hip
 		a.apply_scale = true;
 		a.scale = static_cast<float>(1.0 / sqrt(static_cast<double>(head_dim)));
 		a.out = out;
-		return launch_attn_rows(a, cache_dtype == LITENN_F32, s, rounded);
+		return launch_attn_rows(a, cache_dtype == LITENN_F32, s);
 	}
 
-	bool launch_attn_rows(const RowsAttn& a, bool f32, hipStream_t s, bool rounded)
+	bool launch_attn_rows(const RowsAttn& a, bool f32, hipStream_t s)
 	{
-		rounded = rounded && !f32 && !a.mask && !a.sinks && a.softcap == 0.0f && a.apply_scale;
 		const auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
 		const int piece = f32 ? 4 : 8; // elements of 16 bytes
 		if (a.rows <= 0 || a.heads <= 0 || a.dim % 8 != 0 || a.vdim % 8 != 0 || a.dim <= 0 || a.vdim <= 0 || a.dim > 128 || a.vdim > 128 ||
@@ -715,11 +675,11 @@ namespace litenn_hip
 		}
 		if (a.dim <= 64 && a.vdim <= 64)
 		{
-			launch_dim<64>(a, f32, s, rounded);
+			launch_dim<64>(a, f32, s);
 		}
 		else
 		{
-			launch_dim<128>(a, f32, s, rounded);
+			launch_dim<128>(a, f32, s);
 		}
 		return true;
 	}

@@ -39,8 +39,8 @@ namespace litenn_hip
 	inline bool attn_rows_pays(size_t rows, size_t keys, bool f32) { return rows >= (f32 ? 16u : 8u) && keys >= 96; }
 
 	// Returns false, launching nothing, for shapes it does not take: head sizes that are no multiple of 8 or above 128,
-	// rows that are not whole 16-byte pieces.  `rounded`: queries and weights may be rounded to halves (no options, Float16 keys).
-	bool launch_attn_rows(const RowsAttn& a, bool f32, hipStream_t s, bool rounded = false);
+	// rows that are not whole 16-byte pieces.
+	bool launch_attn_rows(const RowsAttn& a, bool f32, hipStream_t s);
 	bool launch_attn_rows_causal(const float* q, const void* kcache, const void* vcache, int cache_dtype, size_t m,
-	                             size_t past, size_t n_head, size_t n_kv_head, size_t head_dim, float* out, hipStream_t s, bool rounded = false);
+	                             size_t past, size_t n_head, size_t n_kv_head, size_t head_dim, float* out, hipStream_t s);
 } // namespace litenn_hip

@@ -26,7 +26,6 @@
 #include <cstdint>
 
 #include "common.hpp"
-#include "attn_rows.hpp"
 #include "fetch_model.hpp"
 
 namespace litenn_hip
@@ -300,15 +299,6 @@ namespace litenn_hip
 		    !aligned(out))
 		{
 			return false;
-		}
-		// Where 64 rows of a head give half the CUs a workgroup, the 32 x 32 tiles of csrc/attn_rows.hip take them, twice the
-		// products per byte of LDS (us with the host's part: 1024 rows on 2048 keys, 32 heads 149 -> 115, 2048 on 2048 182 -> 137,
-		// 512 on 512 104 -> 73, 1500 on 1600 with 8 heads 97 -> 88; 128 on 128 65 -> 65, 16 on 2016 66 -> 81).  They want the
-		// position on the host, where every call of several rows has it.
-		if (!past_dev && m >= 256 && n_head * ((m + 63) / 64) >= 128 &&
-		    launch_attn_rows_causal(q, kcache, vcache, cache_dtype, m, past_host, n_head, n_kv_head, head_dim, out, s, true))
-		{
-			return true;
 		}
 		const size_t q_tiles = (m + kQTile - 1) / kQTile;
 		if (q_tiles > 65535)
