@@ -16,11 +16,12 @@
 // Scores, softmax and sums are Float32 as in the row kernels.
 //
 // A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
-// a SIMD (250 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
+// a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
 // where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
-// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) take 30 us, with mask, slopes, soft cap and sinks 35,
-// where the row kernel took 1365; one wavefront a SIMD, two of them sharing their keys, took 46 and 59.  Against 64
-// bits 3.8e-7, as before.  Float32 keys and values (three times the products, one wavefront a SIMD): 89 and 101 us.
+// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 35 us, where
+// the row kernel took 1365.  Against 64 bits it is as close (3.8e-7; 150 rows on 700 keys 2.1e-7 and 2.0e-7): the parts'
+// small products have a sum of their own and outputs take one addition per tile, which costs 4 us here and brings
+// Float32 keys from 4.7e-7 to 2.1e-7.  Float32 keys and values (three times the products, one wavefront a SIMD): 98 us.
 #include "common.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
@@ -365,7 +366,7 @@ namespace litenn_hip
 					}
 				}
 				meet(); // the tile's keys are there, the previous tile's values have been used
-				floatx16 s = {};
+				floatx16 s = {}, s_low = {}; // the parts' small products apart: every addition to the large sum rounds
 #pragma unroll
 				for (int st = 0; st < D / 16; ++st)
 				{
@@ -373,13 +374,14 @@ namespace litenn_hip
 					for (int p = 0; p < O::kProducts; ++p)
 					{
 						const frag kf = *reinterpret_cast<const frag*>(k_lds + O::stored_of[p] * kTileBytes + j * RS + 16 * key_slot<D>(j, 2 * st + h));
+						floatx16& to = p == 0 ? s : s_low;
 						if constexpr (kQueriesInLds)
 						{
-							s = O::multiply(kf, p == 0 ? q[st][0] : *reinterpret_cast<const frag*>(q_lds + 1024 * st), s);
+							to = O::multiply(kf, p == 0 ? q[st][0] : *reinterpret_cast<const frag*>(q_lds + 1024 * st), to);
 						}
 						else
 						{
-							s = O::multiply(kf, q[st][O::split_of[p]], s);
+							to = O::multiply(kf, q[st][O::split_of[p]], to);
 						}
 					}
 				}
@@ -393,7 +395,7 @@ namespace litenn_hip
 				{
 					const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
 					const bool visible = live && key >= lo && key < hi;
-					const float v = score_of(s[e] * unscale, mask[e]);
+					const float v = score_of((s[e] + s_low[e]) * unscale, mask[e]);
 					sc[e] = visible ? v : -INFINITY;
 					top = fmaxf(top, sc[e]);
 				}
@@ -412,14 +414,6 @@ namespace litenn_hip
 					O::split(p * O::kWeightScale, e & 7, w[e >> 3]);
 				}
 				run_l = fmaf(run_l, corr, sum);
-				if (__builtin_amdgcn_ballot_w64(corr != 1.0f) != 0)
-				{
-#pragma unroll
-					for (int b = 0; b < D / 32; ++b)
-					{
-						o[b] *= corr;
-					}
-				}
 				// step u: keys 16 u + 4 h + 0..3 and 16 u + 8 + 4 h + 0..3.  Sixteen lanes read four keys' rows of
 				// sixteen dimensions, eight bytes each, and get the four keys of one dimension
 				meet(); // the tile's values are there, its keys have been used
@@ -427,10 +421,11 @@ namespace litenn_hip
 				request(vr, v_piece, ldv, tile_at(step + 1));
 				const int v_row = 4 * h + ((lane & 15) >> 2), v_col = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), v_byte = (lane & 1) * 8;
 #pragma unroll
-				for (int u = 0; u < 2; ++u)
+				for (int b = 0; b < D / 32; ++b)
 				{
+					floatx16 t = {}; // the tile's sum, added at once: the running sum rounds once per tile
 #pragma unroll
-					for (int b = 0; b < D / 32; ++b)
+					for (int u = 0; u < 2; ++u)
 					{
 						frag vf[O::kStored];
 #pragma unroll
@@ -446,8 +441,13 @@ namespace litenn_hip
 #pragma unroll
 						for (int p = 0; p < O::kProducts; ++p)
 						{
-							o[b] = O::multiply(vf[O::stored_of[p]], w[u][O::split_of[p]], o[b]);
+							t = O::multiply(vf[O::stored_of[p]], w[u][O::split_of[p]], t);
 						}
+					}
+#pragma unroll
+					for (int e = 0; e < 16; ++e)
+					{
+						o[b][e] = fmaf(o[b][e], corr, t[e]);
 					}
 				}
 			}
