@@ -6,6 +6,7 @@
 // Float32.  The reference has no counterpart (its linears are f32 MatMul nodes,
 // src/LiteNN/Layer/Linear.h:67-95).
 #include "dense.hpp"
+#include "fetch_model.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -491,11 +492,7 @@ namespace litenn_hip
 			const int wm = wave / WN, wn = wave % WN;
 			const int m0 = tm * BM, n0 = tn * BN;
 			const int k = d.w.k;
-			// this group's share of K, and the steps every group makes
-			const int all_steps = d.w.pitch / kTileK, parts = d.splits * KG, part = static_cast<int>(blockIdx.y) * KG + group;
-			const int first_step = all_steps * part / parts;
-			const int steps = all_steps * (part + 1) / parts - first_step;
-			const int rounds = (all_steps + parts - 1) / parts;
+			const fetch::DenseWalk walk = fetch::dense_walk(d.w.pitch / kTileK, d.splits, KG, static_cast<int>(blockIdx.y), group);
 
 			const int ch = tid & 7, row = tid >> 3; // this thread's piece column and first row
 			const operand* xp[LA];
@@ -632,35 +629,33 @@ namespace litenn_hip
 			};
 			// past the last tile it is requested and staged again: a branch around the loads would make every
 			// wait behind it a wait for all of them
-			// (a group without a step walks on its neighbour's first one and multiplies nothing)
-			const auto at = [&](int step) { return min(first_step + max(0, min(step, steps - 1)), all_steps - 1); };
-			request(at(0), 0);
-			request(at(1), 1);
-			stage(at(0), 0);
+			request(walk.tile(0), 0);
+			request(walk.tile(1), 1);
+			stage(walk.tile(0), 0);
 			__syncthreads();
 			// tile `step` is in LDS buffer `set`, tile step + 1 in the other register set
 			const auto advance = [&](int step, int set) {
-				request(at(step + 2), set);
+				request(walk.tile(step + 2), set);
 				if constexpr (BM * BN < 128 * 128 && !F32)
 				{
 					// on their way before the products, not behind them (the largest tile, whose products take
 					// longer than the loads, runs better scheduled freely)
 					__builtin_amdgcn_sched_barrier(0);
 				}
-				if (KG == 1 || step < steps)
+				if (KG == 1 || walk.multiplies(step))
 				{
 					multiply(set);
 				}
-				stage(at(step + 1), set ^ 1);
+				stage(walk.tile(step + 1), set ^ 1);
 				__syncthreads();
 			};
 			int step = 0;
-			for (; step + 1 < rounds; step += 2)
+			for (; step + 1 < walk.rounds; step += 2)
 			{
 				advance(step, 0);
 				advance(step + 1, 1);
 			}
-			if (step < rounds)
+			if (step < walk.rounds)
 			{
 				advance(step, 0);
 			}

@@ -25,6 +25,24 @@ namespace litenn_hip
 		LITENN_FETCH_FN int imin(int a, int b) { return a < b ? a : b; }
 		LITENN_FETCH_FN int imax(int a, int b) { return a > b ? a : b; }
 
+		// ---- products over bfloat16 weights: the K tiles of a group of wavefronts ----------------
+		// K is cut into `ranges` times `groups` parts, in order, that differ by a tile at most; the groups of a
+		// workgroup take neighbouring ones.  They pass one set of barriers, so all of them go through as many
+		// rounds as the longest part has tiles, multiplying only in their own; a group by itself makes its own.
+		struct DenseWalk
+		{
+			int first, steps, rounds, all;
+			LITENN_FETCH_FN bool multiplies(int round) const { return round < steps; }
+			// the tile of a round that is requested and staged (in rounds that multiply nothing, one that is there)
+			LITENN_FETCH_FN int tile(int round) const { return imin(first + imax(0, imin(round, steps - 1)), all - 1); }
+		};
+		LITENN_FETCH_FN DenseWalk dense_walk(int all, int ranges, int groups, int range, int group)
+		{
+			const int parts = ranges * groups, part = range * groups + group;
+			const int first = all * part / parts, steps = all * (part + 1) / parts - first;
+			return { first, steps, groups == 1 ? steps : (all + parts - 1) / parts, all };
+		}
+
 		// ---- matrix-core GEMM: raw weight blocks of one 256-element chunk per row --------------
 		// A wavefront owns 16 * ng consecutive rows; their chunks land in its LDS slot row after row
 		// as `pieces` 16-byte pieces each.  Formats whose chunks start on 16-byte boundaries take

@@ -629,8 +629,51 @@ static void test_gemm_chunk_ranges()
 	std::printf("tiled GEMM K ranges: %ld chunks walked\n", walked);
 }
 
+// Products over bfloat16 weights: whatever the ranges of K and the groups of wavefronts, every tile of K is
+// multiplied once, the groups of a workgroup make equally many rounds, and only tiles that are there are requested
+// (up to six rounds past the last).
+static void test_dense_walks()
+{
+	using namespace litenn_hip::fetch;
+	long walked = 0;
+	for (int all = 1; all <= 300; ++all)
+	{
+		for (int ranges = 1; ranges <= 4; ++ranges)
+		{
+			for (int groups = 1; groups <= 3; ++groups)
+			{
+				std::vector<int> times(all, 0);
+				for (int range = 0; range < ranges; ++range)
+				{
+					for (int group = 0; group < groups; ++group)
+					{
+						const DenseWalk w = dense_walk(all, ranges, groups, range, group);
+						CHECK(w.rounds == dense_walk(all, ranges, groups, range, 0).rounds, "%d tiles, %d ranges of %d groups", all, ranges, groups);
+						for (int round = 0; round < w.rounds + 6; ++round)
+						{
+							const int tile = w.tile(round);
+							CHECK(tile >= 0 && tile < all, "%d tiles, %d ranges of %d groups: tile %d", all, ranges, groups, tile);
+							if (round < w.rounds && w.multiplies(round))
+							{
+								++times[tile];
+								++walked;
+							}
+						}
+					}
+				}
+				for (int tile = 0; tile < all; ++tile)
+				{
+					CHECK(times[tile] == 1, "%d tiles, %d ranges of %d groups: tile %d %d times", all, ranges, groups, tile, times[tile]);
+				}
+			}
+		}
+	}
+	std::printf("bfloat16 products: %ld tiles of K walked\n", walked);
+}
+
 int main()
 {
+	test_dense_walks();
 	test_gemm_chunk_ranges();
 	test_gemm_weight_pieces();
 	test_gemm_stream_pieces();

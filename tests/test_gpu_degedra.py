@@ -96,6 +96,17 @@ def test_each_mechanism_alone(hip, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [150, 300, 350])
+def test_last_products_in_ranges_of_k(hip, rows, dtype):
+    """The sums over K of 5632 (88 tiles) in four, three and, at 350 rows, three ranges: 22 tiles each, or 29, 29 and 30."""
+    cfg = du.config([du.layer(du.attention(8, 2, 64, 100, 0.125, 64), du.state_space(4, 32, 16, 1, 1, 3), ff=5632)], width=2048)
+    model, plain = pair(hip, cfg, 21, dtype)
+    toks = du.tokens(cfg, rows, 5)
+    assert du.error(model.eval(toks), plain.forward(toks)) <= LIMIT[dtype]
+    model.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("width", [6, 53, 64, 200])
 def test_embedding_norms_and_head(hip, width, dtype):
     """Sublayers whose output norm is zero leave the embedding, the last norm and the capped head."""
