@@ -341,8 +341,8 @@ namespace litenn_hip
 		}
 
 		// ------------------------------------------------------------------
-		// Many rows: BM activation rows x BN weight rows per group of four wavefronts, bfloat16 operands (Float32 ones:
-		// below), K in tiles of 64 double-buffered in LDS (global -> registers two tiles ahead -> LDS
+		// Many rows: BM activation rows x BN weight rows per workgroup, bfloat16 operands (Float32 ones:
+		// below), K in tiles of 64 double-buffered in LDS (global -> registers tiles ahead -> LDS
 		// while the previous tile is multiplied), v_mfma_f32_16x16x32_bf16 with the weights as the A operand, so that a lane
 		// ends up with four consecutive outputs of one activation row.  The 16-byte pieces of a 128-byte
 		// LDS row are permuted by the row's low three bits: the 16 rows a fragment read touches then fall
@@ -466,19 +466,26 @@ namespace litenn_hip
 		// pair give what one of Float32 operands gives, at 48 cycles per 32 elements of K where v_mfma_f32_16x16x4_f32
 		// takes 256.  The activations are taken apart on their way into LDS.
 		//
-		// KG groups of four wavefronts share the tile and cut its K walk into as many ranges, each through buffers of its
-		// own; their sums meet in LDS at the end, in K order.  A step of one group alone is a chain of latencies
-		// (request, LDS, barrier, products that feed each other): with few tiles the ranges fill the SIMDs.
-		template <int BM, int BN, int WM, int WN, int KG, bool F32>
-		__global__ __launch_bounds__(256 * KG) void dense_tile_kernel(const TileArgs args)
+		// Two wavefronts a SIMD hide most of a step's chain of latencies (request, LDS, barrier, products that feed each other):
+		// eight of them on 128 x 128 take 49 us for 2048 x 5632 at 1254 rows, four 70.  S tiles of K travel at any time.
+		// Every output is one chain of products over K in order whatever the form, so that bfloat16 results hang on
+		// the ranges of K alone.
+		//
+		// KG (Float32 operands only): groups of WM x WN wavefronts share the tile and cut its K walk into as many ranges,
+		// each through buffers of its own; their sums meet in LDS at the end, in K order.
+		template <int BM, int BN, int WM, int WN, int KG, int S, bool F32>
+		__global__ __launch_bounds__(64 * WM * WN * KG) void dense_tile_kernel(const TileArgs args)
 		{
-			static_assert(WM * WN == 4, "four wavefronts");
+			constexpr int T = 64 * WM * WN, kRowStep = T / 8; // threads of a group, rows they stage at once
 			constexpr int P = F32 ? 3 : 1; // parts of an activation
 			typedef std::conditional_t<F32, float, uint16_t> operand;
 			constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
-			constexpr int LA = BM / 32, LW = BN / 32; // 16-byte pieces a thread stages per K tile
+			constexpr int LA = BM / kRowStep, LW = BN / kRowStep; // 16-byte pieces a thread stages per K tile
+			static_assert(KG == 1 || F32, "one chain of products over K");
+			static_assert(S % 2 == 0, "register sets and LDS buffers alternate together");
+			static_assert(LA * kRowStep == BM && LW * kRowStep == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile");
 			extern __shared__ __attribute__((aligned(16))) uint16_t tile_lds[]; // per group: activations [2][P][BM][64], weights [2][BN][64]
-			const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+			const int group = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / T);
 			uint16_t* const xs = tile_lds + group * (2 * kTileK * (P * BM + BN));
 			uint16_t* const ws = xs + 2 * P * BM * kTileK;
 			const DenseRows& d = args.d;
@@ -487,7 +494,7 @@ namespace litenn_hip
 			{
 				return;
 			}
-			const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+			const int tid = threadIdx.x & (T - 1), lane = tid & 63, wave = tid >> 6;
 			const int j = lane & 15, g = lane >> 4;
 			const int wm = wave / WN, wn = wave % WN;
 			const int m0 = tm * BM, n0 = tn * BN;
@@ -500,16 +507,16 @@ namespace litenn_hip
 #pragma unroll
 			for (int i = 0; i < LA; ++i)
 			{
-				xp[i] = static_cast<const operand*>(d.a) + static_cast<size_t>(operand_row(d, m0 + row + 32 * i)) * d.lda + ch * 8;
+				xp[i] = static_cast<const operand*>(d.a) + static_cast<size_t>(operand_row(d, m0 + row + kRowStep * i)) * d.lda + ch * 8;
 			}
 #pragma unroll
 			for (int i = 0; i < LW; ++i)
 			{
-				wp[i] = d.w.w + static_cast<size_t>(min(n0 + row + 32 * i, d.w.n - 1)) * d.w.pitch + ch * 8;
+				wp[i] = d.w.w + static_cast<size_t>(min(n0 + row + kRowStep * i, d.w.n - 1)) * d.w.pitch + ch * 8;
 			}
-			// two K tiles travel at any time: tile t in register set t & 1 until it is staged
+			// tile t of K is in register set t % S until it is staged, and then in LDS buffer t % 2
 			constexpr int kWords = F32 ? 2 : 1; // of a piece of eight activations
-			u32x4 rx[2][LA][kWords], rw[2][LW];
+			u32x4 rx[S][LA][kWords], rw[S][LW];
 			const auto request = [&](int step, int set) {
 #pragma unroll
 				for (int i = 0; i < LA; ++i)
@@ -547,7 +554,7 @@ namespace litenn_hip
 #pragma unroll
 				for (int i = 0; i < LA; ++i)
 				{
-					uint16_t* const dst = xs + set * (P * BM * kTileK) + (row + 32 * i) * kTileK + slot;
+					uint16_t* const dst = xs + (set & 1) * (P * BM * kTileK) + (row + kRowStep * i) * kTileK + slot;
 					if constexpr (F32)
 					{
 						u32x4 part[3];
@@ -577,7 +584,7 @@ namespace litenn_hip
 #pragma unroll
 				for (int i = 0; i < LW; ++i)
 				{
-					*reinterpret_cast<u32x4*>(ws + set * (BN * kTileK) + (row + 32 * i) * kTileK + slot) = rw[set][i];
+					*reinterpret_cast<u32x4*>(ws + (set & 1) * (BN * kTileK) + (row + kRowStep * i) * kTileK + slot) = rw[set][i];
 				}
 			};
 
@@ -629,13 +636,16 @@ namespace litenn_hip
 			};
 			// past the last tile it is requested and staged again: a branch around the loads would make every
 			// wait behind it a wait for all of them
-			request(walk.tile(0), 0);
-			request(walk.tile(1), 1);
+#pragma unroll
+			for (int t = 0; t < S; ++t)
+			{
+				request(walk.tile(t), t);
+			}
 			stage(walk.tile(0), 0);
 			__syncthreads();
-			// tile `step` is in LDS buffer `set`, tile step + 1 in the other register set
+			// tile `step` is in LDS, the S - 1 behind it in their register sets
 			const auto advance = [&](int step, int set) {
-				request(walk.tile(step + 2), set);
+				request(walk.tile(step + S), set);
 				if constexpr (BM * BN < 128 * 128 && !F32)
 				{
 					// on their way before the products, not behind them (the largest tile, whose products take
@@ -644,20 +654,27 @@ namespace litenn_hip
 				}
 				if (KG == 1 || walk.multiplies(step))
 				{
-					multiply(set);
+					multiply(set & 1);
 				}
-				stage(walk.tile(step + 1), set ^ 1);
+				stage(walk.tile(step + 1), (set + 1) % S);
 				__syncthreads();
 			};
 			int step = 0;
-			for (; step + 1 < walk.rounds; step += 2)
+			for (; step + S <= walk.rounds; step += S)
 			{
-				advance(step, 0);
-				advance(step + 1, 1);
+#pragma unroll
+				for (int t = 0; t < S; ++t)
+				{
+					advance(step + t, t);
+				}
 			}
-			if (step < walk.rounds)
+#pragma unroll
+			for (int t = 0; t < S - 1; ++t)
 			{
-				advance(step, 0);
+				if (step + t < walk.rounds)
+				{
+					advance(step + t, t);
+				}
 			}
 			if constexpr (KG > 1)
 			{
@@ -670,7 +687,7 @@ namespace litenn_hip
 #pragma unroll
 						for (int b = 0; b < TM; ++b)
 						{
-							handed[((group - 1) * 4 + wave) * (TN * TM * 64) + (a * TM + b) * 64 + lane] = acc[a][b];
+							handed[((group - 1) * (WM * WN) + wave) * (TN * TM * 64) + (a * TM + b) * 64 + lane] = acc[a][b];
 						}
 					}
 				}
@@ -688,7 +705,7 @@ namespace litenn_hip
 #pragma unroll
 						for (int b = 0; b < TM; ++b)
 						{
-							acc[a][b] += handed[(other * 4 + wave) * (TN * TM * 64) + (a * TM + b) * 64 + lane];
+							acc[a][b] += handed[(other * (WM * WN) + wave) * (TN * TM * 64) + (a * TM + b) * 64 + lane];
 						}
 					}
 				}
@@ -724,16 +741,16 @@ namespace litenn_hip
 			dense_row_kernel<R><<<dim3(blocks), dim3(kRowThreads), lds, s>>>(args);
 		}
 
-		template <int BM, int BN, int WM, int WN, int KG, bool F32>
+		template <int BM, int BN, int WM, int WN, int KG, int S, bool F32>
 		void launch_tile(TileArgs& args, hipStream_t s)
 		{
 			constexpr size_t lds = sizeof(uint16_t) * KG * 2 * kTileK * ((F32 ? 3 : 1) * BM + BN);
 			static_assert(lds <= 160 * 1024 && sizeof(float) * (KG - 1) * BM * BN <= lds, "LDS");
-			allow_dynamic_lds(reinterpret_cast<const void*>(&dense_tile_kernel<BM, BN, WM, WN, KG, F32>), lds);
+			allow_dynamic_lds(reinterpret_cast<const void*>(&dense_tile_kernel<BM, BN, WM, WN, KG, S, F32>), lds);
 			args.m_tiles = (args.d.m + BM - 1) / BM;
 			args.n_tiles = (args.d.w.n + BN - 1) / BN;
 			const int per = (args.m_tiles * args.n_tiles + 7) / 8;
-			dense_tile_kernel<BM, BN, WM, WN, KG, F32><<<dim3(8 * per, args.d.splits), dim3(256 * KG), lds, s>>>(args);
+			dense_tile_kernel<BM, BN, WM, WN, KG, S, F32><<<dim3(8 * per, args.d.splits), dim3(64 * WM * WN * KG), lds, s>>>(args);
 		}
 
 		int tiles(const DenseRows& d, int bm, int bn) { return ((d.m + bm - 1) / bm) * ((d.w.n + bn - 1) / bn); }
@@ -783,58 +800,50 @@ namespace litenn_hip
 			return;
 		}
 		TileArgs args{ a, 0, 0 };
-		// Tallest tile that still gives a SIMD two wavefronts, from one workgroup's groups if need be.  Figures: us, kernel
-		// alone, the next smaller choice against the one taken.
-		const int steps = a.w.pitch / kTileK / a.splits;
 		const auto work = [&](int bm, int bn) { return tiles(a, bm, bn) * a.splits; };
 		if (a.f32)
 		{
-			// width 2048 at 500 rows: ff 11264 rows 109 -> 100 (one group), 2048 rows 50 -> 39 (two); 288 workgroups of one group
-			// 59, of two, which have a CU to themselves, 69
+			// Tallest tile that still gives a SIMD two wavefronts, from one workgroup's groups if need be (us, kernel alone, the next
+			// smaller choice against the one taken): width 2048 at 500 rows: ff 11264 rows 109 -> 100 (one group), 2048 rows 50 -> 39
+			// (two); 288 workgroups of one group 59, of two, which have a CU to themselves, 69
 			if (a.m > 32 && work(64, 128) > 256)
 			{
-				launch_tile<64, 128, 2, 2, 1, true>(args, s);
+				launch_tile<64, 128, 2, 2, 1, 2, true>(args, s);
 			}
 			else if (a.m > 32 && work(64, 128) >= 192)
 			{
-				launch_tile<64, 128, 2, 2, 2, true>(args, s);
+				launch_tile<64, 128, 2, 2, 2, 2, true>(args, s);
 			}
 			else // width 2048 at 30 rows: 4096 rows 28 -> 19 against one group's 64 x 64
 			{
-				launch_tile<32, 64, 1, 4, 2, true>(args, s);
+				launch_tile<32, 64, 1, 4, 2, 2, true>(args, s);
 			}
+			return;
 		}
-		else if (a.m > 64 && tiles(a, 128, 128) >= 384) // width 2048 at 777 rows, 6432 rows 53 -> 45
+		// A K step of a form costs so many ns where a CU has r workgroups of it, fitted over 2048 x 5632, 4096 x 14336, 11264 x
+		// 2048, 6432 x 2048 and 6144 x 4096 at 30 to 1254 rows; the form with the least is the fastest of eleven, or within 5 % of
+		// it, at all of these (us for 128 x 128, 64 x 128, 64 x 64, 32 x 64: 2048 x 5632 at 777 rows 48, 40, 41, 51, at 500 rows
+		// 48, 39, 26, 32; 11264 x 2048 at 777 rows 58, 66, 75, 92, at 30 rows 23, 19, 13, 13).  The small tiles, taken where a CU
+		// has one or two, wait for memory: four tiles of K on their way instead of two make 6144 x 4096 27 -> 21 us at 100 rows,
+		// 26 -> 19 at 30.
+		const auto cost = [&](int bm, int bn, int fixed, int per) { return fixed + per * ((work(bm, bn) + 255) / 256); };
+		const int c128 = cost(128, 128, 0, 570), c64 = cost(64, 128, 60, 360), c64n = cost(64, 64, 50, 220), c32 = cost(32, 64, 60, 140);
+		const int least = std::min({ c128, c64, c64n, c32 });
+		if (c128 == least)
 		{
-			launch_tile<128, 128, 2, 2, 1, false>(args, s);
+			launch_tile<128, 128, 4, 2, 1, 2, false>(args, s);
 		}
-		else if (a.m > 64 && (work(128, 64) >= 384 || (a.splits == 1 && work(128, 64) > 256))) // 28672 x 4096 at 100 rows 75 -> 65
+		else if (c64 == least)
 		{
-			launch_tile<128, 64, 2, 2, 1, false>(args, s);
+			launch_tile<64, 128, 2, 4, 1, 2, false>(args, s);
 		}
-		// (a workgroup of two groups has a CU to itself: 2048 x 5632 at 777 rows, 224 of them, 49 -> 42, at 1254 rows, 320, 66 -> 77;
-		// 5632 x 1024 at 300 rows 13 -> 21)
-		else if (a.m > 64 && work(128, 64) >= 192 && steps >= 48)
+		else if (c64n == least)
 		{
-			launch_tile<128, 64, 2, 2, 2, false>(args, s);
+			launch_tile<64, 64, 2, 4, 1, 4, false>(args, s);
 		}
-		else if (a.m > 32 && work(64, 64) > 288) // 5632 x 1024 at 300 rows 16 -> 13; of 320 workgroups 11.7 with one group, 12.6 with two
+		else
 		{
-			launch_tile<64, 64, 2, 2, 1, false>(args, s);
-		}
-		else if (a.m > 32 && work(64, 64) >= 192) // 6144 x 4096 at 100 rows 29 (one group) -> 23
-		{
-			launch_tile<64, 64, 2, 2, 2, false>(args, s);
-		}
-		// short walks have nothing to share, long ones run at the memory's rate (32000 x 1024, 2048, 4096 at one row: one group 15, 33, 54,
-		// two 16, 28, 56)
-		else if (work(32, 64) > 384 && (steps <= 16 || steps >= 64))
-		{
-			launch_tile<32, 64, 1, 4, 1, false>(args, s);
-		}
-		else // 4096 x 1536 at 100 rows 12 -> 9, width 2048 at 30 rows 149 -> 123 for all products
-		{
-			launch_tile<32, 64, 1, 4, 2, false>(args, s);
+			launch_tile<32, 64, 1, 4, 1, 4, false>(args, s);
 		}
 	}
 } // namespace litenn_hip

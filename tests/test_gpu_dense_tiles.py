@@ -1,5 +1,5 @@
-"""Products over bfloat16 weights at the edges of the rules that pick a tile and of the K walk that two groups of
-wavefronts share (a single step of 64, odd numbers of steps, ragged K), in both operand types.
+"""Products over bfloat16 weights at the edges of the rules that pick a tile and of the K walk (a single step of 64, odd
+numbers of steps, ragged K; with Float32 operands two groups of wavefronts may share it), in both operand types.
 
 Bounds: bfloat16 operands are exact, Float32 ones are taken apart exactly, so what is left are Float32 sums of k
 products, about sqrt(log2 k) 2^-24 of |x| |W| / sqrt(k); 1e-6 is four times what is seen."""
@@ -11,9 +11,9 @@ from test_gpu_layer_ops import NAN16, NAN32, bf16_tensor, padded_bits, pitch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(49200, 64, 65), (12300, 200, 129),                    # 128 x 128, 128 x 64
-          (6210, 3100, 130), (3100, 64, 200), (3137, 192, 193),  # 128 x 64 and 64 x 64 on two groups
-          (6200, 320, 250), (12290, 100, 250),                   # Float32: 64 x 128 on two groups, on one
+SHAPES = [(49200, 64, 65), (12300, 200, 129),                    # bfloat16 128 x 128, 32 x 64; Float32 64 x 128
+          (6210, 3100, 130), (3100, 64, 200), (3137, 192, 193),  # 32 x 64, 64 x 64; 32 x 64 on two groups
+          (6200, 320, 250), (12290, 100, 250),                   # 64 x 128, 128 x 128; 64 x 128 on two groups, on one
           (40, 64, 33), (700, 1088, 40), (1030, 4096, 7)]        # 32 x 64
 
 
@@ -35,6 +35,21 @@ def test_tiles(hip, f32, n, k, m):
     got = hip.linear_bf16(bf16_tensor(hip, w), n, k, xt, m).numpy()
     size = np.linalg.norm(x.astype(np.float64), axis=1) * np.linalg.norm(wf) / np.sqrt(k)
     assert (np.linalg.norm(got - x.astype(np.float64) @ wf.T, axis=1) / size).max() <= 1e-6
+
+
+@pytest.mark.parametrize("k", [130, 300, 500])
+def test_bfloat16_rows_are_the_same_bits_in_every_form(hip, k):
+    """A row's sums run over K in one order, however many rows go with it: 128 x 128 at 500 rows, then 32 x 64, 64 x 64 and
+    64 x 128."""
+    n, rows = 5632, 500
+    rng = np.random.default_rng(k)
+    w, x = (padded_bits(rng.normal(0, 1, (r, k)).astype(np.float32)) for r in (n, rows))
+    wt = bf16_tensor(hip, w)
+    want = hip.linear_bf16(wt, n, k, bf16_tensor(hip, x), rows).numpy()
+    exact = from_bfloat16(x)[:9].astype(np.float64) @ from_bfloat16(w).astype(np.float64).T
+    assert np.linalg.norm(want[:9] - exact) <= 1e-6 * np.linalg.norm(exact)
+    for m in (20, 100, 150, 250):
+        assert np.array_equal(hip.linear_bf16(wt, n, k, bf16_tensor(hip, x[:m]), m).numpy(), want[:m]), m
 
 
 def test_float32_extremes_stay_in_their_rows(hip):
