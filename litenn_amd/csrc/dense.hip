@@ -6,7 +6,6 @@
 // Float32.  The reference has no counterpart (its linears are f32 MatMul nodes,
 // src/LiteNN/Layer/Linear.h:67-95).
 #include "dense.hpp"
-#include "fetch_model.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -756,16 +755,7 @@ namespace litenn_hip
 		int tiles(const DenseRows& d, int bm, int bn) { return ((d.m + bm - 1) / bm) * ((d.w.n + bn - 1) / bn); }
 	} // namespace
 
-	// Few tiles: K is walked in up to four ranges at once, enough for about two workgroups per CU and none
-	// shorter than 16 tiles of K.
-	int dense_rows_splits(const DenseMatrix& w, int m)
-	{
-		DenseRows d;
-		d.w = w;
-		d.m = m;
-		const int t = m <= 32 ? tiles(d, 32, 64) : tiles(d, 64, 64);
-		return std::max(1, std::min({ kDenseMaxSplits, (512 + t / 2) / t, w.pitch / kTileK / 16 }));
-	}
+	int dense_rows_splits(const DenseMatrix& w, int m) { return fetch::dense_ranges(w.n, w.pitch / kTileK, m); }
 
 	size_t dense_row_max_k() { return kRowLdsLimit / sizeof(float) / (kFlight * kRowBlock) * (kFlight * kRowBlock); }
 

@@ -3,6 +3,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "fetch_model.hpp"
 
 namespace litenn_hip
 {
@@ -77,7 +78,7 @@ namespace litenn_hip
 		ClampedGlu act;
 		float softcap = 0.0f; // kOutF32: > 0: c becomes softcap tanh(c / softcap)
 	};
-	constexpr int kDenseMaxSplits = 4;
+	constexpr int kDenseMaxSplits = fetch::kDenseMaxRanges;
 	int dense_rows_splits(const DenseMatrix& w, int m);
 	void launch_dense_rows(const DenseRows& a, hipStream_t s);
 } // namespace litenn_hip

@@ -43,6 +43,26 @@ namespace litenn_hip
 			return { first, steps, groups == 1 ? steps : (all + parts - 1) / parts, all };
 		}
 
+		// The ranges of K a sublayer's last product of m rows is walked in at once, each with sums of its own
+		// [m, ld] behind the one before: where there are few tiles, enough for about two workgroups per CU and
+		// none shorter than 16 tiles of K.
+		constexpr int kDenseMaxRanges = 4, kDenseRangedRows = 1024;
+		inline int dense_ranges(int n, int k_tiles, int m)
+		{
+			if (m > kDenseRangedRows)
+			{
+				return 1;
+			}
+			const int tiles = ((m + (m <= 32 ? 31 : 63)) / (m <= 32 ? 32 : 64)) * ((n + 63) / 64);
+			return imax(1, imin(kDenseMaxRanges, imin((512 + tiles / 2) / tiles, k_tiles / 16)));
+		}
+		// rows of sums that passes of up to `rows` rows write: a short pass in ranges may write more than a long one
+		inline size_t dense_sum_rows(size_t rows)
+		{
+			const size_t ranged = kDenseMaxRanges * (rows < kDenseRangedRows ? rows : kDenseRangedRows);
+			return rows > ranged ? rows : ranged;
+		}
+
 		// ---- matrix-core GEMM: raw weight blocks of one 256-element chunk per row --------------
 		// A wavefront owns 16 * ng consecutive rows; their chunks land in its LDS slot row after row
 		// as `pieces` 16-byte pieces each.  Formats whose chunks start on 16-byte boundaries take

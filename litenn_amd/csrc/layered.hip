@@ -31,7 +31,6 @@ namespace litenn_hip
 		constexpr int kRowsMin = 4;        // from here on a pass runs on the matrix cores
 		constexpr int kExpandMin = 16;     // from here on attention expands the cached latents
 		constexpr int kPassRows = 4096;    // most tokens of a pass (LITENN_HIP_PASS_ROWS)
-		constexpr int kSplitRows = 1024;   // up to here a sublayer's last product may walk K in several ranges at once
 		constexpr int kAlignRows = 8;      // first row of every part of a concatenated matrix
 
 		struct MixerState
@@ -585,7 +584,7 @@ namespace litenn_hip
 			struct { void** p; size_t bytes; } bufs[] = {
 				{ reinterpret_cast<void**>(&x), 4 * rows * desc.width },
 				{ reinterpret_cast<void**>(&proj), 4 * rows * ld_proj },
-				{ reinterpret_cast<void**>(&y), 4 * rows * ld_y * (rows <= kSplitRows ? kDenseMaxSplits : 1) },
+				{ reinterpret_cast<void**>(&y), 4 * fetch::dense_sum_rows(rows) * ld_y },
 				{ reinterpret_cast<void**>(&q), 4 * rows * ld_q },
 				{ reinterpret_cast<void**>(&absorbed), 4 * absorbed_floats },
 				{ reinterpret_cast<void**>(&partial), 4 * partial_floats },
@@ -965,7 +964,7 @@ namespace litenn_hip
 				d.c = y;
 				d.ldc = ld_y;
 				d.f32 = f32;
-				d.splits = parts = rows <= kSplitRows ? dense_rows_splits(w, rows) : 1;
+				d.splits = parts = dense_rows_splits(w, rows);
 				d.split_stride = part_stride;
 				launch_dense_rows(d, stream);
 				pending = after;

@@ -671,9 +671,37 @@ static void test_dense_walks()
 	std::printf("bfloat16 products: %ld tiles of K walked\n", walked);
 }
 
+// The sums of a sublayer's last product lie in a buffer made for the longest pass so far: any shorter one's, in
+// its ranges of K, must fit (widths and K of layered decoders, and small odd ones).
+static void test_dense_sum_rows()
+{
+	using namespace litenn_hip::fetch;
+	long passes = 0, ranged = 0;
+	for (int cap = 1; cap <= 4300; cap += cap < 1000 || cap > 1030 ? 37 : 1)
+	{
+		const size_t room = dense_sum_rows(cap);
+		for (int rows = 1; rows <= cap; ++rows)
+		{
+			for (int n : { 1, 50, 88, 640, 1024, 2048, 4096 })
+			{
+				for (int k : { 64, 1000, 2048, 2816, 5632, 14336 })
+				{
+					const int ranges = dense_ranges(n, (k + 63) / 64, rows);
+					CHECK(ranges >= 1 && ranges <= kDenseMaxRanges && ranges <= (k + 63) / 64 && static_cast<size_t>(ranges) * rows <= room,
+					      "%d ranges of %d rows (%d x %d) in room for %zu, made for passes of %d", ranges, rows, n, k, room, cap);
+					++passes;
+					ranged += ranges > 1;
+				}
+			}
+		}
+	}
+	std::printf("sums in ranges of K: %ld of %ld passes\n", ranged, passes);
+}
+
 int main()
 {
 	test_dense_walks();
+	test_dense_sum_rows();
 	test_gemm_chunk_ranges();
 	test_gemm_weight_pieces();
 	test_gemm_stream_pieces();

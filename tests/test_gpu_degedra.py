@@ -107,6 +107,20 @@ def test_last_products_in_ranges_of_k(hip, rows, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+def test_a_long_pass_and_then_a_shorter_one(hip, dtype):
+    """1100 tokens in one pass, then 1000, whose last products run in two ranges of K: the logits of a model that never
+    had more than 700 at once."""
+    cfg = du.config([du.layer(du.attention(4, 2, 32, 100, 0.2, 32), du.state_space(2, 32, 16, 1, 1, 3), ff=2816)], width=1024)
+    toks = du.tokens(cfg, 2100, 5)
+    logits = []
+    for cuts in ([1100, 1000], [700]):
+        model = hip.create_model(cfg, du.random_weights(cfg, 22), dtype=dtype, context_length=2100)
+        logits.append(feed(model, toks, cuts))
+        model.close()
+    assert du.error(*logits) <= LIMIT[dtype]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("width", [6, 53, 64, 200])
 def test_embedding_norms_and_head(hip, width, dtype):
     """Sublayers whose output norm is zero leave the embedding, the last norm and the capped head."""
