@@ -225,9 +225,10 @@ namespace litenn_hip
 				}
 				if (a.softcap != 0.0f)
 				{
-					// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range
-					const float ex = exp_f32(__fmul_rn(v, 2.0f));
-					v = __fmul_rn(__fsub_rn(ex, 1.0f), __builtin_amdgcn_rcpf(__fadd_rn(ex, 1.0f)));
+					// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range.  (A
+					// division: the reciprocal instruction gives 0 above 2^126, which exp reaches short of its range's end.)
+					const float ex = expf(__fmul_rn(v, 2.0f));
+					v = __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
 					if (a.apply_cap)
 					{
 						v = __fmul_rn(v, a.softcap);

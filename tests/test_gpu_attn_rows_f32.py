@@ -82,6 +82,26 @@ def test_options(hip, dtype, m, keys, heads, kv, dim, causal):
     assert worst(got, want) <= 2e-6
 
 
+@pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
+@pytest.mark.parametrize("m", [7, 40])
+def test_scores_that_saturate_the_soft_cap(hip, dtype, m):
+    """Capped scores of 43.7 to 44.3, where exp(2x) comes to the end of its range, beside small ones: tanh is 1, on
+    either side of the number of rows from which the matrix cores are used."""
+    keys, heads, dim, cap = 128, 2, 64, 20.0
+    rng = np.random.default_rng(6)
+    k = np.zeros((keys, 1, dim), np.float32)
+    k[:, 0, 0] = np.where(np.arange(keys) % 3 == 0, np.linspace(43.7, 44.3, keys), rng.uniform(0.9, 1.1, keys)).astype(np.float16)
+    k[0::2, 0, 0] *= -1
+    v = rng.standard_normal((keys, 1, dim)).astype(np.float32)
+    if dtype == DT_F16:
+        k, v = k.astype(np.float16), v.astype(np.float16)
+    q = np.zeros((m, heads, dim), np.float32)
+    q[:, :, 0] = cap
+    T = hip.Tensor.from_numpy
+    got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=1.0, logit_softcap=cap, causal=False).numpy()
+    assert worst(got, plain(*(a.astype(np.float64) for a in (q, k, v)), 1.0, 0, softcap=cap, causal=False)) <= 2e-6
+
+
 @pytest.mark.parametrize("m,keys,heads,dim,vdim,window,at", [(16, 100, 3, 24, 40, 96, 84), (50, 150, 2, 128, 64, 97, 100), (96, 96, 4, 128, 128, 200, 0)])
 def test_float32_windows(hip, m, keys, heads, dim, vdim, window, at):
     rng = np.random.default_rng(4)
