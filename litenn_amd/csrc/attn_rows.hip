@@ -9,19 +9,21 @@
 // live beside its outputs, and the weights leave the first product in the registers the second one takes (the
 // order of the keys inside a step is chosen to match; ds_read_b64_tr_b16 turns four keys' rows into the value
 // operand).  No operand is rounded to 16 bits:
-//   * Float16 keys and values are exact; a query (scaled by a power of two per row) and a softmax weight (scaled
-//     by 2^14) are two halves each, hi + lo: two products per operand pair.
-//   * Float32 keys, values, queries and weights are three bfloat16 values each, which carry their 24 bits; the
-//     six products whose terms reach 2^-24 are formed.
+//   * Float16 keys and values are exact; a query (its row scaled to 2^14) and a softmax weight (times 2^14) are two halves
+//     each, hi + lo / 4096, off by 2^-24 of itself at most down to 2^-27 of the row's largest (of a weight of 1), and by
+//     2^-51 of that below: two products per operand pair, in a sum each.
+//   * Float32 keys, values, queries and weights are three bfloat16 values each, exactly; of their nine products the three
+//     below 2^-26 of the pair's, a quarter of what a Float32 rounding takes, are left out.
 // Scores, softmax and sums are Float32 as in the row kernels.
 //
 // A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
 // a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
 // where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
-// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 35 us, where
-// the row kernel took 1365.  Against 64 bits it is as close (3.8e-7; 150 rows on 700 keys 2.1e-7 and 2.0e-7): the parts'
-// small products have a sum of their own and outputs take one addition per tile, which costs 4 us here and brings
-// Float32 keys from 4.7e-7 to 2.1e-7.  Float32 keys and values (three times the products, one wavefront a SIMD): 98 us.
+// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 42 us, where
+// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 113 us.  Sums are
+// short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
+// addition per tile, which costs 4 us and leaves the error against 64 bits below the row kernel's (mean of six inputs, 1e-7:
+// these rows 3.75 and 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
 #include "common.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
@@ -41,17 +43,6 @@ namespace litenn_hip
 
 		constexpr int kKeys = 32; // keys of a tile, queries of a wavefront
 
-		// exp(d) for d <= 0 to about two units in the last place: the product with log2 e is carried in two floats
-		__device__ __forceinline__ float exp_f32(float d)
-		{
-			constexpr float kHi = 1.44269502f, kLo = 1.92596299e-8f, kLn2 = 0.693147182f;
-			d = d < -126.0f ? -126.0f : d; // (NaN stays)
-			const float t = d * kHi;
-			const float r = fmaf(d, kLo, fmaf(d, kHi, -t));
-			const float e = __builtin_amdgcn_exp2f(t);
-			return fmaf(e, r * kLn2, e);
-		}
-
 		// How a Float32 operand is taken apart, and which products of the parts are formed
 		struct HalfOperands // keys and values as they are
 		{
@@ -59,11 +50,11 @@ namespace litenn_hip
 			typedef uint16_t stored;
 			static constexpr int kStored = 1, kSplit = 2, kProducts = 2; // pieces of a key or value, of a query or weight
 			static constexpr int stored_of[2] = { 0, 0 }, split_of[2] = { 0, 1 };
-			static constexpr float kWeightScale = 16384.0f;
+			static constexpr float kWeightScale = 16384.0f, kLowScale = 1.0f / 4096.0f;
 			static __device__ __forceinline__ void split(float v, int e, frag (&out)[2])
 			{
 				out[0][e] = static_cast<_Float16>(v);
-				out[1][e] = static_cast<_Float16>(v - static_cast<float>(out[0][e]));
+				out[1][e] = static_cast<_Float16>((v - static_cast<float>(out[0][e])) * (1.0f / kLowScale));
 			}
 			static __device__ __forceinline__ floatx16 multiply(frag a, frag b, floatx16 c)
 			{
@@ -76,7 +67,7 @@ namespace litenn_hip
 			typedef float stored;
 			static constexpr int kStored = 3, kSplit = 3, kProducts = 6;
 			static constexpr int stored_of[6] = { 0, 0, 1, 1, 0, 2 }, split_of[6] = { 0, 1, 0, 1, 2, 0 };
-			static constexpr float kWeightScale = 1.0f;
+			static constexpr float kWeightScale = 1.0f, kLowScale = 1.0f;
 			static __device__ __forceinline__ void split(float v, int e, frag (&out)[3])
 			{
 				out[0][e] = static_cast<__bf16>(v);
@@ -188,7 +179,7 @@ namespace litenn_hip
 				if constexpr (O::kSplit == 2)
 				{
 					mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-					shift = mx > 0.0f ? min(8 - ilogbf(mx), 126) : 0;
+					shift = mx > 0.0f ? min(14 - ilogbf(mx), 126) : 0;
 					unscale = ldexpf(1.0f, -shift);
 				}
 #pragma unroll
@@ -367,7 +358,7 @@ namespace litenn_hip
 					}
 				}
 				meet(); // the tile's keys are there, the previous tile's values have been used
-				floatx16 s = {}, s_low = {}; // the parts' small products apart: every addition to the large sum rounds
+				floatx16 s = {}, s_odd = {}, s_low = {}; // the parts' small products apart: every addition to a large sum rounds
 #pragma unroll
 				for (int st = 0; st < D / 16; ++st)
 				{
@@ -375,7 +366,7 @@ namespace litenn_hip
 					for (int p = 0; p < O::kProducts; ++p)
 					{
 						const frag kf = *reinterpret_cast<const frag*>(k_lds + O::stored_of[p] * kTileBytes + j * RS + 16 * key_slot<D>(j, 2 * st + h));
-						floatx16& to = p == 0 ? s : s_low;
+						floatx16& to = p > 0 ? s_low : st % 2 == 0 ? s : s_odd;
 						if constexpr (kQueriesInLds)
 						{
 							to = O::multiply(kf, p == 0 ? q[st][0] : *reinterpret_cast<const frag*>(q_lds + 1024 * st), to);
@@ -396,25 +387,34 @@ namespace litenn_hip
 				{
 					const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
 					const bool visible = live && key >= lo && key < hi;
-					const float v = score_of((s[e] + s_low[e]) * unscale, mask[e]);
+					const float v = score_of(fmaf(s_low[e], O::kLowScale, s[e] + s_odd[e]) * unscale, mask[e]);
 					sc[e] = visible ? v : -INFINITY;
 					top = fmaxf(top, sc[e]);
 				}
 				top = fmaxf(top, __shfl_xor(top, 32, 64));
 				const float new_m = fmaxf(run_m, top);
 				const float ref_m = new_m == -INFINITY ? 0.0f : new_m; // (no visible key yet: every exponent is -inf)
-				const float corr = exp_f32(run_m - ref_m);
+				const float corr = expf(run_m - ref_m);
 				run_m = new_m;
-				float sum = 0.0f;
+				float sums[16];
 				frag w[2][O::kSplit];
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
 				{
-					const float p = exp_f32(sc[e] - ref_m);
-					sum += p;
+					const float p = expf(sc[e] - ref_m);
+					sums[e] = p;
 					O::split(p * O::kWeightScale, e & 7, w[e >> 3]);
 				}
-				run_l = fmaf(run_l, corr, sum);
+#pragma unroll
+				for (int half = 8; half > 0; half /= 2)
+				{
+#pragma unroll
+					for (int e = 0; e < half; ++e)
+					{
+						sums[e] += sums[e + half];
+					}
+				}
+				run_l = fmaf(run_l, corr, sums[0]);
 				// step u: keys 16 u + 4 h + 0..3 and 16 u + 8 + 4 h + 0..3.  Sixteen lanes read four keys' rows of
 				// sixteen dimensions, eight bytes each, and get the four keys of one dimension
 				meet(); // the tile's values are there, its keys have been used
@@ -424,11 +424,16 @@ namespace litenn_hip
 #pragma unroll
 				for (int b = 0; b < D / 32; ++b)
 				{
-					floatx16 t = {}; // the tile's sum, added at once: the running sum rounds once per tile
+					if constexpr (O::kSplit == 2)
+					{
+						__builtin_amdgcn_sched_barrier(0); // (one block of dimensions after the other: four at once are more than the registers hold)
+					}
+					// the tile's sum, the small products' first, added at once: the running sum rounds once per tile
+					floatx16 t = {}, t_low = {};
+					frag vf[2][O::kStored];
 #pragma unroll
 					for (int u = 0; u < 2; ++u)
 					{
-						frag vf[O::kStored];
 #pragma unroll
 						for (int p = 0; p < O::kStored; ++p)
 						{
@@ -437,13 +442,26 @@ namespace litenn_hip
 							const uint8_t* const at = v_lds + p * kTileBytes + v_byte;
 							const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + r0 * RS + 16 * value_slot<D>(r0, 4 * b + v_col))));
 							const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + r1 * RS + 16 * value_slot<D>(r1, 4 * b + v_col))));
-							vf[p] = __builtin_bit_cast(frag, u32x4{ x.x, x.y, y.x, y.y });
+							vf[u][p] = __builtin_bit_cast(frag, u32x4{ x.x, x.y, y.x, y.y });
 						}
 #pragma unroll
-						for (int p = 0; p < O::kProducts; ++p)
+						for (int p = O::kProducts - 1; p > 0; --p)
 						{
-							t = O::multiply(vf[O::stored_of[p]], w[u][O::split_of[p]], t);
+							t_low = O::multiply(vf[u][O::stored_of[p]], w[u][O::split_of[p]], t_low);
 						}
+					}
+					if constexpr (O::kSplit == 2)
+					{
+						t = t_low * O::kLowScale; // (and the large products go on top: no registers for two sums)
+					}
+#pragma unroll
+					for (int u = 0; u < 2; ++u)
+					{
+						t = O::multiply(vf[u][0], w[u][0], t);
+					}
+					if constexpr (O::kSplit > 2)
+					{
+						t += t_low;
 					}
 #pragma unroll
 					for (int e = 0; e < 16; ++e)
@@ -485,7 +503,7 @@ namespace litenn_hip
 					const float* src = xch + (other * QW + qw) * kWaveFloats;
 					const float other_m = src[D / 2 * 64 + lane], other_l = src[(D / 2 + 1) * 64 + lane];
 					const float all_m = fmaxf(run_m, other_m), ref_m = all_m == -INFINITY ? 0.0f : all_m;
-					const float w0 = exp_f32(run_m - ref_m), w1 = exp_f32(other_m - ref_m);
+					const float w0 = expf(run_m - ref_m), w1 = expf(other_m - ref_m);
 					run_m = all_m;
 					run_l = run_l * w0 + other_l * w1;
 #pragma unroll
@@ -572,8 +590,8 @@ namespace litenn_hip
 				// the sink joins the row maximum and the denominator, not the values (FlashAttnExt.h:184-212)
 				const float sink = a.sinks[head];
 				const float all_m = fmaxf(run_m, sink);
-				weight = exp_f32(run_m - all_m);
-				total = run_l * weight + exp_f32(sink - all_m);
+				weight = expf(run_m - all_m);
+				total = run_l * weight + expf(sink - all_m);
 			}
 			const float inv = weight / total * (a.out_scale / O::kWeightScale);
 			float* const out = a.out + static_cast<size_t>(row) * a.ldo + static_cast<size_t>(head) * a.vdim;

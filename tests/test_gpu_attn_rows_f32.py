@@ -2,7 +2,7 @@
 edges of its tiles (32 queries, 32 keys, heads of 64 and 128 and sizes between), through every entry point that
 reaches it.
 
-Bound: operands keep 22 bits and more, scores, softmax and sums are Float32 as in the row kernel the suite holds to
+Bound: operands are off by 2^-24 of themselves at most, scores, softmax and sums are Float32 as in the row kernel the suite holds to
 2e-5 elsewhere; 2e-6 of a row's norm is four times what is seen."""
 import numpy as np
 import pytest
@@ -100,6 +100,30 @@ def test_scores_that_saturate_the_soft_cap(hip, dtype, m):
     T = hip.Tensor.from_numpy
     got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=1.0, logit_softcap=cap, causal=False).numpy()
     assert worst(got, plain(*(a.astype(np.float64) for a in (q, k, v)), 1.0, 0, softcap=cap, causal=False)) <= 2e-6
+
+
+@pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_operands_far_below_their_rows_largest(hip, dtype, dim):
+    """A query's small elements beside one 2^26 times as large that meets zeros, and values of keys whose weights are
+    2^-30 and 2^-36 of the largest: each counts with its own 24 bits."""
+    m, keys, heads = 40, 200, 2
+    q, k, v = inputs(7, m, keys, heads, 1, dim, DT_F32)
+    q[:, :, 5] = np.float32(2.0 ** 26)
+    k[:, :, 5] = 0.0
+    k, v = k.astype(np.float16), v.astype(np.float16)
+    T = hip.Tensor.from_numpy
+
+    def error(q, k, v):
+        k, v = (a.astype(np.float16 if dtype == DT_F16 else np.float32) for a in (k, v))
+        got = hip.attn_rows(T(q), T(k), T(v), m, keys - m, heads, 1, dim, precise=True).numpy()
+        return worst(got, plain(*(a.astype(np.float64) for a in (q, k, v)), dim ** -0.5, keys - m))
+    assert error(q, k, v) <= 2e-6
+    q[:], k[:] = 0.0, 0.0
+    q[:, :, 0] = np.sqrt(dim)
+    k[1:, 0, 0] = np.where(np.arange(keys - 1) % 2, -30 * np.log(2.0), -36 * np.log(2.0))
+    v[0], v[1:] = 1e-4 * v[0], 3e4 * np.sign(v[1:])
+    assert error(q, k, v) <= 2e-6
 
 
 @pytest.mark.parametrize("m,keys,heads,dim,vdim,window,at", [(16, 100, 3, 24, 40, 96, 84), (50, 150, 2, 128, 64, 97, 100), (96, 96, 4, 128, 128, 200, 0)])
