@@ -145,8 +145,9 @@ int litenn_hip_permute(int dev, void* dst, int dtype, const size_t* src_shape, s
  * single-row launches): weights and activations are rounded to fp16 once each (activation rows are first scaled
  * by a power of two into the fp16 range), products accumulate in f32; relative L2 error about
  * 4e-4.  LITENN_HIP_MATMUL_PRECISE in `flags` keeps f32 operands for any m: Q4_0, Q8_0, Q4_K, Q5_K and Q6_K
- * on the matrix cores (weights as exact integers, every activation as two halves that carry its Float32 digits,
- * block scales and sums in f32: the streaming GEMV's accuracy), 2 to 8 rows in one launch without scratch, more with
+ * on the matrix cores (weights as exact integers, every activation as two halves, off by 2^-24 of itself at most down to
+ * 2^-28 of its row's largest and by 2^-52 of the largest below that, block scales and sums in f32: the streaming GEMV's
+ * accuracy), 2 to 8 rows in one launch without scratch, more with
  * k <= 16384 in scratch of the device's memory pool or in a given workspace if it has 4.125 * m * k bytes and some
  * (m rounded up to 32, k to 256); without such room, and for the other formats, row by row through the GEMV, which
  * needs none.

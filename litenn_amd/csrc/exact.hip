@@ -7,9 +7,10 @@
 //     sub-scales, integer times sub-scale: at most 63 * 16 and some) are exact in binary16 and are what
 //     the matrix cores multiply; the block's Float32 scale is applied to the Float32 sum of its
 //     products.
-//   * An activation is scaled by a power of two per row and taken apart into two binary16 values, hi =
-//     half(x) and lo = half(x - hi), which together carry 22 to 24 significant bits; both are
-//     multiplied by the same integers and accumulate in the same Float32 registers.
+//   * An activation is scaled by a power of two (per row, for few rows per row and 256 elements) to at most 2^15 and
+//     taken apart into two binary16 values, hi = half(x) and lo = half(4096 (x - hi)): off by 2^-24 of itself at most down
+//     to 2^-28 of the largest, by 2^-52 of that below.  Both are multiplied by the integers, lo by the integers / 4096
+//     (exact as well), and accumulate in the same Float32 registers.
 //   * The minimum term of Q4_K and Q5_K, dmin * sum_j m_j (sum of sub-block j's activations), is one
 //     more product per 256 elements: the eight sums, taken apart the same way, against the eight
 //     six-bit minima.
@@ -20,7 +21,7 @@
 // What bounds it: few rows are the weights' stream and the launch; many rows, the LDS reads of the fragments (two
 // per pair of products) and the latency in front of them: a product issues every 100 cycles and SIMD where
 // it takes 32.  Row by row through the streaming kernel the same calls took, us, before -> now with the rows'
-// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 45; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
+// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 46.7; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
 //
 // v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
 // weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
@@ -47,6 +48,7 @@ namespace litenn_hip
 		constexpr int kStageBytes = 8 * kFrag;           // one tile, 64 elements: (hi, lo) x 4 steps
 		constexpr int kTileChunkBytes = 4 * kStageBytes; // one tile, 256 elements
 		constexpr float kSumScale = 1.0f / 64.0f; // sums of 32 activations back into the binary16 range
+		constexpr float kLowScale = 1.0f / 4096.0f; // of the low parts: small activations beside a large one keep their bits
 
 		// ---- weight blocks -> binary16 integers -------------------------------------------------------
 		// A wavefront copies the raw blocks of its 32 NG rows for one 256-element chunk into a slot of its own in
@@ -80,6 +82,11 @@ namespace litenn_hip
 		// bytes 0, 1 and 2, 3 of v as the halves 1024 + byte (0x6400 | byte)
 		__device__ __forceinline__ half2v biased01(uint32_t v) { return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)); }
 		__device__ __forceinline__ half2v biased23(uint32_t v) { return as_half2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)); }
+
+		// the factors of the low parts
+		__device__ __forceinline__ half8 lowered(half8 v) { return v * static_cast<_Float16>(kLowScale); }
+		// factors of sub-block sums: lanes (r, 0) hold those of the high parts, lanes (r, 1) of the low ones
+		__device__ __forceinline__ half8 for_sums(half8 v, int h) { return v * static_cast<_Float16>(h ? kLowScale : 1.0f); }
 
 		__device__ __forceinline__ half8 join(half2v a, half2v b, half2v c, half2v d)
 		{
@@ -440,7 +447,7 @@ namespace litenn_hip
 						const float v = ldexpf(held[u][e], shift);
 						hi[e] = static_cast<_Float16>(v);
 						const float rest = v - static_cast<float>(hi[e]);
-						lo[e] = static_cast<_Float16>(fabsf(v) <= 65504.0f ? rest : 0.0f); // (inf - inf)
+						lo[e] = static_cast<_Float16>(fabsf(v) <= 65504.0f ? rest * (1.0f / kLowScale) : 0.0f); // (inf - inf)
 						sum += static_cast<double>(v);
 					}
 					uint8_t* dst = frags + static_cast<size_t>(it >> 1) * (2 * kFrag) + (it & 1) * 512;
@@ -455,7 +462,7 @@ namespace litenn_hip
 					const float v = static_cast<float>(sum * kSumScale);
 					const _Float16 hi = static_cast<_Float16>(v);
 					const double rest = sum * kSumScale - static_cast<double>(static_cast<float>(hi));
-					const _Float16 lo = static_cast<_Float16>(fabsf(v) <= 65504.0f ? static_cast<float>(rest) : 0.0f);
+					const _Float16 lo = static_cast<_Float16>(fabsf(v) <= 65504.0f ? static_cast<float>(rest * (1.0f / kLowScale)) : 0.0f);
 					uint8_t* dst = sums + static_cast<size_t>(it >> 5) * kFrag + ((it >> 2) & 7) * 2;
 					*reinterpret_cast<_Float16*>(dst) = hi;
 					*reinterpret_cast<_Float16*>(dst + 512) = lo;
@@ -732,11 +739,12 @@ namespace litenn_hip
 #pragma unroll
 						for (int s = 0; s < 4; ++s)
 						{
-							half8 b[NG];
+							half8 b[NG], b_low[NG];
 #pragma unroll
 							for (int q = 0; q < NG; ++q)
 							{
 								b[q] = F::frag(head[q], raw[q], st, s);
+								b_low[q] = lowered(b[q]);
 							}
 							const int step = 4 * st + s;
 							const bool fresh = step % min(F::kScaleSteps, 8) == 0;
@@ -761,7 +769,7 @@ namespace litenn_hip
 								for (int q = 0; q < NG; ++q)
 								{
 									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b[q], fresh ? floatx16{} : p[q][t], 0, 0, 0);
-									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b[q], p[q][t], 0, 0, 0);
+									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b_low[q], p[q][t], 0, 0, 0);
 								}
 							}
 							if constexpr (!kShared)
@@ -823,7 +831,7 @@ namespace litenn_hip
 						const float d = F::chunk_scale(head[q]);
 						if constexpr (F::kMins)
 						{
-							const half8 b = F::centre_frag(head[q]);
+							const half8 b = for_sums(F::centre_frag(head[q]), h);
 #pragma unroll
 							for (int t = 0; t < MT; ++t)
 							{
@@ -841,7 +849,7 @@ namespace litenn_hip
 						}
 						if constexpr (F::kMins)
 						{
-							const half8 b = F::min_frag(head[q]);
+							const half8 b = for_sums(F::min_frag(head[q]), h);
 							const float dm = F::min_scale(head[q]) * (1.0f / kSumScale);
 #pragma unroll
 							for (int t = 0; t < MT; ++t)
@@ -1024,7 +1032,7 @@ namespace litenn_hip
 					{
 						v[e] *= scale;
 						hi[e] = static_cast<_Float16>(v[e]);
-						lo[e] = static_cast<_Float16>(fmaxf(v[e] - static_cast<float>(hi[e]), -16.0f)); // (inf - inf: any number will do)
+						lo[e] = static_cast<_Float16>(fmaxf((v[e] - static_cast<float>(hi[e])) * (1.0f / kLowScale), -32768.0f)); // (inf - inf: any number will do)
 						sum += v[e];
 					}
 					*reinterpret_cast<half4*>(frag_to + 16 * i) = hi;
@@ -1038,7 +1046,7 @@ namespace litenn_hip
 						const float s = sum * kSumScale;
 						const _Float16 high = static_cast<_Float16>(s);
 						*reinterpret_cast<_Float16*>(frags + sum_at + sum_row * i) = high;
-						*reinterpret_cast<_Float16*>(frags + sum_at + sum_row * i + sum_low) = static_cast<_Float16>(fmaxf(s - static_cast<float>(high), -16.0f));
+						*reinterpret_cast<_Float16*>(frags + sum_at + sum_row * i + sum_low) = static_cast<_Float16>(fmaxf((s - static_cast<float>(high)) * (1.0f / kLowScale), -32768.0f));
 					}
 				}
 			};
@@ -1087,12 +1095,13 @@ namespace litenn_hip
 								if (st == 3)
 								{
 									sums = r < 16 ? *reinterpret_cast<const half8*>(sums_from) : half8{}; // (into the high parts' rows alone)
-									p = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, F::centre_frag(head), p, 0, 0, 0);
+									p = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, for_sums(F::centre_frag(head), h), p, 0, 0, 0);
 								}
 #pragma unroll
 								for (int e = 0; e < NE; ++e)
 								{
-									sum[e] = st == 0 ? p[e] + p[e + 8] : sum[e] + (p[e] + p[e + 8]);
+									const float both = fmaf(p[e + 8], kLowScale, p[e]);
+									sum[e] = st == 0 ? both : sum[e] + both;
 								}
 							}
 						}
@@ -1104,7 +1113,8 @@ namespace litenn_hip
 #pragma unroll
 								for (int e = 0; e < NE; ++e)
 								{
-									sum[e] = at == F::kScaleSteps - 1 ? d * (p[e] + p[e + 8]) : fmaf(d, p[e] + p[e + 8], sum[e]);
+									const float both = fmaf(p[e + 8], kLowScale, p[e]);
+									sum[e] = at == F::kScaleSteps - 1 ? d * both : fmaf(d, both, sum[e]);
 								}
 							}
 						}
@@ -1125,7 +1135,7 @@ namespace litenn_hip
 				const float d = F::chunk_scale(head);
 				if constexpr (F::kMins)
 				{
-					const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, F::min_frag(head), floatx16{}, 0, 0, 0);
+					const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, for_sums(F::min_frag(head), h), floatx16{}, 0, 0, 0);
 					const float dm = F::min_scale(head) * (1.0f / kSumScale);
 #pragma unroll
 					for (int e = 0; e < NE; ++e)

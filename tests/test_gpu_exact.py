@@ -119,3 +119,27 @@ def test_a_workspace_that_holds_the_rows_is_used_and_a_smaller_one_is_enough(hip
         got = y.numpy()
         assert np.array_equal(got, want) == same
         assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(3, 70, 768), (8, 33, 256), (40, 130, 768), (300, 5200, 512)])
+def test_activations_far_below_their_rows_largest_keep_their_bits(hip, fmt, m, n, k):
+    """A sub-block of zero weights hides one large activation.  Down to 2^-28 of it an activation is off by 2^-24 of itself at
+    most, so that the bound above holds for the others."""
+    wq = synth.model_weights(fmt, n, k, 31, m).copy()
+    rows = wq.reshape(n, -1)
+    if fmt in (Q4_0, Q8_0):
+        rows[:, :2] = 0  # the first block's scale
+    elif fmt == Q6_K:
+        rows[:, 192] = 0  # the first sub-block's scale
+    else:
+        rows[:, [4, 8]] &= 0xC0  # its scale and its minimum
+    w = np_decoders.decode(fmt, wq, k).astype(np.float64)
+    assert not w[:, :16].any()
+    x = synth.activations(m, k, 32, m)
+    x[:, 0] = np.float32(2.0) ** (24 - 7 * np.arange(m) % 25).astype(np.float32)
+    got = hip.mul_mat_q(fmt, hip.Tensor.from_numpy(wq), n, k, hip.Tensor.from_numpy(x), flags=MATMUL_PRECISE).numpy()
+    rest = x.astype(np.float64)
+    rest[:, 0] = 0.0
+    size = np.linalg.norm(rest, axis=1) * np.linalg.norm(w) / np.sqrt(k)
+    assert (np.linalg.norm(got - rest @ w.T, axis=1) / size).max() <= 1e-6
