@@ -226,6 +226,11 @@ namespace litenn_hip
 			}
 			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
 			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.w.x); }
+			// element l of sub-block j
+			static __device__ __forceinline__ int code(const uint8_t* block, int j, int l)
+			{
+				return (block[16 + (j >> 1) * 32 + l] >> (4 * (j & 1))) & 15;
+			}
 			static __device__ __forceinline__ half8 min_frag(const Head& hd) { return bytes_minus(minima(hd.w, 0), minima(hd.w, 1), 0.0f); }
 			static __device__ __forceinline__ half8 centre_frag(const Head& hd) { return centres(scales(hd.w, 0), scales(hd.w, 1), kCentre); }
 			static __device__ __forceinline__ float min_scale(const Head& hd) { return -f16_bits_to_f32(hd.w.x >> 16); }
@@ -257,6 +262,10 @@ namespace litenn_hip
 			}
 			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
 			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.w.x); }
+			static __device__ __forceinline__ int code(const uint8_t* block, int j, int l)
+			{
+				return ((block[48 + (j >> 1) * 32 + l] >> (4 * (j & 1))) & 15) | ((block[16 + l] >> j) & 1) << 4;
+			}
 			static __device__ __forceinline__ half8 min_frag(const Head& hd)
 			{
 				return bytes_minus(Q4_KX::minima(hd.w, 0), Q4_KX::minima(hd.w, 1), 0.0f);
@@ -296,6 +305,36 @@ namespace litenn_hip
 			}
 			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return f16_bits_to_f32(hd.d); }
 		};
+
+		// A weight row times the activations x(k), the terms formed as the streaming kernel forms them: for results that an
+		// infinite activation leaves infinite or NaN, which centred integers would give another sign or no number.
+		template <typename F, typename X>
+		__device__ __forceinline__ float plain_dot(const uint8_t* row, int chunks, X x)
+		{
+			float total = 0.0f;
+#pragma unroll 1
+			for (int c = 0; c < chunks; ++c, row += F::kChunkBytes)
+			{
+				const float d = f16_bits_to_f32(row[0] | row[1] << 8), dmin = f16_bits_to_f32(row[2] | row[3] << 8);
+#pragma unroll 1
+				for (int j = 0; j < 8; ++j)
+				{
+					const uint8_t* const sc = row + 4;
+					const int s = j < 4 ? sc[j] & 63 : (sc[j + 4] & 15) | (sc[j - 4] >> 6) << 4;
+					const int m = j < 4 ? sc[j + 4] & 63 : sc[j + 4] >> 4 | (sc[j] >> 6) << 4;
+					float sum = 0.0f, off = 0.0f;
+#pragma unroll 1
+					for (int l = 0; l < 32; ++l)
+					{
+						const float v = x(kChunk * c + 32 * j + l);
+						sum = fmaf(static_cast<float>(F::code(row, j, l)), v, sum);
+						off += v;
+					}
+					total += d * (static_cast<float>(s) * sum) - dmin * (static_cast<float>(m) * off);
+				}
+			}
+			return total;
+		}
 
 		// 16-byte pieces of a row's chunk, the last one moved back so that it ends with the chunk.  The rows of a slot are a
 		// multiple of 16 bytes but not of 32 apart: 32 lanes then read over 64 banks two to a bank.
@@ -919,6 +958,7 @@ namespace litenn_hip
 
 			// lane (r, h) holds weight row r and activation rows 8 (e / 4) + 4 h + e % 4
 			const float* factors = reinterpret_cast<const float*>(xs + at.factors);
+			uint32_t again[NG] = {}; // results that are not finite
 #pragma unroll
 			for (int t = 0; t < MT; ++t)
 			{
@@ -936,6 +976,11 @@ namespace litenn_hip
 							if (col < n)
 							{
 								const size_t o = static_cast<size_t>(mm) * n + col;
+								if (F::kMins && !(fabsf(acc[q][t][e]) <= 3.402823466e38f))
+								{
+									again[q] |= 1u << (16 * t + e);
+									continue;
+								}
 								float v = acc[q][t][e] * us;
 								if (residual)
 								{
@@ -944,6 +989,26 @@ namespace litenn_hip
 								y[o] = v;
 							}
 						}
+					}
+				}
+			}
+			if constexpr (F::kMins)
+			{
+#pragma unroll
+				for (int q = 0; q < NG; ++q)
+				{
+					const int col = n_base + kTile * q + r;
+					while (__builtin_expect(again[q] != 0, 0))
+					{
+						const int i = __ffs(again[q]) - 1, e = i & 15, mm = (mt_base + (i >> 4)) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
+						again[q] &= again[q] - 1;
+						const uint8_t* const parts = xs + static_cast<size_t>(mm / kTile) * chunks * kTileChunkBytes + (mm % kTile) * 16;
+						const float v = factors[mm] * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
+							const uint8_t* const at = parts + static_cast<size_t>(i >> 4) * (2 * kFrag) + ((i >> 3) & 1) * 512 + (i & 7) * 2;
+							return fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(at + kFrag)), kLowScale, static_cast<float>(*reinterpret_cast<const _Float16*>(at)));
+						});
+						const size_t o = static_cast<size_t>(mm) * n + col;
+						y[o] = residual ? residual[o] + v : v;
 					}
 				}
 			}
@@ -1019,8 +1084,8 @@ namespace litenn_hip
 					{
 						v[e] = there ? xv[i][e] : 0.0f;
 					}
-					// Times 2^shift the largest is in [2^14, 2^15); the inverse stays a normal number.  (An infinity, or a NaN
-					// aside from it, leaves the row's results infinite or NaN whatever becomes of the chunk's other elements.)
+					// Times 2^shift the largest is in [2^14, 2^15); the inverse stays a normal number.  (An infinity leaves the row's
+					// results infinite or NaN whatever becomes of the chunk's other elements, a NaN has no part in the largest.)
 					const float mx = wave_max_nonnegative(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
 					const int shift = min(141 - static_cast<int>(static_cast<uint32_t>(__float_as_int(mx)) >> 23), 126);
 					const float scale = __int_as_float((127 + shift) << 23);
@@ -1191,6 +1256,14 @@ namespace litenn_hip
 				}
 				if (col < n)
 				{
+					if constexpr (F::kMins)
+					{
+						if (__builtin_expect(!(fabsf(v) <= 3.402823466e38f), 0))
+						{
+							const float* const from = x + static_cast<size_t>(row) * k;
+							v = plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) { return from[i]; });
+						}
+					}
 					const size_t o = static_cast<size_t>(row) * n + col;
 					y[o] = residual ? residual[o] + v : v;
 				}

@@ -143,3 +143,18 @@ def test_activations_far_below_their_rows_largest_keep_their_bits(hip, fmt, m, n
     rest[:, 0] = 0.0
     size = np.linalg.norm(rest, axis=1) * np.linalg.norm(w) / np.sqrt(k)
     assert (np.linalg.norm(got - rest @ w.T, axis=1) / size).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt", [Q4_K, Q5_K])
+@pytest.mark.parametrize("m,n,k", [(6, 70, 768), (40, 130, 512), (300, 5200, 256)])
+def test_infinite_activations_give_the_infinities_that_one_row_by_itself_gives(hip, fmt, m, n, k):
+    wq = synth.model_weights(fmt, n, k, 5, 4)  # (scales of either sign, so that some sums are infinite and no NaN)
+    x = synth.activations(m, k, 6, 4)
+    x[0, 3], x[1, 200], x[2, [70, 90]], x[3, [10, 255]] = np.inf, -np.inf, np.inf, [-np.inf, np.inf]
+    w, t = hip.Tensor.from_numpy(wq), hip.Tensor.from_numpy
+    got = hip.mul_mat_q(fmt, w, n, k, t(x), flags=MATMUL_PRECISE).numpy()
+    want = np.concatenate([hip.mul_mat_q(fmt, w, n, k, t(x[i:i + 1]), flags=MATMUL_PRECISE).numpy() for i in range(4)])
+    signed = np.isinf(want)  # (where that is no number, the several rows' sums, formed in another order, may be one)
+    assert signed.sum() >= 8
+    assert np.array_equal(got[:4][signed], want[signed]) and not np.isfinite(got[:4]).any()
+    assert np.isfinite(got[4:]).all()
