@@ -148,9 +148,10 @@ int litenn_hip_permute(int dev, void* dst, int dtype, const size_t* src_shape, s
  * on the matrix cores (weights as exact integers, every activation as two halves, off by 2^-24 of itself at most down to
  * 2^-28 of its row's largest and by 2^-52 of the largest below that, block scales and sums in f32: the streaming GEMV's
  * accuracy), 2 to 8 rows in one launch without scratch, more with
- * k <= 16384 in scratch of the device's memory pool or in a given workspace if it has 4.125 * m * k bytes and some
- * (m rounded up to 32, k to 256); without such room, and for the other formats, row by row through the GEMV, which
- * needs none.
+ * k <= 16384 in scratch of the device's memory pool, or in a given workspace of at least
+ * litenn_hip_mul_mat_q_precise_workspace_bytes(m, k) (16-byte aligned; 0 where none is used); with a smaller one, on a
+ * stream that is being captured without one, and for the other formats, row by row through the GEMV, which needs none
+ * and adds in another order.
  * The matrix-core path needs a device workspace of litenn_hip_mul_mat_q_workspace_bytes(m, k):
  * litenn_hip_mul_mat_q takes it from the device's memory pool in stream order (hipMallocAsync /
  * hipFreeAsync on the call's stream: no wait for the stream, opts->synchronize is honoured; only
@@ -167,6 +168,7 @@ int litenn_hip_permute(int dev, void* dst, int dtype, const size_t* src_shape, s
 int litenn_hip_mul_mat_q(int dev, int fmt, const void* wq, size_t n, size_t k, const void* x, int x_dtype, size_t m,
                          void* y, const void* residual, unsigned flags, const litenn_hip_exec* opts);
 size_t litenn_hip_mul_mat_q_workspace_bytes(size_t m, size_t k);
+size_t litenn_hip_mul_mat_q_precise_workspace_bytes(size_t m, size_t k);
 /* Measurement aid, no reference counterpart: writes into out (capacity bytes, always terminated)
  * which instance of the streaming single-row kernel the calling thread's last m == 1 matmul or
  * linear group launched and with what geometry, e.g.

@@ -91,6 +91,7 @@ SIGNATURES = {
     "litenn_hip_permute": [_i, _vp, _i, _szp, _sz, _vp, _szp, _ex],
     "litenn_hip_mul_mat_q": [_i, _i, _vp, _sz, _sz, _vp, _i, _sz, _vp, _vp, _u, _ex],
     "litenn_hip_mul_mat_q_workspace_bytes": [_sz, _sz],
+    "litenn_hip_mul_mat_q_precise_workspace_bytes": [_sz, _sz],
     "litenn_hip_gemv_last_launch": [C.c_char_p, _sz],
     "litenn_hip_gemm_last_launch": [C.c_char_p, _sz],
     "litenn_hip_mul_mat_q_ws": [_i, _i, _vp, _sz, _sz, _vp, _i, _sz, _vp, _vp, _u, _vp, _sz, _ex],
@@ -147,6 +148,7 @@ SIGNATURES = {
 _RESTYPES = {
     "litenn_hip_gla_workspace_bytes": C.c_size_t,
     "litenn_hip_last_error": C.c_char_p, "litenn_hip_llama_model": C.c_void_p, "litenn_hip_mul_mat_q_workspace_bytes": C.c_size_t,
+    "litenn_hip_mul_mat_q_precise_workspace_bytes": C.c_size_t,
     "litenn_gguf_close": None, "litenn_gguf_version": C.c_uint, "litenn_gguf_tensor_count": C.c_size_t,
     "litenn_gguf_metadata_count": C.c_size_t, "litenn_gguf_metadata_key": C.c_char_p,
 }

@@ -16,6 +16,7 @@ namespace litenn_hip
 	                const float* residual, hipStream_t stream);
 	size_t gemm_scratch_halves(size_t m, size_t k);
 	size_t exact_scratch_bytes(size_t m, size_t k);
+	bool exact_rows_take(size_t m, size_t k);
 	bool exact_gemm_takes(int fmt, const void* wq, size_t n, size_t k);
 	bool launch_exact_rows(const float* x, size_t m, size_t k, const float* norm_w, double eps, const float* up,
 	                       void* scratch, hipStream_t stream);
@@ -779,6 +780,11 @@ static constexpr size_t kExactMinRows = 8;
 extern "C" size_t litenn_hip_mul_mat_q_workspace_bytes(size_t m, size_t k)
 {
 	return m >= kMatrixCoreMinRows ? 2 * gemm_scratch_halves(m, k) : 0;
+}
+
+extern "C" size_t litenn_hip_mul_mat_q_precise_workspace_bytes(size_t m, size_t k)
+{
+	return m > kFewRows && exact_rows_take(m, k) ? exact_scratch_bytes(m, k) : 0;
 }
 
 extern "C" int litenn_hip_mul_mat_q(int dev, int fmt, const void* wq, size_t n, size_t k, const void* x, int x_dtype,

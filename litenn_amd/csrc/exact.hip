@@ -1401,6 +1401,12 @@ namespace litenn_hip
 		return RowsLayout(tiles, chunks).bytes;
 	}
 
+	// Whether launch_exact_rows takes rows of this number and width.
+	bool exact_rows_take(size_t m, size_t k)
+	{
+		return m > 0 && m <= (size_t{ 1 } << 20) && k > 0 && k % 32 == 0 && k <= static_cast<size_t>(kHeldItems) * 256 * 8;
+	}
+
 	// Whether launch_exact_gemm takes a matrix: one of the formats above, rows that start on 2 bytes.
 	bool exact_gemm_takes(int fmt, const void* wq, size_t n, size_t k)
 	{
@@ -1419,8 +1425,7 @@ namespace litenn_hip
 	                       hipStream_t stream)
 	{
 		const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-		if (!scratch || m == 0 || m > (size_t{ 1 } << 20) || k == 0 || k % 32 != 0 || k > static_cast<size_t>(kHeldItems) * 256 * 8 ||
-		    !aligned(x) || !aligned(scratch) || !aligned(norm_w) || !aligned(up) || (norm_w && up))
+		if (!scratch || !exact_rows_take(m, k) || !aligned(x) || !aligned(scratch) || !aligned(norm_w) || !aligned(up) || (norm_w && up))
 		{
 			return false;
 		}

@@ -158,3 +158,25 @@ def test_infinite_activations_give_the_infinities_that_one_row_by_itself_gives(h
     assert signed.sum() >= 8
     assert np.array_equal(got[:4][signed], want[signed]) and not np.isfinite(got[:4]).any()
     assert np.isfinite(got[4:]).all()
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [(Q4_K, 9, 40, 256), (Q8_0, 33, 200, 1056), (Q6_K, 64, 70, 512)])
+def test_a_workspace_of_the_size_asked_for_is_used(hip, fmt, m, n, k):
+    import ctypes as C
+    from litenn_amd import _lib
+    lib = _lib.load()
+    size = lib.litenn_hip_mul_mat_q_precise_workspace_bytes(m, k)
+    wq, x = synth.model_weights(fmt, n, k, 5, 2), synth.activations(m, k, 6, 2)
+    w, xt = hip.Tensor.from_numpy(wq), hip.Tensor.from_numpy(x)
+    want = hip.mul_mat_q(fmt, w, n, k, xt, flags=MATMUL_PRECISE).numpy()
+    room = hip.Tensor.from_numpy(np.zeros(size, np.uint8))
+    y = hip.Tensor.from_numpy(np.full((m, n), np.nan, np.float32))
+    _lib.check(lib.litenn_hip_mul_mat_q_ws(0, fmt, w.ptr, n, k, xt.ptr, 0, m, y.ptr, None, MATMUL_PRECISE, room.ptr, C.c_size_t(size), None))
+    assert np.array_equal(y.numpy(), want) and room.numpy().any()
+
+
+@pytest.mark.parametrize("m,k,some", [(1, 512, False), (8, 512, False), (9, 16384, True), (9, 16640, False), (40, 48, False)])
+def test_a_workspace_is_asked_for_where_one_is_used(hip, m, k, some):
+    from litenn_amd import _lib
+    size = _lib.load().litenn_hip_mul_mat_q_precise_workspace_bytes(m, k)
+    assert (size >= 4 * m * k) == some and (size > 0) == some
