@@ -43,9 +43,9 @@ namespace litenn_hip
 			return 0;
 		}
 
-		int ensure_base(litenn_hip_model* m, size_t rows, size_t logit_rows)
+		int ensure_base(litenn_hip_model* m, size_t rows, size_t logit_rows, unsigned flags)
 		{
-			if (m->ensure_rows(rows) != 0)
+			if (m->ensure_rows(rows, flags) != 0)
 			{
 				return 1;
 			}
@@ -200,7 +200,7 @@ namespace litenn_hip
 				++pick_end;
 			}
 			const size_t logit_rows = pick_end > next_pick ? first + count - picks[next_pick].first : 1;
-			if (ensure_base(m, pass, logit_rows) != 0)
+			if (ensure_base(m, pass, logit_rows, flags) != 0)
 			{
 				return 1;
 			}
@@ -268,7 +268,7 @@ namespace litenn_hip
 			return fail_hip(m->action, guard.error());
 		}
 		const size_t pass = std::min(n_prompt, m->pass_rows());
-		if (ensure_base(m, pass, 1) != 0)
+		if (ensure_base(m, pass, 1, flags) != 0)
 		{
 			return 1;
 		}

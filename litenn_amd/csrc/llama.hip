@@ -114,8 +114,8 @@ struct litenn_hip_llama : litenn_hip_model
 	float *x = nullptr, *xn = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *attn = nullptr, *gate = nullptr,
 	      *gate2 = nullptr, *up = nullptr;
 	size_t xn_floats = 0; // what xn holds (rows x embedding_length, three times that for short prompts)
-	void* xh = nullptr; // fp16 copy of a matmul's activations (multi-row path), 16-row padded
-	size_t xh_halves = 0; // its size: room for the widest matmul, and for two copies of the embedding width
+	void* xh = nullptr; // a matmul's activations as the matrix cores take them (multi-row path)
+	size_t xh_halves = 0; // its size
 	// single-row attention: key chunks per head, their meeting place and arrival counters
 	size_t attn_splits = 1;
 	float* attn_partial = nullptr;
@@ -130,7 +130,7 @@ struct litenn_hip_llama : litenn_hip_model
 
 	~litenn_hip_llama() override;
 	int check_complete() override;
-	int ensure_rows(size_t rows) override;
+	int ensure_rows(size_t rows, unsigned flags) override;
 	void prepare() override;
 	void forward(const int32_t* ids, size_t rows, size_t logit_rows, unsigned flags, int past) override;
 	bool give_up_waiting() override;
@@ -159,7 +159,33 @@ namespace
 		m->cap_rows = 0;
 	}
 
-	int ensure_scratch(litenn_hip_llama* m, size_t rows)
+	// Halves that the rows of the model's matmuls take on their way to the matrix cores: rounded to fp16 (q/k/v projections in
+	// two formats share a launch that wants them in both fragment orders), or, for matrices that meet Float32
+	// operands, taken apart into two halves each.
+	size_t matmul_halves(const litenn_hip_llama* m, size_t rows, unsigned flags)
+	{
+		const size_t d = m->p.embedding_length, ff = m->p.feed_forward_length;
+		const size_t qw = static_cast<size_t>(m->p.head_count) * m->head_dim;
+		size_t widest = 0;
+		const auto look_at = [&](const Weight& w) {
+			if (((flags & LITENN_HIP_MATMUL_PRECISE) || w.k % 256 != 0) && exact_gemm_takes(w.fmt, w.data, w.n, w.k))
+			{
+				widest = std::max(widest, w.k);
+			}
+		};
+		look_at(m->output.data ? m->output : m->tok_embd);
+		for (const Layer& L : m->layers)
+		{
+			for (const Weight* w : { &L.wq, &L.wk, &L.wv, &L.wo, &L.gate, &L.up, &L.down })
+			{
+				look_at(*w);
+			}
+		}
+		const size_t rounded = std::max(gemm_scratch_halves(rows, std::max({ d, qw, ff })), 2 * gemm_scratch_halves(rows, d));
+		return widest ? std::max(rounded, (exact_scratch_bytes(rows, widest) + 1) / 2) : rounded;
+	}
+
+	int ensure_scratch(litenn_hip_llama* m, size_t rows, unsigned flags)
 	{
 		const size_t d = m->p.embedding_length;
 		const size_t qw = static_cast<size_t>(m->p.head_count) * m->head_dim;
@@ -180,12 +206,17 @@ namespace
 			{
 				LITENN_HIP_TRY(kAction, hipMalloc(reinterpret_cast<void**>(b.p), sizeof(float) * rows * b.n));
 			}
-			// (q/k/v projections in two formats share a launch that wants the rows in both fragment orders)
-			m->xh_halves = std::max(gemm_scratch_halves(rows, std::max({ d, qw, ff })), 2 * gemm_scratch_halves(rows, d));
-			// or, with Float32 operands, the rows taken apart into two halves each
-			m->xh_halves = std::max(m->xh_halves, (exact_scratch_bytes(rows, std::max({ d, qw, ff })) + 1) / 2);
-			LITENN_HIP_TRY(kAction, hipMalloc(&m->xh, 2 * m->xh_halves));
 			m->cap_rows = rows;
+		}
+		const size_t halves = m->xh && rows == 1 ? 0 : matmul_halves(m, m->cap_rows, flags); // (a single row uses none)
+		if (!m->xh || halves > m->xh_halves)
+		{
+			decoder_drop_graph(m);
+			(void)hipFree(m->xh);
+			m->xh = nullptr;
+			m->xh_halves = 0;
+			LITENN_HIP_TRY(kAction, hipMalloc(&m->xh, 2 * halves));
+			m->xh_halves = halves;
 		}
 		return 0;
 	}
@@ -594,7 +625,7 @@ namespace
 
 int litenn_hip_llama::check_complete() { return check_tensors(this); }
 
-int litenn_hip_llama::ensure_rows(size_t rows) { return ensure_scratch(this, rows); }
+int litenn_hip_llama::ensure_rows(size_t rows, unsigned flags) { return ensure_scratch(this, rows, flags); }
 
 void litenn_hip_llama::prepare() { (void)block_fused_ready(this); }
 

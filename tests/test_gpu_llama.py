@@ -396,3 +396,19 @@ def test_generation_through_every_chunk_count(hip, oracle):
     for a, b in zip(dev.get_kv(1), kv):
         assert np.array_equal(a, b)
     dev.close()
+
+
+@pytest.mark.parametrize("fmt,ff", [(Q4_0, 320), (Q4_K, 512)])
+def test_float32_operands_after_rounded_ones(hip, fmt, ff):
+    """Rows taken apart want more room than rounded ones: it is taken at the first pass that asks for Float32 operands, behind
+    which the model gives what one that never did anything else gives."""
+    cfg = synth.LLaMAConfig("two-ways", 2, 256, 4, 2, ff, 300, 256, formats={"default": fmt})
+    tokens = np.arange(90, dtype=np.int32) % 300
+    alone = [hip_model(hip, cfg, 5).eval(tokens, precise=precise) for precise in (False, True)]
+    steps = [hip_model(hip, cfg, 5).generate(tokens, 6, precise=precise)[0] for precise in (False, True)]
+    model = hip_model(hip, cfg, 5)
+    for precise in (False, True, False, True):
+        model.reset()
+        assert np.array_equal(model.generate(tokens, 6, precise=precise)[0], steps[precise])
+        model.reset()
+        assert np.array_equal(model.eval(tokens, precise=precise), alone[precise])
