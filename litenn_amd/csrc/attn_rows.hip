@@ -305,7 +305,8 @@ namespace litenn_hip
 				}
 				else
 				{
-					__builtin_amdgcn_wave_barrier(); // (a wavefront's LDS accesses keep their order)
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
+					__builtin_amdgcn_wave_barrier();
 				}
 			};
 

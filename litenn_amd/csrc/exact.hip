@@ -725,6 +725,7 @@ namespace litenn_hip
 					}
 				}
 				weights.deposit(moving, lane);
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 				if constexpr (kShared)
 				{
 					deposit(staged[0], 0);
@@ -902,7 +903,10 @@ namespace litenn_hip
 							}
 						}
 					}
-					weights.deposit(moving, lane); // (the wavefront's own reads of the slot are behind it in its instruction stream)
+					// (a wavefront's LDS accesses keep their order: the slot's reads, the next chunk, its reads)
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+					weights.deposit(moving, lane);
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 				}
 			}
 
