@@ -769,13 +769,10 @@ static bool is_weight_format(int fmt)
 // tile costs about as much as three single-row GEMVs (Q4_K 14336 x 4096: 14.6 us against 8.2 each).
 static constexpr size_t kMatrixCoreMinRows = 4;
 
-// Up to this many rows with Float32 operands share the weights in one launch that needs no scratch (Q4_K 14336 x 4096 at
-// 8 rows 19.4 us, through scratch 25.6; the next row would double the fragments).
+// Up to this many rows with Float32 operands share the weights in one launch that needs no scratch, more through scratch
+// (Q4_K 14336 x 4096 at 8 rows 19.4 us, through scratch 25.6; the next row would double the fragments).
 static constexpr size_t kFewRows = 8;
 
-// From this many rows on a matmul with Float32 operands shares the weights between its rows through scratch (formats
-// or rows that the form above does not take go one by one below it).
-static constexpr size_t kExactMinRows = 8;
 
 extern "C" size_t litenn_hip_mul_mat_q_workspace_bytes(size_t m, size_t k)
 {
@@ -902,7 +899,7 @@ extern "C" int litenn_hip_mul_mat_q_ws(int dev, int fmt, const void* wq, size_t 
 	// Several rows with Float32 operands share the weights on the matrix cores (csrc/exact.hip) where there is room for
 	// the rows taken apart: in the caller's workspace, or, where none was given, from the device's memory pool.  A
 	// call that finds no room, or whose stream is being captured, streams the weights row by row, which needs none.
-	if (m >= kExactMinRows && exact_gemm_takes(fmt, wq, n, k))
+	if (m > kFewRows && exact_gemm_takes(fmt, wq, n, k))
 	{
 		const size_t need = exact_scratch_bytes(m, k);
 		StreamScratch scratch(s);

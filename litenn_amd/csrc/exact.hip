@@ -51,7 +51,7 @@ namespace litenn_hip
 		constexpr float kLowScale = 1.0f / 4096.0f; // of the low parts: small activations beside a large one keep their bits
 
 		// ---- weight blocks -> binary16 integers -------------------------------------------------------
-		// A wavefront copies the raw blocks of its 32 NG rows for one 256-element chunk into a slot of its own in
+		// A wavefront copies the raw blocks of its 32 rows for one 256-element chunk into a slot of its own in
 		// LDS, 16-byte pieces in a row's order (eight neighbouring lanes fetch one 128-byte line; a lane that
 		// fetched its own row's bytes instead took 29 us for Q8_0 4096 x 4096, most of it in the vector memory
 		// path).  From there lane (r, h) = (lane % 32, lane / 32) takes, of weight row r, elements 16 s + 8 h .. + 7
@@ -542,16 +542,16 @@ namespace litenn_hip
 			}
 		}
 
-		// A wavefront's share of the weights on their way: the raw blocks of 32 NG rows for one chunk, from memory (where
+		// A wavefront's share of the weights on their way: the raw blocks of 32 rows for one chunk, from memory (where
 		// they lie on 2 bytes) to the wavefront's slot in LDS (where a row's chunk begins on 16).  The P pieces of a row fall
 		// into groups of 16, 8, 4, 2 and 1 (the bits of P); a load takes one group of as many rows as there are lanes for, so
 		// that a lane's place in the row stays the same from load to load and its addresses are one sum.  Nothing behind
 		// the matrix is fetched: rows behind the last are the last, and a row's chunk that is not whole comes element
 		// by element, its missing part being the row's last two bytes.
-		template <typename F, int NG>
+		template <typename F>
 		struct WeightPieces
 		{
-			static constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>(), kRows = NG * kTile;
+			static constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>(), kRows = kTile;
 			static constexpr int loads_of(int width) { return (P & width) != 0 ? (kRows * width + 63) / 64 : 0; }
 			static constexpr int kLoads = loads_of(16) + loads_of(8) + loads_of(4) + loads_of(2) + loads_of(1);
 			static constexpr int kSlotBytes = kRows * kStride;
@@ -610,18 +610,18 @@ namespace litenn_hip
 			{
 				each(lane, [&](int i, int row, int piece) { *reinterpret_cast<u32x4*>(slot + row * kStride + 16 * piece) = moving[i]; });
 			}
-			// the lane's row of group q in the slot
-			__device__ __forceinline__ lds_bytes_t chunk(int q, int lane) const { return (lds_bytes_t)(slot) + (kTile * q + (lane & 31)) * kStride; }
+			// the lane's row in the slot
+			__device__ __forceinline__ lds_bytes_t chunk(int lane) const { return (lds_bytes_t)(slot) + (lane & 31) * kStride; }
 		};
 
-		// A wavefront multiplies NG groups of 32 weight rows by MT tiles of 32 activation rows over one of KS
+		// A wavefront multiplies 32 weight rows by MT tiles of 32 activation rows over one of KS
 		// ranges of K; the KS sums meet in LDS at the end, added in K order.  Two levels of sums, a chunk's and
 		// the range's, keep the rounding of long rows down.  WN wavefronts side by side share the activation
 		// fragments of a range through LDS (two buffers of one 64-element stage, the next two stages travelling
 		// through registers while the current one is multiplied); with WN = 1 nobody shares them and they go to
 		// registers directly, each refilled for the next stage once it has been used.  The raw blocks of the
 		// next chunk travel through registers into the wavefront's slot meanwhile.
-		template <typename F, int NG, int MT, int WN, int KS>
+		template <typename F, int MT, int WN, int KS>
 		__global__ __launch_bounds__(64 * WN * KS) void exact_gemm_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                  const float* residual, int k, int m, int m_tiles,
 		                                                                  int chunks, size_t row_bytes)
@@ -629,7 +629,7 @@ namespace litenn_hip
 			constexpr bool kShared = WN > 1;
 			constexpr int kPieces = kShared ? MT * 8 / WN : 1; // 1 KB pieces a wavefront stages
 			static_assert(!kShared || kPieces * WN == MT * 8, "activation pieces / wavefront split");
-			typedef WeightPieces<F, NG> W;
+			typedef WeightPieces<F> W;
 			constexpr int kRingBytes = kShared ? KS * 2 * MT * kStageBytes : 0;
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
 			int grid_x, grid_y;
@@ -643,7 +643,7 @@ namespace litenn_hip
 			const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 			const int part = wave / WN, wv = wave % WN;
 			const int r = lane & 31, h = lane >> 5;
-			const int n_base = (block_x * WN + wv) * (NG * kTile);
+			const int n_base = (block_x * WN + wv) * kTile;
 			const int mt_base = grid_y * MT;
 			const int per = (chunks + KS - 1) / KS;
 			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
@@ -662,15 +662,11 @@ namespace litenn_hip
 				sum_tiles[t] = xs + at.sums + tile * chunks * kFrag + lane * 16;
 			}
 
-			floatx16 acc[NG][MT], p[NG][MT], first[F::kMins ? NG : 1][MT]; // first: of the chunk's first half, where kScaleSteps is 16
+			floatx16 acc[MT], p[MT], first[MT]; // first: of the chunk's first half, where kScaleSteps is 16
 #pragma unroll
-			for (int q = 0; q < NG; ++q)
+			for (int t = 0; t < MT; ++t)
 			{
-#pragma unroll
-				for (int t = 0; t < MT; ++t)
-				{
-					acc[q][t] = floatx16{};
-				}
+				acc[t] = floatx16{};
 			}
 
 			// ---- activations
@@ -741,17 +737,13 @@ namespace litenn_hip
 				const int c = c_begin + i;
 				const bool live = c < c_end; // (uniform: a shorter range only passes the barriers)
 				const int next = min(c + 1, c_end - 1);
-				typename F::Head head[NG];
-				floatx16 sum[F::kScaleSteps < 16 ? NG : 1][MT]; // the chunk's
+				typename F::Head head;
+				floatx16 sum[MT]; // the chunk's, where kScaleSteps is less
 				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
 				if (live)
 				{
 					weights.request(moving, next, lane);
-#pragma unroll
-					for (int q = 0; q < NG; ++q)
-					{
-						head[q] = F::head(weights.chunk(q, lane), h);
-					}
+					head = F::head(weights.chunk(lane), h);
 					if constexpr (F::kMins)
 					{
 #pragma unroll
@@ -766,12 +758,7 @@ namespace litenn_hip
 				{
 					if (live)
 					{
-						typename F::Raw raw[NG];
-#pragma unroll
-						for (int q = 0; q < NG; ++q)
-						{
-							raw[q] = F::load(weights.chunk(q, lane), st, h, blocks);
-						}
+						const typename F::Raw raw = F::load(weights.chunk(lane), st, h, blocks);
 						if constexpr (kShared)
 						{
 							request(staged[st & 1], st < 2 ? c : next, (st + 2) & 3);
@@ -779,13 +766,7 @@ namespace litenn_hip
 #pragma unroll
 						for (int s = 0; s < 4; ++s)
 						{
-							half8 b[NG], b_low[NG];
-#pragma unroll
-							for (int q = 0; q < NG; ++q)
-							{
-								b[q] = F::frag(head[q], raw[q], st, s);
-								b_low[q] = lowered(b[q]);
-							}
+							const half8 b = F::frag(head, raw, st, s), b_low = lowered(b);
 							const int step = 4 * st + s;
 							const bool fresh = step % min(F::kScaleSteps, 8) == 0;
 #pragma unroll
@@ -805,12 +786,8 @@ namespace litenn_hip
 										a[e] = direct[t][s][e];
 									}
 								}
-#pragma unroll
-								for (int q = 0; q < NG; ++q)
-								{
-									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b[q], fresh ? floatx16{} : p[q][t], 0, 0, 0);
-									p[q][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b_low[q], p[q][t], 0, 0, 0);
-								}
+								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b, fresh ? floatx16{} : p[t], 0, 0, 0);
+								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b_low, p[t], 0, 0, 0);
 							}
 							if constexpr (!kShared)
 							{
@@ -821,13 +798,9 @@ namespace litenn_hip
 								if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
 								{
 #pragma unroll
-									for (int q = 0; q < NG; ++q)
+									for (int t = 0; t < MT; ++t)
 									{
-#pragma unroll
-										for (int t = 0; t < MT; ++t)
-										{
-											first[q][t] = p[q][t];
-										}
+										first[t] = p[t];
 									}
 								}
 							}
@@ -835,18 +808,14 @@ namespace litenn_hip
 							{
 								if (step % F::kScaleSteps == F::kScaleSteps - 1)
 								{
+									const float d = F::scale(head, raw, st, s);
 #pragma unroll
-									for (int q = 0; q < NG; ++q)
+									for (int t = 0; t < MT; ++t)
 									{
-										const float d = F::scale(head[q], raw[q], st, s);
 #pragma unroll
-										for (int t = 0; t < MT; ++t)
+										for (int e = 0; e < 16; ++e)
 										{
-#pragma unroll
-											for (int e = 0; e < 16; ++e)
-											{
-												sum[q][t][e] = step == F::kScaleSteps - 1 ? d * p[q][t][e] : fmaf(d, p[q][t][e], sum[q][t][e]);
-											}
+											sum[t][e] = step == F::kScaleSteps - 1 ? d * p[t][e] : fmaf(d, p[t][e], sum[t][e]);
 										}
 									}
 								}
@@ -865,41 +834,37 @@ namespace litenn_hip
 				}
 				if (live)
 				{
-#pragma unroll
-					for (int q = 0; q < NG; ++q)
+					const float d = F::chunk_scale(head);
+					if constexpr (F::kMins)
 					{
-						const float d = F::chunk_scale(head[q]);
-						if constexpr (F::kMins)
-						{
-							const half8 b = for_sums(F::centre_frag(head[q]), h);
-#pragma unroll
-							for (int t = 0; t < MT; ++t)
-							{
-								p[q][t] = first[q][t] + __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, p[q][t], 0, 0, 0);
-							}
-						}
+						const half8 b = for_sums(F::centre_frag(head), h);
 #pragma unroll
 						for (int t = 0; t < MT; ++t)
 						{
+							p[t] = first[t] + __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, p[t], 0, 0, 0);
+						}
+					}
+#pragma unroll
+					for (int t = 0; t < MT; ++t)
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							acc[t][e] = fmaf(d, F::kScaleSteps < 16 ? sum[t][e] : p[t][e], acc[t][e]);
+						}
+					}
+					if constexpr (F::kMins)
+					{
+						const half8 b = for_sums(F::min_frag(head), h);
+						const float dm = F::min_scale(head) * (1.0f / kSumScale);
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+							const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, floatx16{}, 0, 0, 0);
 #pragma unroll
 							for (int e = 0; e < 16; ++e)
 							{
-								acc[q][t][e] = fmaf(d, F::kScaleSteps < 16 ? sum[q % (F::kScaleSteps < 16 ? NG : 1)][t][e] : p[q][t][e], acc[q][t][e]);
-							}
-						}
-						if constexpr (F::kMins)
-						{
-							const half8 b = for_sums(F::min_frag(head[q]), h);
-							const float dm = F::min_scale(head[q]) * (1.0f / kSumScale);
-#pragma unroll
-							for (int t = 0; t < MT; ++t)
-							{
-								const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, floatx16{}, 0, 0, 0);
-#pragma unroll
-								for (int e = 0; e < 16; ++e)
-								{
-									acc[q][t][e] = fmaf(dm, s[e], acc[q][t][e]);
-								}
+								acc[t][e] = fmaf(dm, s[e], acc[t][e]);
 							}
 						}
 					}
@@ -918,17 +883,13 @@ namespace litenn_hip
 				if (part > 0)
 				{
 #pragma unroll
-					for (int q = 0; q < NG; ++q)
+					for (int t = 0; t < MT; ++t)
 					{
 #pragma unroll
-						for (int t = 0; t < MT; ++t)
+						for (int e = 0; e < 16; e += 4)
 						{
-#pragma unroll
-							for (int e = 0; e < 16; e += 4)
-							{
-								float4* dst = reinterpret_cast<float4*>(handed + (((part - 1) * WN + wv) * NG * MT + q * MT + t) * 64) + (e / 4) * 64 + lane;
-								*dst = float4{ acc[q][t][e], acc[q][t][e + 1], acc[q][t][e + 2], acc[q][t][e + 3] };
-							}
+							float4* dst = reinterpret_cast<float4*>(handed + (((part - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane;
+							*dst = float4{ acc[t][e], acc[t][e + 1], acc[t][e + 2], acc[t][e + 3] };
 						}
 					}
 				}
@@ -941,20 +902,16 @@ namespace litenn_hip
 				for (int other = 1; other < KS; ++other)
 				{
 #pragma unroll
-					for (int q = 0; q < NG; ++q)
+					for (int t = 0; t < MT; ++t)
 					{
 #pragma unroll
-						for (int t = 0; t < MT; ++t)
+						for (int e = 0; e < 16; e += 4)
 						{
-#pragma unroll
-							for (int e = 0; e < 16; e += 4)
-							{
-								const float4 v = *(reinterpret_cast<const float4*>(handed + (((other - 1) * WN + wv) * NG * MT + q * MT + t) * 64) + (e / 4) * 64 + lane);
-								acc[q][t][e] += v.x;
-								acc[q][t][e + 1] += v.y;
-								acc[q][t][e + 2] += v.z;
-								acc[q][t][e + 3] += v.w;
-							}
+							const float4 v = *(reinterpret_cast<const float4*>(handed + (((other - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane);
+							acc[t][e] += v.x;
+							acc[t][e + 1] += v.y;
+							acc[t][e + 2] += v.z;
+							acc[t][e + 3] += v.w;
 						}
 					}
 				}
@@ -962,7 +919,7 @@ namespace litenn_hip
 
 			// lane (r, h) holds weight row r and activation rows 8 (e / 4) + 4 h + e % 4
 			const float* factors = reinterpret_cast<const float*>(xs + at.factors);
-			uint32_t again[NG] = {}; // results that are not finite
+			uint32_t again = 0; // results that are not finite
 #pragma unroll
 			for (int t = 0; t < MT; ++t)
 			{
@@ -973,47 +930,39 @@ namespace litenn_hip
 					if (mm < m)
 					{
 						const float us = factors[mm];
-#pragma unroll
-						for (int q = 0; q < NG; ++q)
+						const int col = n_base + r;
+						if (col < n)
 						{
-							const int col = n_base + kTile * q + r;
-							if (col < n)
+							const size_t o = static_cast<size_t>(mm) * n + col;
+							if (F::kMins && !(fabsf(acc[t][e]) <= 3.402823466e38f))
 							{
-								const size_t o = static_cast<size_t>(mm) * n + col;
-								if (F::kMins && !(fabsf(acc[q][t][e]) <= 3.402823466e38f))
-								{
-									again[q] |= 1u << (16 * t + e);
-									continue;
-								}
-								float v = acc[q][t][e] * us;
-								if (residual)
-								{
-									v = residual[o] + v;
-								}
-								y[o] = v;
+								again |= 1u << (16 * t + e);
+								continue;
 							}
+							float v = acc[t][e] * us;
+							if (residual)
+							{
+								v = residual[o] + v;
+							}
+							y[o] = v;
 						}
 					}
 				}
 			}
 			if constexpr (F::kMins)
 			{
-#pragma unroll
-				for (int q = 0; q < NG; ++q)
+				const int col = n_base + r;
+				while (__builtin_expect(again != 0, 0))
 				{
-					const int col = n_base + kTile * q + r;
-					while (__builtin_expect(again[q] != 0, 0))
-					{
-						const int i = __ffs(again[q]) - 1, e = i & 15, mm = (mt_base + (i >> 4)) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
-						again[q] &= again[q] - 1;
-						const uint8_t* const parts = xs + static_cast<size_t>(mm / kTile) * chunks * kTileChunkBytes + (mm % kTile) * 16;
-						const float v = factors[mm] * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
-							const uint8_t* const at = parts + static_cast<size_t>(i >> 4) * (2 * kFrag) + ((i >> 3) & 1) * 512 + (i & 7) * 2;
-							return fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(at + kFrag)), kLowScale, static_cast<float>(*reinterpret_cast<const _Float16*>(at)));
-						});
-						const size_t o = static_cast<size_t>(mm) * n + col;
-						y[o] = residual ? residual[o] + v : v;
-					}
+					const int i = __ffs(again) - 1, e = i & 15, mm = (mt_base + (i >> 4)) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
+					again &= again - 1;
+					const uint8_t* const parts = xs + static_cast<size_t>(mm / kTile) * chunks * kTileChunkBytes + (mm % kTile) * 16;
+					const float v = factors[mm] * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
+						const uint8_t* const at = parts + static_cast<size_t>(i >> 4) * (2 * kFrag) + ((i >> 3) & 1) * 512 + (i & 7) * 2;
+						return fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(at + kFrag)), kLowScale, static_cast<float>(*reinterpret_cast<const _Float16*>(at)));
+					});
+					const size_t o = static_cast<size_t>(mm) * n + col;
+					y[o] = residual ? residual[o] + v : v;
 				}
 			}
 		}
@@ -1034,7 +983,6 @@ namespace litenn_hip
 			static constexpr int kSums = 32 * kHalf;                      // sub-block sums: [hi, lo][row][8 halves]
 			static constexpr int kUnused = kSums + 2 * kPart; // what lanes with nothing to write write
 			static constexpr int kBytes = kUnused + 256;
-			static constexpr int kValues = MR > 8 ? 8 : 4; // results of a lane
 		};
 
 		template <typename F, int MR, int KS>
@@ -1042,8 +990,8 @@ namespace litenn_hip
 		                                                            const float* residual, int n, int k, int m, int chunks, size_t row_bytes)
 		{
 			typedef FewRows<MR> R;
-			typedef WeightPieces<F, 1> W;
-			constexpr int NE = R::kValues;
+			typedef WeightPieces<F> W;
+			constexpr int NE = 4; // results of a lane
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][slot, fragments]; later the KS sums
 			const int lane = threadIdx.x & 63;
 			const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1141,7 +1089,7 @@ namespace litenn_hip
 				request_x(min(c + 1, c_end - 1));
 				weights.request(arrived, min(c + 2, c_end - 1), lane);
 				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
-				lds_bytes_t const chunk = weights.chunk(0, lane);
+				lds_bytes_t const chunk = weights.chunk(lane);
 				const typename F::Head head = F::head(chunk, h);
 				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
 				floatx16 p;
@@ -1288,12 +1236,12 @@ namespace litenn_hip
 			hipStream_t stream;
 		};
 
-		template <typename F, int NG, int MT, int WN, int KS>
+		template <typename F, int MT, int WN, int KS>
 		void launch_variant(const ExactCall& c)
 		{
 			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * 2 * MT * kStageBytes : 0) +
-			                         static_cast<size_t>(WN) * KS * WeightPieces<F, NG>::kSlotBytes;
-			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * NG * MT * 64 * 64;
+			                         static_cast<size_t>(WN) * KS * WeightPieces<F>::kSlotBytes;
+			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * MT * 64 * 64;
 			constexpr size_t lds = rings > sums ? rings : sums;
 			static_assert(lds <= 160 * 1024, "LDS");
 			ExactMats mats{};
@@ -1307,12 +1255,12 @@ namespace litenn_hip
 					mats.y[i] = c.y[i];
 					mats.n[i] = c.n[i];
 					mats.first_block[i] = blocks;
-					blocks += (c.n[i] + WN * NG * kTile - 1) / (WN * NG * kTile);
+					blocks += (c.n[i] + WN * kTile - 1) / (WN * kTile);
 				}
 			}
-			const auto kernel = &exact_gemm_kernel<F, NG, MT, WN, KS>;
+			const auto kernel = &exact_gemm_kernel<F, MT, WN, KS>;
 			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
-			exact_gemm_kernel<F, NG, MT, WN, KS><<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
+			exact_gemm_kernel<F, MT, WN, KS><<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
 			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
 		}
 
@@ -1323,26 +1271,28 @@ namespace litenn_hip
 			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each
 			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 262 against 301 of the
 			// forms below, at 64 rows 53 against 62.  Not for Q6_K, whose scaling per step wants the registers.
-			if (F::kScaleSteps > 1 && (strips + 3) / 4 * ((c.m_tiles + 1) / 2) >= 200 && c.m_tiles > 1)
+			if constexpr (F::kScaleSteps > 1)
 			{
-				launch_variant<F, 1, 2, 4, 2>(c);
+				if ((strips + 3) / 4 * ((c.m_tiles + 1) / 2) >= 200 && c.m_tiles > 1)
+				{
+					return launch_variant<F, 2, 4, 2>(c);
+				}
 			}
 			// Otherwise a wavefront keeps to itself and the ranges of K fill the card.  Q6_K saves a second decode with two
 			// tiles once there are enough of them (4096 x 14336 at 300 rows 168 against 207; at 45 rows 52 against 44).
-			else if (F::kScaleSteps == 1 && units >= 512 && c.m_tiles > 1)
+			else if (units >= 512 && c.m_tiles > 1)
 			{
-				launch_variant<F, 1, 2, 1, 8>(c);
+				return launch_variant<F, 2, 1, 8>(c);
 			}
-			// Eight ranges while there are few tiles (Q8_0 4096 x 4096 at 3 rows 14.7 against 16.6 with four, Q6_K
-			// 4096 x 14336 at 45 rows 44 against 54), four from there on (Q4_K 14336 x 4096 at 8 rows 18.1 against
-			// 20.7 with eight) and for short rows (Q8_0 1024 x 1024 7.2 against 8.1).
-			else if (units <= 256 && c.chunks >= 8)
+			// Eight ranges while there are few tiles (Q6_K 4096 x 14336 at 45 rows 44 against 54 with four), four from there
+			// on (Q4_K 14336 x 4096 at 8 rows 18.1 against 20.7 with eight) and for short rows (Q8_0 1024 x 1024 7.2 against 8.1).
+			if (units <= 256 && c.chunks >= 8)
 			{
-				launch_variant<F, 1, 1, 1, 8>(c);
+				launch_variant<F, 1, 1, 8>(c);
 			}
 			else
 			{
-				launch_variant<F, 1, 1, 1, 4>(c);
+				launch_variant<F, 1, 1, 4>(c);
 			}
 		}
 
@@ -1360,7 +1310,7 @@ namespace litenn_hip
 		template <typename F, int MR, int KS>
 		void launch_few(const FewCall& c)
 		{
-			constexpr size_t tiles = static_cast<size_t>(KS) * (WeightPieces<F, 1>::kSlotBytes + FewRows<MR>::kBytes);
+			constexpr size_t tiles = static_cast<size_t>(KS) * (WeightPieces<F>::kSlotBytes + FewRows<MR>::kBytes);
 			constexpr size_t sums = static_cast<size_t>(KS) * MR * kTile * sizeof(float);
 			constexpr size_t lds = tiles > sums ? tiles : sums;
 			static_assert(lds <= 160 * 1024, "LDS");
@@ -1389,7 +1339,7 @@ namespace litenn_hip
 		{
 			switch (c.m)
 			{
-			case 1: case 2: launch_few_rows<F, 2>(c); break;
+			case 2: launch_few_rows<F, 2>(c); break;
 			case 3: launch_few_rows<F, 3>(c); break;
 			case 4: launch_few_rows<F, 4>(c); break;
 			case 5: case 6: launch_few_rows<F, 6>(c); break;
@@ -1472,12 +1422,12 @@ namespace litenn_hip
 		}
 	}
 
-	// Y[M, N] = X . deq(W)^T (+ residual, which may alias y) for at most 8 rows, a matrix that exact_gemm_takes.
-	// Returns false, launching nothing, for more.
+	// Y[M, N] = X . deq(W)^T (+ residual, which may alias y) for 2 to 8 rows, a matrix that exact_gemm_takes.
+	// Returns false, launching nothing, for others.
 	bool launch_exact_few(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y, const float* residual,
 	                      hipStream_t stream)
 	{
-		if (m == 0 || m > 8 || k < 4)
+		if (m < 2 || m > 8 || k < 4)
 		{
 			return false;
 		}
