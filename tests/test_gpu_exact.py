@@ -180,3 +180,10 @@ def test_a_workspace_is_asked_for_where_one_is_used(hip, m, k, some):
     from litenn_amd import _lib
     size = _lib.load().litenn_hip_mul_mat_q_precise_workspace_bytes(m, k)
     assert (size >= 4 * m * k) == some and (size > 0) == some
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(300, 5200, 1280), (300, 2000, 4352)])
+def test_forms_of_two_tiles_over_several_chunks(hip, fmt, m, n, k):
+    """Ranges of three chunks and two (four wavefronts on shared activations), of three, three and two (Q6_K's form)."""
+    assert errors(hip, fmt, m, n, k, residual=fmt == Q4_0).max() <= 1e-6
