@@ -755,7 +755,7 @@ namespace litenn_hip
 				}
 				const float new_m = fmaxf(run_m, sc);
 				const float corr = softmax_weight(run_m, new_m);
-				const float pw = expf(sc - new_m);
+				const float pw = softmax_weight(sc, new_m); // (a mask may hide the first keys)
 				run_l = fmaf(run_l, corr, pw);
 #pragma unroll
 				for (int e = 0; e < E; ++e)

@@ -103,6 +103,19 @@ def test_scores_that_saturate_the_soft_cap(hip, dtype, m):
 
 
 @pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
+@pytest.mark.parametrize("m", [1, 7, 40])
+def test_a_mask_that_hides_the_first_keys(hip, dtype, m):
+    keys, heads, dim = 130, 2, 64
+    q, k, v = inputs(8, m, keys, heads, 1, dim, dtype)
+    mask = np.zeros((m, keys), np.float32)
+    mask[:, :37] = -np.inf
+    T = hip.Tensor.from_numpy
+    got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=dim ** -0.5, mask=T(mask), causal=False).numpy()
+    want = plain(*(a.astype(np.float64) for a in (q, k, v)), dim ** -0.5, 0, mask=mask.astype(np.float64), slopes=[1.0] * heads, causal=False)
+    assert worst(got, want) <= 2e-6
+
+
+@pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
 @pytest.mark.parametrize("dim", [64, 128])
 def test_operands_far_below_their_rows_largest(hip, dtype, dim):
     """A query's small elements beside one 2^26 times as large that meets zeros, and values of keys whose weights are
