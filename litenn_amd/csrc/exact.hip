@@ -15,13 +15,13 @@
 //     more product per 256 elements: the eight sums, taken apart the same way, against the eight
 //     six-bit minima.
 //
-// Against 64 bits the result is as close as the streaming kernel's (relative L2 0.8e-7 to 1.2e-7 over
-// K = 256 .. 14336 and every format; the streaming kernel has 0.9e-7 to 2.6e-7).
+// Against 64 bits the result is closer than the streaming kernel's in every format and form (relative L2 over K = 256 ..
+// 14336, mean of six inputs, 0.7e-7 to 1.2e-7; the streaming kernel 0.9e-7 to 2.5e-7).
 //
 // What bounds it: few rows are the weights' stream and the launch; many rows, the LDS reads of the fragments (two
 // per pair of products) and the latency in front of them: a product issues every 100 cycles and SIMD where
 // it takes 32.  Row by row through the streaming kernel the same calls took, us, before -> now with the rows'
-// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 46.7; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
+// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 46; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
 //
 // v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
 // weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
@@ -133,8 +133,8 @@ namespace litenn_hip
 		//   Head          what the lane needs of the chunk as a whole
 		//   kMins         whether a minimum term follows each chunk.  The integers are then taken about kCentre, the middle of
 		//                 their range, lower, and what that takes from the sum is added back per chunk, a product more over the
-		//                 sub-blocks' sums: the sums on the way stay as small as the result (relative error at Q5_K, 33 rows
-		//                 of 2048, 1.66e-7 without it)
+		//                 sub-blocks' sums, together with the minima, much of which it cancels: the sums on the way stay as small
+		//                 as the result (relative error at Q5_K, 33 rows of 2048, 1.66e-7 without it)
 		// Rows whose last chunk is not whole (blocks of 32 only) load their last block again in the missing blocks'
 		// places and scale it by 0 (`blocks` whole blocks of the chunk are there).
 		struct Q4_0X
@@ -513,6 +513,21 @@ namespace litenn_hip
 			}
 		}
 
+		// The sums of neighbouring ranges of K, then of neighbouring pairs: a shorter chain rounds less.  v[0] is the result.
+		template <typename V, int N>
+		__device__ __forceinline__ void add_in_pairs(V (&v)[N])
+		{
+#pragma unroll
+			for (int apart = 1; apart < N; apart *= 2)
+			{
+#pragma unroll
+				for (int i = 0; i + apart < N; i += 2 * apart)
+				{
+					v[i] += v[i + apart];
+				}
+			}
+		}
+
 		// ---- the product ------------------------------------------------------------------------------
 		struct ExactMats
 		{
@@ -837,34 +852,29 @@ namespace litenn_hip
 					const float d = F::chunk_scale(head);
 					if constexpr (F::kMins)
 					{
-						const half8 b = for_sums(F::centre_frag(head), h);
-#pragma unroll
-						for (int t = 0; t < MT; ++t)
-						{
-							p[t] = first[t] + __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, p[t], 0, 0, 0);
-						}
-					}
-#pragma unroll
-					for (int t = 0; t < MT; ++t)
-					{
-#pragma unroll
-						for (int e = 0; e < 16; ++e)
-						{
-							acc[t][e] = fmaf(d, F::kScaleSteps < 16 ? sum[t][e] : p[t][e], acc[t][e]);
-						}
-					}
-					if constexpr (F::kMins)
-					{
-						const half8 b = for_sums(F::min_frag(head), h);
+						const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
 						const float dm = F::min_scale(head) * (1.0f / kSumScale);
 #pragma unroll
 						for (int t = 0; t < MT; ++t)
 						{
-							const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], b, floatx16{}, 0, 0, 0);
+							const floatx16 c = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
+							const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
 #pragma unroll
 							for (int e = 0; e < 16; ++e)
 							{
-								acc[t][e] = fmaf(dm, s[e], acc[t][e]);
+								acc[t][e] += fmaf(d, first[t][e] + p[t][e], fmaf(d, c[e], dm * s[e]));
+							}
+						}
+					}
+					else
+					{
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+#pragma unroll
+							for (int e = 0; e < 16; ++e)
+							{
+								acc[t][e] = fmaf(d, sum[t][e], acc[t][e]);
 							}
 						}
 					}
@@ -899,19 +909,23 @@ namespace litenn_hip
 					return;
 				}
 #pragma unroll
-				for (int other = 1; other < KS; ++other)
+				for (int t = 0; t < MT; ++t)
 				{
 #pragma unroll
-					for (int t = 0; t < MT; ++t)
+					for (int e = 0; e < 16; e += 4)
 					{
+						floatx4 v[KS];
+						v[0] = floatx4{ acc[t][e], acc[t][e + 1], acc[t][e + 2], acc[t][e + 3] };
 #pragma unroll
-						for (int e = 0; e < 16; e += 4)
+						for (int other = 1; other < KS; ++other)
 						{
-							const float4 v = *(reinterpret_cast<const float4*>(handed + (((other - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane);
-							acc[t][e] += v.x;
-							acc[t][e + 1] += v.y;
-							acc[t][e + 2] += v.z;
-							acc[t][e + 3] += v.w;
+							v[other] = *(reinterpret_cast<const floatx4*>(handed + (((other - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane);
+						}
+						add_in_pairs(v);
+#pragma unroll
+						for (int i = 0; i < 4; ++i)
+						{
+							acc[t][e + i] = v[0][i];
 						}
 					}
 				}
@@ -1070,12 +1084,7 @@ namespace litenn_hip
 			const uint8_t* const frag_from = frags + h * R::kHalf + (r >> 4) * R::kPart + min(r & 15, m - 1) * 16;
 			const uint8_t* const sums_from = frags + R::kSums + h * R::kPart + min(r & 15, m - 1) * 16;
 
-			float acc[NE];
-#pragma unroll
-			for (int e = 0; e < NE; ++e)
-			{
-				acc[e] = 0.0f;
-			}
+			float acc[2][NE] = {}; // of every other chunk
 			u32x4 moving[2][W::kLoads]; // the next two chunks
 			if (c_begin < c_end)
 			{
@@ -1083,7 +1092,7 @@ namespace litenn_hip
 				request_x(c_begin);
 				weights.request(moving[1], min(c_begin + 1, c_end - 1), lane);
 			}
-			const auto step = [&](int c, u32x4 (&arrived)[W::kLoads]) {
+			const auto step = [&](int c, u32x4 (&arrived)[W::kLoads], float (&acc)[NE]) {
 				weights.deposit(arrived, lane);
 				deposit_x(c);
 				request_x(min(c + 1, c_end - 1));
@@ -1093,8 +1102,7 @@ namespace litenn_hip
 				const typename F::Head head = F::head(chunk, h);
 				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
 				floatx16 p;
-				half8 sums;
-				float sum[NE];
+				float sum[NE], low[NE]; // low: the low parts', where kScaleSteps is 16
 #pragma unroll
 				for (int st = 0; st < 4; ++st)
 				{
@@ -1109,16 +1117,11 @@ namespace litenn_hip
 						{
 							if (s == 3)
 							{
-								if (st == 3)
-								{
-									sums = r < 16 ? *reinterpret_cast<const half8*>(sums_from) : half8{}; // (into the high parts' rows alone)
-									p = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, for_sums(F::centre_frag(head), h), p, 0, 0, 0);
-								}
 #pragma unroll
 								for (int e = 0; e < NE; ++e)
 								{
-									const float both = fmaf(p[e + 8], kLowScale, p[e]);
-									sum[e] = st == 0 ? both : sum[e] + both;
+									sum[e] = st == 0 ? p[e] : sum[e] + p[e];
+									low[e] = st == 0 ? p[e + 8] : low[e] + p[e + 8];
 								}
 							}
 						}
@@ -1152,12 +1155,14 @@ namespace litenn_hip
 				const float d = F::chunk_scale(head);
 				if constexpr (F::kMins)
 				{
+					const half8 sums = r < 16 ? *reinterpret_cast<const half8*>(sums_from) : half8{}; // (into the high parts' rows alone)
+					const floatx16 centre = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, for_sums(F::centre_frag(head), h), floatx16{}, 0, 0, 0);
 					const floatx16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums, for_sums(F::min_frag(head), h), floatx16{}, 0, 0, 0);
 					const float dm = F::min_scale(head) * (1.0f / kSumScale);
 #pragma unroll
 					for (int e = 0; e < NE; ++e)
 					{
-						sum[e] = fmaf(dm, s[e], d * sum[e]);
+						sum[e] = fmaf(d, fmaf(low[e], kLowScale, sum[e]), fmaf(d, centre[e], dm * s[e]));
 					}
 				}
 				else
@@ -1179,10 +1184,10 @@ namespace litenn_hip
 			};
 			for (int c = c_begin; c < c_end; c += 2)
 			{
-				step(c, moving[0]);
+				step(c, moving[0], acc[0]);
 				if (c + 1 < c_end)
 				{
-					step(c + 1, moving[1]);
+					step(c + 1, moving[1], acc[1]);
 				}
 			}
 			__syncthreads();
@@ -1193,19 +1198,21 @@ namespace litenn_hip
 				const int row = 8 * (e / 4) + 4 * h + (e & 3);
 				if (row < m)
 				{
-					handed[(part * MR + row) * kTile + r] = acc[e];
+					handed[(part * MR + row) * kTile + r] = acc[0][e] + acc[1][e];
 				}
 			}
 			__syncthreads();
 			for (int i = threadIdx.x; i < m * kTile; i += 64 * KS)
 			{
 				const int row = i / kTile, col = n_base + i % kTile;
-				float v = handed[i];
+				float ranges[KS];
 #pragma unroll
-				for (int p = 1; p < KS; ++p)
+				for (int p = 0; p < KS; ++p)
 				{
-					v += handed[p * MR * kTile + i];
+					ranges[p] = handed[p * MR * kTile + i];
 				}
+				add_in_pairs(ranges);
+				float v = ranges[0];
 				if (col < n)
 				{
 					if constexpr (F::kMins)

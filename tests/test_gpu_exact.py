@@ -187,3 +187,18 @@ def test_a_workspace_is_asked_for_where_one_is_used(hip, m, k, some):
 def test_forms_of_two_tiles_over_several_chunks(hip, fmt, m, n, k):
     """Ranges of three chunks and two (four wavefronts on shared activations), of three, three and two (Q6_K's form)."""
     assert errors(hip, fmt, m, n, k, residual=fmt == Q4_0).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,k", [(3, 256), (3, 4096), (45, 4096)])
+def test_several_rows_are_no_further_off_than_rows_one_by_one(hip, fmt, m, k):
+    """Error against 64 bits, mean of six inputs."""
+    n, many, one = 300, [], []
+    T = hip.Tensor.from_numpy
+    for seed in range(6):
+        wq, x = synth.model_weights(fmt, n, k, 40, seed), synth.activations(m, k, 41, seed)
+        w, want = T(wq), x.astype(np.float64) @ np_decoders.decode(fmt, wq, k).astype(np.float64).T
+        off = lambda got: np.linalg.norm(got - want) / np.linalg.norm(want)
+        many.append(off(hip.mul_mat_q(fmt, w, n, k, T(x), flags=MATMUL_PRECISE).numpy()))
+        one.append(off(np.concatenate([hip.mul_mat_q(fmt, w, n, k, T(x[i:i + 1]), flags=MATMUL_PRECISE).numpy() for i in range(m)])))
+    assert np.mean(many) <= np.mean(one)
