@@ -899,7 +899,7 @@ extern "C" int litenn_hip_mul_mat_q_ws(int dev, int fmt, const void* wq, size_t 
 	// Several rows with Float32 operands share the weights on the matrix cores (csrc/exact.hip) where there is room for
 	// the rows taken apart: in the caller's workspace, or, where none was given, from the device's memory pool.  A
 	// call that finds no room, or whose stream is being captured, streams the weights row by row, which needs none.
-	if (m > kFewRows && exact_gemm_takes(fmt, wq, n, k))
+	if (m > kFewRows && exact_rows_take(m, k) && exact_gemm_takes(fmt, wq, n, k))
 	{
 		const size_t need = exact_scratch_bytes(m, k);
 		StreamScratch scratch(s);
