@@ -641,8 +641,8 @@ namespace litenn_hip
 			else
 			{
 				// Eight wavefronts on a head's rows, one workgroup to a CU, while all of them fit the 256 CUs at once and each wavefront
-				// has two tiles; else four, two workgroups to a CU (us for eight and four: 200 rows on 1000 keys 35 and 39, 16 on
-				// 4000 79 and 105, 128 on 128 19 and 14, 512 on 1024 64 and 47, 1500 on 4000 447 and 401).
+				// has two tiles; else four, two workgroups to a CU (kernel's us for eight and four, every option: 200 rows on 1000
+				// keys 45 and 55, 16 on 4000 112 and 170, 128 on 128 24 and 17, 512 on 1024 84 and 68, 1500 on 4000 667 and 591).
 				const size_t groups = static_cast<size_t>(a.heads) * ((a.rows + 31) / 32);
 				if (groups <= 256 && a.keys >= 512)
 				{

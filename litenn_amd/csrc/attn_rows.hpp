@@ -33,9 +33,9 @@ namespace litenn_hip
 		size_t ldo = 0;
 	};
 
-	// Whether the rows are many enough, and the keys they see, for the tiles to pay (us against the row kernels, 32 heads of
-	// 128: Float16 keys, 12 rows on 100 keys 13 against 20, 32 rows on 32 keys 14 against 13, 8 on 1024 26 against 131;
-	// Float32 keys, 8 rows on 300 keys 37 against 37, heads of 64 24 against 19).
+	// Whether the rows are many enough, and the keys they see, for the tiles to pay (kernel's us against the row kernel's, 32 heads
+	// of 128 over 8: Float16 keys, 8 rows on 96 keys 14.0 against 14.7, 12 on 100 13 against 20, 8 on 1024 31 against 110; Float32
+	// keys, 16 rows on 96 keys 19 against 26, on 300 35 against 71, heads of 64 22.8 against 22.4).
 	inline bool attn_rows_pays(size_t rows, size_t keys, bool f32) { return rows >= (f32 ? 16u : 8u) && keys >= 96; }
 
 	// Returns false, launching nothing, for shapes it does not take: head sizes that are no multiple of 8 or above 128,
