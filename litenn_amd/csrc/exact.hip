@@ -151,7 +151,8 @@ namespace litenn_hip
 				for (int b = 0; b < 2; ++b)
 				{
 					const int block = 2 * st + b;
-					r.d[b] = block < blocks ? load2(chunk + 18 * block) : 0u;
+					const uint32_t d = load2(chunk + 18 * block); // (there, whatever it is: not a branch)
+					r.d[b] = block < blocks ? d : 0u;
 					r.q[b] = load8(chunk + 8 * h, 18 * block + 2);
 				}
 				return r;
@@ -180,7 +181,8 @@ namespace litenn_hip
 				for (int b = 0; b < 2; ++b)
 				{
 					const int block = 2 * st + b;
-					r.d[b] = block < blocks ? load2(chunk + 34 * block) : 0u;
+					const uint32_t d = load2(chunk + 34 * block); // (there, whatever it is: not a branch)
+					r.d[b] = block < blocks ? d : 0u;
 					r.q[2 * b] = load8(chunk + 8 * h, 34 * block + 2);
 					r.q[2 * b + 1] = load8(chunk + 8 * h, 34 * block + 18);
 				}
@@ -629,13 +631,391 @@ namespace litenn_hip
 			__device__ __forceinline__ lds_bytes_t chunk(int lane) const { return (lds_bytes_t)(slot) + (lane & 31) * kStride; }
 		};
 
-		// A wavefront multiplies 32 weight rows by MT tiles of 32 activation rows over one of KS
-		// ranges of K; the KS sums meet in LDS at the end, added in K order.  Two levels of sums, a chunk's and
-		// the range's, keep the rounding of long rows down.  WN wavefronts side by side share the activation
-		// fragments of a range through LDS (two buffers of one 64-element stage, the next two stages travelling
-		// through registers while the current one is multiplied); with WN = 1 nobody shares them and they go to
-		// registers directly, each refilled for the next stage once it has been used.  The raw blocks of the
-		// next chunk travel through registers into the wavefront's slot meanwhile.
+		// What of the product a workgroup and its wavefront take, and the way out of their sums: shared by both forms below.
+		// A wavefront multiplies 32 weight rows by MT tiles of 32 activation rows over one of KS ranges of K; the KS sums meet in
+		// LDS at the end, added in K order.  Two levels of sums, a chunk's and the range's, keep the rounding of long rows down.
+		template <typename F, int MT, int WN, int KS>
+		struct ExactPlace
+		{
+			const uint8_t* w;
+			float* y;
+			int n, lane, part, wv, n_base, mt_base, c_begin, c_end, per;
+
+			__device__ __forceinline__ ExactPlace(const ExactMats& mats, int chunks)
+			{
+				int grid_x, grid_y;
+				exact_grid_position(grid_x, grid_y);
+				const int which = (grid_x >= mats.first_block[1]) + (grid_x >= mats.first_block[2]);
+				w = which == 0 ? mats.w[0] : (which == 1 ? mats.w[1] : mats.w[2]);
+				y = which == 0 ? mats.y[0] : (which == 1 ? mats.y[1] : mats.y[2]);
+				n = which == 0 ? mats.n[0] : (which == 1 ? mats.n[1] : mats.n[2]);
+				const int block_x = grid_x - (which == 0 ? 0 : (which == 1 ? mats.first_block[1] : mats.first_block[2]));
+				lane = threadIdx.x & 63;
+				const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+				part = wave / WN, wv = wave % WN;
+				n_base = (block_x * WN + wv) * kTile;
+				mt_base = grid_y * MT;
+				per = (chunks + KS - 1) / KS;
+				c_begin = part * per, c_end = min(c_begin + per, chunks);
+			}
+
+			// the sums of all ranges, scaled, go out; every wavefront of the workgroup calls it
+			__device__ __forceinline__ void finish(floatx16 (&acc)[MT], uint8_t* lds, const uint8_t* xs, const RowsLayout& at, const float* residual,
+			                                       int m, int chunks, size_t row_bytes) const
+			{
+				const int r = lane & 31, h = lane >> 5;
+				if constexpr (KS > 1)
+				{
+					// ranges 1 .. KS - 1 hand their sums to range 0
+					__syncthreads();
+					floatx16* const handed = reinterpret_cast<floatx16*>(lds);
+					if (part > 0)
+					{
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+#pragma unroll
+							for (int e = 0; e < 16; e += 4)
+							{
+								float4* dst = reinterpret_cast<float4*>(handed + (((part - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane;
+								*dst = float4{ acc[t][e], acc[t][e + 1], acc[t][e + 2], acc[t][e + 3] };
+							}
+						}
+					}
+					__syncthreads();
+					if (part > 0)
+					{
+						return;
+					}
+#pragma unroll
+					for (int t = 0; t < MT; ++t)
+					{
+#pragma unroll
+						for (int e = 0; e < 16; e += 4)
+						{
+							floatx4 v[KS];
+							v[0] = floatx4{ acc[t][e], acc[t][e + 1], acc[t][e + 2], acc[t][e + 3] };
+#pragma unroll
+							for (int other = 1; other < KS; ++other)
+							{
+								v[other] = *(reinterpret_cast<const floatx4*>(handed + (((other - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane);
+							}
+							add_in_pairs(v);
+#pragma unroll
+							for (int i = 0; i < 4; ++i)
+							{
+								acc[t][e + i] = v[0][i];
+							}
+						}
+					}
+				}
+
+				// lane (r, h) holds weight row r and activation rows 8 (e / 4) + 4 h + e % 4.  Everything is asked for before the first
+				// store: a factor and a residual at a time, each waited for, were 10 us of every workgroup.
+				const float* factors = reinterpret_cast<const float*>(xs + at.factors);
+				const int col = n_base + r;
+				uint32_t again = 0; // results that are not finite
+#pragma unroll
+				for (int t = 0; t < MT; ++t)
+				{
+					const int first = (mt_base + t) * kTile + 4 * h;
+					if ((mt_base + t) * kTile >= m)
+					{
+						break;
+					}
+					floatx4 us[4];
+					float res[16];
+#pragma unroll
+					for (int e = 0; e < 16; e += 4)
+					{
+						us[e / 4] = *reinterpret_cast<const floatx4*>(factors + first + 2 * e);
+					}
+					if (residual)
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							res[e] = residual[static_cast<size_t>(min(first + 8 * (e / 4) + (e & 3), m - 1)) * n + min(col, n - 1)];
+						}
+					}
+					if (col < n)
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							const int mm = first + 8 * (e / 4) + (e & 3);
+							if (mm < m)
+							{
+								if (F::kMins && !(fabsf(acc[t][e]) <= 3.402823466e38f))
+								{
+									again |= 1u << (16 * t + e);
+									continue;
+								}
+								const float v = acc[t][e] * us[e / 4][e & 3];
+								y[static_cast<size_t>(mm) * n + col] = residual ? res[e] + v : v;
+							}
+						}
+					}
+				}
+				if constexpr (F::kMins)
+				{
+					while (__builtin_expect(again != 0, 0))
+					{
+						const int i = __ffs(again) - 1, e = i & 15, mm = (mt_base + (i >> 4)) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
+						again &= again - 1;
+						const uint8_t* const parts = xs + static_cast<size_t>(mm / kTile) * chunks * kTileChunkBytes + (mm % kTile) * 16;
+						const float v = factors[mm] * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
+							const uint8_t* const at = parts + static_cast<size_t>(i >> 4) * (2 * kFrag) + ((i >> 3) & 1) * 512 + (i & 7) * 2;
+							return fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(at + kFrag)), kLowScale, static_cast<float>(*reinterpret_cast<const _Float16*>(at)));
+						});
+						const size_t o = static_cast<size_t>(mm) * n + col;
+						y[o] = residual ? residual[o] + v : v;
+					}
+				}
+			}
+		};
+
+		// WN wavefronts side by side share the activation fragments of a range through LDS: two buffers of one 64-element stage,
+		// the next stage travelling through registers while the current one is multiplied.  The raw blocks of the next
+		// chunk travel through registers into the wavefront's slot meanwhile.  What a step of 16 elements multiplies is in
+		// registers when it begins: the step before asks for its activations ahead of its own products and decodes its
+		// weights behind them, and a stage's last products follow the barrier, so that they cover the next stage's first reads.
+		template <typename F, int MT, int WN, int KS>
+		__global__ __launch_bounds__(64 * WN * KS) void exact_shared_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
+		                                                                    const float* residual, int k, int m, int m_tiles,
+		                                                                    int chunks, size_t row_bytes)
+		{
+			constexpr int kPieces = MT * 8 / WN; // 1 KB pieces a wavefront stages
+			static_assert(kPieces * WN == MT * 8, "activation pieces / wavefront split");
+			typedef WeightPieces<F> W;
+			constexpr int kRingBytes = KS * 2 * MT * kStageBytes;
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
+			const ExactPlace<F, MT, WN, KS> place(mats, chunks);
+			const int lane = place.lane, h = lane >> 5;
+			const int c_begin = place.c_begin, c_end = place.c_end;
+			const W weights(lds + kRingBytes + (place.part * WN + place.wv) * W::kSlotBytes, place.w, place.n_base, place.n, row_bytes);
+			u32x4 moving[W::kLoads];
+
+			const RowsLayout at(m_tiles, chunks);
+			const uint8_t* sum_tiles[MT];
+#pragma unroll
+			for (int t = 0; t < MT; ++t)
+			{
+				sum_tiles[t] = xs + at.sums + static_cast<size_t>(min(place.mt_base + t, m_tiles - 1)) * chunks * kFrag + lane * 16;
+			}
+
+			floatx16 acc[MT], p[MT];
+			floatx16 held[MT]; // the chunk's sums so far or, where one scale is all of it, its first half
+#pragma unroll
+			for (int t = 0; t < MT; ++t)
+			{
+				acc[t] = floatx16{};
+			}
+
+			u32x4 staged[kPieces]; // the next stage on its way
+			uint8_t* const ring = lds + place.part * (2 * MT * kStageBytes);
+			const uint8_t* from[kPieces];
+#pragma unroll
+			for (int i = 0; i < kPieces; ++i)
+			{
+				const int piece = i * WN + place.wv;
+				from[i] = xs + static_cast<size_t>(min(place.mt_base + (piece >> 3), m_tiles - 1)) * chunks * kTileChunkBytes + (piece & 7) * kFrag;
+			}
+			const auto request = [&](u32x4 (&into)[kPieces], int c, int st) {
+#pragma unroll
+				for (int i = 0; i < kPieces; ++i)
+				{
+					into[i] = *reinterpret_cast<const u32x4*>(from[i] + static_cast<size_t>(c) * kTileChunkBytes + st * kStageBytes + lane * 16);
+				}
+			};
+			const auto deposit = [&](const u32x4 (&from)[kPieces], int buffer) {
+#pragma unroll
+				for (int i = 0; i < kPieces; ++i)
+				{
+					*reinterpret_cast<u32x4*>(ring + buffer * (MT * kStageBytes) + (i * WN + place.wv) * kFrag + lane * 16) = from[i];
+				}
+			};
+
+			half8 a[2][MT][2], b[2]; // of this step and the next
+			const auto read = [&](int buffer, int s, int into) {
+#pragma unroll
+				for (int t = 0; t < MT; ++t)
+				{
+#pragma unroll
+					for (int e = 0; e < 2; ++e)
+					{
+						a[into][t][e] = *reinterpret_cast<const half8*>(ring + buffer * (MT * kStageBytes) + t * kStageBytes + (2 * s + e) * kFrag + lane * 16);
+					}
+				}
+			};
+
+			typename F::Head head, next_head;
+			typename F::Raw raw, next_raw;
+			const auto blocks_of = [&](int c) { return k / F::kBlock - c * (kChunk / F::kBlock); };
+			if (c_begin < c_end)
+			{
+				weights.request(moving, c_begin, lane);
+				request(staged, c_begin, 0);
+				weights.deposit(moving, lane);
+				deposit(staged, 0);
+				request(staged, c_begin, 1);
+				weights.request(moving, min(c_begin + 1, c_end - 1), lane);
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+			}
+			__syncthreads();
+			if (c_begin < c_end)
+			{
+				head = F::head(weights.chunk(lane), h);
+				raw = F::load(weights.chunk(lane), 0, h, blocks_of(c_begin));
+				read(0, 0, 0);
+				b[0] = F::frag(head, raw, 0, 0);
+			}
+			for (int c = c_begin; c < c_end; ++c)
+			{
+				const int next = min(c + 1, c_end - 1);
+				half8 sum_frag[MT];
+#pragma unroll
+				for (int st = 0; st < 4; ++st)
+				{
+#pragma unroll
+					for (int s = 0; s < 4; ++s)
+					{
+						const int step = 4 * st + s, mine = s & 1, other = mine ^ 1;
+						if (s < 3)
+						{
+							read(st & 1, s + 1, other);
+						}
+						if (s == 0)
+						{
+							// (the buffer was read last before the barrier that this stage began with)
+							deposit(staged, (st + 1) & 1);
+							request(staged, st < 2 ? c : next, (st + 2) & 3);
+							if (st == 3)
+							{
+								// (a wavefront's LDS accesses keep their order: the slot's reads, the next chunk, its reads)
+								__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+								weights.deposit(moving, lane);
+								__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+								weights.request(moving, min(c + 2, c_end - 1), lane);
+							}
+						}
+						if (F::kMins && step == 11)
+						{
+#pragma unroll
+							for (int t = 0; t < MT; ++t)
+							{
+								sum_frag[t] = *reinterpret_cast<const half8*>(sum_tiles[t] + static_cast<size_t>(c) * kFrag);
+							}
+						}
+						if (s == 2)
+						{
+							if (st == 3)
+							{
+								next_head = F::head(weights.chunk(lane), h);
+							}
+							next_raw = F::load(weights.chunk(lane), (st + 1) & 3, h, blocks_of(st < 3 ? c : next));
+						}
+						if (s == 3)
+						{
+							__syncthreads();
+							read((st + 1) & 1, 0, other);
+						}
+						__builtin_amdgcn_sched_barrier(0);
+						const half8 low = lowered(b[mine]);
+						const bool fresh = step % min(F::kScaleSteps, 8) == 0;
+#pragma unroll
+						for (int e = 0; e < 2; ++e)
+						{
+#pragma unroll
+							for (int t = 0; t < MT; ++t)
+							{
+								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mine][t][e], e == 0 ? b[mine] : low, fresh && e == 0 ? floatx16{} : p[t], 0, 0, 0);
+							}
+						}
+						if (s < 3)
+						{
+							b[other] = F::frag(head, raw, st, s + 1);
+						}
+						else
+						{
+							b[other] = F::frag(st < 3 ? head : next_head, next_raw, (st + 1) & 3, 0);
+						}
+						if constexpr (F::kMins)
+						{
+							if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
+							{
+#pragma unroll
+								for (int t = 0; t < MT; ++t)
+								{
+									held[t] = p[t];
+								}
+							}
+						}
+						if constexpr (F::kScaleSteps < 16)
+						{
+							if (step % F::kScaleSteps == F::kScaleSteps - 1)
+							{
+								const float d = F::scale(head, raw, st, s);
+#pragma unroll
+								for (int t = 0; t < MT; ++t)
+								{
+#pragma unroll
+									for (int e = 0; e < 16; ++e)
+									{
+										held[t][e] = step == F::kScaleSteps - 1 ? d * p[t][e] : fmaf(d, p[t][e], held[t][e]);
+									}
+								}
+							}
+						}
+						__builtin_amdgcn_sched_barrier(0);
+					}
+					raw = next_raw;
+				}
+				const float d = F::chunk_scale(head);
+				if constexpr (F::kMins)
+				{
+					const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
+					const float dm = F::min_scale(head) * (1.0f / kSumScale);
+#pragma unroll
+					for (int t = 0; t < MT; ++t)
+					{
+						const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
+						const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
+						}
+					}
+				}
+				else
+				{
+#pragma unroll
+					for (int t = 0; t < MT; ++t)
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							acc[t][e] = fmaf(d, held[t][e], acc[t][e]);
+						}
+					}
+				}
+				head = next_head;
+			}
+			// a shorter range only passes the barriers
+			for (int i = max(c_end - c_begin, 0); i < place.per; ++i)
+			{
+#pragma unroll
+				for (int st = 0; st < 4; ++st)
+				{
+					__syncthreads();
+				}
+			}
+			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes);
+		}
+
+		// The same with less held ahead.  WN > 1: the fragments pass through the same two buffers, two stages on their way; with WN =
+		// 1 nobody shares them and they go to registers directly, each refilled for the next stage once it has been used.
 		template <typename F, int MT, int WN, int KS>
 		__global__ __launch_bounds__(64 * WN * KS) void exact_gemm_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                  const float* residual, int k, int m, int m_tiles,
@@ -647,23 +1027,11 @@ namespace litenn_hip
 			typedef WeightPieces<F> W;
 			constexpr int kRingBytes = kShared ? KS * 2 * MT * kStageBytes : 0;
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
-			int grid_x, grid_y;
-			exact_grid_position(grid_x, grid_y);
-			const int which = (grid_x >= mats.first_block[1]) + (grid_x >= mats.first_block[2]);
-			const uint8_t* w = which == 0 ? mats.w[0] : (which == 1 ? mats.w[1] : mats.w[2]);
-			float* y = which == 0 ? mats.y[0] : (which == 1 ? mats.y[1] : mats.y[2]);
-			const int n = which == 0 ? mats.n[0] : (which == 1 ? mats.n[1] : mats.n[2]);
-			const int block_x = grid_x - (which == 0 ? 0 : (which == 1 ? mats.first_block[1] : mats.first_block[2]));
-			const int lane = threadIdx.x & 63;
-			const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-			const int part = wave / WN, wv = wave % WN;
-			const int r = lane & 31, h = lane >> 5;
-			const int n_base = (block_x * WN + wv) * kTile;
-			const int mt_base = grid_y * MT;
-			const int per = (chunks + KS - 1) / KS;
-			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
+			const ExactPlace<F, MT, WN, KS> place(mats, chunks);
+			const int lane = place.lane, part = place.part, wv = place.wv, h = lane >> 5, mt_base = place.mt_base;
+			const int c_begin = place.c_begin, c_end = place.c_end, per = place.per;
 
-			const W weights(lds + kRingBytes + wave * W::kSlotBytes, w, n_base, n, row_bytes);
+			const W weights(lds + kRingBytes + (part * WN + wv) * W::kSlotBytes, place.w, place.n_base, place.n, row_bytes);
 			u32x4 moving[W::kLoads];
 
 			const RowsLayout at(m_tiles, chunks);
@@ -885,100 +1253,7 @@ namespace litenn_hip
 				}
 			}
 
-			if constexpr (KS > 1)
-			{
-				// ranges 1 .. KS - 1 hand their sums to range 0
-				__syncthreads();
-				floatx16* const handed = reinterpret_cast<floatx16*>(lds);
-				if (part > 0)
-				{
-#pragma unroll
-					for (int t = 0; t < MT; ++t)
-					{
-#pragma unroll
-						for (int e = 0; e < 16; e += 4)
-						{
-							float4* dst = reinterpret_cast<float4*>(handed + (((part - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane;
-							*dst = float4{ acc[t][e], acc[t][e + 1], acc[t][e + 2], acc[t][e + 3] };
-						}
-					}
-				}
-				__syncthreads();
-				if (part > 0)
-				{
-					return;
-				}
-#pragma unroll
-				for (int t = 0; t < MT; ++t)
-				{
-#pragma unroll
-					for (int e = 0; e < 16; e += 4)
-					{
-						floatx4 v[KS];
-						v[0] = floatx4{ acc[t][e], acc[t][e + 1], acc[t][e + 2], acc[t][e + 3] };
-#pragma unroll
-						for (int other = 1; other < KS; ++other)
-						{
-							v[other] = *(reinterpret_cast<const floatx4*>(handed + (((other - 1) * WN + wv) * MT + t) * 64) + (e / 4) * 64 + lane);
-						}
-						add_in_pairs(v);
-#pragma unroll
-						for (int i = 0; i < 4; ++i)
-						{
-							acc[t][e + i] = v[0][i];
-						}
-					}
-				}
-			}
-
-			// lane (r, h) holds weight row r and activation rows 8 (e / 4) + 4 h + e % 4
-			const float* factors = reinterpret_cast<const float*>(xs + at.factors);
-			uint32_t again = 0; // results that are not finite
-#pragma unroll
-			for (int t = 0; t < MT; ++t)
-			{
-#pragma unroll
-				for (int e = 0; e < 16; ++e)
-				{
-					const int mm = (mt_base + t) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
-					if (mm < m)
-					{
-						const float us = factors[mm];
-						const int col = n_base + r;
-						if (col < n)
-						{
-							const size_t o = static_cast<size_t>(mm) * n + col;
-							if (F::kMins && !(fabsf(acc[t][e]) <= 3.402823466e38f))
-							{
-								again |= 1u << (16 * t + e);
-								continue;
-							}
-							float v = acc[t][e] * us;
-							if (residual)
-							{
-								v = residual[o] + v;
-							}
-							y[o] = v;
-						}
-					}
-				}
-			}
-			if constexpr (F::kMins)
-			{
-				const int col = n_base + r;
-				while (__builtin_expect(again != 0, 0))
-				{
-					const int i = __ffs(again) - 1, e = i & 15, mm = (mt_base + (i >> 4)) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
-					again &= again - 1;
-					const uint8_t* const parts = xs + static_cast<size_t>(mm / kTile) * chunks * kTileChunkBytes + (mm % kTile) * 16;
-					const float v = factors[mm] * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
-						const uint8_t* const at = parts + static_cast<size_t>(i >> 4) * (2 * kFrag) + ((i >> 3) & 1) * 512 + (i & 7) * 2;
-						return fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(at + kFrag)), kLowScale, static_cast<float>(*reinterpret_cast<const _Float16*>(at)));
-					});
-					const size_t o = static_cast<size_t>(mm) * n + col;
-					y[o] = residual ? residual[o] + v : v;
-				}
-			}
+			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes);
 		}
 
 		// ---- few rows: up to MR activation rows, one launch, no scratch ---------------------------------
@@ -1243,6 +1518,21 @@ namespace litenn_hip
 			hipStream_t stream;
 		};
 
+		// Four wavefronts over one chunk's scale have the registers to hold two steps' operands (Q4_K 28672 x 4096 at 300 rows 253
+		// -> 238 us); sums that are scaled every step or two have not.
+		template <typename F, int MT, int WN, int KS>
+		constexpr auto variant()
+		{
+			if constexpr (WN > 1 && F::kMins)
+			{
+				return &exact_shared_kernel<F, MT, WN, KS>;
+			}
+			else
+			{
+				return &exact_gemm_kernel<F, MT, WN, KS>;
+			}
+		}
+
 		template <typename F, int MT, int WN, int KS>
 		void launch_variant(const ExactCall& c)
 		{
@@ -1265,9 +1555,9 @@ namespace litenn_hip
 					blocks += (c.n[i] + WN * kTile - 1) / (WN * kTile);
 				}
 			}
-			const auto kernel = &exact_gemm_kernel<F, MT, WN, KS>;
+			const auto kernel = variant<F, MT, WN, KS>();
 			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
-			exact_gemm_kernel<F, MT, WN, KS><<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
+			kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
 			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
 		}
 
@@ -1276,7 +1566,7 @@ namespace litenn_hip
 		{
 			const int strips = (c.total_rows + kTile - 1) / kTile, units = strips * c.m_tiles;
 			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each
-			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 262 against 301 of the
+			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 238 against 301 of the
 			// forms below, at 64 rows 53 against 62.  Not for Q6_K, whose scaling per step wants the registers.
 			if constexpr (F::kScaleSteps > 1)
 			{
