@@ -359,17 +359,19 @@ namespace litenn_hip
 			}
 		};
 
-		constexpr int kHeldItems = 8; // 8-element items of a row per thread: rows up to 16384 wide
+		constexpr int kMostItems = 2048; // 8-element items of a row: rows up to 16384 wide
 
 		// One workgroup per row.  The producers of csrc/gemm.hip's pre-pass may run first: RMSNorm with f64
 		// accumulation (norm_w) or SwiGLU's silu(x) * up.
-		__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
+		template <int T>
+		__global__ __launch_bounds__(T) void split_rows_kernel(const float* __restrict__ x, uint8_t* __restrict__ out,
 		                                                         int m, int m_pad, int k, int chunks,
 		                                                         const float* __restrict__ norm_w, double eps,
 		                                                         const float* __restrict__ up)
 		{
-			__shared__ float red[4];
-			__shared__ double red64[4];
+			constexpr int kHeldItems = kMostItems / T, kWaves = T / 64;
+			__shared__ float red[kWaves];
+			__shared__ double red64[kWaves];
 			// eight rows share every 128-byte line of the layout: XCD x (workgroups are dealt out round-robin)
 			// takes the row octets x, x + 8, ... so that its L2 puts whole lines together
 			const int xcd = blockIdx.x & 7, nth = blockIdx.x >> 3;
@@ -390,7 +392,7 @@ namespace litenn_hip
 #pragma unroll
 			for (int u = 0; u < kHeldItems; ++u)
 			{
-				const int it = threadIdx.x + 256 * u;
+				const int it = threadIdx.x + T * u;
 #pragma unroll
 				for (int e = 0; e < 8; ++e)
 				{
@@ -435,12 +437,17 @@ namespace litenn_hip
 					red64[threadIdx.x >> 6] = ss;
 				}
 				__syncthreads();
-				const double total = red64[0] + red64[1] + red64[2] + red64[3];
+				double total = red64[0];
+#pragma unroll
+				for (int i = 1; i < kWaves; ++i)
+				{
+					total += red64[i];
+				}
 				const double inv = 1.0 / sqrt(total / static_cast<double>(k) + eps);
 #pragma unroll
 				for (int u = 0; u < kHeldItems; ++u)
 				{
-					const int it = threadIdx.x + 256 * u;
+					const int it = threadIdx.x + T * u;
 					if (row < m && 8 * it < k)
 					{
 						const float4 wa = *reinterpret_cast<const float4*>(norm_w + 8 * it);
@@ -471,13 +478,17 @@ namespace litenn_hip
 				red[threadIdx.x >> 6] = mx;
 			}
 			__syncthreads();
-			mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+#pragma unroll
+			for (int i = 0; i < kWaves; ++i)
+			{
+				mx = fmaxf(mx, red[i]);
+			}
 			// x 2^shift has its largest magnitude in [2^14, 2^15); the inverse stays a normal number
 			const int shift = mx > 0.0f ? min(14 - ilogbf(mx), 126) : 0;
 #pragma unroll
 			for (int u = 0; u < kHeldItems; ++u)
 			{
-				const int it = threadIdx.x + 256 * u;
+				const int it = threadIdx.x + T * u;
 				double sum = 0.0;
 				if (it < items)
 				{
@@ -1655,7 +1666,7 @@ namespace litenn_hip
 	// Whether launch_exact_rows takes rows of this number and width.
 	bool exact_rows_take(size_t m, size_t k)
 	{
-		return m > 0 && m <= (size_t{ 1 } << 20) && k > 0 && k % 32 == 0 && k <= static_cast<size_t>(kHeldItems) * 256 * 8;
+		return m > 0 && m <= (size_t{ 1 } << 20) && k > 0 && k % 32 == 0 && k <= static_cast<size_t>(kMostItems) * 8;
 	}
 
 	// Whether launch_exact_gemm takes a matrix: one of the formats above, rows that start on 2 bytes.
@@ -1682,8 +1693,21 @@ namespace litenn_hip
 		}
 		const int chunks = static_cast<int>((k + kChunk - 1) / kChunk);
 		const int m_pad = static_cast<int>((m + kTile - 1) / kTile * kTile);
-		split_rows_kernel<<<dim3(static_cast<unsigned>((m_pad + 63) / 64 * 64)), dim3(256), 0, stream>>>(
-		    x, static_cast<uint8_t*>(scratch), static_cast<int>(m), m_pad, static_cast<int>(k), chunks, norm_w, eps, up);
+		const auto launch = [&](auto kernel, int threads) {
+			kernel<<<dim3(static_cast<unsigned>((m_pad + 63) / 64 * 64)), dim3(threads), 0, stream>>>(
+			    x, static_cast<uint8_t*>(scratch), static_cast<int>(m), m_pad, static_cast<int>(k), chunks, norm_w, eps, up);
+		};
+		// Few rows leave a workgroup a CU to itself: more threads, fewer elements in a chain (us, 256 / 512 / 1024 threads: 64
+		// rows of 14336 9.9, 7.8, 7.4; 20 rows of 4096 5.5, 4.4, 4.0); many rows share a CU (300 rows of 14336 with SwiGLU 18.4,
+		// 17.8, 18.1, of 4096 8.5, 7.9, 8.4).
+		if (m <= 128)
+		{
+			launch(&split_rows_kernel<1024>, 1024);
+		}
+		else
+		{
+			launch(&split_rows_kernel<512>, 512);
+		}
 		return true;
 	}
 
