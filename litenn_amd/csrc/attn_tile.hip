@@ -12,7 +12,7 @@
 // output) triples are merged once at the end.
 //
 //   S^T[key, q]  = K[key, :] . Q[q, :]        A = key tile (row-major in LDS), B = Q (registers)
-//   O^T[d, q]   += V^T[d, key] . P^T[key, q]  A = value tile staged dimension-major, B = P
+//   O^T[d, q]   += V^T[d, key] . P^T[key, q]  A = value tile (row-major in LDS, read transposed), B = P
 //
 // Computing the transposed products keeps the query in the lane index of every result, so
 // the softmax weights leave the first contraction in exactly the register layout the second
@@ -43,7 +43,9 @@ namespace litenn_hip
 		constexpr int kKeyTile = 64;   // keys staged per step
 		constexpr int kDim = 128;      // head width this kernel is written for
 		constexpr int kKStride = 136;  // halves between staged key rows: 16 rows x 16 bytes fall on 64 distinct banks
-		constexpr int kVtStride = 72;  // halves between staged value columns (dimension-major)
+		// A staged value row is kDim halves, its 32-byte columns permuted by the row: sixteen lanes read 32 bytes of four
+		// neighbouring rows, 32 lanes of eight, which then cover all banks.
+		__device__ __forceinline__ int value_at(int key, int piece) { return key * kDim + ((piece ^ ((key & 7) << 1)) << 3); }
 
 		__device__ __forceinline__ half2v pack2(float a, float b)
 		{
@@ -51,8 +53,9 @@ namespace litenn_hip
 			return __builtin_convertvector(f, half2v); // v_cvt_pk_f16_f32
 		}
 
-		constexpr int kTileHalves = kKeyTile * kKStride + kDim * kVtStride; // one half's key + value buffers
+		constexpr int kTileHalves = kKeyTile * kKStride + kKeyTile * kDim; // one half's key + value buffers
 		constexpr size_t kAttnTileLds = 2 * kTileHalves * sizeof(_Float16);
+		static_assert((8 * 1024 + 512) * sizeof(float) <= kAttnTileLds, "the halves' results");
 
 		__global__ __launch_bounds__(512) void attn_tile_kernel(const float* __restrict__ q,
 		                                                         const uint16_t* __restrict__ kcache,
@@ -64,7 +67,7 @@ namespace litenn_hip
 			extern __shared__ __attribute__((aligned(16))) _Float16 attn_lds[];
 			const int part = threadIdx.x >> 8; // which half of the workgroup: key tiles part, part + 2, ...
 			_Float16* const k_lds = attn_lds + part * kTileHalves;
-			_Float16* const vt_lds = k_lds + kKeyTile * kKStride;
+			_Float16* const v_lds = k_lds + kKeyTile * kKStride;
 			const int tid = threadIdx.x & 255;
 			const int lane = tid & 63;
 			const int wave = tid >> 6;
@@ -102,26 +105,19 @@ namespace litenn_hip
 				q_frag[st] = half8{ p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y };
 			}
 			const int my_limit = past + my_q_clamped; // last key position this query sees
+			const int first_limit = past + min(q_first + 16 * __builtin_amdgcn_readfirstlane(wave), m - 1); // and the wavefront's first
 
-			// staging: keys row-major (thread = 16-byte piece of a key row, consecutive lanes consecutive
-			// pieces), values dimension-major (thread = one key, 64 consecutive bytes of its row)
+			// staging, row-major: thread = 16-byte piece of a row, consecutive lanes consecutive pieces
 			u32x4 k_reg[4], v_reg[4];
-			const int v_key = tid & 63;
-			const int v_part0 = (tid >> 6) * 4;
 			const auto fetch = [&](int kt) {
 #pragma unroll
 				for (int i = 0; i < 4; ++i)
 				{
 					const int c = tid + 256 * i;
 					const int key = fetch::attn_tile_key(kt, kKeyTile, c >> 4, kv_len);
-					k_reg[i] = *reinterpret_cast<const u32x4*>(kbase + static_cast<size_t>(key) * kvw + (c & 15) * 8);
-				}
-				const int key = fetch::attn_tile_key(kt, kKeyTile, v_key, kv_len);
-				const uint16_t* vr = vbase + static_cast<size_t>(key) * kvw + v_part0 * 8;
-#pragma unroll
-				for (int i = 0; i < 4; ++i)
-				{
-					v_reg[i] = *reinterpret_cast<const u32x4*>(vr + 8 * i);
+					const size_t at = static_cast<size_t>(key) * kvw + (c & 15) * 8;
+					k_reg[i] = *reinterpret_cast<const u32x4*>(kbase + at);
+					v_reg[i] = *reinterpret_cast<const u32x4*>(vbase + at);
 				}
 			};
 			const auto stage = [&]() {
@@ -130,20 +126,18 @@ namespace litenn_hip
 				{
 					const int c = tid + 256 * i;
 					*reinterpret_cast<u32x4*>(&k_lds[(c >> 4) * kKStride + (c & 15) * 8]) = k_reg[i];
+					*reinterpret_cast<u32x4*>(&v_lds[value_at(c >> 4, c & 15)]) = v_reg[i];
 				}
-				uint16_t* vt = reinterpret_cast<uint16_t*>(vt_lds);
-#pragma unroll
-				for (int i = 0; i < 4; ++i)
-				{
-					const uint32_t w[4] = { v_reg[i].x, v_reg[i].y, v_reg[i].z, v_reg[i].w };
-#pragma unroll
-					for (int e = 0; e < 4; ++e)
-					{
-						const int d = (v_part0 + i) * 8 + 2 * e;
-						vt[d * kVtStride + v_key] = static_cast<uint16_t>(w[e] & 0xffffu);
-						vt[(d + 1) * kVtStride + v_key] = static_cast<uint16_t>(w[e] >> 16);
-					}
-				}
+			};
+			// Transposed read of four keys of sixteen dimensions: lane j of sixteen names eight bytes of one key's row and gets
+			// the four keys of dimension j.  (Turned on their way into LDS, two bytes at a time, they took a quarter of
+			// the kernel: 1024 rows of 32 heads behind 1024 and behind none, 90 us on average, 70 with this, 63 with masks and
+			// rescaling only in tiles that need them.)
+			const auto values = [&](int key, int db) {
+				typedef short short4v __attribute__((ext_vector_type(4)));
+				typedef __attribute__((address_space(3))) short4v* lds_short4;
+				return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+				    (lds_short4)(&v_lds[value_at(key + (j >> 2), 2 * db + ((j & 3) >> 1)) + (j & 1) * 4])));
 			};
 
 			floatx4 o[8];
@@ -178,19 +172,29 @@ namespace litenn_hip
 						s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, q_frag[st], s[b], 0, 0, 0);
 					}
 				}
-				// causal mask, tile maximum of the query (its keys are spread over four lanes)
+				// causal mask where the tile holds a key that one of the wavefront's queries does not see; the query's maximum (its
+				// keys are spread over four lanes)
 				const int key0 = kt * kKeyTile + 4 * g;
+				if (kt * kKeyTile + kKeyTile - 1 > first_limit || kt >= n_key_tiles)
+				{
+#pragma unroll
+					for (int b = 0; b < 4; ++b)
+					{
+#pragma unroll
+						for (int r = 0; r < 4; ++r)
+						{
+							s[b][r] = (key0 + 16 * b + r <= limit) ? s[b][r] : -INFINITY;
+						}
+					}
+				}
 				float tile_m = -INFINITY;
-				float sv[4][4];
 #pragma unroll
 				for (int b = 0; b < 4; ++b)
 				{
-					const float v4[4] = { s[b].x, s[b].y, s[b].z, s[b].w };
 #pragma unroll
 					for (int r = 0; r < 4; ++r)
 					{
-						sv[b][r] = (key0 + 16 * b + r <= limit) ? v4[r] : -INFINITY;
-						tile_m = fmaxf(tile_m, sv[b][r]);
+						tile_m = fmaxf(tile_m, s[b][r]);
 					}
 				}
 				tile_m = fmaxf(tile_m, __shfl_xor(tile_m, 16, 64));
@@ -209,8 +213,8 @@ namespace litenn_hip
 #pragma unroll
 					for (int r = 0; r < 4; ++r)
 					{
-						p[r] = __expf(sv[2 * ks][r] - ref_m);
-						p[4 + r] = __expf(sv[2 * ks + 1][r] - ref_m);
+						p[r] = __expf(s[2 * ks][r] - ref_m);
+						p[4 + r] = __expf(s[2 * ks + 1][r] - ref_m);
 					}
 #pragma unroll
 					for (int e = 0; e < 8; ++e)
@@ -222,18 +226,23 @@ namespace litenn_hip
 					p_frag[ks] = half8{ p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y };
 				}
 				run_l = fmaf(run_l, corr, sum);
+				if (__any(corr != 1.0f)) // (past the first tiles a maximum seldom moves)
+				{
+#pragma unroll
+					for (int db = 0; db < 8; ++db)
+					{
+						o[db] *= corr;
+					}
+				}
 				// O^T: eight blocks of 16 dimensions; contraction index 8 g + e of step ks stands for
 				// key 16 (2 ks) + 4 g + e (e < 4) and key 16 (2 ks + 1) + 4 g + e - 4 (e >= 4)
 #pragma unroll
 				for (int db = 0; db < 8; ++db)
 				{
-					o[db] *= corr;
 #pragma unroll
 					for (int ks = 0; ks < 2; ++ks)
 					{
-						const _Float16* col = &vt_lds[(16 * db + j) * kVtStride + 32 * ks + 4 * g];
-						const half4 lo = *reinterpret_cast<const half4*>(col);
-						const half4 hi = *reinterpret_cast<const half4*>(col + 16);
+						const half4 lo = values(32 * ks + 4 * g, db), hi = values(32 * ks + 16 + 4 * g, db);
 						const half8 a = half8{ lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w };
 						o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, p_frag[ks], o[db], 0, 0, 0);
 					}
@@ -242,9 +251,9 @@ namespace litenn_hip
 
 			run_l += __shfl_xor(run_l, 16, 64);
 			run_l += __shfl_xor(run_l, 32, 64);
-			// the odd half hands its triple to the even half through its own (now idle) buffers
+			// the odd half hands its triple to the even half through the (now idle) buffers
 			__syncthreads();
-			float* const xch = reinterpret_cast<float*>(attn_lds + kTileHalves);
+			float* const xch = reinterpret_cast<float*>(attn_lds);
 			if (part == 1)
 			{
 #pragma unroll

@@ -643,21 +643,36 @@ namespace litenn_hip
 		}
 
 		// Matrix-core form: a workgroup takes 64 query rows of one head (16 per wavefront) and walks the
-		// keys any of them sees in tiles of 64, staged in LDS (keys row-major, values transposed).  Both
+		// keys any of them sees in tiles of 64, staged row-major in LDS (values are read transposed).  Both
 		// products are formed transposed (keys x queries, value dimensions x queries), so that a query
 		// stays in one lane column: the softmax weights leave the first product in the register layout
 		// the second one takes, and the running maximum and sum live beside the outputs.  DK and DV are the
 		// head sizes rounded up; what lies beyond the true sizes is zero in LDS and in the queries.
-		constexpr int kWinQ = 64, kWinKeys = 64, kWinVStride = 72;
+		constexpr int kWinQ = 64, kWinKeys = 64;
 
-		template <int DK, int DV>
-		__global__ __launch_bounds__(256) void window_attn_tile_kernel(const WindowAttn a)
+		// A staged value row is DV halves, its 32-byte columns permuted by the row: sixteen lanes read 32 bytes of four
+		// neighbouring rows, 32 lanes of eight, which then cover all banks.
+		template <int DV>
+		__device__ __forceinline__ int win_value_at(int key, int piece)
 		{
-			constexpr int KS = DK + 8;
+			constexpr int kSame = DV < 128 ? 128 / DV : 1, kColumns = DV < 128 ? DV / 16 : 8; // rows that lie side by side on the banks
+			return key * DV + ((piece ^ (((key / kSame) & (kColumns - 1)) << 1)) << 3);
+		}
+
+		// PARTS = 2: a workgroup is two halves of four wavefronts, one for the even key tiles and one for the odd ones, each
+		// with its own buffers; their (maximum, sum, outputs) meet at the end.  A query tile is a chain of up to 17 key tiles
+		// otherwise, with one wavefront a SIMD where there are few of them.  us for 777 rows of 16 heads of 128, window 1024, 31.7 ->
+		// 19.2, 2048 rows of 32 heads 114 -> 76: values turned by the LDS read instead of two bytes at a time on their way in,
+		// masks and rescaling only in tiles that need them, queries and gates asked for all at once.
+		template <int DK, int DV, int PARTS>
+		__global__ __launch_bounds__(256 * PARTS) void window_attn_tile_kernel(const WindowAttn a)
+		{
+			constexpr int KS = DK + 8, kPart = kWinKeys * (KS + DV);
 			extern __shared__ __attribute__((aligned(16))) uint16_t win_lds[];
-			uint16_t* const k_lds = win_lds;                 // [kWinKeys][KS]
-			uint16_t* const v_lds = win_lds + kWinKeys * KS; // [DV][kWinVStride]
-			const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+			const int part = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+			uint16_t* const k_lds = win_lds + part * kPart; // [kWinKeys][KS]
+			uint16_t* const v_lds = k_lds + kWinKeys * KS;  // [kWinKeys][DV], permuted
+			const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
 			const int j = lane & 15, g = lane >> 4;
 			const int h = blockIdx.x;
 			const int tile = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y);
@@ -666,6 +681,9 @@ namespace litenn_hip
 			const int my_q = q_first + 16 * wave + j;
 			const int my_row = min(my_q, a.rows - 1);
 			const int my_pos = a.q_base + my_row;
+			// of the wavefront's queries
+			const int wave_q = q_first + 16 * __builtin_amdgcn_readfirstlane(wave);
+			const int first_pos = a.q_base + min(wave_q, a.rows - 1), last_pos = a.q_base + min(wave_q + 15, a.rows - 1);
 			// key rows (relative to key_base) any query of the tile sees
 			const int lo = max(0, a.q_base + q_first - a.shape.window + 1 - a.key_base);
 			const int hi = min(a.keys, a.q_base + min(q_first + kWinQ, a.rows) - a.key_base);
@@ -676,17 +694,38 @@ namespace litenn_hip
 			bf16x8 q_frag[DK / 32];
 			{
 				const float* q = a.q + static_cast<size_t>(my_row) * a.ldq + static_cast<size_t>(h) * dim;
-#pragma unroll
-				for (int st = 0; st < DK / 32; ++st)
+				if ((dim & 7) == 0) // whole groups of eight: all on their way before the first is looked at
 				{
-					uint32_t w[4];
+					floatx4 v[DK / 32][2];
 #pragma unroll
-					for (int e = 0; e < 4; ++e)
+					for (int st = 0; st < DK / 32; ++st)
 					{
-						const int d = 32 * st + 8 * g + 2 * e;
-						w[e] = d < dim ? pack_bf16(q[d], d + 1 < dim ? q[d + 1] : 0.0f) : 0u;
+						const int d = 32 * st + 8 * g;
+						const floatx4_a4* at = reinterpret_cast<const floatx4_a4*>(q + (d < dim ? d : 0));
+						v[st][0] = at[0], v[st][1] = at[1];
 					}
-					q_frag[st] = __builtin_bit_cast(bf16x8, u32x4{ w[0], w[1], w[2], w[3] });
+#pragma unroll
+					for (int st = 0; st < DK / 32; ++st)
+					{
+						const u32x4 w = { pack_bf16(v[st][0].x, v[st][0].y), pack_bf16(v[st][0].z, v[st][0].w),
+							              pack_bf16(v[st][1].x, v[st][1].y), pack_bf16(v[st][1].z, v[st][1].w) };
+						q_frag[st] = __builtin_bit_cast(bf16x8, 32 * st + 8 * g < dim ? w : u32x4{ 0u, 0u, 0u, 0u });
+					}
+				}
+				else
+				{
+#pragma unroll
+					for (int st = 0; st < DK / 32; ++st)
+					{
+						uint32_t w[4];
+#pragma unroll
+						for (int e = 0; e < 4; ++e)
+						{
+							const int d = 32 * st + 8 * g + 2 * e;
+							w[e] = d < dim ? pack_bf16(q[d], d + 1 < dim ? q[d + 1] : 0.0f) : 0u;
+						}
+						q_frag[st] = __builtin_bit_cast(bf16x8, u32x4{ w[0], w[1], w[2], w[3] });
+					}
 				}
 			}
 			floatx4 o[DV / 16];
@@ -697,9 +736,8 @@ namespace litenn_hip
 			}
 			float run_m = -INFINITY, run_l = 0.0f;
 			constexpr int KP = DK / 8, VP = DV / 8;              // 16-byte pieces of a row
-			constexpr int KN = kWinKeys * KP / 256, VN = VP / 4; // pieces a thread stages
+			constexpr int KN = kWinKeys * KP / 256, VN = kWinKeys * VP / 256; // pieces a thread stages
 			u32x4 kr[KN], vr[VN];
-			const int v_key = tid & 63, v_piece = (tid >> 6) * VN;
 			const auto request = [&](int base) {
 #pragma unroll
 				for (int i = 0; i < KN; ++i)
@@ -708,17 +746,19 @@ namespace litenn_hip
 					kr[i] = d < dim ? *reinterpret_cast<const u32x4*>(keys + static_cast<size_t>(window_row(a, key)) * a.ldkv + d)
 					                : u32x4{ 0u, 0u, 0u, 0u };
 				}
-				const uint16_t* v = values + static_cast<size_t>(window_row(a, min(base + v_key, hi - 1))) * a.ldkv;
 #pragma unroll
 				for (int i = 0; i < VN; ++i)
 				{
-					const int e = (v_piece + i) * 8;
-					vr[i] = e < vdim ? *reinterpret_cast<const u32x4*>(v + e) : u32x4{ 0u, 0u, 0u, 0u };
+					const int c = tid + 256 * i, key = min(base + c / VP, hi - 1), e = (c % VP) * 8;
+					vr[i] = e < vdim ? *reinterpret_cast<const u32x4*>(values + static_cast<size_t>(window_row(a, key)) * a.ldkv + e)
+					                 : u32x4{ 0u, 0u, 0u, 0u };
 				}
 			};
-			request(lo);
-			for (int base = lo; base < hi; base += kWinKeys)
+			request(lo + part * kWinKeys);
+			// (a half whose last tile lies behind the last key stages that key again and hides it)
+			for (int from = lo; from < hi; from += PARTS * kWinKeys)
 			{
+				const int base = from + part * kWinKeys;
 				__syncthreads(); // the previous tile has been consumed
 #pragma unroll
 				for (int i = 0; i < KN; ++i)
@@ -729,18 +769,10 @@ namespace litenn_hip
 #pragma unroll
 				for (int i = 0; i < VN; ++i)
 				{
-#pragma unroll
-					for (int e = 0; e < 4; ++e)
-					{
-						const int d = (v_piece + i) * 8 + 2 * e;
-						v_lds[d * kWinVStride + v_key] = static_cast<uint16_t>(vr[i][e] & 0xffffu);
-						v_lds[(d + 1) * kWinVStride + v_key] = static_cast<uint16_t>(vr[i][e] >> 16);
-					}
+					const int c = tid + 256 * i;
+					*reinterpret_cast<u32x4*>(&v_lds[win_value_at<DV>(c / VP, c % VP)]) = vr[i];
 				}
-				if (base + kWinKeys < hi)
-				{
-					request(base + kWinKeys);
-				}
+				request(base + PARTS * kWinKeys);
 				__syncthreads();
 				// lane (j, g) gets keys base + 16 b + 4 g + 0..3 of query j
 				floatx4 s[4];
@@ -755,8 +787,34 @@ namespace litenn_hip
 						s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, q_frag[st], s[b], 0, 0, 0);
 					}
 				}
+				// the mask where the tile holds a key that one of the wavefront's queries does not see
 				const int pos0 = a.key_base + base + 4 * g;
 				float sv[4][4];
+				if (a.key_base + base + kWinKeys - 1 > first_pos || last_pos - (a.key_base + base) >= a.shape.window)
+				{
+#pragma unroll
+					for (int b = 0; b < 4; ++b)
+					{
+#pragma unroll
+						for (int r = 0; r < 4; ++r)
+						{
+							const int back = my_pos - (pos0 + 16 * b + r);
+							sv[b][r] = back >= 0 && back < a.shape.window ? s[b][r] * scale2 : -INFINITY;
+						}
+					}
+				}
+				else
+				{
+#pragma unroll
+					for (int b = 0; b < 4; ++b)
+					{
+#pragma unroll
+						for (int r = 0; r < 4; ++r)
+						{
+							sv[b][r] = s[b][r] * scale2;
+						}
+					}
+				}
 				float top = -INFINITY;
 #pragma unroll
 				for (int b = 0; b < 4; ++b)
@@ -764,8 +822,6 @@ namespace litenn_hip
 #pragma unroll
 					for (int r = 0; r < 4; ++r)
 					{
-						const int back = my_pos - (pos0 + 16 * b + r);
-						sv[b][r] = back >= 0 && back < a.shape.window ? s[b][r] * scale2 : -INFINITY;
 						top = fmaxf(top, sv[b][r]);
 					}
 				}
@@ -797,17 +853,28 @@ namespace litenn_hip
 					                                               pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]) });
 				}
 				run_l = fmaf(run_l, corr, sum);
+				if (__any(corr != 1.0f)) // (past the first tiles a maximum seldom moves)
+				{
+#pragma unroll
+					for (int b = 0; b < DV / 16; ++b)
+					{
+						o[b] *= corr;
+					}
+				}
 				// contraction index 8 g + e of step ks stands for key 16 (2 ks) + 4 g + e (e < 4) and key
 				// 16 (2 ks + 1) + 4 g + e - 4 (e >= 4)
 #pragma unroll
 				for (int b = 0; b < DV / 16; ++b)
 				{
-					o[b] *= corr;
 #pragma unroll
 					for (int ks = 0; ks < 2; ++ks)
 					{
-						const uint16_t* col = &v_lds[(16 * b + j) * kWinVStride + 32 * ks + 4 * g];
-						const uint2 x = *reinterpret_cast<const uint2*>(col), y = *reinterpret_cast<const uint2*>(col + 16);
+						// four keys of sixteen dimensions: lane j of sixteen names eight bytes of a row and gets dimension j
+						typedef short short4v __attribute__((ext_vector_type(4)));
+						typedef __attribute__((address_space(3))) short4v* lds_short4;
+						const int key = 32 * ks + 4 * g + (j >> 2), piece = 2 * b + ((j & 3) >> 1), in = (j & 1) * 4;
+						const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(&v_lds[win_value_at<DV>(key, piece) + in])));
+						const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(&v_lds[win_value_at<DV>(key + 16, piece) + in])));
 						const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{ x.x, x.y, y.x, y.y });
 						o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, p_frag[ks], o[b], 0, 0, 0);
 					}
@@ -815,6 +882,38 @@ namespace litenn_hip
 			}
 			run_l += __shfl_xor(run_l, 16, 64);
 			run_l += __shfl_xor(run_l, 32, 64);
+			if constexpr (PARTS == 2)
+			{
+				static_assert(sizeof(float) * (DV / 16 * 1024 + 512) <= sizeof(uint16_t) * 2 * kPart, "the halves' results");
+				float* const handed = reinterpret_cast<float*>(win_lds);
+				__syncthreads();
+				if (part == 1)
+				{
+#pragma unroll
+					for (int b = 0; b < DV / 16; ++b)
+					{
+						*reinterpret_cast<floatx4*>(handed + (b * 256 + tid) * 4) = o[b];
+					}
+					handed[DV / 16 * 1024 + tid] = run_m;
+					handed[DV / 16 * 1024 + 256 + tid] = run_l;
+				}
+				__syncthreads();
+				if (part == 1)
+				{
+					return;
+				}
+				// (one of the two may not have seen a key of this query)
+				const float other_m = handed[DV / 16 * 1024 + tid], other_l = handed[DV / 16 * 1024 + 256 + tid];
+				const float all_m = fmaxf(run_m, other_m), ref_m = all_m == -INFINITY ? 0.0f : all_m;
+				const float w0 = exp2_f32(run_m - ref_m), w1 = exp2_f32(other_m - ref_m);
+				run_m = all_m;
+				run_l = run_l * w0 + other_l * w1;
+#pragma unroll
+				for (int b = 0; b < DV / 16; ++b)
+				{
+					o[b] = o[b] * w0 + *reinterpret_cast<const floatx4*>(handed + (b * 256 + tid) * 4) * w1;
+				}
+			}
 			if (my_q >= a.rows)
 			{
 				return;
@@ -830,6 +929,27 @@ namespace litenn_hip
 			const float inv = weight / total * a.out_scale;
 			uint16_t* out = static_cast<uint16_t*>(a.out) + static_cast<size_t>(my_q) * a.ldo + static_cast<size_t>(h) * vdim;
 			const float* gate = a.gate ? a.gate + static_cast<size_t>(my_q) * a.ldg + static_cast<size_t>(h) * vdim : nullptr;
+			floatx4 gates[DV / 16];
+			if (gate)
+			{
+				if ((vdim & 3) == 0) // whole groups of four, all on their way at once
+				{
+#pragma unroll
+					for (int b = 0; b < DV / 16; ++b)
+					{
+						const int e = 16 * b + 4 * g;
+						gates[b] = *reinterpret_cast<const floatx4_a4*>(gate + (e < vdim ? e : 0));
+					}
+				}
+				else
+				{
+#pragma unroll
+					for (int b = 0; b < DV / 16; ++b)
+					{
+						gates[b] = load_columns(gate, 16 * b + 4 * g, vdim);
+					}
+				}
+			}
 #pragma unroll
 			for (int b = 0; b < DV / 16; ++b)
 			{
@@ -842,7 +962,7 @@ namespace litenn_hip
 #pragma unroll
 						for (int r = 0; r < 4; ++r)
 						{
-							v[r] *= e + r < vdim ? sigmoid_f32(gate[e + r]) : 0.0f;
+							v[r] *= e + r < vdim ? sigmoid_f32(gates[b][r]) : 0.0f;
 						}
 					}
 					if ((vdim & 3) == 0 && (reinterpret_cast<size_t>(a.out) & 7) == 0)
@@ -1467,10 +1587,22 @@ namespace litenn_hip
 		template <int DK, int DV>
 		void launch_window_tile(const WindowAttn& a, hipStream_t s)
 		{
-			constexpr size_t lds = sizeof(uint16_t) * (kWinKeys * (DK + 8) + DV * kWinVStride);
-			allow_dynamic_lds(reinterpret_cast<const void*>(&window_attn_tile_kernel<DK, DV>), lds);
-			window_attn_tile_kernel<DK, DV>
-			    <<<dim3(a.shape.heads, (a.rows + kWinQ - 1) / kWinQ), dim3(256), lds, s>>>(a);
+			const dim3 grid(a.shape.heads, (a.rows + kWinQ - 1) / kWinQ);
+			const auto launch = [&](auto kernel, int parts) {
+				const size_t lds = sizeof(uint16_t) * parts * kWinKeys * (DK + 8 + DV);
+				allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+				kernel<<<grid, dim3(256 * parts), lds, s>>>(a);
+			};
+			// Two halves where a CU has one workgroup at most (us, one part against two, heads of 128: 208 workgroups 24.7 and 19.2,
+			// 256 22.2 and 19.9, 416 29.8 and 33.6, 1024 76 and 95); wider heads have not the registers for two wavefronts a SIMD.
+			if constexpr (DK <= 128 && DV <= 128)
+			{
+				if (grid.x * static_cast<size_t>(grid.y) <= 256)
+				{
+					return launch(&window_attn_tile_kernel<DK, DV, 2>, 2);
+				}
+			}
+			launch(&window_attn_tile_kernel<DK, DV, 1>, 1);
 		}
 
 		template <int DK>

@@ -235,3 +235,12 @@ def test_gla_step(hip, heads, dim, vdim, rank):
 def test_gla_bfloat16_output_only_rounds_the_result(hip):
     run, _, _keep, _, gated, _ = gla_case(hip, 80, 2, 44, 32, 11, 6.0, (-1.0, 4.0))
     assert rel_l2(bf16_values(hip, run(True, DT_BF16)), gated) <= 3e-3
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(1, 128, 128), (3, 30, 50), (5, 24, 126), (9, 128, 72)])
+@pytest.mark.parametrize("m,keys,window", [(63, 63, 40), (65, 129, 64), (192, 257, 193), (2000, 2000, 150), (1900, 1964, 5000)])
+def test_window_attention_of_few_and_many_workgroups(hip, m, keys, window, heads, dim, vdim):
+    """Up to 256 tiles of 64 queries the key tiles are halved among a workgroup's wavefronts, beyond they are not: odd and
+    even numbers of key tiles, queries whose keys all lie in one half, heads that are no whole pieces."""
+    got, plain = window_case(hip, DT_BF16, m, keys, heads, dim, vdim, window, 0, keys - m, dim ** -0.5)
+    assert rel_l2(got, plain()) <= WINDOW_LIMIT[DT_BF16]
