@@ -10,6 +10,8 @@
 #include <algorithm>
 #include <type_traits>
 
+#pragma clang diagnostic ignored "-Winline-asm" // m0 is named as clobbered although it is reserved
+
 namespace litenn_hip
 {
 	namespace
@@ -721,6 +723,169 @@ namespace litenn_hip
 			}
 		}
 
+		// ------------------------------------------------------------------
+		// The same product of bfloat16 operands that lie on 16 bytes: tiles of K go from memory into a ring of S buffers in LDS
+		// directly (global_load_lds_dwordx4: 8 rows of 128 bytes at a time, lane l fills bytes 16 l, so it is the address that
+		// is permuted), and a wavefront's fragments of half a tile are read while the other half is multiplied.  One barrier a
+		// tile, in its middle: behind it the next tile is there and this one's buffer is free.  Outputs are the chains of
+		// products over K that dense_tile_kernel forms, bit for bit.
+		//
+		// What bounds it: small tiles, the rate at which a CU takes operands from L2 (70 to 80 GB/s a CU, about 30 bytes a cycle;
+		// a ring twice as deep changes nothing); large ones, the products (256 x 256 on 2048 x 28672 x 4096: 1125 TFLOP/s).  us
+		// against dense_tile_kernel: 2048 rows by 28672 x 4096 527 -> 427, by 4096 x 4096 79 -> 63, 777 rows by 2048 x 5632 45 ->
+		// 32, by 11264 x 2048 62 -> 55, 100 rows by 4096 x 4096 19.9 -> 12.7.
+		// ------------------------------------------------------------------
+		template <int BM, int BN, int WM, int WN, int S>
+		__global__ __launch_bounds__(64 * WM * WN, 2) void dense_ring_kernel(const TileArgs args)
+		{
+			constexpr int W = WM * WN, TM = BM / WM / 16, TN = BN / WN / 16;
+			constexpr int kRowBytes = 2 * kTileK, kStage = (BM + BN) * kRowBytes; // [BM activations, BN weights][64]
+			constexpr int LA = BM / 8 / W, LW = BN / 8 / W, L = LA + LW;         // 1 KB pieces a wavefront moves per tile
+			static_assert(LA * 8 * W == BM && LW * 8 * W == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile");
+			static_assert((S - 1) * L < 64, "loads that a wait can count");
+			extern __shared__ __attribute__((aligned(16))) uint8_t ring_lds[];
+			const DenseRows& d = args.d;
+			int tm, tn;
+			if (!tile_of(args, tm, tn))
+			{
+				return;
+			}
+			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int j = lane & 15, g = lane >> 4;
+			const int wm = wave / WN, wn = wave % WN;
+			const int m0 = tm * BM, n0 = tn * BN;
+			const fetch::DenseWalk walk = fetch::dense_walk(d.w.pitch / kTileK, d.splits, 1, static_cast<int>(blockIdx.y), 0);
+
+			// piece i of a wavefront: rows 8 (i W + wave) .. + 7 of the activations, then of the weights
+			uint32_t from[L];
+			{
+				const int row = lane >> 3, at = ((lane & 7) ^ row) * 16;
+#pragma unroll
+				for (int i = 0; i < LA; ++i)
+				{
+					from[i] = static_cast<uint32_t>(operand_row(d, m0 + 8 * (i * W + wave) + row)) * static_cast<uint32_t>(2 * d.lda) + at;
+				}
+#pragma unroll
+				for (int i = 0; i < LW; ++i)
+				{
+					from[LA + i] = static_cast<uint32_t>(min(n0 + 8 * (i * W + wave) + row, d.w.n - 1)) * static_cast<uint32_t>(2 * d.w.pitch) + at;
+				}
+			}
+			const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t*)(ring_lds)));
+			const auto request = [&](int step, int buffer) {
+				const size_t k_bytes = static_cast<size_t>(walk.tile(step)) * kRowBytes;
+				const uint8_t* const a = static_cast<const uint8_t*>(d.a) + k_bytes;
+				const uint8_t* const w = reinterpret_cast<const uint8_t*>(d.w.w) + k_bytes;
+				const uint32_t to = lds_base + buffer * kStage + wave * 1024;
+#pragma unroll
+				for (int i = 0; i < L; ++i)
+				{
+					asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+					             :
+					             : "s"(to + i * (W * 1024)), "v"(from[i]), "s"(i < LA ? a : w)
+					             : "memory", "m0");
+				}
+			};
+			// this lane's piece of the first fragment, by half of the tile
+			const uint8_t* x_at[2];
+			const uint8_t* w_at[2];
+#pragma unroll
+			for (int ks = 0; ks < 2; ++ks)
+			{
+				const int piece = ((4 * ks + g) ^ (j & 7)) * 16;
+				x_at[ks] = ring_lds + (wm * (BM / WM) + j) * kRowBytes + piece;
+				w_at[ks] = ring_lds + (BM + wn * (BN / WN) + j) * kRowBytes + piece;
+			}
+			bf16x8 wf[2][TN], xf[2][TM];
+			const auto read = [&](int ks, int buffer) {
+#pragma unroll
+				for (int a = 0; a < TN; ++a)
+				{
+					wf[ks][a] = *reinterpret_cast<const bf16x8*>(w_at[ks] + buffer * kStage + a * (16 * kRowBytes));
+				}
+#pragma unroll
+				for (int b = 0; b < TM; ++b)
+				{
+					xf[ks][b] = *reinterpret_cast<const bf16x8*>(x_at[ks] + buffer * kStage + b * (16 * kRowBytes));
+				}
+			};
+			floatx4 acc[TN][TM];
+#pragma unroll
+			for (int a = 0; a < TN; ++a)
+			{
+#pragma unroll
+				for (int b = 0; b < TM; ++b)
+				{
+					acc[a][b] = floatx4{ 0.0f, 0.0f, 0.0f, 0.0f };
+				}
+			}
+			const auto multiply = [&](int ks) {
+#pragma unroll
+				for (int a = 0; a < TN; ++a)
+				{
+#pragma unroll
+					for (int b = 0; b < TM; ++b)
+					{
+						acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][a], xf[ks][b], acc[a][b], 0, 0, 0);
+					}
+				}
+			};
+			// behind the k-th activation there may be anything: the last tile's is zeroed once it is there
+			const int last_tile = d.w.pitch / kTileK - 1, last_valid = d.w.k - last_tile * kTileK;
+			const auto trim = [&](int step, int buffer) {
+				if (last_valid == kTileK || step >= walk.rounds || walk.tile(step) != last_tile)
+				{
+					return;
+				}
+				for (int i = threadIdx.x; i < BM * 8; i += 64 * W)
+				{
+					const int row = i >> 3, left = last_valid - 8 * ((i & 7) ^ (row & 7));
+					uint16_t* const piece = reinterpret_cast<uint16_t*>(ring_lds + buffer * kStage + i * 16);
+					for (int e = max(left, 0); e < 8; ++e)
+					{
+						piece[e] = 0;
+					}
+				}
+				__syncthreads();
+			};
+#pragma unroll
+			for (int t = 0; t < S; ++t)
+			{
+				request(t, t); // (past the range's last tile that one comes again: every wait counts the same)
+			}
+			// all but the last N pieces have arrived, this wavefront's reads too; then the others say the same
+			asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * L) : "memory");
+			trim(0, 0);
+			read(0, 0);
+			int buffer = 0;
+			for (int step = 0; step < walk.rounds; ++step)
+			{
+				read(1, buffer);
+				__builtin_amdgcn_sched_barrier(0);
+				multiply(0);
+				__builtin_amdgcn_sched_barrier(0);
+				asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
+				request(step + S, buffer);
+				buffer = buffer == S - 1 ? 0 : buffer + 1;
+				trim(step + 1, buffer);
+				read(0, buffer);
+				__builtin_amdgcn_sched_barrier(0);
+				multiply(1);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); // (nothing may arrive in LDS that is another workgroup's)
+#pragma unroll
+			for (int b = 0; b < TM; ++b)
+			{
+				const int m = m0 + wm * (BM / WM) + 16 * b + j;
+#pragma unroll
+				for (int a = 0; a < TN; ++a)
+				{
+					store_outputs<uint16_t>(d, m, n0 + wn * (BN / WN) + 16 * a + 4 * g, acc[a][b]);
+				}
+			}
+		}
+
 		constexpr size_t kRowLdsLimit = 152 * 1024;
 
 		size_t row_lds_bytes(int pitch, int& groups)
@@ -750,6 +915,18 @@ namespace litenn_hip
 			args.n_tiles = (args.d.w.n + BN - 1) / BN;
 			const int per = (args.m_tiles * args.n_tiles + 7) / 8;
 			dense_tile_kernel<BM, BN, WM, WN, KG, S, F32><<<dim3(8 * per, args.d.splits), dim3(64 * WM * WN * KG), lds, s>>>(args);
+		}
+
+		template <int BM, int BN, int WM, int WN, int S>
+		void launch_ring(TileArgs& args, hipStream_t s)
+		{
+			constexpr size_t lds = static_cast<size_t>(S) * (BM + BN) * kTileK * sizeof(uint16_t);
+			static_assert(lds <= 160 * 1024, "LDS");
+			allow_dynamic_lds(reinterpret_cast<const void*>(&dense_ring_kernel<BM, BN, WM, WN, S>), lds);
+			args.m_tiles = (args.d.m + BM - 1) / BM;
+			args.n_tiles = (args.d.w.n + BN - 1) / BN;
+			const int per = (args.m_tiles * args.n_tiles + 7) / 8;
+			dense_ring_kernel<BM, BN, WM, WN, S><<<dim3(8 * per, args.d.splits), dim3(64 * WM * WN), lds, s>>>(args);
 		}
 
 		int tiles(const DenseRows& d, int bm, int bn) { return ((d.m + bm - 1) / bm) * ((d.w.n + bn - 1) / bn); }
@@ -809,6 +986,30 @@ namespace litenn_hip
 				launch_tile<32, 64, 1, 4, 2, 2, true>(args, s);
 			}
 			return;
+		}
+		// A tile of K costs so many ns of every workgroup a CU has in a row, in the form that is the fastest or within 3 % of it at
+		// all but one of 20 shapes from 20 x 11264 x 2048 to 2048 x 4096 x 14336 (2048 x 4096 x 4096, 7 %): 256 x 256 1660, 128 x 256 990, 64 x
+		// 128 320, 64 x 64 195, 32 x 64 142; 128 x 128 590 by itself, 475 where others share the CU, and 550 there when rows are so
+		// long that their tiles leave the caches.  us for 256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64, 32 x 64: 2048 x 28672 x
+		// 4096 427, 450, 470, 674, 830, 1194; 777 x 2048 x 5632 126, 72, 54, 32, 36, 51; 500 x 2048 x 5632 126, 71, 55, 30, 21, 28;
+		// 100 x 4096 x 4096 86, 52, 39, 22, 14.7, 12.6.
+		const auto on16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+		const auto reach = [](size_t rows, size_t pitch) { return rows * pitch * sizeof(uint16_t) <= 0xffffffffu; }; // 32-bit offsets
+		if (on16(a.a) && on16(a.w.w) && a.lda % 8 == 0 && reach(std::max(a.m, a.a_ring), a.lda) && reach(a.w.n, a.w.pitch))
+		{
+			const auto in_a_row = [&](int bm, int bn) { return (work(bm, bn) + 255) / 256; };
+			const int r128 = in_a_row(128, 128);
+			const int cost[] = { 1660 * in_a_row(256, 256), 990 * in_a_row(128, 256), (r128 == 1 ? 590 : a.w.pitch <= 6144 ? 475 : 550) * r128,
+				                 320 * in_a_row(64, 128), 195 * in_a_row(64, 64), 142 * in_a_row(32, 64) };
+			switch (std::min_element(cost, cost + 6) - cost)
+			{
+			case 0: return launch_ring<256, 256, 2, 4, 2>(args, s);
+			case 1: return launch_ring<128, 256, 2, 4, 3>(args, s);
+			case 2: return launch_ring<128, 128, 2, 2, 2>(args, s);
+			case 3: return launch_ring<64, 128, 2, 4, 3>(args, s);
+			case 4: return launch_ring<64, 64, 2, 2, 4>(args, s);
+			default: return launch_ring<32, 64, 1, 4, 4>(args, s);
+			}
 		}
 		// A K step of a form costs so many ns where a CU has r workgroups of it, fitted over 2048 x 5632, 4096 x 14336, 11264 x
 		// 2048, 6432 x 2048 and 6144 x 4096 at 30 to 1254 rows; the form with the least is the fastest of eleven, or within 5 % of

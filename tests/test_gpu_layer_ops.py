@@ -4,6 +4,7 @@ import pytest
 
 import np_kulurax as ref
 from conftest import rel_l2
+from litenn_amd import _lib
 from litenn_amd.formats import DT_BF16, DT_F32
 from litenn_amd.model import from_bfloat16, to_bfloat16
 
@@ -63,6 +64,23 @@ def test_linear_bf16_larger(hip, n, k, m):
     xb = padded_bits(rng.normal(0, 1, (m, k)).astype(np.float32))
     y = hip.linear_bf16(bf16_tensor(hip, w), n, k, bf16_tensor(hip, xb), m).numpy()
     assert rel_l2(y, from_bfloat16(xb).astype(np.float64) @ from_bfloat16(w).astype(np.float64).T) <= 2e-6
+
+
+@pytest.mark.parametrize("n,k,m", [(8192, 300, 2048), (8000, 6200, 1000), (8000, 300, 1000), (4000, 333, 300), (2030, 64, 490), (2030, 1, 490),
+                                   (4090, 65, 40), (4100, 191, 20)])
+def test_linear_bf16_in_every_form(hip, n, k, m):
+    """256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64, 32 x 64 in turn: rows fewer than a tile's, fewer tiles of K than
+    a ring has buffers, a last tile that is not whole behind none, one and many.  Operands off their 16 bytes give the same."""
+    rng = np.random.default_rng([n, k, m])
+    w, xb = padded_bits(rng.normal(0, 1, (n, k)).astype(np.float32)), padded_bits(rng.normal(0, 1, (m, k)).astype(np.float32), NAN16)
+    y = hip.linear_bf16(bf16_tensor(hip, w), n, k, bf16_tensor(hip, xb), m).numpy()
+    want = from_bfloat16(xb)[:, :k].astype(np.float64) @ from_bfloat16(w)[:, :k].astype(np.float64).T
+    assert rel_l2(y, want) <= 2e-6
+    moved = np.concatenate([np.zeros(1, np.uint16), xb.ravel()]).reshape(1, -1)
+    t, out = bf16_tensor(hip, moved), hip.Tensor((m, n), DT_F32)
+    wt = bf16_tensor(hip, w)
+    _lib.check(_lib.load().litenn_hip_linear_bf16(0, wt.ptr, n, k, pitch(k), t.ptr + 2, DT_BF16, m, out.ptr, None))
+    assert np.array_equal(out.numpy(), y)
 
 
 def plain_window_attn(q, k, v, q_pos, k_pos, window, scale, sink):
