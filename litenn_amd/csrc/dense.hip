@@ -8,6 +8,7 @@
 #include "dense.hpp"
 
 #include <algorithm>
+#include <iterator>
 #include <type_traits>
 
 #pragma clang diagnostic ignored "-Winline-asm" // m0 is named as clobbered although it is reserved
@@ -730,10 +731,10 @@ namespace litenn_hip
 		// tile, in its middle: behind it the next tile is there and this one's buffer is free.  Outputs are the chains of
 		// products over K that dense_tile_kernel forms, bit for bit.
 		//
-		// What bounds it: small tiles, the rate at which a CU takes operands from L2 (70 to 80 GB/s a CU, about 30 bytes a cycle;
-		// a ring twice as deep changes nothing); large ones, the products (256 x 256 on 2048 x 28672 x 4096: 1125 TFLOP/s).  us
-		// against dense_tile_kernel: 2048 rows by 28672 x 4096 527 -> 427, by 4096 x 4096 79 -> 63, 777 rows by 2048 x 5632 45 ->
-		// 32, by 11264 x 2048 62 -> 55, 100 rows by 4096 x 4096 19.9 -> 12.7.
+		// What bounds it: small tiles, the rate at which a CU takes operands from L2 (70 to 80 GB/s a CU, about 30 bytes a cycle; a
+		// ring twice as deep changes nothing), and a tenth or two for weights that come from HBM (a wavefront that touches
+		// them ahead of the others costs more than that); large ones, the products (256 x 256 on 2048 x 28672 x 4096: 1040 TFLOP/s
+		// with the weights from HBM, 1125 without).
 		// ------------------------------------------------------------------
 		template <int BM, int BN, int WM, int WN, int S>
 		__global__ __launch_bounds__(64 * WM * WN, 2) void dense_ring_kernel(const TileArgs args)
@@ -987,28 +988,32 @@ namespace litenn_hip
 			}
 			return;
 		}
-		// A tile of K costs so many ns of every workgroup a CU has in a row, in the form that is the fastest or within 3 % of it at
-		// all but one of 20 shapes from 20 x 11264 x 2048 to 2048 x 4096 x 14336 (2048 x 4096 x 4096, 7 %): 256 x 256 1660, 128 x 256 990, 64 x
-		// 128 320, 64 x 64 195, 32 x 64 142; 128 x 128 590 by itself, 475 where others share the CU, and 550 there when rows are so
-		// long that their tiles leave the caches.  us for 256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64, 32 x 64: 2048 x 28672 x
-		// 4096 427, 450, 470, 674, 830, 1194; 777 x 2048 x 5632 126, 72, 54, 32, 36, 51; 500 x 2048 x 5632 126, 71, 55, 30, 21, 28;
-		// 100 x 4096 x 4096 86, 52, 39, 22, 14.7, 12.6.
+		// Time = workgroups a CU has in a row, each a fixed part and so many ns a tile of K, fitted to 18 shapes from 100 x 4096 x 4096
+		// to 2048 x 28672 x 4096 with weights from HBM (more of them in turn than the 256 MB cache holds; a model's are never
+		// there either, and tuned with weights that are, the choice cost a tenth).  The form it picks is 1 % slower than the best
+		// in the mean, 11 % at 777 x 6432 x 2048.  us for 256 x 256, 128 x 256, 192 x 128, 128 x 192, 128 x 64, 64 x 128, 64 x 64, 32 x 64
+		// and the best of dense_tile_kernel: 2048 x 28672 x 4096 462, 488, 487, 541, 672, 684, 802, 1184 and 551; 777 x 11264 x 2048 68,
+		// 72, 52, 63, 66, 69, 79, 108 and 63; 777 x 2048 x 5632 133, 79, 82, 65, 38, 41, 45, 60 and 46; 500 x 2048 x 5632 140, 82, 83, 66,
+		// 40, 42, 28, 36 and 31; 100 x 4096 x 4096 95, 59, 60, 48, 29, 30, 20, 15.5 and 20.
 		const auto on16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
 		const auto reach = [](size_t rows, size_t pitch) { return rows * pitch * sizeof(uint16_t) <= 0xffffffffu; }; // 32-bit offsets
 		if (on16(a.a) && on16(a.w.w) && a.lda % 8 == 0 && reach(std::max(a.m, a.a_ring), a.lda) && reach(a.w.n, a.w.pitch))
 		{
-			const auto in_a_row = [&](int bm, int bn) { return (work(bm, bn) + 255) / 256; };
-			const int r128 = in_a_row(128, 128);
-			const int cost[] = { 1660 * in_a_row(256, 256), 990 * in_a_row(128, 256), (r128 == 1 ? 590 : a.w.pitch <= 6144 ? 475 : 550) * r128,
-				                 320 * in_a_row(64, 128), 195 * in_a_row(64, 64), 142 * in_a_row(32, 64) };
-			switch (std::min_element(cost, cost + 6) - cost)
+			const auto cost = [&](int bm, int bn, int fixed, int step) {
+				return static_cast<long long>((work(bm, bn) + 255) / 256) * (fixed + static_cast<long long>(step) * (a.w.pitch / kTileK / a.splits));
+			};
+			const long long costs[] = { cost(256, 256, 7900, 1475), cost(128, 256, 3700, 867), cost(192, 128, 5700, 663), cost(128, 192, 3900, 725),
+				                        cost(128, 64, 100, 372),    cost(64, 128, 400, 382),   cost(64, 64, 300, 256),    cost(32, 64, 700, 179) };
+			switch (std::min_element(std::begin(costs), std::end(costs)) - costs)
 			{
 			case 0: return launch_ring<256, 256, 2, 4, 2>(args, s);
 			case 1: return launch_ring<128, 256, 2, 4, 3>(args, s);
-			case 2: return launch_ring<128, 128, 2, 2, 2>(args, s);
-			case 3: return launch_ring<64, 128, 2, 4, 3>(args, s);
-			case 4: return launch_ring<64, 64, 2, 2, 4>(args, s);
-			default: return launch_ring<32, 64, 1, 4, 4>(args, s);
+			case 2: return launch_ring<192, 128, 4, 2, 2>(args, s);
+			case 3: return launch_ring<128, 192, 2, 4, 3>(args, s);
+			case 4: return launch_ring<128, 64, 4, 2, 3>(args, s);
+			case 5: return launch_ring<64, 128, 2, 4, 3>(args, s);
+			case 6: return launch_ring<64, 64, 2, 2, 4>(args, s);
+			default: return launch_ring<32, 64, 1, 4, 6>(args, s);
 			}
 		}
 		// A K step of a form costs so many ns where a CU has r workgroups of it, fitted over 2048 x 5632, 4096 x 14336, 11264 x

@@ -66,11 +66,12 @@ def test_linear_bf16_larger(hip, n, k, m):
     assert rel_l2(y, from_bfloat16(xb).astype(np.float64) @ from_bfloat16(w).astype(np.float64).T) <= 2e-6
 
 
-@pytest.mark.parametrize("n,k,m", [(8192, 300, 2048), (8000, 6200, 1000), (8000, 300, 1000), (4000, 333, 300), (2030, 64, 490), (2030, 1, 490),
-                                   (4090, 65, 40), (4100, 191, 20)])
+@pytest.mark.parametrize("n,k,m", [(8192, 300, 2048), (8000, 4300, 1000), (11200, 2050, 760), (6432, 1290, 777), (8000, 300, 1000),
+                                   (11264, 700, 300), (2030, 700, 490), (4090, 700, 100), (2030, 65, 490), (2030, 1, 490), (4100, 64, 20)])
 def test_linear_bf16_in_every_form(hip, n, k, m):
-    """256 x 256, 128 x 256, 128 x 128, 64 x 128, 64 x 64, 32 x 64 in turn: rows fewer than a tile's, fewer tiles of K than
-    a ring has buffers, a last tile that is not whole behind none, one and many.  Operands off their 16 bytes give the same."""
+    """256 x 256, 128 x 256, 192 x 128, 128 x 192, 128 x 64, 64 x 128, 64 x 64, 32 x 64 in turn: rows fewer than a tile's, fewer
+    tiles of K than a ring has buffers, a last tile that is not whole behind none, one and many.  Operands off their 16 bytes
+    give the same."""
     rng = np.random.default_rng([n, k, m])
     w, xb = padded_bits(rng.normal(0, 1, (n, k)).astype(np.float32)), padded_bits(rng.normal(0, 1, (m, k)).astype(np.float32), NAN16)
     y = hip.linear_bf16(bf16_tensor(hip, w), n, k, bf16_tensor(hip, xb), m).numpy()
