@@ -451,8 +451,17 @@ namespace litenn_hip
 
 		// A Float32 as three values whose upper halves are bfloat16 and whose sum it is: eight significant bits, the next
 		// eight, the rest.  An infinity or a NaN is the first one, the others zero.
+		template <bool FINITE>
 		__device__ __forceinline__ void cut_in_three(uint32_t bits, uint32_t (&part)[3])
 		{
+			if constexpr (FINITE)
+			{
+				part[0] = bits & 0xffff0000u;
+				const float rest = __uint_as_float(bits) - __uint_as_float(part[0]);
+				part[1] = __float_as_uint(rest) & 0xffff0000u;
+				part[2] = __float_as_uint(rest - __uint_as_float(part[1]));
+				return;
+			}
 			const bool special = (bits & 0x7f800000u) == 0x7f800000u;
 			const uint32_t quiet = (bits & 0x007fffffu) != 0u ? 0x00400000u : 0u;
 			part[0] = (bits | (special ? quiet : 0u)) & 0xffff0000u;
@@ -466,7 +475,8 @@ namespace litenn_hip
 		// F32: Float32 operands.  The weights are bfloat16 as they are; an activation is the sum of three bfloat16 values
 		// of eight bits each, cut off its front one after the other, which is exact, so that three products per operand
 		// pair give what one of Float32 operands gives, at 48 cycles per 32 elements of K where v_mfma_f32_16x16x4_f32
-		// takes 256.  The activations are taken apart on their way into LDS.
+		// takes 256.  The activations are taken apart on their way into LDS, without a look at infinities where a piece's
+		// magnitudes add up to a number (64 x 128 on 500 x 11264 x 2048 100 -> 88 us; eight wavefronts instead of four 88 -> 85).
 		//
 		// Two wavefronts a SIMD hide most of a step's chain of latencies (request, LDS, barrier, products that feed each other):
 		// eight of them on 128 x 128 take 49 us for 2048 x 5632 at 1254 rows, four 70.  S tiles of K travel at any time.
@@ -560,17 +570,33 @@ namespace litenn_hip
 					if constexpr (F32)
 					{
 						u32x4 part[3];
+						const auto cut = [&](auto finite) {
 #pragma unroll
-						for (int e = 0; e < 4; ++e)
-						{
-							uint32_t lo[3], hi[3];
-							cut_in_three(rx[set][i][e / 2][2 * (e % 2)], lo);
-							cut_in_three(rx[set][i][e / 2][2 * (e % 2) + 1], hi);
-#pragma unroll
-							for (int p = 0; p < 3; ++p)
+							for (int e = 0; e < 4; ++e)
 							{
-								part[p][e] = __builtin_amdgcn_perm(hi[p], lo[p], 0x07060302u); // the upper halves
+								uint32_t lo[3], hi[3];
+								cut_in_three<decltype(finite)::value>(rx[set][i][e / 2][2 * (e % 2)], lo);
+								cut_in_three<decltype(finite)::value>(rx[set][i][e / 2][2 * (e % 2) + 1], hi);
+#pragma unroll
+								for (int p = 0; p < 3; ++p)
+								{
+									part[p][e] = __builtin_amdgcn_perm(hi[p], lo[p], 0x07060302u); // the upper halves
+								}
 							}
+						};
+						float sum = 0.0f; // of magnitudes: one that is no number or infinite shows in it
+#pragma unroll
+						for (int e = 0; e < 8; ++e)
+						{
+							sum += fabsf(__uint_as_float(rx[set][i][e / 4][e % 4]));
+						}
+						if (__builtin_expect(__any(!(sum <= 3.402823466e38f)), 0))
+						{
+							cut(std::false_type{});
+						}
+						else
+						{
+							cut(std::true_type{});
 						}
 #pragma unroll
 						for (int p = 0; p < 3; ++p)
@@ -971,20 +997,35 @@ namespace litenn_hip
 		const auto work = [&](int bm, int bn) { return tiles(a, bm, bn) * a.splits; };
 		if (a.f32)
 		{
-			// Tallest tile that still gives a SIMD two wavefronts, from one workgroup's groups if need be (us, kernel alone, the next
-			// smaller choice against the one taken): width 2048 at 500 rows: ff 11264 rows 109 -> 100 (one group), 2048 rows 50 -> 39
-			// (two); 288 workgroups of one group 59, of two, which have a CU to themselves, 69
+			// Beyond 256 tiles of 64 x 128 a product is one chain over K, up to there two halves (results hang on this alone).  us a
+			// tile of K takes of each workgroup a CU has in a row, fitted to 16 shapes from 30 x 4096 x 2048 to 1000 x 11264 x 4096; us
+			// for 64 x 128, 64 x 256: 500 rows by 11264 x 2048 85, 95, by 6432 x 2048 57, 51; for 64 x 128, 64 x 64, 32 x 64 in halves: 300
+			// rows by 4096 x 4096 58, 78, 70, 500 by 2048 x 5632 76, 59, 66, 100 by 2048 x 2048 28, 20, 15.
+			const auto in_a_row = [&](int bm, int bn) { return (work(bm, bn) + 255) / 256; };
 			if (a.m > 32 && work(64, 128) > 256)
 			{
-				launch_tile<64, 128, 2, 2, 1, 2, true>(args, s);
+				if (83 * in_a_row(64, 128) <= 147 * in_a_row(64, 256))
+				{
+					launch_tile<64, 128, 2, 4, 1, 2, true>(args, s);
+				}
+				else
+				{
+					launch_tile<64, 256, 2, 4, 1, 2, true>(args, s);
+				}
+				return;
 			}
-			else if (a.m > 32 && work(64, 128) >= 192)
-			{
-				launch_tile<64, 128, 2, 2, 2, 2, true>(args, s);
-			}
-			else // width 2048 at 30 rows: 4096 rows 28 -> 19 against one group's 64 x 64
+			const int tall = 88 * in_a_row(64, 128), square = 64 * in_a_row(64, 64), low = 37 * in_a_row(32, 64);
+			if (a.m <= 32 || low <= std::min(tall, square))
 			{
 				launch_tile<32, 64, 1, 4, 2, 2, true>(args, s);
+			}
+			else if (tall <= square)
+			{
+				launch_tile<64, 128, 2, 4, 2, 2, true>(args, s);
+			}
+			else
+			{
+				launch_tile<64, 64, 2, 4, 2, 2, true>(args, s);
 			}
 			return;
 		}
