@@ -1036,6 +1036,7 @@ namespace litenn_hip
 		// and the best of dense_tile_kernel: 2048 x 28672 x 4096 462, 488, 487, 541, 672, 684, 802, 1184 and 551; 777 x 11264 x 2048 68,
 		// 72, 52, 63, 66, 69, 79, 108 and 63; 777 x 2048 x 5632 133, 79, 82, 65, 38, 41, 45, 60 and 46; 500 x 2048 x 5632 140, 82, 83, 66,
 		// 40, 42, 28, 36 and 31; 100 x 4096 x 4096 95, 59, 60, 48, 29, 30, 20, 15.5 and 20.
+		// 32 x 32 against 32 x 64: 30 x 4096 x 14336 38 and 54, 60 x 2048 x 5632 15.5 and 22, 3 x 28672 x 4096 43.2 and 42.4.
 		const auto on16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
 		const auto reach = [](size_t rows, size_t pitch) { return rows * pitch * sizeof(uint16_t) <= 0xffffffffu; }; // 32-bit offsets
 		if (on16(a.a) && on16(a.w.w) && a.lda % 8 == 0 && reach(std::max(a.m, a.a_ring), a.lda) && reach(a.w.n, a.w.pitch))
@@ -1044,7 +1045,8 @@ namespace litenn_hip
 				return static_cast<long long>((work(bm, bn) + 255) / 256) * (fixed + static_cast<long long>(step) * (a.w.pitch / kTileK / a.splits));
 			};
 			const long long costs[] = { cost(256, 256, 7900, 1475), cost(128, 256, 3700, 867), cost(192, 128, 5700, 663), cost(128, 192, 3900, 725),
-				                        cost(128, 64, 100, 372),    cost(64, 128, 400, 382),   cost(64, 64, 300, 256),    cost(32, 64, 700, 179) };
+				                        cost(128, 64, 100, 372),    cost(64, 128, 400, 382),   cost(64, 64, 300, 256),    cost(32, 64, 700, 179),
+				                        cost(32, 32, 300, 145) };
 			switch (std::min_element(std::begin(costs), std::end(costs)) - costs)
 			{
 			case 0: return launch_ring<256, 256, 2, 4, 2>(args, s);
@@ -1054,7 +1056,8 @@ namespace litenn_hip
 			case 4: return launch_ring<128, 64, 4, 2, 3>(args, s);
 			case 5: return launch_ring<64, 128, 2, 4, 3>(args, s);
 			case 6: return launch_ring<64, 64, 2, 2, 4>(args, s);
-			default: return launch_ring<32, 64, 1, 4, 6>(args, s);
+			case 7: return launch_ring<32, 64, 1, 4, 6>(args, s);
+			default: return launch_ring<32, 32, 2, 2, 8>(args, s);
 			}
 		}
 		// A K step of a form costs so many ns where a CU has r workgroups of it, fitted over 2048 x 5632, 4096 x 14336, 11264 x

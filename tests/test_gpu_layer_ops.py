@@ -67,9 +67,9 @@ def test_linear_bf16_larger(hip, n, k, m):
 
 
 @pytest.mark.parametrize("n,k,m", [(8192, 300, 2048), (8000, 4300, 1000), (11200, 2050, 760), (6432, 1290, 777), (8000, 300, 1000),
-                                   (11264, 700, 300), (2030, 700, 490), (4090, 700, 100), (2030, 65, 490), (2030, 1, 490), (4100, 64, 20)])
+                                   (11264, 700, 300), (2030, 700, 490), (4090, 700, 100), (2000, 700, 33), (2030, 65, 490), (2030, 1, 490), (4100, 64, 20)])
 def test_linear_bf16_in_every_form(hip, n, k, m):
-    """256 x 256, 128 x 256, 192 x 128, 128 x 192, 128 x 64, 64 x 128, 64 x 64, 32 x 64 in turn: rows fewer than a tile's, fewer
+    """256 x 256, 128 x 256, 192 x 128, 128 x 192, 128 x 64, 64 x 128, 64 x 64, 32 x 64, 32 x 32 in turn: rows fewer than a tile's, fewer
     tiles of K than a ring has buffers, a last tile that is not whole behind none, one and many.  Operands off their 16 bytes
     give the same."""
     rng = np.random.default_rng([n, k, m])
