@@ -19,11 +19,12 @@
 // A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
 // a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
 // where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
-// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 42 us, where
-// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 113 us.  Sums are
+// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 36 us, where
+// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 91 us.  (43 and 109 with
+// a branch for each score's options, every tile masked and the cap's tangent always in the layer's form.)  Sums are
 // short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
 // addition per tile, which costs 4 us and leaves the error against 64 bits below the row kernel's (mean of six inputs, 1e-7:
-// these rows 3.75 and 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
+// these rows, whose small capped scores the row kernel's tangent rounds, 1.34 and 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
 #include "common.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
@@ -89,9 +90,22 @@ namespace litenn_hip
 			{
 				head_log2 <<= 1;
 			}
-			const double m0 = pow(2.0, -max_bias / static_cast<double>(head_log2));
-			const double m1 = pow(2.0, -(max_bias / 2.0) / static_cast<double>(head_log2));
-			return head < head_log2 ? pow(m0, static_cast<double>(head + 1)) : pow(m1, static_cast<double>(2 * (head - head_log2) + 1));
+			// (its powers of 2 to a power are one power of 2)
+			const int times = head < head_log2 ? 2 * (head + 1) : 2 * (head - head_log2) + 1;
+			return exp2(-(max_bias / 2.0) / static_cast<double>(head_log2) * static_cast<double>(times));
+		}
+
+		// tanh up to kSmallTangent: its series to x^11, the next term 1.2e-8 of it
+		constexpr float kSmallTangent = 0.35f;
+		__device__ __forceinline__ float small_tanh(float x)
+		{
+			const float x2 = x * x;
+			float p = -1382.0f / 155925.0f;
+			p = fmaf(p, x2, 62.0f / 2835.0f);
+			p = fmaf(p, x2, -17.0f / 315.0f);
+			p = fmaf(p, x2, 2.0f / 15.0f);
+			p = fmaf(p, x2, -1.0f / 3.0f);
+			return fmaf(x, x2 * p, x);
 		}
 
 		// Rows of keys and values lie 2 D bytes apart in LDS, their 16-byte pieces permuted by the row so that the 64 banks
@@ -132,6 +146,8 @@ namespace litenn_hip
 			const auto sees_from = [&](int i) { return static_cast<int>(max(0ll, q_at + i - a.window + 1)); };
 			const auto sees_to = [&](int i) { return a.causal ? static_cast<int>(min(static_cast<long long>(keys), q_at + i + 1)) : keys; };
 			const int lo = sees_from(row_c), hi = sees_to(row_c);
+			// keys that all of the wavefront's queries see
+			const int wave_lo = sees_from(min(q_first + 32 * qw + 31, a.rows - 1)), wave_hi = sees_to(min(q_first + 32 * qw, a.rows - 1));
 			const int first = sees_from(q_first), last = sees_to(min(q_first + 32 * QW, a.rows) - 1);
 			const int tiles = (last - first + kKeys - 1) / kKeys;
 			const int steps = (tiles + KW - 1) / KW;
@@ -208,6 +224,12 @@ namespace litenn_hip
 			const float slope = a.mask && a.max_bias > 0.0 ? static_cast<float>(row_alibi_slope(head, a.heads, a.max_bias)) : 1.0f;
 			const float* const mask_row = a.mask ? a.mask + static_cast<size_t>(row_c) * keys : nullptr;
 
+			// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range.  (A
+			// division: the reciprocal instruction gives 0 above 2^126, which exp reaches short of its range's end.)
+			const auto layer_tanh = [](float v) {
+				const float ex = expf(__fmul_rn(v, 2.0f));
+				return __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
+			};
 			// a dot product's score (the causal mask and the window aside)
 			const auto score_of = [&](float v, float mv) {
 				if (a.apply_scale)
@@ -216,10 +238,7 @@ namespace litenn_hip
 				}
 				if (a.softcap != 0.0f)
 				{
-					// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range.  (A
-					// division: the reciprocal instruction gives 0 above 2^126, which exp reaches short of its range's end.)
-					const float ex = expf(__fmul_rn(v, 2.0f));
-					v = __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
+					v = layer_tanh(v);
 					if (a.apply_cap)
 					{
 						v = __fmul_rn(v, a.softcap);
@@ -227,7 +246,7 @@ namespace litenn_hip
 				}
 				if (a.mask)
 				{
-					v = __fadd_rn(v, __fmul_rn(mv, slope)); // (a slope of 1 leaves the mask as it is)
+					v = __fadd_rn(v, __fmul_rn(mv, slope));
 				}
 				return v;
 			};
@@ -386,10 +405,73 @@ namespace litenn_hip
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
 				{
-					const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
-					const bool visible = live && key >= lo && key < hi;
-					const float v = score_of(fmaf(s_low[e], O::kLowScale, s[e] + s_odd[e]) * unscale, mask[e]);
-					sc[e] = visible ? v : -INFINITY;
+					sc[e] = fmaf(s_low[e], O::kLowScale, s[e] + s_odd[e]) * unscale;
+				}
+				// (an option at a time over all sixteen: a branch for each score's options was a tenth of the tile)
+				if (a.apply_scale)
+				{
+#pragma unroll
+					for (int e = 0; e < 16; ++e)
+					{
+						sc[e] = __fmul_rn(sc[e], a.scale);
+					}
+				}
+				if (a.softcap != 0.0f)
+				{
+					// Capped scores are a small part of the cap as a rule: where all of the wavefront's are, the tangent's series takes
+					// seven instructions where the layer's form takes 35, and is closer (that form cancels: 1e-6 of a score of
+					// cap / 30, which was most of the error against 64 bits, 3.7e-7 -> 1.3e-7).
+					float most = 0.0f;
+#pragma unroll
+					for (int e = 0; e < 16; ++e)
+					{
+						most = fmaxf(most, fabsf(sc[e])); // (a NaN stays one in either form)
+					}
+					if (__all(most <= kSmallTangent))
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							sc[e] = small_tanh(sc[e]);
+						}
+					}
+					else
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							sc[e] = layer_tanh(sc[e]);
+						}
+					}
+					if (a.apply_cap)
+					{
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							sc[e] = __fmul_rn(sc[e], a.softcap);
+						}
+					}
+				}
+				if (a.mask)
+				{
+#pragma unroll
+					for (int e = 0; e < 16; ++e)
+					{
+						sc[e] = __fadd_rn(sc[e], __fmul_rn(mask[e], slope)); // (a slope of 1 leaves the mask as it is)
+					}
+				}
+				if (!live || base < wave_lo || base + kKeys > wave_hi) // (a key that one of the wavefront's queries does not see)
+				{
+#pragma unroll
+					for (int e = 0; e < 16; ++e)
+					{
+						const int key = base + 8 * (e / 4) + 4 * h + (e & 3);
+						sc[e] = live && key >= lo && key < hi ? sc[e] : -INFINITY;
+					}
+				}
+#pragma unroll
+				for (int e = 0; e < 16; ++e)
+				{
 					top = fmaxf(top, sc[e]);
 				}
 				top = fmaxf(top, __shfl_xor(top, 32, 64));

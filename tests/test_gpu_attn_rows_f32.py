@@ -168,3 +168,19 @@ def test_a_value_that_is_not_finite_stays_with_the_queries_that_see_it(hip, dtyp
     assert np.all(got[m - 10:, :, 3] == np.inf) and np.all(np.isnan(got[m - 5:, :, 90]))
     rest = np.delete(got, [3, 90], axis=2), np.delete(clean, [3, 90], axis=2)
     assert np.linalg.norm(rest[0] - rest[1]) <= 2e-6 * np.linalg.norm(rest[1])
+
+
+@pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
+@pytest.mark.parametrize("spread", [0.02, 0.32, 0.345, 0.355, 1.0, 8.0])
+@pytest.mark.parametrize("m,keys", [(33, 129), (64, 96), (40, 700)])
+def test_soft_caps_on_both_sides_of_the_series(hip, dtype, spread, m, keys):
+    """The largest score is `spread` of the cap: the series' tiles alone, both kinds and the layer's form alone; key tiles that
+    all queries see whole, and the ones where the first and the last key of a tile is the first that one does not."""
+    heads, dim, cap = 3, 64, 7.0
+    q, k, v = inputs(5, m, keys, heads, 1, dim, dtype)
+    s = np.abs(np.einsum("ihd,jd->hij", q.astype(np.float64), k[:, 0].astype(np.float64))).max()
+    q *= np.float32(spread * cap / s)
+    T = hip.Tensor.from_numpy
+    got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=1.0, logit_softcap=cap,
+                             query_position_offset=keys - m).numpy()
+    assert worst(got, plain(*(a.astype(np.float64) for a in (q, k, v)), 1.0, keys - m, softcap=cap)) <= 4e-6
