@@ -182,5 +182,5 @@ def test_soft_caps_on_both_sides_of_the_series(hip, dtype, spread, m, keys):
     q *= np.float32(spread * cap / s)
     T = hip.Tensor.from_numpy
     got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=1.0, logit_softcap=cap,
-                             query_position_offset=keys - m).numpy()
+                             causal=True, query_position_offset=keys - m).numpy()
     assert worst(got, plain(*(a.astype(np.float64) for a in (q, k, v)), 1.0, keys - m, softcap=cap)) <= 4e-6
