@@ -15,7 +15,8 @@ namespace litenn_hip
 	namespace
 	{
 		// counters[0] = past length, counters[1] = tokens emitted so far, counters[2] = steps this model
-		// has run (never reset: it names a step in the values its workgroups hand to each other)
+		// has run (never reset: it names a step in the values its workgroups hand to each other), counters[3] = workgroups of the
+		// arg-max that have arrived (0 between launches)
 		__global__ void set_counters_kernel(int* counters, int past, int emitted)
 		{
 			counters[0] = past;

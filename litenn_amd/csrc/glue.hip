@@ -866,10 +866,12 @@ namespace litenn_hip
 			}
 		}
 
-		// ---- arg-max of one long row in two launches (the decoder's vocabulary) -------------------
-		// Many workgroups scan a chunk each; one wavefront merges their (value, index) pairs, stores
-		// the token and advances the decoder's device-side counters {past length, tokens emitted}.
-		constexpr int kArgmaxChunk = 2048;
+		// ---- arg-max of one long row (the decoder's vocabulary) -----------------------------------
+		// Many workgroups scan a chunk each; the last to arrive merges their (value, index) pairs, stores the token and
+		// advances the decoder's device-side counters {past length, tokens emitted, steps run, workgroups arrived}.  The
+		// pairs cross between workgroups as the attention splits' triples do.  A launch of one wavefront that merged them,
+		// and chunks of 2048, took 8.7 us for 32000 values where this takes 4.5.
+		constexpr int kArgmaxChunk = 1024;
 
 		__device__ __forceinline__ void argmax_take(float ov, int oi, float& best, int& best_i)
 		{
@@ -880,21 +882,31 @@ namespace litenn_hip
 			}
 		}
 
-		__global__ __launch_bounds__(256) void argmax_partial_kernel(const float* __restrict__ x, int n,
-		                                                              float* __restrict__ pv, int* __restrict__ pi)
+		// counters[3] is 0 before and after; out may be null
+		__global__ __launch_bounds__(256) void argmax_step_kernel(const float* __restrict__ x, int n, float* pv, int* pi,
+		                                                           int32_t* __restrict__ next, int* counters, int past_inc,
+		                                                           int32_t* __restrict__ out)
 		{
 			__shared__ float bv[4];
 			__shared__ int bi[4];
+			__shared__ int s_last;
 			const int begin = blockIdx.x * kArgmaxChunk, end = min(n, begin + kArgmaxChunk);
+			float v[kArgmaxChunk / 256];
+#pragma unroll
+			for (int i = 0; i < kArgmaxChunk / 256; ++i)
+			{
+				v[i] = x[min(begin + static_cast<int>(threadIdx.x) + 256 * i, end - 1)];
+			}
 			float best = -INFINITY;
 			int best_i = 0x7fffffff;
-			for (int i = begin + threadIdx.x; i < end; i += 256)
+#pragma unroll
+			for (int i = 0; i < kArgmaxChunk / 256; ++i)
 			{
-				const float v = x[i];
-				if (v > best || best_i == 0x7fffffff)
+				const int at = begin + static_cast<int>(threadIdx.x) + 256 * i;
+				if (at < end && (v[i] > best || best_i == 0x7fffffff))
 				{
-					best = v;
-					best_i = i;
+					best = v[i];
+					best_i = at;
 				}
 			}
 			for (int off = 32; off > 0; off >>= 1)
@@ -913,22 +925,22 @@ namespace litenn_hip
 				{
 					argmax_take(bv[wv], bi[wv], best, best_i);
 				}
-				pv[blockIdx.x] = best;
-				pi[blockIdx.x] = best_i;
+				__hip_atomic_store(pv + blockIdx.x, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+				__hip_atomic_store(pi + blockIdx.x, best_i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+				asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+				s_last = __hip_atomic_fetch_add(counters + 3, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == static_cast<int>(gridDim.x) - 1;
 			}
-		}
-
-		// one wavefront; counters = {past length, tokens emitted, steps run}, out may be null
-		__global__ __launch_bounds__(64) void argmax_merge_step_kernel(const float* __restrict__ pv,
-		                                                                const int* __restrict__ pi, int blocks,
-		                                                                int32_t* __restrict__ next, int* counters,
-		                                                                int past_inc, int32_t* __restrict__ out)
-		{
-			float best = -INFINITY;
-			int best_i = 0x7fffffff;
-			for (int b = threadIdx.x; b < blocks; b += 64)
+			__syncthreads();
+			if (!s_last || threadIdx.x >= 64)
 			{
-				argmax_take(pv[b], pi[b], best, best_i);
+				return;
+			}
+			best = -INFINITY;
+			best_i = 0x7fffffff;
+			for (int b = threadIdx.x; b < static_cast<int>(gridDim.x); b += 64)
+			{
+				argmax_take(__hip_atomic_load(pv + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
+				            __hip_atomic_load(pi + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), best, best_i);
 			}
 			for (int off = 32; off > 0; off >>= 1)
 			{
@@ -945,6 +957,7 @@ namespace litenn_hip
 				}
 				counters[0] += past_inc;
 				counters[2] += 1;
+				__hip_atomic_store(counters + 3, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // for the next launch on this stream
 			}
 		}
 
@@ -1280,8 +1293,7 @@ namespace litenn_hip
 		const int blocks = static_cast<int>((n + kArgmaxChunk - 1) / kArgmaxChunk);
 		float* pv = static_cast<float*>(scratch);
 		int* pi = reinterpret_cast<int*>(pv + blocks);
-		argmax_partial_kernel<<<dim3(blocks), dim3(256), 0, s>>>(x, static_cast<int>(n), pv, pi);
-		argmax_merge_step_kernel<<<dim3(1), dim3(64), 0, s>>>(pv, pi, blocks, next, counters, past_inc, out);
+		argmax_step_kernel<<<dim3(blocks), dim3(256), 0, s>>>(x, static_cast<int>(n), pv, pi, next, counters, past_inc, out);
 	}
 
 	void launch_add_int(int* p, int v, hipStream_t s) { add_int_kernel<<<1, 1, 0, s>>>(p, v); }

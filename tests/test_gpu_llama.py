@@ -412,3 +412,28 @@ def test_float32_operands_after_rounded_ones(hip, fmt, ff):
         assert np.array_equal(model.generate(tokens, 6, precise=precise)[0], steps[precise])
         model.reset()
         assert np.array_equal(model.eval(tokens, precise=precise), alone[precise])
+
+
+@pytest.mark.parametrize("vocab", [7, 1023, 1024, 1025, 2050, 66000])
+def test_the_first_of_equal_logits_is_taken(hip, vocab):
+    """Vocabularies at the edges of the arg-max's chunks, and more chunks than a wavefront has lanes; every logit of the first
+    half comes again in the second."""
+    cfg = synth.tiny_llama(Q8_0, block_count=1, d_model=256, heads=2, kv_heads=1, ff=256, vocab=vocab, context_length=32)
+
+    def tensors():
+        for kind, layer, fmt, payload, n, k in synth.llama_tensors(cfg, 3):
+            if kind == "output":
+                rows = payload.reshape(n, -1).copy()
+                rows[vocab // 2:2 * (vocab // 2)] = rows[:vocab // 2]
+                payload = rows.reshape(payload.shape)
+            yield kind, layer, fmt, payload, n, k
+    m = hip_model(hip, cfg, 3, tensors=tensors())
+    prompt = synth.prompt_tokens(cfg, 5, 9)
+    got = [m.generate(prompt, 12)[0].tolist() if m.reset() is None else None for _ in range(2)]
+    assert got[0] == got[1]
+    m.reset()
+    logits, want = m.eval(prompt)[-1], []
+    for _ in range(12):
+        want.append(int(np.argmax(logits)))
+        logits = m.eval(want[-1:])[0]
+    assert got[0] == want
