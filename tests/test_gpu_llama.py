@@ -437,3 +437,17 @@ def test_the_first_of_equal_logits_is_taken(hip, vocab):
         want.append(int(np.argmax(logits)))
         logits = m.eval(want[-1:])[0]
     assert got[0] == want
+
+
+@pytest.mark.parametrize("head_dim,rope", [(6, 6), (6, 2), (8, 8), (8, 2), (12, 6), (20, 10), (128, 64)])
+@pytest.mark.parametrize("kv", [DT_F16, DT_F32])
+def test_rotations_that_end_inside_four_features(hip, oracle, head_dim, rope, kv):
+    """Heads of whole groups of four features and others, rotations of all of a group, half of it and none."""
+    cfg = synth.tiny_llama(Q8_0, block_count=2, d_model=16 * head_dim, heads=16, kv_heads=4, ff=32, vocab=50, context_length=64)
+    cfg.rope_dimension_count = rope
+    toks = synth.prompt_tokens(cfg, 40, 2)
+    ref, dev = oracle_model(oracle, cfg, 4, kv_f16=(kv == DT_F16)), hip_model(hip, cfg, 4, kv_dtype=kv)
+    assert rel_l2(dev.eval(toks[:33]), ref.eval(toks[:33])) < 1e-4
+    assert rel_l2(dev.eval(toks[33:]), ref.eval(toks[33:])) < 1e-4
+    for got, want in zip(dev.get_kv(1), ref.get_kv(1)):
+        assert rel_l2(got, want) < 1e-3
