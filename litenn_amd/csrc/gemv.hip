@@ -2247,9 +2247,10 @@ namespace litenn_hip
 	void launch_get_rows_q(int fmt, const void* table, size_t rows, size_t k, const int32_t* ids, size_t n_ids,
 	                       float* out, int* err_flag, hipStream_t stream)
 	{
-		// an element a thread while that is 512 workgroups and fewer (one row of 4096 6.1 -> 4.8 us, 20 rows 8.1 -> 3.7)
+		// an element a thread while that is 8192 workgroups and fewer (us, rows of 4096: one 6.1 -> 4.8, 20 8.1 -> 3.7, 300 8.8 -> 7.6,
+		// 1024 18.6 -> 20.5)
 		const size_t pieces = (k + 255) / 256;
-		const bool cut = n_ids * pieces <= 512;
+		const bool cut = n_ids * pieces <= 8192;
 		get_rows_q_kernel<<<dim3(n_ids, cut ? pieces : 1), dim3(cut || k < 4096 ? 256 : 1024), 0, stream>>>(
 		    fmt, static_cast<const uint8_t*>(table), static_cast<int>(rows), static_cast<int>(k), row_bytes(fmt, k), ids, out, err_flag);
 	}
