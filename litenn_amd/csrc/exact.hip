@@ -21,7 +21,7 @@
 // What bounds it: few rows are the weights' stream and the launch; many rows, the LDS reads of the fragments (two
 // per pair of products) and the latency in front of them: a product issues every 100 cycles and SIMD where
 // it takes 32.  Row by row through the streaming kernel the same calls took, us, before -> now with the rows'
-// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 46; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1400.
+// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 43; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1310.
 //
 // v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
 // weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
