@@ -659,20 +659,23 @@ namespace litenn_hip
 			return key * DV + ((piece ^ (((key / kSame) & (kColumns - 1)) << 1)) << 3);
 		}
 
-		// PARTS = 2: a workgroup is two halves of four wavefronts, one for the even key tiles and one for the odd ones, each
-		// with its own buffers; their (maximum, sum, outputs) meet at the end.  A query tile is a chain of up to 17 key tiles
-		// otherwise, with one wavefront a SIMD where there are few of them.  us for 777 rows of 16 heads of 128, window 1024, 31.7 ->
-		// 19.2, 2048 rows of 32 heads 114 -> 76: values turned by the LDS read instead of two bytes at a time on their way in,
-		// masks and rescaling only in tiles that need them, queries and gates asked for all at once.
+		// PARTS = 2: eight wavefronts, two to sixteen queries: both form the scores and the weights of every key, each half of
+		// the value dimensions, so that a query's bits are the same whichever of the two forms it takes.  A query tile is a chain of
+		// up to 17 key tiles, with one wavefront a SIMD where there are few of them.
+		// us for 777 rows of 16 heads of 128, window 1024, 26.1 -> 24.3, 100 rows 10.5 -> 9.2.  (Halves that take the key tiles
+		// in turn and meet at the end take 22.2 and 12.0, but round their weights to bfloat16 against maxima of their own: a row's
+		// bits hung on how many heads and rows went with it.)  Values turned by the LDS read instead of two bytes at a time on
+		// their way in, masks and rescaling only in tiles that need them, queries and gates asked for all at once: 777 rows
+		// 34.5 -> 26.1, 2048 rows of 32 heads 102 -> 71.
 		template <int DK, int DV, int PARTS>
 		__global__ __launch_bounds__(256 * PARTS) void window_attn_tile_kernel(const WindowAttn a)
 		{
-			constexpr int KS = DK + 8, kPart = kWinKeys * (KS + DV);
+			constexpr int KS = DK + 8, kThreads = 256 * PARTS, kBlocks = DV / 16 / PARTS; // 16 value dimensions a block
 			extern __shared__ __attribute__((aligned(16))) uint16_t win_lds[];
-			const int part = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
-			uint16_t* const k_lds = win_lds + part * kPart; // [kWinKeys][KS]
-			uint16_t* const v_lds = k_lds + kWinKeys * KS;  // [kWinKeys][DV], permuted
-			const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
+			uint16_t* const k_lds = win_lds;               // [kWinKeys][KS]
+			uint16_t* const v_lds = k_lds + kWinKeys * KS; // [kWinKeys][DV], permuted
+			const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3;
+			const int first_block = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8) * kBlocks;
 			const int j = lane & 15, g = lane >> 4;
 			const int h = blockIdx.x;
 			const int tile = static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y);
@@ -728,51 +731,49 @@ namespace litenn_hip
 					}
 				}
 			}
-			floatx4 o[DV / 16];
+			floatx4 o[kBlocks];
 #pragma unroll
-			for (int b = 0; b < DV / 16; ++b)
+			for (int b = 0; b < kBlocks; ++b)
 			{
 				o[b] = floatx4{ 0.0f, 0.0f, 0.0f, 0.0f };
 			}
 			float run_m = -INFINITY, run_l = 0.0f;
 			constexpr int KP = DK / 8, VP = DV / 8;              // 16-byte pieces of a row
-			constexpr int KN = kWinKeys * KP / 256, VN = kWinKeys * VP / 256; // pieces a thread stages
+			constexpr int KN = kWinKeys * KP / kThreads, VN = kWinKeys * VP / kThreads; // pieces a thread stages
 			u32x4 kr[KN], vr[VN];
 			const auto request = [&](int base) {
 #pragma unroll
 				for (int i = 0; i < KN; ++i)
 				{
-					const int c = tid + 256 * i, key = min(base + c / KP, hi - 1), d = (c % KP) * 8;
+					const int c = tid + kThreads * i, key = min(base + c / KP, hi - 1), d = (c % KP) * 8;
 					kr[i] = d < dim ? *reinterpret_cast<const u32x4*>(keys + static_cast<size_t>(window_row(a, key)) * a.ldkv + d)
 					                : u32x4{ 0u, 0u, 0u, 0u };
 				}
 #pragma unroll
 				for (int i = 0; i < VN; ++i)
 				{
-					const int c = tid + 256 * i, key = min(base + c / VP, hi - 1), e = (c % VP) * 8;
+					const int c = tid + kThreads * i, key = min(base + c / VP, hi - 1), e = (c % VP) * 8;
 					vr[i] = e < vdim ? *reinterpret_cast<const u32x4*>(values + static_cast<size_t>(window_row(a, key)) * a.ldkv + e)
 					                 : u32x4{ 0u, 0u, 0u, 0u };
 				}
 			};
-			request(lo + part * kWinKeys);
-			// (a half whose last tile lies behind the last key stages that key again and hides it)
-			for (int from = lo; from < hi; from += PARTS * kWinKeys)
+			request(lo);
+			for (int base = lo; base < hi; base += kWinKeys)
 			{
-				const int base = from + part * kWinKeys;
 				__syncthreads(); // the previous tile has been consumed
 #pragma unroll
 				for (int i = 0; i < KN; ++i)
 				{
-					const int c = tid + 256 * i;
+					const int c = tid + kThreads * i;
 					*reinterpret_cast<u32x4*>(&k_lds[(c / KP) * KS + (c % KP) * 8]) = kr[i];
 				}
 #pragma unroll
 				for (int i = 0; i < VN; ++i)
 				{
-					const int c = tid + 256 * i;
+					const int c = tid + kThreads * i;
 					*reinterpret_cast<u32x4*>(&v_lds[win_value_at<DV>(c / VP, c % VP)]) = vr[i];
 				}
-				request(base + PARTS * kWinKeys);
+				request(base + kWinKeys);
 				__syncthreads();
 				// lane (j, g) gets keys base + 16 b + 4 g + 0..3 of query j
 				floatx4 s[4];
@@ -856,7 +857,7 @@ namespace litenn_hip
 				if (__any(corr != 1.0f)) // (past the first tiles a maximum seldom moves)
 				{
 #pragma unroll
-					for (int b = 0; b < DV / 16; ++b)
+					for (int b = 0; b < kBlocks; ++b)
 					{
 						o[b] *= corr;
 					}
@@ -864,7 +865,7 @@ namespace litenn_hip
 				// contraction index 8 g + e of step ks stands for key 16 (2 ks) + 4 g + e (e < 4) and key
 				// 16 (2 ks + 1) + 4 g + e - 4 (e >= 4)
 #pragma unroll
-				for (int b = 0; b < DV / 16; ++b)
+				for (int b = 0; b < kBlocks; ++b)
 				{
 #pragma unroll
 					for (int ks = 0; ks < 2; ++ks)
@@ -872,7 +873,7 @@ namespace litenn_hip
 						// four keys of sixteen dimensions: lane j of sixteen names eight bytes of a row and gets dimension j
 						typedef short short4v __attribute__((ext_vector_type(4)));
 						typedef __attribute__((address_space(3))) short4v* lds_short4;
-						const int key = 32 * ks + 4 * g + (j >> 2), piece = 2 * b + ((j & 3) >> 1), in = (j & 1) * 4;
+						const int key = 32 * ks + 4 * g + (j >> 2), piece = 2 * (first_block + b) + ((j & 3) >> 1), in = (j & 1) * 4;
 						const uint2 x = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(&v_lds[win_value_at<DV>(key, piece) + in])));
 						const uint2 y = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(&v_lds[win_value_at<DV>(key + 16, piece) + in])));
 						const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{ x.x, x.y, y.x, y.y });
@@ -882,38 +883,6 @@ namespace litenn_hip
 			}
 			run_l += __shfl_xor(run_l, 16, 64);
 			run_l += __shfl_xor(run_l, 32, 64);
-			if constexpr (PARTS == 2)
-			{
-				static_assert(sizeof(float) * (DV / 16 * 1024 + 512) <= sizeof(uint16_t) * 2 * kPart, "the halves' results");
-				float* const handed = reinterpret_cast<float*>(win_lds);
-				__syncthreads();
-				if (part == 1)
-				{
-#pragma unroll
-					for (int b = 0; b < DV / 16; ++b)
-					{
-						*reinterpret_cast<floatx4*>(handed + (b * 256 + tid) * 4) = o[b];
-					}
-					handed[DV / 16 * 1024 + tid] = run_m;
-					handed[DV / 16 * 1024 + 256 + tid] = run_l;
-				}
-				__syncthreads();
-				if (part == 1)
-				{
-					return;
-				}
-				// (one of the two may not have seen a key of this query)
-				const float other_m = handed[DV / 16 * 1024 + tid], other_l = handed[DV / 16 * 1024 + 256 + tid];
-				const float all_m = fmaxf(run_m, other_m), ref_m = all_m == -INFINITY ? 0.0f : all_m;
-				const float w0 = exp2_f32(run_m - ref_m), w1 = exp2_f32(other_m - ref_m);
-				run_m = all_m;
-				run_l = run_l * w0 + other_l * w1;
-#pragma unroll
-				for (int b = 0; b < DV / 16; ++b)
-				{
-					o[b] = o[b] * w0 + *reinterpret_cast<const floatx4*>(handed + (b * 256 + tid) * 4) * w1;
-				}
-			}
 			if (my_q >= a.rows)
 			{
 				return;
@@ -929,31 +898,31 @@ namespace litenn_hip
 			const float inv = weight / total * a.out_scale;
 			uint16_t* out = static_cast<uint16_t*>(a.out) + static_cast<size_t>(my_q) * a.ldo + static_cast<size_t>(h) * vdim;
 			const float* gate = a.gate ? a.gate + static_cast<size_t>(my_q) * a.ldg + static_cast<size_t>(h) * vdim : nullptr;
-			floatx4 gates[DV / 16];
+			floatx4 gates[kBlocks];
 			if (gate)
 			{
 				if ((vdim & 3) == 0) // whole groups of four, all on their way at once
 				{
 #pragma unroll
-					for (int b = 0; b < DV / 16; ++b)
+					for (int b = 0; b < kBlocks; ++b)
 					{
-						const int e = 16 * b + 4 * g;
+						const int e = 16 * (first_block + b) + 4 * g;
 						gates[b] = *reinterpret_cast<const floatx4_a4*>(gate + (e < vdim ? e : 0));
 					}
 				}
 				else
 				{
 #pragma unroll
-					for (int b = 0; b < DV / 16; ++b)
+					for (int b = 0; b < kBlocks; ++b)
 					{
-						gates[b] = load_columns(gate, 16 * b + 4 * g, vdim);
+						gates[b] = load_columns(gate, 16 * (first_block + b) + 4 * g, vdim);
 					}
 				}
 			}
 #pragma unroll
-			for (int b = 0; b < DV / 16; ++b)
+			for (int b = 0; b < kBlocks; ++b)
 			{
-				const int e = 16 * b + 4 * g;
+				const int e = 16 * (first_block + b) + 4 * g;
 				if (e < vdim)
 				{
 					floatx4 v = o[b] * inv;
@@ -1589,12 +1558,13 @@ namespace litenn_hip
 		{
 			const dim3 grid(a.shape.heads, (a.rows + kWinQ - 1) / kWinQ);
 			const auto launch = [&](auto kernel, int parts) {
-				const size_t lds = sizeof(uint16_t) * parts * kWinKeys * (DK + 8 + DV);
+				constexpr size_t lds = sizeof(uint16_t) * kWinKeys * (DK + 8 + DV);
 				allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
 				kernel<<<grid, dim3(256 * parts), lds, s>>>(a);
 			};
-			// Two halves where a CU has one workgroup at most (us, one part against two, heads of 128: 208 workgroups 24.7 and 19.2,
-			// 256 22.2 and 19.9, 416 29.8 and 33.6, 1024 76 and 95); wider heads have not the registers for two wavefronts a SIMD.
+			// Eight wavefronts where a CU has one workgroup at most (us, four against eight, heads of 128: 32 workgroups 10.5 and 9.1,
+			// 208 26.1 and 24.2, 256 33.5 and 31.6, 320 24.0 and 24.0, 512 42.9 and 48.9); wider heads have not the registers for two
+			// wavefronts a SIMD.
 			if constexpr (DK <= 128 && DV <= 128)
 			{
 				if (grid.x * static_cast<size_t>(grid.y) <= 256)

@@ -259,7 +259,25 @@ def test_gla_bfloat16_output_only_rounds_the_result(hip):
 @pytest.mark.parametrize("heads,dim,vdim", [(1, 128, 128), (3, 30, 50), (5, 24, 126), (9, 128, 72)])
 @pytest.mark.parametrize("m,keys,window", [(63, 63, 40), (65, 129, 64), (192, 257, 193), (2000, 2000, 150), (1900, 1964, 5000)])
 def test_window_attention_of_few_and_many_workgroups(hip, m, keys, window, heads, dim, vdim):
-    """Up to 256 tiles of 64 queries the key tiles are halved among a workgroup's wavefronts, beyond they are not: odd and
-    even numbers of key tiles, queries whose keys all lie in one half, heads that are no whole pieces."""
+    """Up to 256 tiles of 64 queries two wavefronts share a query's value dimensions, beyond one has them all: odd and even
+    numbers of key tiles, heads that are no whole pieces."""
     got, plain = window_case(hip, DT_BF16, m, keys, heads, dim, vdim, window, 0, keys - m, dim ** -0.5)
     assert rel_l2(got, plain()) <= WINDOW_LIMIT[DT_BF16]
+
+
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 64), (40, 126), (128, 24)])
+@pytest.mark.parametrize("m,keys,window", [(129, 300, 290), (500, 500, 1000), (700, 764, 130)])
+def test_window_attention_of_a_head_is_the_same_bits_whoever_goes_along(hip, m, keys, window, dim, vdim):
+    """A head alone and as one of as many as make more than 256 tiles of 64 queries, the first rows with and without the others."""
+    heads = 257 // -(-m // 64) + 1
+    rng = np.random.default_rng([m, keys, dim, vdim])
+    q = rng.normal(0, 1, (m, heads, dim)).astype(np.float32)
+    k, v = (to_bfloat16(rng.normal(0, 1, (keys, heads, d)).astype(np.float32)) for d in (dim, vdim))
+
+    def run(rows, used):
+        kv = np.concatenate([a[:keys - m + rows, :used].reshape(keys - m + rows, -1) for a in (k, v)], axis=1)
+        out = hip.window_attn(hip.Tensor.from_numpy(np.ascontiguousarray(q[:rows, :used])), bf16_tensor(hip, kv), rows, keys - m + rows,
+                              used, dim, vdim, window, dim ** -0.5, 0, keys - m)
+        return bf16_values(hip, out).reshape(rows, used, vdim)
+    every = run(m, heads)
+    assert np.array_equal(run(m, 1), every[:, :1]) and np.array_equal(run(m // 2, heads), every[:m // 2])
