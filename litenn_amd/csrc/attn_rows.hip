@@ -19,8 +19,8 @@
 // A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
 // a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
 // where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
-// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 36 us, where
-// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 91 us.  (43 and 109 with
+// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 34 us, where
+// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 93 us.  (40 and 108 with
 // a branch for each score's options, every tile masked and the cap's tangent always in the layer's form.)  Sums are
 // short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
 // addition per tile, which costs 4 us and leaves the error against 64 bits below the row kernel's (mean of six inputs, 1e-7:
@@ -230,6 +230,9 @@ namespace litenn_hip
 				const float ex = expf(__fmul_rn(v, 2.0f));
 				return __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
 			};
+			// Up to kSmallTangent its series, which is closer (the layer's form cancels: 1e-6 of a score of cap / 30).  Which of the
+			// two hangs on the score alone: neither hidden keys nor other queries change a query's bits.
+			const auto in_series = [](float v) { return fabsf(v) <= kSmallTangent; };
 			// a dot product's score (the causal mask and the window aside)
 			const auto score_of = [&](float v, float mv) {
 				if (a.apply_scale)
@@ -238,7 +241,7 @@ namespace litenn_hip
 				}
 				if (a.softcap != 0.0f)
 				{
-					v = layer_tanh(v);
+					v = in_series(v) ? small_tanh(v) : layer_tanh(v);
 					if (a.apply_cap)
 					{
 						v = __fmul_rn(v, a.softcap);
@@ -418,16 +421,16 @@ namespace litenn_hip
 				}
 				if (a.softcap != 0.0f)
 				{
-					// Capped scores are a small part of the cap as a rule: where all of the wavefront's are, the tangent's series takes
-					// seven instructions where the layer's form takes 35, and is closer (that form cancels: 1e-6 of a score of
-					// cap / 30, which was most of the error against 64 bits, 3.7e-7 -> 1.3e-7).
+					// Capped scores are a small part of the cap as a rule: the series takes seven instructions, the layer's form 35 more
+					// where a lane of the wavefront has a score that wants it (the call above with caps of 30 and 4: 34.2 and 38.9 us,
+					// with Float32 keys and a cap of 0.5 108; error against 64 bits 1.3e-7 where the layer's form alone has 3.7e-7).
 					float most = 0.0f;
 #pragma unroll
 					for (int e = 0; e < 16; ++e)
 					{
 						most = fmaxf(most, fabsf(sc[e])); // (a NaN stays one in either form)
 					}
-					if (__all(most <= kSmallTangent))
+					if (__all(in_series(most)))
 					{
 #pragma unroll
 						for (int e = 0; e < 16; ++e)
@@ -440,7 +443,14 @@ namespace litenn_hip
 #pragma unroll
 						for (int e = 0; e < 16; ++e)
 						{
-							sc[e] = layer_tanh(sc[e]);
+							const float near = small_tanh(sc[e]);
+							float far = layer_tanh(sc[e]);
+							asm("" : "+v"(far)); // (a choice, not a branch for each score)
+							sc[e] = in_series(sc[e]) ? near : far;
+							if (e == 7)
+							{
+								__builtin_amdgcn_sched_barrier(0); // (sixteen at once want registers that spill)
+							}
 						}
 					}
 					if (a.apply_cap)

@@ -184,3 +184,22 @@ def test_soft_caps_on_both_sides_of_the_series(hip, dtype, spread, m, keys):
     got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=1.0, logit_softcap=cap,
                              causal=True, query_position_offset=keys - m).numpy()
     assert worst(got, plain(*(a.astype(np.float64) for a in (q, k, v)), 1.0, keys - m, softcap=cap)) <= 4e-6
+
+
+@pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
+@pytest.mark.parametrize("m,keys", [(33, 129), (64, 64), (40, 700)])
+def test_soft_caps_of_a_query_hang_on_its_own_scores_alone(hip, dtype, m, keys):
+    """Keys that the first rows do not see, and the other queries, grow beyond the series' range: the first rows keep their bits."""
+    heads, dim, seen = 3, 64, m // 3
+    q, k, v = inputs(6, m, keys, heads, 1, dim, dtype)
+    T = hip.Tensor.from_numpy
+
+    def run(q, k):
+        got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, 1, dim, scale=0.01, logit_softcap=7.0, causal=True,
+                                 query_position_offset=keys - m).numpy()
+        return got[:seen]
+    hidden, others = k.copy(), q.copy()
+    hidden[keys - m + seen:] *= 16
+    others[seen:] *= 300
+    want = run(q, k)
+    assert np.array_equal(run(q, hidden), want) and np.array_equal(run(others, k), want)
