@@ -1029,34 +1029,29 @@ namespace litenn_hip
 			}
 			return;
 		}
-		// Time = workgroups a CU has in a row, each a fixed part and so many ns a tile of K, fitted to 18 shapes from 100 x 4096 x 4096
-		// to 2048 x 28672 x 4096 with weights from HBM (more of them in turn than the 256 MB cache holds; a model's are never
-		// there either, and tuned with weights that are, the choice cost a tenth).  The form it picks is 1 % slower than the best
-		// in the mean, 11 % at 777 x 6432 x 2048.  us for 256 x 256, 128 x 256, 192 x 128, 128 x 192, 128 x 64, 64 x 128, 64 x 64, 32 x 64
-		// and the best of dense_tile_kernel: 2048 x 28672 x 4096 462, 488, 487, 541, 672, 684, 802, 1184 and 551; 777 x 11264 x 2048 68,
-		// 72, 52, 63, 66, 69, 79, 108 and 63; 777 x 2048 x 5632 133, 79, 82, 65, 38, 41, 45, 60 and 46; 500 x 2048 x 5632 140, 82, 83, 66,
-		// 40, 42, 28, 36 and 31; 100 x 4096 x 4096 95, 59, 60, 48, 29, 30, 20, 15.5 and 20.
-		// 32 x 32 against 32 x 64: 30 x 4096 x 14336 38 and 54, 60 x 2048 x 5632 15.5 and 22, 3 x 28672 x 4096 43.2 and 42.4.
+		// us, weights from HBM, for 256 x 256, 128 x 256, 192 x 128 (three buffers), 128 x 192, 128 x 128 (three), 128 x 64, 64 x 128,
+		// 64 x 64, 32 x 64, 32 x 32 and the best of dense_tile_kernel: 2048 x 28672 x 4096 451, 468, 523, 529, 573, 650, 670, more, more, more and 528;
+		// 639 x 4096 x 14336 313, 195, 151, 161, 133, 162, 169, 162, 196, 254 and 136; 777 x 2048 x 5632 132, 79, 63, 64, 50, 39, 42, 46,
+		// 62, 71 and 44; 320 x 6160 x 2048 58, 35, 29, 30, 24, 28, 21, 24, 30, 39 and 22; 33 x 4096 x 14336 in four ranges 80, 52, 43, 42,
+		// 35, 29, 32, 23, 29, 34 and 24; 17 x 13888 x 4096 90, 58, 47, 46, 38, 32, 35, 27, 26, 26 and 26.  Two buffers instead of
+		// three: 1280 x 6432 x 2048 128 x 128 40 and 52, 192 x 128 46 (777 x 11264 x 2048 49 and 57).
 		const auto on16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
 		const auto reach = [](size_t rows, size_t pitch) { return rows * pitch * sizeof(uint16_t) <= 0xffffffffu; }; // 32-bit offsets
 		if (on16(a.a) && on16(a.w.w) && a.lda % 8 == 0 && reach(std::max(a.m, a.a_ring), a.lda) && reach(a.w.n, a.w.pitch))
 		{
-			const auto cost = [&](int bm, int bn, int fixed, int step) {
-				return static_cast<long long>((work(bm, bn) + 255) / 256) * (fixed + static_cast<long long>(step) * (a.w.pitch / kTileK / a.splits));
-			};
-			const long long costs[] = { cost(256, 256, 7900, 1475), cost(128, 256, 3700, 867), cost(192, 128, 5700, 663), cost(128, 192, 3900, 725),
-				                        cost(128, 64, 100, 372),    cost(64, 128, 400, 382),   cost(64, 64, 300, 256),    cost(32, 64, 700, 179),
-				                        cost(32, 32, 300, 145) };
-			switch (std::min_element(std::begin(costs), std::end(costs)) - costs)
+			switch (fetch::dense_form(a.w.n, a.w.pitch / kTileK, a.m, a.splits))
 			{
-			case 0: return launch_ring<256, 256, 2, 4, 2>(args, s);
-			case 1: return launch_ring<128, 256, 2, 4, 3>(args, s);
-			case 2: return launch_ring<192, 128, 4, 2, 2>(args, s);
-			case 3: return launch_ring<128, 192, 2, 4, 3>(args, s);
-			case 4: return launch_ring<128, 64, 4, 2, 3>(args, s);
-			case 5: return launch_ring<64, 128, 2, 4, 3>(args, s);
-			case 6: return launch_ring<64, 64, 2, 2, 4>(args, s);
-			case 7: return launch_ring<32, 64, 1, 4, 6>(args, s);
+			case fetch::kDense256x256: return launch_ring<256, 256, 2, 4, 2>(args, s);
+			case fetch::kDense128x256: return launch_ring<128, 256, 2, 4, 3>(args, s);
+			case fetch::kDense192x128: return launch_ring<192, 128, 4, 2, 2>(args, s);
+			case fetch::kDense192x128x3: return launch_ring<192, 128, 4, 2, 3>(args, s);
+			case fetch::kDense128x192: return launch_ring<128, 192, 2, 4, 3>(args, s);
+			case fetch::kDense128x128: return launch_ring<128, 128, 4, 2, 2>(args, s);
+			case fetch::kDense128x128x3: return launch_ring<128, 128, 4, 2, 3>(args, s);
+			case fetch::kDense128x64: return launch_ring<128, 64, 4, 2, 3>(args, s);
+			case fetch::kDense64x128: return launch_ring<64, 128, 2, 4, 3>(args, s);
+			case fetch::kDense64x64: return launch_ring<64, 64, 2, 2, 4>(args, s);
+			case fetch::kDense32x64: return launch_ring<32, 64, 1, 4, 6>(args, s);
 			default: return launch_ring<32, 32, 2, 2, 8>(args, s);
 			}
 		}

@@ -63,6 +63,52 @@ namespace litenn_hip
 			return rows > ranged ? rows : ranged;
 		}
 
+		// The form a product of bfloat16 operands takes, activation rows x weight rows of a tile; the two with a digit behind
+		// differ in the buffers of their ring.  (All give the same bits.)
+		enum DenseForm
+		{
+			kDense256x256, kDense128x256, kDense192x128, kDense192x128x3, kDense128x192, kDense128x128, kDense128x128x3,
+			kDense128x64, kDense64x128, kDense64x64, kDense32x64, kDense32x32, kDenseForms
+		};
+		// The form of least time, where a CU has r workgroups of it: ns of a workgroup by itself (a fixed part and one a tile of K) and
+		// of two that share a CU, r / 2 pairs and the odd one; a form whose ring leaves room for one only takes them in a row.
+		// Fitted to 925 products with weights from HBM (25 matrices of the layered decoders' widths, 37 numbers of rows
+		// from 17 to 2048): 0.3 % slower than the fastest form in the mean, 15 % at most, and at matrices kept out of the fit 0.5 %.
+		// With one time for a workgroup whether it shares its CU or not, and without 128 x 128, tiles in a row took up to 1.6 times
+		// as long: us for 639 x 4096 x 14336 in 192 x 128 with two buffers 201, 128 x 128 with three 132; 178 rows in three
+		// ranges 78, 45; 1100 x 2048 x 5632 85, 51.
+		inline DenseForm dense_form(int n, int k_tiles, int m, int ranges)
+		{
+			struct Cost
+			{
+				int rows, columns, alone, alone_tile, pair, pair_tile;
+			};
+			constexpr Cost costs[kDenseForms] = {
+				{ 256, 256, 19800, 1350, 0, 0 },     { 128, 256, 8760, 860, 0, 0 },    { 192, 128, 6580, 860, 10510, 1120 },
+				{ 192, 128, 7380, 660, 0, 0 },       { 128, 192, 7370, 690, 0, 0 },    { 128, 128, 4350, 770, 8090, 900 },
+				{ 128, 128, 5180, 560, 0, 0 },       { 128, 64, 3650, 420, 5360, 640 }, { 64, 128, 3570, 450, 5460, 720 },
+				{ 64, 64, 3230, 290, 3570, 450 },    { 32, 64, 2830, 240, 3130, 330 }, { 32, 32, 2840, 170, 2820, 270 },
+			};
+			const int tiles_of_k = imax(1, k_tiles / ranges);
+			int best = 0;
+			long long least = -1;
+			for (int form = 0; form < kDenseForms; ++form)
+			{
+				const Cost& c = costs[form];
+				const long long workgroups = static_cast<long long>((m + c.rows - 1) / c.rows) * ((n + c.columns - 1) / c.columns) * ranges;
+				const long long in_a_cu = (workgroups + 255) / 256;
+				const long long alone = c.alone + static_cast<long long>(c.alone_tile) * tiles_of_k;
+				const long long pair = c.pair + static_cast<long long>(c.pair_tile) * tiles_of_k;
+				const long long time = c.pair ? in_a_cu / 2 * pair + in_a_cu % 2 * alone : in_a_cu * alone;
+				if (least < 0 || time < least)
+				{
+					least = time;
+					best = form;
+				}
+			}
+			return static_cast<DenseForm>(best);
+		}
+
 		// ---- matrix-core GEMM: raw weight blocks of one 256-element chunk per row --------------
 		// A wavefront owns 16 * ng consecutive rows; their chunks land in its LDS slot row after row
 		// as `pieces` 16-byte pieces each.  Formats whose chunks start on 16-byte boundaries take

@@ -671,6 +671,54 @@ static void test_dense_walks()
 	std::printf("bfloat16 products: %ld tiles of K walked\n", walked);
 }
 
+// The form a product of bfloat16 operands takes against what all of them took (us on the card, weights from HBM, forms in
+// the order of DenseForm, 0 not measured): never 5 % more than the fastest.
+static void test_dense_forms()
+{
+	using namespace litenn_hip::fetch;
+	struct Measured
+	{
+		int n, k, ranges, m;
+		double us[kDenseForms];
+	};
+	const Measured measured[] = {
+		{ 4096, 14336, 1, 639, { 313.1, 195.0, 201.1, 150.6, 160.5, 191.6, 132.7, 162.2, 168.8, 162.3, 195.9, 254.4 } },
+		{ 4096, 14336, 3, 178, { 117.1, 72.4, 77.8, 60.2, 58.3, 68.3, 45.8, 55.3, 65.4, 63.8, 73.7, 88.5 } },
+		{ 4096, 14336, 4, 33, { 79.5, 52.2, 55.6, 42.5, 41.9, 51.9, 34.5, 28.5, 32.0, 23.3, 28.5, 34.2 } },
+		{ 4096, 4096, 4, 96, { 31.5, 22.2, 21.0, 17.6, 19.1, 19.6, 16.0, 13.6, 14.1, 14.4, 17.6, 21.7 } },
+		{ 28672, 4096, 1, 178, { 105.7, 69.6, 75.2, 61.7, 98.6, 75.4, 83.2, 90.2, 87.8, 102.1, 129.7, 166.0 } },
+		{ 28672, 4096, 1, 2048, { 450.6, 467.7, 467.8, 523.4, 529.0, 490.6, 573.0, 650.3, 669.8, 0, 0, 0 } },
+		{ 13888, 4096, 1, 17, { 89.6, 57.6, 62.0, 46.8, 45.9, 58.5, 38.3, 32.2, 35.0, 26.8, 25.5, 25.6 } },
+		{ 6160, 2048, 1, 320, { 58.4, 35.3, 37.2, 29.1, 29.6, 33.3, 24.0, 28.2, 21.4, 23.6, 30.3, 38.9 } },
+		{ 6432, 2048, 1, 1280, { 62.4, 67.4, 46.1, 57.7, 59.4, 40.0, 51.8, 57.4, 57.7, 67.0, 84.5, 123.7 } },
+		{ 11264, 2048, 1, 777, { 60.5, 66.6, 48.6, 56.7, 59.3, 68.7, 64.3, 63.2, 67.8, 75.8, 100.1, 140.9 } },
+		{ 2048, 5632, 1, 777, { 131.8, 79.3, 83.3, 62.8, 63.7, 77.5, 49.8, 39.0, 42.3, 46.0, 61.6, 71.2 } },
+		{ 2048, 5632, 2, 512, { 80.1, 48.4, 48.0, 37.8, 40.3, 44.0, 33.7, 26.2, 27.1, 29.6, 39.9, 51.1 } },
+		{ 1024, 2816, 2, 48, { 34.6, 23.8, 24.2, 19.1, 19.6, 22.5, 16.3, 12.8, 15.0, 10.7, 8.9, 6.9 } },
+	};
+	for (const Measured& p : measured)
+	{
+		double least = p.us[0];
+		for (double us : p.us)
+		{
+			least = us > 0.0 && us < least ? us : least;
+		}
+		const DenseForm form = dense_form(p.n, p.k / 64, p.m, p.ranges);
+		CHECK(p.us[form] > 0.0 && p.us[form] <= 1.05 * least, "%d x %d x %d in %d ranges: form %d", p.m, p.n, p.k, p.ranges, static_cast<int>(form));
+	}
+	for (int m = 1; m <= 4096; m += 1 + m / 3) // any size has one
+	{
+		for (int n = 1; n <= 40000; n += 1 + n / 2)
+		{
+			for (int tiles : { 1, 2, 3, 7, 64, 300 })
+			{
+				const int form = dense_form(n, tiles, m, dense_ranges(n, tiles, m));
+				CHECK(form >= 0 && form < kDenseForms, "%d x %d x %d tiles: form %d", m, n, tiles, form);
+			}
+		}
+	}
+}
+
 // The sums of a sublayer's last product lie in a buffer made for the longest pass so far: any shorter one's, in
 // its ranges of K, must fit (widths and K of layered decoders, and small odd ones).
 static void test_dense_sum_rows()
@@ -698,9 +746,18 @@ static void test_dense_sum_rows()
 	std::printf("sums in ranges of K: %ld of %ld passes\n", ranged, passes);
 }
 
-int main()
+int main(int argc, char** argv)
 {
+	if (argc > 1) // n k m ...: the forms of these products
+	{
+		for (int i = 1; i + 2 < argc; i += 3)
+		{
+			std::printf("%d\n", static_cast<int>(litenn_hip::fetch::dense_form(std::atoi(argv[i]), (std::atoi(argv[i + 1]) + 63) / 64, std::atoi(argv[i + 2]), 1)));
+		}
+		return 0;
+	}
 	test_dense_walks();
+	test_dense_forms();
 	test_dense_sum_rows();
 	test_gemm_chunk_ranges();
 	test_gemm_weight_pieces();

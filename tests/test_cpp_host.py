@@ -44,3 +44,14 @@ def test_fetch_patterns_stay_inside_their_tensors():
     assert p.returncode == 0, p.stdout[-3000:] + p.stderr
     assert "fetch bounds ok" in p.stdout and "FAIL" not in p.stdout
     assert "pieces behind the tensor before the fix, 0 now" in p.stdout
+
+
+def dense_forms(products):
+    """The forms of products of bfloat16 operands (n, k, m), as numbers of csrc/fetch_model.hpp's DenseForm."""
+    p = subprocess.run([hip_build.FETCH_TEST_BIN, *(str(v) for s in products for v in s)], capture_output=True, text=True, timeout=60)
+    return [int(f) for f in p.stdout.split()]
+
+
+def test_products_that_the_gpu_tests_multiply_take_every_form():
+    from test_gpu_layer_ops import EVERY_FORM
+    assert set(dense_forms(EVERY_FORM)) == set(range(12))

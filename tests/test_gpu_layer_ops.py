@@ -66,12 +66,16 @@ def test_linear_bf16_larger(hip, n, k, m):
     assert rel_l2(y, from_bfloat16(xb).astype(np.float64) @ from_bfloat16(w).astype(np.float64).T) <= 2e-6
 
 
-@pytest.mark.parametrize("n,k,m", [(8192, 300, 2048), (8000, 4300, 1000), (11200, 2050, 760), (6432, 1290, 777), (8000, 300, 1000),
-                                   (11264, 700, 300), (2030, 700, 490), (4090, 700, 100), (2000, 700, 33), (2030, 65, 490), (2030, 1, 490), (4100, 64, 20)])
+# products that between them take every form of csrc/fetch_model.hpp's dense_form (tests/test_cpp_host.py holds them to it)
+EVERY_FORM = [(8192, 300, 2048), (8000, 4300, 1000), (11200, 2050, 760), (6432, 1290, 777), (8000, 300, 1000),
+              (11264, 700, 300), (2030, 700, 490), (4090, 700, 100), (2000, 700, 33), (2030, 65, 490), (2030, 1, 490), (4100, 64, 20),
+              (12300, 700, 1000), (11200, 300, 500), (11200, 300, 130), (11200, 300, 70), (20000, 65, 250), (28600, 65, 130), (11200, 130, 377)]
+
+
+@pytest.mark.parametrize("n,k,m", EVERY_FORM)
 def test_linear_bf16_in_every_form(hip, n, k, m):
-    """256 x 256, 128 x 256, 192 x 128, 128 x 192, 128 x 64, 64 x 128, 64 x 64, 32 x 64, 32 x 32 in turn: rows fewer than a tile's, fewer
-    tiles of K than a ring has buffers, a last tile that is not whole behind none, one and many.  Operands off their 16 bytes
-    give the same."""
+    """Rows fewer than a tile's, fewer tiles of K than a ring has buffers, a last tile that is not whole behind none, one and
+    many.  Operands off their 16 bytes give the same."""
     rng = np.random.default_rng([n, k, m])
     w, xb = padded_bits(rng.normal(0, 1, (n, k)).astype(np.float32)), padded_bits(rng.normal(0, 1, (m, k)).astype(np.float32), NAN16)
     y = hip.linear_bf16(bf16_tensor(hip, w), n, k, bf16_tensor(hip, xb), m).numpy()
