@@ -972,10 +972,9 @@ namespace litenn_hip
 			for (int i = 0; i < kArgmaxChunk / 256; ++i)
 			{
 				const int at = begin + static_cast<int>(threadIdx.x) + 256 * i;
-				if (at < end && (v[i] > best || best_i == 0x7fffffff))
+				if (at < end)
 				{
-					best = v[i];
-					best_i = at;
+					argmax_take(v[i], at, best, best_i); // (a NaN is not: it would hide what comes behind it)
 				}
 			}
 			for (int off = 32; off > 0; off >>= 1)

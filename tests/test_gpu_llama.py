@@ -439,6 +439,32 @@ def test_the_first_of_equal_logits_is_taken(hip, vocab):
     assert got[0] == want
 
 
+@pytest.mark.parametrize("first", [0, 1024, 1280])
+def test_logits_that_are_not_numbers_hide_no_other(hip, first):
+    """256 NaN in a row, which is what the lanes of a workgroup look at first, and the largest logits behind them."""
+    cfg = synth.tiny_llama(Q8_0, block_count=1, d_model=256, heads=2, kv_heads=1, ff=256, vocab=2048, context_length=32)
+
+    def tensors():
+        for kind, layer, fmt, payload, n, k in synth.llama_tensors(cfg, 3):
+            if kind == "output":
+                blocks = payload.reshape(n, -1, 34).copy()
+                rows = np.arange(n)
+                blocks[(rows < first) | (rows >= first + 768), :, :2] = 0  # logits of zero
+                blocks[first:first + 256, :, :2] = np.frombuffer(np.float16(np.nan).tobytes(), np.uint8)
+                payload = blocks.reshape(payload.shape)
+            yield kind, layer, fmt, payload, n, k
+    m = hip_model(hip, cfg, 3, tensors=tensors())
+    prompt = synth.prompt_tokens(cfg, 5, 9)
+    got = m.generate(prompt, 8)[0].tolist()
+    m.reset()
+    logits, want = m.eval(prompt)[-1], []
+    for _ in range(8):
+        assert np.isnan(logits[first:first + 256]).all() and np.nanmax(logits) > 0
+        want.append(int(np.nanargmax(logits)))
+        logits = m.eval(want[-1:])[0]
+    assert got == want
+
+
 @pytest.mark.parametrize("head_dim,rope", [(6, 6), (6, 2), (8, 8), (8, 2), (12, 6), (20, 10), (128, 64)])
 @pytest.mark.parametrize("kv", [DT_F16, DT_F32])
 def test_rotations_that_end_inside_four_features(hip, oracle, head_dim, rope, kv):
