@@ -796,6 +796,7 @@ namespace litenn_hip
 		                                                                    const float* residual, int k, int m, int m_tiles,
 		                                                                    int chunks, size_t row_bytes)
 		{
+			static_assert(F::kMins && F::kScaleSteps == 16, "one scale for a chunk, minima beside it");
 			constexpr int kPieces = MT * 8 / WN; // 1 KB pieces a wavefront stages
 			static_assert(kPieces * WN == MT * 8, "activation pieces / wavefront split");
 			typedef WeightPieces<F> W;
@@ -816,7 +817,7 @@ namespace litenn_hip
 			}
 
 			floatx16 acc[MT], p[MT];
-			floatx16 held[MT]; // the chunk's sums so far or, where one scale is all of it, its first half
+			floatx16 held[MT]; // the chunk's first half
 #pragma unroll
 			for (int t = 0; t < MT; ++t)
 			{
@@ -910,7 +911,7 @@ namespace litenn_hip
 								weights.request(moving, min(c + 2, c_end - 1), lane);
 							}
 						}
-						if (F::kMins && step == 11)
+						if (step == 11)
 						{
 #pragma unroll
 							for (int t = 0; t < MT; ++t)
@@ -933,7 +934,7 @@ namespace litenn_hip
 						}
 						__builtin_amdgcn_sched_barrier(0);
 						const half8 low = lowered(b[mine]);
-						const bool fresh = step % min(F::kScaleSteps, 8) == 0;
+						const bool fresh = step % 8 == 0;
 #pragma unroll
 						for (int e = 0; e < 2; ++e)
 						{
@@ -951,31 +952,12 @@ namespace litenn_hip
 						{
 							b[other] = F::frag(st < 3 ? head : next_head, next_raw, (st + 1) & 3, 0);
 						}
-						if constexpr (F::kMins)
+						if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
 						{
-							if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
+#pragma unroll
+							for (int t = 0; t < MT; ++t)
 							{
-#pragma unroll
-								for (int t = 0; t < MT; ++t)
-								{
-									held[t] = p[t];
-								}
-							}
-						}
-						if constexpr (F::kScaleSteps < 16)
-						{
-							if (step % F::kScaleSteps == F::kScaleSteps - 1)
-							{
-								const float d = F::scale(head, raw, st, s);
-#pragma unroll
-								for (int t = 0; t < MT; ++t)
-								{
-#pragma unroll
-									for (int e = 0; e < 16; ++e)
-									{
-										held[t][e] = step == F::kScaleSteps - 1 ? d * p[t][e] : fmaf(d, p[t][e], held[t][e]);
-									}
-								}
+								held[t] = p[t];
 							}
 						}
 						__builtin_amdgcn_sched_barrier(0);
@@ -983,32 +965,17 @@ namespace litenn_hip
 					raw = next_raw;
 				}
 				const float d = F::chunk_scale(head);
-				if constexpr (F::kMins)
+				const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
+				const float dm = F::min_scale(head) * (1.0f / kSumScale);
+#pragma unroll
+				for (int t = 0; t < MT; ++t)
 				{
-					const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
-					const float dm = F::min_scale(head) * (1.0f / kSumScale);
+					const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
+					const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
 #pragma unroll
-					for (int t = 0; t < MT; ++t)
+					for (int e = 0; e < 16; ++e)
 					{
-						const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
-						const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
-#pragma unroll
-						for (int e = 0; e < 16; ++e)
-						{
-							acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
-						}
-					}
-				}
-				else
-				{
-#pragma unroll
-					for (int t = 0; t < MT; ++t)
-					{
-#pragma unroll
-						for (int e = 0; e < 16; ++e)
-						{
-							acc[t][e] = fmaf(d, held[t][e], acc[t][e]);
-						}
+						acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
 					}
 				}
 				head = next_head;
