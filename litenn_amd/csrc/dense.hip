@@ -2,7 +2,7 @@
 //
 // One row (decode) streams the weights once through registers with Float32 activations in LDS; many
 // rows (prompt) run on the matrix cores, either with bfloat16 operands or, where Float32 operands are
-// asked for, with v_mfma_f32_16x16x4_f32 and the weights widened exactly.  Every accumulation is
+// asked for, with each activation taken apart exactly into three bfloat16 values.  Every accumulation is
 // Float32.  The reference has no counterpart (its linears are f32 MatMul nodes,
 // src/LiteNN/Layer/Linear.h:67-95).
 #include "dense.hpp"
@@ -10,8 +10,6 @@
 #include <algorithm>
 #include <iterator>
 #include <type_traits>
-
-#pragma clang diagnostic ignored "-Winline-asm" // m0 is named as clobbered although it is reserved
 
 namespace litenn_hip
 {
@@ -807,10 +805,13 @@ namespace litenn_hip
 #pragma unroll
 				for (int i = 0; i < L; ++i)
 				{
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm" // m0 is named as clobbered although it is reserved
 					asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
 					             :
 					             : "s"(to + i * (W * 1024)), "v"(from[i]), "s"(i < LA ? a : w)
 					             : "memory", "m0");
+#pragma clang diagnostic pop
 				}
 			};
 			// this lane's piece of the first fragment, by half of the tile
