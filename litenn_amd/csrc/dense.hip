@@ -998,37 +998,14 @@ namespace litenn_hip
 		const auto work = [&](int bm, int bn) { return tiles(a, bm, bn) * a.splits; };
 		if (a.f32)
 		{
-			// Beyond 256 tiles of 64 x 128 a product is one chain over K, up to there two halves (results hang on this alone).  us a
-			// tile of K takes of each workgroup a CU has in a row, fitted to 16 shapes from 30 x 4096 x 2048 to 1000 x 11264 x 4096; us
-			// for 64 x 128, 64 x 256: 500 rows by 11264 x 2048 85, 95, by 6432 x 2048 57, 51; for 64 x 128, 64 x 64, 32 x 64 in halves: 300
-			// rows by 4096 x 4096 58, 78, 70, 500 by 2048 x 5632 76, 59, 66, 100 by 2048 x 2048 28, 20, 15.
-			const auto in_a_row = [&](int bm, int bn) { return (work(bm, bn) + 255) / 256; };
-			if (a.m > 32 && work(64, 128) > 256)
+			switch (fetch::dense_f32_form(a.w.n, a.m, a.splits))
 			{
-				if (83 * in_a_row(64, 128) <= 147 * in_a_row(64, 256))
-				{
-					launch_tile<64, 128, 2, 4, 1, 2, true>(args, s);
-				}
-				else
-				{
-					launch_tile<64, 256, 2, 4, 1, 2, true>(args, s);
-				}
-				return;
+			case fetch::kF32Chain64x128: return launch_tile<64, 128, 2, 4, 1, 2, true>(args, s);
+			case fetch::kF32Chain64x256: return launch_tile<64, 256, 2, 4, 1, 2, true>(args, s);
+			case fetch::kF32Halves64x128: return launch_tile<64, 128, 2, 4, 2, 2, true>(args, s);
+			case fetch::kF32Halves64x64: return launch_tile<64, 64, 2, 4, 2, 2, true>(args, s);
+			default: return launch_tile<32, 64, 1, 4, 2, 2, true>(args, s);
 			}
-			const int tall = 88 * in_a_row(64, 128), square = 64 * in_a_row(64, 64), low = 37 * in_a_row(32, 64);
-			if (a.m <= 32 || low <= std::min(tall, square))
-			{
-				launch_tile<32, 64, 1, 4, 2, 2, true>(args, s);
-			}
-			else if (tall <= square)
-			{
-				launch_tile<64, 128, 2, 4, 2, 2, true>(args, s);
-			}
-			else
-			{
-				launch_tile<64, 64, 2, 4, 2, 2, true>(args, s);
-			}
-			return;
 		}
 		// us, weights from HBM, for 256 x 256, 128 x 256, 192 x 128 (three buffers), 128 x 192, 128 x 128 (three), 128 x 64, 64 x 128,
 		// 64 x 64, 32 x 64, 32 x 32 and the best of dense_tile_kernel: 2048 x 28672 x 4096 451, 468, 523, 529, 573, 650, 670, more, more, more and 528;

@@ -109,6 +109,28 @@ namespace litenn_hip
 			return static_cast<DenseForm>(best);
 		}
 
+		// The form a product of Float32 operands takes.  Beyond 256 tiles of 64 x 128 it is one chain over K, up to there, and for
+		// 32 rows and fewer, two halves: results hang on this alone.  Time is what a tile of K takes of each workgroup that a CU
+		// has in a row, tens of ns, fitted to 16 shapes from 30 x 4096 x 2048 to 1000 x 11264 x 4096; us for 64 x 128 and 64 x 256: 512
+		// rows by 11264 x 2048 75, 85, by 7200 x 2048 52, 46; for 64 x 128, 64 x 64, 32 x 64 in halves: 512 rows by 2048 x 5632 in two
+		// ranges 44, 57, 59, 64 by 11264 x 2048 31, 23, 26, 96 by 2048 x 2048 in two ranges 18, 13, 11.
+		enum DenseF32Form { kF32Chain64x128, kF32Chain64x256, kF32Halves32x64, kF32Halves64x128, kF32Halves64x64, kDenseF32Forms };
+		inline DenseF32Form dense_f32_form(int n, int m, int ranges)
+		{
+			const auto workgroups = [&](int rows, int columns) { return ((m + rows - 1) / rows) * ((n + columns - 1) / columns) * ranges; };
+			const auto in_a_row = [&](int rows, int columns) { return (workgroups(rows, columns) + 255) / 256; };
+			if (m > 32 && workgroups(64, 128) > 256)
+			{
+				return 83 * in_a_row(64, 128) <= 147 * in_a_row(64, 256) ? kF32Chain64x128 : kF32Chain64x256;
+			}
+			const int tall = 88 * in_a_row(64, 128), square = 64 * in_a_row(64, 64), low = 37 * in_a_row(32, 64);
+			if (m <= 32 || low <= imin(tall, square))
+			{
+				return kF32Halves32x64;
+			}
+			return tall <= square ? kF32Halves64x128 : kF32Halves64x64;
+		}
+
 		// ---- matrix-core GEMM: raw weight blocks of one 256-element chunk per row --------------
 		// A wavefront owns 16 * ng consecutive rows; their chunks land in its LDS slot row after row
 		// as `pieces` 16-byte pieces each.  Formats whose chunks start on 16-byte boundaries take

@@ -748,11 +748,13 @@ static void test_dense_sum_rows()
 
 int main(int argc, char** argv)
 {
-	if (argc > 1) // n k m ...: the forms of these products
+	if (argc > 1) // n k m ...: the forms of these products, with bfloat16 and with Float32 operands
 	{
 		for (int i = 1; i + 2 < argc; i += 3)
 		{
-			std::printf("%d\n", static_cast<int>(litenn_hip::fetch::dense_form(std::atoi(argv[i]), (std::atoi(argv[i + 1]) + 63) / 64, std::atoi(argv[i + 2]), 1)));
+			const int n = std::atoi(argv[i]), k_tiles = (std::atoi(argv[i + 1]) + 63) / 64, m = std::atoi(argv[i + 2]);
+			std::printf("%d %d\n", static_cast<int>(litenn_hip::fetch::dense_form(n, k_tiles, m, 1)),
+			            static_cast<int>(litenn_hip::fetch::dense_f32_form(n, m, 1)));
 		}
 		return 0;
 	}

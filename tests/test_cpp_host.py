@@ -47,11 +47,17 @@ def test_fetch_patterns_stay_inside_their_tensors():
 
 
 def dense_forms(products):
-    """The forms of products of bfloat16 operands (n, k, m), as numbers of csrc/fetch_model.hpp's DenseForm."""
+    """The forms of products (n, k, m) as numbers of csrc/fetch_model.hpp's DenseForm and DenseF32Form."""
     p = subprocess.run([hip_build.FETCH_TEST_BIN, *(str(v) for s in products for v in s)], capture_output=True, text=True, timeout=60)
-    return [int(f) for f in p.stdout.split()]
+    return list(zip(*(map(int, line.split()) for line in p.stdout.splitlines())))
 
 
 def test_products_that_the_gpu_tests_multiply_take_every_form():
+    import test_gpu_dense_tiles as tiles
     from test_gpu_layer_ops import EVERY_FORM
-    assert set(dense_forms(EVERY_FORM)) == set(range(12))
+    assert set(dense_forms(EVERY_FORM)[0]) == set(range(12))
+    assert set(dense_forms(tiles.SHAPES)[1]) == set(range(5))
+    # one row's bits in one form after the other
+    n, rows = tiles.SAME_BITS[0], tiles.SAME_BITS[1:]
+    for k in tiles.SAME_BITS_K:
+        assert len(set(dense_forms([(n, k, m) for m in rows])[0])) >= 8

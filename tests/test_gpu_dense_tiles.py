@@ -11,10 +11,14 @@ from test_gpu_layer_ops import NAN16, NAN32, bf16_tensor, padded_bits, pitch
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(49200, 64, 65), (12300, 200, 129),                    # bfloat16 128 x 128, 32 x 64; Float32 64 x 128
-          (6210, 3100, 130), (3100, 64, 200), (3137, 192, 193),  # 32 x 64, 64 x 64; 32 x 64 on two groups
-          (6200, 320, 250), (12290, 100, 250),                   # 64 x 128, 128 x 128; 64 x 128 on two groups, on one
-          (40, 64, 33), (700, 1088, 40), (1030, 4096, 7)]        # 32 x 64
+# the forms of csrc/fetch_model.hpp that they take (tests/test_cpp_host.py holds SHAPES to all of Float32's, SAME_BITS to
+# most of bfloat16's)
+SHAPES = [(49200, 64, 65), (12300, 200, 129), (12290, 100, 250),                   # Float32 64 x 256
+          (11264, 200, 500), (11200, 205, 760), (11200, 64, 500),                  # 64 x 128 as one chain
+          (6200, 320, 250),                                                        # 64 x 128 on two groups
+          (3137, 192, 193),                                                        # 64 x 64 on two groups
+          (6210, 3100, 130), (3100, 64, 200), (40, 64, 33), (700, 1088, 40), (1030, 4096, 7)]  # 32 x 64 on two groups
+SAME_BITS, SAME_BITS_K = (5632, 1430, 20, 43, 100, 150, 250, 270, 330, 500, 710, 970, 1031), (130, 300, 500)
 
 
 @pytest.mark.parametrize("n,k,m", SHAPES)
@@ -37,18 +41,17 @@ def test_tiles(hip, f32, n, k, m):
     assert (np.linalg.norm(got - x.astype(np.float64) @ wf.T, axis=1) / size).max() <= 1e-6
 
 
-@pytest.mark.parametrize("k", [130, 300, 500])
+@pytest.mark.parametrize("k", SAME_BITS_K)
 def test_bfloat16_rows_are_the_same_bits_in_every_form(hip, k):
-    """A row's sums run over K in one order, however many rows go with it: 128 x 128 at 500 rows, then 32 x 64, 64 x 64 and
-    64 x 128."""
-    n, rows = 5632, 500
+    """A row's sums run over K in one order, however many rows go with it: from 192 x 128 at 1430 rows to 32 x 32 at 20."""
+    n, rows, *fewer = SAME_BITS
     rng = np.random.default_rng(k)
     w, x = (padded_bits(rng.normal(0, 1, (r, k)).astype(np.float32)) for r in (n, rows))
     wt = bf16_tensor(hip, w)
     want = hip.linear_bf16(wt, n, k, bf16_tensor(hip, x), rows).numpy()
     exact = from_bfloat16(x)[:9].astype(np.float64) @ from_bfloat16(w).astype(np.float64).T
     assert np.linalg.norm(want[:9] - exact) <= 1e-6 * np.linalg.norm(exact)
-    for m in (20, 100, 150, 250):
+    for m in fewer:
         assert np.array_equal(hip.linear_bf16(wt, n, k, bf16_tensor(hip, x[:m]), m).numpy(), want[:m]), m
 
 
