@@ -8,7 +8,6 @@
 #include "dense.hpp"
 
 #include <algorithm>
-#include <iterator>
 #include <type_traits>
 
 namespace litenn_hip
@@ -767,7 +766,7 @@ namespace litenn_hip
 			constexpr int kRowBytes = 2 * kTileK, kStage = (BM + BN) * kRowBytes; // [BM activations, BN weights][64]
 			constexpr int LA = BM / 8 / W, LW = BN / 8 / W, L = LA + LW;         // 1 KB pieces a wavefront moves per tile
 			static_assert(LA * 8 * W == BM && LW * 8 * W == BN && TM * WM * 16 == BM && TN * WN * 16 == BN, "tile");
-			static_assert((S - 1) * L < 64, "loads that a wait can count");
+			static_assert((S - 1) * L < 64 && S <= fetch::kDenseMaxBuffers, "loads that a wait can count");
 			extern __shared__ __attribute__((aligned(16))) uint8_t ring_lds[];
 			const DenseRows& d = args.d;
 			int tm, tn;

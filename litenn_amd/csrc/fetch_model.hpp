@@ -43,6 +43,9 @@ namespace litenn_hip
 			return { first, steps, groups == 1 ? steps : (all + parts - 1) / parts, all };
 		}
 
+		// buffers of a ring at most: a kernel asks for tiles that many rounds past the one it multiplies
+		constexpr int kDenseMaxBuffers = 8;
+
 		// The ranges of K a sublayer's last product of m rows is walked in at once, each with sums of its own
 		// [m, ld] behind the one before: where there are few tiles, enough for about two workgroups per CU and
 		// none shorter than 16 tiles of K.

@@ -631,7 +631,7 @@ static void test_gemm_chunk_ranges()
 
 // Products over bfloat16 weights: whatever the ranges of K and the groups of wavefronts, every tile of K is
 // multiplied once, the groups of a workgroup make equally many rounds, and only tiles that are there are requested
-// (up to six rounds past the last).
+// (up to a ring's buffers past the last round).
 static void test_dense_walks()
 {
 	using namespace litenn_hip::fetch;
@@ -649,7 +649,7 @@ static void test_dense_walks()
 					{
 						const DenseWalk w = dense_walk(all, ranges, groups, range, group);
 						CHECK(w.rounds == dense_walk(all, ranges, groups, range, 0).rounds, "%d tiles, %d ranges of %d groups", all, ranges, groups);
-						for (int round = 0; round < w.rounds + 6; ++round)
+						for (int round = 0; round < w.rounds + kDenseMaxBuffers; ++round)
 						{
 							const int tile = w.tile(round);
 							CHECK(tile >= 0 && tile < all, "%d tiles, %d ranges of %d groups: tile %d", all, ranges, groups, tile);
