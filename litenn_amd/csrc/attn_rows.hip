@@ -19,8 +19,8 @@
 // A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
 // a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
 // where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
-// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 34 us, where
-// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 93 us.  (40 and 108 with
+// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 34 us (37 on inputs not in the caches), where
+// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 92 us.  (41 and 109 with
 // a branch for each score's options, every tile masked and the cap's tangent always in the layer's form.)  Sums are
 // short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
 // addition per tile, which costs 4 us and leaves the error against 64 bits below the row kernel's (mean of six inputs, 1e-7:
@@ -422,8 +422,8 @@ namespace litenn_hip
 				if (a.softcap != 0.0f)
 				{
 					// Capped scores are a small part of the cap as a rule: the series takes seven instructions, the layer's form 35 more
-					// where a lane of the wavefront has a score that wants it (the call above with caps of 30 and 4: 34.2 and 38.9 us,
-					// with Float32 keys and a cap of 0.5 108; error against 64 bits 1.3e-7 where the layer's form alone has 3.7e-7).
+					// where a lane of the wavefront has a score that wants it (the call above with caps of 30 and 4: 34 and 39 us,
+					// with Float32 keys and a cap of 0.5 107; error against 64 bits 1.3e-7 where the layer's form alone has 3.7e-7).
 					float most = 0.0f;
 #pragma unroll
 					for (int e = 0; e < 16; ++e)

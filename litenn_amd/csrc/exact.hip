@@ -1664,9 +1664,10 @@ namespace litenn_hip
 			kernel<<<dim3(static_cast<unsigned>((m_pad + 63) / 64 * 64)), dim3(threads), 0, stream>>>(
 			    x, static_cast<uint8_t*>(scratch), static_cast<int>(m), m_pad, static_cast<int>(k), chunks, norm_w, eps, up);
 		};
-		// Few rows leave a workgroup a CU to itself: more threads, fewer elements in a chain (us, 256 / 512 / 1024 threads: 64
-		// rows of 14336 9.9, 7.8, 7.4; 20 rows of 4096 5.5, 4.4, 4.0); many rows share a CU (300 rows of 14336 with SwiGLU 18.4,
-		// 17.8, 18.1, of 4096 8.5, 7.9, 8.4).
+		// Few rows leave a workgroup a CU to itself: more threads, fewer elements in a chain, and it pays at every width (us, 256 /
+		// 512 / 1024 threads: 64 rows of 14336 10.8, 8.7, 8.3, of 4096 5.9, 5.0, 4.8, of 2048 5.0, 4.3, 4.0, of 1024 4.9, 4.1, 3.9; 9 of
+		// 1024 4.2, 3.6, 3.5; 128 of 1024 5.1, 4.3, 4.1); beyond 256 rows they share a CU (300 rows of 14336 14.2, 13.0, 14.0, of 4096
+		// 9.3, 9.2, 9.4, of 1024 6.6, 6.0, 6.7).  From 129 to 256 the two are 0.1 to 0.4 apart.
 		if (m <= 128)
 		{
 			launch(&split_rows_kernel<1024>, 1024);
