@@ -48,7 +48,7 @@ SINGLE = {
     "gla_odd": ku.config([ku.linear_attention(heads=5, dim=7, vdim=11, tau=3.0)], vocab=67, width=50),
     "gla_ones": ku.config([ku.linear_attention(heads=1, dim=1, vdim=1, tau=1.0)], vocab=5, width=6),
     "odd_width": ku.config([ku.attention(), ku.linear_attention()], width=53),
-    # head sizes of every tile form
+    # head sizes of every form of the window's tiles, and beyond
     "attention_wide": ku.config([ku.attention(heads=2, dim=136, vdim=200, kv_rank=300, q_rank=520, window=70, scale=0.1)]),
     "attention_mid": ku.config([ku.attention(heads=2, dim=96, vdim=72, kv_rank=64, q_rank=64, window=64, scale=0.1)]),
     "attention_unequal": ku.config([ku.attention(heads=2, dim=32, vdim=256, kv_rank=128, q_rank=128, window=33)]),

@@ -40,8 +40,8 @@ NAN16, NAN32 = 0x7FC0, np.float32(np.nan)
 @pytest.mark.parametrize("n,k", [(1, 1), (7, 5), (130, 64), (65, 100), (300, 320), (96, 4096), (2049, 513), (4100, 96), (33, 8192)])
 @pytest.mark.parametrize("m", [1, 2, 5, 31, 33, 64, 129, 200])
 def test_linear_bf16(hip, n, k, m):
-    """Every tile form, ragged in all three extents; what lies behind a row's last activation is never used
-    (it is NaN here)."""
+    """Small tiles, ragged in all three extents (EVERY_FORM has the others); what lies behind a row's last activation is never
+    used (it is NaN here)."""
     rng = np.random.default_rng([n, k, m])
     w = padded_bits(rng.normal(0, 1, (n, k)).astype(np.float32))
     x = rng.normal(0, 1, (m, k)).astype(np.float32)
