@@ -16,15 +16,17 @@
 //     below 2^-26 of the pair's, a quarter of what a Float32 rounding takes, are left out.
 // Scores, softmax and sums are Float32 as in the row kernels.
 //
-// A tile is one chain in its wavefront (16 products, softmax, 16 products), so what counts is that two wavefronts fit
-// a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
-// where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with
-// no barrier.  200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 34 us (37 on inputs not in the caches), where
-// the row kernel took 1365; Float32 keys and values (three times the products, one wavefront a SIMD) 92 us.  (41 and 109 with
-// a branch for each score's options, every tile masked and the cap's tangent always in the layer's form.)  Sums are
-// short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
+// A tile is one chain in its wavefront (16 products, softmax, 16 products) that the vector ALUs bound: 600 instructions at four
+// cycles beside 1024 cycles of products.  So what counts is how few there are (a whole tile's rows lie at one distance from a
+// uniform address, weights take an exponential for arguments of one sign, places in LDS are a register and a constant), that two
+// wavefronts fit a SIMD (256 registers: one of keys and values is in flight at a time, the second halves of the queries are in LDS
+// where all wavefronts have the same), that no load hangs on a branch, and that every wavefront has its own keys, with no barrier.
+// 200 rows on 1000 keys (32 heads of 128 over 8) with mask, slopes, soft cap and sinks take 27.6 us (38.5 with 1000 instructions a
+// tile, 31 registers spilled and the groups merged by one of them), where the row kernel took 1365; causal, with Float32 keys and
+// values (three times the products, one wavefront a SIMD), 57 (85 in pairs of wavefronts that share their keys, on half the SIMDs).
+// Sums are short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
 // addition per tile, which costs 4 us and leaves the error against 64 bits below the row kernel's (mean of six inputs, 1e-7:
-// these rows, whose small capped scores the row kernel's tangent rounds, 1.34 and 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
+// these rows, whose small capped scores the row kernel's tangent rounds, 1.30 and 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
 #include "common.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
@@ -108,15 +110,30 @@ namespace litenn_hip
 			return fmaf(x, x2 * p, x);
 		}
 
-		// Rows of keys and values lie 2 D bytes apart in LDS, their 16-byte pieces permuted by the row so that the 64 banks
-		// are covered evenly: keys are read as a piece of each of 16 rows, values as 64 bytes of each of four.
-		template <int D>
-		__device__ __forceinline__ int key_slot(int row, int piece) { return piece ^ (D == 128 ? row & 15 : (row >> 1) & 7); }
-		template <int D>
-		__device__ __forceinline__ int value_slot(int row, int piece)
+		// exp(x) for x at most 0, or NaN: the product's rounding is put back behind the power of two, which below 2^-126 is 0.
+		// Seven instructions where expf, which reduces its range and looks for its ends, takes thirteen.
+		__device__ __forceinline__ float exp_of_nonpositive(float x)
 		{
-			return piece ^ (D == 128 ? (row & 3) << 2 | ((row >> 2) & 3) : (row & 2) << 1);
+			constexpr float kLog2e = 1.44269504088896341f, kLog2eRest = 1.925963033e-8f, kLn2 = 0.69314718055994531f;
+			x = __builtin_elementwise_maximum(x, -256.0f); // (an infinity would leave no number; a NaN stays one)
+			const float high = x * kLog2e;
+			const float low = fmaf(x, kLog2eRest, fmaf(x, kLog2e, -high));
+			const float p = __builtin_amdgcn_exp2f(high);
+			return fmaf(p * low, kLn2, p);
 		}
+
+		// Rows of keys lie 16 bytes further apart in LDS than they are long, rows of values 64, which spreads a piece of each of 16
+		// keys, and 64 bytes of each of four values, over all 64 banks.  (Pieces permuted by their row want a register for each
+		// place that is read: 31 of them spilled.)
+		template <int D>
+		constexpr int key_stride() { return 2 * D + 16; }
+		template <int D>
+		constexpr int value_stride() { return 2 * D + 64; }
+		// A wavefront that shares its Float32 tiles with nobody puts the values where the keys were: four of them fit a CU's LDS
+		template <typename O, int QW>
+		constexpr bool one_buffer() { return O::kStored > 1 && QW == 1; }
+		template <typename O, int D, int QW>
+		constexpr int group_bytes() { return O::kStored * kKeys * (one_buffer<O, QW>() ? value_stride<D>() : key_stride<D>() + value_stride<D>()); }
 
 		// A workgroup takes 32 QW query rows of one head; its KW groups of QW wavefronts take the key tiles in turn,
 		// each group with its own buffers, and merge at the end.
@@ -125,8 +142,10 @@ namespace litenn_hip
 		{
 			typedef typename O::frag frag;
 			typedef typename O::stored stored;
-			constexpr int RS = 2 * D, kTileBytes = kKeys * RS; // of one part of the keys or the values
-			constexpr int kGroupBytes = 2 * O::kStored * kTileBytes;
+			constexpr int kKeyStride = key_stride<D>(), kValueStride = value_stride<D>();
+			constexpr int kKeyBytes = kKeys * kKeyStride, kValueBytes = kKeys * kValueStride; // of one part of a tile
+			constexpr bool kOneBuffer = one_buffer<O, QW>();
+			constexpr int kGroupBytes = group_bytes<O, D, QW>();
 			// The second half of the queries waits in LDS where every wavefront has the same ones and registers are short
 			constexpr bool kQueriesInLds = O::kSplit == 2 && QW == 1 && D == 128;
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KW][keys, values], queries; later the groups' results
@@ -162,40 +181,172 @@ namespace litenn_hip
 			// ---- the wavefront's queries: B operand of the first product, times 2^shift
 			frag q[D / 16][O::kSplit];
 			float unscale = 1.0f;
+			floatx4 raw[D / 8]; // asked for ahead of the first tile's keys and values
 			{
 				// (whole groups of eight; one behind the head's last loads the first again and is dropped: the loads must not
 				// hang on branches, or each waits for the one before)
 				const float* src = a.q + static_cast<size_t>(row_c) * a.ldq + static_cast<size_t>(head) * a.dim;
-				float v[D / 16][8];
-				float mx = 0.0f;
 #pragma unroll
 				for (int s = 0; s < D / 16; ++s)
 				{
 					const int d = 16 * s + 8 * h;
 					const floatx4_a4* at = reinterpret_cast<const floatx4_a4*>(src + (d < a.dim ? d : 0));
-					const floatx4 x = at[0], y = at[1];
+					raw[2 * s] = at[0], raw[2 * s + 1] = at[1];
+				}
+			}
+			// ---- staging: a thread moves 8-element pieces of rows
+			uint8_t* const k_lds = lds + group * kGroupBytes;
+			uint8_t* const v_lds = kOneBuffer ? k_lds : k_lds + O::kStored * kKeyBytes;
+			constexpr int kRowPieces = D / 8, kPieces = kKeys * kRowPieces / (64 * QW), kRowStep = 64 * QW / kRowPieces;
+			static_assert(kPieces * 64 * QW == kKeys * kRowPieces && kRowStep * kRowPieces == 64 * QW, "pieces per thread");
+			constexpr int kWords = sizeof(stored) / 2; // 16-byte words of a piece
+			const int piece_row = tid / kRowPieces, piece = tid % kRowPieces; // first row, and the same column in all of them
+			u32x4 kr[kPieces][kWords], vr[kPieces][kWords];
+			const uint32_t ldk = static_cast<uint32_t>(a.ldk), ldv = static_cast<uint32_t>(a.ldv);
+			// (a piece behind the head's last loads the first again and goes nowhere)
+			const uint32_t k_off = static_cast<uint32_t>(piece_row) * ldk + (8 * piece < a.dim ? 8 * piece : 0);
+			const uint32_t v_off = static_cast<uint32_t>(piece_row) * ldv + (8 * piece < a.vdim ? 8 * piece : 0);
+			const auto request = [&](u32x4 (&into)[kPieces][kWords], const stored* from, uint32_t ld, uint32_t off, int tile) __attribute__((always_inline)) {
+				// A whole tile that does not wrap lies at one distance from a uniform address; others go row by row
+				const int key = first + tile * kKeys;
+				const int at0 = buffer_row(key);
+				if (key + kKeys <= last && (a.ring <= 0 || at0 + kKeys <= a.ring) && ld <= (1u << 26)) // (offsets of 32 bits)
+				{
+					const stored* const rows = from + static_cast<uint64_t>(static_cast<uint32_t>(at0)) * ld;
+#pragma unroll
+					for (int i = 0; i < kPieces; ++i)
+					{
+#pragma unroll
+						for (int w = 0; w < kWords; ++w)
+						{
+							into[i][w] = *reinterpret_cast<const u32x4*>(rows + static_cast<uint64_t>(kRowStep * i) * ld + 4 * w + off);
+						}
+					}
+					return;
+				}
+#pragma unroll
+				for (int i = 0; i < kPieces; ++i)
+				{
+					const uint32_t at = buffer_row(min(key + piece_row + kRowStep * i, last - 1));
+#pragma unroll
+					for (int w = 0; w < kWords; ++w)
+					{
+						into[i][w] = *reinterpret_cast<const u32x4*>(from + static_cast<uint64_t>(at) * ld + 4 * w + (off - static_cast<uint32_t>(piece_row) * ld));
+					}
+				}
+			};
+			const auto store_piece = [&](uint8_t* dst, int part_bytes, const u32x4 (&v)[kWords]) __attribute__((always_inline)) {
+				if constexpr (O::kStored == 1)
+				{
+					*reinterpret_cast<u32x4*>(dst) = v[0];
+				}
+				else
+				{
+					frag f[O::kStored];
 #pragma unroll
 					for (int e = 0; e < 8; ++e)
 					{
-						v[s][e] = e < 4 ? x[e & 3] : y[e & 3];
+						O::split(__uint_as_float(v[e / 4][e % 4]), e, f);
+					}
+#pragma unroll
+					for (int p = 0; p < O::kStored; ++p)
+					{
+						*reinterpret_cast<frag*>(dst + p * part_bytes) = f[p];
 					}
 				}
-#pragma unroll
-				for (int s = 0; s < D / 16; ++s)
+			};
+			const auto deposit = [&](u32x4 (&pieces)[kPieces][kWords], uint8_t* to, int stride, int part_bytes, int dim) __attribute__((always_inline)) {
+				const bool there = 8 * piece < dim;
+				if (kOneBuffer && !there) // (the buffer holds both in turn, and not in the same places)
 				{
 #pragma unroll
-					for (int e = 0; e < 8; ++e)
+					for (int i = 0; i < kPieces; ++i)
 					{
-						v[s][e] = 16 * s + 8 * h < a.dim ? v[s][e] : 0.0f;
-						const float m = fabsf(v[s][e]);
-						mx = m <= 3.402823466e38f ? fmaxf(mx, m) : mx;
+#pragma unroll
+						for (int w = 0; w < kWords; ++w)
+						{
+							pieces[i][w] = u32x4{ 0u, 0u, 0u, 0u };
+						}
 					}
 				}
-				int shift = 0;
+				if (kOneBuffer || there)
+				{
+#pragma unroll
+					for (int i = 0; i < kPieces; ++i)
+					{
+						store_piece(to + (piece_row + kRowStep * i) * stride + 16 * piece, part_bytes, pieces[i]);
+					}
+				}
+			};
+			const auto deposit_keys = [&]() { deposit(kr, k_lds, kKeyStride, kKeyBytes, a.dim); };
+			const auto deposit_values = [&]() { deposit(vr, v_lds, kValueStride, kValueBytes, a.vdim); };
+			if (!kOneBuffer && (a.dim < D || a.vdim < D)) // (uniform) pieces behind the head's last stay zero
+			{
+				for (int at = tid * 16; at < kGroupBytes; at += 64 * QW * 16)
+				{
+					*reinterpret_cast<u32x4*>(k_lds + at) = u32x4{ 0u, 0u, 0u, 0u };
+				}
+				if constexpr (QW > 1)
+				{
+					__syncthreads();
+				}
+			}
+			const auto meet = [&]() {
+				if constexpr (QW > 1)
+				{
+					__syncthreads();
+				}
+				else
+				{
+					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
+					__builtin_amdgcn_wave_barrier();
+				}
+			};
+
+			// Keys travel while the previous tile's values are used and go into LDS once its scores are formed, values the
+			// other way round: one of the two is in registers at a time.
+			const auto tile_at = [&](int step) { return min(step * KW + group, tiles - 1); };
+			if (steps > 0)
+			{
+				request(kr, kb, ldk, k_off, tile_at(0));
+				request(vr, vb, ldv, v_off, tile_at(0));
+			}
+			__builtin_amdgcn_sched_barrier(0); // (the first tile travels while the queries are taken apart)
+			{
+				if (a.dim < D) // (uniform)
+				{
+#pragma unroll
+					for (int s = 0; s < D / 8; ++s)
+					{
+						raw[s] = 16 * (s >> 1) + 8 * h < a.dim ? raw[s] : floatx4{};
+					}
+				}
+				float scale = 1.0f;
 				if constexpr (O::kSplit == 2)
 				{
+					float mx = 0.0f;
+#pragma unroll
+					for (int s = 0; s < D / 8; ++s)
+					{
+						mx = fmaxf(mx, fmaxf(fmaxf(fabsf(raw[s].x), fabsf(raw[s].y)), fmaxf(fabsf(raw[s].z), fabsf(raw[s].w))));
+					}
+					if (__any(mx > 3.402823466e38f)) // (of the finite ones, then)
+					{
+						mx = 0.0f;
+#pragma unroll
+						for (int s = 0; s < D / 8; ++s)
+						{
+#pragma unroll
+							for (int e = 0; e < 4; ++e)
+							{
+								const float m = fabsf(raw[s][e]);
+								mx = m <= 3.402823466e38f ? fmaxf(mx, m) : mx;
+							}
+						}
+					}
 					mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-					shift = mx > 0.0f ? min(14 - ilogbf(mx), 126) : 0;
+					const int shift = mx > 0.0f ? min(14 - ilogbf(mx), 126) : 0;
+					scale = ldexpf(1.0f, shift);
 					unscale = ldexpf(1.0f, -shift);
 				}
 #pragma unroll
@@ -204,7 +355,7 @@ namespace litenn_hip
 #pragma unroll
 					for (int e = 0; e < 8; ++e)
 					{
-						O::split(ldexpf(v[s][e], shift), e, q[s]);
+						O::split(raw[2 * s + e / 4][e & 3] * scale, e, q[s]);
 					}
 				}
 			}
@@ -222,6 +373,7 @@ namespace litenn_hip
 				__syncthreads();
 			}
 			const float slope = a.mask && a.max_bias > 0.0 ? static_cast<float>(row_alibi_slope(head, a.heads, a.max_bias)) : 1.0f;
+			const float factor = a.apply_scale ? unscale * a.scale : unscale; // (a power of two and the scale: one rounding for both)
 			const float* const mask_row = a.mask ? a.mask + static_cast<size_t>(row_c) * keys : nullptr;
 
 			// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range.  (A
@@ -254,84 +406,6 @@ namespace litenn_hip
 				return v;
 			};
 
-			// ---- staging: a thread moves 8-element pieces of rows
-			uint8_t* const k_lds = lds + group * kGroupBytes;
-			uint8_t* const v_lds = k_lds + O::kStored * kTileBytes;
-			constexpr int kRowPieces = D / 8, kPieces = kKeys * kRowPieces / (64 * QW), kRowStep = 64 * QW / kRowPieces;
-			static_assert(kPieces * 64 * QW == kKeys * kRowPieces && kRowStep * kRowPieces == 64 * QW, "pieces per thread");
-			constexpr int kWords = sizeof(stored) / 2; // 16-byte words of a piece
-			const int piece_row = tid / kRowPieces, piece = tid % kRowPieces; // first row, and the same column in all of them
-			u32x4 kr[kPieces][kWords], vr[kPieces][kWords];
-			const uint32_t ldk = static_cast<uint32_t>(a.ldk), ldv = static_cast<uint32_t>(a.ldv);
-			// (a piece behind the head's last loads the first again and is zeroed on its way into LDS)
-			const stored* const k_piece = kb + (8 * piece < a.dim ? 8 * piece : 0);
-			const stored* const v_piece = vb + (8 * piece < a.vdim ? 8 * piece : 0);
-			const auto request = [&](u32x4 (&into)[kPieces][kWords], const stored* from, uint32_t ld, int tile) {
-#pragma unroll
-				for (int i = 0; i < kPieces; ++i)
-				{
-					const uint32_t at = buffer_row(min(first + tile * kKeys + piece_row + kRowStep * i, last - 1));
-#pragma unroll
-					for (int w = 0; w < kWords; ++w)
-					{
-						into[i][w] = *reinterpret_cast<const u32x4*>(from + static_cast<uint64_t>(at) * ld + 4 * w);
-					}
-				}
-			};
-			const auto store_piece = [&](uint8_t* dst, const u32x4 (&w)[kWords], bool there) {
-				u32x4 v[kWords];
-#pragma unroll
-				for (int i = 0; i < kWords; ++i)
-				{
-					v[i] = there ? w[i] : u32x4{ 0u, 0u, 0u, 0u };
-				}
-				if constexpr (O::kStored == 1)
-				{
-					*reinterpret_cast<u32x4*>(dst) = v[0];
-				}
-				else
-				{
-					frag f[O::kStored];
-#pragma unroll
-					for (int e = 0; e < 8; ++e)
-					{
-						O::split(__uint_as_float(v[e / 4][e % 4]), e, f);
-					}
-#pragma unroll
-					for (int p = 0; p < O::kStored; ++p)
-					{
-						*reinterpret_cast<frag*>(dst + p * kTileBytes) = f[p];
-					}
-				}
-			};
-			const auto deposit_keys = [&]() {
-#pragma unroll
-				for (int i = 0; i < kPieces; ++i)
-				{
-					const int key = piece_row + kRowStep * i;
-					store_piece(k_lds + key * RS + 16 * key_slot<D>(key, piece), kr[i], 8 * piece < a.dim);
-				}
-			};
-			const auto deposit_values = [&]() {
-#pragma unroll
-				for (int i = 0; i < kPieces; ++i)
-				{
-					const int key = piece_row + kRowStep * i;
-					store_piece(v_lds + key * RS + 16 * value_slot<D>(key, piece), vr[i], 8 * piece < a.vdim);
-				}
-			};
-			const auto meet = [&]() {
-				if constexpr (QW > 1)
-				{
-					__syncthreads();
-				}
-				else
-				{
-					__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
-					__builtin_amdgcn_wave_barrier();
-				}
-			};
-
 			floatx16 o[D / 32];
 #pragma unroll
 			for (int b = 0; b < D / 32; ++b)
@@ -339,14 +413,9 @@ namespace litenn_hip
 				o[b] = floatx16{};
 			}
 			float run_m = -INFINITY, run_l = 0.0f; // run_l: of this lane's keys
-			// Keys travel while the previous tile's values are used and go into LDS once its scores are formed, values the
-			// other way round: one of the two is in registers at a time.
-			const auto tile_at = [&](int step) { return min(step * KW + group, tiles - 1); };
 			if (steps > 0)
 			{
-				request(kr, k_piece, ldk, tile_at(0));
 				deposit_keys();
-				request(vr, v_piece, ldv, tile_at(0));
 			}
 			for (int step = 0; step < steps; ++step)
 			{
@@ -388,7 +457,7 @@ namespace litenn_hip
 #pragma unroll
 					for (int p = 0; p < O::kProducts; ++p)
 					{
-						const frag kf = *reinterpret_cast<const frag*>(k_lds + O::stored_of[p] * kTileBytes + j * RS + 16 * key_slot<D>(j, 2 * st + h));
+						const frag kf = *reinterpret_cast<const frag*>(k_lds + O::stored_of[p] * kKeyBytes + j * kKeyStride + 16 * (2 * st + h));
 						floatx16& to = p > 0 ? s_low : st % 2 == 0 ? s : s_odd;
 						if constexpr (kQueriesInLds)
 						{
@@ -401,24 +470,16 @@ namespace litenn_hip
 					}
 				}
 				deposit_values();
-				request(kr, k_piece, ldk, tile_at(step + 1));
+				request(kr, kb, ldk, k_off, tile_at(step + 1));
 				// lane (j, h) holds keys base + 8 (e / 4) + 4 h + e % 4 of query j
 				float sc[16];
 				float top = -INFINITY;
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
 				{
-					sc[e] = fmaf(s_low[e], O::kLowScale, s[e] + s_odd[e]) * unscale;
+					sc[e] = fmaf(s_low[e], O::kLowScale, s[e] + s_odd[e]) * factor;
 				}
 				// (an option at a time over all sixteen: a branch for each score's options was a tenth of the tile)
-				if (a.apply_scale)
-				{
-#pragma unroll
-					for (int e = 0; e < 16; ++e)
-					{
-						sc[e] = __fmul_rn(sc[e], a.scale);
-					}
-				}
 				if (a.softcap != 0.0f)
 				{
 					// Capped scores are a small part of the cap as a rule: the series takes seven instructions, the layer's form 35 more
@@ -467,7 +528,7 @@ namespace litenn_hip
 #pragma unroll
 					for (int e = 0; e < 16; ++e)
 					{
-						sc[e] = __fadd_rn(sc[e], __fmul_rn(mask[e], slope)); // (a slope of 1 leaves the mask as it is)
+						sc[e] = fmaf(mask[e], slope, sc[e]);
 					}
 				}
 				if (!live || base < wave_lo || base + kKeys > wave_hi) // (a key that one of the wavefront's queries does not see)
@@ -494,7 +555,7 @@ namespace litenn_hip
 #pragma unroll
 				for (int e = 0; e < 16; ++e)
 				{
-					const float p = expf(sc[e] - ref_m);
+					const float p = exp_of_nonpositive(sc[e] - ref_m);
 					sums[e] = p;
 					O::split(p * O::kWeightScale, e & 7, w[e >> 3]);
 				}
@@ -511,8 +572,11 @@ namespace litenn_hip
 				// step u: keys 16 u + 4 h + 0..3 and 16 u + 8 + 4 h + 0..3.  Sixteen lanes read four keys' rows of
 				// sixteen dimensions, eight bytes each, and get the four keys of one dimension
 				meet(); // the tile's values are there, its keys have been used
-				deposit_keys();
-				request(vr, v_piece, ldv, tile_at(step + 1));
+				if constexpr (!kOneBuffer)
+				{
+					deposit_keys();
+				}
+				request(vr, vb, ldv, v_off, tile_at(step + 1));
 				const int v_row = 4 * h + ((lane & 15) >> 2), v_col = ((lane >> 4) & 1) * 2 + ((lane & 3) >> 1), v_byte = (lane & 1) * 8;
 #pragma unroll
 				for (int b = 0; b < D / 32; ++b)
@@ -531,10 +595,9 @@ namespace litenn_hip
 						for (int p = 0; p < O::kStored; ++p)
 						{
 							typedef __attribute__((address_space(3))) short4v* lds_short4;
-							const int r0 = 16 * u + v_row, r1 = r0 + 8;
-							const uint8_t* const at = v_lds + p * kTileBytes + v_byte;
-							const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + r0 * RS + 16 * value_slot<D>(r0, 4 * b + v_col))));
-							const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + r1 * RS + 16 * value_slot<D>(r1, 4 * b + v_col))));
+							const uint8_t* const at = v_lds + p * kValueBytes + v_row * kValueStride + 16 * v_col + v_byte;
+							const u32x2 x = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + 16 * u * kValueStride + 64 * b)));
+							const u32x2 y = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4)(at + (16 * u + 8) * kValueStride + 64 * b)));
 							vf[u][p] = __builtin_bit_cast(frag, u32x4{ x.x, x.y, y.x, y.y });
 						}
 #pragma unroll
@@ -562,58 +625,70 @@ namespace litenn_hip
 						o[b][e] = fmaf(o[b][e], corr, t[e]);
 					}
 				}
+				if constexpr (kOneBuffer)
+				{
+					meet();
+					deposit_keys();
+				}
 			}
 			run_l += __shfl_xor(run_l, 32, 64);
 
-			if constexpr (KW > 1)
+			// The groups hand (maximum, sum, outputs) over through LDS, and each takes a share of the dimensions: quads of them, as
+			// they lie in o, group by group.  (One group that took all of them in turn: 1.2 us more of 39 with eight groups.)
+			constexpr int kQuads = D / 8 / KW; // of this wavefront
+			static_assert(kQuads * KW * 8 == D, "quads and groups");
+			float r[kQuads][4];
 			{
-				// groups 1 .. KW - 1 hand (maximum, sum, outputs) to group 0, which takes them in order
 				float* const xch = reinterpret_cast<float*>(lds);
 				constexpr int kWaveFloats = (D / 2 + 2) * 64; // of one wavefront: outputs, maximum, sum
 				__syncthreads();
-				if (group > 0)
+				float* const dst = xch + (group * QW + qw) * kWaveFloats;
+#pragma unroll
+				for (int b = 0; b < D / 32; ++b)
 				{
-					float* dst = xch + ((group - 1) * QW + qw) * kWaveFloats;
 #pragma unroll
-					for (int b = 0; b < D / 32; ++b)
+					for (int e = 0; e < 16; e += 4)
 					{
-#pragma unroll
-						for (int e = 0; e < 16; e += 4)
-						{
-							*reinterpret_cast<float4*>(dst + ((b * 16 + e) / 4 * 64 + lane) * 4) = float4{ o[b][e], o[b][e + 1], o[b][e + 2], o[b][e + 3] };
-						}
+						*reinterpret_cast<float4*>(dst + ((b * 16 + e) / 4 * 64 + lane) * 4) = float4{ o[b][e], o[b][e + 1], o[b][e + 2], o[b][e + 3] };
 					}
-					dst[D / 2 * 64 + lane] = run_m;
-					dst[(D / 2 + 1) * 64 + lane] = run_l;
 				}
+				dst[D / 2 * 64 + lane] = run_m;
+				dst[(D / 2 + 1) * 64 + lane] = run_l;
 				__syncthreads();
-				if (group > 0)
+				float m[KW], weight[KW];
+#pragma unroll
+				for (int i = 0; i < KW; ++i)
 				{
-					return;
+					m[i] = xch[(i * QW + qw) * kWaveFloats + D / 2 * 64 + lane];
+					run_m = i == 0 ? m[0] : fmaxf(run_m, m[i]);
 				}
-				for (int other = 0; other < KW - 1; ++other)
+				const float ref_m = run_m == -INFINITY ? 0.0f : run_m;
+#pragma unroll
+				for (int i = 0; i < KW; ++i)
 				{
-					const float* src = xch + (other * QW + qw) * kWaveFloats;
-					const float other_m = src[D / 2 * 64 + lane], other_l = src[(D / 2 + 1) * 64 + lane];
-					const float all_m = fmaxf(run_m, other_m), ref_m = all_m == -INFINITY ? 0.0f : all_m;
-					const float w0 = expf(run_m - ref_m), w1 = expf(other_m - ref_m);
-					run_m = all_m;
-					run_l = run_l * w0 + other_l * w1;
+					weight[i] = expf(m[i] - ref_m);
+					const float l = xch[(i * QW + qw) * kWaveFloats + (D / 2 + 1) * 64 + lane] * weight[i];
+					run_l = i == 0 ? l : run_l + l;
+				}
 #pragma unroll
-					for (int b = 0; b < D / 32; ++b)
+				for (int i = 0; i < KW; ++i)
+				{
+#pragma unroll
+					for (int n = 0; n < kQuads; ++n)
 					{
-#pragma unroll
-						for (int e = 0; e < 16; e += 4)
-						{
-							const float4 t = *reinterpret_cast<const float4*>(src + ((b * 16 + e) / 4 * 64 + lane) * 4);
-							o[b][e] = o[b][e] * w0 + t.x * w1;
-							o[b][e + 1] = o[b][e + 1] * w0 + t.y * w1;
-							o[b][e + 2] = o[b][e + 2] * w0 + t.z * w1;
-							o[b][e + 3] = o[b][e + 3] * w0 + t.w * w1;
-						}
+						const float4 t = *reinterpret_cast<const float4*>(xch + (i * QW + qw) * kWaveFloats + ((group * kQuads + n) * 64 + lane) * 4);
+						r[n][0] = i == 0 ? t.x * weight[0] : fmaf(t.x, weight[i], r[n][0]);
+						r[n][1] = i == 0 ? t.y * weight[0] : fmaf(t.y, weight[i], r[n][1]);
+						r[n][2] = i == 0 ? t.z * weight[0] : fmaf(t.z, weight[i], r[n][2]);
+						r[n][3] = i == 0 ? t.w * weight[0] : fmaf(t.w, weight[i], r[n][3]);
 					}
 				}
 			}
+			// the first of the quad's dimensions
+			const auto dim_of = [&](int n) {
+				const int quad = group * kQuads + n;
+				return 32 * (quad >> 2) + 8 * (quad & 3) + 4 * h;
+			};
 			if (row >= a.rows)
 			{
 				return;
@@ -623,12 +698,12 @@ namespace litenn_hip
 			// so that it gets what Float32 arithmetic gives it.
 			bool finite = fabsf(run_l) <= 3.402823466e38f;
 #pragma unroll
-			for (int b = 0; b < D / 32; ++b)
+			for (int n = 0; n < kQuads; ++n)
 			{
 #pragma unroll
-				for (int e = 0; e < 16; ++e)
+				for (int i = 0; i < 4; ++i)
 				{
-					finite = finite && fabsf(o[b][e]) <= 3.402823466e38f;
+					finite = finite && fabsf(r[n][i]) <= 3.402823466e38f;
 				}
 			}
 			if (__builtin_expect(!finite, 0))
@@ -647,9 +722,13 @@ namespace litenn_hip
 				run_m = -INFINITY;
 				run_l = 0.0f;
 #pragma unroll
-				for (int b = 0; b < D / 32; ++b)
+				for (int n = 0; n < kQuads; ++n)
 				{
-					o[b] = floatx16{};
+#pragma unroll
+					for (int i = 0; i < 4; ++i)
+					{
+						r[n][i] = 0.0f;
+					}
 				}
 				for (int key = lo; key < hi; ++key)
 				{
@@ -666,13 +745,13 @@ namespace litenn_hip
 					run_m = new_m;
 					run_l = fmaf(run_l, corr, p);
 #pragma unroll
-					for (int b = 0; b < D / 32; ++b)
+					for (int n = 0; n < kQuads; ++n)
 					{
 #pragma unroll
-						for (int e = 0; e < 16; ++e)
+						for (int i = 0; i < 4; ++i)
 						{
-							const int d = 32 * b + 8 * (e / 4) + 4 * h + (e & 3);
-							o[b][e] = fmaf(p * O::kWeightScale, d < a.vdim ? widen(vr0[d]) : 0.0f, o[b][e] * corr);
+							const int d = dim_of(n) + i;
+							r[n][i] = fmaf(p * O::kWeightScale, d < a.vdim ? widen(vr0[d]) : 0.0f, r[n][i] * corr);
 						}
 					}
 				}
@@ -690,24 +769,20 @@ namespace litenn_hip
 			float* const out = a.out + static_cast<size_t>(row) * a.ldo + static_cast<size_t>(head) * a.vdim;
 			const float* const gate = a.gate ? a.gate + static_cast<size_t>(row) * a.ldg + static_cast<size_t>(head) * a.vdim : nullptr;
 #pragma unroll
-			for (int b = 0; b < D / 32; ++b)
+			for (int n = 0; n < kQuads; ++n)
 			{
-#pragma unroll
-				for (int e = 0; e < 16; e += 4)
+				const int d = dim_of(n);
+				if (d < a.vdim) // (whole groups of eight)
 				{
-					const int d = 32 * b + 2 * e + 4 * h;
-					if (d < a.vdim) // (whole groups of eight)
+					float4 v = { r[n][0] * inv, r[n][1] * inv, r[n][2] * inv, r[n][3] * inv };
+					if (gate)
 					{
-						float4 v = { o[b][e] * inv, o[b][e + 1] * inv, o[b][e + 2] * inv, o[b][e + 3] * inv };
-						if (gate)
-						{
-							v.x *= sigmoid_f32(gate[d]);
-							v.y *= sigmoid_f32(gate[d + 1]);
-							v.z *= sigmoid_f32(gate[d + 2]);
-							v.w *= sigmoid_f32(gate[d + 3]);
-						}
-						*reinterpret_cast<float4*>(out + d) = v;
+						v.x *= sigmoid_f32(gate[d]);
+						v.y *= sigmoid_f32(gate[d + 1]);
+						v.z *= sigmoid_f32(gate[d + 2]);
+						v.w *= sigmoid_f32(gate[d + 3]);
 					}
+					*reinterpret_cast<float4*>(out + d) = v;
 				}
 			}
 		}
@@ -715,8 +790,8 @@ namespace litenn_hip
 		template <typename O, int D, int QW, int KW>
 		void launch_form(const RowsAttn& a, hipStream_t s)
 		{
-			constexpr size_t tiles = static_cast<size_t>(KW) * O::kStored * kKeys * 4 * D + (O::kSplit == 2 && QW == 1 && D == 128 ? 64 * D : 0);
-			constexpr size_t merge = static_cast<size_t>(KW - 1) * QW * (D / 2 + 2) * 64 * sizeof(float);
+			constexpr size_t tiles = static_cast<size_t>(KW) * group_bytes<O, D, QW>() + (O::kSplit == 2 && QW == 1 && D == 128 ? 64 * D : 0);
+			constexpr size_t merge = static_cast<size_t>(KW) * QW * (D / 2 + 2) * 64 * sizeof(float);
 			constexpr size_t lds = tiles > merge ? tiles : merge;
 			static_assert(lds <= 160 * 1024, "LDS");
 			allow_dynamic_lds(reinterpret_cast<const void*>(&attn_rows_kernel<O, D, QW, KW>), lds);
@@ -726,17 +801,30 @@ namespace litenn_hip
 		template <int D>
 		void launch_dim(const RowsAttn& a, bool f32, hipStream_t s)
 		{
+			// us of both forms, 32 heads over 8 unless said, the rows on the keys behind
+			const size_t groups = static_cast<size_t>(a.heads) * ((a.rows + 31) / 32);
 			if (f32)
 			{
-				launch_form<FloatOperands, D, 2, 2>(a, s);
+				// Four wavefronts with keys of their own while their workgroups, one to a CU, fit the card at once, or twice over where
+				// half of them see half the keys and fewer (200 rows on 1000 keys 57 against 79 for two pairs that share their keys, 512
+				// on 512 of 16 heads 33 against 44, 700 on 700 of 16 44 and 57); pairs, which take their tiles apart once, from there on
+				// (300 on 1000 79 against 91, 1000 on 1000 93 and 133).
+				if (groups <= 256 || (groups <= 512 && a.keys == a.rows))
+				{
+					launch_form<FloatOperands, D, 1, 4>(a, s);
+				}
+				else
+				{
+					launch_form<FloatOperands, D, 2, 2>(a, s);
+				}
 			}
 			else
 			{
-				// Eight wavefronts on a head's rows, one workgroup to a CU, while all of them fit the 256 CUs at once and each wavefront
-				// has two tiles; else four, two workgroups to a CU (kernel's us for eight and four, every option: 200 rows on 1000
-				// keys 45 and 55, 16 on 4000 112 and 170, 128 on 128 24 and 17, 512 on 1024 84 and 68, 1500 on 4000 667 and 591).
-				const size_t groups = static_cast<size_t>(a.heads) * ((a.rows + 31) / 32);
-				if (groups <= 256 && a.keys >= 512)
+				// Eight wavefronts on a head's rows, one workgroup to a CU, while all of them fit the 256 CUs at once and have more than
+				// a tile or two each; four, two workgroups to a CU, for few keys and, heads of 128 on long runs of keys aside, for
+				// many rows (eight and four: 200 on 1000 24 and 27, 16 on 2000 32 and 44, 128 on 400 17.4 and 18.2, on 300 17.4 and
+				// 15.9, on 128 14.1 and 10.7, 512 on 512 30 and 27, 1000 on 2000 121 and 141; heads of 64, 300 on 1000 27 and 20).
+				if (groups <= 256 ? a.keys >= 384 : D == 128 && a.keys >= 1000)
 				{
 					launch_form<HalfOperands, D, 1, 8>(a, s);
 				}
@@ -752,7 +840,7 @@ namespace litenn_hip
 	bool launch_attn_rows_causal(const float* q, const void* kcache, const void* vcache, int cache_dtype, size_t m,
 	                             size_t past, size_t n_head, size_t n_kv_head, size_t head_dim, float* out, hipStream_t s)
 	{
-		if (!attn_rows_pays(m, past + m, cache_dtype == LITENN_F32) || m > 0x3fffffffu || n_head > 65535 || past + m > 0x3fffffffu)
+		if (!attn_rows_pay_causal(m, past + m, cache_dtype == LITENN_F32) || m > 0x3fffffffu || n_head > 65535 || past + m > 0x3fffffffu)
 		{
 			return false;
 		}

@@ -1298,7 +1298,7 @@ namespace litenn_hip
 	                     size_t query_offset, float* out, hipStream_t s)
 	{
 		const double score_scale = logit_softcap != 0.0 ? scale / logit_softcap : scale;
-		if (attn_rows_pays(m, keys, cache_dtype == LITENN_F32))
+		if (attn_rows_pay_options(m, keys, n_head, cache_dtype == LITENN_F32))
 		{
 			RowsAttn a;
 			a.q = q;

@@ -1721,7 +1721,7 @@ namespace litenn_hip
 		const dim3 rows(a.rows, a.shape.heads);
 		if (a.f32)
 		{
-			if (attn_rows_pays(a.rows, std::min(a.keys, a.shape.window), true))
+			if (attn_rows_pay_window(a.rows, std::min(a.keys, a.shape.window)))
 			{
 				RowsAttn r;
 				r.q = a.q;
