@@ -5,10 +5,12 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <cstring>
 
 namespace litenn_hip
 {
 	size_t argmax_step_scratch_bytes(size_t n);
+	void launch_zero_ints(int* p, size_t n, hipStream_t s);
 	void launch_argmax_step(const float* x, size_t n, void* scratch, int32_t* next, int* counters, int past_inc,
 	                        int32_t* out, hipStream_t s);
 
@@ -26,15 +28,56 @@ namespace litenn_hip
 
 		constexpr int kWaitRanOut = -2;
 
-		int check_error_flag(litenn_hip_model* m)
+		// What a pass leaves for the host goes to pinned memory from the device itself, the error word with it: n words from `from`
+		// to `to`, sixteen bytes a thread where both allow.  A copy to memory that is not pinned waits for the pass, stages and
+		// waits again: ten small launches and 32000 logits 136 us with two such copies, 57 this way (the host's own copy is 1 of them).
+		// (A run too long for the pinned memory, whose own length is what counts, is copied.)
+		__global__ __launch_bounds__(256) void deliver_kernel(const uint32_t* __restrict__ from, uint32_t* __restrict__ to, size_t n, size_t quads,
+		                                                      const int* __restrict__ err, int* __restrict__ err_to)
+		{
+			const size_t at = blockIdx.x * size_t{ 256 } + threadIdx.x, threads = gridDim.x * size_t{ 256 };
+			for (size_t i = at; i < quads; i += threads)
+			{
+				reinterpret_cast<uint4*>(to)[i] = reinterpret_cast<const uint4*>(from)[i];
+			}
+			for (size_t i = 4 * quads + at; i < n; i += threads)
+			{
+				to[i] = from[i];
+			}
+			if (err_to && at == 0)
+			{
+				*err_to = *err;
+			}
+		}
+
+		constexpr size_t kPinnedWords = size_t{ 1 } << 18; // and the error word behind them
+
+		// words [first, first + n) of the pinned memory from `from` (null: none), the error word last of all
+		void deliver(litenn_hip_model* m, const void* from, size_t first, size_t n, bool last)
+		{
+			uint32_t* const to = m->pinned + first;
+			const bool wide = ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15u) == 0;
+			const size_t quads = wide ? n / 4 : 0, blocks = ((wide ? quads : n) + 255) / 256;
+			deliver_kernel<<<dim3(static_cast<unsigned>(std::max<size_t>(1, std::min<size_t>(blocks, 256)))), dim3(256), 0, m->stream>>>(
+			    static_cast<const uint32_t*>(from), to, n, quads, m->d_err, last ? reinterpret_cast<int*>(m->pinned + kPinnedWords) : nullptr);
+		}
+
+		// Waits for the pass and looks at its error word, which was delivered or is copied here.
+		int check_error_flag(litenn_hip_model* m, bool delivered)
 		{
 			int flag = 0;
-			LITENN_HIP_TRY(m->action, hipMemcpyAsync(&flag, m->d_err, sizeof(int), hipMemcpyDeviceToHost, m->stream));
+			if (!delivered)
+			{
+				LITENN_HIP_TRY(m->action, hipMemcpyAsync(&flag, m->d_err, sizeof(int), hipMemcpyDeviceToHost, m->stream));
+			}
 			LITENN_HIP_TRY(m->action, hipStreamSynchronize(m->stream));
+			if (delivered)
+			{
+				std::memcpy(&flag, m->pinned + kPinnedWords, sizeof(int));
+			}
 			if (flag)
 			{
-				const int zero = 0;
-				(void)hipMemcpy(m->d_err, &zero, sizeof(int), hipMemcpyHostToDevice);
+				launch_zero_ints(m->d_err, 1, m->stream); // (on the model's stream: the legacy one fails while another thread captures)
 				if (flag & 2)
 				{
 					return kWaitRanOut;
@@ -121,6 +164,11 @@ namespace litenn_hip
 		    (e = hipMemsetAsync(m->d_next, 0, sizeof(int32_t), m->stream)) != hipSuccess)
 		{
 			return e;
+		}
+		if (hipHostMalloc(reinterpret_cast<void**>(&m->pinned), sizeof(uint32_t) * (kPinnedWords + 1), hipHostMallocDefault) != hipSuccess)
+		{
+			(void)hipGetLastError();
+			m->pinned = nullptr; // results are copied, then
 		}
 		return hipMalloc(&m->argmax_scratch, argmax_step_scratch_bytes(static_cast<size_t>(m->vocab)));
 	}
@@ -215,6 +263,9 @@ namespace litenn_hip
 				set_counters_kernel<<<1, 1, 0, s>>>(m->d_counters, m->past, 0);
 				m->forward(m->d_tokens, count, logit_rows, flags, m->past);
 				LITENN_HIP_TRY(m->action, hipGetLastError());
+				const bool wants_last = last_logits && first + count == rows;
+				const size_t words = (pick_end - next_pick + (wants_last ? 1 : 0)) * vocab;
+				const bool delivered = m->pinned && words <= kPinnedWords;
 				for (size_t i = next_pick; i < pick_end;)
 				{
 					// consecutive rows that land in consecutive places travel together
@@ -223,17 +274,28 @@ namespace litenn_hip
 					{
 						++j;
 					}
+					if (delivered)
+					{
+						deliver(m, m->logits + (picks[i].first - first_logit) * vocab, (i - next_pick) * vocab, vocab * (j - i), j == pick_end && !wants_last);
+						i = j;
+						continue;
+					}
 					LITENN_HIP_TRY(m->action,
 					               hipMemcpyAsync(out + picks[i].second * vocab, m->logits + (picks[i].first - first_logit) * vocab,
 					                              sizeof(float) * vocab * (j - i), hipMemcpyDeviceToHost, s));
 					i = j;
 				}
-				if (last_logits && first + count == rows)
+				if (delivered && (wants_last || pick_end == next_pick))
+				{
+					deliver(m, m->logits + (logit_rows - 1) * vocab, (pick_end - next_pick) * vocab, wants_last ? vocab : 0, true);
+				}
+				else if (wants_last)
 				{
 					LITENN_HIP_TRY(m->action, hipMemcpyAsync(last_logits, m->logits + (logit_rows - 1) * vocab,
 					                                         sizeof(float) * vocab, hipMemcpyDeviceToHost, s));
 				}
-				const int rc = check_error_flag(m);
+				LITENN_HIP_TRY(m->action, hipGetLastError());
+				const int rc = check_error_flag(m, delivered);
 				if (rc == kWaitRanOut && attempt == 0 && m->give_up_waiting())
 				{
 					continue; // and once more through the other form
@@ -241,6 +303,17 @@ namespace litenn_hip
 				if (rc != 0)
 				{
 					return rc == kWaitRanOut ? fail(m->action, "a wait inside the decoder step ran out") : 1;
+				}
+				if (delivered)
+				{
+					for (size_t i = next_pick; i < pick_end; ++i)
+					{
+						std::memcpy(out + picks[i].second * vocab, m->pinned + (i - next_pick) * vocab, sizeof(float) * vocab);
+					}
+					if (wants_last)
+					{
+						std::memcpy(last_logits, m->pinned + (pick_end - next_pick) * vocab, sizeof(float) * vocab);
+					}
 				}
 				break;
 			}
@@ -390,15 +463,25 @@ namespace litenn_hip
 		}
 		GEN_TRY(hipEventRecord(ev[2], s));
 		GEN_TRY(hipGetLastError());
-		GEN_TRY(hipMemcpyAsync(out_tokens, m->d_out, sizeof(int32_t) * n_new, hipMemcpyDeviceToHost, s));
 		int step_flag = 0;
-		GEN_TRY(hipMemcpyAsync(&step_flag, m->d_err, sizeof(int), hipMemcpyDeviceToHost, s));
-		GEN_TRY(hipStreamSynchronize(s));
+		if (m->pinned && n_new <= kPinnedWords)
+		{
+			deliver(m, m->d_out, 0, n_new, true);
+			GEN_TRY(hipGetLastError());
+			GEN_TRY(hipStreamSynchronize(s));
+			std::memcpy(out_tokens, m->pinned, sizeof(int32_t) * n_new);
+			std::memcpy(&step_flag, m->pinned + kPinnedWords, sizeof(int));
+		}
+		else
+		{
+			GEN_TRY(hipMemcpyAsync(out_tokens, m->d_out, sizeof(int32_t) * n_new, hipMemcpyDeviceToHost, s));
+			GEN_TRY(hipMemcpyAsync(&step_flag, m->d_err, sizeof(int), hipMemcpyDeviceToHost, s));
+			GEN_TRY(hipStreamSynchronize(s));
+		}
 		if ((step_flag & 2) && m->give_up_waiting())
 		{
 			// the tokens are void; once more, from the prompt, through the other form (`past` has not moved)
-			const int zero = 0;
-			GEN_TRY(hipMemcpy(m->d_err, &zero, sizeof(int), hipMemcpyHostToDevice));
+			launch_zero_ints(m->d_err, 1, s);
 			cleanup();
 			return decoder_generate(m, prompt, n_prompt, n_new, out_tokens, flags, prefill_ms, decode_ms);
 		}
@@ -446,6 +529,10 @@ litenn_hip_model::~litenn_hip_model()
 		{
 			(void)hipFree(ptr);
 		}
+	}
+	if (pinned)
+	{
+		(void)hipHostFree(pinned);
 	}
 	if (stream)
 	{

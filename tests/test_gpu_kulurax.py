@@ -380,3 +380,21 @@ def test_models_of_both_kinds_side_by_side(hip, oracle):
     as_model._h = ctypes.c_void_p()  # one owner
     llama.close()
     other.close()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_wanted_rows_are_the_rows_of_a_whole_run(hip, dtype):
+    """Results that come back through pinned memory (up to 2^18 words), in runs and out of order, and ones that are copied."""
+    cfg = ku.config([ku.attention(heads=1, dim=8, vdim=8, window=16)], vocab=67, width=50)
+    model, _ = pair(hip, cfg, 23, dtype, context_length=4100)
+    toks = np.random.default_rng(5).integers(0, 67, 4000)
+    whole = model.eval(toks)  # 268000 words
+    model.reset()
+    part = model.eval(toks[:3911])  # 262037
+    assert ku.error(part, whole[:3911]) <= LIMIT[dtype]
+    for want in ([3999], [0], [7, 8, 9, 3000, 2, 2], list(range(100, 200)) + [5], []):
+        model.reset()
+        got = model.eval(toks, want=want)
+        assert got.shape == (len(want), 67)
+        if want:
+            assert ku.error(got, whole[want]) <= LIMIT[dtype]
