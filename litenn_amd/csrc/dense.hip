@@ -959,7 +959,10 @@ namespace litenn_hip
 		int tiles(const DenseRows& d, int bm, int bn) { return ((d.m + bm - 1) / bm) * ((d.w.n + bn - 1) / bn); }
 	} // namespace
 
-	int dense_rows_splits(const DenseMatrix& w, int m) { return fetch::dense_ranges(w.n, w.pitch / kTileK, m); }
+	int dense_rows_splits(const DenseMatrix& w, int m, bool f32)
+	{
+		return f32 ? fetch::dense_f32_ranges(w.n, w.pitch / kTileK, m) : fetch::dense_ranges(w.n, w.pitch / kTileK, m);
+	}
 
 	size_t dense_row_max_k() { return kRowLdsLimit / sizeof(float) / (kFlight * kRowBlock) * (kFlight * kRowBlock); }
 

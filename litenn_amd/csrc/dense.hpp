@@ -79,7 +79,7 @@ namespace litenn_hip
 		float softcap = 0.0f; // kOutF32: > 0: c becomes softcap tanh(c / softcap)
 	};
 	constexpr int kDenseMaxSplits = fetch::kDenseMaxRanges;
-	int dense_rows_splits(const DenseMatrix& w, int m);
+	int dense_rows_splits(const DenseMatrix& w, int m, bool f32);
 	void launch_dense_rows(const DenseRows& a, hipStream_t s);
 } // namespace litenn_hip
 

@@ -46,26 +46,6 @@ namespace litenn_hip
 		// buffers of a ring at most: a kernel asks for tiles that many rounds past the one it multiplies
 		constexpr int kDenseMaxBuffers = 8;
 
-		// The ranges of K a sublayer's last product of m rows is walked in at once, each with sums of its own
-		// [m, ld] behind the one before: where there are few tiles, enough for about two workgroups per CU and
-		// none shorter than 16 tiles of K.
-		constexpr int kDenseMaxRanges = 4, kDenseRangedRows = 1024;
-		inline int dense_ranges(int n, int k_tiles, int m)
-		{
-			if (m > kDenseRangedRows)
-			{
-				return 1;
-			}
-			const int tiles = ((m + (m <= 32 ? 31 : 63)) / (m <= 32 ? 32 : 64)) * ((n + 63) / 64);
-			return imax(1, imin(kDenseMaxRanges, imin((512 + tiles / 2) / tiles, k_tiles / 16)));
-		}
-		// rows of sums that passes of up to `rows` rows write: a short pass in ranges may write more than a long one
-		inline size_t dense_sum_rows(size_t rows)
-		{
-			const size_t ranged = kDenseMaxRanges * (rows < kDenseRangedRows ? rows : kDenseRangedRows);
-			return rows > ranged ? rows : ranged;
-		}
-
 		// The form a product of bfloat16 operands takes, activation rows x weight rows of a tile; the two with a digit behind
 		// differ in the buffers of their ring.  (All give the same bits.)
 		enum DenseForm
@@ -80,7 +60,12 @@ namespace litenn_hip
 		// With one time for a workgroup whether it shares its CU or not, and without 128 x 128, tiles in a row took up to 1.6 times
 		// as long: us for 639 x 4096 x 14336 in 192 x 128 with two buffers 201, 128 x 128 with three 132; 178 rows in three
 		// ranges 78, 45; 1100 x 2048 x 5632 85, 51.
-		inline DenseForm dense_form(int n, int k_tiles, int m, int ranges)
+		struct DenseChoice
+		{
+			DenseForm form;
+			long long ns;
+		};
+		inline DenseChoice dense_choice(int n, int k_tiles, int m, int ranges)
 		{
 			struct Cost
 			{
@@ -109,7 +94,51 @@ namespace litenn_hip
 					best = form;
 				}
 			}
-			return static_cast<DenseForm>(best);
+			return { static_cast<DenseForm>(best), least };
+		}
+		inline DenseForm dense_form(int n, int k_tiles, int m, int ranges) { return dense_choice(n, k_tiles, m, ranges).form; }
+
+		// The ranges of K a sublayer's last product of m rows is walked in at once, each with sums of its own [m, ld] behind the one
+		// before, none shorter than 16 tiles of K.  Float32 operands: where there are few tiles, enough for about two workgroups per CU.
+		// bfloat16: as many as take least time, a range's sums being written and read again at 4500 bytes a ns.  (By the rule of the
+		// Float32 operands 777 x 2048 x 5632 had one range, whose 224 tiles of 128 x 64 wait for L2: 37.8 us, and 30.6 in three
+		// with 2.9 for the sums; 777 x 2048 x 4096 28.8, and 24.8 in two with 2.3; a 4096-wide prompt of 639 tokens, two
+		// layers, 1085 and 1008.)
+		constexpr int kDenseMaxRanges = 4, kDenseRangedRows = 1024;
+		inline int dense_ranges(int n, int k_tiles, int m)
+		{
+			if (m > kDenseRangedRows)
+			{
+				return 1;
+			}
+			int best = 1;
+			long long least = -1;
+			for (int ranges = 1; ranges <= imax(1, imin(kDenseMaxRanges, k_tiles / 16)); ++ranges)
+			{
+				const long long sums = static_cast<long long>(ranges - 1) * m * n * 16 / 9000;
+				const long long ns = dense_choice(n, k_tiles, m, ranges).ns + sums;
+				if (least < 0 || ns < least)
+				{
+					least = ns;
+					best = ranges;
+				}
+			}
+			return best;
+		}
+		inline int dense_f32_ranges(int n, int k_tiles, int m)
+		{
+			if (m > kDenseRangedRows)
+			{
+				return 1;
+			}
+			const int tiles = ((m + (m <= 32 ? 31 : 63)) / (m <= 32 ? 32 : 64)) * ((n + 63) / 64);
+			return imax(1, imin(kDenseMaxRanges, imin((512 + tiles / 2) / tiles, k_tiles / 16)));
+		}
+		// rows of sums that passes of up to `rows` rows write: a short pass in ranges may write more than a long one
+		inline size_t dense_sum_rows(size_t rows)
+		{
+			const size_t ranged = kDenseMaxRanges * (rows < kDenseRangedRows ? rows : kDenseRangedRows);
+			return rows > ranged ? rows : ranged;
 		}
 
 		// The form a product of Float32 operands takes.  Beyond 256 tiles of 64 x 128 it is one chain over K, up to there, and for

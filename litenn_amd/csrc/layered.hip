@@ -964,7 +964,7 @@ namespace litenn_hip
 				d.c = y;
 				d.ldc = ld_y;
 				d.f32 = f32;
-				d.splits = parts = dense_rows_splits(w, rows);
+				d.splits = parts = dense_rows_splits(w, rows, f32);
 				d.split_stride = part_stride;
 				launch_dense_rows(d, stream);
 				pending = after;
