@@ -477,3 +477,21 @@ def test_rotations_that_end_inside_four_features(hip, oracle, head_dim, rope, kv
     assert rel_l2(dev.eval(toks[33:]), ref.eval(toks[33:])) < 1e-4
     for got, want in zip(dev.get_kv(1), ref.get_kv(1)):
         assert rel_l2(got, want) < 1e-3
+
+
+@pytest.mark.parametrize("fmt", [Q4_0, Q4_K])
+@pytest.mark.parametrize("kv", [DT_F16, DT_F32])
+@pytest.mark.parametrize("rows,precise", [(2, True), (7, False), (40, True), (40, False), (130, True), (130, False)])
+def test_last_logits_are_those_of_a_whole_run(hip, fmt, kv, rows, precise):
+    """Only the rows whose logits are asked for go through the last block: their logits, the caches and what follows are
+    those of a run that asks for all (products of one row keep Float32 operands, of several Float16 ones unless precise)."""
+    cfg = synth.tiny_llama(fmt, block_count=2, d_model=512, heads=4, kv_heads=2, ff=1024, vocab=777, context_length=160)
+    toks = synth.prompt_tokens(cfg, rows + 1, 3)
+    whole, last = (hip_model(hip, cfg, 5, kv_dtype=kv) for _ in range(2))
+    bound = 1e-4 if precise or rows < 4 else 4e-3
+    want = whole.eval(toks[:rows], precise=precise)[-1]
+    assert rel_l2(last.eval(toks[:rows], all_logits=False, precise=precise), want) < bound
+    for layer in range(2):
+        for a, b in zip(whole.get_kv(layer), last.get_kv(layer)):
+            assert np.array_equal(a, b)
+    assert rel_l2(last.eval(toks[rows:], all_logits=False), whole.eval(toks[rows:], all_logits=False)) < 1e-6
