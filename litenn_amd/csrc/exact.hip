@@ -993,7 +993,11 @@ namespace litenn_hip
 		}
 
 		// The same with less held ahead.  WN > 1: the fragments pass through the same two buffers, two stages on their way; with WN =
-		// 1 nobody shares them and they go to registers directly, each refilled for the next stage once it has been used.
+		// 1 nobody shares them and they go to registers directly, each refilled for a later step once it has been used.  Nobody is
+		// waited for there either: a wavefront walks its own range with no branch in a chunk's steps, which the compiler orders as
+		// one run.  With two tiles only two steps' fragments are held (four: 32 more registers, the sums' and scales' loads waited
+		// for in turn).  Q6_K 4096 x 14336, 1000 rows: 630 us with a branch a stage and four steps, 608 with two, 595 without the
+		// branches; 14336 x 4096, 45 rows: 52.1 -> 50.0; one tile (Q4_0, Q8_0): 1 to 4 %.
 		template <typename F, int MT, int WN, int KS>
 		__global__ __launch_bounds__(64 * WN * KS) void exact_gemm_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                  const float* residual, int k, int m, int m_tiles,
@@ -1031,8 +1035,9 @@ namespace litenn_hip
 			}
 
 			// ---- activations
-			half8 direct[kShared ? 1 : MT][4][2]; // WN = 1
-			u32x4 staged[2][kPieces];             // WN > 1: the next two stages on their way
+			constexpr int kHeld = MT > 1 ? 2 : 4; // steps whose fragments are here or on their way, WN = 1
+			half8 direct[kShared ? 1 : MT][kHeld][2];
+			u32x4 staged[2][kPieces]; // WN > 1: the next two stages on their way
 			uint8_t* const ring = lds + part * (2 * MT * kStageBytes);
 			const auto request = [&](u32x4 (&into)[kPieces], int c, int st) {
 #pragma unroll
@@ -1058,7 +1063,7 @@ namespace litenn_hip
 #pragma unroll
 					for (int e = 0; e < 2; ++e)
 					{
-						direct[t][s][e] = *reinterpret_cast<const half8*>(tiles[t] + static_cast<size_t>(c) * kTileChunkBytes +
+						direct[t][s % kHeld][e] = *reinterpret_cast<const half8*>(tiles[t] + static_cast<size_t>(c) * kTileChunkBytes +
 						                                                  st * kStageBytes + (2 * s + e) * kFrag);
 					}
 				}
@@ -1076,7 +1081,7 @@ namespace litenn_hip
 				else
 				{
 #pragma unroll
-					for (int s = 0; s < 4; ++s)
+					for (int s = 0; s < kHeld; ++s)
 					{
 						fetch_direct(c_begin, 0, s);
 					}
@@ -1093,10 +1098,11 @@ namespace litenn_hip
 				__syncthreads();
 			}
 			int buffer = 0;
-			for (int i = 0; i < per; ++i)
+			const int trips = kShared ? per : c_end - c_begin;
+			for (int i = 0; i < trips; ++i)
 			{
 				const int c = c_begin + i;
-				const bool live = c < c_end; // (uniform: a shorter range only passes the barriers)
+				const bool live = !kShared || c < c_end; // (uniform: a shorter range only passes the barriers)
 				const int next = min(c + 1, c_end - 1);
 				typename F::Head head;
 				floatx16 sum[MT]; // the chunk's, where kScaleSteps is less
@@ -1144,7 +1150,7 @@ namespace litenn_hip
 									}
 									else
 									{
-										a[e] = direct[t][s][e];
+										a[e] = direct[t][s % kHeld][e];
 									}
 								}
 								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b, fresh ? floatx16{} : p[t], 0, 0, 0);
@@ -1152,7 +1158,7 @@ namespace litenn_hip
 							}
 							if constexpr (!kShared)
 							{
-								fetch_direct(st < 3 ? c : next, (st + 1) & 3, s);
+								fetch_direct(step + kHeld < 16 ? c : next, ((step + kHeld) & 15) / 4, (s + kHeld) % 4);
 							}
 							if constexpr (F::kMins)
 							{
