@@ -805,13 +805,20 @@ def bench_layered(ln, which, names, prompts, n_new=128, window=1024, vocab=32000
             for side, (pre, dec) in best.items():
                 if side in cfgs:
                     w_bytes = synth.layered_decode_weight_bytes(cfgs[side])
-                    flops = synth.layered_prefill_flops(cfgs[side], n_prompt)
+                    # (the last layer's output projections and feed-forward half take the last row alone)
+                    last = f"l{len(cfgs[side]['layers']) - 1}."
+                    one_row = sum(2.0 * s[0] * s[1] for n, s in synth.TENSOR_SHAPES[cfgs[side]["architecture"]](cfgs[side]).items()
+                                  if n.startswith(last) and (n.endswith(".o") or ".mlp." in n))
+                    flops = synth.layered_prefill_flops(cfgs[side], n_prompt) - one_row * (n_prompt - 1)
                 else:
                     w_bytes = lcfg.matmul_weight_bytes_per_token()
                     per_token = sum(2.0 * s[0] * s[1] for kind, s in lcfg.tensor_shapes().items()
                                     if kind not in ("token_embd", "output")) * lcfg.block_count
-                    flops = per_token * n_prompt + 2.0 * vocab * lcfg.embedding_length + \
-                        4.0 * lcfg.block_count * lcfg.embedding_length * n_prompt * (n_prompt + 1) / 2
+                    # (behind the last block's keys and values the last row alone)
+                    one_row = sum(2.0 * s[0] * s[1] for kind, s in lcfg.tensor_shapes().items()
+                                  if kind == "attn_output" or kind.startswith("ffn_"))
+                    flops = per_token * n_prompt - one_row * (n_prompt - 1) + 2.0 * vocab * lcfg.embedding_length + \
+                        4.0 * lcfg.embedding_length * n_prompt * ((lcfg.block_count - 1) * (n_prompt + 1) / 2 + 1)
                 step_us = dec / (n_new - 1) * 1e3
                 run[side] = {"prefill_ms": round(pre, 3), "prefill_tokens_per_s": round(n_prompt / pre * 1e3, 1),
                              "prefill_tflops": round(flops / pre / 1e9, 1),
