@@ -487,7 +487,7 @@ namespace litenn_hip
 #pragma unroll
 				for (int u = 0; u < kUnroll; ++u)
 				{
-					// keys past the chunk re-read a valid one and get weight zero below
+					// keys past the chunk re-read a valid one and count for nothing below
 					const int t = min(from + 16 * u, t_end - 1);
 					k_raw[u] = Load::load(kbase + static_cast<size_t>(t) * kvw, first, per, head_dim);
 					v_raw[u] = Load::load(vbase + static_cast<size_t>(t) * kvw, first, per, head_dim);
@@ -558,8 +558,8 @@ namespace litenn_hip
 					s[u] = (t0 + 16 * u < t_end) ? acc : -INFINITY;
 					step_m = fmaxf(step_m, s[u]);
 				}
-				// step_m is finite: the first key of the step is always inside the chunk
-				const float corr = expf(run_m - step_m);
+				const float ref_m = step_m == -INFINITY ? 0.0f : step_m; // (every score so far -inf: weights of zero)
+				const float corr = expf(run_m - ref_m);
 				run_l *= corr;
 #pragma unroll
 				for (int e = 0; e < E; ++e)
@@ -569,12 +569,15 @@ namespace litenn_hip
 #pragma unroll
 				for (int u = 0; u < kUnroll; ++u)
 				{
-					const float p = expf(s[u] - step_m);
+					const float p = expf(s[u] - ref_m);
 					run_l += p;
-#pragma unroll
-					for (int e = 0; e < E; ++e)
+					if (u == 0 || t0 + 16 * u < t_end) // (an infinite value would meet a weight of zero)
 					{
-						o[e] = fmaf(p, vf[u][e], o[e]);
+#pragma unroll
+						for (int e = 0; e < E; ++e)
+						{
+							o[e] = fmaf(p, vf[u][e], o[e]);
+						}
 					}
 				}
 				run_m = step_m;
@@ -592,9 +595,9 @@ namespace litenn_hip
 						acc = fmaf(qv[e], kn[e], acc);
 					}
 					const float sc = row16_sum(acc) * scale;
-					const float step_m = fmaxf(run_m, sc);
-					const float corr = expf(run_m - step_m);
-					const float pw = expf(sc - step_m);
+					const float step_m = fmaxf(run_m, sc), ref_m = step_m == -INFINITY ? 0.0f : step_m;
+					const float corr = expf(run_m - ref_m);
+					const float pw = expf(sc - ref_m);
 					run_l = fmaf(run_l, corr, pw);
 #pragma unroll
 					for (int e = 0; e < E; ++e)
@@ -703,9 +706,10 @@ namespace litenn_hip
 #pragma unroll
 				for (int sidx = 0; sidx < kMaxAttnSplits; ++sidx)
 				{
+					// (chunks there are not re-read the last one's, whose outputs may be infinite)
 					const float w = sidx < splits ? softmax_weight(pm[sidx], mm) : 0.0f;
 					ll = fmaf(pl[sidx], w, ll);
-					oo = fmaf(po[sidx], w, oo);
+					oo = fmaf(sidx < splits ? po[sidx] : 0.0f, w, oo);
 				}
 				dst[tid] = oo / ll;
 			}

@@ -133,6 +133,39 @@ def test_attention_with_large_scores(hip, oracle, cache_dtype):
         assert rel_l2(got, want) < 1e-5, (m, past, H, KH, hd)
 
 
+@pytest.mark.parametrize("cache_dtype", [DT_F32, DT_F16])
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("keys", [1, 3, 10, 16, 40, 49, 65, 100, 129, 1000, 3001])
+def test_one_row_over_infinite_keys_and_values(hip, cache_dtype, hd, keys):
+    """An infinite value gives an infinity, also at the end of a chunk of keys, and keys whose score is -inf count for nothing:
+    the row by itself (chunks of keys) and as the last of two (no chunks)."""
+    rng = np.random.default_rng(43)
+    heads = 4
+    q = rng.standard_normal((2, heads * hd)).astype(np.float32)
+    q[:, ::hd] = -1.0  # times a key that is infinite there: -inf
+    k, v = (rng.standard_normal((keys, heads * hd)).astype(np.float16).astype(np.float32) for _ in range(2))
+    v[keys - 1, 5::hd] = np.inf
+    v[keys // 3, 6::hd] = -np.inf
+    hidden = [t for t in range(keys) if t % 16 in (1, 5, 15) and t not in (keys - 1, keys // 3)]
+    k[hidden, 0::hd] = np.inf
+    kc, vc = (T(hip, a, np.float16 if cache_dtype == DT_F16 else np.float32) for a in (k, v))
+    want = np.empty((heads, hd))
+    for h in range(heads):
+        at = slice(h * hd, (h + 1) * hd)
+        with np.errstate(invalid="ignore"):
+            s = k[:, at].astype(np.float64) @ q[1, at] / math.sqrt(hd)
+        w = np.exp(s - s.max())
+        use = w > 0  # (weights of these scores are zero or far from it)
+        want[h] = w[use] / w.sum() @ v[use, at].astype(np.float64)
+    want = want.reshape(-1)
+    for m in (1, 2):
+        if keys >= m:
+            got = hip.attn_decode(T(hip, q[2 - m:]), kc, vc, m, keys - m, heads, heads, hd).numpy()[-1]
+            finite = np.isfinite(want)
+            assert np.array_equal(got[~finite], want[~finite]), m
+            assert rel_l2(got[finite], want[finite]) < 1e-5, m
+
+
 def _attention_want(oracle, q, k, v, past, H, KH, hd):
     want = np.empty_like(q)
     for h in range(H):
