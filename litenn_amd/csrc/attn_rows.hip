@@ -135,6 +135,14 @@ namespace litenn_hip
 		template <typename O, int D, int QW>
 		constexpr int group_bytes() { return O::kStored * kKeys * (one_buffer<O, QW>() ? value_stride<D>() : key_stride<D>() + value_stride<D>()); }
 
+		// The second half of the queries waits in LDS where every wavefront has the same ones and registers are short: behind all
+		// buffers, or, where that keeps a second workgroup of four wavefronts off the CU (83968 bytes, and 75776 without), in the 64
+		// bytes that set one row of values apart from the next.  (1000 rows on 1000 keys 67 and 49 us.)
+		template <typename O, int D, int QW>
+		constexpr bool queries_in_lds() { return O::kSplit == 2 && QW == 1 && D == 128; }
+		template <typename O, int D, int QW, int KW>
+		constexpr bool queries_between_values() { return queries_in_lds<O, D, QW>() && KW == 4; }
+
 		// A workgroup takes 32 QW query rows of one head; its KW groups of QW wavefronts take the key tiles in turn,
 		// each group with its own buffers, and merge at the end.
 		template <typename O, int D, int QW, int KW>
@@ -146,8 +154,7 @@ namespace litenn_hip
 			constexpr int kKeyBytes = kKeys * kKeyStride, kValueBytes = kKeys * kValueStride; // of one part of a tile
 			constexpr bool kOneBuffer = one_buffer<O, QW>();
 			constexpr int kGroupBytes = group_bytes<O, D, QW>();
-			// The second half of the queries waits in LDS where every wavefront has the same ones and registers are short
-			constexpr bool kQueriesInLds = O::kSplit == 2 && QW == 1 && D == 128;
+			constexpr bool kQueriesInLds = queries_in_lds<O, D, QW>(), kQueriesBetween = queries_between_values<O, D, QW, KW>();
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KW][keys, values], queries; later the groups' results
 			const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 			const int group = wave / QW, qw = wave % QW;
@@ -286,7 +293,7 @@ namespace litenn_hip
 				{
 					*reinterpret_cast<u32x4*>(k_lds + at) = u32x4{ 0u, 0u, 0u, 0u };
 				}
-				if constexpr (QW > 1)
+				if constexpr (QW > 1 || kQueriesBetween)
 				{
 					__syncthreads();
 				}
@@ -359,15 +366,17 @@ namespace litenn_hip
 					}
 				}
 			}
-			uint8_t* const q_lds = lds + KW * kGroupBytes + lane * 16;
+			uint8_t* const q_lds = kQueriesBetween ? lds + kKeyBytes + (lane >> 2) * kValueStride + 2 * D + 16 * (lane & 3) : lds + KW * kGroupBytes + 16 * lane;
+			const auto q_step = [](int s) { return kQueriesBetween ? (s >> 1) * kGroupBytes + (s & 1) * 16 * kValueStride : 1024 * s; };
 			if constexpr (kQueriesInLds)
 			{
+				static_assert(!kQueriesBetween || (kValueStride == 2 * D + 64 && D / 32 <= KW && kKeys == 32), "16 rows a step, two steps a group");
 				if (group == 0)
 				{
 #pragma unroll
 					for (int s = 0; s < D / 16; ++s)
 					{
-						*reinterpret_cast<frag*>(q_lds + 1024 * s) = q[s][1];
+						*reinterpret_cast<frag*>(q_lds + q_step(s)) = q[s][1];
 					}
 				}
 				__syncthreads();
@@ -461,7 +470,7 @@ namespace litenn_hip
 						floatx16& to = p > 0 ? s_low : st % 2 == 0 ? s : s_odd;
 						if constexpr (kQueriesInLds)
 						{
-							to = O::multiply(kf, p == 0 ? q[st][0] : *reinterpret_cast<const frag*>(q_lds + 1024 * st), to);
+							to = O::multiply(kf, p == 0 ? q[st][0] : *reinterpret_cast<const frag*>(q_lds + q_step(st)), to);
 						}
 						else
 						{
@@ -790,10 +799,11 @@ namespace litenn_hip
 		template <typename O, int D, int QW, int KW>
 		void launch_form(const RowsAttn& a, hipStream_t s)
 		{
-			constexpr size_t tiles = static_cast<size_t>(KW) * group_bytes<O, D, QW>() + (O::kSplit == 2 && QW == 1 && D == 128 ? 64 * D : 0);
+			constexpr size_t tiles = static_cast<size_t>(KW) * group_bytes<O, D, QW>() + (queries_in_lds<O, D, QW>() && !queries_between_values<O, D, QW, KW>() ? 64 * D : 0);
 			constexpr size_t merge = static_cast<size_t>(KW) * QW * (D / 2 + 2) * 64 * sizeof(float);
 			constexpr size_t lds = tiles > merge ? tiles : merge;
 			static_assert(lds <= 160 * 1024, "LDS");
+			static_assert(O::kStored > 1 || KW > 4 || 2 * lds <= 160 * 1024, "two workgroups of four wavefronts a CU");
 			allow_dynamic_lds(reinterpret_cast<const void*>(&attn_rows_kernel<O, D, QW, KW>), lds);
 			attn_rows_kernel<O, D, QW, KW><<<dim3(a.heads, (a.rows + 32 * QW - 1) / (32 * QW)), dim3(64 * QW * KW), lds, s>>>(a);
 		}
@@ -821,10 +831,11 @@ namespace litenn_hip
 			else
 			{
 				// Eight wavefronts on a head's rows, one workgroup to a CU, while all of them fit the 256 CUs at once and have more than
-				// a tile or two each; four, two workgroups to a CU, for few keys and, heads of 128 on long runs of keys aside, for
-				// many rows (eight and four: 200 on 1000 24 and 27, 16 on 2000 32 and 44, 128 on 400 17.4 and 18.2, on 300 17.4 and
-				// 15.9, on 128 14.1 and 10.7, 512 on 512 30 and 27, 1000 on 2000 121 and 141; heads of 64, 300 on 1000 27 and 20).
-				if (groups <= 256 ? a.keys >= 384 : D == 128 && a.keys >= 1000)
+				// a tile or two each; four, two workgroups to a CU, for few keys and for many rows (eight and four: 200 on 1000 24 and
+				// 27, 16 on 2000 31 and 43, 128 on 400 17.3 and 18.1, on 300 17.3 and 15.9, on 128 13.8 and 10.6, 512 on 512 29 and 20,
+				// on 1024 41 and 32, 1000 on 2000 121 and 98, 1500 on 4000 306 and 272; heads of 64, 300 on 1000 26 and 19, 1000 on 4000
+				// 136 and 120).
+				if (groups <= 256 && a.keys >= 384)
 				{
 					launch_form<HalfOperands, D, 1, 8>(a, s);
 				}
