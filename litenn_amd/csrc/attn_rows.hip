@@ -30,6 +30,7 @@
 #include "common.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
+#include "fetch_model.hpp"
 
 #include <cmath>
 
@@ -811,15 +812,9 @@ namespace litenn_hip
 		template <int D>
 		void launch_dim(const RowsAttn& a, bool f32, hipStream_t s)
 		{
-			// us of both forms, 32 heads over 8 unless said, the rows on the keys behind
-			const size_t groups = static_cast<size_t>(a.heads) * ((a.rows + 31) / 32);
 			if (f32)
 			{
-				// Four wavefronts with keys of their own while their workgroups, one to a CU, fit the card at once, or twice over where
-				// half of them see half the keys and fewer (200 rows on 1000 keys 57 against 79 for two pairs that share their keys, 512
-				// on 512 of 16 heads 33 against 44, 700 on 700 of 16 44 and 57); pairs, which take their tiles apart once, from there on
-				// (300 on 1000 79 against 91, 1000 on 1000 93 and 133).
-				if (groups <= 256 || (groups <= 512 && a.keys == a.rows))
+				if (fetch::rows_float_alone({ a.rows, a.keys, a.causal, a.q_at, a.window }, a.heads, D))
 				{
 					launch_form<FloatOperands, D, 1, 4>(a, s);
 				}
@@ -830,11 +825,12 @@ namespace litenn_hip
 			}
 			else
 			{
+				const size_t groups = static_cast<size_t>(a.heads) * ((a.rows + 31) / 32);
 				// Eight wavefronts on a head's rows, one workgroup to a CU, while all of them fit the 256 CUs at once and have more than
-				// a tile or two each; four, two workgroups to a CU, for few keys and for many rows (eight and four: 200 on 1000 24 and
-				// 27, 16 on 2000 31 and 43, 128 on 400 17.3 and 18.1, on 300 17.3 and 15.9, on 128 13.8 and 10.6, 512 on 512 29 and 20,
-				// on 1024 41 and 32, 1000 on 2000 121 and 98, 1500 on 4000 306 and 272; heads of 64, 300 on 1000 26 and 19, 1000 on 4000
-				// 136 and 120).
+				// a tile or two each; four, two workgroups to a CU, for few keys and for many rows (us of eight and four, 32 heads over
+				// 8, rows on keys: 200 on 1000 24 and 27, 16 on 2000 31 and 43, 128 on 400 17.3 and 18.1, on 300 17.3 and 15.9, on 128
+				// 13.8 and 10.6, 512 on 512 29 and 20, on 1024 41 and 32, 1000 on 2000 121 and 98, 1500 on 4000 306 and 272; heads of 64,
+				// 300 on 1000 26 and 19, 1000 on 4000 136 and 120).
 				if (groups <= 256 && a.keys >= 384)
 				{
 					launch_form<HalfOperands, D, 1, 8>(a, s);

@@ -25,6 +25,56 @@ namespace litenn_hip
 		LITENN_FETCH_FN int imin(int a, int b) { return a < b ? a : b; }
 		LITENN_FETCH_FN int imax(int a, int b) { return a > b ? a : b; }
 
+		// ---- attention of many rows: what a block of 32 query rows sees ---------------------------
+		struct RowsSeen
+		{
+			int rows, keys;
+			bool causal;
+			long long q_at, window; // query i sees keys max(0, q_at + i - window + 1) .. (causal: q_at + i)
+			// tiles of 32 keys that rows first .. first + count - 1 see
+			int tiles(int first, int count) const
+			{
+				const long long end = first + count < rows ? first + count : rows;
+				const long long to = causal && q_at + end < keys ? q_at + end : keys;
+				const long long from = q_at + first - window + 1 > 0 ? q_at + first - window + 1 : 0;
+				return to > from ? static_cast<int>((to - from + 31) / 32) : 0;
+			}
+		};
+		// What up to 512 workgroups of `block` rows take, one to a CU and the longest first: a fixed part and a step for every `per` tiles of
+		// keys (tenths of a us).  From the 257th on one waits for the shortest that is left before it.
+		struct RowsCost
+		{
+			int once, twice, step; // fixed parts of a workgroup and of two in a row
+		};
+		inline int rows_time(const RowsSeen& a, int heads, int block, int per, RowsCost c)
+		{
+			const int blocks = (a.rows + block - 1) / block;
+			const auto steps = [&](int b) { return (a.tiles(block * b, block) + per - 1) / per; };
+			int time = c.once + c.step * steps(blocks - 1);
+			for (int b = blocks - 1 - 256 / heads; b >= 0; --b)
+			{
+				const int last = (blocks - b) * heads - 1; // of the block's workgroups, in the order of their start
+				time = imax(time, c.twice + c.step * (steps(b) + steps(blocks - 1 - imax(0, 511 - last) / heads)));
+			}
+			return time;
+		}
+		// Whether Float32 tiles go through four wavefronts of a workgroup of 32 rows, each with keys of its own, or through two pairs
+		// of 64 rows that share theirs: four tiles a step, or two in less time.  Up to 256 workgroups four wavefronts are the faster
+		// form, beyond 512 pairs, between the two what the steps take.  us of four and of pairs, 32 heads of 128 unless said: 200
+		// rows on 1000 keys 54 and 79, 1000 on 1000 133 and 93; causal, 300 on 300 28.9 and 30.6, on 301 34.8 and 31.8, on 1000 91 and
+		// 79, 512 on 512 45.7 and 44.6, of 64 26.5 and 29.6, 700 of 16 heads on 700 43 and 57, on 1000 70 and 80; every key seen
+		// by all, 300 on 300 51 and 31.
+		inline bool rows_float_alone(const RowsSeen& a, int heads, int dim)
+		{
+			const long long groups = static_cast<long long>(heads) * ((a.rows + 31) / 32);
+			if (groups <= 256 || groups > 512)
+			{
+				return groups <= 256;
+			}
+			return dim > 64 ? rows_time(a, heads, 32, 4, { 98, 180, 55 }) < rows_time(a, heads, 64, 2, { 90, 160, 43 })
+			                : rows_time(a, heads, 32, 4, { 64, 123, 31 }) < rows_time(a, heads, 64, 2, { 61, 110, 29 });
+		}
+
 		// ---- products over bfloat16 weights: the K tiles of a group of wavefronts ----------------
 		// K is cut into `ranges` times `groups` parts, in order, that differ by a tile at most; the groups of a
 		// workgroup take neighbouring ones.  They pass one set of barriers, so all of them go through as many

@@ -746,6 +746,77 @@ static void test_dense_sum_rows()
 	std::printf("sums in ranges of K: %ld of %ld passes\n", ranged, passes);
 }
 
+// Attention of many rows over Float32 keys: the keys that a block of rows sees, and the form taken against what both take (us on
+// the card): never 5 % more than the faster one, whether or not rows and keys are equally many.
+static void test_rows_forms()
+{
+	using namespace litenn_hip::fetch;
+	for (const RowsSeen a : { RowsSeen{ 70, 70, true, 0, 1ll << 62 }, RowsSeen{ 70, 71, true, 1, 1ll << 62 }, RowsSeen{ 33, 400, true, 367, 40 },
+	                          RowsSeen{ 40, 300, false, 0, 1ll << 62 }, RowsSeen{ 40, 90, true, 100, 1ll << 62 }, RowsSeen{ 1, 1, true, 0, 1 } })
+	{
+		for (int first = 0; first < a.rows; first += 32)
+		{
+			int low = a.keys, high = -1;
+			for (int i = first; i < a.rows && i < first + 32; ++i)
+			{
+				for (int key = 0; key < a.keys; ++key)
+				{
+					if (key > a.q_at + i - a.window && (!a.causal || key <= a.q_at + i))
+					{
+						low = imin(low, key);
+						high = imax(high, key);
+					}
+				}
+			}
+			CHECK(a.tiles(first, 32) == (high - low + 32) / 32, "%d rows on %d keys, rows from %d: %d tiles", a.rows, a.keys, first, a.tiles(first, 32));
+		}
+	}
+	struct Measured
+	{
+		int rows, keys, heads, dim;
+		bool causal;
+		double alone, pairs;
+	};
+	const Measured measured[] = {
+		{ 300, 300, 32, 128, true, 28.9, 30.6 }, { 300, 301, 32, 128, true, 34.8, 31.8 }, { 300, 320, 32, 128, true, 34.6, 31.5 },
+		{ 300, 350, 32, 128, true, 34.9, 35.4 }, { 300, 400, 32, 128, true, 41.3, 39.9 }, { 300, 500, 32, 128, true, 52.1, 44.8 },
+		{ 300, 1000, 32, 128, true, 90.9, 79.2 }, { 512, 512, 32, 128, true, 45.7, 44.6 }, { 512, 513, 32, 128, true, 52.0, 49.7 },
+		{ 512, 700, 32, 128, true, 63.4, 58.5 }, { 512, 1024, 32, 128, true, 89.6, 79.9 }, { 700, 700, 16, 128, true, 43.3, 56.9 },
+		{ 700, 701, 16, 128, true, 46.9, 57.9 }, { 700, 1000, 16, 128, true, 69.5, 79.6 }, { 700, 1500, 16, 128, true, 111.5, 114.3 },
+		{ 1024, 1024, 16, 128, true, 67.3, 79.2 }, { 1024, 1500, 16, 128, true, 112.5, 115.7 }, { 400, 400, 24, 128, true, 33.9, 38.4 },
+		{ 400, 500, 24, 128, true, 46.5, 44.8 }, { 1200, 1200, 8, 128, true, 65.0, 91.2 }, { 1200, 2400, 8, 128, true, 145.8, 174.7 },
+		{ 2000, 2000, 8, 128, true, 111.4, 148.1 }, { 2000, 3000, 8, 128, true, 201.6, 217.9 }, { 3000, 3000, 4, 128, true, 142.3, 213.3 },
+		{ 3000, 4000, 4, 128, true, 206.4, 286.0 }, { 300, 300, 32, 128, false, 51.3, 31.4 }, { 512, 512, 24, 128, false, 61.3, 44.5 },
+		{ 700, 700, 16, 128, false, 85.0, 57.9 }, { 700, 128, 16, 128, false, 28.1, 18.0 }, { 1100, 2000, 8, 128, false, 195.7, 149.9 },
+		{ 1100, 1100, 8, 128, false, 118.3, 88.1 }, { 64, 300, 200, 128, false, 55.1, 32.6 }, { 64, 300, 200, 128, true, 54.9, 32.7 },
+		{ 30, 300, 300, 128, true, 54.9, 59.2 }, { 200, 1000, 32, 128, true, 53.9, 78.6 }, { 512, 512, 16, 128, true, 32.0, 43.7 },
+		{ 1000, 1000, 32, 128, true, 132.7, 92.6 }, { 600, 600, 32, 128, true, 63.8, 52.8 }, { 512, 512, 32, 64, true, 26.5, 29.6 },
+		{ 512, 700, 32, 64, true, 37.1, 38.7 }, { 700, 700, 16, 64, true, 25.2, 37.8 }, { 700, 1000, 16, 64, true, 40.2, 53.1 },
+		{ 300, 300, 32, 64, true, 17.0, 20.3 }, { 300, 1000, 32, 64, true, 52.6, 53.1 }, { 300, 400, 32, 64, true, 24.2, 26.6 },
+		{ 1024, 1024, 16, 64, true, 39.4, 52.7 }, { 1024, 1500, 16, 64, true, 65.9, 76.5 }, { 2000, 3000, 8, 64, true, 114.9, 143.1 },
+		{ 512, 1024, 32, 64, true, 52.4, 53.1 },
+	};
+	for (const Measured& p : measured)
+	{
+		const bool alone = rows_float_alone({ p.rows, p.keys, p.causal, p.causal ? p.keys - p.rows : 0, 1ll << 62 }, p.heads, p.dim);
+		const double least = p.alone < p.pairs ? p.alone : p.pairs;
+		CHECK((alone ? p.alone : p.pairs) <= 1.05 * least, "%d rows on %d keys, %d heads of %d, causal %d: alone %d", p.rows, p.keys, p.heads, p.dim, p.causal, alone);
+	}
+	for (int heads : { 1, 3, 8, 24, 255, 256, 257, 300, 512, 513 }) // any size has one
+	{
+		for (int rows = 1; rows <= 3000; rows += 1 + rows / 5)
+		{
+			for (bool causal : { false, true })
+			{
+				const RowsSeen a{ rows, rows + 7, causal, 7, 1ll << 62 };
+				const long long groups = static_cast<long long>(heads) * ((rows + 31) / 32);
+				CHECK(rows_float_alone(a, heads, 64) || groups > 256, "%d rows of %d heads", rows, heads);
+				CHECK(groups > 512 || (rows_time(a, heads, 32, 4, { 98, 180, 55 }) > 98 && rows_time(a, heads, 64, 2, { 90, 160, 43 }) > 90), "%d rows of %d heads", rows, heads);
+			}
+		}
+	}
+}
+
 int main(int argc, char** argv)
 {
 	if (argc > 1) // n k m ...: the forms of these products, with bfloat16 and with Float32 operands
@@ -758,6 +829,7 @@ int main(int argc, char** argv)
 		}
 		return 0;
 	}
+	test_rows_forms();
 	test_dense_walks();
 	test_dense_forms();
 	test_dense_sum_rows();

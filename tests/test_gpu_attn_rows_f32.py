@@ -50,7 +50,8 @@ def worst(got, want):
 CASES = [(16, 96, 3, 3, 128), (31, 129, 8, 2, 128), (32, 97, 4, 1, 64), (33, 128, 8, 8, 128), (65, 160, 2, 1, 64), (100, 333, 16, 4, 128),
          (40, 200, 2, 2, 72), (17, 500, 5, 5, 8), (16, 511, 3, 3, 128), (35, 529, 4, 2, 128), (16, 800, 3, 1, 64), (40, 512, 129, 43, 8),
          # four and eight groups on either side of 256 workgroups, Float32 tiles of a wavefront's own and in pairs
-         (101, 417, 16, 4, 128), (65, 1003, 32, 8, 128), (290, 290, 16, 16, 128), (290, 1001, 32, 8, 128), (97, 130, 96, 96, 120)]
+         (101, 417, 16, 4, 128), (65, 1003, 32, 8, 128), (290, 290, 16, 16, 128), (290, 1001, 32, 8, 128), (97, 130, 96, 96, 120),
+         (290, 291, 32, 8, 128), (350, 352, 24, 8, 64)]
 
 
 @pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
@@ -66,7 +67,8 @@ def test_causal_rows(hip, dtype, m, keys, heads, kv, dim):
 
 @pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
 @pytest.mark.parametrize("m,keys,heads,kv,dim", [(16, 96, 6, 3, 128), (37, 130, 8, 8, 64), (33, 545, 8, 4, 128), (20, 2050, 2, 2, 64),
-                                                   (4, 128, 2, 1, 120), (5, 1029, 3, 1, 128), (32, 75, 24, 8, 64)])
+                                                   (4, 128, 2, 1, 120), (5, 1029, 3, 1, 128), (32, 75, 24, 8, 64),
+                                                   (130, 137, 64, 8, 128)])
 @pytest.mark.parametrize("causal", [True, False])
 def test_options(hip, dtype, m, keys, heads, kv, dim, causal):
     q, k, v = inputs(2, m, keys, heads, kv, dim, dtype)
