@@ -26,6 +26,7 @@
 // v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
 // weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
 #include "common.hpp"
+#include "fetch_model.hpp"
 
 #include <algorithm>
 
@@ -1549,9 +1550,9 @@ namespace litenn_hip
 		void launch_exact_format(const ExactCall& c)
 		{
 			const int strips = (c.total_rows + kTile - 1) / kTile, units = strips * c.m_tiles;
-			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each
-			// decoded weight meets two tiles (us, kernel alone): Q4_K 28672 x 4096 at 300 rows 238 against 301 of the
-			// forms below, at 64 rows 53 against 62.  Not for Q6_K, whose scaling per step wants the registers.
+			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each decoded weight meets two
+			// tiles (us, kernel alone, weights from HBM, here and below): Q4_K 28672 x 4096 at 300 rows 226 against 313 of the
+			// forms below, at 64 rows 47 against 64.  Not for Q6_K, whose scaling per step wants the registers.
 			if constexpr (F::kScaleSteps > 1)
 			{
 				if ((strips + 3) / 4 * ((c.m_tiles + 1) / 2) >= 200 && c.m_tiles > 1)
@@ -1559,14 +1560,14 @@ namespace litenn_hip
 					return launch_variant<F, 2, 4, 2>(c);
 				}
 			}
-			// Otherwise a wavefront keeps to itself and the ranges of K fill the card.  Q6_K saves a second decode with two
-			// tiles once there are enough of them (4096 x 14336 at 300 rows 168 against 207; at 45 rows 52 against 44).
-			else if (units >= 512 && c.m_tiles > 1)
+			// Otherwise a wavefront keeps to itself and the ranges of K fill the card, in Q6_K with two tiles where these are enough.
+			else if (fetch::exact_two_tiles(strips, c.m_tiles))
 			{
 				return launch_variant<F, 2, 1, 8>(c);
 			}
-			// Eight ranges while there are few tiles (Q6_K 4096 x 14336 at 45 rows 44 against 54 with four), four from there
-			// on (Q4_K 14336 x 4096 at 8 rows 18.1 against 20.7 with eight) and for short rows (Q8_0 1024 x 1024 7.2 against 8.1).
+			// Eight ranges while there are few tiles (Q6_K 4096 x 14336 at 45 rows 41 against 46 with four, at 16 43 against 47), four
+			// from there on (Q4_K 14336 x 4096 at 45 rows 37 against 44 with eight, at 16 equal) and for short rows (Q8_0 1024 x 1024 at
+			// 16 rows 5.8 against 6.0).
 			if (units <= 256 && c.chunks >= 8)
 			{
 				launch_variant<F, 1, 1, 8>(c);

@@ -25,6 +25,19 @@ namespace litenn_hip
 		LITENN_FETCH_FN int imin(int a, int b) { return a < b ? a : b; }
 		LITENN_FETCH_FN int imax(int a, int b) { return a > b ? a : b; }
 
+		// ---- products of quantised weights with Float32 operands ----------------------------------
+		// Whether Q6_K takes two 32-row tiles of activations a wavefront, which saves a second decode, K in eight ranges and one workgroup
+		// to a CU.  Not for up to 256 tiles, which have a CU each, nor where up to 512 of one tile are all on the card at once and these
+		// are not.  us of a call, weights from HBM, one tile and two: 4096 x 14336, 64 rows 51 and 71, 96 rows 82 and 67, 160 115
+		// and 118, 300 190 and 181; 4128 x 4096, 33 rows 32 and 30; 1024 x 11008, 400 rows 78 and 62; 2100 x 4096, 200 rows 34 and 50.
+		// (From 512 on one tile would sometimes be faster, 14336 x 4096 at 96 rows 76 and 93, 45 56 and 53, but walks K in four
+		// ranges, which rounds more: K = 14336 1.23e-7 of the result, eight 1.16e-7.)
+		inline bool exact_two_tiles(int strips, int m_tiles)
+		{
+			const int ones = strips * m_tiles, twos = strips * ((m_tiles + 1) / 2);
+			return m_tiles > 1 && (ones >= 512 || (ones > 256 && twos <= 256));
+		}
+
 		// ---- attention of many rows: what a block of 32 query rows sees ---------------------------
 		struct RowsSeen
 		{

@@ -817,6 +817,34 @@ static void test_rows_forms()
 	}
 }
 
+// Q6_K with Float32 operands, one tile of activations a wavefront or two, against what a call takes either way (us on the card,
+// weights from HBM): up to 512 tiles never 5 % more than the faster one.
+static void test_exact_forms()
+{
+	struct Measured
+	{
+		int n, k, m;
+		double one, two;
+	};
+	const Measured measured[] = {
+		{ 4096, 14336, 33, 50.7, 70.6 }, { 4096, 14336, 45, 50.7, 70.5 }, { 4096, 14336, 64, 51.3, 70.9 }, { 4096, 14336, 65, 81.1, 65.7 },
+		{ 4096, 14336, 96, 81.7, 67.0 }, { 4096, 14336, 97, 82.3, 69.8 }, { 4096, 14336, 128, 83.4, 70.9 }, { 4096, 4096, 33, 24.8, 30.1 },
+		{ 4096, 4096, 64, 25.0, 30.6 }, { 4096, 4096, 96, 33.4, 31.6 }, { 4096, 4096, 128, 34.1, 32.4 }, { 8192, 4096, 33, 33.8, 31.3 },
+		{ 8192, 4096, 64, 34.2, 32.3 }, { 1024, 4096, 64, 23.8, 27.9 }, { 1024, 4096, 200, 25.5, 31.6 }, { 1024, 4096, 300, 34.1, 32.8 },
+		{ 1024, 4096, 512, 37.6, 35.5 }, { 2048, 5632, 64, 28.1, 36.2 }, { 2048, 5632, 128, 30.1, 38.1 }, { 2048, 5632, 200, 42.8, 38.6 },
+		{ 2720, 14336, 65, 49.7, 64.7 }, { 2720, 14336, 96, 50.0, 64.7 }, { 4128, 4096, 33, 32.2, 30.4 }, { 4128, 4096, 64, 32.5, 30.6 },
+		{ 4128, 14336, 33, 78.1, 70.3 }, { 4128, 14336, 64, 78.5, 70.8 }, { 7000, 4096, 33, 34.2, 31.3 }, { 7000, 4096, 64, 34.4, 32.2 },
+		{ 512, 2048, 600, 28.4, 27.9 }, { 512, 2048, 1000, 35.6, 31.7 }, { 1024, 11008, 270, 63.9, 58.0 }, { 1024, 11008, 400, 78.5, 62.0 },
+		{ 2100, 4096, 128, 31.6, 30.6 }, { 2100, 4096, 150, 32.3, 31.5 }, { 2100, 4096, 200, 33.5, 50.4 },
+	};
+	for (const Measured& p : measured)
+	{
+		const bool two = litenn_hip::fetch::exact_two_tiles((p.n + 31) / 32, (p.m + 31) / 32);
+		CHECK((two ? p.two : p.one) <= 1.05 * (p.one < p.two ? p.one : p.two), "%d x %d x %d: two tiles %d", p.m, p.n, p.k, two);
+	}
+	CHECK(!litenn_hip::fetch::exact_two_tiles(4000, 1) && litenn_hip::fetch::exact_two_tiles(448, 3), "one tile, and many");
+}
+
 int main(int argc, char** argv)
 {
 	if (argc > 1) // n k m ...: the forms of these products, with bfloat16 and with Float32 operands
@@ -830,6 +858,7 @@ int main(int argc, char** argv)
 		return 0;
 	}
 	test_rows_forms();
+	test_exact_forms();
 	test_dense_walks();
 	test_dense_forms();
 	test_dense_sum_rows();

@@ -183,9 +183,9 @@ def test_a_workspace_is_asked_for_where_one_is_used(hip, m, k, some):
 
 
 @pytest.mark.parametrize("fmt", FORMATS)
-@pytest.mark.parametrize("m,n,k", [(300, 5200, 1280), (300, 2000, 4352)])
+@pytest.mark.parametrize("m,n,k", [(300, 5200, 1280), (300, 2000, 4352), (33, 4100, 4352), (200, 2100, 768), (96, 7000, 512)])
 def test_forms_of_two_tiles_over_several_chunks(hip, fmt, m, n, k):
-    """Ranges of three chunks and two (four wavefronts on shared activations), of three, three and two (Q6_K's form)."""
+    """Ranges of three chunks and two (four wavefronts on shared activations; two tiles of Q6_K), and sizes beside them."""
     assert errors(hip, fmt, m, n, k, residual=fmt == Q4_0).max() <= 1e-6
 
 
