@@ -495,3 +495,31 @@ def test_last_logits_are_those_of_a_whole_run(hip, fmt, kv, rows, precise):
         for a, b in zip(whole.get_kv(layer), last.get_kv(layer)):
             assert np.array_equal(a, b)
     assert rel_l2(last.eval(toks[rows:], all_logits=False), whole.eval(toks[rows:], all_logits=False)) < 1e-6
+
+
+@pytest.mark.parametrize("fmt", [Q4_0, Q4_K])
+@pytest.mark.parametrize("earlier", [0, 37])
+@pytest.mark.parametrize("first", [0, 40, 100, 114, 115, 127, 129])
+def test_wanted_rows_with_float16_operands_are_those_of_a_whole_run(hip, fmt, earlier, first):
+    """A prompt of 130 rows, of which the last block takes those from the first wanted one on: tiles of many rows, of few, and one
+    row, behind cached tokens and not (Float16 operands round each block's activations once: 4e-3, caches to the bit)."""
+    import ctypes
+    from litenn_amd import _lib
+    cfg = synth.tiny_llama(fmt, block_count=2, d_model=512, heads=4, kv_heads=2, ff=1024, vocab=777, context_length=200)
+    toks = synth.prompt_tokens(cfg, earlier + 130, 3)
+    whole, some = (hip_model(hip, cfg, 5) for _ in range(2))
+    for model in (whole, some):
+        if earlier:
+            model.eval(toks[:earlier], all_logits=False, precise=False)
+    want = whole.eval(toks[earlier:], precise=False)
+    as_model = hip.Model(ctypes.c_void_p(_lib.load().litenn_hip_llama_model(some._h)))
+    rows = sorted({first, (first + 129) // 2, 129})
+    got = as_model.eval(toks[earlier:], want=rows, precise=False)
+    as_model._h = ctypes.c_void_p()  # one owner
+    for i, row in enumerate(rows):
+        assert rel_l2(got[i], want[row]) < 4e-3, row
+    for layer in range(2):
+        for a, b in zip(whole.get_kv(layer), some.get_kv(layer)):
+            assert np.array_equal(a, b)
+    for model in (whole, some):
+        model.close()
