@@ -166,8 +166,8 @@ namespace litenn_hip
 		// bfloat16: as many as take least time, a range's sums being written and read again at 4500 bytes a ns.  (By the rule of the
 		// Float32 operands 777 x 2048 x 5632 had one range, whose 224 tiles of 128 x 64 wait for L2: 37.8 us, and 30.6 in three
 		// with 2.9 for the sums; 777 x 2048 x 4096 28.8, and 24.8 in two with 2.3; a 4096-wide prompt of 639 tokens, two
-		// layers, 1085 and 1008.  The model leaves out some 2 us that a second range takes at any size: 2048 x 2048 takes 16.0 in one
-		// range and 18.5 in two at 400 rows, both with the norm behind it.)
+		// layers, 1085 and 1008.)  And 1.5 us for sums being there at all, which is what two ranges that save nothing take longer in
+		// the mean: 2048 x 2048 in one and in two, the norm behind it included, 400 rows 16.0 and 18.5, 777 21.6 and 23.3.
 		constexpr int kDenseMaxRanges = 4, kDenseRangedRows = 1024;
 		inline int dense_ranges(int n, int k_tiles, int m)
 		{
@@ -179,7 +179,7 @@ namespace litenn_hip
 			long long least = -1;
 			for (int ranges = 1; ranges <= imax(1, imin(kDenseMaxRanges, k_tiles / 16)); ++ranges)
 			{
-				const long long sums = static_cast<long long>(ranges - 1) * m * n * 16 / 9000;
+				const long long sums = ranges > 1 ? 1500 + static_cast<long long>(ranges - 1) * m * n * 16 / 9000 : 0;
 				const long long ns = dense_choice(n, k_tiles, m, ranges).ns + sums;
 				if (least < 0 || ns < least)
 				{
