@@ -37,7 +37,7 @@ namespace litenn_hip
 	//
 	// The causal row kernel: Float16 keys of 64, 8 rows on 96 10.7 / 7.3, of 128, 24 on 1000 29 / 21; Float32 keys, 48 on 1000 65 / 53.
 	// (Below some 20000 / sqrt(keys) rows of all heads together its 128-wide form is the faster one, 8 on 128 4.9 / 9.8, 30 on 300
-	// 14.6 / 15.0: the line does not follow it there, it goes by what rows and keys give in heads of 64 and in Float32 keys too.)
+	// 14.6 / 15.0: it could have a line of its own there, which is not drawn.)
 	inline bool attn_rows_pay_causal(size_t rows, size_t keys, bool f32) { return rows >= (f32 ? 16u : 8u) && keys >= 96; }
 	// The row kernel with options: a key at a time.  Float16 keys of 128: 2 rows on 48 9.0 / 10.6, on 64 10.5 / 10.4, on 96 14 / 10, on 1000
 	// 130 / 20, 64 on 64 29 / 10; heads of 64 on 64 keys 8.7 / 7.8.  Float32 keys: 2 rows on 96 14.9 / 14.9, of 64 8.7 / 9.8 and on
