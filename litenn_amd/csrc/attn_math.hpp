@@ -1,6 +1,6 @@
 // litenn-hip: the arithmetic of one new row's attention step that more than one kernel shares: the
 // separately rounded RoPE rotation, the cache type's rounding of the new key and value, the merge
-// weight of partial softmax triples, and the device-scope accesses through which workgroups hand
+// weight of partial softmax triples, the soft cap's tangent, and the device-scope accesses through which workgroups hand
 // values to each other inside one launch.
 #pragma once
 
@@ -33,6 +33,29 @@ namespace litenn_hip
 	{
 		return m == -INFINITY ? 0.0f : expf(m - m_all);
 	}
+
+	// ---- the soft cap's tangent
+	// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range.  (A division: the
+	// reciprocal instruction gives 0 above 2^126, which exp reaches short of its range's end.)
+	__device__ __forceinline__ float layer_tanh(float x)
+	{
+		const float ex = expf(__fmul_rn(x, 2.0f));
+		return __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
+	}
+	// Up to kSmallTangent its series to x^11, the next term 1.2e-8 of it, which is closer (the layer's form cancels: 1e-6 of a score of
+	// cap / 30).  Which of the two hangs on the score alone: neither hidden keys nor other queries change a query's bits.
+	constexpr float kSmallTangent = 0.35f;
+	__device__ __forceinline__ float small_tanh(float x)
+	{
+		const float x2 = x * x;
+		float p = -1382.0f / 155925.0f;
+		p = fmaf(p, x2, 62.0f / 2835.0f);
+		p = fmaf(p, x2, -17.0f / 315.0f);
+		p = fmaf(p, x2, 2.0f / 15.0f);
+		p = fmaf(p, x2, -1.0f / 3.0f);
+		return fmaf(x, x2 * p, x);
+	}
+	__device__ __forceinline__ float capped_tanh(float x) { return fabsf(x) <= kSmallTangent ? small_tanh(x) : layer_tanh(x); }
 
 	template <typename KV>
 	__device__ __forceinline__ float through_cache(float v);

@@ -26,8 +26,9 @@
 // values (three times the products, one wavefront a SIMD), 57 (85 in pairs of wavefronts that share their keys, on half the SIMDs).
 // Sums are short chains: scores in two sums, the parts' small products in one of their own, the weights' sum as a tree, outputs one
 // addition per tile, which costs 4 us and leaves the error against 64 bits below the row kernel's (mean of six inputs, 1e-7:
-// these rows, whose small capped scores the row kernel's tangent rounds, 1.30 and 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
+// these rows 1.30 and, the tangent in the layer's form throughout, 3.78, 150 rows on 700 keys 1.86 and 2.02, with Float32 keys 1.64 and 2.03).
 #include "common.hpp"
+#include "attn_math.hpp"
 #include "layer_device.hpp"
 #include "attn_rows.hpp"
 #include "fetch_model.hpp"
@@ -96,19 +97,6 @@ namespace litenn_hip
 			// (its powers of 2 to a power are one power of 2)
 			const int times = head < head_log2 ? 2 * (head + 1) : 2 * (head - head_log2) + 1;
 			return exp2(-(max_bias / 2.0) / static_cast<double>(head_log2) * static_cast<double>(times));
-		}
-
-		// tanh up to kSmallTangent: its series to x^11, the next term 1.2e-8 of it
-		constexpr float kSmallTangent = 0.35f;
-		__device__ __forceinline__ float small_tanh(float x)
-		{
-			const float x2 = x * x;
-			float p = -1382.0f / 155925.0f;
-			p = fmaf(p, x2, 62.0f / 2835.0f);
-			p = fmaf(p, x2, -17.0f / 315.0f);
-			p = fmaf(p, x2, 2.0f / 15.0f);
-			p = fmaf(p, x2, -1.0f / 3.0f);
-			return fmaf(x, x2 * p, x);
 		}
 
 		// exp(x) for x at most 0, or NaN: the product's rounding is put back behind the power of two, which below 2^-126 is 0.
@@ -386,15 +374,6 @@ namespace litenn_hip
 			const float factor = a.apply_scale ? unscale * a.scale : unscale; // (a power of two and the scale: one rounding for both)
 			const float* const mask_row = a.mask ? a.mask + static_cast<size_t>(row_c) * keys : nullptr;
 
-			// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1), NaN beyond exp's range.  (A
-			// division: the reciprocal instruction gives 0 above 2^126, which exp reaches short of its range's end.)
-			const auto layer_tanh = [](float v) {
-				const float ex = expf(__fmul_rn(v, 2.0f));
-				return __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
-			};
-			// Up to kSmallTangent its series, which is closer (the layer's form cancels: 1e-6 of a score of cap / 30).  Which of the
-			// two hangs on the score alone: neither hidden keys nor other queries change a query's bits.
-			const auto in_series = [](float v) { return fabsf(v) <= kSmallTangent; };
 			// a dot product's score (the causal mask and the window aside)
 			const auto score_of = [&](float v, float mv) {
 				if (a.apply_scale)
@@ -403,7 +382,7 @@ namespace litenn_hip
 				}
 				if (a.softcap != 0.0f)
 				{
-					v = in_series(v) ? small_tanh(v) : layer_tanh(v);
+					v = capped_tanh(v);
 					if (a.apply_cap)
 					{
 						v = __fmul_rn(v, a.softcap);
@@ -501,7 +480,7 @@ namespace litenn_hip
 					{
 						most = fmaxf(most, fabsf(sc[e])); // (a NaN stays one in either form)
 					}
-					if (__all(in_series(most)))
+					if (__all(most <= kSmallTangent))
 					{
 #pragma unroll
 						for (int e = 0; e < 16; ++e)
@@ -517,7 +496,7 @@ namespace litenn_hip
 							const float near = small_tanh(sc[e]);
 							float far = layer_tanh(sc[e]);
 							asm("" : "+v"(far)); // (a choice, not a branch for each score)
-							sc[e] = in_series(sc[e]) ? near : far;
+							sc[e] = fabsf(sc[e]) <= kSmallTangent ? near : far;
 							if (e == 7)
 							{
 								__builtin_amdgcn_sched_barrier(0); // (sixteen at once want registers that spill)

@@ -39,13 +39,7 @@ namespace litenn_hip
 	// (Below some 20000 / sqrt(keys) rows of all heads together its 128-wide form is the faster one, 8 on 128 4.9 / 9.8, 30 on 300
 	// 14.6 / 15.0: it could have a line of its own there, which is not drawn.)
 	inline bool attn_rows_pay_causal(size_t rows, size_t keys, bool f32) { return rows >= (f32 ? 16u : 8u) && keys >= 96; }
-	// The row kernel with options: a key at a time.  Float16 keys of 128: 2 rows on 48 9.0 / 10.6, on 64 10.5 / 10.4, on 96 14 / 10, on 1000
-	// 130 / 20, 64 on 64 29 / 10; heads of 64 on 64 keys 8.7 / 7.8.  Float32 keys: 2 rows on 96 14.9 / 14.9, of 64 8.7 / 9.8 and on
-	// 128 10.2 / 9.5, 24 on 64 24 / 14.5 and of 64 9.2 / 9.2, 64 on 1000 850 / 54, with a soft cap 20 on 100 35 / 15.
-	inline bool attn_rows_pay_options(size_t rows, size_t keys, size_t heads, bool f32)
-	{
-		return f32 ? keys >= 96 || (keys >= 64 && rows * heads >= 768) : keys >= 64;
-	}
+	// The row kernel with options: fetch::rows_options_tiles (fetch_model.hpp).
 	// The window's row kernel with Float32 keys (a layer of a prompt in both, 2048 wide): 48 and 64 rows on themselves equal, 80 7 to
 	// 13 us apart, 32 four us the other way.
 	inline bool attn_rows_pay_window(size_t rows, size_t keys) { return rows >= 16 && keys > 64; }

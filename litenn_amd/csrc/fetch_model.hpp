@@ -88,6 +88,30 @@ namespace litenn_hip
 			                : rows_time(a, heads, 32, 4, { 64, 123, 31 }) < rows_time(a, heads, 64, 2, { 61, 110, 29 });
 		}
 
+		// Whether a call with options takes the tiles, or the row kernel with options, a key at a time and a workgroup for each row of a
+		// head, whose time grows from some 500 of them on (us of that kernel and of the tiles, 32 heads over 8 unless said).
+		// Float16 keys of 128: 2 rows on 48 9.0 / 10.6, on 64 10.5 / 10.4, on 96 14 / 10, on 1000 130 / 20, 64 on 64 29 / 10; heads of
+		// 64 on 64 keys 8.7 / 7.8; of 72 on 64 9.2 / 10.8, on 80 10.5 / 10.7.  Float32 keys: 2 rows on 96 14.9 / 14.9, of 64 8.5 / 9.1
+		// and on 128 10.1 / 9.1, 24 on 64 24 / 14.5 and of 64 9.2 / 9.2, 64 on 1000 850 / 54, with a soft cap 20 on 100 35 / 15.
+		// Float32 heads of 72 to 112 take the tiles of 128, and five to seven elements a lane in the row kernel: 4 rows of 80 on 96
+		// 8.8 / 14.8, on 200 14.5 / 20.5, on 600 34.3 / 37.3, of 96 on 1000 54.3 / 53.4, 128 heads, 4 rows of 80 on 300 19.7 / 26.4, of 96
+		// 29.8 / 26.1, 8 rows of 80 on 96 14.8 / 13.9, of 96 20.2 / 13.7 and on 64 14.9 / 13.7.  (From 16 rows
+		// on 96 keys on they stay on the tiles, whose error against 64 bits is the smaller one, 1.4e-7 and 1.6.)
+		inline bool rows_options_tiles(size_t rows, size_t keys, size_t heads, size_t dim, bool f32)
+		{
+			const size_t groups = rows * heads;
+			if (dim <= 64 || dim > 112 || (rows >= 16 && keys >= 96))
+			{
+				return f32 ? keys >= 96 || (keys >= 64 && groups >= 768) : keys >= 64;
+			}
+			if (!f32)
+			{
+				return keys >= (groups >= 768 ? 64u : 80u);
+			}
+			const size_t load = dim > 80 ? groups + groups / 2 : groups;
+			return keys >= (load >= 1536 ? 64u : load >= 1024 ? 112u : load > 512 ? 300u : 800u);
+		}
+
 		// ---- products over bfloat16 weights: the K tiles of a group of wavefronts ----------------
 		// K is cut into `ranges` times `groups` parts, in order, that differ by a tile at most; the groups of a
 		// workgroup take neighbouring ones.  They pass one set of barriers, so all of them go through as many

@@ -6,6 +6,7 @@
 #include "common.hpp"
 #include "attn_rows.hpp"
 #include "attn_math.hpp"
+#include "fetch_model.hpp"
 
 #include <algorithm>
 
@@ -809,9 +810,7 @@ namespace litenn_hip
 				}
 				if (x.softcap != 0.0f)
 				{
-					// AddTanh as the layer lowers it (Activation.h:34-50): (exp(2x) - 1) / (exp(2x) + 1)
-					const float ex = expf(__fmul_rn(sc, 2.0f));
-					sc = __fdiv_rn(__fsub_rn(ex, 1.0f), __fadd_rn(ex, 1.0f));
+					sc = capped_tanh(sc);
 					if (x.apply_cap)
 					{
 						sc = __fmul_rn(sc, x.softcap);
@@ -1302,7 +1301,7 @@ namespace litenn_hip
 	                     size_t query_offset, float* out, hipStream_t s)
 	{
 		const double score_scale = logit_softcap != 0.0 ? scale / logit_softcap : scale;
-		if (attn_rows_pay_options(m, keys, n_head, cache_dtype == LITENN_F32))
+		if (fetch::rows_options_tiles(m, keys, n_head, head_dim, cache_dtype == LITENN_F32))
 		{
 			RowsAttn a;
 			a.q = q;

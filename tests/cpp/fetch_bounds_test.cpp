@@ -868,6 +868,37 @@ static void test_rows_forms()
 	}
 }
 
+// Attention with options, a key at a time or tiles, against what a call takes either way (us on the card, no soft cap): never 6 % more
+// than the faster one.
+static void test_options_forms()
+{
+	struct Measured
+	{
+		int rows, keys, heads, dim;
+		bool f32;
+		double row, tiles;
+	};
+	const Measured measured[] = {
+		{ 1, 96, 32, 72, true, 8.7, 14.6 }, { 4, 128, 32, 72, true, 10.4, 14.8 }, { 12, 96, 32, 72, true, 9.1, 13.8 }, { 8, 300, 32, 72, true, 19.4, 25.8 },
+		{ 8, 96, 128, 72, true, 13.6, 13.9 }, { 8, 128, 128, 72, true, 16.6, 13.9 }, { 12, 64, 128, 72, true, 15.0, 14.0 }, { 1, 160, 32, 80, true, 11.9, 20.1 },
+		{ 4, 96, 32, 80, true, 8.8, 14.8 }, { 4, 200, 32, 80, true, 14.5, 20.5 }, { 2, 600, 32, 80, true, 34.1, 37.0 }, { 4, 1000, 32, 80, true, 54.3, 53.8 },
+		{ 4, 300, 128, 80, true, 19.7, 26.4 }, { 4, 96, 128, 80, true, 9.4, 15.0 }, { 8, 64, 128, 80, true, 11.5, 13.9 }, { 8, 112, 128, 80, true, 16.6, 14.0 },
+		{ 1, 112, 32, 96, true, 9.4, 14.6 }, { 2, 1000, 32, 96, true, 55.5, 53.4 }, { 8, 600, 32, 96, true, 33.5, 36.6 }, { 12, 200, 32, 96, true, 17.9, 19.7 },
+		{ 12, 300, 32, 96, true, 24.3, 25.3 }, { 8, 64, 128, 96, true, 14.9, 13.7 }, { 4, 200, 128, 96, true, 21.7, 20.6 }, { 4, 400, 32, 104, true, 23.0, 31.9 },
+		{ 2, 96, 128, 104, true, 8.9, 14.9 }, { 8, 128, 128, 104, true, 23.7, 13.9 }, { 16, 200, 32, 104, true, 19.5, 20.2 }, { 2, 64, 32, 72, false, 9.2, 10.8 },
+		{ 4, 80, 32, 72, false, 10.5, 10.7 }, { 24, 64, 32, 72, false, 10.3, 10.1 }, { 8, 96, 32, 96, false, 12.5, 10.3 }, { 4, 80, 128, 104, false, 12.0, 10.8 },
+		{ 12, 64, 128, 104, false, 21.7, 10.0 }, { 4, 64, 32, 64, true, 7.0, 9.1 }, { 4, 112, 32, 64, true, 9.2, 9.2 }, { 8, 96, 32, 64, true, 8.6, 8.8 },
+		{ 24, 64, 32, 64, true, 9.0, 8.7 }, { 2, 200, 32, 64, true, 13.6, 12.3 }, { 2, 64, 32, 32, true, 7.2, 9.2 }, { 8, 128, 32, 32, true, 10.6, 8.9 },
+		{ 2, 96, 32, 128, true, 14.9, 14.3 }, { 2, 64, 32, 128, true, 11.4, 14.3 }, { 8, 128, 32, 128, true, 18.6, 13.7 }, { 4, 112, 32, 120, true, 16.0, 15.0 },
+		{ 2, 64, 32, 64, false, 8.7, 7.0 }, { 2, 64, 32, 128, false, 10.5, 9.8 }, { 8, 96, 32, 128, false, 13.9, 9.4 }, { 12, 64, 128, 64, false, 16.7, 6.4 },
+	};
+	for (const Measured& p : measured)
+	{
+		const bool tiles = litenn_hip::fetch::rows_options_tiles(p.rows, p.keys, p.heads, p.dim, p.f32);
+		CHECK((tiles ? p.tiles : p.row) <= 1.06 * (p.row < p.tiles ? p.row : p.tiles), "%d rows on %d keys, %d heads of %d: tiles %d", p.rows, p.keys, p.heads, p.dim, tiles);
+	}
+}
+
 // Q6_K with Float32 operands, one tile of activations a wavefront or two, against what a call takes either way (us on the card,
 // weights from HBM): up to 512 tiles never 5 % more than the faster one.
 static void test_exact_forms()
@@ -909,6 +940,7 @@ int main(int argc, char** argv)
 		return 0;
 	}
 	test_rows_forms();
+	test_options_forms();
 	test_exact_forms();
 	test_dense_walks();
 	test_dense_forms();

@@ -88,6 +88,25 @@ def test_options(hip, dtype, m, keys, heads, kv, dim, causal):
 
 
 @pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
+@pytest.mark.parametrize("m,keys,heads,kv,dim", [(4, 79, 8, 8, 72), (4, 80, 8, 4, 80), (1, 130, 32, 8, 112), (4, 799, 4, 2, 104), (4, 800, 4, 2, 104),
+                                                   (8, 111, 64, 8, 96), (15, 299, 36, 4, 88), (15, 300, 36, 4, 88), (16, 96, 4, 4, 80), (12, 64, 128, 8, 96)])
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+def test_options_of_few_rows(hip, dtype, m, keys, heads, kv, dim, softcap):
+    """Heads between 64 and 128, on either side of where the tiles begin."""
+    q, k, v = inputs(4, m, keys, heads, kv, dim, dtype)
+    rng = np.random.default_rng(5)
+    mask = -np.abs(rng.standard_normal((m, keys))).astype(np.float32)
+    mask[:, :20] = -np.inf
+    sinks = rng.standard_normal(heads).astype(np.float32)
+    T = hip.Tensor.from_numpy
+    got = hip.flash_attn_ext(T(q), T(k), T(v), m, keys, heads, kv, dim, scale=dim ** -0.5, logit_softcap=softcap, mask=T(mask),
+                             sinks=T(sinks), causal=True, query_position_offset=keys - m).numpy()
+    want = plain(*(a.astype(np.float64) for a in (q, k, v)), dim ** -0.5, keys - m, sinks=sinks, softcap=softcap,
+                 mask=mask.astype(np.float64), slopes=[1.0] * heads)
+    assert worst(got, want) <= 2e-6
+
+
+@pytest.mark.parametrize("dtype", [DT_F16, DT_F32])
 @pytest.mark.parametrize("m", [7, 40])
 def test_scores_that_saturate_the_soft_cap(hip, dtype, m):
     """Capped scores of 43.7 to 44.3, where exp(2x) comes to the end of its range, beside small ones: tanh is 1, on
