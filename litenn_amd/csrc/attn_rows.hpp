@@ -39,10 +39,7 @@ namespace litenn_hip
 	// (Below some 20000 / sqrt(keys) rows of all heads together its 128-wide form is the faster one, 8 on 128 4.9 / 9.8, 30 on 300
 	// 14.6 / 15.0: it could have a line of its own there, which is not drawn.)
 	inline bool attn_rows_pay_causal(size_t rows, size_t keys, bool f32) { return rows >= (f32 ? 16u : 8u) && keys >= 96; }
-	// The row kernel with options: fetch::rows_options_tiles (fetch_model.hpp).
-	// The window's row kernel with Float32 keys (a layer of a prompt in both, 2048 wide): 48 and 64 rows on themselves equal, 80 7 to
-	// 13 us apart, 32 four us the other way.
-	inline bool attn_rows_pay_window(size_t rows, size_t keys) { return rows >= 16 && keys > 64; }
+	// The row kernel with options and the window's: fetch::rows_options_tiles, rows_window_tiles (fetch_model.hpp).
 
 	// Returns false, launching nothing, for shapes it does not take: head sizes that are no multiple of 8 or above 128,
 	// rows that are not whole 16-byte pieces.

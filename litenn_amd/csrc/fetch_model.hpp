@@ -112,6 +112,17 @@ namespace litenn_hip
 			return keys >= (load >= 1536 ? 64u : load >= 1024 ? 112u : load > 512 ? 300u : 800u);
 		}
 
+		// The same for a window with Float32 keys, a row of which sees `keys`.  A layer of a prompt, 2048 wide, in both: 48 and 64 rows on
+		// themselves equal, 80 7 to 13 us apart, 32 four us the other way.  Below 96 keys heads that leave much of the tiles of 128
+		// empty want some 1400 rows of all heads (the call alone, us of the row kernel and of the tiles, 66 keys): 4 heads of 128 with
+		// values of 64, 64 rows 11.3 / 15.2, 16 heads 13.2 / 15.3, 48 heads, 32 rows 16.3 / 15.3; of 80, 4 heads, 64 rows 13.1 / 15.7,
+		// 16 heads, 80 rows 15.6 / 15.9, 100 17.1 / 15.9; of 128 14.3 / 15.3, 16.4 / 15.5, 22.9 / 15.5; of 64 9.5 / 9.6, 10.4 / 9.7.
+		inline bool rows_window_tiles(size_t rows, size_t keys, size_t heads, size_t dim, size_t vdim)
+		{
+			const bool filled = (dim <= 64 && vdim <= 64) || dim + vdim > 224;
+			return rows >= 16 && keys > 64 && (keys >= 96 || filled || rows * heads >= 1400);
+		}
+
 		// ---- products over bfloat16 weights: the K tiles of a group of wavefronts ----------------
 		// K is cut into `ranges` times `groups` parts, in order, that differ by a tile at most; the groups of a
 		// workgroup take neighbouring ones.  They pass one set of barriers, so all of them go through as many

@@ -5,6 +5,7 @@
 // Norms, positions, scores, softmax and everything inside a recurrence are Float32.  The reference
 // has no counterpart of these layers.
 #include "attn_rows.hpp"
+#include "fetch_model.hpp"
 #include "layer_device.hpp"
 
 #include <algorithm>
@@ -1721,7 +1722,7 @@ namespace litenn_hip
 		const dim3 rows(a.rows, a.shape.heads);
 		if (a.f32)
 		{
-			if (attn_rows_pay_window(a.rows, std::min(a.keys, a.shape.window)))
+			if (fetch::rows_window_tiles(a.rows, std::min(a.keys, a.shape.window), a.shape.heads, a.shape.dim, a.shape.vdim))
 			{
 				RowsAttn r;
 				r.q = a.q;

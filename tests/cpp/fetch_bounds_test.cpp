@@ -897,6 +897,24 @@ static void test_options_forms()
 		const bool tiles = litenn_hip::fetch::rows_options_tiles(p.rows, p.keys, p.heads, p.dim, p.f32);
 		CHECK((tiles ? p.tiles : p.row) <= 1.06 * (p.row < p.tiles ? p.row : p.tiles), "%d rows on %d keys, %d heads of %d: tiles %d", p.rows, p.keys, p.heads, p.dim, tiles);
 	}
+	struct Window
+	{
+		int rows, keys, heads, dim, vdim;
+		double row, tiles;
+	};
+	const Window windows[] = { // (10 %)
+		{ 64, 66, 4, 128, 64, 11.3, 15.2 }, { 16, 80, 16, 128, 64, 11.9, 14.4 }, { 64, 80, 16, 128, 64, 14.0, 15.3 }, { 32, 80, 48, 128, 64, 19.7, 15.3 },
+		{ 48, 80, 48, 128, 64, 25.6, 15.4 }, { 16, 66, 4, 80, 80, 13.1, 14.8 }, { 48, 66, 16, 80, 80, 13.6, 15.9 }, { 80, 80, 16, 80, 80, 16.3, 15.9 },
+		{ 100, 80, 16, 80, 80, 18.2, 15.9 }, { 200, 66, 48, 80, 80, 61.3, 24.5 }, { 64, 66, 4, 128, 128, 14.3, 15.3 }, { 16, 80, 48, 128, 128, 25.2, 14.6 },
+		{ 64, 84, 16, 128, 128, 18.0, 15.5 }, { 20, 66, 48, 64, 64, 10.4, 9.4 }, { 32, 66, 4, 64, 64, 9.4, 9.6 },
+	};
+	for (const Window& p : windows)
+	{
+		const bool tiles = litenn_hip::fetch::rows_window_tiles(p.rows, p.keys, p.heads, p.dim, p.vdim);
+		const double least = p.row < p.tiles ? p.row : p.tiles;
+		CHECK((tiles ? p.tiles : p.row) <= 1.1 * least, "window, %d rows on %d keys, %d heads of %d and %d: tiles %d", p.rows, p.keys, p.heads, p.dim, p.vdim, tiles);
+	}
+	CHECK(!litenn_hip::fetch::rows_window_tiles(15, 500, 16, 128, 128) && !litenn_hip::fetch::rows_window_tiles(500, 64, 16, 128, 128), "few rows or keys");
 }
 
 // Q6_K with Float32 operands, one tile of activations a wavefront or two, against what a call takes either way (us on the card,

@@ -163,7 +163,8 @@ def test_operands_far_below_their_rows_largest(hip, dtype, dim):
     assert error(q, k, v) <= 2e-6
 
 
-@pytest.mark.parametrize("m,keys,heads,dim,vdim,window,at", [(16, 100, 3, 24, 40, 96, 84), (50, 150, 2, 128, 64, 97, 100), (96, 96, 4, 128, 128, 200, 0)])
+@pytest.mark.parametrize("m,keys,heads,dim,vdim,window,at", [(16, 100, 3, 24, 40, 96, 84), (50, 150, 2, 128, 64, 97, 100), (96, 96, 4, 128, 128, 200, 0),
+                                                                 (40, 95, 3, 80, 80, 200, 55), (40, 90, 35, 80, 80, 70, 50), (17, 65, 2, 64, 64, 65, 48)])
 def test_float32_windows(hip, m, keys, heads, dim, vdim, window, at):
     rng = np.random.default_rng(4)
     q = rng.standard_normal((m, heads, dim)).astype(np.float32)
