@@ -995,11 +995,11 @@ namespace litenn_hip
 
 		// The same with less held ahead.  WN > 1: the fragments pass through the same two buffers, two stages on their way; with WN =
 		// 1 nobody shares them and they go to registers directly, each refilled for a later step once it has been used.  Nobody is
-		// waited for there either: a wavefront walks its own range with no branch in a chunk's steps, which the compiler orders as
-		// one run.  With two tiles only two steps' fragments are held (four: 32 more registers, the sums' and scales' loads waited
-		// for in turn).  Q6_K 4096 x 14336, 1000 rows: 630 us with a branch a stage and four steps, 608 with two, 595 without the
-		// branches; 14336 x 4096, 45 rows: 52.1 -> 50.0; one tile (Q4_0, Q8_0): 1 to 4 %.
-		template <typename F, int MT, int WN, int KS>
+		// waited for there either: in one run (ONE_RUN) a wavefront walks its own range with no branch in a chunk's steps, which the
+		// compiler orders as a whole; else stage by stage.  With two tiles only two steps' fragments are held (four: 32 more
+		// registers, the sums' and scales' loads waited for in turn).  Q6_K 4096 x 14336, 1000 rows: 630 us with a branch a stage
+		// and four steps, 608 with two, 595 without the branches; 14336 x 4096, 45 rows: 52.1 -> 50.0; one tile (Q4_0, Q8_0): 1 to 4 %.
+		template <typename F, int MT, int WN, int KS, bool ONE_RUN>
 		__global__ __launch_bounds__(64 * WN * KS) void exact_gemm_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                  const float* residual, int k, int m, int m_tiles,
 		                                                                  int chunks, size_t row_bytes)
@@ -1007,6 +1007,7 @@ namespace litenn_hip
 			constexpr bool kShared = WN > 1;
 			constexpr int kPieces = kShared ? MT * 8 / WN : 1; // 1 KB pieces a wavefront stages
 			static_assert(!kShared || kPieces * WN == MT * 8, "activation pieces / wavefront split");
+			static_assert(kShared ? !ONE_RUN : ONE_RUN || MT == 1, "barriers; a stage held");
 			typedef WeightPieces<F> W;
 			constexpr int kRingBytes = kShared ? KS * 2 * MT * kStageBytes : 0;
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
@@ -1099,11 +1100,11 @@ namespace litenn_hip
 				__syncthreads();
 			}
 			int buffer = 0;
-			const int trips = kShared ? per : c_end - c_begin;
+			const int trips = ONE_RUN ? c_end - c_begin : per;
 			for (int i = 0; i < trips; ++i)
 			{
 				const int c = c_begin + i;
-				const bool live = !kShared || c < c_end; // (uniform: a shorter range only passes the barriers)
+				const bool live = ONE_RUN || c < c_end; // (uniform: a shorter range only passes the barriers)
 				const int next = min(c + 1, c_end - 1);
 				typename F::Head head;
 				floatx16 sum[MT]; // the chunk's, where kScaleSteps is less
@@ -1157,9 +1158,13 @@ namespace litenn_hip
 								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[0], b, fresh ? floatx16{} : p[t], 0, 0, 0);
 								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[1], b_low, p[t], 0, 0, 0);
 							}
-							if constexpr (!kShared)
+							if constexpr (ONE_RUN)
 							{
 								fetch_direct(step + kHeld < 16 ? c : next, ((step + kHeld) & 15) / 4, (s + kHeld) % 4);
+							}
+							else if constexpr (!kShared) // (the next stage's same step, said so: Q4_0 in 164 registers instead of 186)
+							{
+								fetch_direct(st < 3 ? c : next, (st + 1) & 3, s);
 							}
 							if constexpr (F::kMins)
 							{
@@ -1505,7 +1510,7 @@ namespace litenn_hip
 
 		// Four wavefronts over one chunk's scale have the registers to hold two steps' operands (Q4_K 28672 x 4096 at 300 rows 253
 		// -> 238 us); sums that are scaled every step or two have not.
-		template <typename F, int MT, int WN, int KS>
+		template <typename F, int MT, int WN, int KS, bool ONE_RUN>
 		constexpr auto variant()
 		{
 			if constexpr (WN > 1 && F::kMins)
@@ -1514,11 +1519,11 @@ namespace litenn_hip
 			}
 			else
 			{
-				return &exact_gemm_kernel<F, MT, WN, KS>;
+				return &exact_gemm_kernel<F, MT, WN, KS, ONE_RUN>;
 			}
 		}
 
-		template <typename F, int MT, int WN, int KS>
+		template <typename F, int MT, int WN, int KS, bool ONE_RUN = WN == 1>
 		void launch_variant(const ExactCall& c)
 		{
 			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * 2 * MT * kStageBytes : 0) +
@@ -1540,7 +1545,7 @@ namespace litenn_hip
 					blocks += (c.n[i] + WN * kTile - 1) / (WN * kTile);
 				}
 			}
-			const auto kernel = variant<F, MT, WN, KS>();
+			const auto kernel = variant<F, MT, WN, KS, ONE_RUN>();
 			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
 			kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
 			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
@@ -1570,12 +1575,20 @@ namespace litenn_hip
 			// 16 rows 5.8 against 6.0).
 			if (units <= 256 && c.chunks >= 8)
 			{
-				launch_variant<F, 1, 1, 8>(c);
+				return launch_variant<F, 1, 1, 8>(c);
 			}
-			else
+			// Stage by stage where many tiles of activations meet few strips: in one run wavefronts drift apart, and loads of what others
+			// brought into L2 come too late (Q4_0 512 x 8192, 1000 rows: 2.6 and 4.0 million misses).  us of stages and of a run: that
+			// one 78 and 100, Q4_K 1024 x 8192, 777 rows 106 and 129, 2048 x 8192, 640 rows 140 and 164, 4096 x 4096, 300 rows 60 and 59;
+			// the other way round 14336 x 4096, 45 rows 41.6 and 39.9, Q8_0 45.7 and 44.0.
+			if constexpr (F::kScaleSteps > 1)
 			{
-				launch_variant<F, 1, 1, 4>(c);
+				if (units > 256 && 12 * c.m_tiles >= strips)
+				{
+					return launch_variant<F, 1, 1, 4, false>(c);
+				}
 			}
+			launch_variant<F, 1, 1, 4>(c);
 		}
 
 		struct FewCall
