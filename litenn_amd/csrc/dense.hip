@@ -59,6 +59,25 @@ namespace litenn_hip
 			return v;
 		}
 
+		__device__ __forceinline__ floatx4 load_piece(const uint16_t* x, int i, int k)
+		{
+			floatx4 v = { 0.0f, 0.0f, 0.0f, 0.0f };
+			if (i + 3 < k)
+			{
+				const uint2 w = *reinterpret_cast<const uint2*>(x + i);
+				v = floatx4{ bf16_to_f32(w.x & 0xffffu), bf16_to_f32(w.x >> 16), bf16_to_f32(w.y & 0xffffu), bf16_to_f32(w.y >> 16) };
+			}
+			else
+			{
+#pragma unroll
+				for (int e = 0; e < 3; ++e)
+				{
+					v[e] = i + e < k ? bf16_to_f32(x[i + e]) : 0.0f;
+				}
+			}
+			return v;
+		}
+
 		__device__ __forceinline__ float square_sum(const floatx4& v, float acc)
 		{
 			acc = fmaf(v.x, v.x, acc);
@@ -221,6 +240,14 @@ namespace litenn_hip
 				for (int i = k + threadIdx.x; i < 2 * half; i += kRowThreads)
 				{
 					row_lds[row_slot(i, half)] = 0.0f;
+				}
+			}
+			else if (d.x16)
+			{
+#pragma unroll 4
+				for (int p = threadIdx.x; p < pieces; p += kRowThreads)
+				{
+					put(p, load_piece(d.x16, 4 * p, k));
 				}
 			}
 			else

@@ -28,7 +28,7 @@ namespace litenn_hip
 	// ---- one activation row (decode): Float32 activations, weights streamed once ----------------
 	enum DensePrologue
 	{
-		kRowPlain = 0,    // x as it is
+		kRowPlain = 0,    // x (or x16) as it is
 		kRowAddNorm = 1,  // x' = x + norm(sub) sub_w (sub may be null); x' -> x_out if given; norm(x') norm_w, or x' without norm_w
 		kRowHeadGate = 2, // per head of `vdim`: norm(x) norm_w, then times silu(gate)
 	};
@@ -36,6 +36,7 @@ namespace litenn_hip
 	{
 		DenseMatrix w;
 		const float* x = nullptr; // [k]
+		const uint16_t* x16 = nullptr; // [k] bfloat16 in x's place, on 8 bytes, kRowPlain
 		float* y = nullptr;       // [n], or [n / 2] with glu
 		int prologue = kRowPlain;
 		const float* sub = nullptr;

@@ -30,6 +30,7 @@ namespace litenn_hip
 
 		constexpr int kRowsMin = 4;        // from here on a pass runs on the matrix cores
 		constexpr int kExpandMin = 16;     // from here on attention expands the cached latents
+		constexpr int kAttnRows = 64;      // a prompt's queries are taken in tiles of so many: a tile's bits hang on its rows
 		constexpr int kPassRows = 4096;    // most tokens of a pass (LITENN_HIP_PASS_ROWS)
 		constexpr int kAlignRows = 8;      // first row of every part of a concatenated matrix
 
@@ -64,6 +65,7 @@ namespace litenn_hip
 			// norms ahead of the sublayers (null where there are none) and behind them
 			const float *norm1 = nullptr, *norm1b = nullptr, *norm2 = nullptr, *norm2b = nullptr;
 			DenseMatrix in, out; // concatenated input projections, output projection
+			int kept = 0;        // the first of `in`'s rows that make what caches and states hold
 			std::vector<MixerState> mixers;
 			// feed-forward
 			DenseMatrix gate_up, down;
@@ -246,15 +248,18 @@ namespace litenn_hip
 			return s.vector;
 		}
 
-		// weights of one mixer: its input projections join `parts`, its output projection `outs`
-		void build_mixer(const std::string& mix, MixerState& M, std::vector<Part>& parts, std::vector<std::pair<std::string, int>>& outs)
+		// weights of one mixer: its input projections join `parts`, or `kept` where caches and states hold them, its output
+		// projection `outs`
+		void build_mixer(const std::string& mix, MixerState& M, std::vector<Part>& parts, std::vector<Part>& kept,
+		                 std::vector<std::pair<std::string, int>>& outs)
 		{
 			const MixerDesc& m = M.desc;
 			const int values = m.heads * m.vdim, keys = m.heads * m.dim;
 			switch (m.kind)
 			{
 			case MixerKind::LatentAttention: {
-				parts.insert(parts.end(), { { mix + "dq", m.q_rank, &M.at_q }, { mix + "dkv", m.kv_rank, &M.at_latent }, { mix + "g", values, &M.at_gate } });
+				parts.insert(parts.end(), { { mix + "dq", m.q_rank, &M.at_q }, { mix + "g", values, &M.at_gate } });
+				kept.push_back({ mix + "dkv", m.kv_rank, &M.at_latent });
 				M.q_norm = vector(mix + "dq.norm", m.q_rank);
 				M.latent_norm = vector(mix + "dkv.norm", m.kv_rank);
 				M.sink = vector(mix + "sink", m.heads);
@@ -269,17 +274,18 @@ namespace litenn_hip
 				break;
 			}
 			case MixerKind::GatedLinearAttention:
-				parts.insert(parts.end(), { { mix + "q", keys, &M.at_q }, { mix + "k", keys, &M.at_k }, { mix + "v", values, &M.at_v },
-				                            { mix + "g", values, &M.at_gate }, { mix + "a1", m.decay_rank, &M.at_low } });
+				parts.insert(parts.end(), { { mix + "q", keys, &M.at_q }, { mix + "g", values, &M.at_gate } });
+				kept.insert(kept.end(), { { mix + "k", keys, &M.at_k }, { mix + "v", values, &M.at_v }, { mix + "a1", m.decay_rank, &M.at_low } });
 				M.a2 = matrix({ { mix + "a2", keys, nullptr } }, m.decay_rank);
 				M.a2_bias = vector(mix + "a2.b", keys);
 				M.head_norm = vector(mix + "norm", m.vdim);
 				break;
 			case MixerKind::GroupedAttention:
-				parts.insert(parts.end(), { { mix + "q", keys, &M.at_q }, { mix + "k", m.kv_heads * m.dim, &M.at_k } });
+				parts.push_back({ mix + "q", keys, &M.at_q });
+				kept.push_back({ mix + "k", m.kv_heads * m.dim, &M.at_k });
 				if (!m.values_are_keys)
 				{
-					parts.push_back({ mix + "v", m.kv_heads * m.vdim, &M.at_v });
+					kept.push_back({ mix + "v", m.kv_heads * m.vdim, &M.at_v });
 				}
 				if (m.projection_norm)
 				{
@@ -293,7 +299,7 @@ namespace litenn_hip
 				break;
 			case MixerKind::StateSpace: {
 				const int channels = values + 2 * m.groups * m.state;
-				parts.push_back({ mix + "in", values + channels + m.heads, &M.at_in });
+				kept.insert(kept.begin(), { mix + "in", values + channels + m.heads, &M.at_in }); // (gates first)
 				M.conv_w = columns(mix + "conv", channels, m.taps);
 				M.conv_b = vector(mix + "conv.b", channels);
 				M.dt_bias = vector(mix + "dt_bias", m.heads);
@@ -315,7 +321,7 @@ namespace litenn_hip
 			{
 				L.norm1b = vector(p + "norm1b", width);
 			}
-			std::vector<Part> parts;
+			std::vector<Part> parts, kept;
 			std::vector<std::pair<std::string, int>> outs;
 			L.mixers.resize(L.desc.mixers.size()); // before their members' addresses go into `parts`
 			for (size_t i = 0; i < L.mixers.size(); ++i)
@@ -326,9 +332,18 @@ namespace litenn_hip
 				{
 					M.at_mid += before.second;
 				}
-				build_mixer(p + "mix." + M.desc.name, M, parts, outs);
+				build_mixer(p + "mix." + M.desc.name, M, parts, kept, outs);
 			}
+			parts.insert(parts.end(), kept.begin(), kept.end());
 			L.in = matrix(parts, width);
+			L.kept = *kept.front().at;
+			for (const MixerState& M : L.mixers)
+			{
+				if (M.desc.kind == MixerKind::StateSpace && M.at_in == L.kept)
+				{
+					L.kept += M.desc.heads * M.desc.vdim / kAlignRows * kAlignRows; // behind the gates
+				}
+			}
 			for (MixerState& M : L.mixers)
 			{
 				if (M.desc.kind == MixerKind::GroupedAttention && M.desc.values_are_keys)
@@ -761,21 +776,27 @@ namespace litenn_hip
 			launch_mixer_finish(a ? &attn : nullptr, a ? a->desc.weight : 1.0f, a ? row_mid + a->at_mid : nullptr, b ? &norm : nullptr, stream);
 		}
 
-		// the same for a prompt's rows: from proj to mid
-		void mix_rows(const LayerState& L, int rows, int past, const Position& pos)
+		// the same for a prompt's rows: from proj to mid, of rows `first` .. (and of some ahead of them)
+		void mix_rows(const LayerState& L, int rows, int first, int past, const Position& pos)
 		{
+			const size_t operand = f32 ? 4 : 2;
 			for (const MixerState& M : L.mixers)
 			{
-				void* out = static_cast<uint8_t*>(mid) + (f32 ? 4 : 2) * static_cast<size_t>(M.at_mid);
+				uint8_t* out = static_cast<uint8_t*>(mid) + operand * static_cast<size_t>(M.at_mid);
 				if (M.desc.kind == MixerKind::GroupedAttention)
 				{
 					GroupedAttn a = grouped_args(M);
 					a.rows = rows;
 					a.pos = pos;
+					a.q_from = first;
 					launch_grouped_append(a, stream);
 					WindowAttn w = grouped_window(a, past);
+					const int from = first / kAttnRows * kAttnRows;
+					w.q += static_cast<size_t>(from) * w.ldq;
+					w.q_base += from;
+					w.rows -= from;
 					w.out_scale = M.desc.weight;
-					w.out = out;
+					w.out = out + operand * static_cast<size_t>(from) * ld_mid;
 					w.ldo = ld_mid;
 					launch_window_attn(w, stream);
 				}
@@ -784,61 +805,88 @@ namespace litenn_hip
 					Ssm a = ssm_args(M);
 					a.rows = rows;
 					a.pos = pos;
+					a.out_from = first;
 					launch_ssm_rows(a, stream);
 					GatedNorm g = gated_norm_args(M);
-					g.y = a.in;
+					g.y = a.in + static_cast<size_t>(first) * ld_proj;
 					g.ldy = ld_proj;
-					g.out = out;
+					g.out = out + operand * static_cast<size_t>(first) * ld_mid;
 					g.ldo = ld_mid;
-					g.rows = rows;
+					g.rows = rows - first;
 					g.f32 = f32;
 					launch_gated_norm(g, stream);
 				}
 			}
 		}
 
+		// A row on its way through the layers: x is the residual stream, `pending` the norm weight of the sublayer output in
+		// y that is still to be added to it.
+		struct OneRow
+		{
+			LayeredModel& m;
+			const float* x;
+			int spare; // of xt: takes the next sum
+			const float* pending = nullptr;
+
+			// norm(x + norm(y)) norm_w through `w`
+			void enter(const DenseMatrix& w, const float* norm_w, float* dst, bool glu = false, const ClampedGlu& act = ClampedGlu{}, float softcap = 0.0f)
+			{
+				DenseRow r;
+				r.w = w;
+				r.x = x;
+				r.y = dst;
+				r.softcap = softcap;
+				r.prologue = pending || norm_w ? kRowAddNorm : kRowPlain;
+				r.norm_w = norm_w;
+				r.eps = m.desc.eps;
+				r.glu = glu;
+				r.act = act;
+				if (pending)
+				{
+					r.sub = m.y;
+					r.sub_w = pending;
+					r.x_out = m.xt[spare];
+				}
+				launch_dense_row(r, m.stream);
+				if (pending)
+				{
+					x = m.xt[spare];
+					spare ^= 1;
+				}
+				pending = nullptr;
+			}
+			void leave(const DenseMatrix& w, const float* src, const float* after, const uint16_t* src16 = nullptr)
+			{
+				DenseRow r;
+				r.w = w;
+				r.x = src;
+				r.x16 = src16;
+				r.y = m.y;
+				launch_dense_row(r, m.stream);
+				pending = after;
+			}
+			void feed_forward(const LayerState& L)
+			{
+				if (L.desc.ff > 0)
+				{
+					enter(L.gate_up, L.norm2, m.row_mid, true, L.desc.act);
+					leave(L.down, m.row_mid, L.norm2b);
+				}
+			}
+			void logits(float* out) { enter(m.head, m.final_norm, out, false, ClampedGlu{}, m.desc.logit_softcap); }
+		};
+
 		// the token at position counters[0] + offset; logits to `out` unless null
 		void forward_token(const int32_t* id, int offset, float* out)
 		{
 			const Position pos{ d_counters, offset };
 			launch_embed_rows(embed, id, 1, turns, pos, xt[0], d_err, stream);
-			int at = 0;                // xt[at] is the residual stream, `pending` still to be added
-			const float* pending = nullptr; // norm weight of the sublayer output in y
-			// norm(x + norm(y)) norm_w through `w`
-			const auto enter = [&](const DenseMatrix& w, const float* norm_w, float* dst, bool glu, const ClampedGlu& act, float softcap = 0.0f) {
-				DenseRow r;
-				r.w = w;
-				r.x = xt[at];
-				r.y = dst;
-				r.softcap = softcap;
-				r.prologue = pending || norm_w ? kRowAddNorm : kRowPlain;
-				r.norm_w = norm_w;
-				r.eps = desc.eps;
-				r.glu = glu;
-				r.act = act;
-				if (pending)
-				{
-					r.sub = y;
-					r.sub_w = pending;
-					r.x_out = xt[at ^ 1];
-				}
-				launch_dense_row(r, stream);
-				at ^= pending ? 1 : 0;
-				pending = nullptr;
-			};
-			const auto leave = [&](const DenseMatrix& w, const float* src, const float* after) {
-				DenseRow r;
-				r.w = w;
-				r.x = src;
-				r.y = y;
-				launch_dense_row(r, stream);
-				pending = after;
-			};
+			OneRow row{ *this, xt[0], 1 };
 			for (LayerState& L : layers)
 			{
 				const MixerState& M = L.mixers[0];
 				const MixerDesc& m = M.desc;
-				enter(L.in, L.norm1, proj, false, ClampedGlu{});
+				row.enter(L.in, L.norm1, proj);
 				if (m.kind == MixerKind::LatentAttention)
 				{
 					DenseRow r;
@@ -871,7 +919,7 @@ namespace litenn_hip
 					a.partial = partial;
 					a.splits = M.splits;
 					launch_latent_step(a, stream);
-					leave(L.out, row_mid, L.norm1b);
+					row.leave(L.out, row_mid, L.norm1b);
 				}
 				else if (m.kind == MixerKind::GatedLinearAttention)
 				{
@@ -888,22 +936,18 @@ namespace litenn_hip
 					r.vdim = m.vdim;
 					r.eps = desc.eps;
 					launch_dense_row(r, stream);
-					pending = L.norm1b;
+					row.pending = L.norm1b;
 				}
 				else
 				{
 					mix_token(L, pos);
-					leave(L.out, row_mid, L.norm1b);
+					row.leave(L.out, row_mid, L.norm1b);
 				}
-				if (L.desc.ff > 0)
-				{
-					enter(L.gate_up, L.norm2, row_mid, true, L.desc.act);
-					leave(L.down, row_mid, L.norm2b);
-				}
+				row.feed_forward(L);
 			}
 			if (out)
 			{
-				enter(head, final_norm, out, false, ClampedGlu{}, desc.logit_softcap);
+				row.logits(out);
 			}
 		}
 
@@ -972,19 +1016,52 @@ namespace litenn_hip
 				launch_dense_rows(d, stream);
 				pending = after;
 			};
+			const auto operand_row = [&](void* p, int row, int ld) { return static_cast<uint8_t*>(p) + static_cast<size_t>(row) * ld * (f32 ? 4 : 2); };
 			for (LayerState& L : layers)
 			{
 				const MixerState& M = L.mixers[0];
+				// Nothing reads what the last layer makes of a row whose logits are not asked for, but for keys, values and states:
+				// n rows alone, from `first` on, have queries and gates and go on behind the mixer, one row as a step's row does.  us
+				// with every row's queries and attention and one row in the prompt's tiles, against this: 2048 tokens of two
+				// 4096-wide Kulurax layers 1729 -> 1499, 40 tokens 432 -> 404; 777 tokens of three 2048-wide Degedra layers 776 ->
+				// 729, 500 of two in 32 bits 577 -> 531, 16 of two 1024-wide ones 219 -> 207.  (Of a whole model's layers that is a few
+				// percent.)  The row's error against 64 bits falls by 10 to 30 %: its operands are not rounded.
+				const int n = &L == &layers.back() ? logit_rows : rows, first = rows - n;
+				const bool one = n == 1;
+				// (attention in 32 bits takes a few rows the slower the fewer they are, and looks at what comes out of all of them)
+				const int asked = f32 ? first / kAttnRows * kAttnRows : first;
 				enter(L.norm1, 0, rows);
-				product(L.in, h, ld_h, rows, proj, ld_proj, kOutF32);
+				OneRow row{ *this, x + static_cast<size_t>(first) * desc.width, 0 };
+				if (asked > 0)
+				{
+					DenseMatrix ahead = L.in, kept = L.in;
+					ahead.n = L.kept;
+					kept.n -= L.kept;
+					kept.w += static_cast<size_t>(L.kept) * kept.pitch;
+					product(kept, h, ld_h, rows, proj + L.kept, ld_proj, kOutF32);
+					float* const to = proj + static_cast<size_t>(asked) * ld_proj;
+					if (rows - asked == 1)
+					{
+						row.enter(ahead, L.norm1, to);
+					}
+					else
+					{
+						product(ahead, operand_row(h, asked, ld_h), ld_h, rows - asked, to, ld_proj, kOutF32);
+					}
+				}
+				else
+				{
+					product(L.in, h, ld_h, rows, proj, ld_proj, kOutF32);
+				}
 				if (M.desc.kind == MixerKind::LatentAttention)
 				{
-					attend(M, rows, past, pos);
+					attend(M, rows, asked, past, pos);
 				}
 				else if (M.desc.kind == MixerKind::GatedLinearAttention)
 				{
 					Gla g = gla_args(M);
 					g.rows = rows;
+					g.out_from = asked;
 					g.out = mid;
 					g.ldo = ld_mid;
 					g.f32 = f32;
@@ -994,12 +1071,17 @@ namespace litenn_hip
 				}
 				else
 				{
-					mix_rows(L, rows, past, pos);
+					mix_rows(L, rows, asked, past, pos);
 				}
-				// Behind the last layer's states nothing reads a row whose logits are not asked for: it goes on with the others
-				// alone.  (2048 tokens of two 4096-wide layers 2361 -> 1708 us; of a whole model's layers that is a few percent.)
-				const int n = &L == &layers.back() ? logit_rows : rows, first = rows - n;
-				leave(L.out, static_cast<const char*>(mid) + static_cast<size_t>(first) * ld_mid * (f32 ? 4 : 2), L.norm1b, first, n);
+				if (one)
+				{
+					const void* const from = operand_row(mid, first, ld_mid);
+					row.leave(L.out, static_cast<const float*>(f32 ? from : nullptr), L.norm1b, static_cast<const uint16_t*>(f32 ? nullptr : from));
+					row.feed_forward(L);
+					row.logits(logits);
+					return;
+				}
+				leave(L.out, operand_row(mid, first, ld_mid), L.norm1b, first, n);
 				if (L.desc.ff > 0)
 				{
 					enter(L.norm2, first, n);
@@ -1020,21 +1102,39 @@ namespace litenn_hip
 			launch_dense_rows(d, stream);
 		}
 
-		void attend(const MixerState& M, int rows, int past, const Position& pos)
+		// queries of rows `first` .. (and some ahead of them), keys of all rows
+		void attend(const MixerState& M, int rows, int first, int past, const Position& pos)
 		{
 			const MixerDesc& m = M.desc;
-			AddNorm n; // queries' latent
-			n.x = proj + M.at_q;
-			n.ldx = ld_proj;
-			n.norm_w = M.q_norm;
-			n.out = mid;
-			n.ldo = ld_mid;
-			n.rows = rows;
-			n.width = m.q_rank;
-			n.eps = desc.eps;
-			n.f32 = f32;
-			launch_add_norm(n, stream);
-			product(M.uq, mid, ld_mid, rows, q, ld_q, kOutF32);
+			const size_t operand = f32 ? 4 : 2;
+			const auto queries = [&](int from) { return q + static_cast<size_t>(from) * ld_q; };
+			const auto columns_of = [&](int from, int at) { return proj + static_cast<size_t>(from) * ld_proj + at; };
+			if (rows - first == 1)
+			{
+				DenseRow r;
+				r.w = M.uq;
+				r.x = columns_of(first, M.at_q);
+				r.y = queries(first);
+				r.prologue = kRowAddNorm;
+				r.norm_w = M.q_norm;
+				r.eps = desc.eps;
+				launch_dense_row(r, stream);
+			}
+			else
+			{
+				AddNorm n; // queries' latent
+				n.x = columns_of(first, M.at_q);
+				n.ldx = ld_proj;
+				n.norm_w = M.q_norm;
+				n.out = mid;
+				n.ldo = ld_mid;
+				n.rows = rows - first;
+				n.width = m.q_rank;
+				n.eps = desc.eps;
+				n.f32 = f32;
+				launch_add_norm(n, stream);
+				product(M.uq, mid, ld_mid, rows - first, queries(first), ld_q, kOutF32);
+			}
 			launch_latent_append(proj + M.at_latent, ld_proj, M.latent_norm, desc.eps, rows, pos, M.cache, stream);
 			if (rows < kExpandMin)
 			{
@@ -1043,22 +1143,25 @@ namespace litenn_hip
 				a.cache = M.cache;
 				a.uk = M.uk;
 				a.uv = M.uv;
-				a.q = q;
+				a.q = queries(first);
 				a.ldq = ld_q;
-				a.gate = proj + M.at_gate;
+				a.gate = columns_of(first, M.at_gate);
 				a.ldg = ld_proj;
-				a.out = mid;
+				a.out = static_cast<uint8_t*>(mid) + operand * static_cast<size_t>(first) * ld_mid;
 				a.ldo = ld_mid;
 				a.out_f32 = f32;
-				a.rows = rows;
+				a.rows = rows - first;
 				a.pos = pos;
+				a.pos.add += first;
 				a.absorbed = absorbed;
 				a.partial = partial;
-				a.splits = latent_step_splits(m.heads, rows, m.window);
+				a.splits = latent_step_splits(m.heads, a.rows, m.window);
 				launch_latent_step(a, stream);
 				return;
 			}
-			const int base = std::max(0, past - m.window + 1);
+			// the keys that a query of the tiles sees
+			const int from = first / kAttnRows * kAttnRows;
+			const int base = std::max(0, past + from - m.window + 1);
 			const int keys = past + rows - base;
 			DenseRows d;
 			d.w = M.ukv;
@@ -1074,7 +1177,7 @@ namespace litenn_hip
 			launch_dense_rows(d, stream);
 			WindowAttn w;
 			w.shape = latent_shape(M);
-			w.q = q;
+			w.q = queries(from);
 			w.ldq = ld_q;
 			w.kv = kv;
 			w.ldkv = ld_kv;
@@ -1083,11 +1186,11 @@ namespace litenn_hip
 			w.v_head = static_cast<size_t>(m.vdim);
 			w.keys = keys;
 			w.key_base = base;
-			w.rows = rows;
-			w.q_base = past;
-			w.gate = proj + M.at_gate;
+			w.rows = rows - from;
+			w.q_base = past + from;
+			w.gate = columns_of(from, M.at_gate);
 			w.ldg = ld_proj;
-			w.out = mid;
+			w.out = static_cast<uint8_t*>(mid) + operand * static_cast<size_t>(from) * ld_mid;
 			w.ldo = ld_mid;
 			w.f32 = f32;
 			launch_window_attn(w, stream);

@@ -1264,7 +1264,7 @@ namespace litenn_hip
 			float(*const ls)[kSlabStride] = ks + kChunk; // log decays summed from the block's first token
 			float(*const totals)[kSlab] = reinterpret_cast<float(*)[kSlab]>(lds + 3 * kChunk * kSlabStride); // a block's whole sum
 			const int dim = a.shape.dim, vdim = a.shape.vdim, pitch = gla_state_pitch(vdim), heads = a.shape.heads;
-			const int h = blockIdx.x, chunk = blockIdx.y;
+			const int h = blockIdx.x, chunk = static_cast<int>(blockIdx.y) + a.out_from / kChunk;
 			const int row0 = chunk * kChunk, count = min(kChunk, a.rows - row0);
 			const int lane = threadIdx.x & 63;
 			const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1600,13 +1600,18 @@ namespace litenn_hip
 			gla_state_kernel<NC><<<dim3(a.shape.heads * slabs, chunks), dim3(256 * NC), 0, s>>>(a);
 			const int quads = a.shape.heads * a.shape.dim * (gla_state_pitch(a.shape.vdim) >> 2);
 			gla_scan_kernel<<<dim3((quads + 255) / 256), dim3(256), 0, s>>>(a, chunks);
+			if (a.out_from >= a.rows)
+			{
+				return;
+			}
+			const dim3 grid(a.shape.heads, chunks - a.out_from / kChunk);
 			if (a.f32)
 			{
-				gla_out_kernel<NC, float><<<dim3(a.shape.heads, chunks), dim3(256 * NC), 0, s>>>(a);
+				gla_out_kernel<NC, float><<<grid, dim3(256 * NC), 0, s>>>(a);
 			}
 			else
 			{
-				gla_out_kernel<NC, uint16_t><<<dim3(a.shape.heads, chunks), dim3(256 * NC), 0, s>>>(a);
+				gla_out_kernel<NC, uint16_t><<<grid, dim3(256 * NC), 0, s>>>(a);
 			}
 		}
 

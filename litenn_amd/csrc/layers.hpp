@@ -133,6 +133,7 @@ namespace litenn_hip
 		void* out = nullptr;
 		int ldo = 0;
 		bool f32 = false;
+		int out_from = 0;              // the first row whose output is asked for (some rows ahead of it may be written too)
 		float* log_decay = nullptr;    // scratch [rows, heads dim]
 		float* chunk_states = nullptr; // scratch: gla_chunk_floats()
 	};
@@ -181,6 +182,7 @@ namespace litenn_hip
 		// many rows
 		float* q_out = nullptr;    // [rows, ldq]
 		int ldq = 0;
+		int q_from = 0;            // the first row whose query is asked for
 		// one row
 		float* partial = nullptr;  // scratch: grouped_step_partial_floats()
 		int splits = 1;
@@ -208,7 +210,8 @@ namespace litenn_hip
 		Position pos;
 		// one row: y [heads vdim]
 		float* y = nullptr;
-		// many rows: y silu(z) takes the place of z
+		// many rows: y silu(z) takes the place of z, from row out_from on (in some rows ahead of it too)
+		int out_from = 0;
 		float* xbc = nullptr;          // scratch [rows, ssm_ldx()]
 		float* steps = nullptr;        // scratch [2, rows, heads]: dt, then log decays in units of log 2
 		float* chunk_states = nullptr; // scratch: ssm_chunk_floats()

@@ -116,13 +116,15 @@ namespace litenn_hip
 			const int k_at = (q_cols + 3) & ~3, half = a.rot.dims >> 1;
 			float* q_out = a.q_out + static_cast<size_t>(row) * a.ldq;
 			T* rows = static_cast<T*>(c.rows) + static_cast<size_t>(position % c.ring) * c.row_pitch();
+			const bool asked = row >= a.q_from;
 			if constexpr (KEPT > 0)
 			{
 				floatx4 x[KEPT], w[KEPT];
 #pragma unroll
 				for (int i = 0; i < KEPT; ++i)
 				{
-					x[i] = load_either(q, q_cols, k, k_cols, 4 * (tid + 256 * i));
+					const int e = 4 * (tid + 256 * i);
+					x[i] = asked || e >= k_at ? load_either(q, q_cols, k, k_cols, e) : floatx4{ 0.0f, 0.0f, 0.0f, 0.0f };
 				}
 #pragma unroll
 				for (int i = 0; i < KEPT; ++i)
@@ -156,7 +158,7 @@ namespace litenn_hip
 						}
 						return x0 * scale;
 					};
-					for (int e = 4 * tid; e < q_cols; e += 1024)
+					for (int e = 4 * tid; asked && e < q_cols; e += 1024)
 					{
 						const int d = e % c.dim;
 						*reinterpret_cast<floatx4*>(q_out + e) = turned(e - d, d, q_scale);
@@ -169,7 +171,7 @@ namespace litenn_hip
 				}
 				else
 				{
-					for (int e = tid; e < q_cols; e += 256)
+					for (int e = tid; asked && e < q_cols; e += 256)
 					{
 						const int d = e % c.dim;
 						q_out[e] = rotated(lds, nullptr, q_scale, e - d, d, a.rot, cs, sn);
@@ -184,10 +186,10 @@ namespace litenn_hip
 			else
 			{
 				rotary_angles(a.rot, position, cs, sn);
-				const float q_scale = projection_scale(q, a.q_norm, q_cols, a.eps, red);
+				const float q_scale = asked ? projection_scale(q, a.q_norm, q_cols, a.eps, red) : 0.0f; // (uniform)
 				const float k_scale = projection_scale(k, a.k_norm, k_cols, a.eps, red);
 				__syncthreads();
-				for (int e = tid; e < q_cols; e += 256)
+				for (int e = tid; asked && e < q_cols; e += 256)
 				{
 					const int d = e % c.dim;
 					q_out[e] = rotated(q, a.q_norm, q_scale, e - d, d, a.rot, cs, sn);
@@ -1142,7 +1144,7 @@ namespace litenn_hip
 			__shared__ float dts[kChunk];
 			const int pitch = ssm_state_pitch(a.vdim), ldx = a.ldx(), vdim = a.vdim;
 			const int h = static_cast<int>(blockIdx.x) % a.heads, v0 = static_cast<int>(blockIdx.x) / a.heads * kSlice;
-			const int chunk = blockIdx.y, row0 = chunk * kChunk, count = min(kChunk, a.rows - row0);
+			const int chunk = static_cast<int>(blockIdx.y) + a.out_from / kChunk, row0 = chunk * kChunk, count = min(kChunk, a.rows - row0);
 			const int lane = threadIdx.x & 63;
 			const int block = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 			const int j = lane & 15, g = lane >> 4;
@@ -1414,7 +1416,10 @@ namespace litenn_hip
 		const int scan_blocks = (a.heads * a.state * (ssm_state_pitch(a.vdim) >> 2) + 255) / 256;
 		const int ring_blocks = (std::min(a.rows, a.taps) * a.channels() + 255) / 256;
 		ssm_scan_kernel<<<dim3(scan_blocks + ring_blocks), dim3(256), 0, s>>>(a, chunks, scan_blocks);
-		ssm_out_kernel<<<dim3(a.heads * slices, chunks), dim3(256), 0, s>>>(a);
+		if (a.out_from < a.rows)
+		{
+			ssm_out_kernel<<<dim3(a.heads * slices, chunks - a.out_from / kChunk), dim3(256), 0, s>>>(a);
+		}
 	}
 
 	void launch_gated_norm(const GatedNorm& a, hipStream_t s)
