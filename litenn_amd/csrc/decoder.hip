@@ -4,6 +4,7 @@
 #include "decoder.hpp"
 
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 
@@ -18,22 +19,36 @@ namespace litenn_hip
 	{
 		// counters[0] = past length, counters[1] = tokens emitted so far, counters[2] = steps this model
 		// has run (never reset: it names a step in the values its workgroups hand to each other), counters[3] = workgroups of the
-		// arg-max that have arrived (0 between launches)
-		__global__ void set_counters_kernel(int* counters, int past, int emitted)
+		// arg-max that have arrived (0 between launches); n ids from `from`, which may be pinned memory of the host
+		__global__ __launch_bounds__(256) void begin_pass_kernel(int* counters, int past, int emitted, const int32_t* __restrict__ from, int32_t* __restrict__ ids, int n)
 		{
-			counters[0] = past;
-			counters[1] = emitted;
-			counters[2] += 1;
+			const int i = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+			if (i < n)
+			{
+				ids[i] = from[i];
+			}
+			if (i == 0)
+			{
+				counters[0] = past;
+				counters[1] = emitted;
+				counters[2] += 1;
+			}
 		}
 
 		constexpr int kWaitRanOut = -2;
+
+		constexpr size_t kPinnedWords = size_t{ 1 } << 18; // and the error word behind them
+		constexpr size_t kPinnedIds = size_t{ 1 } << 16;   // and a run's ids behind that, where it has no more
+		constexpr size_t kMostDeliverers = 256;            // and a word for each workgroup that delivers
+		constexpr size_t kPinnedIdsAt = kPinnedWords + 4, kPinnedDoneAt = kPinnedIdsAt + kPinnedIds;
 
 		// What a pass leaves for the host goes to pinned memory from the device itself, the error word with it: n words from `from`
 		// to `to`, sixteen bytes a thread where both allow.  A copy to memory that is not pinned waits for the pass, stages and
 		// waits again: ten small launches and 32000 logits 136 us with two such copies, 57 this way (the host's own copy is 1 of them).
 		// (A run too long for the pinned memory, whose own length is what counts, is copied.)
+		// The pass's last launch also has every workgroup write `pass` behind what it delivered: see wait_for_pass.
 		__global__ __launch_bounds__(256) void deliver_kernel(const uint32_t* __restrict__ from, uint32_t* __restrict__ to, size_t n, size_t quads,
-		                                                      const int* __restrict__ err, int* __restrict__ err_to)
+		                                                      const int* __restrict__ err, int* __restrict__ err_to, uint32_t* __restrict__ done, uint32_t pass)
 		{
 			const size_t at = blockIdx.x * size_t{ 256 } + threadIdx.x, threads = gridDim.x * size_t{ 256 };
 			for (size_t i = at; i < quads; i += threads)
@@ -48,18 +63,78 @@ namespace litenn_hip
 			{
 				*err_to = *err;
 			}
+			if (done)
+			{
+				__threadfence_system(); // every thread's own words are there
+				__syncthreads();
+				if (threadIdx.x == 0)
+				{
+					__hip_atomic_store(done + blockIdx.x, pass, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+				}
+			}
 		}
 
-		constexpr size_t kPinnedWords = size_t{ 1 } << 18; // and the error word behind them
-
-		// words [first, first + n) of the pinned memory from `from` (null: none), the error word last of all
+		// words [first, first + n) of the pinned memory from `from` (null: none), the error word and the marks of the pass last of all
 		void deliver(litenn_hip_model* m, const void* from, size_t first, size_t n, bool last)
 		{
 			uint32_t* const to = m->pinned + first;
 			const bool wide = ((reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(to)) & 15u) == 0;
-			const size_t quads = wide ? n / 4 : 0, blocks = ((wide ? quads : n) + 255) / 256;
-			deliver_kernel<<<dim3(static_cast<unsigned>(std::max<size_t>(1, std::min<size_t>(blocks, 256)))), dim3(256), 0, m->stream>>>(
-			    static_cast<const uint32_t*>(from), to, n, quads, m->d_err, last ? reinterpret_cast<int*>(m->pinned + kPinnedWords) : nullptr);
+			const size_t quads = wide ? n / 4 : 0, wanted = ((wide ? quads : n) + 255) / 256;
+			const size_t blocks = std::max<size_t>(1, std::min<size_t>(wanted, kMostDeliverers));
+			if (last)
+			{
+				m->passes += 1;
+				m->deliverers = static_cast<int>(blocks);
+			}
+			deliver_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, m->stream>>>(
+			    static_cast<const uint32_t*>(from), to, n, quads, m->d_err, last ? reinterpret_cast<int*>(m->pinned + kPinnedWords) : nullptr,
+			    last ? m->pinned + kPinnedDoneAt : nullptr, m->passes);
+		}
+
+		// Waits until the pass's last launch has delivered.  The runtime's own wait sleeps until an interrupt, which costs a pass
+		// some 10 us (four empty launches and the wait 17.7 us, with a look at the marks in its place 14.2, twelve 65 and 37; 16 tokens of a
+		// 1024-wide LLaMA block 87 -> 74, of two Degedra layers 204 -> 185), so the host
+		// looks at the marks itself for as long as a pass of a few layers or tokens may take, and sleeps only then.
+		hipError_t wait_for_pass(litenn_hip_model* m)
+		{
+			const uint32_t* const done = m->pinned + kPinnedDoneAt;
+			const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+			for (int block = 0, looks = 0; block < m->deliverers;)
+			{
+				if (__atomic_load_n(done + block, __ATOMIC_ACQUIRE) == m->passes)
+				{
+					++block;
+				}
+				else if ((++looks & 63) == 0 && std::chrono::steady_clock::now() > until)
+				{
+					return hipStreamSynchronize(m->stream); // (which also reports what went wrong)
+				}
+			}
+			return hipSuccess;
+		}
+
+		// The ids of a pass, tokens first .. first + count of a run of `rows` that begins behind `past`, and its counters, in one
+		// launch out of pinned memory: a copy from memory that is not pinned is staged and costs the host as much as two launches
+		// (16 prompt tokens 90 -> 87 us).  Each pass of a run has its own place there, and a run is waited for before the next one.
+		hipError_t begin_pass(litenn_hip_model* m, const int32_t* tokens, size_t rows, size_t first, size_t count, int past)
+		{
+			const bool through_pinned = m->pinned && rows <= kPinnedIds;
+			if (through_pinned)
+			{
+				std::memcpy(m->pinned + kPinnedIdsAt + first, tokens + first, sizeof(int32_t) * count);
+			}
+			else
+			{
+				const hipError_t e = hipMemcpyAsync(m->d_tokens, tokens + first, sizeof(int32_t) * count, hipMemcpyHostToDevice, m->stream);
+				if (e != hipSuccess)
+				{
+					return e;
+				}
+			}
+			const int n = through_pinned ? static_cast<int>(count) : 0;
+			begin_pass_kernel<<<dim3(static_cast<unsigned>(std::max(1, (n + 255) / 256))), dim3(256), 0, m->stream>>>(
+			    m->d_counters, past, 0, through_pinned ? reinterpret_cast<const int32_t*>(m->pinned + kPinnedIdsAt + first) : nullptr, m->d_tokens, n);
+			return hipSuccess;
 		}
 
 		// Waits for the pass and looks at its error word, which was delivered or is copied here.
@@ -70,7 +145,7 @@ namespace litenn_hip
 			{
 				LITENN_HIP_TRY(m->action, hipMemcpyAsync(&flag, m->d_err, sizeof(int), hipMemcpyDeviceToHost, m->stream));
 			}
-			LITENN_HIP_TRY(m->action, hipStreamSynchronize(m->stream));
+			LITENN_HIP_TRY(m->action, delivered ? wait_for_pass(m) : hipStreamSynchronize(m->stream));
 			if (delivered)
 			{
 				std::memcpy(&flag, m->pinned + kPinnedWords, sizeof(int));
@@ -165,10 +240,14 @@ namespace litenn_hip
 		{
 			return e;
 		}
-		if (hipHostMalloc(reinterpret_cast<void**>(&m->pinned), sizeof(uint32_t) * (kPinnedWords + 1), hipHostMallocDefault) != hipSuccess)
+		if (hipHostMalloc(reinterpret_cast<void**>(&m->pinned), sizeof(uint32_t) * (kPinnedDoneAt + kMostDeliverers), hipHostMallocDefault) != hipSuccess)
 		{
 			(void)hipGetLastError();
 			m->pinned = nullptr; // results are copied, then
+		}
+		else
+		{
+			std::memset(m->pinned + kPinnedDoneAt, 0, sizeof(uint32_t) * kMostDeliverers); // no pass has the number 0 (but one in 2^32)
 		}
 		return hipMalloc(&m->argmax_scratch, argmax_step_scratch_bytes(static_cast<size_t>(m->vocab)));
 	}
@@ -258,9 +337,7 @@ namespace litenn_hip
 			for (int attempt = 0;; ++attempt)
 			{
 				m->state_lost = m->stateful(); // until the pass is known to have run
-				LITENN_HIP_TRY(m->action, hipMemcpyAsync(m->d_tokens, tokens + first, sizeof(int32_t) * count,
-				                                         hipMemcpyHostToDevice, s));
-				set_counters_kernel<<<1, 1, 0, s>>>(m->d_counters, m->past, 0);
+				LITENN_HIP_TRY(m->action, begin_pass(m, tokens, rows, first, count, m->past));
 				m->forward(m->d_tokens, count, logit_rows, flags, m->past);
 				LITENN_HIP_TRY(m->action, hipGetLastError());
 				const bool wants_last = last_logits && first + count == rows;
@@ -404,8 +481,7 @@ namespace litenn_hip
 		{
 			const size_t count = std::min(pass, n_prompt - first);
 			const int past = m->past + static_cast<int>(first);
-			GEN_TRY(hipMemcpyAsync(m->d_tokens, prompt + first, sizeof(int32_t) * count, hipMemcpyHostToDevice, s));
-			set_counters_kernel<<<1, 1, 0, s>>>(m->d_counters, past, 0);
+			GEN_TRY(begin_pass(m, prompt, n_prompt, first, count, past));
 			if (first == 0)
 			{
 				GEN_TRY(hipEventRecord(ev[0], s)); // the first pass's ids are on their way: the clock starts here

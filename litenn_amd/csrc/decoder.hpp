@@ -30,6 +30,8 @@ struct litenn_hip_model
 	int* d_counters = nullptr;      // {past, emitted, steps run}
 	int* d_err = nullptr;
 	uint32_t* pinned = nullptr;     // host memory that a pass's results go to (null: there was none to be had)
+	uint32_t passes = 0;            // delivered so far, by so many workgroups the last time
+	int deliverers = 0;
 	std::vector<void*> owned;       // device buffers freed with the model
 	int past = 0;
 	bool state_lost = false;        // a pass failed half-way through a state that cannot be rolled back

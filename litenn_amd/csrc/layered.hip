@@ -91,6 +91,8 @@ namespace litenn_hip
 		std::vector<LayerState> layers;
 		std::map<std::string, Slot> slots;
 		int max_pass = kPassRows;
+		float* states = nullptr; // of all recurrences
+		size_t state_total = 0;  // floats
 
 		// scratch for cap_rows tokens
 		size_t cap_rows = 0;
@@ -383,7 +385,7 @@ namespace litenn_hip
 				M.splits = latent_step_splits(m.heads, 1, m.window);
 				break;
 			case MixerKind::GatedLinearAttention:
-				M.state = static_cast<float*>(allocate(sizeof(float) * state_floats(m)));
+				state_total += state_floats(m);
 				break;
 			case MixerKind::GroupedAttention:
 				M.heads.ring = ring;
@@ -395,7 +397,7 @@ namespace litenn_hip
 				M.splits = grouped_step_splits(m.heads, m.kv_heads, m.dim, m.vdim, m.window);
 				break;
 			case MixerKind::StateSpace:
-				M.state = static_cast<float*>(allocate(sizeof(float) * state_floats(m)));
+				state_total += state_floats(m);
 				M.ring = static_cast<float*>(allocate(sizeof(float) * m.taps * static_cast<size_t>(ssm_args(M).channels())));
 				break;
 			}
@@ -448,6 +450,20 @@ namespace litenn_hip
 				}
 				widest_mid = std::max({ widest_mid, mid_cols, L.desc.ff });
 				proj_cols = std::max(proj_cols, L.in.n);
+			}
+			// the states side by side, so that one launch clears them
+			states = state_total > 0 ? static_cast<float*>(allocate(sizeof(float) * state_total)) : nullptr;
+			float* state = states;
+			for (LayerState& L : layers)
+			{
+				for (MixerState& M : L.mixers)
+				{
+					if (M.desc.kind == MixerKind::GatedLinearAttention || M.desc.kind == MixerKind::StateSpace)
+					{
+						M.state = state;
+						state += state_floats(M.desc);
+					}
+				}
 			}
 			const auto up4 = [](int n) { return (n + 3) & ~3; };
 			ld_proj = up4(proj_cols);
@@ -620,15 +636,10 @@ namespace litenn_hip
 
 		int reset_state() override
 		{
-			for (const LayerState& L : layers)
+			constexpr size_t kMost = size_t{ 1 } << 30; // words of a launch
+			for (size_t at = 0; at < state_total; at += kMost)
 			{
-				for (const MixerState& M : L.mixers)
-				{
-					if (M.state)
-					{
-						launch_zero_ints(reinterpret_cast<int*>(M.state), state_floats(M.desc), stream);
-					}
-				}
+				launch_zero_ints(reinterpret_cast<int*>(states + at), std::min(kMost, state_total - at), stream);
 			}
 			LITENN_HIP_TRY(action, hipGetLastError());
 			return 0;
