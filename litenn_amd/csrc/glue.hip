@@ -159,7 +159,7 @@ namespace litenn_hip
 		template <typename KV>
 		__global__ void rope_qkv_append_kernel(float* __restrict__ q, const float* __restrict__ k,
 		                                       const float* __restrict__ v, KV* __restrict__ kcache,
-		                                       KV* __restrict__ vcache, const int* __restrict__ past_dev, int m,
+		                                       KV* __restrict__ vcache, const int* __restrict__ past_dev, int m, int q_from,
 		                                       int n_head, int n_kv_head, int head_dim, int rope_dims,
 		                                       const float* __restrict__ cos_t, const float* __restrict__ sin_t)
 		{
@@ -182,7 +182,7 @@ namespace litenn_hip
 			if (h < n_head)
 			{
 				float* base = q + (static_cast<size_t>(row) * n_head + h) * head_dim + 2 * p;
-				if (2 * p < rope_dims)
+				if (2 * p < rope_dims && row >= q_from)
 				{
 					float o0, o1;
 					rotate(base[0], base[1], cos_t[static_cast<size_t>(pos) * half + p],
@@ -222,7 +222,7 @@ namespace litenn_hip
 		__global__ __launch_bounds__(256) void rope_qkv_append_quads_kernel(float* __restrict__ q, const float* __restrict__ k,
 		                                                                     const float* __restrict__ v, KV* __restrict__ kcache,
 		                                                                     KV* __restrict__ vcache, const int* __restrict__ past_dev,
-		                                                                     uint32_t q_width, uint32_t kv_width, uint32_t head_dim,
+		                                                                     uint32_t q_from, uint32_t q_width, uint32_t kv_width, uint32_t head_dim,
 		                                                                     uint32_t rope_dims, const float* __restrict__ cos_t,
 		                                                                     const float* __restrict__ sin_t)
 		{
@@ -236,6 +236,10 @@ namespace litenn_hip
 			const size_t row = blockIdx.y;
 			const size_t pos = static_cast<size_t>(*past_dev) + row;
 			const bool is_q = at < q_width, is_v = at >= q_width + kv_width;
+			if (is_q && blockIdx.y < q_from)
+			{
+				return;
+			}
 			const uint32_t in = is_q ? at : at - q_width - (is_v ? kv_width : 0);
 			const float* const src = is_q ? q + row * q_width + in : (is_v ? v : k) + row * kv_width + in;
 			float4_a4 x = *reinterpret_cast<const float4_a4*>(src);
@@ -1083,8 +1087,9 @@ namespace litenn_hip
 		}
 	}
 
+	// queries of rows q_from .. m - 1, keys and values of all m
 	void launch_rope_qkv_append(float* q, const float* k, const float* v, void* kcache, void* vcache, int cache_dtype,
-	                            const int* past_dev, size_t m, size_t n_head, size_t n_kv_head, size_t head_dim,
+	                            const int* past_dev, size_t m, size_t q_from, size_t n_head, size_t n_kv_head, size_t head_dim,
 	                            size_t rope_dims, const float* cos_t, const float* sin_t, hipStream_t s)
 	{
 		const size_t width = (n_head + 2 * n_kv_head) * head_dim;
@@ -1093,7 +1098,7 @@ namespace litenn_hip
 			const auto launch = [&](auto* kc, auto* vc) {
 				typedef std::remove_pointer_t<decltype(kc)> KV;
 				rope_qkv_append_quads_kernel<KV><<<dim3(static_cast<unsigned>((width / 4 + 255) / 256), static_cast<unsigned>(m)), dim3(256), 0, s>>>(
-				    q, k, v, kc, vc, past_dev, static_cast<uint32_t>(n_head * head_dim), static_cast<uint32_t>(n_kv_head * head_dim),
+				    q, k, v, kc, vc, past_dev, static_cast<uint32_t>(q_from), static_cast<uint32_t>(n_head * head_dim), static_cast<uint32_t>(n_kv_head * head_dim),
 				    static_cast<uint32_t>(head_dim), static_cast<uint32_t>(rope_dims), cos_t, sin_t);
 			};
 			if (cache_dtype == LITENN_F16)
@@ -1111,14 +1116,14 @@ namespace litenn_hip
 		if (cache_dtype == LITENN_F16)
 		{
 			rope_qkv_append_kernel<uint16_t><<<grid, block, 0, s>>>(
-			    q, k, v, static_cast<uint16_t*>(kcache), static_cast<uint16_t*>(vcache), past_dev, static_cast<int>(m),
+			    q, k, v, static_cast<uint16_t*>(kcache), static_cast<uint16_t*>(vcache), past_dev, static_cast<int>(m), static_cast<int>(q_from),
 			    static_cast<int>(n_head), static_cast<int>(n_kv_head), static_cast<int>(head_dim),
 			    static_cast<int>(rope_dims), cos_t, sin_t);
 		}
 		else
 		{
 			rope_qkv_append_kernel<float><<<grid, block, 0, s>>>(
-			    q, k, v, static_cast<float*>(kcache), static_cast<float*>(vcache), past_dev, static_cast<int>(m),
+			    q, k, v, static_cast<float*>(kcache), static_cast<float*>(vcache), past_dev, static_cast<int>(m), static_cast<int>(q_from),
 			    static_cast<int>(n_head), static_cast<int>(n_kv_head), static_cast<int>(head_dim),
 			    static_cast<int>(rope_dims), cos_t, sin_t);
 		}

@@ -58,7 +58,7 @@ namespace litenn_hip
 	                       float* out, int* err_flag, hipStream_t stream);
 	void launch_rmsnorm(const float* x, const float* w, double eps, size_t m, size_t d, float* y, hipStream_t s);
 	void launch_rope_qkv_append(float* q, const float* k, const float* v, void* kcache, void* vcache, int cache_dtype,
-	                            const int* past_dev, size_t m, size_t n_head, size_t n_kv_head, size_t head_dim,
+	                            const int* past_dev, size_t m, size_t q_from, size_t n_head, size_t n_kv_head, size_t head_dim,
 	                            size_t rope_dims, const float* cos_t, const float* sin_t, hipStream_t s);
 	bool attn_step_fusable(const float* q, const float* k, const float* v, const void* kcache, const void* vcache,
 	                       size_t head_dim, size_t rope_dims, const float* cos_t, const float* sin_t);
@@ -243,6 +243,16 @@ namespace
 	constexpr size_t kGemmMinRows = 4;
 	// From this many rows on the prompt's attention runs tiled on the matrix cores.
 	constexpr size_t kAttnTileMinRows = 16;
+
+	// Whether the one row that goes on behind the last block's keys and values has its query made alone: a launch more (5 to 8 us
+	// where the others are short) against the other rows' queries, 2 rows d width operations.  us of a block's whole pass, all
+	// queries and one, Float32 operands: 4096 wide, 130 rows 141 and 128, 300 rows 166 and 151; 2048 wide, 300 rows 106 and 107, 112 and 105
+	// in Q8_0; rounded ones: 4096 wide, 250 rows 140 and 143, 300 rows 135 and 134, 152 and 133, 600 rows 166 and 152; 2048 wide,
+	// 1400 rows 152 and 131.
+	bool own_query(size_t rows, size_t d, size_t width, bool rounded)
+	{
+		return rows >= kGemmMinRows && rows * d * width >= (rounded ? size_t{ 1 } << 32 : size_t{ 100 } << 24);
+	}
 
 	bool is_quantised(const Weight& w) { return w.fmt != LITENN_FMT_F16 && w.fmt != LITENN_FMT_F32; }
 
@@ -536,7 +546,7 @@ namespace
 			}
 			else
 			{
-				launch_rope_qkv_append(m->q, m->k, m->v, L.kcache, L.vcache, m->p.kv_dtype, past_dev, 1, H, KH, hd,
+				launch_rope_qkv_append(m->q, m->k, m->v, L.kcache, L.vcache, m->p.kv_dtype, past_dev, 1, 0, H, KH, hd,
 				                       rope_dims, m->cos_t, m->sin_t, s);
 				launch_attn_decode(m->q, L.kcache, L.vcache, m->p.kv_dtype, 1, past_dev, 0, H, KH, hd, m->attn,
 				                   m->attn_splits, m->attn_partial, m->attn_counters, s);
@@ -566,20 +576,34 @@ namespace
 		launch_get_rows_q(m->tok_embd.fmt, m->tok_embd.data, m->tok_embd.n, d, ids, rows, m->x, m->d_err, s);
 		for (Layer& L : m->layers)
 		{
+			// Behind the last block's keys and values nothing reads a row whose logits are not asked for: n rows go on, one row as a
+			// step's row does, from its query on.  (A prompt that wants one row's logits saves most of one block: 300 tokens of two
+			// 8B-shape blocks, Float32 operands, 1246 -> 776 us; with the query of that row
+			// alone 735 -> 716, 2048 tokens of three 7B-shape blocks in two portions 2860 -> 2726; of a whole model's 32 blocks that is some
+			// 2 to 3 %.)
+			const size_t n = &L == &m->layers.back() && d % 4 == 0 ? logit_rows : rows, behind = rows - n; // (rows on 16 bytes)
+			float* const q = m->q + behind * H * hd;
+			float* const x = m->x + behind * d;
 			const Weight* qkv[3] = { &L.wq, &L.wk, &L.wv };
 			float* qkv_out[3] = { m->q, m->k, m->v };
+			const bool own = n == 1 && own_query(rows, d, H * hd, !(flags & LITENN_HIP_MATMUL_PRECISE));
+			const int from = own ? 1 : 0;
+			if (own)
+			{
+				group(m, 1, qkv, &q, x, nullptr, L.attn_norm, false, s);
+			}
 			// consecutive projections of one format share a launch (and its fused norm), and so do q and
 			// k in Q4_K or Q5_K beside a Q6_K v
 			const int qkv_fmt[3] = { L.wq.fmt, L.wk.fmt, L.wv.fmt };
 			const void* qkv_w[3] = { L.wq.data, L.wk.data, L.wv.data };
 			const size_t qkv_n[3] = { L.wq.n, L.wk.n, L.wv.n };
-			const bool mixed = L.wq.fmt != L.wk.fmt || L.wk.fmt != L.wv.fmt;
+			const bool mixed = qkv_fmt[from] != L.wk.fmt || L.wk.fmt != L.wv.fmt;
 			const bool one_launch = mixed && rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE) &&
-			                        L.wq.k == L.wk.k && L.wk.k == L.wv.k &&
-			                        launch_gemm_group_mixed(qkv_fmt, 3, qkv_w, qkv_n, L.wq.k, m->x, rows, qkv_out, L.attn_norm,
-			                                                m->p.rms_norm_epsilon, m->xh, m->xh_halves, s);
+			                        qkv[from]->k == L.wk.k && L.wk.k == L.wv.k &&
+			                        launch_gemm_group_mixed(qkv_fmt + from, 3 - from, qkv_w + from, qkv_n + from, L.wk.k, m->x, rows,
+			                                                qkv_out + from, L.attn_norm, m->p.rms_norm_epsilon, m->xh, m->xh_halves, s);
 			const bool exact = rows >= kGemmMinRows && (flags & LITENN_HIP_MATMUL_PRECISE); // (formats do not matter to its rows)
-			for (int i = 0; i < 3 && !one_launch;)
+			for (int i = from; i < 3 && !one_launch;)
 			{
 				int j = i + 1;
 				while (j < 3 && (exact || qkv[j]->fmt == qkv[i]->fmt) && qkv[j]->k == qkv[i]->k)
@@ -590,14 +614,8 @@ namespace
 				             flags, s);
 				i = j;
 			}
-			launch_rope_qkv_append(m->q, m->k, m->v, L.kcache, L.vcache, m->p.kv_dtype, past_dev, rows, H, KH, hd,
+			launch_rope_qkv_append(m->q, m->k, m->v, L.kcache, L.vcache, m->p.kv_dtype, past_dev, rows, behind, H, KH, hd,
 			                       m->p.rope_dimension_count, m->cos_t, m->sin_t, s);
-			// Behind the last block's keys and values nothing reads a row whose logits are not asked for: it goes on with the
-			// others alone.  (A prompt that wants one row's logits saves most of one block: 300 tokens of two 8B-shape blocks, Float32
-			// operands, 1246 -> 776 us; of a whole model's 32 blocks that is some 2 %.)
-			const size_t n = &L == &m->layers.back() && d % 4 == 0 ? logit_rows : rows, behind = rows - n; // (rows on 16 bytes)
-			const float* const q = m->q + behind * H * hd;
-			float* const x = m->x + behind * d;
 			// a prompt's rows go through the matrix cores (fp16 operands) unless f32 operands are asked for
 			if (n < kAttnTileMinRows || (flags & LITENN_HIP_MATMUL_PRECISE) ||
 			    !launch_attn_tile(q, L.kcache, L.vcache, m->p.kv_dtype, n, attn_past_dev, attn_past + behind, H, KH, hd, m->attn, s))
