@@ -571,16 +571,16 @@ namespace litenn_hip
 			}
 		}
 
-		// A wavefront's share of the weights on their way: the raw blocks of 32 rows for one chunk, from memory (where
+		// A wavefront's share of the weights on their way: the raw blocks of 32 (or 16) rows for one chunk, from memory (where
 		// they lie on 2 bytes) to the wavefront's slot in LDS (where a row's chunk begins on 16).  The P pieces of a row fall
 		// into groups of 16, 8, 4, 2 and 1 (the bits of P); a load takes one group of as many rows as there are lanes for, so
 		// that a lane's place in the row stays the same from load to load and its addresses are one sum.  Nothing behind
 		// the matrix is fetched: rows behind the last are the last, and a row's chunk that is not whole comes element
 		// by element, its missing part being the row's last two bytes.
-		template <typename F>
+		template <typename F, int ROWS = kTile>
 		struct WeightPieces
 		{
-			static constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>(), kRows = kTile;
+			static constexpr int P = slot_pieces<F>(), kStride = slot_stride<F>(), kRows = ROWS;
 			static constexpr int loads_of(int width) { return (P & width) != 0 ? (kRows * width + 63) / 64 : 0; }
 			static constexpr int kLoads = loads_of(16) + loads_of(8) + loads_of(4) + loads_of(2) + loads_of(1);
 			static constexpr int kSlotBytes = kRows * kStride;
@@ -640,7 +640,7 @@ namespace litenn_hip
 				each(lane, [&](int i, int row, int piece) { *reinterpret_cast<u32x4*>(slot + row * kStride + 16 * piece) = moving[i]; });
 			}
 			// the lane's row in the slot
-			__device__ __forceinline__ lds_bytes_t chunk(int lane) const { return (lds_bytes_t)(slot) + (lane & 31) * kStride; }
+			__device__ __forceinline__ lds_bytes_t chunk(int lane) const { return (lds_bytes_t)(slot) + (lane & (kRows - 1)) * kStride; }
 		};
 
 		// What of the product a workgroup and its wavefront take, and the way out of their sums: shared by both forms below.
@@ -1247,14 +1247,16 @@ namespace litenn_hip
 		}
 
 		// ---- few rows: up to MR activation rows, one launch, no scratch ---------------------------------
-		// A workgroup takes 32 weight rows; its KS wavefronts take ranges of K and meet in LDS at the end.  Each takes
+		// A workgroup takes 16 weight rows; its KS wavefronts take ranges of K and meet in LDS at the end.  Each takes
 		// the activations apart by itself, a chunk of 256 at a time and with a power of two per chunk and row: a
 		// lane holds four neighbouring elements of every row, and the parts go to fragments in the wavefront's LDS.
-		// Rows 0 .. MR - 1 of a fragment are the high parts, 16 .. 16 + MR - 1 the low ones, so that one product forms both;
-		// their sums lie in one lane (elements e and e + 8 of the result).  Bound by a wavefront's chain per chunk (blocks
-		// and activations into LDS, 16 products); a row more costs its preparation, 32 instructions.  us against the streaming
-		// kernel once per row: Q8_0 4096 x 4096 at 3 rows 10.9 / 18.2, Q4_K 14336 x 4096 at 4 rows 15.8 / 31.1, Q6_K 4096 x
-		// 14336 at 7 rows 33 / 90.
+		// v_mfma_f32_16x16x32_f16 (16x16x16 where every 16 elements have a scale) with the activations as A, the high parts of row
+		// i as its row i, the low ones as row 8 + i: lane (r, g) = (lane % 16, lane / 16) holds weight row r's results of
+		// activation rows 4 (g % 2) .., the high parts' where g < 2 and the low ones' else, which are summed apart and meet at the end.
+		// Bound by a wavefront's chain per chunk (blocks and activations into LDS, 8 products, 16 in Q6_K); a row more costs its
+		// preparation, 32 instructions.  us against 32 weight rows a workgroup (below), which leave half the card idle here: Q8_0
+		// 4096 x 4096 at 3 rows 10.4 -> 7.9, Q4_K 8.3 -> 6.9, Q6_K 4096 x 14336 at 2 rows 22.4 -> 15.0, at 8 rows 32.6 -> 24.5.  Error
+		// against 64 bits up to 8 % lower.
 		template <int MR>
 		struct FewRows
 		{
@@ -1263,48 +1265,43 @@ namespace litenn_hip
 			static constexpr int kUnused = kSums + 2 * kPart; // what lanes with nothing to write write
 			static constexpr int kBytes = kUnused + 256;
 		};
-
-		template <typename F, int MR, int KS>
-		__global__ __launch_bounds__(64 * KS, 2) void exact_few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, float* y,
-		                                                            const float* residual, int n, int k, int m, int chunks, size_t row_bytes)
+		// A range's activations on their way into fragments in the wavefront's LDS
+		template <typename F, int MR>
+		struct FewActivations
 		{
 			typedef FewRows<MR> R;
-			typedef WeightPieces<F> W;
-			constexpr int NE = 4; // results of a lane
-			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][slot, fragments]; later the KS sums
-			const int lane = threadIdx.x & 63;
-			const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-			const int r = lane & 31, h = lane >> 5;
-			const int n_base = blockIdx.x * kTile;
-			const int per = (chunks + KS - 1) / KS;
-			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
-			uint8_t* const mine = lds + part * (W::kSlotBytes + R::kBytes);
-			uint8_t* const frags = mine + W::kSlotBytes;
-			const W weights(mine, w, n_base, n, row_bytes);
-
-			// (nothing here may hang on a branch or look at what it loads: the next chunk's loads would be waited for at once)
 			floatx4 xv[MR];
 			const float* rows[MR];
-#pragma unroll
-			for (int i = 0; i < MR; ++i)
+			float unscale[MR];
+			uint8_t* frags;
+			uint8_t* frag_to;
+			int lane, k, sum_at, sum_row, sum_low;
+
+			__device__ __forceinline__ FewActivations(const float* x, int m, int k_, uint8_t* frags_, int lane_) : frags(frags_), lane(lane_), k(k_)
 			{
-				rows[i] = x + static_cast<size_t>(min(i, m - 1)) * k;
+#pragma unroll
+				for (int i = 0; i < MR; ++i)
+				{
+					rows[i] = x + static_cast<size_t>(min(i, m - 1)) * k;
+				}
+				// lane l holds elements 4 l .. 4 l + 3: group of eight l / 2, its first or second four
+				frag_to = frags + (lane >> 1) * R::kHalf + (lane & 1) * 8;
+				// the sub-block sum of lanes 8 j .. 8 j + 7 is lane 8 j's to write, the others' go nowhere
+				sum_at = (lane & 7) == 0 ? R::kSums + (lane >> 3) * 2 : R::kUnused + lane * 4;
+				sum_row = (lane & 7) == 0 ? 16 : 0, sum_low = (lane & 7) == 0 ? R::kPart : 2;
 			}
-			const auto request_x = [&](int c) {
+			// (nothing here may hang on a branch or look at what it loads: the next chunk's loads would be waited for at once)
+			__device__ __forceinline__ void request(int c)
+			{
 				const int at = min(c * kChunk + 4 * lane, k - 4);
 #pragma unroll
 				for (int i = 0; i < MR; ++i)
 				{
 					xv[i] = *reinterpret_cast<const floatx4_a4*>(rows[i] + at);
 				}
-			};
-			float unscale[MR];
-			// lane l holds elements 4 l .. 4 l + 3: step l / 4, half l / 2 % 2, first or second four of its eight
-			uint8_t* const frag_to = frags + (lane >> 1) * R::kHalf + (lane & 1) * 8;
-			// the sub-block sum of lanes 8 j .. 8 j + 7 is lane 8 j's to write, the others' go nowhere
-			const int sum_at = (lane & 7) == 0 ? R::kSums + (lane >> 3) * 2 : R::kUnused + lane * 4;
-			const int sum_row = (lane & 7) == 0 ? 16 : 0, sum_low = (lane & 7) == 0 ? R::kPart : 2;
-			const auto deposit_x = [&](int c) {
+			}
+			__device__ __forceinline__ void deposit(int c)
+			{
 				const bool there = F::kBlock == kChunk || c * kChunk + 4 * lane < k;
 #pragma unroll
 				for (int i = 0; i < MR; ++i)
@@ -1345,7 +1342,322 @@ namespace litenn_hip
 						*reinterpret_cast<_Float16*>(frags + sum_at + sum_row * i + sum_low) = static_cast<_Float16>(fmaxf((s - static_cast<float>(high)) * (1.0f / kLowScale), -32768.0f));
 					}
 				}
+			}
+		};
+
+		constexpr int kFewTile = 16; // weight rows of a workgroup
+
+		// What lane (r, g) multiplies of weight row r: of step s = 2 st + u elements 32 s + 8 g .. + 7, or, where kStep is 16, of step s
+		// = 4 st + u elements 16 s + 4 g .. + 3.  `chunk` is the row's in the slot; st one of four stages of 64 elements.
+		template <typename F>
+		struct FewWeights;
+
+		template <>
+		struct FewWeights<Q4_0X>
+		{
+			static constexpr int kStep = 32;
+			struct Head {};
+			struct Raw { u32x2 q[2]; uint32_t d[2]; };
+			static __device__ __forceinline__ Head head(lds_bytes_t, int) { return {}; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int g, int blocks)
+			{
+				Raw r;
+#pragma unroll
+				for (int u = 0; u < 2; ++u)
+				{
+					const int block = 2 * st + u;
+					const uint32_t d = load2(chunk + 18 * block); // (there, whatever it is: not a branch)
+					r.d[u] = block < blocks ? d : 0u;
+					r.q[u] = load8(chunk + 8 * (g & 1), 18 * block + 2);
+				}
+				return r;
+			}
+			static __device__ __forceinline__ half8 frag(const Head&, const Raw& r, int, int u, int g)
+			{
+				const int sh = 4 * (g >> 1);
+				return bytes_minus((r.q[u].x >> sh) & 0x0f0f0f0fu, (r.q[u].y >> sh) & 0x0f0f0f0fu, 8.0f);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw& r, int, int u) { return f16_bits_to_f32(r.d[u]); }
+			static __device__ __forceinline__ float chunk_scale(const Head&) { return 1.0f; }
+		};
+
+		template <>
+		struct FewWeights<Q8_0X>
+		{
+			static constexpr int kStep = 32;
+			struct Head {};
+			struct Raw { u32x2 q[2]; uint32_t d[2]; };
+			static __device__ __forceinline__ Head head(lds_bytes_t, int) { return {}; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int g, int blocks)
+			{
+				Raw r;
+#pragma unroll
+				for (int u = 0; u < 2; ++u)
+				{
+					const int block = 2 * st + u;
+					const uint32_t d = load2(chunk + 34 * block); // (there, whatever it is: not a branch)
+					r.d[u] = block < blocks ? d : 0u;
+					r.q[u] = load8(chunk + 8 * g, 34 * block + 2);
+				}
+				return r;
+			}
+			static __device__ __forceinline__ half8 frag(const Head&, const Raw& r, int, int u, int)
+			{
+				return bytes_minus(r.q[u].x ^ 0x80808080u, r.q[u].y ^ 0x80808080u, 128.0f);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw& r, int, int u) { return f16_bits_to_f32(r.d[u]); }
+			static __device__ __forceinline__ float chunk_scale(const Head&) { return 1.0f; }
+		};
+
+		template <>
+		struct FewWeights<Q4_KX>
+		{
+			static constexpr int kStep = 32;
+			typedef Q4_KX::Head Head;
+			struct Raw { u32x2 q; };
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return { load16(chunk) }; }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int g, int) { return { load8(chunk + 8 * g, 16 + 32 * st) }; }
+			static __device__ __forceinline__ half8 frag(const Head& hd, const Raw& r, int st, int u, int)
+			{
+				const int sh = 4 * u, sub = 2 * st + u;
+				const uint32_t s = (Q4_KX::scales(hd.w, sub >> 2) >> (8 * (sub & 3))) & 0xffu;
+				return bytes_times((r.q.x >> sh) & 0x0f0f0f0fu, (r.q.y >> sh) & 0x0f0f0f0fu, s, Q4_KX::kCentre);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
+			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return Q4_KX::chunk_scale(hd); }
+		};
+
+		template <>
+		struct FewWeights<Q5_KX>
+		{
+			static constexpr int kStep = 32;
+			typedef Q5_KX::Head Head;
+			struct Raw { u32x2 q; };
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int g)
+			{
+				const u32x2 fifth = load8(chunk + 8 * g, 16);
+				return { load16(chunk), { fifth, fifth } };
+			}
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int g, int) { return { load8(chunk + 8 * g, 48 + 32 * st) }; }
+			static __device__ __forceinline__ half8 frag(const Head& hd, const Raw& r, int st, int u, int)
+			{
+				const int sh = 4 * u, sub = 2 * st + u;
+				const uint32_t s = (Q4_KX::scales(hd.w, sub >> 2) >> (8 * (sub & 3))) & 0xffu;
+				const u32x2 f = hd.fifth[0]; // bit `sub` of a byte is its element's fifth bit
+				return bytes_times(((r.q.x >> sh) & 0x0f0f0f0fu) | (((f.x >> sub) & 0x01010101u) << 4),
+				                   ((r.q.y >> sh) & 0x0f0f0f0fu) | (((f.y >> sub) & 0x01010101u) << 4), s, Q5_KX::kCentre);
+			}
+			static __device__ __forceinline__ float scale(const Head&, const Raw&, int, int) { return 1.0f; }
+			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return Q5_KX::chunk_scale(hd); }
+		};
+
+		template <>
+		struct FewWeights<Q6_KX>
+		{
+			static constexpr int kStep = 16;
+			typedef Q6_KX::Head Head;
+			struct Raw { uint32_t low[2][2], high[2]; }; // half st / 2 of the block: [32 x (first, second)][16-element run]
+			static __device__ __forceinline__ Head head(lds_bytes_t chunk, int) { return Q6_KX::head(chunk, 0); }
+			static __device__ __forceinline__ Raw load(lds_bytes_t chunk, int st, int g, int)
+			{
+				typedef const __attribute__((address_space(3))) uint32_t* words_t;
+				const words_t low = (words_t)(chunk + 64 * (st >> 1) + 4 * g), high = (words_t)(chunk + 128 + 32 * (st >> 1) + 4 * g);
+				return { { { low[0], low[4] }, { low[8], low[12] } }, { high[0], high[4] } };
+			}
+			// quarter i = 2 (st % 2) + u / 2 of the half, elements 16 (u % 2) + 4 g .. of its 32
+			static __device__ __forceinline__ half4 frag(const Head&, const Raw& r, int st, int u, int)
+			{
+				const int sh = 4 * (st & 1), top = 2 * (2 * (st & 1) + (u >> 1));
+				const uint32_t v = ((r.low[u >> 1][u & 1] >> sh) & 0x0f0f0f0fu) | (((r.high[u & 1] >> top) & 0x03030303u) << 4);
+				const _Float16 m = static_cast<_Float16>(-1024.0f - 32.0f);
+				const half2v a = biased01(v) + half2v{ m, m }, b = biased23(v) + half2v{ m, m };
+				return half4{ a.x, a.y, b.x, b.y };
+			}
+			static __device__ __forceinline__ float scale(const Head& hd, const Raw& r, int st, int u) { return Q6_KX::scale(hd, {}, st, u); }
+			static __device__ __forceinline__ float chunk_scale(const Head& hd) { return Q6_KX::chunk_scale(hd); }
+		};
+
+		template <typename F, int MR, int KS>
+		__global__ __launch_bounds__(64 * KS, 2) void exact_few_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, float* y,
+		                                                            const float* residual, int n, int k, int m, int chunks, size_t row_bytes)
+		{
+			typedef FewRows<MR> R;
+			typedef FewWeights<F> D;
+			typedef WeightPieces<F, kFewTile> W;
+			constexpr int NE = 4; // results of a lane
+			constexpr int kSteps = 64 / D::kStep; // of a stage
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][slot, fragments]; later the KS sums
+			const int lane = threadIdx.x & 63;
+			const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int r = lane & 15, g = lane >> 4;
+			const int n_base = blockIdx.x * kFewTile;
+			const int per = (chunks + KS - 1) / KS;
+			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
+			uint8_t* const mine = lds + part * (W::kSlotBytes + R::kBytes);
+			uint8_t* const frags = mine + W::kSlotBytes;
+			const W weights(mine, w, n_base, n, row_bytes);
+
+			FewActivations<F, MR> xs(x, m, k, frags, lane);
+			// A's row r: high parts of activation row r, low ones of row r - 8 (rows that are not there repeat the last)
+			const uint8_t* const frag_row = frags + (r >> 3) * R::kPart + min(r & 7, m - 1) * 16;
+			const uint8_t* const frag_from = D::kStep == 32 ? frag_row + g * R::kHalf : frag_row + (g >> 1) * R::kHalf + (g & 1) * 8;
+			const uint8_t* const sums_from = frags + R::kSums + (r >> 3) * R::kPart + min(r & 7, m - 1) * 16;
+
+			float acc[2][NE] = {}; // of every other chunk
+			u32x4 moving[2][W::kLoads]; // the next two chunks
+			if (c_begin < c_end)
+			{
+				weights.request(moving[0], c_begin, lane);
+				xs.request(c_begin);
+				weights.request(moving[1], min(c_begin + 1, c_end - 1), lane);
+			}
+			const auto step = [&](int c, u32x4 (&arrived)[W::kLoads], float (&acc)[NE]) {
+				weights.deposit(arrived, lane);
+				xs.deposit(c);
+				xs.request(min(c + 1, c_end - 1));
+				weights.request(arrived, min(c + 2, c_end - 1), lane);
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
+				const int blocks = k / F::kBlock - c * (kChunk / F::kBlock);
+				lds_bytes_t const chunk = weights.chunk(lane);
+				const typename D::Head head = D::head(chunk, g);
+				floatx4 stage, sum[2]; // sum: of the chunk's halves (two shorter chains round less)
+#pragma unroll
+				for (int st = 0; st < 4; ++st)
+				{
+					const typename D::Raw raw = D::load(chunk, st, g, blocks);
+					floatx4& half = sum[st >> 1];
+#pragma unroll
+					for (int u = 0; u < kSteps; ++u)
+					{
+						const int at = kSteps * st + u;
+						floatx4 p;
+						if constexpr (D::kStep == 32)
+						{
+							const half8 a = *reinterpret_cast<const half8*>(frag_from + 4 * at * R::kHalf);
+							p = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, D::frag(head, raw, st, u, g), floatx4{}, 0, 0, 0);
+						}
+						else
+						{
+							const half4 a = *reinterpret_cast<const half4*>(frag_from + 2 * at * R::kHalf);
+							p = __builtin_amdgcn_mfma_f32_16x16x16f16(a, D::frag(head, raw, st, u, g), floatx4{}, 0, 0, 0);
+						}
+						if constexpr (F::kMins)
+						{
+							stage = u == 0 ? p : stage + p;
+							if (u == kSteps - 1)
+							{
+								half = (st & 1) == 0 ? stage : half + stage;
+							}
+						}
+						else
+						{
+							const float d = D::scale(head, raw, st, u);
+#pragma unroll
+							for (int e = 0; e < NE; ++e)
+							{
+								half[e] = (st & 1) == 0 && u == 0 ? d * p[e] : fmaf(d, p[e], half[e]);
+							}
+						}
+					}
+				}
+				const float d = D::chunk_scale(head);
+				floatx4 total = sum[0] + sum[1];
+				if constexpr (F::kMins)
+				{
+					// eight sums of a row's high or low parts; the high ones' products are short enough to be summed exactly
+					const half8 sums = g == 0 ? *reinterpret_cast<const half8*>(sums_from) : half8{};
+					const floatx4 centre = __builtin_amdgcn_mfma_f32_16x16x32_f16(sums, F::centre_frag(head), floatx4{}, 0, 0, 0);
+					const floatx4 s = __builtin_amdgcn_mfma_f32_16x16x32_f16(sums, F::min_frag(head), floatx4{}, 0, 0, 0);
+					const float dm = F::min_scale(head) * (1.0f / kSumScale);
+#pragma unroll
+					for (int e = 0; e < NE; ++e)
+					{
+						total[e] = fmaf(d, total[e], fmaf(d, centre[e], dm * s[e]));
+					}
+				}
+				else
+				{
+					total *= d;
+				}
+#pragma unroll
+				for (int e = 0; e < NE; ++e)
+				{
+					const float even = xs.unscale[e < MR ? e : 0], odd = xs.unscale[e + 4 < MR ? e + 4 : 0]; // (values: a choice of places would keep them in memory)
+					acc[e] = fmaf(total[e], g & 1 ? odd : even, acc[e]);
+				}
+				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 			};
+			for (int c = c_begin; c < c_end; c += 2)
+			{
+				step(c, moving[0], acc[0]);
+				if (c + 1 < c_end)
+				{
+					step(c + 1, moving[1], acc[1]);
+				}
+			}
+			__syncthreads();
+			float* const handed = reinterpret_cast<float*>(lds); // [KS][activation row][weight row]
+#pragma unroll
+			for (int e = 0; e < NE; ++e)
+			{
+				const int row = 4 * (g & 1) + e;
+				const float high = acc[0][e] + acc[1][e], low = __shfl_xor(high, 32, 64);
+				if (g < 2 && row < m)
+				{
+					handed[(part * MR + row) * kFewTile + r] = fmaf(low, kLowScale, high);
+				}
+			}
+			__syncthreads();
+			for (int i = threadIdx.x; i < m * kFewTile; i += 64 * KS)
+			{
+				const int row = i / kFewTile, col = n_base + i % kFewTile;
+				float ranges[KS];
+#pragma unroll
+				for (int p = 0; p < KS; ++p)
+				{
+					ranges[p] = handed[p * MR * kFewTile + i];
+				}
+				add_in_pairs(ranges);
+				float v = ranges[0];
+				if (col < n)
+				{
+					if constexpr (F::kMins)
+					{
+						if (__builtin_expect(!(fabsf(v) <= 3.402823466e38f), 0))
+						{
+							const float* const from = x + static_cast<size_t>(row) * k;
+							v = plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) { return from[i]; });
+						}
+					}
+					const size_t o = static_cast<size_t>(row) * n + col;
+					y[o] = residual ? residual[o] + v : v;
+				}
+			}
+		}
+
+		// The same where there are many weight rows: 32 of them share a wavefront's preparation of the activations, on
+		// v_mfma_f32_32x32x16_f16 with rows 0 .. MR - 1 of a fragment the high parts and 16 .. 16 + MR - 1 the low ones, so that one
+		// product forms both; their sums lie in one lane (elements e and e + 8 of the result).  us at 3 rows, 16 rows a
+		// workgroup and 32: 14336 x 4096 Q8_0 19.3 and 18.0, Q4_K 17.7 and 14.8, 12000 x 8192 24.9 and 23.6; 6000 x 2048 6.7 and 5.3.
+		template <typename F, int MR, int KS>
+		__global__ __launch_bounds__(64 * KS, 2) void exact_few_wide_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, float* y,
+		                                                            const float* residual, int n, int k, int m, int chunks, size_t row_bytes)
+		{
+			typedef FewRows<MR> R;
+			typedef WeightPieces<F> W;
+			constexpr int NE = 4; // results of a lane
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][slot, fragments]; later the KS sums
+			const int lane = threadIdx.x & 63;
+			const int part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int r = lane & 31, h = lane >> 5;
+			const int n_base = blockIdx.x * kTile;
+			const int per = (chunks + KS - 1) / KS;
+			const int c_begin = part * per, c_end = min(c_begin + per, chunks);
+			uint8_t* const mine = lds + part * (W::kSlotBytes + R::kBytes);
+			uint8_t* const frags = mine + W::kSlotBytes;
+			const W weights(mine, w, n_base, n, row_bytes);
+
+			FewActivations<F, MR> xs(x, m, k, frags, lane);
 			const uint8_t* const frag_from = frags + h * R::kHalf + (r >> 4) * R::kPart + min(r & 15, m - 1) * 16;
 			const uint8_t* const sums_from = frags + R::kSums + h * R::kPart + min(r & 15, m - 1) * 16;
 
@@ -1354,13 +1666,13 @@ namespace litenn_hip
 			if (c_begin < c_end)
 			{
 				weights.request(moving[0], c_begin, lane);
-				request_x(c_begin);
+				xs.request(c_begin);
 				weights.request(moving[1], min(c_begin + 1, c_end - 1), lane);
 			}
 			const auto step = [&](int c, u32x4 (&arrived)[W::kLoads], float (&acc)[NE]) {
 				weights.deposit(arrived, lane);
-				deposit_x(c);
-				request_x(min(c + 1, c_end - 1));
+				xs.deposit(c);
+				xs.request(min(c + 1, c_end - 1));
 				weights.request(arrived, min(c + 2, c_end - 1), lane);
 				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wavefront's LDS accesses keep their order)
 				lds_bytes_t const chunk = weights.chunk(lane);
@@ -1443,7 +1755,8 @@ namespace litenn_hip
 				for (int e = 0; e < NE; ++e)
 				{
 					const int row = 8 * (e / 4) + (e & 3);
-					acc[e] = fmaf(sum[e], h ? unscale[row + 4 < MR ? row + 4 : 0] : unscale[row < MR ? row : 0], acc[e]);
+					const float low4 = xs.unscale[row < MR ? row : 0], high4 = xs.unscale[row + 4 < MR ? row + 4 : 0];
+					acc[e] = fmaf(sum[e], h ? high4 : low4, acc[e]);
 				}
 				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 			};
@@ -1602,30 +1915,36 @@ namespace litenn_hip
 			hipStream_t stream;
 		};
 
-		template <typename F, int MR, int KS>
+		// tile: weight rows of a workgroup
+		template <typename F, int MR, int KS, int TILE>
 		void launch_few(const FewCall& c)
 		{
-			constexpr size_t tiles = static_cast<size_t>(KS) * (WeightPieces<F>::kSlotBytes + FewRows<MR>::kBytes);
-			constexpr size_t sums = static_cast<size_t>(KS) * MR * kTile * sizeof(float);
-			constexpr size_t lds = tiles > sums ? tiles : sums;
+			constexpr size_t parts = static_cast<size_t>(KS) * (WeightPieces<F, TILE>::kSlotBytes + FewRows<MR>::kBytes);
+			constexpr size_t sums = static_cast<size_t>(KS) * MR * TILE * sizeof(float);
+			constexpr size_t lds = parts > sums ? parts : sums;
 			static_assert(lds <= 160 * 1024, "LDS");
-			allow_dynamic_lds(reinterpret_cast<const void*>(&exact_few_kernel<F, MR, KS>), lds);
-			exact_few_kernel<F, MR, KS><<<dim3((c.n + kTile - 1) / kTile), dim3(64 * KS), lds, c.stream>>>(
-			    c.w, c.x, c.y, c.residual, c.n, c.k, c.m, c.chunks, c.row_bytes);
+			constexpr auto kernel = TILE == kFewTile ? &exact_few_kernel<F, MR, KS> : &exact_few_wide_kernel<F, MR, KS>;
+			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+			kernel<<<dim3((c.n + TILE - 1) / TILE), dim3(64 * KS), lds, c.stream>>>(c.w, c.x, c.y, c.residual, c.n, c.k, c.m, c.chunks, c.row_bytes);
 		}
 
 		template <typename F, int MR>
 		void launch_few_rows(const FewCall& c)
 		{
-			// Eight ranges of K where 8192 weight rows and fewer leave CUs idle, else four (us at 3 rows: Q8_0 4096 x 4096 10.9
-			// with eight, 11.8 with four; Q6_K 4096 x 14336 24.7 and 30.2; Q4_0 11008 x 4096 16.4 and 14.3).
-			if (c.n <= 8192 && c.chunks >= 8)
+			// Sixteen weight rows a workgroup while each has a CU to itself (us at 3 rows, sixteen and 32: Q8_0 4096 x 4096 7.8 and 10.3,
+			// 1024 x 4096 6.1 and 8.2, Q6_K 4096 x 14336 16.8 and 24.8; in a second round not: 6000 x 2048 9.0 and 7.7), in eight ranges of K.
+			if (c.n <= 256 * kFewTile)
 			{
-				launch_few<F, MR, 8>(c);
+				launch_few<F, MR, 8, kFewTile>(c);
+			}
+			// Eight ranges of K where 8192 weight rows and fewer leave CUs idle, else four (Q4_0 11008 x 4096 16.4 and 14.3).
+			else if (c.n <= 8192 && c.chunks >= 8)
+			{
+				launch_few<F, MR, 8, kTile>(c);
 			}
 			else
 			{
-				launch_few<F, MR, 4>(c);
+				launch_few<F, MR, 4, kTile>(c);
 			}
 		}
 

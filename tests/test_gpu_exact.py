@@ -67,6 +67,13 @@ def test_few_rows(hip, fmt, m, n, k):
     assert errors(hip, fmt, m, n, k, residual=m % 2 == 0).max() <= 1e-6
 
 
+@pytest.mark.parametrize("fmt", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(2, 15, 256), (3, 17, 2304), (5, 4095, 256), (8, 4096, 512), (3, 4097, 512), (4, 4113, 256)])
+def test_few_rows_where_the_tile_changes(hip, fmt, m, n, k):
+    """Edges of sixteen weight rows, and both sides of the line to 32."""
+    assert errors(hip, fmt, m, n, k, residual=m % 2 == 0).max() <= 1e-6
+
+
 @pytest.mark.parametrize("fmt", [Q4_0, Q8_0])
 @pytest.mark.parametrize("m,n,k", [(2, 17, 32), (4, 33, 288), (7, 40, 1056), (3, 70, 2080)])
 def test_few_rows_that_end_inside_a_chunk(hip, fmt, m, n, k):
