@@ -16,6 +16,8 @@ namespace litenn_hip
 	namespace
 	{
 		// ---------------- embedding ----------------------------------------------------------
+		// Four entries a thread.  Bound by the sines; in half turns they need no reduction of large angles: 2048 rows of 4096 24.6 ->
+		// 16.1 us.
 		__global__ __launch_bounds__(256) void embed_rows_kernel(DenseMatrix table, const int32_t* __restrict__ ids,
 		                                                         const double* __restrict__ turns, Position pos,
 		                                                         float* __restrict__ x, int* __restrict__ err)
@@ -34,19 +36,36 @@ namespace litenn_hip
 			float* xr = x + static_cast<size_t>(row) * table.k;
 			const double p = static_cast<double>(row_position(pos, row));
 			const int i = static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x);
-			if (2 * i < table.k)
+			// the angle in turns, reduced in double: what reaches the Float32 sine, in half turns, is at most one
+			const auto position_vector = [&](int pair, float& sn, float& cs) {
+				const double t0 = p * turns[pair];
+				sincospif(static_cast<float>(2.0 * (t0 - rint(t0))), &sn, &cs);
+			};
+			if (4 * i + 3 < table.k && table.k % 4 == 0)
+			{
+				const uint2 w = *reinterpret_cast<const uint2*>(t + 4 * i);
+				floatx4 v = { bf16_to_f32(w.x & 0xffffu), bf16_to_f32(w.x >> 16), bf16_to_f32(w.y & 0xffffu), bf16_to_f32(w.y >> 16) };
+				if (turns)
+				{
+					float sn[2], cs[2];
+					position_vector(2 * i, sn[0], cs[0]);
+					position_vector(2 * i + 1, sn[1], cs[1]);
+					v += floatx4{ sn[0], cs[0], sn[1], cs[1] };
+				}
+				*reinterpret_cast<floatx4*>(xr + 4 * i) = v;
+				return;
+			}
+			for (int pair = 2 * i; pair < 2 * i + 2 && 2 * pair < table.k; ++pair)
 			{
 				float sn = 0.0f, cs = 0.0f;
 				if (turns)
 				{
-					// the angle in turns, reduced in double: what reaches the Float32 sine is below half a turn
-					const double t0 = p * turns[i];
-					sincosf(static_cast<float>((t0 - rint(t0)) * 6.283185307179586476925), &sn, &cs);
+					position_vector(pair, sn, cs);
 				}
-				xr[2 * i] = bf16_to_f32(t[2 * i]) + sn;
-				if (2 * i + 1 < table.k)
+				xr[2 * pair] = bf16_to_f32(t[2 * pair]) + sn;
+				if (2 * pair + 1 < table.k)
 				{
-					xr[2 * i + 1] = bf16_to_f32(t[2 * i + 1]) + cs;
+					xr[2 * pair + 1] = bf16_to_f32(t[2 * pair + 1]) + cs;
 				}
 			}
 		}
@@ -1627,7 +1646,7 @@ namespace litenn_hip
 	{
 		if (rows > 0)
 		{
-			embed_rows_kernel<<<dim3(rows, (table.k + 511) / 512), dim3(256), 0, s>>>(table, ids, turns, pos, x, err);
+			embed_rows_kernel<<<dim3(rows, (table.k + 1023) / 1024), dim3(256), 0, s>>>(table, ids, turns, pos, x, err);
 		}
 	}
 
