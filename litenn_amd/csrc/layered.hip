@@ -1040,7 +1040,8 @@ namespace litenn_hip
 				const int n = &L == &layers.back() ? logit_rows : rows, first = rows - n;
 				const bool one = n == 1;
 				// (attention in 32 bits takes a few rows the slower the fewer they are, and looks at what comes out of all of them)
-				const int asked = f32 ? first / kAttnRows * kAttnRows : first;
+				const bool by_step = M.desc.kind == MixerKind::LatentAttention && latent_by_step(M, n, past + rows);
+				const int asked = f32 && !by_step ? first / kAttnRows * kAttnRows : first;
 				enter(L.norm1, 0, rows);
 				OneRow row{ *this, x + static_cast<size_t>(first) * desc.width, 0 };
 				if (asked > 0)
@@ -1113,6 +1114,15 @@ namespace litenn_hip
 			launch_dense_rows(d, stream);
 		}
 
+		// Whether `n` queries behind `length` positions attend as a step does, to the cached latents themselves: one does where the
+		// keys it sees are too many to be expanded for it alone.  us of a whole prompt of two layers, expanded and by step, bfloat16:
+		// 2048 wide, 128 tokens 242 and 245, 400 290 and 289, 800 356 and 344, 2048 547 and 523; 4096 wide, 256 tokens 488 and 489, 2048
+		// 1471 and 1446.  In 32 bits, whose expanded attention takes a tile of queries: 128 tokens 315 and 288, 400 441 and 396.
+		bool latent_by_step(const MixerState& M, int n, int length) const
+		{
+			return n == 1 && std::min(length, M.desc.window) >= (f32 ? 64 : 384);
+		}
+
 		// queries of rows `first` .. (and some ahead of them), keys of all rows
 		void attend(const MixerState& M, int rows, int first, int past, const Position& pos)
 		{
@@ -1147,7 +1157,7 @@ namespace litenn_hip
 				product(M.uq, mid, ld_mid, rows - first, queries(first), ld_q, kOutF32);
 			}
 			launch_latent_append(proj + M.at_latent, ld_proj, M.latent_norm, desc.eps, rows, pos, M.cache, stream);
-			if (rows < kExpandMin)
+			if (rows < kExpandMin || latent_by_step(M, rows - first, past + rows))
 			{
 				LatentStep a;
 				a.shape = latent_shape(M);
