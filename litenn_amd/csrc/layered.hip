@@ -791,17 +791,21 @@ namespace litenn_hip
 		void mix_rows(const LayerState& L, int rows, int first, int past, const Position& pos)
 		{
 			const size_t operand = f32 ? 4 : 2;
+			const MixerState *attention = nullptr, *space = nullptr;
+			GroupedAttn a;
+			WindowAttn w;
+			Ssm b;
 			for (const MixerState& M : L.mixers)
 			{
 				uint8_t* out = static_cast<uint8_t*>(mid) + operand * static_cast<size_t>(M.at_mid);
 				if (M.desc.kind == MixerKind::GroupedAttention)
 				{
-					GroupedAttn a = grouped_args(M);
+					attention = &M;
+					a = grouped_args(M);
 					a.rows = rows;
 					a.pos = pos;
 					a.q_from = first;
-					launch_grouped_append(a, stream);
-					WindowAttn w = grouped_window(a, past);
+					w = grouped_window(a, past);
 					const int from = first / kAttnRows * kAttnRows;
 					w.q += static_cast<size_t>(from) * w.ldq;
 					w.q_base += from;
@@ -809,24 +813,39 @@ namespace litenn_hip
 					w.out_scale = M.desc.weight;
 					w.out = out + operand * static_cast<size_t>(from) * ld_mid;
 					w.ldo = ld_mid;
-					launch_window_attn(w, stream);
 				}
 				else
 				{
-					Ssm a = ssm_args(M);
-					a.rows = rows;
-					a.pos = pos;
-					a.out_from = first;
-					launch_ssm_rows(a, stream);
-					GatedNorm g = gated_norm_args(M);
-					g.y = a.in + static_cast<size_t>(first) * ld_proj;
-					g.ldy = ld_proj;
-					g.out = out + operand * static_cast<size_t>(first) * ld_mid;
-					g.ldo = ld_mid;
-					g.rows = rows - first;
-					g.f32 = f32;
-					launch_gated_norm(g, stream);
+					space = &M;
+					b = ssm_args(M);
+					b.rows = rows;
+					b.pos = pos;
+					b.out_from = first;
 				}
+			}
+			if (attention && space)
+			{
+				launch_mixer_rows(a, w, b, stream);
+			}
+			else if (attention)
+			{
+				launch_grouped_append(a, stream);
+				launch_window_attn(w, stream);
+			}
+			else
+			{
+				launch_ssm_rows(b, stream);
+			}
+			if (space)
+			{
+				GatedNorm g = gated_norm_args(*space);
+				g.y = b.in + static_cast<size_t>(first) * ld_proj;
+				g.ldy = ld_proj;
+				g.out = static_cast<uint8_t*>(mid) + operand * (static_cast<size_t>(first) * ld_mid + space->at_mid);
+				g.ldo = ld_mid;
+				g.rows = rows - first;
+				g.f32 = f32;
+				launch_gated_norm(g, stream);
 			}
 		}
 

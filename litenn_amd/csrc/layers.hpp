@@ -225,6 +225,10 @@ namespace litenn_hip
 	size_t ssm_chunk_floats(int rows, const Ssm& shape);
 	void launch_ssm_rows(const Ssm& a, hipStream_t s);
 
+	// A prompt's rows through both mixers, as launch_grouped_append, launch_window_attn and launch_ssm_rows, with what does not
+	// wait for each other in one launch.
+	void launch_mixer_rows(const GroupedAttn& attn, const WindowAttn& window, const Ssm& ssm, hipStream_t s);
+
 	// out = scale w norm(y silu(z)), in `parts` equal parts with a root mean square of their own (z null: y alone)
 	struct GatedNorm
 	{

@@ -5,6 +5,7 @@
 // run on the Float32 matrix instructions).  Norms, angles, scores, softmax and everything inside the recurrence
 // are Float32.  The reference has no counterpart of these layers.
 #include "layer_device.hpp"
+#include "window_tile.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -102,12 +103,12 @@ namespace litenn_hip
 
 		// KEPT > 0: queries and keys of up to 1024 KEPT elements pass through LDS, read once; 0: any number
 		template <typename T, int KEPT>
-		__global__ __launch_bounds__(256) void grouped_append_kernel(const GroupedAttn a)
+		__device__ __forceinline__ void grouped_append_block(const GroupedAttn& a, int row)
 		{
 			__shared__ float red[8];
 			__shared__ __attribute__((aligned(16))) float cs[kGroupedMaxDim / 2], sn[kGroupedMaxDim / 2];
 			__shared__ __attribute__((aligned(16))) float lds[KEPT > 0 ? 1024 * KEPT : 4];
-			const int row = blockIdx.x, position = row_position(a.pos, row), tid = threadIdx.x;
+			const int position = row_position(a.pos, row), tid = threadIdx.x;
 			const HeadCache& c = a.cache;
 			const float* q = a.q + static_cast<size_t>(row) * a.ld;
 			const float* k = a.k + static_cast<size_t>(row) * a.ld;
@@ -214,6 +215,12 @@ namespace litenn_hip
 					operand_store(rows + e / c.vdim * c.head_stride() + c.key_pitch() + e % c.vdim, v[e]);
 				}
 			}
+		}
+
+		template <typename T, int KEPT>
+		__global__ __launch_bounds__(256) void grouped_append_kernel(const GroupedAttn a)
+		{
+			grouped_append_block<T, KEPT>(a, blockIdx.x);
 		}
 
 		// ---------------- one token's attention --------------------------------------------------------
@@ -875,12 +882,14 @@ namespace litenn_hip
 
 		// x | B | C behind convolution and silu, four channels per thread; the last column of workgroups makes the
 		// step sizes and log decays.  TAPS > 0: that many taps, channels a multiple of 4, every input read once; 0: any.
+		// (block `bx` of ssm_conv_blocks in rows `by`)
+		__host__ __device__ inline int ssm_conv_blocks(const Ssm& a) { return (a.ldx() / 4 + 63) / 64 + 1; }
 		template <int TAPS>
-		__global__ __launch_bounds__(256) void ssm_conv_kernel(const Ssm a)
+		__device__ __forceinline__ void ssm_conv_block(const Ssm& a, int bx, int by)
 		{
 			const int inner = a.inner(), channels = a.channels(), ldx = a.ldx();
-			const int block_row = static_cast<int>(blockIdx.y) * 4 * kConvRows;
-			if (blockIdx.x + 1 == gridDim.x)
+			const int block_row = by * 4 * kConvRows;
+			if (bx + 1 == ssm_conv_blocks(a))
 			{
 				const int count = min(4 * kConvRows, a.rows - block_row);
 				for (int i = threadIdx.x; i < count * a.heads; i += 256)
@@ -893,7 +902,7 @@ namespace litenn_hip
 				}
 				return;
 			}
-			const int ch = (static_cast<int>(blockIdx.x) * 64 + static_cast<int>(threadIdx.x & 63)) * 4;
+			const int ch = (bx * 64 + static_cast<int>(threadIdx.x & 63)) * 4;
 			const int row0 = block_row + static_cast<int>(threadIdx.x >> 6) * kConvRows;
 			if (ch >= channels || row0 >= a.rows)
 			{
@@ -980,13 +989,32 @@ namespace litenn_hip
 			}
 		}
 
+		template <int TAPS>
+		__global__ __launch_bounds__(256) void ssm_conv_kernel(const Ssm a)
+		{
+			ssm_conv_block<TAPS>(a, blockIdx.x, blockIdx.y);
+		}
+
+		// Both, which depend on the same projections alone, in one launch: the append's rows first.  777 rows 8.9 and 8.1 us -> 11.6.
+		template <typename T, int KEPT, int TAPS>
+		__global__ __launch_bounds__(256) void mixer_prepare_kernel(const GroupedAttn attn, const Ssm ssm)
+		{
+			const int i = blockIdx.x;
+			if (i < attn.rows)
+			{
+				grouped_append_block<T, KEPT>(attn, i);
+				return;
+			}
+			const int wide = ssm_conv_blocks(ssm);
+			ssm_conv_block<TAPS>(ssm, (i - attn.rows) % wide, (i - attn.rows) / wide);
+		}
+
 		// Sums of a chunk's log decays up to and including every token, and its step sizes (zero behind the last
 		// token), by the first wavefront.
-		__device__ __forceinline__ void chunk_sums(const Ssm& a, int h, int row0, int count, double* sums, float* dts)
+		__device__ __forceinline__ void chunk_sums(const Ssm& a, int h, int row0, int count, double* sums, float* dts, int t)
 		{
-			if (threadIdx.x < kChunk)
+			if (t < kChunk)
 			{
-				const int t = threadIdx.x;
 				const size_t at = static_cast<size_t>(row0 + min(t, count - 1)) * a.heads + h;
 				double l = t < count ? static_cast<double>(a.steps[static_cast<size_t>(a.rows) * a.heads + at]) : 0.0;
 				dts[t] = t < count ? a.steps[at] : 0.0f;
@@ -1036,7 +1064,7 @@ namespace litenn_hip
 				const int row = 16 * part + t;
 				b[t] = live && row < count ? bs[static_cast<size_t>(row0 + row) * ldx + n0 + lane] : 0.0f;
 			}
-			chunk_sums(a, h, row0, count, sums, dts);
+			chunk_sums(a, h, row0, count, sums, dts, threadIdx.x);
 			__syncthreads();
 			const double end = sums[kChunk - 1];
 			if (rest == 0 && threadIdx.x == 0)
@@ -1136,24 +1164,31 @@ namespace litenn_hip
 		}
 
 		// A wavefront makes 64 value columns of a block of 16 tokens of one head; y silu(z) goes where z was.
-		__global__ __launch_bounds__(256) void ssm_out_kernel(const Ssm a)
+		// (by 256 threads, `tid` of them this one; what is not `live` only passes the barriers)
+		struct SsmOutLds
 		{
-			__shared__ __attribute__((aligned(16))) float cs[kChunk][kSlabStride];
-			__shared__ __attribute__((aligned(16))) float bs[kChunk][kSlabStride];
-			__shared__ double sums[kChunk];
-			__shared__ float dts[kChunk];
+			float cs[kChunk][kSlabStride], bs[kChunk][kSlabStride];
+			double sums[kChunk];
+			float dts[kChunk];
+		};
+		__device__ __forceinline__ void ssm_out_block(const Ssm& a, int bx, int by, bool live_block, int tid, SsmOutLds& lds)
+		{
+			auto& cs = lds.cs;
+			auto& bs = lds.bs;
+			auto& sums = lds.sums;
+			auto& dts = lds.dts;
 			const int pitch = ssm_state_pitch(a.vdim), ldx = a.ldx(), vdim = a.vdim;
-			const int h = static_cast<int>(blockIdx.x) % a.heads, v0 = static_cast<int>(blockIdx.x) / a.heads * kSlice;
-			const int chunk = static_cast<int>(blockIdx.y) + a.out_from / kChunk, row0 = chunk * kChunk, count = min(kChunk, a.rows - row0);
-			const int lane = threadIdx.x & 63;
-			const int block = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+			const int h = bx % a.heads, v0 = bx / a.heads * kSlice;
+			const int chunk = by + a.out_from / kChunk, row0 = chunk * kChunk, count = min(kChunk, a.rows - row0);
+			const int lane = tid & 63;
+			const int block = __builtin_amdgcn_readfirstlane(tid >> 6);
 			const int j = lane & 15, g = lane >> 4;
 			const int e0 = v0 + 4 * j;
 			const float* const state = a.chunk_states + (static_cast<size_t>(chunk) * a.heads + h) * a.state * pitch;
 			const float* const xs = a.xbc + h * vdim;
 			const float* const b_in = a.xbc + a.inner() + h / (a.heads / a.groups) * a.state;
 			const float* const c_in = b_in + a.groups * a.state;
-			chunk_sums(a, h, row0, count, sums, dts);
+			chunk_sums(a, h, row0, count, sums, dts, tid);
 
 			floatx4 o[4];      // o[b][r]: value column v0 + 16 g + 4 r + b of token j of the block
 			floatx4 scores[4]; // scores[back][r]: token 4 g + r of `block - back` against token j
@@ -1259,7 +1294,7 @@ namespace litenn_hip
 					}
 				}
 			}
-			if (row >= count)
+			if (row >= count || !live_block)
 			{
 				return;
 			}
@@ -1298,27 +1333,50 @@ namespace litenn_hip
 			}
 		}
 
+		__global__ __launch_bounds__(256) void ssm_out_kernel(const Ssm a)
+		{
+			__shared__ __attribute__((aligned(16))) SsmOutLds lds;
+			ssm_out_block(a, blockIdx.x, blockIdx.y, true, threadIdx.x, lds);
+		}
+
+		// Both mixers' outputs, which wait for different things, in one launch: neither fills the card, and both are chains of
+		// loads and products.  The attention's tiles first, the longest chains ahead, then the recurrence's blocks, PARTS to a
+		// workgroup.  777 rows, 16 heads of 128 and 32 of the recurrence 22.4 and 22.7 us -> 36, whole prompts 2 to 10 % (three layers
+		// 700 -> 665 with the launch above; the same bits).  144 registers leave a CU one workgroup of eight wavefronts; held to 128
+		// they spill (2048 rows 694 -> 746).
+		template <int DK, int DV, int PARTS>
+		__global__ __launch_bounds__(256 * PARTS) void mixer_outputs_kernel(const WindowAttn attn, const Ssm ssm, int tiles, int ssm_wide, int ssm_blocks)
+		{
+			extern __shared__ __attribute__((aligned(16))) uint8_t outputs_lds[];
+			const int i = blockIdx.x, heads = attn.shape.heads;
+			if (i < heads * tiles)
+			{
+				window_tile_block<DK, DV, PARTS>(attn, i % heads, tiles - 1 - i / heads, reinterpret_cast<uint16_t*>(outputs_lds));
+				return;
+			}
+			const int part = PARTS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), block = (i - heads * tiles) * PARTS + part;
+			const int b = min(block, ssm_blocks - 1);
+			ssm_out_block(ssm, b % ssm_wide, b / ssm_wide, block < ssm_blocks, threadIdx.x & 255, reinterpret_cast<SsmOutLds*>(outputs_lds)[part]);
+		}
+
 		bool narrow_heads(const HeadCache& c) { return c.key_pitch() <= 256 && c.value_pitch() <= 256; }
+
+		// the form of the append: thousands of elements of a row that pass through LDS, 0 for more
+		int append_kept(const GroupedAttn& a)
+		{
+			const size_t cols = ((static_cast<size_t>(a.heads) * a.cache.dim + 3) & ~size_t{ 3 }) + static_cast<size_t>(a.cache.heads) * a.cache.dim;
+			return cols <= 2048 ? 2 : cols <= 5120 ? 5 : cols <= 10240 ? 10 : 0;
+		}
 
 		template <typename T>
 		void launch_append(const GroupedAttn& a, hipStream_t s)
 		{
-			const size_t cols = ((static_cast<size_t>(a.heads) * a.cache.dim + 3) & ~size_t{ 3 }) + static_cast<size_t>(a.cache.heads) * a.cache.dim;
-			if (cols <= 2048)
+			switch (append_kept(a))
 			{
-				grouped_append_kernel<T, 2><<<dim3(a.rows), dim3(256), 0, s>>>(a);
-			}
-			else if (cols <= 5120)
-			{
-				grouped_append_kernel<T, 5><<<dim3(a.rows), dim3(256), 0, s>>>(a);
-			}
-			else if (cols <= 10240)
-			{
-				grouped_append_kernel<T, 10><<<dim3(a.rows), dim3(256), 0, s>>>(a);
-			}
-			else
-			{
-				grouped_append_kernel<T, 0><<<dim3(a.rows), dim3(256), 0, s>>>(a);
+			case 2: grouped_append_kernel<T, 2><<<dim3(a.rows), dim3(256), 0, s>>>(a); break;
+			case 5: grouped_append_kernel<T, 5><<<dim3(a.rows), dim3(256), 0, s>>>(a); break;
+			case 10: grouped_append_kernel<T, 10><<<dim3(a.rows), dim3(256), 0, s>>>(a); break;
+			default: grouped_append_kernel<T, 0><<<dim3(a.rows), dim3(256), 0, s>>>(a); break;
 			}
 		}
 
@@ -1395,14 +1453,11 @@ namespace litenn_hip
 		return chunks * a.heads * (static_cast<size_t>(a.state) * ssm_state_pitch(a.vdim) + 1);
 	}
 
-	void launch_ssm_rows(const Ssm& a, hipStream_t s)
+	static int ssm_conv_rows(const Ssm& a) { return (a.rows + 4 * kConvRows - 1) / (4 * kConvRows); }
+
+	static void launch_ssm_conv(const Ssm& a, hipStream_t s)
 	{
-		if (a.rows <= 0)
-		{
-			return;
-		}
-		const int conv_blocks = (a.ldx() / 4 + 63) / 64;
-		const dim3 conv_grid(conv_blocks + 1, (a.rows + 4 * kConvRows - 1) / (4 * kConvRows));
+		const dim3 conv_grid(ssm_conv_blocks(a), ssm_conv_rows(a));
 		switch (a.channels() % 4 == 0 ? a.taps : 0)
 		{
 		case 2: ssm_conv_kernel<2><<<conv_grid, dim3(256), 0, s>>>(a); break;
@@ -1410,15 +1465,114 @@ namespace litenn_hip
 		case 4: ssm_conv_kernel<4><<<conv_grid, dim3(256), 0, s>>>(a); break;
 		default: ssm_conv_kernel<0><<<conv_grid, dim3(256), 0, s>>>(a); break;
 		}
+	}
+
+	// the state every chunk begins with, and the new one
+	static void launch_ssm_states(const Ssm& a, hipStream_t s)
+	{
 		const int chunks = (a.rows + kChunk - 1) / kChunk;
 		const int slabs = (a.state + kSlab - 1) / kSlab, slices = (a.vdim + kSlice - 1) / kSlice;
 		ssm_state_kernel<<<dim3(a.heads * slabs * slices, chunks), dim3(256), 0, s>>>(a);
 		const int scan_blocks = (a.heads * a.state * (ssm_state_pitch(a.vdim) >> 2) + 255) / 256;
 		const int ring_blocks = (std::min(a.rows, a.taps) * a.channels() + 255) / 256;
 		ssm_scan_kernel<<<dim3(scan_blocks + ring_blocks), dim3(256), 0, s>>>(a, chunks, scan_blocks);
-		if (a.out_from < a.rows)
+	}
+
+	// workgroups of the outputs: heads' value slices by chunks
+	static dim3 ssm_out_grid(const Ssm& a)
+	{
+		return a.out_from < a.rows ? dim3(a.heads * ((a.vdim + kSlice - 1) / kSlice), (a.rows + kChunk - 1) / kChunk - a.out_from / kChunk) : dim3(0, 0);
+	}
+
+	void launch_ssm_rows(const Ssm& a, hipStream_t s)
+	{
+		if (a.rows <= 0)
 		{
-			ssm_out_kernel<<<dim3(a.heads * slices, chunks - a.out_from / kChunk), dim3(256), 0, s>>>(a);
+			return;
+		}
+		launch_ssm_conv(a, s);
+		launch_ssm_states(a, s);
+		const dim3 grid = ssm_out_grid(a);
+		if (grid.x > 0)
+		{
+			ssm_out_kernel<<<grid, dim3(256), 0, s>>>(a);
+		}
+	}
+
+	template <typename T, int KEPT>
+	static void launch_prepare(const GroupedAttn& attn, const Ssm& ssm, hipStream_t s)
+	{
+		const unsigned conv = static_cast<unsigned>(ssm_conv_blocks(ssm)) * ssm_conv_rows(ssm);
+		mixer_prepare_kernel<T, KEPT, 4><<<dim3(attn.rows + conv), dim3(256), 0, s>>>(attn, ssm);
+	}
+
+	template <typename T>
+	static bool launch_prepare(const GroupedAttn& attn, const Ssm& ssm, hipStream_t s)
+	{
+		switch (append_kept(attn))
+		{
+		case 2: launch_prepare<T, 2>(attn, ssm, s); return true;
+		case 5: launch_prepare<T, 5>(attn, ssm, s); return true;
+		case 10: launch_prepare<T, 10>(attn, ssm, s); return true;
+		default: return false;
+		}
+	}
+
+	template <int DK, int DV, int PARTS>
+	static void launch_outputs(const WindowAttn& attn, const Ssm& ssm, hipStream_t s)
+	{
+		constexpr size_t lds = std::max(window_tile_lds<DK, DV>(), PARTS * sizeof(SsmOutLds));
+		const int tiles = (attn.rows + kWinQ - 1) / kWinQ;
+		const dim3 grid = ssm_out_grid(ssm);
+		const int blocks = static_cast<int>(grid.x * grid.y);
+		allow_dynamic_lds(reinterpret_cast<const void*>(&mixer_outputs_kernel<DK, DV, PARTS>), lds);
+		mixer_outputs_kernel<DK, DV, PARTS><<<dim3(attn.shape.heads * tiles + (blocks + PARTS - 1) / PARTS), dim3(256 * PARTS), lds, s>>>(
+		    attn, ssm, tiles, static_cast<int>(grid.x), blocks);
+	}
+
+	template <int DK, int DV>
+	static void launch_outputs(const WindowAttn& attn, const Ssm& ssm, hipStream_t s)
+	{
+		if (window_shares_queries(static_cast<size_t>(attn.shape.heads) * ((attn.rows + kWinQ - 1) / kWinQ)))
+		{
+			launch_outputs<DK, DV, 2>(attn, ssm, s);
+		}
+		else
+		{
+			launch_outputs<DK, DV, 1>(attn, ssm, s);
+		}
+	}
+
+	void launch_mixer_rows(const GroupedAttn& attn, const WindowAttn& window, const Ssm& ssm, hipStream_t s)
+	{
+		if (attn.rows <= 0)
+		{
+			return;
+		}
+		const bool four = ssm.channels() % 4 == 0 && ssm.taps == 4;
+		if (!four || !(attn.cache.f32 ? launch_prepare<float>(attn, ssm, s) : launch_prepare<uint16_t>(attn, ssm, s)))
+		{
+			launch_grouped_append(attn, s);
+			launch_ssm_conv(ssm, s);
+		}
+		launch_ssm_states(ssm, s);
+		const dim3 grid = ssm_out_grid(ssm);
+		if (grid.x > 0 && window.rows > 0 && window_takes_tiles(window) && window.shape.dim <= 128 && window.shape.vdim <= 128)
+		{
+			if (window.shape.dim <= 64)
+			{
+				window.shape.vdim <= 64 ? launch_outputs<64, 64>(window, ssm, s) : launch_outputs<64, 128>(window, ssm, s);
+			}
+			else
+			{
+				window.shape.vdim <= 64 ? launch_outputs<128, 64>(window, ssm, s) : launch_outputs<128, 128>(window, ssm, s);
+			}
+			return;
+		}
+		launch_window_attn(window, s);
+		if (grid.x > 0)
+		{
+			ssm_out_kernel<<<grid, dim3(256), 0, s>>>(ssm);
 		}
 	}
 

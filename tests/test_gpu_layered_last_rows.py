@@ -24,6 +24,44 @@ LAST = {
 }
 
 
+@pytest.mark.parametrize("rows", [383, 384, 401])
+def test_one_row_over_cached_latents(hip, rows):
+    """Both sides of the number of keys from which one asked row attends to the latents themselves."""
+    cfg = ku.config([ku.linear_attention(), ku.attention(heads=5, window=390)])
+    w = ku.random_weights(cfg, 21)
+    toks = ku.tokens(cfg, rows, 6)
+    want = np_kulurax.NumpyKulurax(cfg, ku.as_floats(w)).forward(toks)
+    with hip.create_model(cfg, w, dtype="bfloat16", context_length=410) as model:
+        assert ku.error(model.eval(toks, want=[rows - 1]), want[rows - 1:]) <= LIMIT["bfloat16"]
+
+
+# heads and value sizes of every form of the launch that makes both mixers' outputs, at the edges of its tiles (64 queries,
+# chunks of 64 tokens, two blocks of the recurrence to a workgroup), few workgroups and many, four taps and others
+PAIRS = {
+    "64_64": du.layer(du.attention(4, 2, 64, 70, 0.1, 32), du.state_space(3, 64, 128, 1, 1, 4)),
+    "64_odd": du.layer(du.attention(3, 3, 40, 21, 0.2, 40), du.state_space(4, 36, 33, 1, 2, 4)),
+    "128": du.layer(du.attention(8, 2, 128, 100, 0.1, 128), du.state_space(2, 70, 65, 2, 1, 4)),
+    "96": du.layer(du.attention(5, 5, 96, 40, 0.1, 64), du.state_space(1, 20, 20, 1, 1, 4)),
+    "three_taps": du.layer(du.attention(4, 2, 64, 70, 0.1, 32), du.state_space(4, 32, 64, 2, 2, 3)),
+    "beyond": du.layer(du.attention(2, 2, 136, 70, 0.1, 100), du.state_space(2, 32, 64, 1, 1, 4)),
+    "many": du.layer(du.attention(64, 8, 64, 200, 0.1, 32), du.state_space(32, 64, 64, 2, 2, 4)),
+}
+
+
+@pytest.mark.parametrize("dtype", sorted(LIMIT))
+@pytest.mark.parametrize("name", sorted(PAIRS))
+def test_both_mixers_in_one_launch(hip, name, dtype):
+    cfg = du.config([PAIRS[name]])
+    w = du.random_weights(cfg, 8)
+    plain = np_degedra.NumpyDegedra(cfg, du.as_floats(w))
+    toks = ku.tokens(cfg, 330, 6)
+    want = plain.forward(toks)
+    with hip.create_model(cfg, w, dtype=dtype, context_length=330) as model:
+        for rows in (4, 63, 64, 65, 128, 330):
+            model.reset()
+            assert ku.error(model.eval(toks[:rows]), want[:rows]) <= LIMIT[dtype], rows
+
+
 @pytest.mark.parametrize("dtype", sorted(LIMIT))
 @pytest.mark.parametrize("name", sorted(LAST))
 def test_rows_asked_for(hip, name, dtype):
