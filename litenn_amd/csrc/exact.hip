@@ -787,13 +787,22 @@ namespace litenn_hip
 			}
 		};
 
-		// WN wavefronts side by side share the activation fragments of a range through LDS: two buffers of one 64-element stage,
-		// the next stage travelling through registers while the current one is multiplied.  The raw blocks of the next
-		// chunk travel through registers into the wavefront's slot meanwhile.  What a step of 16 elements multiplies is in
-		// registers when it begins: the step before asks for its activations ahead of its own products and decodes its
-		// weights behind them, and a stage's last products follow the barrier, so that they cover the next stage's first reads.
+		// WN wavefronts side by side share the activation fragments of a range through LDS: a ring of 64-element stages that loads fill
+		// directly, two stages ahead, which leaves registers for the sums and time for the blocks of the next chunk (they come from HBM,
+		// and what was asked for behind them arrives behind them).  Those blocks travel through registers into the wavefront's slot.
+		// What a step of 16 elements multiplies is in registers when it begins: the step before asks for its activations ahead of
+		// its own products and decodes its weights behind them, and a stage's last products follow the barrier, so that they cover
+		// the next stage's first reads.
+		// KS = 1 walks both halves of K one after the other and adds them as the two ranges of KS = 2 are added.
+		// Bound by the waits around a barrier per stage (matrix cores 36 % busy, VALU 35, LDS 30).  us, kernel alone, Q4_K 28672 x
+		// 4096 at 300 rows: stages through registers and two buffers 221, ring 216, KS = 1 with two workgroups to a CU 190.
+		constexpr int kRing = 3; // stages: one is multiplied, two are on their way
+		// all but the N youngest of the wavefront's loads are there
+		template <int N>
+		__device__ __forceinline__ void arrived() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+
 		template <typename F, int MT, int WN, int KS>
-		__global__ __launch_bounds__(64 * WN * KS) void exact_shared_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
+		__global__ __launch_bounds__(64 * WN * KS, 2) void exact_shared_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                    const float* residual, int k, int m, int m_tiles,
 		                                                                    int chunks, size_t row_bytes)
 		{
@@ -801,11 +810,11 @@ namespace litenn_hip
 			constexpr int kPieces = MT * 8 / WN; // 1 KB pieces a wavefront stages
 			static_assert(kPieces * WN == MT * 8, "activation pieces / wavefront split");
 			typedef WeightPieces<F> W;
-			constexpr int kRingBytes = KS * 2 * MT * kStageBytes;
-			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][2][MT][stage], [WN KS][slot]; later the KS sums
+			constexpr int kBuffer = MT * kStageBytes, kRingBytes = KS * kRing * kBuffer;
+			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][kRing][MT][stage], [WN KS][slot]; later the KS sums
 			const ExactPlace<F, MT, WN, KS> place(mats, chunks);
 			const int lane = place.lane, h = lane >> 5;
-			const int c_begin = place.c_begin, c_end = place.c_end;
+			const int c_begin = place.c_begin, c_end = place.c_end, half = (chunks + 1) / 2;
 			const W weights(lds + kRingBytes + (place.part * WN + place.wv) * W::kSlotBytes, place.w, place.n_base, place.n, row_bytes);
 			u32x4 moving[W::kLoads];
 
@@ -814,19 +823,19 @@ namespace litenn_hip
 #pragma unroll
 			for (int t = 0; t < MT; ++t)
 			{
-				sum_tiles[t] = xs + at.sums + static_cast<size_t>(min(place.mt_base + t, m_tiles - 1)) * chunks * kFrag + lane * 16;
+				sum_tiles[t] = xs + at.sums + static_cast<size_t>(min(place.mt_base + t, m_tiles - 1)) * chunks * kFrag;
 			}
 
 			floatx16 acc[MT], p[MT];
 			floatx16 held[MT]; // the chunk's first half
+			floatx16 first[KS == 1 ? MT : 1]; // one range: the sums of its first half, added at the end as a range's are
 #pragma unroll
 			for (int t = 0; t < MT; ++t)
 			{
 				acc[t] = floatx16{};
 			}
 
-			u32x4 staged[kPieces]; // the next stage on its way
-			uint8_t* const ring = lds + place.part * (2 * MT * kStageBytes);
+			const uint8_t* const ring = lds + place.part * kRingBytes / KS;
 			const uint8_t* from[kPieces];
 #pragma unroll
 			for (int i = 0; i < kPieces; ++i)
@@ -834,18 +843,19 @@ namespace litenn_hip
 				const int piece = i * WN + place.wv;
 				from[i] = xs + static_cast<size_t>(min(place.mt_base + (piece >> 3), m_tiles - 1)) * chunks * kTileChunkBytes + (piece & 7) * kFrag;
 			}
-			const auto request = [&](u32x4 (&into)[kPieces], int c, int st) {
+			const uint32_t lane_at = lane * 16;
+			const uint32_t ring_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_bytes_t)(ring)));
+			// (as inline assembly: a load into LDS that the compiler knew of would be waited for before every read of LDS)
+			const auto request = [&](int c, int st, int buffer) {
 #pragma unroll
 				for (int i = 0; i < kPieces; ++i)
 				{
-					into[i] = *reinterpret_cast<const u32x4*>(from[i] + static_cast<size_t>(c) * kTileChunkBytes + st * kStageBytes + lane * 16);
-				}
-			};
-			const auto deposit = [&](const u32x4 (&from)[kPieces], int buffer) {
-#pragma unroll
-				for (int i = 0; i < kPieces; ++i)
-				{
-					*reinterpret_cast<u32x4*>(ring + buffer * (MT * kStageBytes) + (i * WN + place.wv) * kFrag + lane * 16) = from[i];
+					const uint8_t* const src = from[i] + static_cast<size_t>(c) * kTileChunkBytes + st * kStageBytes;
+					const uint32_t dst = ring_lds + buffer * kBuffer + (i * WN + place.wv) * kFrag;
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm" // m0 is named as clobbered although it is reserved
+					asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(dst), "v"(lane_at), "s"(src) : "memory", "m0");
+#pragma clang diagnostic pop
 				}
 			};
 
@@ -857,7 +867,7 @@ namespace litenn_hip
 #pragma unroll
 					for (int e = 0; e < 2; ++e)
 					{
-						a[into][t][e] = *reinterpret_cast<const half8*>(ring + buffer * (MT * kStageBytes) + t * kStageBytes + (2 * s + e) * kFrag + lane * 16);
+						a[into][t][e] = *reinterpret_cast<const half8*>(ring + buffer * kBuffer + t * kStageBytes + (2 * s + e) * kFrag + lane * 16);
 					}
 				}
 			};
@@ -868,14 +878,16 @@ namespace litenn_hip
 			if (c_begin < c_end)
 			{
 				weights.request(moving, c_begin, lane);
-				request(staged, c_begin, 0);
+				request(c_begin, 0, 0);
+				request(c_begin, 1, 1);
 				weights.deposit(moving, lane);
-				deposit(staged, 0);
-				request(staged, c_begin, 1);
 				weights.request(moving, min(c_begin + 1, c_end - 1), lane);
 				__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+				arrived<kPieces + W::kLoads>(); // (behind the first stage's: the second's and the next chunk's blocks)
 			}
 			__syncthreads();
+			int buffer = 0;
+			const auto behind = [](int b, int by) { return b + by < kRing ? b + by : b + by - kRing; };
 			if (c_begin < c_end)
 			{
 				head = F::head(weights.chunk(lane), h);
@@ -883,104 +895,139 @@ namespace litenn_hip
 				read(0, 0, 0);
 				b[0] = F::frag(head, raw, 0, 0);
 			}
-			for (int c = c_begin; c < c_end; ++c)
-			{
-				const int next = min(c + 1, c_end - 1);
-				half8 sum_frag[MT];
-#pragma unroll
-				for (int st = 0; st < 4; ++st)
+			const auto walk = [&](int c_from, int c_to) {
+				for (int c = c_from; c < c_to; ++c)
 				{
+					const int next = min(c + 1, c_end - 1);
+					half8 sum_frag[MT];
 #pragma unroll
-					for (int s = 0; s < 4; ++s)
+					for (int st = 0; st < 4; ++st)
 					{
-						const int step = 4 * st + s, mine = s & 1, other = mine ^ 1;
-						if (s < 3)
-						{
-							read(st & 1, s + 1, other);
-						}
-						if (s == 0)
-						{
-							// (the buffer was read last before the barrier that this stage began with)
-							deposit(staged, (st + 1) & 1);
-							request(staged, st < 2 ? c : next, (st + 2) & 3);
-							if (st == 3)
-							{
-								// (a wavefront's LDS accesses keep their order: the slot's reads, the next chunk, its reads)
-								__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-								weights.deposit(moving, lane);
-								__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-								weights.request(moving, min(c + 2, c_end - 1), lane);
-							}
-						}
-						if (step == 11)
-						{
 #pragma unroll
-							for (int t = 0; t < MT; ++t)
-							{
-								sum_frag[t] = *reinterpret_cast<const half8*>(sum_tiles[t] + static_cast<size_t>(c) * kFrag);
-							}
-						}
-						if (s == 2)
+						for (int s = 0; s < 4; ++s)
 						{
-							if (st == 3)
+							const int step = 4 * st + s, mine = s & 1, other = mine ^ 1;
+							if (s < 3)
 							{
-								next_head = F::head(weights.chunk(lane), h);
+								read(buffer, s + 1, other);
 							}
-							next_raw = F::load(weights.chunk(lane), (st + 1) & 3, h, blocks_of(st < 3 ? c : next));
-						}
-						if (s == 3)
-						{
-							__syncthreads();
-							read((st + 1) & 1, 0, other);
-						}
-						__builtin_amdgcn_sched_barrier(0);
-						const half8 low = lowered(b[mine]);
-						const bool fresh = step % 8 == 0;
+							if (s == 0)
+							{
+								if (st == 2)
+								{
 #pragma unroll
-						for (int e = 0; e < 2; ++e)
-						{
-#pragma unroll
-							for (int t = 0; t < MT; ++t)
-							{
-								p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mine][t][e], e == 0 ? b[mine] : low, fresh && e == 0 ? floatx16{} : p[t], 0, 0, 0);
+									for (int t = 0; t < MT; ++t)
+									{
+										sum_frag[t] = *reinterpret_cast<const half8*>(sum_tiles[t] + static_cast<size_t>(c) * kFrag + lane_at);
+									}
+								}
+								if (st == 3)
+								{
+									// (a wavefront's LDS accesses keep their order: the slot's reads, the next chunk, its reads)
+									__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+									weights.deposit(moving, lane);
+									__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+								}
+								// (the buffer was read last before the barrier that this stage began with)
+								request(st < 2 ? c : next, (st + 2) & 3, behind(buffer, 2));
+								if (st == 3)
+								{
+									weights.request(moving, min(c + 2, c_end - 1), lane);
+								}
 							}
-						}
-						if (s < 3)
-						{
-							b[other] = F::frag(head, raw, st, s + 1);
-						}
-						else
-						{
-							b[other] = F::frag(st < 3 ? head : next_head, next_raw, (st + 1) & 3, 0);
-						}
-						if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
-						{
-#pragma unroll
-							for (int t = 0; t < MT; ++t)
+							if (s == 2)
 							{
-								held[t] = p[t];
+								if (st == 3)
+								{
+									next_head = F::head(weights.chunk(lane), h);
+								}
+								next_raw = F::load(weights.chunk(lane), (st + 1) & 3, h, blocks_of(st < 3 ? c : next));
 							}
+							if (s == 3)
+							{
+								// the wavefront's pieces of the next stage are there; behind them are those of the one after it and a chunk's blocks
+								if (st == 3)
+								{
+									arrived<kPieces + W::kLoads>();
+								}
+								else
+								{
+									arrived<kPieces>();
+								}
+								__syncthreads();
+								buffer = behind(buffer, 1);
+								read(buffer, 0, other);
+							}
+							__builtin_amdgcn_sched_barrier(0);
+							const half8 low = lowered(b[mine]);
+							const bool fresh = step % 8 == 0;
+#pragma unroll
+							for (int e = 0; e < 2; ++e)
+							{
+#pragma unroll
+								for (int t = 0; t < MT; ++t)
+								{
+									p[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[mine][t][e], e == 0 ? b[mine] : low, fresh && e == 0 ? floatx16{} : p[t], 0, 0, 0);
+								}
+							}
+							if (s < 3)
+							{
+								b[other] = F::frag(head, raw, st, s + 1);
+							}
+							else
+							{
+								b[other] = F::frag(st < 3 ? head : next_head, next_raw, (st + 1) & 3, 0);
+							}
+							if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
+							{
+#pragma unroll
+								for (int t = 0; t < MT; ++t)
+								{
+									held[t] = p[t];
+								}
+							}
+							__builtin_amdgcn_sched_barrier(0);
 						}
-						__builtin_amdgcn_sched_barrier(0);
+						raw = next_raw;
 					}
-					raw = next_raw;
+					const float d = F::chunk_scale(head);
+					const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
+					const float dm = F::min_scale(head) * (1.0f / kSumScale);
+#pragma unroll
+					for (int t = 0; t < MT; ++t)
+					{
+						const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
+						const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
+#pragma unroll
+						for (int e = 0; e < 16; ++e)
+						{
+							acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
+						}
+					}
+					head = next_head;
 				}
-				const float d = F::chunk_scale(head);
-				const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
-				const float dm = F::min_scale(head) * (1.0f / kSumScale);
+			};
+			if constexpr (KS == 1)
+			{
+				walk(0, min(half, chunks));
 #pragma unroll
 				for (int t = 0; t < MT; ++t)
 				{
-					const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
-					const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
-#pragma unroll
-					for (int e = 0; e < 16; ++e)
-					{
-						acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
-					}
+					first[t] = acc[t];
+					acc[t] = floatx16{};
 				}
-				head = next_head;
+				walk(half, chunks);
+#pragma unroll
+				for (int t = 0; t < MT; ++t)
+				{
+					acc[t] = first[t] + acc[t];
+				}
 			}
+			else
+			{
+				walk(c_begin, c_end);
+			}
+			arrived<0>(); // (nothing may arrive in LDS that is the sums' or another workgroup's)
 			// a shorter range only passes the barriers
 			for (int i = max(c_end - c_begin, 0); i < place.per; ++i)
 			{
@@ -1839,7 +1886,7 @@ namespace litenn_hip
 		template <typename F, int MT, int WN, int KS, bool ONE_RUN = WN == 1>
 		void launch_variant(const ExactCall& c)
 		{
-			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * 2 * MT * kStageBytes : 0) +
+			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * (F::kMins ? kRing : 2) * MT * kStageBytes : 0) +
 			                         static_cast<size_t>(WN) * KS * WeightPieces<F>::kSlotBytes;
 			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * MT * 64 * 64;
 			constexpr size_t lds = rings > sums ? rings : sums;
@@ -1873,8 +1920,19 @@ namespace litenn_hip
 			// forms below, at 64 rows 47 against 64.  Not for Q6_K, whose scaling per step wants the registers.
 			if constexpr (F::kScaleSteps > 1)
 			{
-				if ((strips + 3) / 4 * ((c.m_tiles + 1) / 2) >= 200 && c.m_tiles > 1)
+				const int workgroups = (strips + 3) / 4 * ((c.m_tiles + 1) / 2);
+				if (workgroups >= 200 && c.m_tiles > 1)
 				{
+					// From the 257th on in one range of K, four wavefronts each, two workgroups to a CU: one's barriers, sums and results go
+					// beside the other's products (kernel alone, us, both ranges in one workgroup of eight and one: 672 workgroups of Q5_K 139 ->
+					// 131, 448 of Q4_K 83 -> 75, 1120 217 -> 191; one to a CU they have nobody beside them: 240 47 and 49).  The same sums.
+					if constexpr (F::kMins)
+					{
+						if (workgroups > 256)
+						{
+							return launch_variant<F, 2, 4, 1>(c);
+						}
+					}
 					return launch_variant<F, 2, 4, 2>(c);
 				}
 			}

@@ -196,6 +196,19 @@ def test_forms_of_two_tiles_over_several_chunks(hip, fmt, m, n, k):
     assert errors(hip, fmt, m, n, k, residual=fmt == Q4_0).max() <= 1e-6
 
 
+@pytest.mark.parametrize("fmt", [Q4_K, Q5_K])
+@pytest.mark.parametrize("n,k", [(5185, 256), (5200, 768), (5200, 4352)])
+def test_one_range_of_k_adds_as_two(hip, fmt, n, k):
+    """More than 256 workgroups go over K in one range, fewer in two: a row's sums are the same bits."""
+    wq, x = hip.Tensor.from_numpy(synth.model_weights(fmt, n, k, 51)), synth.activations(450, k, 52)
+    run = lambda rows: hip.mul_mat_q(fmt, wq, n, k, hip.Tensor.from_numpy(rows), flags=MATMUL_PRECISE).numpy()
+    got = run(x)
+    np.testing.assert_array_equal(got[:300].view(np.uint32), run(x[:300]).view(np.uint32))
+    w = np_decoders.decode(fmt, wq.numpy().reshape(n, -1), k).astype(np.float64)
+    size = np.linalg.norm(x.astype(np.float64), axis=1) * np.linalg.norm(w) / np.sqrt(k)
+    assert (np.linalg.norm(got - x.astype(np.float64) @ w.T, axis=1) / size).max() <= 1e-6
+
+
 @pytest.mark.parametrize("fmt", FORMATS)
 @pytest.mark.parametrize("m,k", [(3, 256), (3, 4096), (45, 4096)])
 def test_several_rows_are_no_further_off_than_rows_one_by_one(hip, fmt, m, k):
