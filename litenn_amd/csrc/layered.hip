@@ -757,9 +757,10 @@ namespace litenn_hip
 			return g;
 		}
 
-		// grouped attention and state space, alone or side by side, on one token: from proj to row_mid
-		void mix_token(const LayerState& L, const Position& pos)
+		// grouped attention and state space, alone or side by side, on one token: from a row of proj to row_mid
+		void mix_token(const LayerState& L, const Position& pos, int row = 0)
 		{
+			const size_t at = static_cast<size_t>(row) * ld_proj;
 			GroupedAttn attn;
 			Ssm ssm;
 			GatedNorm norm;
@@ -770,12 +771,16 @@ namespace litenn_hip
 				{
 					a = &M;
 					attn = grouped_args(M);
+					attn.q += at;
+					attn.k += at;
+					attn.v += at;
 					attn.pos = pos;
 				}
 				else
 				{
 					b = &M;
 					ssm = ssm_args(M);
+					ssm.in += at;
 					ssm.pos = pos;
 					norm = gated_norm_args(M);
 					norm.y = row_ssm;
@@ -787,7 +792,7 @@ namespace litenn_hip
 			launch_mixer_finish(a ? &attn : nullptr, a ? a->desc.weight : 1.0f, a ? row_mid + a->at_mid : nullptr, b ? &norm : nullptr, stream);
 		}
 
-		// the same for a prompt's rows: from proj to mid, of rows `first` .. (and of some ahead of them)
+		// the same for a prompt's rows: from proj to mid, of rows `first` .. (and of some ahead of them; of none where first == rows)
 		void mix_rows(const LayerState& L, int rows, int first, int past, const Position& pos)
 		{
 			const size_t operand = f32 ? 4 : 2;
@@ -806,7 +811,7 @@ namespace litenn_hip
 					a.pos = pos;
 					a.q_from = first;
 					w = grouped_window(a, past);
-					const int from = first / kAttnRows * kAttnRows;
+					const int from = first < rows ? first / kAttnRows * kAttnRows : rows;
 					w.q += static_cast<size_t>(from) * w.ldq;
 					w.q_base += from;
 					w.rows -= from;
@@ -1058,8 +1063,13 @@ namespace litenn_hip
 				// percent.)  The row's error against 64 bits falls by 10 to 30 %: its operands are not rounded.
 				const int n = &L == &layers.back() ? logit_rows : rows, first = rows - n;
 				const bool one = n == 1;
+				// One row's attention and recurrence are a step behind a prompt that is a row shorter: a prompt's kernels have a few
+				// workgroups for it, each a chain over all keys or a chunk.  us of both and the part norms, 500 tokens of 2048-wide
+				// layers in 32 bits 53 -> 20 (and 15 -> 7 of the product of up to 32 rows that attention would want), 777 in 16 bits
+				// 28 -> 19.
+				const bool stepped = one && rows > 1 && (M.desc.kind == MixerKind::GroupedAttention || M.desc.kind == MixerKind::StateSpace);
 				// (attention in 32 bits takes a few rows the slower the fewer they are, and looks at what comes out of all of them)
-				const bool by_step = M.desc.kind == MixerKind::LatentAttention && latent_by_step(M, n, past + rows);
+				const bool by_step = stepped || (M.desc.kind == MixerKind::LatentAttention && latent_by_step(M, n, past + rows));
 				const int asked = f32 && !by_step ? first / kAttnRows * kAttnRows : first;
 				enter(L.norm1, 0, rows);
 				OneRow row{ *this, x + static_cast<size_t>(first) * desc.width, 0 };
@@ -1100,14 +1110,26 @@ namespace litenn_hip
 					g.chunk_states = chunk_states;
 					launch_gla_rows(g, stream);
 				}
+				else if (stepped)
+				{
+					mix_rows(L, first, first, past, pos);
+					mix_token(L, Position{ pos.dev, pos.add + first }, first);
+				}
 				else
 				{
 					mix_rows(L, rows, asked, past, pos);
 				}
 				if (one)
 				{
-					const void* const from = operand_row(mid, first, ld_mid);
-					row.leave(L.out, static_cast<const float*>(f32 ? from : nullptr), L.norm1b, static_cast<const uint16_t*>(f32 ? nullptr : from));
+					if (stepped)
+					{
+						row.leave(L.out, row_mid, L.norm1b);
+					}
+					else
+					{
+						const void* const from = operand_row(mid, first, ld_mid);
+						row.leave(L.out, static_cast<const float*>(f32 ? from : nullptr), L.norm1b, static_cast<const uint16_t*>(f32 ? nullptr : from));
+					}
 					row.feed_forward(L);
 					row.logits(logits);
 					return;
