@@ -23,7 +23,8 @@ namespace litenn_hip
 	bool launch_exact_few(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y, const float* residual,
 	                      hipStream_t stream);
 	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
-	                       const float* residual, const void* scratch, hipStream_t stream);
+	                       const float* residual, const void* scratch, float* partial, size_t partial_floats, hipStream_t stream);
+	size_t exact_partial_floats(int fmt, size_t n, size_t k, size_t m);
 	bool launch_gemm(int fmt, const void* wq, size_t n, size_t k, const float* x, size_t m, float* y,
 	                 const float* residual, void* scratch_halves, float* partial, size_t partial_floats,
 	                 hipStream_t stream);
@@ -904,7 +905,14 @@ extern "C" int litenn_hip_mul_mat_q_ws(int dev, int fmt, const void* wq, size_t 
 		const size_t need = exact_scratch_bytes(m, k);
 		StreamScratch scratch(s);
 		void* room = workspace && workspace_bytes >= need ? workspace : nullptr;
-		if (!workspace && scratch.allocate(need) == hipSuccess)
+		// (and for the sums of ranges of K, behind them, where the memory is this call's)
+		const size_t need16 = (need + 15) / 16 * 16;
+		size_t sums = workspace ? 0 : exact_partial_floats(fmt, n, k, m);
+		if (sums && scratch.allocate(need16 + sizeof(float) * sums) == hipSuccess)
+		{
+			room = scratch.get();
+		}
+		else if (sums = 0; !workspace && scratch.allocate(need) == hipSuccess)
 		{
 			room = scratch.get();
 		}
@@ -914,7 +922,7 @@ extern "C" int litenn_hip_mul_mat_q_ws(int dev, int fmt, const void* wq, size_t 
 		}
 		if (room && launch_exact_rows(xf, m, k, nullptr, 0.0, nullptr, room, s))
 		{
-			launch_exact_gemm(fmt, 1, &wq, &n, k, m, &yf, rf, room, s);
+			launch_exact_gemm(fmt, 1, &wq, &n, k, m, &yf, rf, room, sums ? reinterpret_cast<float*>(static_cast<char*>(room) + need16) : nullptr, sums, s);
 			if (scratch.blocking())
 			{
 				const hipError_t launched = hipGetLastError();

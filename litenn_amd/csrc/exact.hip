@@ -804,17 +804,24 @@ namespace litenn_hip
 		template <typename F, int MT, int WN, int KS>
 		__global__ __launch_bounds__(64 * WN * KS, 2) void exact_shared_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                    const float* residual, int k, int m, int m_tiles,
-		                                                                    int chunks, size_t row_bytes)
+		                                                                    int chunks, size_t row_bytes, int flush, size_t range_stride)
 		{
-			static_assert(F::kMins && F::kScaleSteps == 16, "one scale for a chunk, minima beside it");
+			constexpr bool kScaled = F::kScaleSteps < 16; // sums of kScaleSteps steps are scaled and added to the chunk's
+			static_assert(kScaled != F::kMins, "one scale for a chunk has minima beside it");
 			constexpr int kPieces = MT * 8 / WN; // 1 KB pieces a wavefront stages
 			static_assert(kPieces * WN == MT * 8, "activation pieces / wavefront split");
 			typedef WeightPieces<F> W;
 			constexpr int kBuffer = MT * kStageBytes, kRingBytes = KS * kRing * kBuffer;
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][kRing][MT][stage], [WN KS][slot]; later the KS sums
-			const ExactPlace<F, MT, WN, KS> place(mats, chunks);
+			ExactPlace<F, MT, WN, KS> place(mats, chunks);
 			const int lane = place.lane, h = lane >> 5;
-			const int c_begin = place.c_begin, c_end = place.c_end, half = (chunks + 1) / 2;
+			if constexpr (KS == 1)
+			{
+				const int per = (chunks + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
+				place.c_begin = static_cast<int>(blockIdx.z) * per, place.c_end = min(place.c_begin + per, chunks);
+				place.y += blockIdx.z * range_stride;
+			}
+			const int c_begin = place.c_begin, c_end = place.c_end;
 			const W weights(lds + kRingBytes + (place.part * WN + place.wv) * W::kSlotBytes, place.w, place.n_base, place.n, row_bytes);
 			u32x4 moving[W::kLoads];
 
@@ -827,8 +834,9 @@ namespace litenn_hip
 			}
 
 			floatx16 acc[MT], p[MT];
-			floatx16 held[MT]; // the chunk's first half
-			floatx16 first[KS == 1 ? MT : 1]; // one range: the sums of its first half, added at the end as a range's are
+			floatx16 held[MT]; // the chunk's first half; kScaled: its sum so far
+			constexpr bool kFlushed = KS == 1 || kScaled; // every `flush` chunks' sums go to a sum of their own
+			floatx16 total[kFlushed ? MT : 1];
 #pragma unroll
 			for (int t = 0; t < MT; ++t)
 			{
@@ -913,7 +921,7 @@ namespace litenn_hip
 							}
 							if (s == 0)
 							{
-								if (st == 2)
+								if (F::kMins && st == 2)
 								{
 #pragma unroll
 									for (int t = 0; t < MT; ++t)
@@ -960,7 +968,7 @@ namespace litenn_hip
 							}
 							__builtin_amdgcn_sched_barrier(0);
 							const half8 low = lowered(b[mine]);
-							const bool fresh = step % 8 == 0;
+							const bool fresh = step % (kScaled ? F::kScaleSteps : 8) == 0;
 #pragma unroll
 							for (int e = 0; e < 2; ++e)
 							{
@@ -978,7 +986,23 @@ namespace litenn_hip
 							{
 								b[other] = F::frag(st < 3 ? head : next_head, next_raw, (st + 1) & 3, 0);
 							}
-							if (step == 7) // (two sums of eight steps each: a shorter chain rounds less)
+							if constexpr (kScaled)
+							{
+								if (step % F::kScaleSteps == F::kScaleSteps - 1)
+								{
+									const float d = F::scale(head, raw, st, s);
+#pragma unroll
+									for (int t = 0; t < MT; ++t)
+									{
+#pragma unroll
+										for (int e = 0; e < 16; ++e)
+										{
+											held[t][e] = step == F::kScaleSteps - 1 ? d * p[t][e] : fmaf(d, p[t][e], held[t][e]);
+										}
+									}
+								}
+							}
+							if (F::kMins && step == 7) // (two sums of eight steps each: a shorter chain rounds less)
 							{
 #pragma unroll
 								for (int t = 0; t < MT; ++t)
@@ -991,36 +1015,58 @@ namespace litenn_hip
 						raw = next_raw;
 					}
 					const float d = F::chunk_scale(head);
-					const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
-					const float dm = F::min_scale(head) * (1.0f / kSumScale);
-#pragma unroll
-					for (int t = 0; t < MT; ++t)
+					if constexpr (F::kMins)
 					{
-						const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
-						const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
+						const half8 centres = for_sums(F::centre_frag(head), h), minima = for_sums(F::min_frag(head), h);
+						const float dm = F::min_scale(head) * (1.0f / kSumScale);
 #pragma unroll
-						for (int e = 0; e < 16; ++e)
+						for (int t = 0; t < MT; ++t)
 						{
-							acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
+							const floatx16 ce = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], centres, floatx16{}, 0, 0, 0);
+							const floatx16 mi = __builtin_amdgcn_mfma_f32_32x32x16_f16(sum_frag[t], minima, floatx16{}, 0, 0, 0);
+#pragma unroll
+							for (int e = 0; e < 16; ++e)
+							{
+								acc[t][e] += fmaf(d, held[t][e] + p[t][e], fmaf(d, ce[e], dm * mi[e]));
+							}
+						}
+					}
+					else
+					{
+#pragma unroll
+						for (int t = 0; t < MT; ++t)
+						{
+#pragma unroll
+							for (int e = 0; e < 16; ++e)
+							{
+								acc[t][e] = fmaf(d, held[t][e], acc[t][e]);
+							}
 						}
 					}
 					head = next_head;
 				}
 			};
-			if constexpr (KS == 1)
+			if constexpr (kFlushed)
 			{
-				walk(0, min(half, chunks));
 #pragma unroll
 				for (int t = 0; t < MT; ++t)
 				{
-					first[t] = acc[t];
-					acc[t] = floatx16{};
+					total[t] = floatx16{};
 				}
-				walk(half, chunks);
+				for (int c = c_begin; c < c_end; c += flush)
+				{
+					walk(c, min(c + flush, c_end));
+#pragma unroll
+					for (int t = 0; t < MT; ++t)
+					{
+						total[t] += acc[t];
+						acc[t] = floatx16{};
+					}
+				}
 #pragma unroll
 				for (int t = 0; t < MT; ++t)
 				{
-					acc[t] = first[t] + acc[t];
+					acc[t] = total[t];
 				}
 			}
 			else
@@ -1029,7 +1075,7 @@ namespace litenn_hip
 			}
 			arrived<0>(); // (nothing may arrive in LDS that is the sums' or another workgroup's)
 			// a shorter range only passes the barriers
-			for (int i = max(c_end - c_begin, 0); i < place.per; ++i)
+			for (int i = max(c_end - c_begin, 0); KS > 1 && i < place.per; ++i)
 			{
 #pragma unroll
 				for (int st = 0; st < 4; ++st)
@@ -1291,6 +1337,51 @@ namespace litenn_hip
 			}
 
 			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes);
+		}
+
+		// y_i = sum over `ranges` of from_i (+ residual), in double, rounded once; four elements a thread, one matrix a grid row.  Bound by
+		// its bytes and the launch: three ranges of 300 x 4096 in 7 us.
+		constexpr int kMostRanges = 16;
+		__global__ __launch_bounds__(256) void add_ranges_kernel(const ExactMats to, const ExactMats from, int ranges, size_t stride,
+		                                                         const float* residual, int m)
+		{
+			const int which = blockIdx.y;
+			const size_t count = static_cast<size_t>(m) * to.n[which], at = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+			const float* const part = from.y[which];
+			float* const y = to.y[which];
+			if (at + 4 <= count)
+			{
+				floatx4 v[kMostRanges];
+#pragma unroll
+				for (int i = 0; i < kMostRanges; ++i)
+				{
+					v[i] = i < ranges ? *reinterpret_cast<const floatx4_a4*>(part + i * stride + at) : floatx4{};
+				}
+				const floatx4 res = residual ? *reinterpret_cast<const floatx4_a4*>(residual + at) : floatx4{};
+				floatx4 out;
+#pragma unroll
+				for (int e = 0; e < 4; ++e)
+				{
+					double sum = static_cast<double>(v[0][e]);
+#pragma unroll
+					for (int i = 1; i < kMostRanges; ++i)
+					{
+						sum += static_cast<double>(v[i][e]);
+					}
+					out[e] = static_cast<float>(sum + static_cast<double>(res[e]));
+				}
+				*reinterpret_cast<floatx4_a4*>(y + at) = out;
+				return;
+			}
+			for (size_t e = at; e < count; ++e)
+			{
+				double sum = residual ? static_cast<double>(residual[e]) : 0.0;
+				for (int i = 0; i < ranges; ++i)
+				{
+					sum += static_cast<double>(part[i * stride + e]);
+				}
+				y[e] = static_cast<float>(sum);
+			}
 		}
 
 		// ---- few rows: up to MR activation rows, one launch, no scratch ---------------------------------
@@ -1866,33 +1957,15 @@ namespace litenn_hip
 			int k, m, m_tiles, chunks;
 			size_t row_bytes;
 			hipStream_t stream;
+			float* partial; // room for the sums of K's ranges, or null
+			size_t partial_floats;
 		};
 
-		// Four wavefronts over one chunk's scale have the registers to hold two steps' operands (Q4_K 28672 x 4096 at 300 rows 253
-		// -> 238 us); sums that are scaled every step or two have not.
-		template <typename F, int MT, int WN, int KS, bool ONE_RUN>
-		constexpr auto variant()
+		// the matrices, `rows` weight rows a workgroup, side by side in grid x
+		ExactMats grid_mats(const ExactCall& c, int rows, int& blocks)
 		{
-			if constexpr (WN > 1 && F::kMins)
-			{
-				return &exact_shared_kernel<F, MT, WN, KS>;
-			}
-			else
-			{
-				return &exact_gemm_kernel<F, MT, WN, KS, ONE_RUN>;
-			}
-		}
-
-		template <typename F, int MT, int WN, int KS, bool ONE_RUN = WN == 1>
-		void launch_variant(const ExactCall& c)
-		{
-			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * (F::kMins ? kRing : 2) * MT * kStageBytes : 0) +
-			                         static_cast<size_t>(WN) * KS * WeightPieces<F>::kSlotBytes;
-			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * MT * 64 * 64;
-			constexpr size_t lds = rings > sums ? rings : sums;
-			static_assert(lds <= 160 * 1024, "LDS");
 			ExactMats mats{};
-			int blocks = 0;
+			blocks = 0;
 			for (int i = 0; i < 3; ++i)
 			{
 				mats.first_block[i] = 0x7fffffff;
@@ -1902,44 +1975,154 @@ namespace litenn_hip
 					mats.y[i] = c.y[i];
 					mats.n[i] = c.n[i];
 					mats.first_block[i] = blocks;
-					blocks += (c.n[i] + WN * kTile - 1) / (WN * kTile);
+					blocks += (c.n[i] + rows - 1) / rows;
 				}
 			}
-			const auto kernel = variant<F, MT, WN, KS, ONE_RUN>();
+			return mats;
+		}
+
+		template <typename F, int MT, int WN, int KS, bool ONE_RUN = WN == 1>
+		void launch_variant(const ExactCall& c)
+		{
+			constexpr size_t rings = (WN > 1 ? static_cast<size_t>(KS) * 2 * MT * kStageBytes : 0) +
+			                         static_cast<size_t>(WN) * KS * WeightPieces<F>::kSlotBytes;
+			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * MT * 64 * 64;
+			constexpr size_t lds = rings > sums ? rings : sums;
+			static_assert(lds <= 160 * 1024, "LDS");
+			int blocks;
+			const ExactMats mats = grid_mats(c, WN * kTile, blocks);
+			const auto kernel = &exact_gemm_kernel<F, MT, WN, KS, ONE_RUN>;
 			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
 			kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
 			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
+		}
+
+		// `ranges` of K in grid z, none of them empty, leave their sums in c.partial, from where a launch more adds them
+		template <typename F, int KS>
+		void launch_shared(const ExactCall& c, int flush, int ranges = 1)
+		{
+			constexpr int MT = 2, WN = 4;
+			constexpr size_t rings = static_cast<size_t>(KS) * kRing * MT * kStageBytes + static_cast<size_t>(WN) * KS * WeightPieces<F>::kSlotBytes;
+			constexpr size_t sums = static_cast<size_t>(KS - 1) * WN * MT * 64 * 64;
+			constexpr size_t lds = rings > sums ? rings : sums;
+			static_assert(lds <= (KS == 1 ? 80 : 160) * 1024, "LDS");
+			int blocks;
+			ExactMats mats = grid_mats(c, WN * kTile, blocks);
+			const ExactMats out = mats;
+			const size_t stride = static_cast<size_t>(c.m) * c.total_rows;
+			if (ranges > 1)
+			{
+				size_t at = 0;
+				for (int i = 0; i < c.count; ++i)
+				{
+					mats.y[i] = c.partial + at;
+					at += static_cast<size_t>(c.m) * c.n[i];
+				}
+			}
+			constexpr auto kernel = &exact_shared_kernel<F, MT, WN, KS>;
+			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
+			kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT, ranges), dim3(64 * WN * KS), lds, c.stream>>>(
+			    mats, c.xs, ranges > 1 ? nullptr : c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, stride);
+			if (ranges > 1)
+			{
+				const size_t widest = static_cast<size_t>(c.m) * *std::max_element(c.n, c.n + c.count);
+				add_ranges_kernel<<<dim3(static_cast<unsigned>((widest + 1023) / 1024), c.count), dim3(256), 0, c.stream>>>(out, mats, ranges, stride, c.residual, c.m);
+			}
+		}
+
+		// Formats whose weights' slots leave a CU room for two workgroups of the shared form.  (Q4_0 takes fewer bytes, but its sums,
+		// scaled every other step, spill registers there: 104 -> 288 us.)
+		template <typename F>
+		constexpr bool kShares = F::kMins || F::kScaleSteps == 1;
+
+		// Ranges of K for the shared form with grid z, 1 where it does not pay: as many as leave every workgroup its place on the card,
+		// two to a CU.
+		template <typename F>
+		int exact_ranges(int strips, int m_tiles, int chunks)
+		{
+			const int workgroups = (strips + 3) / 4 * ((m_tiles + 1) / 2), most = std::min({ 512 / std::max(workgroups, 1), chunks, kMostRanges });
+			if (most < 2 || m_tiles < 2)
+			{
+				return 1;
+			}
+			const int per = (chunks + most - 1) / most;
+			// Q6_K, us of a call by the forms below and by this (K = 4096, by workgroups: 64 28 and 32, 96 46 and 43, 112 50 and 46, 160
+			// 76 and 59, 240 101 and 74; K = 14336: 64 69 and 70, 96 118 and 99, 128 126 and 115, 160 186 and 147; K = 1024, 128 24 and 27).
+			if constexpr (F::kScaleSteps == 1)
+			{
+				return workgroups >= 80 && chunks >= 16 ? (chunks + per - 1) / per : 1;
+			}
+			// Q4_K and Q5_K, below the 200 workgroups that have a form for themselves: tenths of a us fitted to 40 calls (K = 4096, by
+			// tiles of 32 x 32: 768 34 and 36, 896 44 and 37 or 42 and 40, 960 43 and 46, 1280 55 and 50; K = 14336: 512 70 and 58, 896 129
+			// and 94, 1280 175 and 122; K = 1024, 1280 23 and 29).
+			else
+			{
+				const long long other = 272ll * strips * m_tiles * chunks / 10000, ranged = 210 + 44 * per;
+				return workgroups < 200 && ranged < other ? (chunks + per - 1) / per : 1;
+			}
+		}
+
+		// Chunks that a range of `per` adds up before they join its sum: those for which the roundings, each as large as what has been
+		// summed by then, come to least
+		int chunks_a_sum(int per)
+		{
+			int best = 1;
+			long long least = -1;
+			for (int count = 1; count <= per; ++count)
+			{
+				long long sizes = 0;
+				for (int from = 0; from < per; from += count)
+				{
+					const long long here = std::min(count, per - from);
+					sizes += here * (here + 1) / 2 + (from ? from + here : 0);
+				}
+				if (least < 0 || sizes < least)
+				{
+					least = sizes, best = count;
+				}
+			}
+			return best;
 		}
 
 		template <typename F>
 		void launch_exact_format(const ExactCall& c)
 		{
 			const int strips = (c.total_rows + kTile - 1) / kTile, units = strips * c.m_tiles;
+			const int workgroups = (strips + 3) / 4 * ((c.m_tiles + 1) / 2);
 			// Where 128 x 64 tiles give most CUs a workgroup, four wavefronts share the activations and each decoded weight meets two
 			// tiles (us, kernel alone, weights from HBM, here and below): Q4_K 28672 x 4096 at 300 rows 226 against 313 of the
-			// forms below, at 64 rows 47 against 64.  Not for Q6_K, whose scaling per step wants the registers.
-			if constexpr (F::kScaleSteps > 1)
+			// forms below, at 64 rows 47 against 64; and from there on in one range of K, four wavefronts each, two workgroups to a CU:
+			// one's barriers, sums and results go beside the other's products (672 workgroups of Q5_K 139 -> 131, 448 of Q4_K 83 -> 75,
+			// 1120 217 -> 191; one to a CU they have nobody beside them: 240 47 and 49).  The same sums.
+			if constexpr (kShares<F>)
 			{
-				const int workgroups = (strips + 3) / 4 * ((c.m_tiles + 1) / 2);
+				const int ranges = exact_ranges<F>(strips, c.m_tiles, c.chunks);
+				if (ranges > 1 && static_cast<size_t>(ranges) * c.m * c.total_rows <= c.partial_floats)
+				{
+					return launch_shared<F, 1>(c, chunks_a_sum((c.chunks + ranges - 1) / ranges), ranges);
+				}
+			}
+			if constexpr (F::kMins)
+			{
 				if (workgroups >= 200 && c.m_tiles > 1)
 				{
-					// From the 257th on in one range of K, four wavefronts each, two workgroups to a CU: one's barriers, sums and results go
-					// beside the other's products (kernel alone, us, both ranges in one workgroup of eight and one: 672 workgroups of Q5_K 139 ->
-					// 131, 448 of Q4_K 83 -> 75, 1120 217 -> 191; one to a CU they have nobody beside them: 240 47 and 49).  The same sums.
-					if constexpr (F::kMins)
-					{
-						if (workgroups > 256)
-						{
-							return launch_variant<F, 2, 4, 1>(c);
-						}
-					}
+					return workgroups > 256 ? launch_shared<F, 1>(c, (c.chunks + 1) / 2) : launch_shared<F, 2>(c, c.chunks);
+				}
+			}
+			else if constexpr (F::kScaleSteps > 1)
+			{
+				if (workgroups >= 200 && c.m_tiles > 1)
+				{
 					return launch_variant<F, 2, 4, 2>(c);
 				}
 			}
 			// Otherwise a wavefront keeps to itself and the ranges of K fill the card, in Q6_K with two tiles where these are enough.
-			else if (fetch::exact_two_tiles(strips, c.m_tiles))
+			if constexpr (F::kScaleSteps == 1)
 			{
-				return launch_variant<F, 2, 1, 8>(c);
+				if (fetch::exact_two_tiles(strips, c.m_tiles))
+				{
+					return launch_variant<F, 2, 1, 8>(c);
+				}
 			}
 			// Eight ranges while there are few tiles (Q6_K 4096 x 14336 at 45 rows 41 against 46 with four, at 16 43 against 47), four
 			// from there on (Q4_K 14336 x 4096 at 45 rows 37 against 44 with eight, at 16 equal) and for short rows (Q8_0 1024 x 1024 at
@@ -2076,12 +2259,43 @@ namespace litenn_hip
 		return true;
 	}
 
+	// floats that launch_exact_gemm would leave sums of ranges of K in (0: it takes K in one)
+	size_t exact_partial_floats(int fmt, size_t n, size_t k, size_t m)
+	{
+		const int strips = static_cast<int>((n + kTile - 1) / kTile), tiles = static_cast<int>((m + kTile - 1) / kTile);
+		const int chunks = static_cast<int>((k + kChunk - 1) / kChunk);
+		int ranges = 1;
+		switch (fmt)
+		{
+		case LITENN_FMT_Q4_K: ranges = exact_ranges<Q4_KX>(strips, tiles, chunks); break;
+		case LITENN_FMT_Q5_K: ranges = exact_ranges<Q5_KX>(strips, tiles, chunks); break;
+		case LITENN_FMT_Q6_K: ranges = exact_ranges<Q6_KX>(strips, tiles, chunks); break;
+		default: break;
+		}
+		return ranges > 1 ? static_cast<size_t>(ranges) * m * n : 0;
+	}
+
+	// the same for any number of rows up to m
+	size_t exact_most_partial_floats(int fmt, size_t n, size_t k, size_t m)
+	{
+		size_t most = 0;
+		// (beyond 256 workgroups of 128 x 64 results there are no ranges)
+		const size_t blocks = (n + 4 * kTile - 1) / (4 * kTile), last = std::min(m, 64 * (256 / std::max<size_t>(blocks, 1)));
+		for (size_t rows = std::min<size_t>(kTile, last); rows <= last && rows; rows = rows < last ? std::min(rows + kTile, last) : last + 1)
+		{
+			most = std::max(most, exact_partial_floats(fmt, n, k, rows));
+		}
+		return most;
+	}
+
 	// y_i[M, n_i] = X' . deq(W_i)^T (+ residual, which may alias y; single matrix) for up to three matrices of
-	// one format over rows that launch_exact_rows has taken apart.
+	// one format over rows that launch_exact_rows has taken apart.  partial: room for sums of ranges of K, or null.
 	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
-	                       const float* residual, const void* scratch, hipStream_t stream)
+	                       const float* residual, const void* scratch, float* partial, size_t partial_floats, hipStream_t stream)
 	{
 		ExactCall c{};
+		c.partial = partial;
+		c.partial_floats = partial ? partial_floats : 0;
 		c.count = count;
 		for (int i = 0; i < count; ++i)
 		{

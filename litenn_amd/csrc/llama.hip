@@ -27,7 +27,8 @@ namespace litenn_hip
 	bool launch_exact_rows(const float* x, size_t m, size_t k, const float* norm_w, double eps, const float* up,
 	                       void* scratch, hipStream_t stream);
 	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
-	                       const float* residual, const void* scratch, hipStream_t stream);
+	                       const float* residual, const void* scratch, float* partial, size_t partial_floats, hipStream_t stream);
+	size_t exact_most_partial_floats(int fmt, size_t n, size_t k, size_t m);
 	bool launch_gemm_group(int fmt, int count, const void* const* wq, const size_t* n, size_t k, const float* x,
 	                       size_t m, float* const* y, const float* residual, const float* norm_w, double eps,
 	                       const float* up, void* scratch_halves, float* partial, size_t partial_floats,
@@ -116,6 +117,7 @@ struct litenn_hip_llama : litenn_hip_model
 	size_t xn_floats = 0; // what xn holds (rows x embedding_length, three times that for short prompts)
 	void* xh = nullptr; // a matmul's activations as the matrix cores take them (multi-row path)
 	size_t xh_halves = 0; // its size
+	size_t summed_rows = 0, sum_floats = 0; // rows that sum_floats was found for: what matmuls of up to so many leave sums of ranges of K in
 	// single-row attention: key chunks per head, their meeting place and arrival counters
 	size_t attn_splits = 1;
 	float* attn_partial = nullptr;
@@ -159,10 +161,39 @@ namespace
 		m->cap_rows = 0;
 	}
 
+	// floats that the model's matmuls of up to `rows` rows with Float32 operands leave sums of ranges of K in
+	size_t ranges_sums(const litenn_hip_llama* m, size_t rows)
+	{
+		size_t most = 0;
+		const Layer* before = nullptr;
+		const auto alike = [](const Weight& a, const Weight& b) { return a.fmt == b.fmt && a.n == b.n && a.k == b.k; };
+		const auto look_at = [&](const Weight& w, size_t n) { most = std::max(most, exact_most_partial_floats(w.fmt, n, w.k, rows)); };
+		for (const Layer& L : m->layers)
+		{
+			if (!before || !alike(L.wq, before->wq) || !alike(L.wk, before->wk) || !alike(L.wv, before->wv) || !alike(L.wo, before->wo) ||
+			    !alike(L.gate, before->gate) || !alike(L.up, before->up) || !alike(L.down, before->down))
+			{
+				// (matrices of one format share a launch)
+				for (const Weight* w : { &L.wq, &L.wk, &L.wv, &L.wo, &L.gate, &L.up, &L.down })
+				{
+					look_at(*w, w->n);
+				}
+				look_at(L.wq, L.wq.n + L.wk.n);
+				look_at(L.wk, L.wk.n + L.wv.n);
+				look_at(L.wq, L.wq.n + L.wk.n + L.wv.n);
+				look_at(L.gate, L.gate.n + L.up.n);
+			}
+			before = &L;
+		}
+		const Weight& head = m->output.data ? m->output : m->tok_embd;
+		look_at(head, head.n);
+		return most;
+	}
+
 	// Halves that the rows of the model's matmuls take on their way to the matrix cores: rounded to fp16 (q/k/v projections in
 	// two formats share a launch that wants them in both fragment orders), or, for matrices that meet Float32
-	// operands, taken apart into two halves each.
-	size_t matmul_halves(const litenn_hip_llama* m, size_t rows, unsigned flags)
+	// operands, taken apart into two halves each and, behind them, sums of ranges of K.
+	size_t matmul_halves(litenn_hip_llama* m, size_t rows, unsigned flags)
 	{
 		const size_t d = m->p.embedding_length, ff = m->p.feed_forward_length;
 		const size_t qw = static_cast<size_t>(m->p.head_count) * m->head_dim;
@@ -182,7 +213,13 @@ namespace
 			}
 		}
 		const size_t rounded = std::max(gemm_scratch_halves(rows, std::max({ d, qw, ff })), 2 * gemm_scratch_halves(rows, d));
-		return widest ? std::max(rounded, (exact_scratch_bytes(rows, widest) + 1) / 2) : rounded;
+		if ((flags & LITENN_HIP_MATMUL_PRECISE) && m->summed_rows != rows)
+		{
+			m->sum_floats = ranges_sums(m, rows);
+			m->summed_rows = rows;
+		}
+		const size_t sums = flags & LITENN_HIP_MATMUL_PRECISE ? 2 * m->sum_floats + 128 : 0; // (behind the rows, on 256 bytes)
+		return widest ? std::max(rounded, (exact_scratch_bytes(rows, widest) + 1) / 2 + sums) : rounded;
 	}
 
 	int ensure_scratch(litenn_hip_llama* m, size_t rows, unsigned flags)
@@ -275,6 +312,8 @@ namespace
 		{
 			return false;
 		}
+		const size_t rows_end = (exact_scratch_bytes(rows, k) + 255) / 256 * 256;
+		const size_t room = 2 * m->xh_halves > rows_end ? (2 * m->xh_halves - rows_end) / sizeof(float) : 0;
 		for (int i = 0; i < count;)
 		{
 			const void* w[3];
@@ -285,7 +324,8 @@ namespace
 				w[j - i] = ws[j]->data;
 				n[j - i] = ws[j]->n;
 			}
-			launch_exact_gemm(ws[i]->fmt, j - i, w, n, k, rows, ys + i, residual, m->xh, s);
+			launch_exact_gemm(ws[i]->fmt, j - i, w, n, k, rows, ys + i, residual, m->xh,
+			                  room ? reinterpret_cast<float*>(static_cast<char*>(m->xh) + rows_end) : nullptr, room, s);
 			i = j;
 		}
 		return true;

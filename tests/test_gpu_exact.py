@@ -196,6 +196,31 @@ def test_forms_of_two_tiles_over_several_chunks(hip, fmt, m, n, k):
     assert errors(hip, fmt, m, n, k, residual=fmt == Q4_0).max() <= 1e-6
 
 
+# workgroups of 128 x 64 results on both sides of what pays, ranges that are not all alike, a last row and strip of their own
+RANGED = [(Q6_K, 300, 2049, 4352), (Q6_K, 257, 2048, 4096), (Q6_K, 33, 10241, 4096), (Q6_K, 70, 16300, 4096), (Q6_K, 100, 4096, 14336),
+          (Q4_K, 300, 3300, 7168), (Q5_K, 129, 4097, 7424), (Q4_K, 40, 14336, 4096), (Q5_K, 64, 4000, 14336)]
+
+
+@pytest.mark.parametrize("fmt,m,n,k", RANGED)
+def test_ranges_of_k_whose_sums_a_launch_more_adds(hip, fmt, m, n, k):
+    """In the call's own memory; a caller's workspace has no room for them."""
+    assert errors(hip, fmt, m, n, k, residual=m % 2 == 1).max() <= 1e-6
+
+
+@pytest.mark.parametrize("fmt,m,n,k", RANGED[4:8])
+def test_infinite_activations_in_ranges_of_k(hip, fmt, m, n, k):
+    wq, x = hip.Tensor.from_numpy(synth.model_weights(fmt, n, k, 61)), synth.activations(m, k, 62)
+    run = lambda rows: hip.mul_mat_q(fmt, wq, n, k, hip.Tensor.from_numpy(rows), flags=MATMUL_PRECISE).numpy()
+    clean = run(x)
+    x[3, 5], x[4, k - 1], x[m - 1, k // 2] = np.inf, -np.inf, np.nan
+    got = run(x)
+    assert np.isnan(got[m - 1]).all() and not np.isfinite(got[3:5]).any()
+    for row in (3, 4) if fmt == Q4_K else ():  # (one row of the others may take an infinity off an infinite sum)
+        np.testing.assert_array_equal(got[row], run(x[row:row + 1])[0])
+    rest = [i for i in range(m) if i not in (3, 4, m - 1)]
+    np.testing.assert_array_equal(got[rest], clean[rest])
+
+
 @pytest.mark.parametrize("fmt", [Q4_K, Q5_K])
 @pytest.mark.parametrize("n,k", [(5185, 256), (5200, 768), (5200, 4352)])
 def test_one_range_of_k_adds_as_two(hip, fmt, n, k):
