@@ -18,12 +18,11 @@
 // Against 64 bits the result is closer than the streaming kernel's in every format and form (relative L2 over K = 256 ..
 // 14336, mean of six inputs, 0.7e-7 to 1.2e-7; the streaming kernel 0.9e-7 to 2.5e-7).
 //
-// What bounds it: few rows are the weights' stream and the launch; many rows, the LDS reads of the fragments (two
-// per pair of products) and the latency in front of them: a product issues every 100 cycles and SIMD where
-// it takes 32.  Row by row through the streaming kernel the same calls took, us, before -> now with the rows'
-// pre-pass: Q6_K 4096 x 14336 at 45 rows 571 -> 43; 8B-shape prompt of 300 tokens, two blocks 28100 -> 1310.
+// What bounds it: few rows are the weights' stream and the launch; many rows, no unit alone (the forms below say more).  Row by
+// row through the streaming kernel the same calls took, us, before -> now with the rows' pre-pass: Q6_K 4096 x 14336 at 45 rows
+// 571 -> 43; 8B-shape prompt of 300 tokens, two blocks 28100 -> 650.
 //
-// v_mfma_f32_32x32x16_f16 throughout: D[i][j] += A[i][k] B[k][j] with the activations as A and the
+// v_mfma_f32_32x32x16_f16 but for few rows: D[i][j] += A[i][k] B[k][j] with the activations as A and the
 // weights as B, so that a lane's sixteen results belong to one weight row, whose scale the lane holds.
 #include "common.hpp"
 #include "fetch_model.hpp"
@@ -794,8 +793,10 @@ namespace litenn_hip
 		// its own products and decodes its weights behind them, and a stage's last products follow the barrier, so that they cover
 		// the next stage's first reads.
 		// KS = 1 walks both halves of K one after the other and adds them as the two ranges of KS = 2 are added.
-		// Bound by the waits around a barrier per stage (matrix cores 36 % busy, VALU 35, LDS 30).  us, kernel alone, Q4_K 28672 x
-		// 4096 at 300 rows: stages through registers and two buffers 221, ring 216, KS = 1 with two workgroups to a CU 190.
+		// Bound by no unit alone (matrix cores 38 % busy, VALU 39, LDS 26; 18 % of a wavefront's time are waits for operands and barriers)
+		// and by a last round of few workgroups.  us, kernel alone, Q4_K 28672 x 4096 at 300 rows: stages through registers and two
+		// buffers 221, ring 216, KS = 1 with two workgroups to a CU 190; Q6_K 4096 x 14336, by two tiles a wavefront on their own 172,
+		// here in three ranges 130 and 5 for adding them.
 		constexpr int kRing = 3; // stages: one is multiplied, two are on their way
 		// all but the N youngest of the wavefront's loads are there
 		template <int N>
@@ -1340,7 +1341,7 @@ namespace litenn_hip
 		}
 
 		// y_i = sum over `ranges` of from_i (+ residual), in double, rounded once; four elements a thread, one matrix a grid row.  Bound by
-		// its bytes and the launch: three ranges of 300 x 4096 in 7 us.
+		// its bytes and the launch: three ranges of 300 x 4096 in 5.3 us.
 		constexpr int kMostRanges = 16;
 		__global__ __launch_bounds__(256) void add_ranges_kernel(const ExactMats to, const ExactMats from, int ranges, size_t stride,
 		                                                         const float* residual, int m)
