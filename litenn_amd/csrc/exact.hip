@@ -2036,12 +2036,63 @@ namespace litenn_hip
 		template <typename F>
 		constexpr bool kShares = F::kMins || F::kScaleSteps == 1;
 
-		// Ranges of K for the shared form with grid z, 1 where it does not pay: as many as leave every workgroup its place on the card,
-		// two to a CU.
+		// Chunks that a range of `per` adds up before they join its sum: those for which the roundings, each as large as what has been
+		// summed by then, come to least
+		struct SumLength
+		{
+			int chunks;
+			long long roundings;
+		};
+		SumLength chunks_a_sum(int per)
+		{
+			SumLength best{ 1, -1 };
+			for (int count = 1; count <= per; ++count)
+			{
+				long long sizes = 0;
+				for (int from = 0; from < per; from += count)
+				{
+					const long long here = std::min(count, per - from);
+					sizes += here * (here + 1) / 2 + (from ? from + here : 0);
+				}
+				if (best.roundings < 0 || sizes < best.roundings)
+				{
+					best = { count, sizes };
+				}
+			}
+			return best;
+		}
+
+		constexpr size_t kMostRangedTiles = size_t{ 1 } << 17; // of 32 x 32 sums, all ranges together
+
+		// Ranges of K for the shared form with grid z, 1 where it does not pay: up to 256 workgroups as many as leave every one its place
+		// on the card, two to a CU.
 		template <typename F>
 		int exact_ranges(int strips, int m_tiles, int chunks)
 		{
 			const int workgroups = (strips + 3) / 4 * ((m_tiles + 1) / 2), most = std::min({ 512 / std::max(workgroups, 1), chunks, kMostRanges });
+			// Q6_K on more workgroups: as few ranges as round no more than the eight of the form below, whose wavefronts each read their
+			// activations from L2 (us of a call by that and by this: 4096 x 14336 at 700 rows 385 and 321, 1000 598 and 415, 2000 2051 and
+			// 848, 8192 x 4096 at 300 rows 124 and 103, 14336 x 4096 207 and 155), up to 512 MB of sums.
+			if constexpr (F::kScaleSteps == 1)
+			{
+				if (workgroups > 256 && chunks >= 16)
+				{
+					const long long r = (chunks + 7) / 8;
+					for (int ranges = 2; ranges <= 4; ++ranges)
+					{
+						const int each = (chunks + ranges - 1) / ranges;
+						if (static_cast<long long>(ranges) * strips * m_tiles > static_cast<long long>(kMostRangedTiles))
+						{
+							return 1;
+						}
+						if (ranges * chunks_a_sum(each).roundings + chunks <= 4 * r * (r + 1) + 3 * chunks)
+						{
+							return (chunks + each - 1) / each;
+						}
+					}
+					return 1;
+				}
+			}
 			if (most < 2 || m_tiles < 2)
 			{
 				return 1;
@@ -2063,28 +2114,6 @@ namespace litenn_hip
 			}
 		}
 
-		// Chunks that a range of `per` adds up before they join its sum: those for which the roundings, each as large as what has been
-		// summed by then, come to least
-		int chunks_a_sum(int per)
-		{
-			int best = 1;
-			long long least = -1;
-			for (int count = 1; count <= per; ++count)
-			{
-				long long sizes = 0;
-				for (int from = 0; from < per; from += count)
-				{
-					const long long here = std::min(count, per - from);
-					sizes += here * (here + 1) / 2 + (from ? from + here : 0);
-				}
-				if (least < 0 || sizes < least)
-				{
-					least = sizes, best = count;
-				}
-			}
-			return best;
-		}
-
 		template <typename F>
 		void launch_exact_format(const ExactCall& c)
 		{
@@ -2100,7 +2129,7 @@ namespace litenn_hip
 				const int ranges = exact_ranges<F>(strips, c.m_tiles, c.chunks);
 				if (ranges > 1 && static_cast<size_t>(ranges) * c.m * c.total_rows <= c.partial_floats)
 				{
-					return launch_shared<F, 1>(c, chunks_a_sum((c.chunks + ranges - 1) / ranges), ranges);
+					return launch_shared<F, 1>(c, chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
 				}
 			}
 			if constexpr (F::kMins)
@@ -2280,7 +2309,13 @@ namespace litenn_hip
 	size_t exact_most_partial_floats(int fmt, size_t n, size_t k, size_t m)
 	{
 		size_t most = 0;
-		// (beyond 256 workgroups of 128 x 64 results there are no ranges)
+		const size_t strips = (n + kTile - 1) / kTile;
+		// beyond 256 workgroups of 128 x 64 results there is one number of ranges, and they take most at most rows
+		for (int ranges = 2; ranges <= 4; ++ranges)
+		{
+			most = std::max(most, exact_partial_floats(fmt, n, k, std::min(m, kTile * (kMostRangedTiles / (ranges * strips)))));
+		}
+		// up to there every number of tiles has its own
 		const size_t blocks = (n + 4 * kTile - 1) / (4 * kTile), last = std::min(m, 64 * (256 / std::max<size_t>(blocks, 1)));
 		for (size_t rows = std::min<size_t>(kTile, last); rows <= last && rows; rows = rows < last ? std::min(rows + kTile, last) : last + 1)
 		{

@@ -198,7 +198,8 @@ def test_forms_of_two_tiles_over_several_chunks(hip, fmt, m, n, k):
 
 # workgroups of 128 x 64 results on both sides of what pays, ranges that are not all alike, a last row and strip of their own
 RANGED = [(Q6_K, 300, 2049, 4352), (Q6_K, 257, 2048, 4096), (Q6_K, 33, 10241, 4096), (Q6_K, 70, 16300, 4096), (Q6_K, 100, 4096, 14336),
-          (Q4_K, 300, 3300, 7168), (Q5_K, 129, 4097, 7424), (Q4_K, 40, 14336, 4096), (Q5_K, 64, 4000, 14336)]
+          (Q4_K, 300, 3300, 7168), (Q5_K, 129, 4097, 7424), (Q4_K, 40, 14336, 4096), (Q5_K, 64, 4000, 14336),
+          (Q6_K, 300, 8193, 4096), (Q6_K, 520, 4100, 4352), (Q6_K, 700, 2049, 8448)]
 
 
 @pytest.mark.parametrize("fmt,m,n,k", RANGED)
