@@ -670,9 +670,10 @@ namespace litenn_hip
 				c_begin = part * per, c_end = min(c_begin + per, chunks);
 			}
 
-			// the sums of all ranges, scaled, go out; every wavefront of the workgroup calls it
+			// The sums of all ranges, scaled, go out (not `scaled`: those of one range of several, to which a launch more sees: times
+			// a row's factor a range's sum may overflow where the result does not); every wavefront of the workgroup calls it
 			__device__ __forceinline__ void finish(floatx16 (&acc)[MT], uint8_t* lds, const uint8_t* xs, const RowsLayout& at, const float* residual,
-			                                       int m, int chunks, size_t row_bytes) const
+			                                       int m, int chunks, size_t row_bytes, bool scaled = true) const
 			{
 				const int r = lane & 31, h = lane >> 5;
 				if constexpr (KS > 1)
@@ -739,7 +740,7 @@ namespace litenn_hip
 #pragma unroll
 					for (int e = 0; e < 16; e += 4)
 					{
-						us[e / 4] = *reinterpret_cast<const floatx4*>(factors + first + 2 * e);
+						us[e / 4] = scaled ? *reinterpret_cast<const floatx4*>(factors + first + 2 * e) : floatx4{ 1.0f, 1.0f, 1.0f, 1.0f };
 					}
 					if (residual)
 					{
@@ -775,7 +776,7 @@ namespace litenn_hip
 						const int i = __ffs(again) - 1, e = i & 15, mm = (mt_base + (i >> 4)) * kTile + 8 * (e / 4) + 4 * h + (e & 3);
 						again &= again - 1;
 						const uint8_t* const parts = xs + static_cast<size_t>(mm / kTile) * chunks * kTileChunkBytes + (mm % kTile) * 16;
-						const float v = factors[mm] * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
+						const float v = (scaled ? factors[mm] : 1.0f) * plain_dot<F>(w + static_cast<size_t>(col) * row_bytes, chunks, [&](int i) {
 							const uint8_t* const at = parts + static_cast<size_t>(i >> 4) * (2 * kFrag) + ((i >> 3) & 1) * 512 + (i & 7) * 2;
 							return fmaf(static_cast<float>(*reinterpret_cast<const _Float16*>(at + kFrag)), kLowScale, static_cast<float>(*reinterpret_cast<const _Float16*>(at)));
 						});
@@ -1084,7 +1085,7 @@ namespace litenn_hip
 					__syncthreads();
 				}
 			}
-			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes);
+			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes, KS > 1 || gridDim.z == 1);
 		}
 
 		// The same with less held ahead.  WN > 1: the fragments pass through the same two buffers, two stages on their way; with WN =
@@ -1340,23 +1341,26 @@ namespace litenn_hip
 			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes);
 		}
 
-		// y_i = sum over `ranges` of from_i (+ residual), in double, rounded once; four elements a thread, one matrix a grid row.  Bound by
-		// its bytes and the launch: three ranges of 300 x 4096 in 5.3 us.
+		// y_i = factor of the row times the sum over `ranges` of from_i (+ residual), in double, rounded once.  A workgroup takes 1024
+		// elements of a row (grid x) of one matrix (grid z), four a thread.  Bound by its bytes and the launch: three ranges of 300 x 4096
+		// in 5.3 us.
 		constexpr int kMostRanges = 16;
 		__global__ __launch_bounds__(256) void add_ranges_kernel(const ExactMats to, const ExactMats from, int ranges, size_t stride,
-		                                                         const float* residual, int m)
+		                                                         const float* __restrict__ factors, const float* residual)
 		{
-			const int which = blockIdx.y;
-			const size_t count = static_cast<size_t>(m) * to.n[which], at = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
-			const float* const part = from.y[which];
-			float* const y = to.y[which];
-			if (at + 4 <= count)
+			const int row = blockIdx.x, which = blockIdx.z, n = to.n[which];
+			const int column = (static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x)) * 4;
+			const size_t at = static_cast<size_t>(row) * n + column;
+			const float* const part = from.y[which] + at;
+			float* const y = to.y[which] + at;
+			const double factor = static_cast<double>(factors[row]);
+			if (column + 4 <= n)
 			{
 				floatx4 v[kMostRanges];
 #pragma unroll
 				for (int i = 0; i < kMostRanges; ++i)
 				{
-					v[i] = i < ranges ? *reinterpret_cast<const floatx4_a4*>(part + i * stride + at) : floatx4{};
+					v[i] = i < ranges ? *reinterpret_cast<const floatx4_a4*>(part + i * stride) : floatx4{};
 				}
 				const floatx4 res = residual ? *reinterpret_cast<const floatx4_a4*>(residual + at) : floatx4{};
 				floatx4 out;
@@ -1369,19 +1373,19 @@ namespace litenn_hip
 					{
 						sum += static_cast<double>(v[i][e]);
 					}
-					out[e] = static_cast<float>(sum + static_cast<double>(res[e]));
+					out[e] = static_cast<float>(fma(sum, factor, static_cast<double>(res[e])));
 				}
-				*reinterpret_cast<floatx4_a4*>(y + at) = out;
+				*reinterpret_cast<floatx4_a4*>(y) = out;
 				return;
 			}
-			for (size_t e = at; e < count; ++e)
+			for (int e = 0; column + e < n; ++e)
 			{
-				double sum = residual ? static_cast<double>(residual[e]) : 0.0;
+				double sum = 0.0;
 				for (int i = 0; i < ranges; ++i)
 				{
 					sum += static_cast<double>(part[i * stride + e]);
 				}
-				y[e] = static_cast<float>(sum);
+				y[e] = static_cast<float>(fma(sum, factor, residual ? static_cast<double>(residual[at + e]) : 0.0));
 			}
 		}
 
@@ -2026,8 +2030,9 @@ namespace litenn_hip
 			    mats, c.xs, ranges > 1 ? nullptr : c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, stride);
 			if (ranges > 1)
 			{
-				const size_t widest = static_cast<size_t>(c.m) * *std::max_element(c.n, c.n + c.count);
-				add_ranges_kernel<<<dim3(static_cast<unsigned>((widest + 1023) / 1024), c.count), dim3(256), 0, c.stream>>>(out, mats, ranges, stride, c.residual, c.m);
+				const unsigned widest = static_cast<unsigned>(*std::max_element(c.n, c.n + c.count));
+				add_ranges_kernel<<<dim3(c.m, (widest + 1023) / 1024, c.count), dim3(256), 0, c.stream>>>(
+				    out, mats, ranges, stride, reinterpret_cast<const float*>(c.xs + RowsLayout(c.m_tiles, c.chunks).factors), c.residual);
 			}
 		}
 

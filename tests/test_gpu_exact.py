@@ -208,6 +208,27 @@ def test_ranges_of_k_whose_sums_a_launch_more_adds(hip, fmt, m, n, k):
     assert errors(hip, fmt, m, n, k, residual=m % 2 == 1).max() <= 1e-6
 
 
+@pytest.mark.parametrize("fmt,m,n,k", [(Q4_K, 300, 3301, 7168), (Q5_K, 129, 4097, 7424), (Q6_K, 100, 8195, 4096), (Q6_K, 520, 4101, 4352)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_ranges_of_k_whose_sums_alone_leave_float32(hip, fmt, m, n, k, residual):
+    """Sums of ranges beyond Float32's largest value whose sum is not, and sums among its subnormal ones, which are rounded
+    once: to half of 2^-149."""
+    wq, x = hip.Tensor.from_numpy(synth.model_weights(fmt, n, k, 61)), synth.activations(m, k, 62)
+    x[0] = np.sign(x[0]) * np.float32(3e38)
+    x[1] *= np.float32(1e-38)
+    add = synth.activations(m, n, 63) if residual else np.zeros((m, n), np.float32)
+    add[1] *= np.float32(1e-38)
+    got = hip.mul_mat_q(fmt, wq, n, k, hip.Tensor.from_numpy(x), residual=hip.Tensor.from_numpy(add) if residual else None, flags=MATMUL_PRECISE).numpy()
+    w = np_decoders.decode(fmt, wq.numpy().reshape(n, -1), k).astype(np.float64)
+    want = x[:2].astype(np.float64) @ w.T + add[:2]
+    size = np.linalg.norm(x[:2].astype(np.float64), axis=1)[:, None] * np.linalg.norm(w, axis=1)
+    top = float(np.finfo(np.float32).max)
+    fits = np.abs(want[0]) + 1e-6 * size[0] < top
+    assert 0.5 < fits.mean() < 0.99
+    assert (np.abs(got[0] - want[0]) <= 1e-6 * size[0])[fits].all()
+    assert (np.abs(got[1] - want[1]) <= 1e-6 * size[1] + 2.0 ** -150).all()
+
+
 @pytest.mark.parametrize("fmt,m,n,k", RANGED[4:8])
 def test_infinite_activations_in_ranges_of_k(hip, fmt, m, n, k):
     wq, x = hip.Tensor.from_numpy(synth.model_weights(fmt, n, k, 61)), synth.activations(m, k, 62)
