@@ -1344,7 +1344,7 @@ namespace litenn_hip
 		// y_i = factor of the row times the sum over `ranges` of from_i (+ residual), in double, rounded once.  A workgroup takes 1024
 		// elements of a row (grid x) of one matrix (grid z), four a thread.  Bound by its bytes and the launch: three ranges of 300 x 4096
 		// in 5.3 us.
-		constexpr int kMostRanges = 16;
+		constexpr int kMostRanges = fetch::kMostRanges;
 		__global__ __launch_bounds__(256) void add_ranges_kernel(const ExactMats to, const ExactMats from, int ranges, size_t stride,
 		                                                         const float* __restrict__ factors, const float* residual)
 		{
@@ -2041,82 +2041,11 @@ namespace litenn_hip
 		template <typename F>
 		constexpr bool kShares = F::kMins || F::kScaleSteps == 1;
 
-		// Chunks that a range of `per` adds up before they join its sum: those for which the roundings, each as large as what has been
-		// summed by then, come to least
-		struct SumLength
-		{
-			int chunks;
-			long long roundings;
-		};
-		SumLength chunks_a_sum(int per)
-		{
-			SumLength best{ 1, -1 };
-			for (int count = 1; count <= per; ++count)
-			{
-				long long sizes = 0;
-				for (int from = 0; from < per; from += count)
-				{
-					const long long here = std::min(count, per - from);
-					sizes += here * (here + 1) / 2 + (from ? from + here : 0);
-				}
-				if (best.roundings < 0 || sizes < best.roundings)
-				{
-					best = { count, sizes };
-				}
-			}
-			return best;
-		}
-
-		constexpr size_t kMostRangedTiles = size_t{ 1 } << 17; // of 32 x 32 sums, all ranges together
-
-		// Ranges of K for the shared form with grid z, 1 where it does not pay: up to 256 workgroups as many as leave every one its place
-		// on the card, two to a CU.
+		// as fetch::exact_ranges, for the formats that take the form with ranges
 		template <typename F>
 		int exact_ranges(int strips, int m_tiles, int chunks)
 		{
-			const int workgroups = (strips + 3) / 4 * ((m_tiles + 1) / 2), most = std::min({ 512 / std::max(workgroups, 1), chunks, kMostRanges });
-			// Q6_K on more workgroups: as few ranges as round no more than the eight of the form below, whose wavefronts each read their
-			// activations from L2 (us of a call by that and by this: 4096 x 14336 at 700 rows 385 and 321, 1000 598 and 415, 2000 2051 and
-			// 848, 8192 x 4096 at 300 rows 124 and 103, 14336 x 4096 207 and 155), up to 512 MB of sums.
-			if constexpr (F::kScaleSteps == 1)
-			{
-				if (workgroups > 256 && chunks >= 16)
-				{
-					const long long r = (chunks + 7) / 8;
-					for (int ranges = 2; ranges <= 4; ++ranges)
-					{
-						const int each = (chunks + ranges - 1) / ranges;
-						if (static_cast<long long>(ranges) * strips * m_tiles > static_cast<long long>(kMostRangedTiles))
-						{
-							return 1;
-						}
-						if (ranges * chunks_a_sum(each).roundings + chunks <= 4 * r * (r + 1) + 3 * chunks)
-						{
-							return (chunks + each - 1) / each;
-						}
-					}
-					return 1;
-				}
-			}
-			if (most < 2 || m_tiles < 2)
-			{
-				return 1;
-			}
-			const int per = (chunks + most - 1) / most;
-			// Q6_K, us of a call by the forms below and by this (K = 4096, by workgroups: 64 28 and 32, 96 46 and 43, 112 50 and 46, 160
-			// 76 and 59, 240 101 and 74; K = 14336: 64 69 and 70, 96 118 and 99, 128 126 and 115, 160 186 and 147; K = 1024, 128 24 and 27).
-			if constexpr (F::kScaleSteps == 1)
-			{
-				return workgroups >= 80 && chunks >= 16 ? (chunks + per - 1) / per : 1;
-			}
-			// Q4_K and Q5_K, below the 200 workgroups that have a form for themselves: tenths of a us fitted to 40 calls (K = 4096, by
-			// tiles of 32 x 32: 768 34 and 36, 896 44 and 37 or 42 and 40, 960 43 and 46, 1280 55 and 50; K = 14336: 512 70 and 58, 896 129
-			// and 94, 1280 175 and 122; K = 1024, 1280 23 and 29).
-			else
-			{
-				const long long other = 272ll * strips * m_tiles * chunks / 10000, ranged = 210 + 44 * per;
-				return workgroups < 200 && ranged < other ? (chunks + per - 1) / per : 1;
-			}
+			return fetch::exact_ranges(F::kScaleSteps == 1, strips, m_tiles, chunks);
 		}
 
 		template <typename F>
@@ -2134,7 +2063,7 @@ namespace litenn_hip
 				const int ranges = exact_ranges<F>(strips, c.m_tiles, c.chunks);
 				if (ranges > 1 && static_cast<size_t>(ranges) * c.m * c.total_rows <= c.partial_floats)
 				{
-					return launch_shared<F, 1>(c, chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
+					return launch_shared<F, 1>(c, fetch::chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
 				}
 			}
 			if constexpr (F::kMins)
@@ -2318,7 +2247,7 @@ namespace litenn_hip
 		// beyond 256 workgroups of 128 x 64 results there is one number of ranges, and they take most at most rows
 		for (int ranges = 2; ranges <= 4; ++ranges)
 		{
-			most = std::max(most, exact_partial_floats(fmt, n, k, std::min(m, kTile * (kMostRangedTiles / (ranges * strips)))));
+			most = std::max(most, exact_partial_floats(fmt, n, k, std::min(m, kTile * (fetch::kMostRangedTiles / (ranges * strips)))));
 		}
 		// up to there every number of tiles has its own
 		const size_t blocks = (n + 4 * kTile - 1) / (4 * kTile), last = std::min(m, 64 * (256 / std::max<size_t>(blocks, 1)));

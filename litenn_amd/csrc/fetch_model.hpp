@@ -38,6 +38,85 @@ namespace litenn_hip
 			return m_tiles > 1 && (ones >= 512 || (ones > 256 && twos <= 256));
 		}
 
+		// Chunks that a range of `per` adds up before they join its sum: those for which the roundings, each as large as what has been
+		// summed by then, come to least
+		struct SumLength
+		{
+			int chunks;
+			long long roundings;
+		};
+		inline SumLength chunks_a_sum(int per)
+		{
+			SumLength best{ 1, -1 };
+			for (int count = 1; count <= per; ++count)
+			{
+				long long sizes = 0;
+				for (int from = 0; from < per; from += count)
+				{
+					const long long here = imin(count, per - from);
+					sizes += here * (here + 1) / 2 + (from ? from + here : 0);
+				}
+				if (best.roundings < 0 || sizes < best.roundings)
+				{
+					best = { count, sizes };
+				}
+			}
+			return best;
+		}
+
+		constexpr int kMostRanges = 16;
+		constexpr size_t kMostRangedTiles = size_t{ 1 } << 17; // of 32 x 32 sums, all ranges together
+
+		// Ranges of K for the form that shares activations, with grid z, 1 where it does not pay: up to 256 workgroups of 128 x 64 results
+		// as many as leave every one its place on the card, two to a CU.  by_step: Q6_K, whose steps are scaled one by one (other
+		// formats that take the form, Q4_K and Q5_K, scale chunks).
+		inline int exact_ranges(bool by_step, int strips, int m_tiles, int chunks)
+		{
+			const int workgroups = (strips + 3) / 4 * ((m_tiles + 1) / 2), most = imin(imin(512 / imax(workgroups, 1), chunks), kMostRanges);
+			// One tile of activations leaves the second half of its 64 rows empty: us of a call of Q6_K at 32 rows by the forms without
+			// ranges and by this, 32800 x 4096 75 and 98, 128256 x 4096 221 and 255, at 9 rows 72 and 92, 212 and 226.
+			if (m_tiles < 2)
+			{
+				return 1;
+			}
+			// Q6_K on more workgroups: as few ranges as round no more than the eight of the form without, whose wavefronts each read their
+			// activations from L2 (us of a call by that and by this: 4096 x 14336 at 700 rows 385 and 321, 1000 598 and 415, 2000 2051 and
+			// 848, 8192 x 4096 at 300 rows 124 and 103, 14336 x 4096 207 and 155), up to 512 MB of sums.
+			if (by_step && workgroups > 256 && chunks >= 16)
+			{
+				const long long r = (chunks + 7) / 8;
+				for (int ranges = 2; ranges <= 4; ++ranges)
+				{
+					const int each = (chunks + ranges - 1) / ranges;
+					if (static_cast<long long>(ranges) * strips * m_tiles > static_cast<long long>(kMostRangedTiles))
+					{
+						return 1;
+					}
+					if (ranges * chunks_a_sum(each).roundings + chunks <= 4 * r * (r + 1) + 3 * chunks)
+					{
+						return (chunks + each - 1) / each;
+					}
+				}
+				return 1;
+			}
+			if (most < 2)
+			{
+				return 1;
+			}
+			const int per = (chunks + most - 1) / most;
+			// Q6_K, us of a call by the forms without ranges and by this (K = 4096, by workgroups: 64 28 and 32, 96 46 and 43, 112 50 and 46,
+			// 160 76 and 59, 240 101 and 74; K = 14336: 64 69 and 70, 96 118 and 99, 128 126 and 115, 160 186 and 147; K = 1024, 128 24 and 27).
+			if (by_step)
+			{
+				return workgroups >= 80 && chunks >= 16 ? (chunks + per - 1) / per : 1;
+			}
+			// Q4_K and Q5_K, below the 200 workgroups that have a form for themselves: tenths of a us fitted to 40 calls (K = 4096, by
+			// tiles of 32 x 32: 768 34 and 36, 896 44 and 37 or 42 and 40, 960 43 and 46, 1280 55 and 50; K = 14336: 512 70 and 58, 896 129
+			// and 94, 1280 175 and 122; K = 1024, 1280 23 and 29).
+			const long long other = 272ll * strips * m_tiles * chunks / 10000, ranged = 210 + 44 * per;
+			return workgroups < 200 && ranged < other ? (chunks + per - 1) / per : 1;
+		}
+
 		// ---- attention of many rows: what a block of 32 query rows sees ---------------------------
 		struct RowsSeen
 		{

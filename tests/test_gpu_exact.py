@@ -229,6 +229,12 @@ def test_ranges_of_k_whose_sums_alone_leave_float32(hip, fmt, m, n, k, residual)
     assert (np.abs(got[1] - want[1]) <= 1e-6 * size[1] + 2.0 ** -150).all()
 
 
+@pytest.mark.parametrize("m", [9, 32, 33])
+def test_many_weight_rows_meet_one_tile_of_activations(hip, m):
+    """More workgroups of 128 x 64 results than CUs: up to 32 rows leave half of each empty and take the form without ranges of K."""
+    assert errors(hip, Q6_K, m, 32801, 4096).max() <= 1e-6
+
+
 @pytest.mark.parametrize("fmt,m,n,k", RANGED[4:8])
 def test_infinite_activations_in_ranges_of_k(hip, fmt, m, n, k):
     wq, x = hip.Tensor.from_numpy(synth.model_weights(fmt, n, k, 61)), synth.activations(m, k, 62)
