@@ -2041,13 +2041,6 @@ namespace litenn_hip
 		template <typename F>
 		constexpr bool kShares = F::kMins || F::kScaleSteps == 1;
 
-		// as fetch::exact_ranges, for the formats that take the form with ranges
-		template <typename F>
-		int exact_ranges(int strips, int m_tiles, int chunks)
-		{
-			return fetch::exact_ranges(F::kScaleSteps == 1, strips, m_tiles, chunks);
-		}
-
 		template <typename F>
 		void launch_exact_format(const ExactCall& c)
 		{
@@ -2060,7 +2053,7 @@ namespace litenn_hip
 			// 1120 217 -> 191; one to a CU they have nobody beside them: 240 47 and 49).  The same sums.
 			if constexpr (kShares<F>)
 			{
-				const int ranges = exact_ranges<F>(strips, c.m_tiles, c.chunks);
+				const int ranges = fetch::exact_ranges(F::kScaleSteps == 1, c.total_rows, c.m, c.chunks);
 				if (ranges > 1 && static_cast<size_t>(ranges) * c.m * c.total_rows <= c.partial_floats)
 				{
 					return launch_shared<F, 1>(c, fetch::chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
@@ -2223,19 +2216,18 @@ namespace litenn_hip
 		return true;
 	}
 
-	// floats that launch_exact_gemm would leave sums of ranges of K in (0: it takes K in one)
+	// ranges of K that launch_exact_gemm leaves sums of, where it has room for them
+	static int exact_ranges(int fmt, size_t n, size_t k, size_t m)
+	{
+		return fmt == LITENN_FMT_Q4_K || fmt == LITENN_FMT_Q5_K || fmt == LITENN_FMT_Q6_K
+		           ? fetch::exact_ranges(fmt == LITENN_FMT_Q6_K, static_cast<int>(n), static_cast<int>(m), static_cast<int>((k + kChunk - 1) / kChunk))
+		           : 1;
+	}
+
+	// floats that it leaves them in (0: it takes K in one)
 	size_t exact_partial_floats(int fmt, size_t n, size_t k, size_t m)
 	{
-		const int strips = static_cast<int>((n + kTile - 1) / kTile), tiles = static_cast<int>((m + kTile - 1) / kTile);
-		const int chunks = static_cast<int>((k + kChunk - 1) / kChunk);
-		int ranges = 1;
-		switch (fmt)
-		{
-		case LITENN_FMT_Q4_K: ranges = exact_ranges<Q4_KX>(strips, tiles, chunks); break;
-		case LITENN_FMT_Q5_K: ranges = exact_ranges<Q5_KX>(strips, tiles, chunks); break;
-		case LITENN_FMT_Q6_K: ranges = exact_ranges<Q6_KX>(strips, tiles, chunks); break;
-		default: break;
-		}
+		const int ranges = exact_ranges(fmt, n, k, m);
 		return ranges > 1 ? static_cast<size_t>(ranges) * m * n : 0;
 	}
 
@@ -2249,11 +2241,12 @@ namespace litenn_hip
 		{
 			most = std::max(most, exact_partial_floats(fmt, n, k, std::min(m, kTile * (fetch::kMostRangedTiles / (ranges * strips)))));
 		}
-		// up to there every number of tiles has its own
+		// up to there every number of tiles has its own, and the fewer rows it holds the sooner they pay
 		const size_t blocks = (n + 4 * kTile - 1) / (4 * kTile), last = std::min(m, 64 * (256 / std::max<size_t>(blocks, 1)));
-		for (size_t rows = std::min<size_t>(kTile, last); rows <= last && rows; rows = rows < last ? std::min(rows + kTile, last) : last + 1)
+		for (size_t first = 1; first <= last; first += kTile)
 		{
-			most = std::max(most, exact_partial_floats(fmt, n, k, rows));
+			const int ranges = exact_ranges(fmt, n, k, first);
+			most = std::max(most, ranges > 1 ? static_cast<size_t>(ranges) * std::min(m, first + kTile - 1) * n : 0);
 		}
 		return most;
 	}

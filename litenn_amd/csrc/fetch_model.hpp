@@ -70,8 +70,9 @@ namespace litenn_hip
 		// Ranges of K for the form that shares activations, with grid z, 1 where it does not pay: up to 256 workgroups of 128 x 64 results
 		// as many as leave every one its place on the card, two to a CU.  by_step: Q6_K, whose steps are scaled one by one (other
 		// formats that take the form, Q4_K and Q5_K, scale chunks).
-		inline int exact_ranges(bool by_step, int strips, int m_tiles, int chunks)
+		inline int exact_ranges(bool by_step, int n, int m, int chunks)
 		{
+			const int strips = (n + 31) / 32, m_tiles = (m + 31) / 32, tiles = strips * m_tiles;
 			const int workgroups = (strips + 3) / 4 * ((m_tiles + 1) / 2), most = imin(imin(512 / imax(workgroups, 1), chunks), kMostRanges);
 			// One tile of activations leaves the second half of its 64 rows empty: us of a call of Q6_K at 32 rows by the forms without
 			// ranges and by this, 32800 x 4096 75 and 98, 128256 x 4096 221 and 255, at 9 rows 72 and 92, 212 and 226.
@@ -88,7 +89,7 @@ namespace litenn_hip
 				for (int ranges = 2; ranges <= 4; ++ranges)
 				{
 					const int each = (chunks + ranges - 1) / ranges;
-					if (static_cast<long long>(ranges) * strips * m_tiles > static_cast<long long>(kMostRangedTiles))
+					if (static_cast<long long>(ranges) * tiles > static_cast<long long>(kMostRangedTiles))
 					{
 						return 1;
 					}
@@ -103,18 +104,24 @@ namespace litenn_hip
 			{
 				return 1;
 			}
-			const int per = (chunks + most - 1) / most;
+			const int per = (chunks + most - 1) / most, ranges = (chunks + per - 1) / per;
 			// Q6_K, us of a call by the forms without ranges and by this (K = 4096, by workgroups: 64 28 and 32, 96 46 and 43, 112 50 and 46,
-			// 160 76 and 59, 240 101 and 74; K = 14336: 64 69 and 70, 96 118 and 99, 128 126 and 115, 160 186 and 147; K = 1024, 128 24 and 27).
+			// 160 76 and 59, 240 101 and 74; K = 14336: 64 69 and 70, 96 118 and 99, 128 126 and 115, 160 186 and 147; K = 1024, 128 24 and
+			// 27).  Not where up to 512 single tiles are all on the card at once, though 80 workgroups have a third of their rows empty
+			// (5120 x 4096 at 65 to 96 rows 31 and 38, x 7168 44 and 50, x 14336 79 and 82; at 128 48 and 40, 70 and 52, 125 and 87).
 			if (by_step)
 			{
-				return workgroups >= 80 && chunks >= 16 ? (chunks + per - 1) / per : 1;
+				return workgroups >= 80 && chunks >= 16 && tiles > 512 ? ranges : 1;
 			}
-			// Q4_K and Q5_K, below the 200 workgroups that have a form for themselves: tenths of a us fitted to 40 calls (K = 4096, by
-			// tiles of 32 x 32: 768 34 and 36, 896 44 and 37 or 42 and 40, 960 43 and 46, 1280 55 and 50; K = 14336: 512 70 and 58, 896 129
-			// and 94, 1280 175 and 122; K = 1024, 1280 23 and 29).
-			const long long other = 272ll * strips * m_tiles * chunks / 10000, ranged = 210 + 44 * per;
-			return workgroups < 200 && ranged < other ? (chunks + per - 1) / per : 1;
+			// Q4_K and Q5_K, below the 200 workgroups that have a form for themselves, in tenths of a us.  Without ranges tiles of 32 x 32 go
+			// through the card 256 at a time; with them every workgroup has its chunks, and what they leave is written and read (fitted to
+			// 214 calls, of which none is 2 % slower by the form this takes: K = 4096, by tiles: 768 34 and 36, 896 44 and 37 or 42 and 40, 960
+			// 43 and 46, 1280 55 and 50; K = 14336: 256 of 33 rows 38.5 and 37.7, of 64 40 and 41, Q5_K 41 and 44, 480 63 and 66, 512 66 and
+			// 58, 896 129 and 94, 1280 175 and 122; K = 7168: 512 38 and 40, 768 54 and 50 or 51 and 53; K = 1024, 1280 23 and 29).
+			// The first line is an older fit, which keeps calls off that the second was not fitted to.
+			const bool worth = 210 + 44 * per < 272ll * tiles * chunks / 10000;
+			const long long ranged = 155 + 44 * per + 19ll * ranges * m * n / 1000000, plain = 135 + 45 * chunks * ((tiles + 255) / 256) / 10;
+			return workgroups < 200 && worth && ranged < plain ? ranges : 1;
 		}
 
 		// ---- attention of many rows: what a block of 32 query rows sees ---------------------------

@@ -958,10 +958,17 @@ static void test_exact_ranges()
 	const Measured measured[] = {
 		{ true, 32800, 4096, 9, 72.5, 91.8 }, { true, 32800, 4096, 16, 72.5, 92.6 }, { true, 32800, 4096, 32, 74.8, 97.8 }, { true, 128256, 4096, 9, 211.5, 225.8 },
 		{ true, 128256, 4096, 16, 214.4, 232.6 }, { true, 128256, 4096, 32, 221.1, 253.9 }, { true, 128256, 4096, 64, 373.3, 275.7 },
+		{ false, 4096, 4096, 300, 55.7, 50.8 }, { false, 4096, 14336, 33, 39.1, 37.9 }, { false, 4096, 14336, 64, 40.3, 41.4 }, { false, 4096, 14336, 65, 60.2, 52.2 }, { false, 4096, 14336, 300, 159.7, 115.4 },
+		{ false, 14336, 4096, 64, 40.3, 39.6 }, { false, 4096, 14336, 33, 40.6, 39.8 }, { false, 4096, 14336, 64, 41.7, 44.3 }, { true, 4096, 4096, 300, 73.4, 58.7 }, { true, 14336, 4096, 33, 47.5, 44.5 },
+		{ false, 2048, 14336, 128, 41.9, 42.8 }, { false, 3072, 11008, 160, 54.1, 55.4 }, { false, 3072, 14336, 160, 66.1, 62.2 }, { false, 5120, 14336, 64, 59.7, 46.3 }, { false, 5120, 14336, 90, 63.0, 66.0 },
+		{ false, 5120, 14336, 128, 89.1, 68.6 }, { false, 6144, 7168, 160, 64.9, 64.8 }, { false, 8192, 4096, 192, 58.2, 55.2 }, { false, 8192, 7168, 64, 38.2, 40.2 }, { false, 8192, 7168, 90, 51.3, 53.4 },
+		{ false, 8192, 7168, 128, 65.0, 55.2 }, { false, 8192, 7168, 192, 93.3, 80.8 }, { false, 11008, 7168, 33, 49.0, 43.3 }, { false, 2048, 14336, 128, 43.5, 44.6 }, { false, 5120, 14336, 90, 67.3, 70.4 },
+		{ false, 8192, 4096, 192, 62.3, 57.9 }, { false, 8192, 7168, 64, 40.7, 42.1 }, { true, 5120, 4096, 65, 31.0, 37.9 }, { true, 5120, 4096, 90, 31.3, 38.5 }, { true, 5120, 4096, 128, 47.9, 39.5 },
+		{ true, 5120, 7168, 90, 44.9, 50.7 }, { true, 5120, 7168, 128, 69.9, 52.0 }, { true, 5120, 14336, 65, 78.7, 81.9 }, { true, 6144, 4096, 65, 46.8, 43.5 }, { true, 8192, 7168, 65, 68.4, 61.7 },
 	};
 	for (const Measured& p : measured)
 	{
-		const int ranges = litenn_hip::fetch::exact_ranges(p.by_step, (p.n + 31) / 32, (p.m + 31) / 32, p.k / 256);
+		const int ranges = litenn_hip::fetch::exact_ranges(p.by_step, p.n, p.m, p.k / 256);
 		CHECK((ranges > 1 ? p.ranged : p.without) <= 1.03 * (p.without < p.ranged ? p.without : p.ranged), "%d x %d x %d: %d ranges", p.m, p.n, p.k, ranges);
 	}
 }
