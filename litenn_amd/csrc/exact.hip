@@ -803,7 +803,7 @@ namespace litenn_hip
 		template <int N>
 		__device__ __forceinline__ void arrived() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 
-		template <typename F, int MT, int WN, int KS>
+		template <typename F, int MT, int WN, int KS, bool RANGES>
 		__global__ __launch_bounds__(64 * WN * KS, 2) void exact_shared_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                    const float* residual, int k, int m, int m_tiles,
 		                                                                    int chunks, size_t row_bytes, int flush, size_t range_stride)
@@ -817,8 +817,9 @@ namespace litenn_hip
 			extern __shared__ __attribute__((aligned(16))) uint8_t lds[]; // [KS][kRing][MT][stage], [WN KS][slot]; later the KS sums
 			ExactPlace<F, MT, WN, KS> place(mats, chunks);
 			const int lane = place.lane, h = lane >> 5;
-			if constexpr (KS == 1)
+			if constexpr (RANGES)
 			{
+				static_assert(KS == 1, "ranges of K over workgroups");
 				const int per = (chunks + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
 				place.c_begin = static_cast<int>(blockIdx.z) * per, place.c_end = min(place.c_begin + per, chunks);
 				place.y += blockIdx.z * range_stride;
@@ -1085,7 +1086,7 @@ namespace litenn_hip
 					__syncthreads();
 				}
 			}
-			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes, KS > 1 || gridDim.z == 1);
+			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes, !RANGES);
 		}
 
 		// The same with less held ahead.  WN > 1: the fragments pass through the same two buffers, two stages on their way; with WN =
@@ -2002,8 +2003,8 @@ namespace litenn_hip
 			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
 		}
 
-		// `ranges` of K in grid z, none of them empty, leave their sums in c.partial, from where a launch more adds them
-		template <typename F, int KS>
+		// RANGES: `ranges` of K in grid z, none of them empty, leave their sums in c.partial, from where a launch more adds them
+		template <typename F, int KS, bool RANGES = false>
 		void launch_shared(const ExactCall& c, int flush, int ranges = 1)
 		{
 			constexpr int MT = 2, WN = 4;
@@ -2015,7 +2016,7 @@ namespace litenn_hip
 			ExactMats mats = grid_mats(c, WN * kTile, blocks);
 			const ExactMats out = mats;
 			const size_t stride = static_cast<size_t>(c.m) * c.total_rows;
-			if (ranges > 1)
+			if constexpr (RANGES)
 			{
 				size_t at = 0;
 				for (int i = 0; i < c.count; ++i)
@@ -2024,11 +2025,11 @@ namespace litenn_hip
 					at += static_cast<size_t>(c.m) * c.n[i];
 				}
 			}
-			constexpr auto kernel = &exact_shared_kernel<F, MT, WN, KS>;
+			constexpr auto kernel = &exact_shared_kernel<F, MT, WN, KS, RANGES>;
 			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
 			kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT, ranges), dim3(64 * WN * KS), lds, c.stream>>>(
-			    mats, c.xs, ranges > 1 ? nullptr : c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, stride);
-			if (ranges > 1)
+			    mats, c.xs, RANGES ? nullptr : c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, stride);
+			if constexpr (RANGES)
 			{
 				const unsigned widest = static_cast<unsigned>(*std::max_element(c.n, c.n + c.count));
 				add_ranges_kernel<<<dim3(c.m, (widest + 1023) / 1024, c.count), dim3(256), 0, c.stream>>>(
@@ -2056,7 +2057,7 @@ namespace litenn_hip
 				const int ranges = fetch::exact_ranges(F::kScaleSteps == 1, c.total_rows, c.m, c.chunks);
 				if (ranges > 1 && static_cast<size_t>(ranges) * c.m * c.total_rows <= c.partial_floats)
 				{
-					return launch_shared<F, 1>(c, fetch::chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
+					return launch_shared<F, 1, true>(c, fetch::chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
 				}
 			}
 			if constexpr (F::kMins)
