@@ -208,6 +208,16 @@ namespace litenn_hip
 			const bool filled = (dim <= 64 && vdim <= 64) || dim + vdim > 224;
 			return rows >= 16 && keys > 64 && (keys >= 96 || filled || rows * heads >= 1400);
 		}
+		// The first of a prompt's rows that such a call takes where rows `first` .. alone are asked for: that of their block, or of the one
+		// before where what is left would go by the row kernel, whose rows walk all keys, and a block more does not.  us of a whole
+		// prompt of two layers, two rows asked for, from their own block and now: Kulurax 1024 wide 200 tokens 305 -> 275, 456 388 -> 308,
+		// 712 486 -> 356, Degedra 712 519 -> 409 (and with all rows taken 288, 327, 380, 448).
+		inline int window_rows_from(int rows, int first, int block, size_t keys, size_t heads, size_t dim, size_t vdim)
+		{
+			const int from = first / block * block;
+			const bool again = from > 0 && !rows_window_tiles(rows - from, keys, heads, dim, vdim) && rows_window_tiles(rows - from + block, keys, heads, dim, vdim);
+			return again ? from - block : from;
+		}
 
 		// ---- products over bfloat16 weights: the K tiles of a group of wavefronts ----------------
 		// K is cut into `ranges` times `groups` parts, in order, that differ by a tile at most; the groups of a

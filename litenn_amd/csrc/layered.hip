@@ -1070,7 +1070,7 @@ namespace litenn_hip
 				const bool stepped = one && rows > 1 && (M.desc.kind == MixerKind::GroupedAttention || M.desc.kind == MixerKind::StateSpace);
 				// (attention in 32 bits takes a few rows the slower the fewer they are, and looks at what comes out of all of them)
 				const bool by_step = stepped || (M.desc.kind == MixerKind::LatentAttention && latent_by_step(M, n, past + rows));
-				const int asked = f32 && !by_step ? first / kAttnRows * kAttnRows : first;
+				const int asked = f32 && !by_step ? asked_block(L, rows, first, past + rows) : first;
 				enter(L.norm1, 0, rows);
 				OneRow row{ *this, x + static_cast<size_t>(first) * desc.width, 0 };
 				if (asked > 0)
@@ -1162,6 +1162,21 @@ namespace litenn_hip
 		bool latent_by_step(const MixerState& M, int n, int length) const
 		{
 			return n == 1 && std::min(length, M.desc.window) >= (f32 ? 64 : 384);
+		}
+
+		// the first row that mixers in 32 bits take where rows `first` .. are asked for, behind `length` positions
+		int asked_block(const LayerState& L, int rows, int first, int length) const
+		{
+			int from = first / kAttnRows * kAttnRows;
+			for (const MixerState& M : L.mixers)
+			{
+				const MixerDesc& m = M.desc;
+				if (m.kind == MixerKind::LatentAttention || m.kind == MixerKind::GroupedAttention)
+				{
+					from = std::min(from, fetch::window_rows_from(rows, first, kAttnRows, std::min(length, m.window), m.heads, m.dim, m.vdim));
+				}
+			}
+			return from;
 		}
 
 		// queries of rows `first` .. (and some ahead of them), keys of all rows

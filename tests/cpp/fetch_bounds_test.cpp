@@ -914,6 +914,23 @@ static void test_options_forms()
 		const double least = p.row < p.tiles ? p.row : p.tiles;
 		CHECK((tiles ? p.tiles : p.row) <= 1.1 * least, "window, %d rows on %d keys, %d heads of %d and %d: tiles %d", p.rows, p.keys, p.heads, p.dim, p.vdim, tiles);
 	}
+	// rows that are asked for alone go by the form that all would go by, with a block of 64 ahead of them at most
+	for (int rows = 1; rows <= 900; ++rows)
+	{
+		for (int first = 0; first < rows; ++first)
+		{
+			for (int keys : { rows, rows < 65 ? rows : 65, rows < 90 ? rows : 90 })
+			{
+				for (int dim : { 64, 80, 128 })
+				{
+					const int from = litenn_hip::fetch::window_rows_from(rows, first, 64, keys, 8, dim, dim);
+					const bool all = litenn_hip::fetch::rows_window_tiles(rows, keys, 8, dim, dim), some = litenn_hip::fetch::rows_window_tiles(rows - from, keys, 8, dim, dim);
+					CHECK(from >= 0 && from <= first && first - from < 128 && from % 64 == 0, "%d of %d rows: from %d", rows - first, rows, from);
+					CHECK(some == all || keys < 96, "%d of %d rows on %d keys: from %d", rows - first, rows, keys, from);
+				}
+			}
+		}
+	}
 	CHECK(!litenn_hip::fetch::rows_window_tiles(15, 500, 16, 128, 128) && !litenn_hip::fetch::rows_window_tiles(500, 64, 16, 128, 128), "few rows or keys");
 }
 

@@ -35,6 +35,24 @@ def test_one_row_over_cached_latents(hip, rows):
         assert ku.error(model.eval(toks, want=[rows - 1]), want[rows - 1:]) <= LIMIT["bfloat16"]
 
 
+@pytest.mark.parametrize("name", ["latent", "both"])
+def test_few_asked_rows_behind_whole_tiles(hip, name):
+    """Float32: up to 15 rows past a tile of 64 take the tile before them too."""
+    cfg, weights, plain_form = LAST[name]
+    w = weights(cfg, 21)
+    toks = ku.tokens(cfg, 280, 6)
+    want = plain_form(cfg, ku.as_floats(w)).forward(toks)
+    with hip.create_model(cfg, w, dtype="float32", context_length=300) as model:
+        for past, rows, count in ((0, 130, 2), (0, 207, 15), (37, 194, 2), (37, 208, 16), (0, 143, 16), (0, 200, 9)):
+            model.reset()
+            if past:
+                model.eval(toks[:past], want=[])
+            got = model.eval(toks[past:past + rows], want=list(range(rows - count, rows)))
+            assert ku.error(got, want[past + rows - count:past + rows]) <= LIMIT["float32"], (past, rows, count)
+            got = model.eval(toks[past + rows:past + rows + 1])
+            assert ku.error(got, want[past + rows:past + rows + 1]) <= LIMIT["float32"], (past, rows, count)
+
+
 # heads and value sizes of every form of the launch that makes both mixers' outputs, at the edges of its tiles (64 queries,
 # chunks of 64 tokens, two blocks of the recurrence to a workgroup), few workgroups and many, four taps and others
 PAIRS = {
