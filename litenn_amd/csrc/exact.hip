@@ -806,7 +806,7 @@ namespace litenn_hip
 		template <typename F, int MT, int WN, int KS, bool RANGES>
 		__global__ __launch_bounds__(64 * WN * KS, 2) void exact_shared_kernel(const ExactMats mats, const uint8_t* __restrict__ xs,
 		                                                                    const float* residual, int k, int m, int m_tiles,
-		                                                                    int chunks, size_t row_bytes, int flush, size_t range_stride)
+		                                                                    int chunks, size_t row_bytes, int flush, size_t range_stride, int first_row)
 		{
 			constexpr bool kScaled = F::kScaleSteps < 16; // sums of kScaleSteps steps are scaled and added to the chunk's
 			static_assert(kScaled != F::kMins, "one scale for a chunk has minima beside it");
@@ -822,7 +822,8 @@ namespace litenn_hip
 				static_assert(KS == 1, "ranges of K over workgroups");
 				const int per = (chunks + static_cast<int>(gridDim.z) - 1) / static_cast<int>(gridDim.z);
 				place.c_begin = static_cast<int>(blockIdx.z) * per, place.c_end = min(place.c_begin + per, chunks);
-				place.y += blockIdx.z * range_stride;
+				place.mt_base += first_row / kTile;
+				place.y += static_cast<ptrdiff_t>(blockIdx.z * range_stride) - static_cast<ptrdiff_t>(first_row) * place.n;
 			}
 			const int c_begin = place.c_begin, c_end = place.c_end;
 			const W weights(lds + kRingBytes + (place.part * WN + place.wv) * W::kSlotBytes, place.w, place.n_base, place.n, row_bytes);
@@ -1342,17 +1343,17 @@ namespace litenn_hip
 			place.finish(acc, lds, xs, at, residual, m, chunks, row_bytes);
 		}
 
-		// y_i = factor of the row times the sum over `ranges` of from_i (+ residual), in double, rounded once.  A workgroup takes 1024
-		// elements of a row (grid x) of one matrix (grid z), four a thread.  Bound by its bytes and the launch: three ranges of 300 x 4096
-		// in 5.3 us.
+		// Rows `first` .. of y_i = factor of the row times the sum over `ranges` of from_i (+ residual), in double, rounded once.  A
+		// workgroup takes 1024 elements of a row (grid x) of one matrix (grid z), four a thread.  Bound by its bytes and the launch: three
+		// ranges of 300 x 4096 in 4.6 us.
 		constexpr int kMostRanges = fetch::kMostRanges;
 		__global__ __launch_bounds__(256) void add_ranges_kernel(const ExactMats to, const ExactMats from, int ranges, size_t stride,
-		                                                         const float* __restrict__ factors, const float* residual)
+		                                                         const float* __restrict__ factors, const float* residual, int first)
 		{
-			const int row = blockIdx.x, which = blockIdx.z, n = to.n[which];
+			const int row = first + static_cast<int>(blockIdx.x), which = blockIdx.z, n = to.n[which];
 			const int column = (static_cast<int>(blockIdx.y) * 256 + static_cast<int>(threadIdx.x)) * 4;
 			const size_t at = static_cast<size_t>(row) * n + column;
-			const float* const part = from.y[which] + at;
+			const float* const part = from.y[which] + static_cast<size_t>(blockIdx.x) * n + column;
 			float* const y = to.y[which] + at;
 			const double factor = static_cast<double>(factors[row]);
 			if (column + 4 <= n)
@@ -2003,7 +2004,8 @@ namespace litenn_hip
 			    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes);
 		}
 
-		// RANGES: `ranges` of K in grid z, none of them empty, leave their sums in c.partial, from where a launch more adds them
+		// RANGES: `ranges` of K in grid z, none of them empty, leave their sums in c.partial, from where a launch more adds them, for
+		// as many rows at a time as fetch::ranged_rows says
 		template <typename F, int KS, bool RANGES = false>
 		void launch_shared(const ExactCall& c, int flush, int ranges = 1)
 		{
@@ -2014,26 +2016,31 @@ namespace litenn_hip
 			static_assert(lds <= (KS == 1 ? 80 : 160) * 1024, "LDS");
 			int blocks;
 			ExactMats mats = grid_mats(c, WN * kTile, blocks);
-			const ExactMats out = mats;
-			const size_t stride = static_cast<size_t>(c.m) * c.total_rows;
-			if constexpr (RANGES)
-			{
-				size_t at = 0;
-				for (int i = 0; i < c.count; ++i)
-				{
-					mats.y[i] = c.partial + at;
-					at += static_cast<size_t>(c.m) * c.n[i];
-				}
-			}
 			constexpr auto kernel = &exact_shared_kernel<F, MT, WN, KS, RANGES>;
 			allow_dynamic_lds(reinterpret_cast<const void*>(kernel), lds);
-			kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT, ranges), dim3(64 * WN * KS), lds, c.stream>>>(
-			    mats, c.xs, RANGES ? nullptr : c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, stride);
-			if constexpr (RANGES)
+			if constexpr (!RANGES)
 			{
-				const unsigned widest = static_cast<unsigned>(*std::max_element(c.n, c.n + c.count));
-				add_ranges_kernel<<<dim3(c.m, (widest + 1023) / 1024, c.count), dim3(256), 0, c.stream>>>(
-				    out, mats, ranges, stride, reinterpret_cast<const float*>(c.xs + RowsLayout(c.m_tiles, c.chunks).factors), c.residual);
+				kernel<<<dim3(blocks, (c.m_tiles + MT - 1) / MT), dim3(64 * WN * KS), lds, c.stream>>>(
+				    mats, c.xs, c.residual, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, 0, 0);
+				return;
+			}
+			const ExactMats out = mats;
+			const int rows = fetch::ranged_rows(ranges, c.total_rows, c.m);
+			const size_t stride = static_cast<size_t>(rows) * c.total_rows;
+			size_t at = 0;
+			for (int i = 0; i < c.count; ++i)
+			{
+				mats.y[i] = c.partial + at;
+				at += static_cast<size_t>(rows) * c.n[i];
+			}
+			const unsigned widest = static_cast<unsigned>(*std::max_element(c.n, c.n + c.count));
+			const float* const factors = reinterpret_cast<const float*>(c.xs + RowsLayout(c.m_tiles, c.chunks).factors);
+			for (int first = 0; first < c.m; first += rows)
+			{
+				const int here = std::min(rows, c.m - first);
+				kernel<<<dim3(blocks, (here + MT * kTile - 1) / (MT * kTile), ranges), dim3(64 * WN * KS), lds, c.stream>>>(
+				    mats, c.xs, nullptr, c.k, c.m, c.m_tiles, c.chunks, c.row_bytes, flush, stride, first);
+				add_ranges_kernel<<<dim3(here, (widest + 1023) / 1024, c.count), dim3(256), 0, c.stream>>>(out, mats, ranges, stride, factors, c.residual, first);
 			}
 		}
 
@@ -2055,7 +2062,7 @@ namespace litenn_hip
 			if constexpr (kShares<F>)
 			{
 				const int ranges = fetch::exact_ranges(F::kScaleSteps == 1, c.total_rows, c.m, c.chunks);
-				if (ranges > 1 && static_cast<size_t>(ranges) * c.m * c.total_rows <= c.partial_floats)
+				if (ranges > 1 && static_cast<size_t>(ranges) * fetch::ranged_rows(ranges, c.total_rows, c.m) * c.total_rows <= c.partial_floats)
 				{
 					return launch_shared<F, 1, true>(c, fetch::chunks_a_sum((c.chunks + ranges - 1) / ranges).chunks, ranges);
 				}
@@ -2229,21 +2236,20 @@ namespace litenn_hip
 	size_t exact_partial_floats(int fmt, size_t n, size_t k, size_t m)
 	{
 		const int ranges = exact_ranges(fmt, n, k, m);
-		return ranges > 1 ? static_cast<size_t>(ranges) * m * n : 0;
+		return ranges > 1 ? static_cast<size_t>(ranges) * fetch::ranged_rows(ranges, static_cast<int>(n), static_cast<int>(m)) * n : 0;
 	}
 
 	// the same for any number of rows up to m
 	size_t exact_most_partial_floats(int fmt, size_t n, size_t k, size_t m)
 	{
-		size_t most = 0;
-		const size_t strips = (n + kTile - 1) / kTile;
-		// beyond 256 workgroups of 128 x 64 results there is one number of ranges, and they take most at most rows
-		for (int ranges = 2; ranges <= 4; ++ranges)
-		{
-			most = std::max(most, exact_partial_floats(fmt, n, k, std::min(m, kTile * (fetch::kMostRangedTiles / (ranges * strips)))));
-		}
-		// up to there every number of tiles has its own, and the fewer rows it holds the sooner they pay
+		// beyond 256 workgroups of 128 x 64 results there is one number of ranges, and as many rows as go at a time take most; up to
+		// there every number of tiles has its own, and the fewer rows it holds the sooner they pay
 		const size_t blocks = (n + 4 * kTile - 1) / (4 * kTile), last = std::min(m, 64 * (256 / std::max<size_t>(blocks, 1)));
+		size_t most = 0;
+		if (const int ranges = exact_ranges(fmt, n, k, m); m > last && ranges > 1)
+		{
+			most = static_cast<size_t>(ranges) * std::min<size_t>(m, fetch::ranged_rows_whole(ranges, static_cast<int>(n))) * n;
+		}
 		for (size_t first = 1; first <= last; first += kTile)
 		{
 			const int ranges = exact_ranges(fmt, n, k, first);

@@ -65,7 +65,23 @@ namespace litenn_hip
 		}
 
 		constexpr int kMostRanges = 16;
-		constexpr size_t kMostRangedTiles = size_t{ 1 } << 17; // of 32 x 32 sums, all ranges together
+		// Rows of activations that go through the form with ranges at a time: whole pairs of tiles, about equally many each time, whose
+		// sums bound what a call or a model holds beside its rows.  128 MB of them, or 256 rows up to 256 MB: a launch of fewer rows has
+		// its last round of workgroups and its weights from HBM to itself, one of more finds less in the caches.  us of a call of
+		// Q6_K with 64 MB, 128 and 512: 14336 x 4096 at 700 rows 324, 297, 299, at 2000 834, 834, 878, 28672 x 4096 at 2400 1936, 1971,
+		// 2050; 128256 x 4096 at 300 in three launches 1223, in one 1156.  (By the forms without ranges 28672 x 4096 at 2400 takes 4970.)
+		constexpr long long kRangedFloats = 1ll << 25, kMostRangedFloats = 1ll << 27;
+		inline int ranged_rows_whole(int ranges, int n)
+		{
+			const long long a_row = static_cast<long long>(ranges) * n, some = kRangedFloats / a_row, wide = 2 * kRangedFloats / a_row;
+			const long long rows = some > 256 ? some : wide > 256 ? 256 : wide;
+			return rows < 64 ? 64 : rows < (1 << 24) ? static_cast<int>(rows / 64 * 64) : 1 << 24;
+		}
+		inline int ranged_rows(int ranges, int n, int m)
+		{
+			const int whole = ranged_rows_whole(ranges, n), times = (m + whole - 1) / whole;
+			return times > 1 ? ((m + times - 1) / times + 63) / 64 * 64 : m;
+		}
 
 		// Ranges of K for the form that shares activations, with grid z, 1 where it does not pay: up to 256 workgroups of 128 x 64 results
 		// as many as leave every one its place on the card, two to a CU.  by_step: Q6_K, whose steps are scaled one by one (other
@@ -82,14 +98,14 @@ namespace litenn_hip
 			}
 			// Q6_K on more workgroups: as few ranges as round no more than the eight of the form without, whose wavefronts each read their
 			// activations from L2 (us of a call by that and by this: 4096 x 14336 at 700 rows 385 and 321, 1000 598 and 415, 2000 2051 and
-			// 848, 8192 x 4096 at 300 rows 124 and 103, 14336 x 4096 207 and 155), up to 512 MB of sums.
+			// 848, 8192 x 4096 at 300 rows 124 and 103, 14336 x 4096 207 and 155), some rows at a time where their sums are many.
 			if (by_step && workgroups > 256 && chunks >= 16)
 			{
 				const long long r = (chunks + 7) / 8;
 				for (int ranges = 2; ranges <= 4; ++ranges)
 				{
 					const int each = (chunks + ranges - 1) / ranges;
-					if (static_cast<long long>(ranges) * tiles > static_cast<long long>(kMostRangedTiles))
+					if (static_cast<long long>(ranges) * imin(m, 64) * n > kMostRangedFloats)
 					{
 						return 1;
 					}

@@ -988,6 +988,27 @@ static void test_exact_ranges()
 		const int ranges = litenn_hip::fetch::exact_ranges(p.by_step, p.n, p.m, p.k / 256);
 		CHECK((ranges > 1 ? p.ranged : p.without) <= 1.03 * (p.without < p.ranged ? p.without : p.ranged), "%d x %d x %d: %d ranges", p.m, p.n, p.k, ranges);
 	}
+	// the rows that go at a time: pairs of tiles, all rows among them, and sums within bounds
+	for (int n : { 1, 31, 1000, 4096, 14336, 28672, 65535, 65536, 128256, 262144, 600000, 1 << 20 })
+	{
+		for (int ranges : { 2, 3, 4, 16 })
+		{
+			for (int m = 1; m <= 1 << 20; m += 1 + m / 7)
+			{
+				const int rows = litenn_hip::fetch::ranged_rows(ranges, n, m), times = (m + rows - 1) / rows;
+				const long long sums = static_cast<long long>(ranges) * rows * n, bound = rows > 256 ? 1ll << 25 : rows > 64 ? 1ll << 26 : 1ll << 62;
+				CHECK(rows > 0 && rows <= m + 63 && (times == 1 || rows % 64 == 0) && sums <= bound, "%d ranges of %d, %d rows: %d at a time", ranges, n, m, rows);
+				CHECK(rows <= litenn_hip::fetch::ranged_rows_whole(ranges, n) && (times == 1 ? rows == m : m - (times - 1) * rows > 0), "%d ranges of %d, %d rows: %d at a time", ranges, n, m, rows);
+				const int chosen = litenn_hip::fetch::exact_ranges(true, n, m, 16);
+				CHECK(chosen == 1 || static_cast<long long>(chosen) * litenn_hip::fetch::ranged_rows(chosen, n, m) * n <= 1ll << 27, "%d x %d: %d ranges", n, m, chosen);
+			}
+		}
+	}
+	// more rows than go at a time keep the ranges of fewer
+	for (int m : { 2336, 2337, 2400, 4096, 100000 })
+	{
+		CHECK(litenn_hip::fetch::exact_ranges(true, 28672, m, 16) == 2, "28672 x 4096, %d rows", m);
+	}
 }
 
 int main(int argc, char** argv)

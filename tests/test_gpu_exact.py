@@ -229,6 +229,23 @@ def test_ranges_of_k_whose_sums_alone_leave_float32(hip, fmt, m, n, k, residual)
     assert (np.abs(got[1] - want[1]) <= 1e-6 * size[1] + 2.0 ** -150).all()
 
 
+@pytest.mark.parametrize("fmt,m,n,k,residual", [(Q6_K, 4200, 4099, 4096, True), (Q6_K, 300, 65600, 4096, False)])
+def test_ranges_of_k_for_some_rows_at_a_time(hip, fmt, m, n, k, residual):
+    """More sums than are left at once: rows in two or three launches, a last one that is not whole; each row as in a call of few."""
+    wq, x, add = hip.Tensor.from_numpy(synth.model_weights(fmt, n, k, 71)), synth.activations(m, k, 72), synth.activations(m, n, 73)
+    run = lambda rows: hip.mul_mat_q(fmt, wq, n, k, hip.Tensor.from_numpy(x[rows]), residual=hip.Tensor.from_numpy(add[rows]) if residual else None,
+                                     flags=MATMUL_PRECISE).numpy()
+    got = run(slice(None))
+    for first, end in ((0, 70), (m // 2 - 90, m // 2 + 90), (m - 70, m)):  # (beyond 256 workgroups of 128 x 64 results, as all)
+        if (n + 127) // 128 * ((end - first + 63) // 64) > 256:
+            np.testing.assert_array_equal(got[first:end], run(slice(first, end)))
+    w = np_decoders.decode(fmt, wq.numpy().reshape(n, -1), k).astype(np.float64)
+    for rows in (slice(0, 8), slice(m // 2 - 8, m // 2 + 8), slice(m - 8, m)):
+        size = np.linalg.norm(x[rows].astype(np.float64), axis=1)[:, None] * np.linalg.norm(w) / np.sqrt(n * k) * np.sqrt(k)
+        want = x[rows].astype(np.float64) @ w.T + (add[rows] if residual else 0.0)
+        assert (np.abs(got[rows] - want) <= 1e-5 * size).all() and np.linalg.norm(got[rows] - want) <= 1e-6 * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("m", [9, 32, 33])
 def test_many_weight_rows_meet_one_tile_of_activations(hip, m):
     """More workgroups of 128 x 64 results than CUs: up to 32 rows leave half of each empty and take the form without ranges of K."""
