@@ -8,6 +8,7 @@
 // preallocated KV cache and the current length kept in device memory.  The token loops around
 // it (evaluation, and the greedy loop over a captured single-token step) are decoder.hip's.
 #include "decoder.hpp"
+#include "room.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -115,9 +116,8 @@ struct litenn_hip_llama : litenn_hip_model
 	float *x = nullptr, *xn = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *attn = nullptr, *gate = nullptr,
 	      *gate2 = nullptr, *up = nullptr;
 	size_t xn_floats = 0; // what xn holds (rows x embedding_length, three times that for short prompts)
-	void* xh = nullptr; // a matmul's activations as the matrix cores take them (multi-row path)
-	size_t xh_halves = 0; // its size
-	size_t summed_rows = 0, sum_floats = 0; // rows that sum_floats was found for: what matmuls of up to so many leave sums of ranges of K in
+	Room xh; // a matmul's activations as the matrix cores take them (multi-row path), and behind them sums of ranges of K
+	size_t summed_rows = 0, sum_floats = 0; // rows that sum_floats was found for: what matmuls of up to so many leave such sums in
 	// single-row attention: key chunks per head, their meeting place and arrival counters
 	size_t attn_splits = 1;
 	float* attn_partial = nullptr;
@@ -142,6 +142,10 @@ namespace
 {
 	const char* kAction = "HIP LLaMA";
 
+	// From this many rows on a matmul goes to the matrix cores: one padded tile costs about as much as three
+	// single-row GEMVs (with Float32 operands: 12.5 us + bytes / 2.2 TB/s against 3.3 us + bytes / 5.1 TB/s per row).
+	constexpr size_t kGemmMinRows = 4;
+
 	void free_scratch(litenn_hip_llama* m)
 	{
 		float** bufs[] = { &m->x, &m->xn, &m->q, &m->k, &m->v, &m->attn, &m->gate, &m->gate2, &m->up };
@@ -153,11 +157,11 @@ namespace
 				*b = nullptr;
 			}
 		}
-		if (m->xh)
+		if (m->xh.data)
 		{
-			(void)hipFree(m->xh);
-			m->xh = nullptr;
+			(void)hipFree(m->xh.data);
 		}
+		m->xh = Room();
 		m->cap_rows = 0;
 	}
 
@@ -190,10 +194,14 @@ namespace
 		return most;
 	}
 
-	// Halves that the rows of the model's matmuls take on their way to the matrix cores: rounded to fp16 (q/k/v projections in
+	// Bytes that the rows of the model's matmuls take on their way to the matrix cores: rounded to fp16 (q/k/v projections in
 	// two formats share a launch that wants them in both fragment orders), or, for matrices that meet Float32
-	// operands, taken apart into two halves each and, behind them, sums of ranges of K.
-	size_t matmul_halves(litenn_hip_llama* m, size_t rows, unsigned flags)
+	// operands, taken apart into two halves each.  with_sums: the same and, behind them, sums of ranges of K.
+	struct MatmulBytes
+	{
+		size_t rows, with_sums;
+	};
+	MatmulBytes matmul_bytes(litenn_hip_llama* m, size_t rows, unsigned flags)
 	{
 		const size_t d = m->p.embedding_length, ff = m->p.feed_forward_length;
 		const size_t qw = static_cast<size_t>(m->p.head_count) * m->head_dim;
@@ -213,13 +221,22 @@ namespace
 			}
 		}
 		const size_t rounded = std::max(gemm_scratch_halves(rows, std::max({ d, qw, ff })), 2 * gemm_scratch_halves(rows, d));
-		if ((flags & LITENN_HIP_MATMUL_PRECISE) && m->summed_rows != rows)
+		if (!widest)
+		{
+			return { 2 * rounded, 2 * rounded };
+		}
+		const size_t bytes = std::max(2 * rounded, exact_scratch_bytes(rows, widest));
+		if (!(flags & LITENN_HIP_MATMUL_PRECISE))
+		{
+			return { bytes, bytes };
+		}
+		if (m->summed_rows != rows)
 		{
 			m->sum_floats = ranges_sums(m, rows);
 			m->summed_rows = rows;
 		}
-		const size_t sums = flags & LITENN_HIP_MATMUL_PRECISE ? 2 * m->sum_floats + 128 : 0; // (behind the rows, on 256 bytes)
-		return widest ? std::max(rounded, (exact_scratch_bytes(rows, widest) + 1) / 2 + sums) : rounded;
+		const size_t sums = m->sum_floats;
+		return { bytes, sums ? std::max(bytes, (exact_scratch_bytes(rows, widest) + 255) / 256 * 256 + sizeof(float) * sums) : bytes };
 	}
 
 	int ensure_scratch(litenn_hip_llama* m, size_t rows, unsigned flags)
@@ -245,17 +262,29 @@ namespace
 			}
 			m->cap_rows = rows;
 		}
-		const size_t halves = m->xh && rows == 1 ? 0 : matmul_halves(m, m->cap_rows, flags); // (a single row uses none)
-		if (!m->xh || halves > m->xh_halves)
+		if (m->xh.data && rows == 1) // (a single row uses none)
 		{
-			decoder_drop_graph(m);
-			(void)hipFree(m->xh);
-			m->xh = nullptr;
-			m->xh_halves = 0;
-			LITENN_HIP_TRY(kAction, hipMalloc(&m->xh, 2 * halves));
-			m->xh_halves = halves;
+			return 0;
 		}
-		return 0;
+		const MatmulBytes bytes = matmul_bytes(m, m->cap_rows, flags);
+		hipError_t last = hipSuccess;
+		const bool there = grow_room(
+		    m->xh, bytes.rows, bytes.with_sums,
+		    [&](size_t size) {
+			    void* data = nullptr;
+			    last = hipMalloc(&data, size);
+			    if (last != hipSuccess)
+			    {
+				    (void)hipGetLastError(); // (without room for sums K goes in one range)
+				    data = nullptr;
+			    }
+			    return data;
+		    },
+		    [&](void* data) {
+			    decoder_drop_graph(m);
+			    (void)hipFree(data);
+		    });
+		return there ? 0 : fail_hip(kAction, last);
 	}
 
 	int check_tensors(const litenn_hip_llama* m)
@@ -275,9 +304,6 @@ namespace
 		return 0;
 	}
 
-	// From this many rows on a matmul goes to the matrix cores: one padded tile costs about as much as three
-	// single-row GEMVs (with Float32 operands: 12.5 us + bytes / 2.2 TB/s against 3.3 us + bytes / 5.1 TB/s per row).
-	constexpr size_t kGemmMinRows = 4;
 	// From this many rows on the prompt's attention runs tiled on the matrix cores.
 	constexpr size_t kAttnTileMinRows = 16;
 
@@ -307,13 +333,13 @@ namespace
 			}
 		}
 		const size_t k = ws[0]->k;
-		if (rows < kGemmMinRows || exact_scratch_bytes(rows, k) > 2 * m->xh_halves ||
-		    !launch_exact_rows(x, rows, k, norm_w, m->p.rms_norm_epsilon, up, m->xh, s))
+		if (rows < kGemmMinRows || exact_scratch_bytes(rows, k) > m->xh.bytes ||
+		    !launch_exact_rows(x, rows, k, norm_w, m->p.rms_norm_epsilon, up, m->xh.data, s))
 		{
 			return false;
 		}
 		const size_t rows_end = (exact_scratch_bytes(rows, k) + 255) / 256 * 256;
-		const size_t room = 2 * m->xh_halves > rows_end ? (2 * m->xh_halves - rows_end) / sizeof(float) : 0;
+		const size_t room = m->xh.bytes > rows_end ? (m->xh.bytes - rows_end) / sizeof(float) : 0;
 		for (int i = 0; i < count;)
 		{
 			const void* w[3];
@@ -324,8 +350,8 @@ namespace
 				w[j - i] = ws[j]->data;
 				n[j - i] = ws[j]->n;
 			}
-			launch_exact_gemm(ws[i]->fmt, j - i, w, n, k, rows, ys + i, residual, m->xh,
-			                  room ? reinterpret_cast<float*>(static_cast<char*>(m->xh) + rows_end) : nullptr, room, s);
+			launch_exact_gemm(ws[i]->fmt, j - i, w, n, k, rows, ys + i, residual, m->xh.data,
+			                  room ? reinterpret_cast<float*>(static_cast<char*>(m->xh.data) + rows_end) : nullptr, room, s);
 			i = j;
 		}
 		return true;
@@ -338,7 +364,7 @@ namespace
 		if (rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE))
 		{
 			if (is_quantised(w) && w.k % 256 == 0 &&
-			    launch_gemm(w.fmt, w.data, w.n, w.k, x, rows, y, residual, m->xh, partial, partial ? m->xn_floats : 0, s))
+			    launch_gemm(w.fmt, w.data, w.n, w.k, x, rows, y, residual, m->xh.data, partial, partial ? m->xn_floats : 0, s))
 			{
 				return;
 			}
@@ -375,7 +401,7 @@ namespace
 				n[i] = ws[i]->n;
 			}
 			if (launch_gemm_group(w0.fmt, count, w, n, w0.k, x, rows, ys, residual, norm_w, m->p.rms_norm_epsilon, up,
-			                      m->xh, partial, partial ? m->xn_floats : 0, s))
+			                      m->xh.data, partial, partial ? m->xn_floats : 0, s))
 			{
 				return;
 			}
@@ -641,7 +667,7 @@ namespace
 			const bool one_launch = mixed && rows >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE) &&
 			                        qkv[from]->k == L.wk.k && L.wk.k == L.wv.k &&
 			                        launch_gemm_group_mixed(qkv_fmt + from, 3 - from, qkv_w + from, qkv_n + from, L.wk.k, m->x, rows,
-			                                                qkv_out + from, L.attn_norm, m->p.rms_norm_epsilon, m->xh, m->xh_halves, s);
+			                                                qkv_out + from, L.attn_norm, m->p.rms_norm_epsilon, m->xh.data, m->xh.bytes / 2, s);
 			const bool exact = rows >= kGemmMinRows && (flags & LITENN_HIP_MATMUL_PRECISE); // (formats do not matter to its rows)
 			for (int i = from; i < 3 && !one_launch;)
 			{
@@ -676,7 +702,7 @@ namespace
 			const bool gated = n >= kGemmMinRows && !(flags & LITENN_HIP_MATMUL_PRECISE) && L.gate.fmt == L.up.fmt &&
 			                   L.gate.k == L.up.k && L.gate.n == L.up.n &&
 			                   launch_gemm_gated(L.gate.fmt, L.gate.data, L.up.data, L.gate.n, L.gate.k, x, n, m->gate,
-			                                     L.ffn_norm, m->p.rms_norm_epsilon, m->xh, s);
+			                                     L.ffn_norm, m->p.rms_norm_epsilon, m->xh.data, s);
 			if (!gated)
 			{
 				matmul_group(m, 2, gu, gu_out, x, n, nullptr, L.ffn_norm, nullptr, m->xn, nullptr, flags, s);
@@ -1000,6 +1026,7 @@ extern "C" int litenn_hip_llama_set_tensor(litenn_hip_llama* m, int which, int l
 	target->k = k;
 	decoder_drop_graph(m);
 	m->block_fused = 0; // decided again with the new tensor
+	m->summed_rows = 0;
 	return 0;
 }
 

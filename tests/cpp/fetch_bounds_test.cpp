@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "../../litenn_amd/csrc/fetch_model.hpp"
+#include "../../litenn_amd/csrc/room.hpp"
 
 namespace fm = litenn_hip::fetch;
 
@@ -1011,6 +1012,32 @@ static void test_exact_ranges()
 	}
 }
 
+// Memory that a model holds: what it is faster with is left out where it cannot be had, and not asked for on every call.
+static void test_room()
+{
+	size_t largest = 1000, held = 0, asked = 0;
+	char memory;
+	const auto allocate = [&](size_t bytes) -> void* {
+		++asked;
+		held = bytes <= largest ? bytes : 0;
+		return held ? &memory : nullptr;
+	};
+	const auto release = [&](void* p) {
+		CHECK(p == &memory && held > 0, "released what was held");
+		held = 0;
+	};
+	litenn_hip::Room room;
+	const auto grow = [&](size_t need, size_t want) { return litenn_hip::grow_room(room, need, want, allocate, release); };
+	CHECK(grow(100, 300) && held == 300 && room.bytes == 300 && asked == 1, "the larger one");
+	CHECK(grow(200, 300) && grow(100, 100) && asked == 1, "no less than is there");
+	CHECK(grow(400, 5000) && held == 400 && room.bytes == 400 && asked == 3, "the lesser one where the larger is refused");
+	CHECK(grow(400, 5000) && grow(300, 9000) && held == 400 && asked == 3, "a size that was refused is not asked for again");
+	CHECK(grow(300, 700) && held == 700 && asked == 4, "a smaller one is");
+	CHECK(grow(800, 6000) && held == 800 && asked == 5, "more than is there, the refused size not tried");
+	CHECK(!grow(2000, 2000) && held == 0 && !room.data && room.bytes == 0 && asked == 6, "none");
+	CHECK(grow(500, 900) && held == 900 && asked == 7, "and some again");
+}
+
 int main(int argc, char** argv)
 {
 	if (argc > 1) // n k m ...: the forms of these products, with bfloat16 and with Float32 operands
@@ -1027,6 +1054,7 @@ int main(int argc, char** argv)
 	test_options_forms();
 	test_exact_forms();
 	test_exact_ranges();
+	test_room();
 	test_dense_walks();
 	test_dense_forms();
 	test_dense_ranges();
