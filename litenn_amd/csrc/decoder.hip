@@ -164,7 +164,7 @@ namespace litenn_hip
 
 		int ensure_base(litenn_hip_model* m, size_t rows, size_t logit_rows, unsigned flags)
 		{
-			if (m->ensure_rows(rows, flags) != 0)
+			if (m->ensure_rows(rows, logit_rows, flags) != 0)
 			{
 				return 1;
 			}

@@ -42,8 +42,8 @@ struct litenn_hip_model
 
 	// 0, or non-zero with a message when a tensor is missing
 	virtual int check_complete() = 0;
-	// scratch for passes of up to `rows` tokens (logits and token ids are the base's)
-	virtual int ensure_rows(size_t rows, unsigned flags) = 0;
+	// scratch for passes of up to `rows` tokens of which the last `logit_rows` have logits (these and token ids are the base's)
+	virtual int ensure_rows(size_t rows, size_t logit_rows, unsigned flags) = 0;
 	// decisions that must be made before anything is queued or captured
 	virtual void prepare() {}
 	// the most tokens one pass may carry; longer prompts are fed in passes of this size

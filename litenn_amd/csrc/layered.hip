@@ -567,7 +567,7 @@ namespace litenn_hip
 		size_t pass_rows() const override { return static_cast<size_t>(max_pass); }
 		bool stateful() const override { return true; }
 
-		int ensure_rows(size_t rows, unsigned) override
+		int ensure_rows(size_t rows, size_t, unsigned) override
 		{
 			if (rows <= cap_rows)
 			{

@@ -29,6 +29,7 @@ namespace litenn_hip
 	                       void* scratch, hipStream_t stream);
 	void launch_exact_gemm(int fmt, int count, const void* const* wq, const size_t* n, size_t k, size_t m, float* const* y,
 	                       const float* residual, const void* scratch, float* partial, size_t partial_floats, hipStream_t stream);
+	size_t exact_partial_floats(int fmt, size_t n, size_t k, size_t m);
 	size_t exact_most_partial_floats(int fmt, size_t n, size_t k, size_t m);
 	bool launch_gemm_group(int fmt, int count, const void* const* wq, const size_t* n, size_t k, const float* x,
 	                       size_t m, float* const* y, const float* residual, const float* norm_w, double eps,
@@ -117,7 +118,7 @@ struct litenn_hip_llama : litenn_hip_model
 	      *gate2 = nullptr, *up = nullptr;
 	size_t xn_floats = 0; // what xn holds (rows x embedding_length, three times that for short prompts)
 	Room xh; // a matmul's activations as the matrix cores take them (multi-row path), and behind them sums of ranges of K
-	size_t summed_rows = 0, sum_floats = 0; // rows that sum_floats was found for: what matmuls of up to so many leave such sums in
+	size_t summed_rows = 0, sum_floats = 0; // rows that sum_floats was found for: what the blocks' matmuls of up to so many leave such sums in
 	// single-row attention: key chunks per head, their meeting place and arrival counters
 	size_t attn_splits = 1;
 	float* attn_partial = nullptr;
@@ -132,7 +133,7 @@ struct litenn_hip_llama : litenn_hip_model
 
 	~litenn_hip_llama() override;
 	int check_complete() override;
-	int ensure_rows(size_t rows, unsigned flags) override;
+	int ensure_rows(size_t rows, size_t logit_rows, unsigned flags) override;
 	void prepare() override;
 	void forward(const int32_t* ids, size_t rows, size_t logit_rows, unsigned flags, int past) override;
 	bool give_up_waiting() override;
@@ -165,7 +166,7 @@ namespace
 		m->cap_rows = 0;
 	}
 
-	// floats that the model's matmuls of up to `rows` rows with Float32 operands leave sums of ranges of K in
+	// floats that the blocks' matmuls of up to `rows` rows with Float32 operands leave sums of ranges of K in
 	size_t ranges_sums(const litenn_hip_llama* m, size_t rows)
 	{
 		size_t most = 0;
@@ -189,19 +190,18 @@ namespace
 			}
 			before = &L;
 		}
-		const Weight& head = m->output.data ? m->output : m->tok_embd;
-		look_at(head, head.n);
 		return most;
 	}
 
 	// Bytes that the rows of the model's matmuls take on their way to the matrix cores: rounded to fp16 (q/k/v projections in
 	// two formats share a launch that wants them in both fragment orders), or, for matrices that meet Float32
-	// operands, taken apart into two halves each.  with_sums: the same and, behind them, sums of ranges of K.
+	// operands, taken apart into two halves each.  with_sums: the same and, behind them, sums of ranges of K, of as many rows as the
+	// blocks and (logit_rows) the head have.
 	struct MatmulBytes
 	{
 		size_t rows, with_sums;
 	};
-	MatmulBytes matmul_bytes(litenn_hip_llama* m, size_t rows, unsigned flags)
+	MatmulBytes matmul_bytes(litenn_hip_llama* m, size_t rows, size_t logit_rows, unsigned flags)
 	{
 		const size_t d = m->p.embedding_length, ff = m->p.feed_forward_length;
 		const size_t qw = static_cast<size_t>(m->p.head_count) * m->head_dim;
@@ -212,7 +212,8 @@ namespace
 				widest = std::max(widest, w.k);
 			}
 		};
-		look_at(m->output.data ? m->output : m->tok_embd);
+		const Weight& head = m->output.data ? m->output : m->tok_embd;
+		look_at(head);
 		for (const Layer& L : m->layers)
 		{
 			for (const Weight* w : { &L.wq, &L.wk, &L.wv, &L.wo, &L.gate, &L.up, &L.down })
@@ -235,11 +236,17 @@ namespace
 			m->sum_floats = ranges_sums(m, rows);
 			m->summed_rows = rows;
 		}
-		const size_t sums = m->sum_floats;
+		// (one row of logits, as a prompt that goes on asks for, streams the head)
+		size_t sums = m->sum_floats;
+		if (logit_rows >= kGemmMinRows)
+		{
+			const size_t whole = std::min(rows, (logit_rows + 63) / 64 * 64); // (so that a few more do not grow it again)
+			sums = std::max({ sums, exact_partial_floats(head.fmt, head.n, head.k, logit_rows), exact_partial_floats(head.fmt, head.n, head.k, whole) });
+		}
 		return { bytes, sums ? std::max(bytes, (exact_scratch_bytes(rows, widest) + 255) / 256 * 256 + sizeof(float) * sums) : bytes };
 	}
 
-	int ensure_scratch(litenn_hip_llama* m, size_t rows, unsigned flags)
+	int ensure_scratch(litenn_hip_llama* m, size_t rows, size_t logit_rows, unsigned flags)
 	{
 		const size_t d = m->p.embedding_length;
 		const size_t qw = static_cast<size_t>(m->p.head_count) * m->head_dim;
@@ -266,7 +273,7 @@ namespace
 		{
 			return 0;
 		}
-		const MatmulBytes bytes = matmul_bytes(m, m->cap_rows, flags);
+		const MatmulBytes bytes = matmul_bytes(m, m->cap_rows, logit_rows, flags);
 		hipError_t last = hipSuccess;
 		const bool there = grow_room(
 		    m->xh, bytes.rows, bytes.with_sums,
@@ -737,7 +744,7 @@ namespace
 
 int litenn_hip_llama::check_complete() { return check_tensors(this); }
 
-int litenn_hip_llama::ensure_rows(size_t rows, unsigned flags) { return ensure_scratch(this, rows, flags); }
+int litenn_hip_llama::ensure_rows(size_t rows, size_t logit_rows, unsigned flags) { return ensure_scratch(this, rows, logit_rows, flags); }
 
 void litenn_hip_llama::prepare() { (void)block_fused_ready(this); }
 
