@@ -91,10 +91,12 @@ namespace litenn_hip
 			    last ? m->pinned + kPinnedDoneAt : nullptr, m->passes);
 		}
 
-		// Waits until the pass's last launch has delivered.  The runtime's own wait sleeps until an interrupt, which costs a pass
-		// some 10 us (four empty launches and the wait 17.7 us, with a look at the marks in its place 14.2, twelve 65 and 37; 16 tokens of a
-		// 1024-wide LLaMA block 87 -> 74, of two Degedra layers 204 -> 185), so the host
-		// looks at the marks itself for as long as a pass of a few layers or tokens may take, and sleeps only then.
+		// Waits until the pass's last launch has delivered: the host looks at the marks itself for as long as a pass of a few layers or
+		// tokens may take, and leaves longer ones to the runtime.  The runtime's wait keeps a core busy as well, 1.2 of them, and ends
+		// some 10 us later (four empty launches and the wait 17.7 us, with a look at the marks in its place 14.2, twelve 65 and 37; 16 tokens
+		// of a 1024-wide LLaMA block 80 -> 74, of two Degedra layers 204 -> 185; passes of 250, 800 and 4300 us took 310, 1000 and 5400 us
+		// of the host's time and take 240, 730 and 3600).  More threads than cores lose nothing by it: 12 models' steps on 2 cores
+		// 17300 -> 22900 a second, passes of 1200 us beside two busy processes on 2 cores 1060; a pause between looks changes neither.
 		hipError_t wait_for_pass(litenn_hip_model* m)
 		{
 			const uint32_t* const done = m->pinned + kPinnedDoneAt;

@@ -793,7 +793,8 @@ namespace litenn_hip
 		// What a step of 16 elements multiplies is in registers when it begins: the step before asks for its activations ahead of
 		// its own products and decodes its weights behind them, and a stage's last products follow the barrier, so that they cover
 		// the next stage's first reads.
-		// KS = 1 walks both halves of K one after the other and adds them as the two ranges of KS = 2 are added.
+		// KS = 1 gives every `flush` chunks a sum of their own: half of K's, which are added as the two ranges of KS = 2 are, or, with
+		// RANGES of K over grid z, as many of the range's as round least.
 		// Bound by no unit alone (matrix cores 38 % busy, VALU 39, LDS 26; 18 % of a wavefront's time are waits for operands and barriers)
 		// and by a last round of few workgroups.  us, kernel alone, Q4_K 28672 x 4096 at 300 rows: stages through registers and two
 		// buffers 221, ring 216, KS = 1 with two workgroups to a CU 190; Q6_K 4096 x 14336, by two tiles a wavefront on their own 172,
@@ -1400,7 +1401,7 @@ namespace litenn_hip
 		// activation rows 4 (g % 2) .., the high parts' where g < 2 and the low ones' else, which are summed apart and meet at the end.
 		// Bound by a wavefront's chain per chunk (blocks and activations into LDS, 8 products, 16 in Q6_K); a row more costs its
 		// preparation, 32 instructions.  us against 32 weight rows a workgroup (below), which leave half the card idle here: Q8_0
-		// 4096 x 4096 at 3 rows 10.4 -> 7.9, Q4_K 8.3 -> 6.9, Q6_K 4096 x 14336 at 2 rows 22.4 -> 15.0, at 8 rows 32.6 -> 24.5.  Error
+		// 4096 x 4096 at 3 rows 10.3 -> 7.6, Q4_K 8.3 -> 6.9, Q6_K 4096 x 14336 at 2 rows 22.4 -> 15.0, at 8 rows 32.6 -> 24.5.  Error
 		// against 64 bits up to 8 % lower.
 		template <int MR>
 		struct FewRows
@@ -2137,7 +2138,7 @@ namespace litenn_hip
 		template <typename F, int MR>
 		void launch_few_rows(const FewCall& c)
 		{
-			// Sixteen weight rows a workgroup while each has a CU to itself (us at 3 rows, sixteen and 32: Q8_0 4096 x 4096 7.8 and 10.3,
+			// Sixteen weight rows a workgroup while each has a CU to itself (us at 3 rows, sixteen and 32: Q8_0 4096 x 4096 7.6 and 10.3,
 			// 1024 x 4096 6.1 and 8.2, Q6_K 4096 x 14336 16.8 and 24.8; in a second round not: 6000 x 2048 9.0 and 7.7), in eight ranges of K.
 			if (c.n <= 256 * kFewTile)
 			{

@@ -1,5 +1,6 @@
 """How a pass's ids reach the device and its results the host: runs of more ids than the pinned memory has room for,
 passes of one run, states of all layers cleared by one call, results read at once by several threads."""
+import os
 import threading
 
 import numpy as np
@@ -38,10 +39,10 @@ def test_reset_clears_every_layer(hip):
             assert np.array_equal(model.eval(toks[80:81]), want[1])
 
 
-def test_models_in_threads(hip):
+def eval_in_threads(hip, count):
     cfg = ku.config([ku.linear_attention(mlp=ku.mlp()), ku.attention()])
     toks = ku.tokens(cfg, 60, 3)
-    models = [hip.create_model(cfg, ku.random_weights(cfg, seed), dtype="float32", context_length=64) for seed in range(3)]
+    models = [hip.create_model(cfg, ku.random_weights(cfg, seed), dtype="float32", context_length=64) for seed in range(count)]
     want = [np.concatenate([m.eval(toks[:20], want=[19])] + [m.eval(toks[i:i + 1]) for i in range(20, 60)]) for m in models]
     wrong = []
 
@@ -60,3 +61,17 @@ def test_models_in_threads(hip):
     for m in models:
         m.close()
     assert not wrong
+
+
+def test_models_in_threads(hip):
+    eval_in_threads(hip, 3)
+
+
+def test_models_in_more_threads_than_cores(hip):
+    """Threads that look at the marks of their passes while others, on the same core, have launches to make."""
+    cores = os.sched_getaffinity(0)
+    os.sched_setaffinity(0, sorted(cores)[:1])  # of this thread, and those that it starts
+    try:
+        eval_in_threads(hip, 8)
+    finally:
+        os.sched_setaffinity(0, cores)
